@@ -82,7 +82,10 @@ int dllm_retention(const void*, long, int, int, int, int, const float*, int, int
 long dllm_retention_chunk_lds(int);
 int dllm_retention_chunked(const void*, long, int, int, int, int, const float*, int, int, const float*, float*, float,
                            const int*, const int*, const int*, const int*, float*, void*, int, long, int, float, int,
-                           hipStream_t);
+                           float*, hipStream_t);
+long dllm_chunk_scan_scratch(long, int, int, int, int);
+int dllm_ssd_chunks(const void*, long, const void*, long, int, int, int, int, int, const float*, const float*, const float*, float*,
+                    const int*, const int*, const int*, const int*, int, long, float*, float*, hipStream_t);
 int dllm_heads_norm_gate(const float*, const void*, long, int, long, int, const float*, float, const int*, const int*, int,
                          void*, long, hipStream_t);
 int dllm_resadd_norm(const void*, long, const void*, long, int, const float*, const float*, const float*, float*,
@@ -1454,6 +1457,14 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
      "selective_scan");
 }
 
+// Chunk states of the chunk-parallel recurrences (chunk_scan.hip) for a step of T tokens and S sequences; undefined
+// where the key width is past 128 or the states would pass 4 GB (a step of several hundred thousand tokens).
+static torch::Tensor chunk_scratch(int64_t T, int S, int64_t H, int64_t d, int64_t dv, const torch::Tensor& like) {
+  const long n = dllm_chunk_scan_scratch((long)T, S, (int)H, (int)d, (int)dv);
+  if (n <= 0 || n > (1L << 30)) return {};
+  return torch::empty({n}, like.options().dtype(torch::kFloat32));
+}
+
 void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tensor cos_sin, int64_t rot,
                torch::Tensor decay, torch::Tensor state, double eps, torch::Tensor pos, torch::Tensor qstart,
                torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out,
@@ -1477,11 +1488,12 @@ void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tens
   if (raw) {   // chunked form (prompt portions): f32 scratch [T, H, dv]
     check_f32(*raw, "raw");
     TORCH_CHECK(raw->numel() >= (int64_t)T * H * dv, "raw scratch [T, H, dv]");
-    TORCH_CHECK(dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
+    const auto sc = chunk_scratch(T, m.S, H, d, dv, qkvg);
+    TORCH_CHECK(sc.defined() || dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
     ok(dllm_retention_chunked(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, cos_sin.data_ptr<float>(),
                               (int)cos_sin.size(1), (int)rot, decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps,
                               m.qstart, m.qlen, m.ctx, m.rows, raw->data_ptr<float>(), out.data_ptr(), m.S, (long)T, 0,
-                              1.f / std::sqrt((float)d), 1, stream()),
+                              1.f / std::sqrt((float)d), 1, sc.defined() ? sc.data_ptr<float>() : nullptr, stream()),
        "retention (chunked)");
     return;
   }
@@ -1514,10 +1526,12 @@ void lightning_attention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, t
   TORCH_CHECK(raw.numel() >= (int64_t)T * H * dv, "raw scratch [T, H, dv]");
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
   if (chunked) {
-    TORCH_CHECK(dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
+    const auto sc = chunk_scratch(T, m.S, H, d, dv, qkvg);
+    TORCH_CHECK(sc.defined() || dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
     ok(dllm_retention_chunked(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, decay.data_ptr<float>(), 0, 0,
                               decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps, m.qstart, m.qlen, m.ctx, m.rows,
-                              raw.data_ptr<float>(), out.data_ptr(), m.S, (long)T, 1, 1.f, 0, stream()),
+                              raw.data_ptr<float>(), out.data_ptr(), m.S, (long)T, 1, 1.f, 0,
+                              sc.defined() ? sc.data_ptr<float>() : nullptr, stream()),
        "lightning attention (chunked)");
   } else {
     TORCH_CHECK(dllm_retention_lds((int)d, (int)dv) <= 150 * 1024, "dim x vdim state does not fit the LDS");
@@ -1990,7 +2004,7 @@ void diff_combine(torch::Tensor a, int64_t H, int64_t G, int64_t dv, double lam,
 
 void ssd_scan(torch::Tensor xbc, torch::Tensor proj, int64_t dt_col, int64_t H, int64_t dv, int64_t N, int64_t G,
               torch::Tensor dt_bias, torch::Tensor neg_a, torch::Tensor D, torch::Tensor state, torch::Tensor qstart,
-              torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out) {
+              torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out, bool chunked) {
   const bool f = act_f32(xbc, "xbc");
   check_rows2d(xbc, "xbc");
   check_rows2d(proj, "proj");
@@ -2007,6 +2021,15 @@ void ssd_scan(torch::Tensor xbc, torch::Tensor proj, int64_t dt_col, int64_t H, 
               "state [slots, H, N, dv]");
   TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == xbc.size(0) && out.size(1) == H * dv, "out [T, H dv] f32");
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
+  const auto sc = chunked ? chunk_scratch(xbc.size(0), m.S, H, N, dv, xbc) : torch::Tensor();
+  if (sc.defined()) {
+    const char* gates = (const char*)proj.data_ptr() + dt_col * proj.element_size();
+    ok(dllm_ssd_chunks(xbc.data_ptr(), xbc.stride(0), gates, proj.stride(0), f, (int)H, (int)dv, (int)N, (int)G,
+                       dt_bias.data_ptr<float>(), neg_a.data_ptr<float>(), D.data_ptr<float>(), state.data_ptr<float>(), m.qstart,
+                       m.qlen, m.ctx, m.rows, m.S, (long)xbc.size(0), out.data_ptr<float>(), sc.data_ptr<float>(), stream()),
+       "ssd_scan (chunked)");
+    return;
+  }
   const int rc = dllm_ssd_scan(xbc.data_ptr(), xbc.stride(0), proj.data_ptr(), proj.stride(0), (int)dt_col, f, (int)H, (int)dv,
                                (int)N, (int)G, dt_bias.data_ptr<float>(), neg_a.data_ptr<float>(), D.data_ptr<float>(),
                                state.data_ptr<float>(), m.qstart, m.qlen, m.ctx, m.rows, m.S, out.data_ptr<float>(), stream());

@@ -594,7 +594,7 @@ __global__ void __launch_bounds__(256) retention_kernel(const T* __restrict__ qk
   for (int e = tid; e < d * dv; e += 256) sg[e] = S[e];
 }
 
-// ---------------------------------------------------------------- retention, chunked (prompt portions)
+// ---------------------------------------------------------------- retention, chunked (prompt portions with d > 128)
 // One workgroup per (head, 32-column slice of the value dim, sequence); tokens in chunks of 32.
 // With the chunk's rotated q / k (k scaled) and v slice in LDS and g = decay:
 //   A[t][s] = g^(t-s) q_t . k_s  (s <= t)            scores inside the chunk, f32
@@ -1323,31 +1323,43 @@ extern "C" long dllm_retention_chunk_lds(int d) {
   return 4L * (2L * RC_T * (d + 1) + RC_T * RC_V + RC_T * (RC_T + 1) + (long)d * RC_V + RC_T + 1);
 }
 
-// Chunked form for prompt portions: `raw` is an f32 scratch [T, H, dv].
+extern "C" int dllm_retention_chunks(const void*, long, int, int, int, int, const float*, int, int, const float*, float*, const int*,
+                                     const int*, const int*, const int*, float*, int, long, int, float, float*, hipStream_t);
+
+// Chunked form for prompt portions: `raw` is an f32 scratch [T, H, dv].  `scratch` (dllm_chunk_scan_scratch entries): the
+// chunk-parallel kernels of chunk_scan.hip; null (widths they do not take): chunks in order, one workgroup per
+// (head, 32 value columns, sequence).
 extern "C" int dllm_retention_chunked(const void* qkvg, long ld, int f32, int H, int d, int dv, const float* cos_sin,
                                       int tab_w, int rot, const float* decay, float* state, float eps, const int* qstart,
                                       const int* qlen, const int* ctx, const int* rows, float* raw, void* out, int S,
-                                      long T, int act, float kscale, int finish, hipStream_t st) {
+                                      long T, int act, float kscale, int finish, float* scratch, hipStream_t st) {
   if (S <= 0 || T <= 0) return 0;
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w) return -1;
   const long lds = dllm_retention_chunk_lds(d);
-  if (lds > 150 * 1024) return -2;
+  if (!scratch && lds > 150 * 1024) return -2;
   const dim3 g(H, (dv + RC_V - 1) / RC_V, S);
   const long rows_total = T * H;
   const dim3 gf((unsigned)((rows_total + 3) / 4));
-  if (f32) {
+  if (scratch) {
+    const int rc = dllm_retention_chunks(qkvg, ld, f32, H, d, dv, cos_sin, tab_w, rot, decay, state, qstart, qlen, ctx, rows, raw,
+                                         S, T, act, kscale, scratch, st);
+    if (rc) return rc;
+  } else if (f32) {
     ENSURE_LDS(retention_chunk_kernel<float>, lds);
     hipLaunchKernelGGL(retention_chunk_kernel<float>, g, dim3(256), lds, st, (const float*)qkvg, ld, H, d, dv, cos_sin, tab_w,
                        rot, decay, state, qstart, qlen, ctx, rows, raw, act, kscale);
-    if (finish) hipLaunchKernelGGL(retention_finish_kernel<float>, gf, dim3(256), 0, st, raw, (const float*)qkvg, ld, H, d, dv, eps, qstart,
-                       qlen, S, (float*)out, rows_total);
   } else {
     ENSURE_LDS(retention_chunk_kernel<u16>, lds);
     hipLaunchKernelGGL(retention_chunk_kernel<u16>, g, dim3(256), lds, st, (const u16*)qkvg, ld, H, d, dv, cos_sin, tab_w, rot,
                        decay, state, qstart, qlen, ctx, rows, raw, act, kscale);
-    if (finish) hipLaunchKernelGGL(retention_finish_kernel<u16>, gf, dim3(256), 0, st, raw, (const u16*)qkvg, ld, H, d, dv, eps, qstart, qlen,
-                       S, (u16*)out, rows_total);
   }
+  if (!finish) return (int)hipGetLastError();
+  if (f32)
+    hipLaunchKernelGGL(retention_finish_kernel<float>, gf, dim3(256), 0, st, raw, (const float*)qkvg, ld, H, d, dv, eps, qstart,
+                       qlen, S, (float*)out, rows_total);
+  else
+    hipLaunchKernelGGL(retention_finish_kernel<u16>, gf, dim3(256), 0, st, raw, (const u16*)qkvg, ld, H, d, dv, eps, qstart, qlen,
+                       S, (u16*)out, rows_total);
   return (int)hipGetLastError();
 }
 

@@ -102,7 +102,10 @@ def retention_step_lds(dim: int, vdim: int) -> int:
     return 4 * (dim * vdim + 8 * (2 * dim + 2 * vdim) + 2 * (256 // lj) * vdim)
 
 
-RETENTION_CHUNK_MIN = 4    # average new tokens per sequence from which the chunked kernel runs
+# average new tokens per sequence from which the chunk-parallel kernels run: about 25 us of launches against the serial
+# tokens of one workgroup per head (24 sequences of 8 tokens: 41 against 35 us for 8 heads of 64 x 128, 73 against 109
+# for 16 of 128 x 128; of 16 tokens: 44 against 62 and 80 against 204; 48 of 4: 57 against 23 and 117 against 95)
+RETENTION_CHUNK_MIN = 8
 
 
 def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen, ctx,
@@ -423,18 +426,27 @@ def scan_col_blocks(vdim: int) -> int:
     return (int(vdim) + SCAN_COLS - 1) // SCAN_COLS
 
 
+SSD_CHUNK_MIN = 48     # average new tokens per sequence from which the chunk-parallel kernels run: three launches and the chunk
+                       # states against 0.34 us a token (32 heads of 128 x 64, one sequence: 64 tokens 31 against 24 us, 256
+                       # tokens 40 against 74; 48 sequences: 16 tokens 72 against 64, 32 tokens 86 against 106)
+
+
 def ssd_scan(xbc, proj, dt_col, heads, vdim, n_state, groups, dt_bias, neg_a, D, state, qstart, qlen, ctx,
-             rows) -> torch.Tensor:
+             rows, chunked: Optional[bool] = None) -> torch.Tensor:
     """Mamba-2 recurrence (scalar decay per head, B / C per group of heads): xbc [T, x | B | C]
     convolved and activated, step logits in proj[:, dt_col:dt_col + heads]; dt = softplus(. + bias),
-    S <- exp(neg_a dt) S + dt B x^T, y = S^T C + D x.  state [slots, heads, N, vdim] f32; returns y f32."""
+    S <- exp(neg_a dt) S + dt B x^T, y = S^T C + D x.  state [slots, heads, N, vdim] f32; returns y f32.
+    ``chunked`` (GPU): the chunk-parallel kernels (N <= 128) or the token-by-token one; default by the
+    step's tokens per sequence."""
     ext = _native(xbc)
     if ext is None:
         return ref.ssd_scan(xbc, proj, dt_col, heads, vdim, n_state, groups, dt_bias, neg_a, D, state, qstart, qlen, ctx,
                             rows)
     out = torch.zeros((xbc.shape[0], heads * vdim), dtype=torch.float32, device=xbc.device)
+    if chunked is None:
+        chunked = xbc.shape[0] >= SSD_CHUNK_MIN * qstart.numel()
     ext.ssd_scan(xbc, proj, int(dt_col), int(heads), int(vdim), int(n_state), int(groups), dt_bias, neg_a, D, state,
-                 qstart, qlen, ctx, rows, out)
+                 qstart, qlen, ctx, rows, out, bool(chunked))
     return out
 
 

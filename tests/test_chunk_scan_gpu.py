@@ -1,0 +1,112 @@
+"""Chunk-parallel recurrences (csrc/kernels/chunk_scan.hip) against 64-bit recurrences written out here, at the edges
+of their chunks (64 tokens), tiles (16, 32, 64, 128 wide) and vectors (4 elements), and beside the token-by-token
+kernels.  In 32 bits a result is a sum of at most 64 + d products and one carried state: with roundings of 2^-24 that
+act like a random walk the relative error stays below sqrt(64 + 128) 2^-24 times a few (gates, powers), 4e-6."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from distributed_llm_amd import ops
+from distributed_llm_amd.ops import seqmix
+from test_seqmix_gpu import batch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+EDGES = [([63, 64, 65], [0, 7, 64]), ([1, 0, 200, 16], [3, 2, 0, 0]), ([385], [0])]
+
+
+@pytest.fixture(autouse=True, scope="module")
+def _native():
+    assert ops.native_available(), "HIP extension must be built for GPU tests"
+
+
+def close(got, want, bound):
+    assert torch.isfinite(got).all()
+    assert float((got.double() - want).norm() / want.norm()) < bound
+
+
+def recur(q, k, v, dec, state, qlens, starts, rows):
+    """S <- dec_t S + k_t v_t^T, y_t = S^T q_t in 64 bits, per sequence; state [slots, H, d, dv] is updated."""
+    out, t0 = torch.zeros_like(v), 0
+    for s, (n, a) in enumerate(zip(qlens, starts)):
+        if n == 0:
+            continue
+        S = state[rows[s]].clone() if a else torch.zeros_like(state[0])
+        for t in range(t0, t0 + n):
+            S = dec[t, :, None, None] * S + k[t, :, :, None] * v[t, :, None, :]
+            out[t] = (S * q[t, :, :, None]).sum(1)
+        state[rows[s]] = S
+        t0 += n
+    return out
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", EDGES)
+@pytest.mark.parametrize("H,d,dv,rot", [(2, 64, 128, 64), (3, 20, 70, 10), (1, 128, 130, 0), (2, 33, 7, 32), (2, 96, 32, 6)])
+def test_retention(dt, case, H, d, dv, rot):
+    torch.manual_seed(31)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, pos = batch(qlens, starts)
+    x = torch.randn(T, 2 * H * d + 2 * H * dv, device=DEV).to(dt)
+    table = ops.rope_cos_sin(512, max(rot, 2), 10000.0, DEV)
+    dec = torch.tensor([1.0 - 2.0 ** (-2 - 3 * h) for h in range(H)], device=DEV)
+    st = torch.randn(len(qlens), H, d, dv, device=DEV)
+    s64, s32 = st.double(), st.clone()
+    got = seqmix.retention(x, H, d, dv, table, rot, dec, s32, 1e-6, pos, qstart, qlen, ctx, rows, chunked=True)
+    y = x.double()
+    q, k, v, g = y.split([H * d, H * d, H * dv, H * dv], 1)
+    q, k, h2 = q.view(T, H, d).clone(), k.view(T, H, d).clone(), rot // 2
+    c, s = (table[pos.long()].double()[:, None, i * h2:(i + 1) * h2] for i in range(2))
+    for z in (q, k):
+        a, b = z[..., :h2].clone(), z[..., h2:rot].clone()
+        z[..., :h2], z[..., h2:rot] = a * c - b * s, b * c + a * s
+    o = recur(q, k * d ** -0.5, v.view(T, H, dv), dec.double().expand(T, H), s64, qlens, starts, rows.tolist())
+    o = o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-6)
+    close(got, o.reshape(T, -1) * F.silu(g), 4e-6 if dt == torch.float32 else 4e-3)
+    close(s32, s64, 4e-6)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", EDGES)
+@pytest.mark.parametrize("H,d,dv", [(3, 128, 128), (2, 40, 48), (1, 5, 6)])
+def test_lightning(dt, case, H, d, dv):
+    torch.manual_seed(32)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    x = torch.randn(T, 2 * H * d + 2 * H * dv + 4, device=DEV).to(dt)
+    dec = torch.tensor([0.5, 0.97, 1.0][:H], device=DEV)
+    st, nw = torch.randn(len(qlens), H, d, dv, device=DEV), torch.randn(H * dv, device=DEV)
+    s64, s32 = st.double(), st.clone()
+    got = seqmix.lightning_attention(x, H, d, dv, dec, s32, 1e-5, nw, qstart, qlen, ctx, rows, chunked=True)
+    q, k, v, g, _ = x.double().split([H * d, H * d, H * dv, H * dv, 4], 1)
+    o = recur(F.silu(q).view(T, H, d), F.silu(k).view(T, H, d), F.silu(v).view(T, H, dv), dec.double().expand(T, H), s64, qlens, starts,
+              rows.tolist()).reshape(T, -1)
+    o = o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-5) * nw.double() * torch.sigmoid(g)
+    close(got, o, 4e-6 if dt == torch.float32 else 4e-3)
+    close(s32, s64, 4e-6)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", EDGES)
+@pytest.mark.parametrize("H,dv,N,G", [(4, 64, 128, 2), (3, 40, 20, 3), (2, 130, 33, 1), (2, 7, 5, 2)])
+def test_ssd(dt, case, H, dv, N, G):
+    torch.manual_seed(33)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    xbc = torch.randn(T, H * dv + 2 * G * N, device=DEV).to(dt)
+    proj = torch.randn(T, H + 3, device=DEV).to(dt)
+    # steep and flat decays: a head that forgets within a few tokens, one that keeps everything
+    dt_b, neg_a, D = torch.randn(H, device=DEV), -torch.tensor([8.0, 0.5, 1e-3, 0.05][:H], device=DEV), torch.randn(H, device=DEV)
+    st = torch.randn(len(qlens), H, N, dv, device=DEV)
+    outs = []
+    for chunked in (True, False):
+        s64, s32 = st.double(), st.clone()
+        got = seqmix.ssd_scan(xbc, proj, 2, H, dv, N, G, dt_b, neg_a, D, s32, qstart, qlen, ctx, rows, chunked=chunked)
+        v, B, C = xbc.double().split([H * dv, G * N, G * N], 1)
+        B, C = (z.view(T, G, N).repeat_interleave(H // G, 1) for z in (B, C))
+        step, v = F.softplus(proj[:, 2:2 + H].double() + dt_b.double(), threshold=40), v.view(T, H, dv)
+        o = recur(C, B * step[..., None], v, torch.exp(step * neg_a.double()), s64, qlens, starts, rows.tolist()) + D.double()[:, None] * v
+        close(got, o.reshape(T, -1), 4e-6)
+        close(s32, s64, 4e-6)
+        outs.append(float((got.double() - o.reshape(T, -1)).norm() / o.norm()))
+    assert outs[0] < 2 * outs[1] + 1e-7      # as exact as the token-by-token form
