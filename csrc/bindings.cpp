@@ -24,7 +24,7 @@ int dllm_gemv(const void*, long, const void*, void*, long, int, int, int, int, i
 int dllm_gelu(const void*, void*, long, hipStream_t);
 int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, hipStream_t);
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
-int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, hipStream_t);
+int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, hipStream_t);
 int dllm_scatter_pairs(int*, const int*, int, hipStream_t);
 int dllm_step_fetch(const int*, int*, int, int, int, int, const int*, const int*, int*, int, hipStream_t);
 int dllm_step_store(const int*, int*, int, hipStream_t);
@@ -136,7 +136,7 @@ int dllm_car_vote(int, int*, void*, int*, hipStream_t);
 int dllm_tgemm(const void*, int, int, int, int, int, int, int, hipStream_t, int);
 int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
-                    int*, int*, int*, void*, void*, void*, const int*, hipStream_t);
+                    int*, int*, int*, void*, void*, void*, int, const int*, hipStream_t);
 int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
                   float, hipStream_t);
@@ -426,8 +426,9 @@ void moe_gate(torch::Tensor logits, int64_t k, torch::Tensor ids, torch::Tensor 
 }
 
 // fused router GEMV + top-k (batch-invariant): x [T, H] (row stride % 8), wg [E, H] -> ids/w [T, k]
+// scale multiplies the weights; with shared a token gets one more pair, (E, 1)
 void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids, torch::Tensor w,
-                c10::optional<torch::Tensor> logits) {
+                c10::optional<torch::Tensor> logits, bool shared, double scale) {
   check_bf16(x, "x");
   check_bf16(wg, "router weight");
   check_i32(ids, "ids");
@@ -435,8 +436,8 @@ void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids,
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && wg.dim() == 2 && wg.is_contiguous() && wg.size(1) == x.size(1),
               "x [T, H] row-major, wg [E, H] contiguous");
   const int T = x.size(0), E = wg.size(0), H = x.size(1);
-  TORCH_CHECK(ids.numel() == (int64_t)T * k && w.numel() == (int64_t)T * k && ids.is_contiguous() && w.is_contiguous(),
-              "out shapes");
+  const int64_t n = (int64_t)T * (k + (shared ? 1 : 0));
+  TORCH_CHECK(ids.numel() == n && w.numel() == n && ids.is_contiguous() && w.is_contiguous(), "out shapes");
   float* lp = nullptr;
   if (logits.has_value()) {
     check_f32(*logits, "logits");
@@ -444,7 +445,7 @@ void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids,
     lp = logits->data_ptr<float>();
   }
   ok(dllm_moe_router(x.data_ptr(), x.stride(0), wg.data_ptr(), T, E, H, k, ids.data_ptr<int>(), w.data_ptr<float>(),
-                     lp, stream()),
+                     lp, (int)shared, (float)scale, stream()),
      "moe_router");
 }
 
@@ -912,9 +913,10 @@ void gemv_swiglu(torch::Tensor x, torch::Tensor w, torch::Tensor ssq, int64_t ss
 // Mixtral-style MoE FFN: x [T, H] bf16, ids [T, k] int32, wts [T, k] f32, w13 [E, 2I, H], w2 [E, H, I]
 // -> out [T, H] bf16 (partial sum over this rank's I shard under TP).  Workspace from torch's
 // caching allocator, so the call is graph-capturable.
-// grouped-tgemm MoE (csrc/kernels/moe.hip dllm_moe_ffn_tg): w13 interleaved per 16-row group
+// grouped-tgemm MoE (csrc/kernels/moe.hip dllm_moe_ffn_tg): act_mode 0: w13 [E, 2I, H] interleaved per 16-row
+// group; 1: squared-ReLU experts, w13 [E, I, H]
 void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Tensor w13, torch::Tensor w2,
-                torch::Tensor out, std::vector<int64_t> plan) {
+                torch::Tensor out, std::vector<int64_t> plan, int64_t act_mode) {
   check_bf16(x, "x");
   check_i32(ids, "ids");
   check_f32(wts, "wts");
@@ -923,12 +925,13 @@ void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Te
   check_bf16(out, "out");
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && out.is_contiguous(), "x rows 16-B aligned");
   TORCH_CHECK(w13.dim() == 3 && w2.dim() == 3 && w13.is_contiguous() && w2.is_contiguous(), "w13/w2 [E, N, K]");
-  const int64_t T = x.size(0), H = x.size(1), E = w13.size(0), I = w13.size(1) / 2;
+  const int64_t T = x.size(0), H = x.size(1), E = w13.size(0), I = w13.size(1) / (act_mode ? 1 : 2);
   TORCH_CHECK(w13.size(2) == H && w2.size(0) == E && w2.size(1) == H && w2.size(2) == I, "expert weight shapes");
   TORCH_CHECK(H % 64 == 0 && I % 64 == 0 && E <= 64, "H, I multiples of 64; E <= 64");
   TORCH_CHECK(ids.dim() == 2 && ids.size(0) == T && wts.sizes() == ids.sizes() && ids.is_contiguous() &&
                   wts.is_contiguous(), "ids/wts [T, k]");
   TORCH_CHECK(out.size(0) == T && out.size(1) == H, "out shape");
+  TORCH_CHECK(act_mode == 0 || act_mode == 1, "act_mode 0 or 1");
   TORCH_CHECK(plan.size() == 9, "plan: bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2");
   const int bm = (int)plan[0];
   for (int g = 0; g < 2; ++g) {
@@ -947,12 +950,12 @@ void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Te
   auto inv = torch::empty({std::max(P, 1)}, iopt);
   auto tiles = torch::empty({4 * mt + 1}, iopt);
   auto act = torch::empty({std::max(P, 1), I}, x.options());
-  auto y = torch::empty({std::max(P, 1), H}, x.options());
+  auto y = torch::empty({std::max(P, 1), H}, act_mode ? wts.options() : x.options());
   int pl[9];
   for (int i = 0; i < 9; ++i) pl[i] = (int)plan[i];
   ok(dllm_moe_ffn_tg(x.data_ptr(), x.stride(0), T, (int)H, ids.data_ptr<int>(), wts.data_ptr<float>(), k, (int)E,
                      w13.data_ptr(), w2.data_ptr(), (int)I, perm.data_ptr<int>(), inv.data_ptr<int>(),
-                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), out.data_ptr(), pl, stream()),
+                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), out.data_ptr(), (int)act_mode, pl, stream()),
      "moe_ffn_tg");
 }
 
@@ -2500,7 +2503,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("embed_ln", &embed_ln);
   m.def("moe_ffn", &moe_ffn, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
         py::arg("act_mode") = 0);
-  m.def("moe_ffn_tg", &moe_ffn_tg);
+  m.def("moe_ffn_tg", &moe_ffn_tg, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
+        py::arg("plan"), py::arg("act_mode") = 0);
   m.def("tgemm", &tgemm);
   m.def("res_add_ssq", &res_add_ssq);
   m.def("qkv_post", &qkv_post, py::arg("y"), py::arg("ssq"), py::arg("ssq_n"), py::arg("scale"), py::arg("eps"),
@@ -2533,7 +2537,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("mean_pool_l2", &mean_pool_l2);
   m.def("moe_gate", &moe_gate);
   m.def("moe_router", &moe_router, py::arg("x"), py::arg("wg"), py::arg("k"), py::arg("ids"), py::arg("w"),
-        py::arg("logits") = py::none());
+        py::arg("logits") = py::none(), py::arg("shared") = false, py::arg("scale") = 1.0);
   m.def("argmax", &argmax);
   m.def("scatter_pairs", &scatter_pairs);
   m.def("step_fetch", &step_fetch);

@@ -13,6 +13,7 @@
 //   EPI_SWIGLU : act = silu(g) * u with [g | u] = (r . Wgu'^T) * rinv[m]  (interleaved gate/up rows)
 //   EPI_RESADD : r += act . Wd^T  (+ partial sums of squares)
 //   EPI_GELU   : y = gelu(x . W^T + bias)  (encoder FFN; PLAIN and RESADD take the same bias)
+//   EPI_RELU2  : y = relu(x . W^T)^2, EPI_F32 : y = x . W^T kept in f32  (grouped squared-ReLU experts)
 //
 // RMSNorm folding: rmsnorm(r) * gamma . W^T = rinv[m] * (r . (W * gamma)^T), gamma folded into the
 // weight columns once at load time; rinv[m] = rsqrt(sum(r^2) / K + eps) comes from the producer
@@ -44,6 +45,8 @@ using dllm::EPI_RESADD;
 using dllm::EPI_QKV;
 using dllm::EPI_SWIGLU;
 using dllm::EPI_GELU;
+using dllm::EPI_RELU2;
+using dllm::EPI_F32;
 constexpr int BK = 64;
 constexpr int ROWB = BK * 2;  // 128 bytes per staged row
 
@@ -595,6 +598,27 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
       rinv[i][e] = r;
     }
 
+  if constexpr (EPI == EPI_F32) {
+    // straight from the accumulators: the 16 lanes of a row write 64 contiguous bytes
+    static_assert(MF == 16, "16 x 16 x 32 plans");
+    if (fw) {
+      float* yf = reinterpret_cast<float*>(a.Y);
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int m = m0 + rl0 + 16 * i + e;
+          if (m >= M) continue;
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const int n = n0 + wn * WN + 16 * j + cl;
+            if (n < N) yf[(long)m * a.ldy + n] = acc[i][j][e];
+          }
+        }
+    }
+    return;
+  }
+
   // Output staging: every epilogue writes its bf16 results into an LDS image of the tile
   // ([BM][OW + 8] bf16, row pad = one 16-B slot against bank conflicts; the ring is idle now)
   // and the block then copies it out as 16-B row vectors, so global stores are full-width and
@@ -766,6 +790,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
           for (int j = 0; j < FN; ++j) {
             float v = acc[i][j][e] * rinv[i][e] + bcol[j];
             if constexpr (EPI == EPI_GELU) v = gelu_erf(bfr(v));  // GELU of the bf16 linear output
+            if constexpr (EPI == EPI_RELU2) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
             so[rl * OLD + wn * WN + 16 * j + cl] = f2bf(v);
           }
         }
@@ -1051,6 +1076,18 @@ int by_tile(int bm, int bn, int stages, int ks, int nw, int wk, const GemmArgs& 
   return -20;
 }
 
+// the plans of ops.MOE_PLANS, for the epilogues that only grouped calls take
+template <int EPI>
+int by_tile_grouped(int bm, int bn, int stages, int ks, int nw, const GemmArgs& a, hipStream_t st) {
+  if (ks != 1) return -20;
+  if (bm == 64 && bn == 128 && stages == 3 && nw == 4) return launch_fit<64, 128, EPI, 3, 1, 4>(a, st);
+  if (bm == 64 && bn == 64 && stages == 6 && nw == 4) return launch_fit<64, 64, EPI, 6, 1, 4>(a, st);
+  if (bm == 128 && bn == 128 && stages == 4 && nw == 8) return launch_fit<128, 128, EPI, 4, 1, 8>(a, st);
+  if (bm == 256 && bn == 128 && stages == 3 && nw == 8) return launch_fit<256, 128, EPI, 3, 1, 8>(a, st);
+  if (bm == 256 && bn == 256 && stages == 2 && nw == 8) return launch_fit<256, 256, EPI, 2, 1, 8>(a, st);
+  return -20;
+}
+
 // Residual-stream helpers for the paths the GEMM epilogue cannot cover (first layer's embedding,
 // tensor-parallel all-reduced outputs, MoE outputs): one wave per row, 16-B vectors.
 //   res_add_ssq: r = bf16(h + r) in place (h may be null: r unchanged) and the row's partial sums
@@ -1303,6 +1340,8 @@ extern "C" int dllm_tgemm(const void* args, int bm, int bn, int stages, int ks, 
     case EPI_QKV: return by_tile<EPI_QKV>(bm, bn, stages, ks, nw, wk, a, stream);
     case EPI_SWIGLU: return by_tile<EPI_SWIGLU>(bm, bn, stages, ks, nw, wk, a, stream);
     case EPI_GELU: return by_tile<EPI_GELU>(bm, bn, stages, ks, nw, wk, a, stream);
+    case EPI_RELU2: return a.g_tiles && wk == 1 ? by_tile_grouped<EPI_RELU2>(bm, bn, stages, ks, nw, a, stream) : -6;
+    case EPI_F32: return a.g_tiles && wk == 1 ? by_tile_grouped<EPI_F32>(bm, bn, stages, ks, nw, a, stream) : -6;
     default: return -6;
   }
 }

@@ -66,5 +66,6 @@ struct GemmArgs {
   // they share G activation and 32 / G weight panels; tgemm.hip tgemm_kernel)
   int raster;
 };
-enum { EPI_PLAIN = 0, EPI_RESADD = 1, EPI_QKV = 2, EPI_SWIGLU = 3, EPI_GELU = 4 };
+// RELU2 (y = relu(.)^2) and F32 (Y is float [M, N], no staging): grouped mode only
+enum { EPI_PLAIN = 0, EPI_RESADD = 1, EPI_QKV = 2, EPI_SWIGLU = 3, EPI_GELU = 4, EPI_RELU2 = 5, EPI_F32 = 6 };
 }  // namespace dllm

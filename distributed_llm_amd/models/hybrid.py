@@ -21,9 +21,10 @@ they do not take and for f32 models), everything between them on the HIP kernels
              the down projection) -> out-proj.  Steps of longer prompt portions make every head's keys
              and values from the latents they read, in scratch pages, and run the grouped-query kernel
              on them instead
-  experts    fused router (f32 softmax top-k, renormalised) -> grouped squared-ReLU expert GEMMs, or
-             the dense form (all experts' columns, unused ones gated to zero) for f32 models and
-             unaligned widths -> plus the shared expert
+  experts    fused router (f32 softmax top-k, renormalised) -> grouped squared-ReLU expert GEMMs (a shared
+             expert of the same width runs with them as one more expert of every token), or the dense
+             form (all experts' columns, unused ones gated to zero) for f32 models and unaligned widths
+             -> plus the shared expert
   delta      one fused projection (q | k | v | gate | beta | decay logits) -> causal conv + SiLU ->
              gated delta rule (unit q / k, decay, beta, f32 state per slot, per-head norm and SiLU
              gate in the kernel) -> out-proj
@@ -489,6 +490,12 @@ class HybridModel:
                 else:
                     w1 = torch.stack([t[p + f"mlp.e{e}.up"] for e in range(f.experts)])   # [E, ff, W]
                 w2 = torch.stack([t[p + f"mlp.e{e}.down"] for e in range(f.experts)])     # [E, W, ff]
+                if (f.act == "relu2" and f.shared_ff == f.ff and f.experts < 64 and f.top <= 8 and dt == torch.bfloat16
+                        and dev.type == "cuda" and W % 64 == 0 and f.ff % 64 == 0):
+                    # a shared expert as wide as the routed ones is one more expert that every token runs
+                    w1 = torch.cat([w1, t[p + "mlp.shared.up"][None]], 0)
+                    w2 = torch.cat([w2, t[p + "mlp.shared.down"][None]], 0)
+                    D["shared_in"] = True
                 grouped = (dt == torch.bfloat16 and dev.type == "cuda" and W % 32 == 0 and f.ff % 32 == 0
                            and f.experts <= 64)
                 if f.act == "swiglu" and grouped and W % 64 == 0 and f.ff % 64 == 0:
@@ -501,7 +508,7 @@ class HybridModel:
                     D["w2"] = put(w2)
                 else:   # dense form: one down projection over every expert's columns
                     D["w2d"] = put(w2.permute(1, 0, 2).reshape(W, f.experts * f.ff))
-                if f.shared_ff:
+                if f.shared_ff and "shared_in" not in D:
                     D["sh_up"], D["sh_down"] = put(t[p + "mlp.shared.up"]), put(t[p + "mlp.shared.down"])
                     if f.act == "swiglu":     # gate rows, then up rows
                         D["sh_up"] = put(torch.cat([t[p + "mlp.shared.gate"], t[p + "mlp.shared.up"]], 0))
@@ -568,7 +575,8 @@ class HybridModel:
                     continue
                 b = x.numel() * x.element_size()
                 if k in ("w1", "w2", "w2d") and top_only and isinstance(S.mlp, MoESpec):
-                    b = b * S.mlp.top // S.mlp.experts
+                    e = int("shared_in" in L)
+                    b = b * (S.mlp.top + e) // (S.mlp.experts + e)
                 n += b
         return n
 
@@ -1006,14 +1014,17 @@ class HybridModel:
     def _experts(self, L, f: MoESpec, x):
         if f.act == "swiglu":
             return self._experts_swiglu(L, f, x)
+        if "shared_in" in L:
+            ids, w = ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
+            return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"])
         if f.experts > 64 or f.top > 8:      # beyond the router kernels' register budget: library top-k
             val, ids = torch.topk(torch.softmax(F.linear(x.float(), L["router"].float()), -1), f.top, -1)
-            ids, w = ids.to(torch.int32), val / (val.sum(-1, keepdim=True) + 1e-20)
+            ids, w = ids.to(torch.int32), val / (val.sum(-1, keepdim=True) + 1e-20) * f.scale
         elif x.is_cuda and x.dtype == torch.bfloat16:
-            ids, w = ops.moe_router(x, L["router"], f.top)      # f32 logits, softmax over the chosen = s / sum s
+            ids, w = ops.moe_router(x, L["router"], f.top, scale=f.scale)   # f32 logits, softmax over the chosen = s / sum s
         else:
             ids, w = ops.moe_gate(F.linear(x.float(), L["router"].float()), f.top)
-        w = w * f.scale
+            w = w * f.scale
         if "w2" in L and (not x.is_cuda or seqmix.moe_ffn_relu2_ok(x, L["w1"])):
             y = seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"])
         else:

@@ -406,18 +406,25 @@ def moe_gate(logits: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     return ids, w
 
 
-def moe_router(x: torch.Tensor, wg: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:
+def moe_router(x: torch.Tensor, wg: torch.Tensor, k: int, shared: bool = False,
+               scale: float = 1.0) -> Tuple[torch.Tensor, torch.Tensor]:
     """Router projection + top-k in one kernel (csrc/kernels/elementwise.hip moe_router_kernel):
     fp32 logits x . wg^T with a per-token fixed reduction order, so routing is batch-invariant (a
     padded graph batch picks the same experts as the eager batch; a vendor GEMM's split varies
-    with M).  x [T, H] bf16, wg [E, H] bf16 -> ids [T, k] int32, renormalised weights [T, k] f32."""
+    with M).  x [T, H] bf16, wg [E, H] bf16 -> ids [T, k] int32, renormalised weights times ``scale``
+    [T, k] f32.  ``shared``: one more pair per token, expert E with weight 1 (a shared expert stored
+    behind the routed ones)."""
     ext = _native(x)
     if ext is None or x.shape[1] > 8192 or x.shape[1] % 8 or x.stride(0) % 8 or x.data_ptr() % 16 or wg.data_ptr() % 16:
-        return moe_gate(torch.nn.functional.linear(x.float(), wg.float()), k)
-    T = x.shape[0]
-    ids = torch.empty((T, k), dtype=torch.int32, device=x.device)
-    w = torch.empty((T, k), dtype=torch.float32, device=x.device)
-    ext.moe_router(x if x.stride(1) == 1 else x.contiguous(), wg.contiguous(), k, ids, w)
+        ids, w = moe_gate(torch.nn.functional.linear(x.float(), wg.float()), k)
+        w = w if scale == 1.0 else w * scale
+        if shared:
+            ids, w = torch.cat([ids, torch.full_like(ids[:, :1], wg.shape[0])], 1), torch.cat([w, torch.ones_like(w[:, :1])], 1)
+        return ids, w
+    T, n = x.shape[0], k + int(shared)
+    ids = torch.empty((T, n), dtype=torch.int32, device=x.device)
+    w = torch.empty((T, n), dtype=torch.float32, device=x.device)
+    ext.moe_router(x if x.stride(1) == 1 else x.contiguous(), wg.contiguous(), k, ids, w, None, bool(shared), float(scale))
     return ids, w
 
 

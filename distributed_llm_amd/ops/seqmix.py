@@ -30,7 +30,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import _native, reference as ref
+from . import _native, moe_plan, reference as ref
 
 LAT_ROWS = 16      # (token, head) rows per workgroup of the latent attention kernel; a tile entry
                    # (sequence, first token) covers max(1, 16 // heads) tokens (AttnMeta.latent_tiles)
@@ -218,14 +218,24 @@ def relu2_scale(x: torch.Tensor, gate: Optional[torch.Tensor] = None, ff: int = 
 
 
 def moe_ffn_relu2(x, ids, wts, w1, w2) -> torch.Tensor:
-    """Top-k experts with a squared-ReLU activation and no gate projection on the grouped MFMA
-    kernels of the SwiGLU experts (csrc/kernels/moe.hip, activation mode 1)."""
+    """Top-k experts with a squared-ReLU activation and no gate projection (csrc/kernels/moe.hip, activation
+    mode 1): on the LDS-tiled grouped GEMM where it takes the widths (multiples of 64), else on the
+    32-row grouped kernels."""
     ext = _native(x)
     if ext is None:
         return ref.moe_ffn_relu2(x, ids, wts, w1, w2)
     out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
-    ext.moe_ffn(x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w1, w2, out, 1)
+    ids, wts = ids.to(torch.int32).contiguous(), wts.float().contiguous()
+    if moe_ffn_relu2_tg_ok(x, w1):
+        ext.moe_ffn_tg(x, ids, wts, w1, w2, out, list(moe_plan(x.shape[0] * ids.shape[1])), 1)
+    else:
+        ext.moe_ffn(x, ids, wts, w1, w2, out, 1)
     return out
+
+
+def moe_ffn_relu2_tg_ok(x: torch.Tensor, w1: torch.Tensor) -> bool:
+    """Widths of the LDS-tiled grouped GEMM."""
+    return moe_ffn_relu2_ok(x, w1) and x.shape[1] % 64 == 0 and w1.shape[1] % 64 == 0 and x.data_ptr() % 16 == 0
 
 
 def moe_ffn_relu2_ok(x: torch.Tensor, w1: torch.Tensor) -> bool:
