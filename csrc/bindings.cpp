@@ -73,6 +73,9 @@ int dllm_qk_norm_prep(const void*, long, int, const float*, int, int, int, int, 
 int dllm_diff_combine(const float*, void*, int, long, int, int, int, float, float, float, hipStream_t);
 int dllm_conv_silu(const void*, long, int, const float*, const float*, void*, const int*, const int*, const int*,
                    const int*, void*, int, int, int, int, int, int, hipStream_t);
+long dllm_scan_chunks_scratch(long, int, int, int);
+int dllm_scan_chunks(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*, const void*, long,
+                     float*, void*, int, const int*, const int*, const int*, const int*, void*, int, long, int, int, float*, hipStream_t);
 int dllm_selective_scan(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*,
                         const void*, long, float*, void*, int, const int*, const int*, const int*, const int*, void*, int,
                         int, int, hipStream_t);
@@ -1431,7 +1434,8 @@ void causal_conv_silu(torch::Tensor x, torch::Tensor w, torch::Tensor b, torch::
 
 void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bias, torch::Tensor A, torch::Tensor dbc,
                     int64_t dt_rank, torch::Tensor D, torch::Tensor xz, torch::Tensor ssm, torch::Tensor conv,
-                    torch::Tensor qstart, torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out) {
+                    torch::Tensor qstart, torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out,
+                    bool chunked) {
   const bool f = act_f32(xc, "xc");
   for (auto* t : {&dt_raw, &dbc, &xz, &out, &conv})
     TORCH_CHECK(t->is_cuda() && t->scalar_type() == xc.scalar_type(), "activations share one dtype");
@@ -1453,6 +1457,16 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
   TORCH_CHECK(conv.is_contiguous() && conv.dim() == 3 && conv.size(0) == ssm.size(0) && conv.size(2) == C,
               "conv_state [slots, K - 1, C]");
   auto m = seq_meta(qstart, qlen, ctx, rows, ssm.size(0));
+  const long ns = chunked ? dllm_scan_chunks_scratch(T, m.S, C, N) : 0;
+  if (ns > 0 && ns <= (1L << 30)) {      // chunk-parallel form (prompt portions)
+    auto sc = torch::empty({ns}, xc.options().dtype(torch::kFloat32));
+    ok(dllm_scan_chunks(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(), dbc.data_ptr(),
+                        dbc.stride(0), (int)dt_rank, D.data_ptr<float>(), xz.data_ptr(), xz.stride(0), ssm.data_ptr<float>(),
+                        conv.data_ptr(), (int)conv.size(1), m.qstart, m.qlen, m.ctx, m.rows, out.data_ptr(), m.S, (long)T, C, N,
+                        sc.data_ptr<float>(), stream()),
+       "selective_scan (chunked)");
+    return;
+  }
   ok(dllm_selective_scan(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(),
                          dbc.data_ptr(), dbc.stride(0), (int)dt_rank, D.data_ptr<float>(), xz.data_ptr(), xz.stride(0),
                          ssm.data_ptr<float>(), conv.data_ptr(), (int)conv.size(1), m.qstart, m.qlen, m.ctx, m.rows,

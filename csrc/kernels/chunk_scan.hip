@@ -28,6 +28,7 @@
 // there (bf16 rows): sums 154, carry 53, outputs 250 us.  One prompt of 4096 tokens, with its norm and gate: retention
 // with 8 heads of 64 x 128 104 us, with 16 of 128 x 128 230 us, against 1900 and 2910 us for chunks in order
 // (seqmix.hip); Mamba-2 with 32 heads of 128 x 64 178 us against 1390 us token by token (outer_scan.hip).
+#include "chunks.h"
 #include "common.h"
 
 namespace {
@@ -97,34 +98,6 @@ template <typename T> __device__ __forceinline__ float4 ld_qk(const ScanArgs& a,
   return x;
 }
 
-__device__ __forceinline__ int wave_scan_i(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o);
-    if (lane >= o) v += u;
-  }
-  return v;
-}
-
-// chunk number `flat` over all sequences -> its sequence and place there; false past the last one
-__device__ __forceinline__ bool find_chunk(const int* qlen, int S, int flat, int& s, int& c) {
-  const int lane = threadIdx.x & 63;
-  int base = 0;
-  for (int i0 = 0; i0 < S; i0 += 64) {
-    const int n = i0 + lane < S ? (max(qlen[i0 + lane], 0) + CS_L - 1) / CS_L : 0;
-    const int up = wave_scan_i(n, lane);
-    const unsigned long long m = __ballot(base + up > flat);
-    if (m) {
-      const int l = __ffsll((unsigned long long)m) - 1;
-      s = i0 + l;
-      c = flat - base - (__shfl(up, l) - __shfl(n, l));
-      return true;
-    }
-    base += __shfl(up, 63);
-  }
-  return false;
-}
-
 // one token's step and logarithm of decay, and the sum of logarithms over the chunk up to it (a lane per token)
 template <typename T>
 __device__ __forceinline__ void ssd_gates(const ScanArgs& a, int h, int tok0, int nt, float& dt, double& sum) {
@@ -151,7 +124,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   __shared__ float wt[CS_L];
   int s, c;
-  if (!find_chunk(a.qlen, a.S, blockIdx.x, s, c)) return;
+  if (!dllm::find_chunk<CS_L>(a.qlen, a.S, blockIdx.x, s, c)) return;
   const int h = blockIdx.y, v0 = blockIdx.z * CS_VC;
   const int n = a.qlen[s], t0 = c * CS_L, nt = min(CS_L, n - t0), tok0 = a.qstart[s] + t0, p0 = a.ctx[s] - n + t0;
   float* Ks = sm;                    // [L][KS]: keys times their weight
@@ -231,13 +204,10 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
 template <bool SSD, typename V>
 __global__ void __launch_bounds__(256) chunk_carry_kernel(ScanArgs a) {
   constexpr int W = sizeof(V) / 4, AHEAD = 4;
-  const int s = blockIdx.z, h = blockIdx.y, lane = threadIdx.x & 63;
+  const int s = blockIdx.z, h = blockIdx.y;
   const int n = a.qlen[s];
   if (n <= 0) return;
-  int first = 0;      // chunks of the sequences before this one
-  for (int i = lane; i < s; i += 64) first += (max(a.qlen[i], 0) + CS_L - 1) / CS_L;
-#pragma unroll
-  for (int o = 32; o; o >>= 1) first += __shfl_xor(first, o);
+  const int first = dllm::chunks_before<CS_L>(a.qlen, s);
   const int nc = min((n + CS_L - 1) / CS_L, a.nchunks - first);
   const long per = (long)a.d * a.dv, e = ((long)blockIdx.x * 256 + threadIdx.x) * W;
   if (e >= per) return;
@@ -276,7 +246,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   __shared__ float wt[CS_L + 1];       // retention: powers of the decay; ssd: steps
   __shared__ double lg[CS_L];          // ssd: sums of log decays
   int s, c;
-  if (!find_chunk(a.qlen, a.S, blockIdx.x, s, c)) return;
+  if (!dllm::find_chunk<CS_L>(a.qlen, a.S, blockIdx.x, s, c)) return;
   const int h = blockIdx.y, v0 = blockIdx.z * CS_VC;
   const int n = a.qlen[s], t0 = c * CS_L, nt = min(CS_L, n - t0), tok0 = a.qstart[s] + t0, p0 = a.ctx[s] - n + t0;
   float* Ks = sm;                      // [L][KS], then the state [KD][VS] from the start of sm

@@ -1,0 +1,229 @@
+// Chunk-parallel selective scan (Mamba-1) for prompt portions (gfx950, wave64); decode steps and short portions run the
+// token-by-token kernel of seqmix.hip.  Per channel and state
+//
+//     S_t = exp(dt_t A) S_(t-1) + dt_t x_t B_t,   y_t = sum_n S_t C_t + D x_t,   out = y silu(z)
+//
+// With chunks of 32 tokens: scan_sum runs every chunk from a zero state and keeps its end and the sum of its steps
+// (the chunk's decay is exp(A sum dt)); scan_carry walks the chunks, one multiply-add per state; scan_out runs every
+// chunk again from its true start and writes the outputs.  A thread has one channel with all its states in
+// registers: no sums across lanes, B and C rows are broadcast from LDS, and the 64 channels of a wave read and write
+// whole rows.  All of it in f32.
+//
+// What bounds it: the exponentials, one per token, channel and state in either pass (4001 tokens x 2048 channels x 16
+// states: 131M, 14 us of the transcendental unit a pass) and the 20 plain instructions a token and state around them.
+// One sequence of 4096 tokens there: sums 42, carry 21, outputs 48 us; token by token 128 workgroups take 884 us.
+#include "chunks.h"
+#include "common.h"
+
+namespace {
+
+template <typename T> __device__ __forceinline__ float ldf(const T* p);
+template <> __device__ __forceinline__ float ldf<u16>(const u16* p) { return bf2f(*p); }
+template <> __device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
+template <typename T> __device__ __forceinline__ void stf(T* p, float v);
+template <> __device__ __forceinline__ void stf<u16>(u16* p, float v) { *p = f2bf(v); }
+template <> __device__ __forceinline__ void stf<float>(float* p, float v) { *p = v; }
+// exp(dt A): bf16 models on the hardware's exponential, as in the token-by-token kernel, with log2 e in A
+template <typename T> struct Decay;
+template <> struct Decay<u16> {
+  static __device__ __forceinline__ float pre(float a) { return a * 1.44269504088896f; }
+  static __device__ __forceinline__ float f(float x) { return __builtin_amdgcn_exp2f(x); }
+};
+template <> struct Decay<float> {
+  static __device__ __forceinline__ float pre(float a) { return a; }
+  static __device__ __forceinline__ float f(float x) { return expf(x); }
+};
+
+// log(1 + e^x) within a few ulp and a quarter of log1pf(expf(x))'s instructions: max(x, 0) + log1p(u) with u = e^-|x|
+// (the product with log2 e carried in two parts) and log1p(u) = 2 atanh(z), z = u / (2 + u) <= 1 / 3, as its power series
+__device__ __forceinline__ float softplus_f(float x) {
+  const float t = fmaxf(-fabsf(x), -104.f), hi = t * 1.44269504f, lo = fmaf(t, 1.44269504f, -hi) + t * 1.92596299e-8f;
+  float u = __builtin_amdgcn_exp2f(hi);
+  u = fmaf(u * lo, 0.693147181f, u);
+  const float z = u * __builtin_amdgcn_rcpf(2.f + u), w = z * z;
+  float p = fmaf(w, 1.f / 15.f, 1.f / 13.f);
+  p = fmaf(w, p, 1.f / 11.f);
+  p = fmaf(w, p, 1.f / 9.f);
+  p = fmaf(w, p, 1.f / 7.f);
+  p = fmaf(w, p, 1.f / 5.f);
+  p = fmaf(w, p, 1.f / 3.f);
+  p = fmaf(w, p, 1.f);
+  return x == x ? fmaxf(x, 0.f) + 2.f * z * p : x;
+}
+
+// z sigmoid(z); results rounded to bf16 take the hardware's exponential and reciprocal
+template <typename T> __device__ __forceinline__ float silu_t(float z) {
+  if constexpr (sizeof(T) == 2) return z * __builtin_amdgcn_rcpf(1.f + __expf(-z));
+  return z / (1.f + expf(-z));
+}
+
+constexpr int SC_L = 32;      // tokens per chunk
+constexpr int SC_AHEAD = 8;   // tokens whose inputs are in flight
+
+template <typename T> struct MambaArgs {
+  const T *xc, *dt_raw, *dbc, *xz;
+  long ldd, ldz;
+  int dt_rank;
+  const float *dt_bias, *A, *D;
+  float* ssm;
+  T* conv;
+  int Km1;
+  const int *qstart, *qlen, *ctx, *rows;
+  T* out;
+  int S, C, N, nchunks;
+  float *ends, *steps;      // [chunks][N][C], [chunks][C]
+};
+
+// OUT = false: scan_sum, true: scan_out.  NP >= N states in registers (the padded ones stay zero).
+template <typename T, int NP, bool OUT>
+__global__ void __launch_bounds__(256) scan_chunk_kernel(MambaArgs<T> a) {
+  constexpr int W = OUT ? 2 * NP : NP;      // staged numbers per token: B (and C)
+  __shared__ __attribute__((aligned(16))) float bc[SC_L * W];
+  int s, ch;
+  if (!dllm::find_chunk<SC_L>(a.qlen, a.S, blockIdx.y, s, ch)) return;
+  const int n = a.qlen[s], t0 = ch * SC_L, nt = min(SC_L, n - t0), p0 = a.ctx[s] - n;
+  const long tok0 = a.qstart[s] + t0;
+  for (int e = threadIdx.x; e < SC_L * W; e += 256) {
+    const int t = e / W, k = e % W, i = k < NP ? k : k - NP;
+    bc[e] = t < nt && i < a.N ? ldf(a.dbc + (tok0 + t) * a.ldd + a.dt_rank + (k < NP ? 0 : a.N) + i) : 0.f;
+  }
+  __syncthreads();
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= a.C) return;
+  float A[NP], S[NP];
+  float* ends = a.ends + (long)blockIdx.y * a.N * a.C + c;
+  const bool carried = OUT && (ch > 0 || p0 > 0);
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    A[i] = i < a.N ? Decay<T>::pre(a.A[(long)c * a.N + i]) : 0.f;
+    S[i] = carried && i < a.N ? ends[(long)i * a.C] : 0.f;
+  }
+  const float dtb = a.dt_bias[c], skip = OUT ? a.D[c] : 0.f;
+  float sum = 0.f;
+  auto group = [&](int u0, int m) {      // tokens u0 .. u0 + m - 1 of the chunk; m is SC_AHEAD but for the last group
+    float raw[SC_AHEAD], x[SC_AHEAD], z[SC_AHEAD];
+#pragma unroll
+    for (int j = 0; j < SC_AHEAD; ++j) {
+      const long tok = tok0 + u0 + min(j, m - 1);
+      raw[j] = ldf(a.dt_raw + tok * a.C + c);
+      x[j] = ldf(a.xc + tok * a.C + c);
+      z[j] = OUT ? ldf(a.xz + tok * a.ldz + a.C + c) : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < SC_AHEAD; ++j) {
+      if (j >= m) break;
+      const float dt = softplus_f(raw[j] + dtb), dx = dt * x[j];
+      const float4* b4 = reinterpret_cast<const float4*>(bc + (u0 + j) * W);
+      float y = 0.f;
+#pragma unroll
+      for (int i = 0; i < NP; i += 4) {
+        const float4 b = b4[i / 4];
+        const float bv[4] = {b.x, b.y, b.z, b.w};
+        const float4 cc = OUT ? b4[(NP + i) / 4] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float cv[4] = {cc.x, cc.y, cc.z, cc.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          S[i + k] = Decay<T>::f(dt * A[i + k]) * S[i + k] + dx * bv[k];
+          if (OUT) y += S[i + k] * cv[k];
+        }
+      }
+      if (OUT) stf(a.out + (tok0 + u0 + j) * a.C + c, (y + skip * x[j]) * silu_t<T>(z[j]));
+      else sum += dt;
+    }
+  };
+  int u0 = 0;
+  for (; u0 + SC_AHEAD <= nt; u0 += SC_AHEAD) group(u0, SC_AHEAD);
+  if (u0 < nt) group(u0, nt - u0);
+  if constexpr (!OUT) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      if (i < a.N) ends[(long)i * a.C] = S[i];
+    a.steps[(long)blockIdx.y * a.C + c] = sum;
+  } else if (t0 + nt == n && a.Km1 > 0) {
+    // the last K-1 inputs of the sequence: new tokens where there are enough, else the slot's older ones
+    T* cs = a.conv + (long)a.rows[s] * a.Km1 * a.C + c;
+    const long q0 = a.qstart[s];
+    float u[8];
+    for (int k = 0; k < a.Km1; ++k) {
+      const int i = n - a.Km1 + k;
+      u[k] = i >= 0 ? ldf(a.xz + (q0 + i) * a.ldz + c) : (p0 > 0 ? ldf(cs + (long)(a.Km1 + i) * a.C) : 0.f);
+    }
+    for (int k = 0; k < a.Km1; ++k) stf(cs + (long)k * a.C, u[k]);
+  }
+}
+
+// chunk ends -> the state before every chunk, in place, and the state behind the last one into the slot
+template <typename T> __global__ void __launch_bounds__(256) scan_carry_kernel(MambaArgs<T> a) {
+  constexpr int AHEAD = 8;
+  const int s = blockIdx.z, i = blockIdx.y;
+  const int n = a.qlen[s];
+  if (n <= 0) return;
+  const int first = dllm::chunks_before<SC_L>(a.qlen, s);
+  const int nc = min((n + SC_L - 1) / SC_L, a.nchunks - first);
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= a.C) return;
+  float* st = a.ssm + ((long)a.rows[s] * a.C + c) * a.N + i;
+  float* u = a.ends + ((long)first * a.N + i) * a.C + c;
+  const float* d = a.steps + (long)first * a.C + c;
+  const float A = a.A[(long)c * a.N + i];
+  float S = a.ctx[s] - n > 0 ? *st : 0.f;
+  for (int c0 = 0; c0 < nc; c0 += AHEAD) {
+    float x[AHEAD], g[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const long k = min(c0 + j, nc - 1);
+      x[j] = u[k * a.N * a.C];
+      g[j] = d[k * a.C];
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      if (c0 + j >= nc) break;
+      u[(long)(c0 + j) * a.N * a.C] = S;
+      S = expf(A * g[j]) * S + x[j];
+    }
+  }
+  *st = S;
+}
+
+template <typename T, int NP> void launch(const MambaArgs<T>& a, hipStream_t st) {
+  const dim3 g((a.C + 255) / 256, a.nchunks), b(256);
+  hipLaunchKernelGGL((scan_chunk_kernel<T, NP, false>), g, b, 0, st, a);
+  hipLaunchKernelGGL(scan_carry_kernel<T>, dim3((a.C + 255) / 256, a.N, a.S), b, 0, st, a);
+  hipLaunchKernelGGL((scan_chunk_kernel<T, NP, true>), g, b, 0, st, a);
+}
+
+template <typename T>
+int run(const void* xc, const void* dt_raw, const float* dt_bias, const float* A, const void* dbc, long ldd, int dt_rank,
+        const float* D, const void* xz, long ldz, float* ssm, void* conv, int Km1, const int* qstart, const int* qlen,
+        const int* ctx, const int* rows, void* out, int S, long tokens, int C, int N, float* scratch, hipStream_t st) {
+  MambaArgs<T> a{(const T*)xc, (const T*)dt_raw, (const T*)dbc, (const T*)xz, ldd, ldz, dt_rank, dt_bias, A, D, ssm, (T*)conv,
+                 Km1, qstart, qlen, ctx, rows, (T*)out, S, C, N, (int)(tokens / SC_L) + S, scratch, nullptr};
+  a.steps = scratch + (long)a.nchunks * N * C;
+  if (a.nchunks > 65535) return -3;
+  if (N <= 8) launch<T, 8>(a, st);
+  else if (N <= 16) launch<T, 16>(a, st);
+  else launch<T, 32>(a, st);
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+// f32 entries of scratch for a step of T tokens and S sequences; 0: not taken (more states than a thread keeps, or more
+// chunks than a grid's second dimension)
+extern "C" long dllm_scan_chunks_scratch(long T, int S, int C, int N) {
+  const long nc = T / SC_L + S;
+  return N < 1 || N > 32 || nc > 65535 ? 0 : nc * C * (N + 1L);
+}
+
+// the arguments of dllm_selective_scan, and the scratch
+extern "C" int dllm_scan_chunks(const void* xc, const void* dt_raw, int f32, const float* dt_bias, const float* A, const void* dbc,
+                                long ldd, int dt_rank, const float* D, const void* xz, long ldz, float* ssm, void* conv, int Km1,
+                                const int* qstart, const int* qlen, const int* ctx, const int* rows, void* out, int S, long T,
+                                int C, int N, float* scratch, hipStream_t st) {
+  if (S <= 0 || T <= 0) return 0;
+  if (N < 1 || N > 32 || Km1 < 0 || Km1 > 8) return -1;
+  return f32 ? run<float>(xc, dt_raw, dt_bias, A, dbc, ldd, dt_rank, D, xz, ldz, ssm, conv, Km1, qstart, qlen, ctx, rows, out, S, T,
+                          C, N, scratch, st)
+             : run<u16>(xc, dt_raw, dt_bias, A, dbc, ldd, dt_rank, D, xz, ldz, ssm, conv, Km1, qstart, qlen, ctx, rows, out, S, T,
+                        C, N, scratch, st);
+}

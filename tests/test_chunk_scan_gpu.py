@@ -110,3 +110,39 @@ def test_ssd(dt, case, H, dv, N, G):
         close(s32, s64, 4e-6)
         outs.append(float((got.double() - o.reshape(T, -1)).norm() / o.norm()))
     assert outs[0] < 2 * outs[1] + 1e-7      # as exact as the token-by-token form
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", EDGES + [([31, 32, 33, 2], [1, 0, 32, 0])])
+@pytest.mark.parametrize("C,N,R,K", [(256, 16, 8, 4), (70, 5, 3, 2), (300, 32, 0, 1), (8, 17, 4, 4), (264, 33, 2, 3)])
+def test_selective_scan(dt, case, C, N, R, K):
+    """Chunks of 32 tokens, 8 inputs in flight, 256 channels a workgroup, 8 / 16 / 32 states a thread (33: token by token)."""
+    torch.manual_seed(34)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    S = len(qlens)
+    xc, dtr = torch.randn(T, C, device=DEV).to(dt), torch.randn(T, C, device=DEV).to(dt)
+    dbc, xz = torch.randn(T, R + 2 * N + 1, device=DEV).to(dt), torch.randn(T, 2 * C + 3, device=DEV).to(dt)
+    dtb, A, D = torch.randn(C, device=DEV) - 2, -torch.rand(C, N, device=DEV) * 8, torch.randn(C, device=DEV)
+    st, cv = torch.randn(S, C, N, device=DEV), torch.randn(S, K - 1, C, device=DEV).to(dt)
+    step = F.softplus(dtr.double() + dtb.double(), threshold=40)
+    want, s64, t0 = torch.zeros(T, C, dtype=torch.float64, device=DEV), st.double(), 0
+    B, Cm = dbc[:, R:R + N].double(), dbc[:, R + N:R + 2 * N].double()
+    for s, (n, a) in enumerate(zip(qlens, starts)):
+        h = s64[rows[s]].clone() if a else torch.zeros(C, N, dtype=torch.float64, device=DEV)
+        for t in range(t0, t0 + n):
+            h = torch.exp(step[t, :, None] * A.double()) * h + (step[t] * xc[t].double())[:, None] * B[t]
+            want[t] = (h * Cm[t]).sum(1) + D.double() * xc[t].double()
+        if n:
+            s64[rows[s]] = h
+        t0 += n
+    want = want * F.silu(xz[:, C:2 * C].double())
+    errs, convs = [], []
+    for chunked in (True, False):
+        s32, c32 = st.clone(), cv.clone()
+        got = seqmix.selective_scan(xc, dtr, dtb, A, dbc, R, D, xz, s32, c32, qstart, qlen, ctx, rows, chunked=chunked)
+        close(got, want, 4e-6 if dt == torch.float32 else 4e-3)
+        close(s32, s64, 4e-6)
+        errs.append(float((s32.double() - s64).norm() / s64.norm()))
+        convs.append(c32)
+    assert torch.equal(*convs) and errs[0] < 2 * errs[1] + 1e-7      # as exact as the token-by-token form
