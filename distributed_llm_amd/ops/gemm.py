@@ -186,11 +186,27 @@ def _need_tg(M: int, N: int, K: int, bm: int, bn: int, splits: int, ks: int = 1)
 # ----------------------------------------------------------------------------- plans
 
 def _heuristic(M: int, N: int, K: int) -> Tuple:
+    """Plan of a shape nothing timed.  A weight of a few MB is bounded by what one workgroup takes in and by the
+    launch (more waves a workgroup do not help), so: as many workgroups as the columns give, 16 each (32 past
+    4096 columns, or for more rows on a very long K), and K split over workgroups only where one would stream more
+    than 64 KB (32 KB past 16 rows, whose activations it re-reads too) or the rows keep it busy, since slabs
+    and ticket cost 1.3 us at two splits and 2.3 at four.  One or two rows, and four on few columns, take the
+    GEMV (4 columns a workgroup).  us at 1024 columns, this plan against 32
+    columns and up to 16 splits: K 1024: 1 row 2.9 / 6.2, 4 rows 3.9 / 6.3, 16 rows 4.8 / 6.4, 64 rows 7.8 / 9.0;
+    K 4096: 1 row 4.5 / 12.9, 16 rows 8.1 / 13.2, 64 rows 11.5 / 16.9."""
     if M > SKINNY_MAX_M:
         return ("blas",)
-    ntw = 1 if M > 64 else 2
-    tiles = (N + 16 * ntw - 1) // (16 * ntw)
-    splits = max(1, min(16, math.ceil(512 / tiles), K // 256))
+    if M > 64:
+        tiles = (N + 15) // 16
+        return ("skinny", 1, max(1, min(16, math.ceil(512 / tiles), K // 256)))
+    if K % 8 == 0 and (M in (1, 2) or (M == 4 and (N <= 1024 or (N <= 2048 and 2048 <= K <= 4096)))) and M * K * 2 <= 64 * 1024:
+        return ("gemv", 1)
+    ntw = 2 if N > 4096 or (M > 16 and K >= 8192) else 1
+    splits = 1
+    if K > 2048 or (K > 1024 and M > 16) or M > 32:
+        tiles = (N + 16 * ntw - 1) // (16 * ntw)
+        while splits < 4 and tiles * splits * 2 <= 256 and K >= 512 * splits:
+            splits *= 2
     return ("skinny", ntw, splits)
 
 
