@@ -23,11 +23,15 @@
 // accumulator of k . q^T (rows = keys) is, register by register, the A operand of the product with v.  LDS rows are
 // padded by 4 floats: 16-byte reads over 16 rows and 4-byte reads over 4 rows x 16 columns both spread over all banks.
 //
+// Rows go to LDS in two steps, several loads a thread in flight before the first conversion (one at a time the
+// staging took half of either kernel), and SiLU is the hardware's exponential and reciprocal with a compensated argument.
+//
 // What bounds it: 16 heads of 128 x 128 over 6 x 1400 tokens are 12 GFLOP of f32 MFMA a layer (80 us at 157 TFLOP/s) and
 // 0.5 GB of chunk states (100 us at 5.2 TB/s); chunks of 128 would halve the states and need twice the LDS.  Measured
-// there (bf16 rows): sums 154, carry 53, outputs 250 us.  One prompt of 4096 tokens, with its norm and gate: retention
-// with 8 heads of 64 x 128 104 us, with 16 of 128 x 128 230 us, against 1900 and 2910 us for chunks in order
-// (seqmix.hip); Mamba-2 with 32 heads of 128 x 64 178 us against 1390 us token by token (outer_scan.hip).
+// there (bf16 rows): sums 108, carry 53, outputs 158 us (150, 53, 242 with rows staged one load at a time).  One
+// prompt of 4096 tokens, with its norm and gate: retention with 8 heads of 64 x 128 about 80 us against 1900 us
+// for chunks in order (seqmix.hip); Mamba-2 with 32 heads of 128 x 64 about 150 us against 1390 us token by token
+// (outer_scan.hip).
 #include "chunks.h"
 #include "common.h"
 
@@ -56,30 +60,72 @@ struct ScanArgs {
   const int *qstart, *qlen, *ctx, *rows;
   float *state, *chunks, *ends, *out;      // state slots; [chunks][H][d][dv], [chunks][H] A_end (ssd); out [T, H, dv]
   int nchunks;
-  int vec;                    // rows, head offsets and widths allow four elements at a time
+  int vec, rotvec;            // rows, head offsets and widths allow four elements at a time; so do rotation and its table
 };
 
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
+// x sigmoid(x) within a few ulp, without expf's and the division's range handling: the product with log2 e in two
+// parts, the hardware's exponential and reciprocal.  Past the clamp the sigmoid is 1, or below 2^-125 times x.
+__device__ __forceinline__ float silu_f(float x) {
+  const float c = fminf(fmaxf(x, -87.f), 100.f);
+  const float hi = -1.44269504f * c, lo = fmaf(-1.44269504f, c, -hi) - 1.92596299e-8f * c;
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return x * __builtin_amdgcn_rcpf(1.f + fmaf(e * lo, 0.693147181f, e));
+}
 
-// four elements from column i of a row of n (zeros behind it)
-template <typename T> __device__ __forceinline__ float4 ld4(const T* r, int i, int n, int vec) {
-  if (vec) {
-    if (i >= n) return make_float4(0.f, 0.f, 0.f, 0.f);
-    if constexpr (sizeof(T) == 2) {
-      const uint2 u = *reinterpret_cast<const uint2*>(r + i);
-      return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                         __uint_as_float(u.y & 0xffff0000u));
-    } else {
-      return *reinterpret_cast<const float4*>(r + i);
-    }
+// four elements of a row as they lie in memory
+template <typename T> struct Quad;
+template <> struct Quad<u16> {
+  uint2 u;
+  __device__ __forceinline__ void ld(const u16* p) { u = *reinterpret_cast<const uint2*>(p); }
+  __device__ __forceinline__ float4 f() const {
+    return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                       __uint_as_float(u.y & 0xffff0000u));
   }
+};
+template <> struct Quad<float> {
+  float4 u;
+  __device__ __forceinline__ void ld(const float* p) { u = *reinterpret_cast<const float4*>(p); }
+  __device__ __forceinline__ float4 f() const { return u; }
+};
+__device__ __forceinline__ float4 scale4(float4 x, float w) { return make_float4(x.x * w, x.y * w, x.z * w, x.w * w); }
+__device__ __forceinline__ float4 zero4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
+__device__ __forceinline__ float4 silu4(float4 x) { return make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w)); }
+
+// four elements from column i of a row of n, any alignment (zeros behind the row)
+template <typename T> __device__ __forceinline__ float4 ld4(const T* r, int i, int n) {
   return make_float4(i < n ? ldf(r + i) : 0.f, i + 1 < n ? ldf(r + i + 1) : 0.f, i + 2 < n ? ldf(r + i + 2) : 0.f,
                      i + 3 < n ? ldf(r + i + 3) : 0.f);
 }
 
-// four elements of a q / k row: rotated (pairs (i, i + rot / 2)) or SiLU'd
+// four elements of a q / k row, rotated (pairs (i, i + rot / 2)) or SiLU'd: in two steps, so that a thread has the loads
+// of several in flight, or at once for any alignment.  Columns from d on are zeros.
+template <typename T> struct QK {
+  Quad<T> x, p;
+  float4 c, s;
+  __device__ __forceinline__ void ld(const ScanArgs& a, const T* r, int i, int pos) {
+    const int ic = min(i, a.d - 4);
+    x.ld(r + ic);
+    if (a.rot) {
+      const int half = a.rot >> 1, f = ic < a.rot ? (ic < half ? ic : ic - half) : 0;
+      p.ld(r + (ic < a.rot ? (ic < half ? ic + half : ic - half) : ic));
+      const float* cs = a.cos_sin + (long)pos * a.tab_w + f;
+      c = *reinterpret_cast<const float4*>(cs);
+      s = *reinterpret_cast<const float4*>(cs + half);
+    }
+  }
+  __device__ __forceinline__ float4 get(const ScanArgs& a, int i) const {
+    float4 v = x.f();
+    if (a.rot && i < a.rot) {
+      const float4 q = p.f();
+      const float g = i < (a.rot >> 1) ? -1.f : 1.f;
+      v = make_float4(v.x * c.x + g * q.x * s.x, v.y * c.y + g * q.y * s.y, v.z * c.z + g * q.z * s.z, v.w * c.w + g * q.w * s.w);
+    }
+    if (a.act) v = silu4(v);
+    return i < a.d ? v : zero4();
+  }
+};
 template <typename T> __device__ __forceinline__ float4 ld_qk(const ScanArgs& a, const T* r, int i, int pos) {
-  float4 x = ld4(r, i, a.d, a.vec);
+  float4 x = ld4(r, i, a.d);
   if (i < a.rot) {
     float v[4] = {x.x, x.y, x.z, x.w};
     const int half = a.rot >> 1;
@@ -94,8 +140,64 @@ template <typename T> __device__ __forceinline__ float4 ld_qk(const ScanArgs& a,
     }
     x = make_float4(v[0], v[1], v[2], v[3]);
   }
-  if (a.act) x = make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w));
-  return x;
+  return a.act ? silu4(x) : x;
+}
+
+// the chunk's keys [L][KD + 4], times kscale and, with wt, a weight per token; rows past nt are zeros
+template <typename T, int KD>
+__device__ __forceinline__ void stage_keys(const ScanArgs& a, float* Ks, const T* kp, int nt, int p0, const float* wt) {
+  constexpr int IT = CS_L * KD / 1024, U = IT < 4 ? IT : 4;
+  if (a.vec && (!a.rot || a.rotvec)) {
+#pragma unroll
+    for (int it = 0; it < IT; it += U) {
+      QK<T> x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = threadIdx.x + 256 * (it + u), t = min(e / (KD / 4), nt - 1);
+        x[u].ld(a, kp + t * a.ld, (e % (KD / 4)) * 4, p0 + t);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int e = threadIdx.x + 256 * (it + u), t = e / (KD / 4), i = (e % (KD / 4)) * 4;
+        const float w = t < nt ? (wt ? wt[t] : 1.f) * a.kscale : 0.f;
+        *reinterpret_cast<float4*>(Ks + t * (KD + 4) + i) = t < nt ? scale4(x[u].get(a, i), w) : zero4();
+      }
+    }
+  } else {
+    for (int e = threadIdx.x; e < CS_L * KD / 4; e += 256) {
+      const int t = e / (KD / 4), i = (e % (KD / 4)) * 4;
+      *reinterpret_cast<float4*>(Ks + t * (KD + 4) + i) =
+          t < nt ? scale4(ld_qk(a, kp + t * a.ld, i, p0 + t), (wt ? wt[t] : 1.f) * a.kscale) : zero4();
+    }
+  }
+}
+
+// the chunk's values [L][16 NV + 4] from column 0 of vp, n of them in a row; rows past nt are zeros
+template <typename T, int NV>
+__device__ __forceinline__ void stage_values(const ScanArgs& a, float* Vs, const T* vp, int nt, int n) {
+  constexpr int IT = CS_L * NV / 64, VS = 16 * NV + 4;
+  if (a.vec) {
+    Quad<T> x[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int e = threadIdx.x + 256 * it;
+      x[it].ld(vp + min(e / (4 * NV), nt - 1) * a.ldv + min((e % (4 * NV)) * 4, n - 4));
+    }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int e = threadIdx.x + 256 * it, t = e / (4 * NV), i = (e % (4 * NV)) * 4;
+      float4 v = x[it].f();
+      if (a.act) v = silu4(v);
+      *reinterpret_cast<float4*>(Vs + t * VS + i) = t < nt && i < n ? v : zero4();
+    }
+  } else {
+    for (int e = threadIdx.x; e < CS_L * NV * 4; e += 256) {
+      const int t = e / (4 * NV), i = (e % (4 * NV)) * 4;
+      float4 v = zero4();
+      if (t < nt) v = ld4(vp + t * a.ldv, i, n);
+      *reinterpret_cast<float4*>(Vs + t * VS + i) = a.act ? silu4(v) : v;
+    }
+  }
 }
 
 // one token's step and logarithm of decay, and the sum of logarithms over the chunk up to it (a lane per token)
@@ -140,32 +242,12 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
       wt[lane] = dt * expf((float)(end - sum));
       if (lane == 0 && v0 == 0) a.ends[(long)blockIdx.x * a.H + h] = expf((float)end);
     } else {
-      wt[lane] = lane < nt ? a.kscale * powf(a.decay[h], (float)(nt - 1 - lane)) : 0.f;
+      wt[lane] = lane < nt ? powf(a.decay[h], (float)(nt - 1 - lane)) : 0.f;
     }
   }
+  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC));
   __syncthreads();
-  const T* kp = (const T*)a.k + (long)(h / a.kdiv) * a.d;
-  for (int e = tid; e < CS_L * KD / 4; e += 256) {
-    const int t = e / (KD / 4), i = (e % (KD / 4)) * 4;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < nt) {
-      const T* r = kp + (long)(tok0 + t) * a.ld;
-      x = SSD ? ld4(r, i, a.d, a.vec) : ld_qk(a, r, i, p0 + t);
-      const float w = wt[t];
-      x = make_float4(x.x * w, x.y * w, x.z * w, x.w * w);
-    }
-    *reinterpret_cast<float4*>(Ks + t * KS + i) = x;
-  }
-  const T* vp = (const T*)a.v + (long)h * a.dv + v0;
-  for (int e = tid; e < CS_L * NV * 4; e += 256) {
-    const int t = e / (NV * 4), i = (e % (NV * 4)) * 4;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < nt) {
-      x = ld4(vp + (long)(tok0 + t) * a.ldv, i, a.dv - v0, a.vec);
-      if (!SSD && a.act) x = make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w));
-    }
-    *reinterpret_cast<float4*>(Vs + t * VS + i) = x;
-  }
+  stage_keys<T, KD>(a, Ks, (const T*)a.k + (long)tok0 * a.ld + (long)(h / a.kdiv) * a.d, nt, p0, wt);
   __syncthreads();
   const int wr = wave % WR, wc = wave / WR;
   f32x4 acc[NR][NC];
@@ -265,36 +347,28 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
       if (lane == 0) wt[CS_L] = powf(a.decay[h], (float)CS_L);
     }
   }
-  const long kh = (long)(h / a.kdiv) * a.d;
-  const T* kp = (const T*)a.k + kh;
-  for (int e = tid; e < CS_L * KD / 4; e += 256) {
-    const int t = e / (KD / 4), i = (e % (KD / 4)) * 4;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < nt) {
-      const T* r = kp + (long)(tok0 + t) * a.ld;
-      x = SSD ? ld4(r, i, a.d, a.vec) : ld_qk(a, r, i, p0 + t);
-      x = make_float4(x.x * a.kscale, x.y * a.kscale, x.z * a.kscale, x.w * a.kscale);
-    }
-    *reinterpret_cast<float4*>(Ks + t * KS + i) = x;
-  }
-  const T* vp = (const T*)a.v + (long)h * a.dv + v0;
-  for (int e = tid; e < CS_L * NV * 4; e += 256) {
-    const int t = e / (NV * 4), i = (e % (NV * 4)) * 4;
-    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (t < nt) {
-      x = ld4(vp + (long)(tok0 + t) * a.ldv, i, a.dv - v0, a.vec);
-      if (!SSD && a.act) x = make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w));
-    }
-    *reinterpret_cast<float4*>(Vs + t * VS + i) = x;
-  }
+  const long kh = (long)tok0 * a.ld + (long)(h / a.kdiv) * a.d;
+  stage_keys<T, KD>(a, Ks, (const T*)a.k + kh, nt, p0, nullptr);
+  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC));
   // the wave's queries: row lr, dims 16 b + 4 g4 ..
-  const int tq = 16 * wave + lr;
+  const int tq = 16 * wave + lr, tl = min(tq, nt - 1);
   float4 q[NB];
   {
-    const T* r = (const T*)a.q + kh + (long)(tok0 + min(tq, nt - 1)) * a.ld;
+    const T* r = (const T*)a.q + kh + tl * a.ld;
+    if (a.vec && (!a.rot || a.rotvec)) {
+      constexpr int U = NB < 4 ? NB : 4;
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      q[b] = SSD ? ld4(r, 16 * b + 4 * g4, a.d, a.vec) : ld_qk(a, r, 16 * b + 4 * g4, p0 + min(tq, nt - 1));
+      for (int b = 0; b < NB; b += U) {
+        QK<T> x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u].ld(a, r, 16 * (b + u) + 4 * g4, p0 + tl);
+#pragma unroll
+        for (int u = 0; u < U; ++u) q[b + u] = x[u].get(a, 16 * (b + u) + 4 * g4);
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) q[b] = ld_qk(a, r, 16 * b + 4 * g4, p0 + tl);
+    }
   }
   __syncthreads();
   f32x4 acc[NV];
@@ -333,15 +407,32 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   if (c > 0 || p0 > 0) {      // (the same for the whole workgroup) a sequence starts from a zero state
     __syncthreads();
     const float* st = a.chunks + ((long)blockIdx.x * a.H + h) * a.d * a.dv + v0;
-    const int vec = a.dv % 4 == 0;
-    for (int e = tid; e < KD * NV * 4; e += 256) {
-      const int r = e / (NV * 4), i = (e % (NV * 4)) * 4;
-      *reinterpret_cast<float4*>(sm + r * VS + i) =
-          r < a.d ? ld4(st + (long)r * a.dv, i, a.dv - v0, vec) : make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr int IT = KD * NV / 64, U = IT < 8 ? IT : 8;
+    if (a.dv % 4 == 0) {
+      const int n = min(a.dv - v0, CS_VC);
+#pragma unroll
+      for (int it = 0; it < IT; it += U) {
+        float4 x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int e = tid + 256 * (it + u);
+          x[u] = *reinterpret_cast<const float4*>(st + (long)min(e / (4 * NV), a.d - 1) * a.dv + min((e % (4 * NV)) * 4, n - 4));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int e = tid + 256 * (it + u), r = e / (4 * NV), i = (e % (4 * NV)) * 4;
+          *reinterpret_cast<float4*>(sm + r * VS + i) = r < a.d && i < n ? x[u] : zero4();
+        }
+      }
+    } else {
+      for (int e = tid; e < KD * NV * 4; e += 256) {
+        const int r = e / (4 * NV), i = (e % (4 * NV)) * 4;
+        *reinterpret_cast<float4*>(sm + r * VS + i) = r < a.d ? ld4(st + (long)r * a.dv, i, a.dv - v0) : zero4();
+      }
     }
     const float w = SSD ? expf((float)lq) : wt[tq + 1];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) q[b] = make_float4(q[b].x * w, q[b].y * w, q[b].z * w, q[b].w * w);
+    for (int b = 0; b < NB; ++b) q[b] = scale4(q[b], w);
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -406,6 +497,7 @@ template <bool SSD> int run_chunks(ScanArgs& a, int f32, long T, float* scratch,
   a.nchunks = (int)(T / CS_L) + a.S;
   a.chunks = scratch;
   a.ends = scratch + (long)a.nchunks * a.H * a.d * a.dv;
+  a.rotvec = a.rot % 8 == 0 && a.tab_w % 4 == 0 && (uintptr_t)a.cos_sin % 16 == 0;
   if (f32) {
     a.vec = vec_ok<float>(a);
     return launch_chunks<float, SSD>(a, st);
