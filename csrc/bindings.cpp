@@ -98,7 +98,8 @@ int dllm_gelu_erf(const void*, void*, int, long, hipStream_t);
 int dllm_conv_refill(const void*, long, int, void*, int, int, const int*, const int*, const int*, const int*, int,
                      hipStream_t);
 int dllm_delta_rule(const void*, long, const void*, long, int, int, int, int, int, const float*, const float*, const float*,
-                    float, float*, const int*, const int*, const int*, const int*, float*, void*, int, long, hipStream_t);
+                    float, float*, const int*, const int*, const int*, const int*, float*, void*, int, long, float*, hipStream_t);
+int dllm_delta_pre(int);
 int dllm_attn_prep(const void*, long, int, int, int, int, int, const float*, int, int, float, const float*, const int*,
                    const int*, void*, void*, void*, long, int, hipStream_t);
 int dllm_gqa_tile_tokens(int, int, int);
@@ -1667,7 +1668,7 @@ void conv_state_refill(torch::Tensor x, torch::Tensor state, torch::Tensor qstar
 
 void delta_rule(torch::Tensor qkv, torch::Tensor gba, int64_t H, int64_t G, int64_t d, int64_t dv, torch::Tensor neg_a,
                 torch::Tensor dt_bias, torch::Tensor norm_w, double eps, torch::Tensor state, torch::Tensor qstart,
-                torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out) {
+                torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out, bool tiled) {
   const bool f = act_f32(qkv, "qkv");
   check_rows2d(qkv, "qkv");
   check_rows2d(gba, "gba");
@@ -1689,10 +1690,13 @@ void delta_rule(torch::Tensor qkv, torch::Tensor gba, int64_t H, int64_t G, int6
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
   // f32 outputs before the per-head norm: written and read for tokens of live sequences only
   auto raw = torch::empty({T, H, dv}, torch::TensorOptions().dtype(torch::kFloat32).device(qkv.device()));
+  const int64_t pw = tiled ? dllm_delta_pre((int)d) : 0;
+  torch::Tensor pre;
+  if (pw) pre = torch::empty({T * H * pw}, raw.options());
   ok(dllm_delta_rule(qkv.data_ptr(), qkv.stride(0), gba.data_ptr(), gba.stride(0), f, (int)H, (int)G, (int)d, (int)dv,
                      neg_a.data_ptr<float>(), dt_bias.data_ptr<float>(), norm_w.data_ptr<float>(), (float)eps,
                      state.data_ptr<float>(), m.qstart, m.qlen, m.ctx, m.rows, raw.data_ptr<float>(), out.data_ptr(), m.S,
-                     (long)T, stream()),
+                     (long)T, pw ? pre.data_ptr<float>() : nullptr, stream()),
      "delta_rule");
 }
 

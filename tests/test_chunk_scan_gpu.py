@@ -146,3 +146,47 @@ def test_selective_scan(dt, case, C, N, R, K):
         errs.append(float((s32.double() - s64).norm() / s64.norm()))
         convs.append(c32)
     assert torch.equal(*convs) and errs[0] < 2 * errs[1] + 1e-7      # as exact as the token-by-token form
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", EDGES + [([128, 15, 17], [64, 1, 0])])
+@pytest.mark.parametrize("H,G,d,dv", [(4, 2, 128, 128), (3, 3, 64, 40), (2, 1, 36, 20), (2, 2, 33, 17), (1, 1, 4, 4), (2, 1, 104, 130)])
+@pytest.mark.parametrize("steep", [0.0, 4.0])
+def test_delta_rule(dt, case, H, G, d, dv, steep):
+    """Tiles of 16 tokens, padded key widths 64 / 128, 16 value columns, rows that are no whole vectors; decays near 1 and
+    steep, and keys that repeat, for which the triangular system is furthest from the identity."""
+    torch.manual_seed(35)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    S = len(qlens)
+    qkv = torch.randn(T, 2 * G * d + H * dv, device=DEV)
+    qkv[::3, G * d:2 * G * d] = qkv[:1, G * d:2 * G * d]
+    qkv, gba = qkv.to(dt), torch.randn(T, H * dv + 2 * H + 3, device=DEV).to(dt)
+    na, dtb, nw = -torch.rand(H, device=DEV) * (0.05 + steep), torch.randn(H, device=DEV), torch.randn(dv, device=DEV)
+    st = torch.randn(S, H, dv, d, device=DEV) * 0.5
+    q, k, v = qkv.double().split([G * d, G * d, H * dv], 1)
+    q, k = (z.view(T, G, d) * torch.rsqrt((z.view(T, G, d) ** 2).sum(-1, keepdim=True) + 1e-6) for z in (q, k))
+    q, k = (q * d ** -0.5).repeat_interleave(H // G, 1), k.repeat_interleave(H // G, 1)
+    v, gate, beta, al = v.view(T, H, dv), *(gba[:, a:b].double() for a, b in ((0, H * dv), (H * dv, H * dv + H), (H * dv + H, H * dv + 2 * H)))
+    beta, g = torch.sigmoid(beta), torch.exp(na.double() * F.softplus(al + dtb.double(), threshold=40))
+    want, s64, t0 = torch.zeros(T, H, dv, dtype=torch.float64, device=DEV), st.double(), 0
+    for s, (n, a) in enumerate(zip(qlens, starts)):
+        M = s64[rows[s]].clone() if a else torch.zeros(H, dv, d, dtype=torch.float64, device=DEV)
+        for t in range(t0, t0 + n):
+            M = g[t, :, None, None] * M
+            u = beta[t, :, None] * (v[t] - (M * k[t, :, None]).sum(-1))
+            M = M + u[:, :, None] * k[t, :, None]
+            want[t] = (M * q[t, :, None]).sum(-1)
+        if n:
+            s64[rows[s]] = M
+        t0 += n
+    want = (want * torch.rsqrt((want * want).mean(-1, keepdim=True) + 1e-6) * nw.double()).reshape(T, -1) * F.silu(gate)
+    errs = []
+    for tiled in (True, False):
+        s32 = st.clone()
+        got = seqmix.delta_rule(qkv, gba, H, G, d, dv, na, dtb, nw, 1e-6, s32, qstart, qlen, ctx, rows, tiled=tiled)
+        close(got, want, 8e-6 if dt == torch.float32 else 4e-3)
+        close(s32, s64, 8e-6)
+        errs.append((float((s32.double() - s64).norm() / s64.norm()), float((got.double() - want).norm() / want.norm())))
+    # as exact as token by token, but for the inverse's own roundings: two of 2^-24 more
+    assert errs[0][0] < 1.5 * errs[1][0] + 2.0 ** -23 and errs[0][1] < 1.5 * errs[1][1] + 2.0 ** -23
