@@ -16,6 +16,9 @@
 //               four rows), f32 online softmax per row, then a lane owns value dims for the weighted
 //               sum (one V read feeds four rows).  The output is multiplied by sigmoid(gate).
 //
+//   gqa_f32     the f32 form on the f32 matrix cores: a wave per 16-key page, no LDS until the waves of a
+//               workgroup meet (whole pages of 16 keys, widths up to 128; paged_gqa takes the rest).
+//
 //   paged_gqa_mfma  the bf16 form on the matrix cores: 64 rows per workgroup, 16 per wave, so a row's
 //               softmax never leaves its wave.  Q stays in registers as MFMA operands; a 64-key tile is
 //               staged once for the four waves (K row-major, V already transposed in its page);
@@ -346,7 +349,10 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(const float* __restri
   for (int i = lane; i < dv; i += 64) stf(out + u * dv + i, (a1[i] - lam * a2[i]) * sc);
 }
 
-constexpr int GA_ROWS = 16;   // rows per workgroup: 4 per wave
+constexpr int GA_ROWS = 16;   // rows per workgroup
+// up to a workgroup per CU, 8 waves share a workgroup's keys, past that 4 (16 heads of 64, us with 8 / 4: 128 workgroups of 400
+// keys 15.1 / 17.6, 8 of 2000 39.7 / 53.3, 480 of 60 12.9 / 8.8, 2016 of up to 250 65.5 / 48.9)
+constexpr int GQF_WIDE = 256;
 
 // KT keys per tile (64, or 32 when the tile would not fit the LDS), NJ = ceil(dv / 64)
 template <typename T, int NJ>
@@ -484,6 +490,161 @@ __global__ void __launch_bounds__(256) paged_gqa_kernel(const T* __restrict__ q,
       else stf(out + tok * ldo + (long)h * dv + jx, o);
     }
   }
+}
+
+// ---------------------------------------------------------------- f32 on the matrix cores
+// A wave takes a 16-key page at a time, alone: S^T = K Q^T (keys 4 g4 + i of a lane against row lr), so that a row's softmax
+// is four registers and two lane exchanges, and its weights are at once the right operand of O^T = V^T P^T.  Every operand
+// comes from where it lies, 16 bytes a lane (contraction step x of lane group g4 stands for dim 16 b + 4 g4 + x, or key
+// 4 g4 + x): no LDS and no barrier until the NW waves of a workgroup, which take every NW-th page, meet at the end.  The next
+// page's keys and values travel while one is computed.  Bounded by one page's load and 32 small products at decode, by the
+// f32 matrix rate (139 TF/s) over prompts.  16 query heads of 64 on 4 key heads: two sequences
+// of 400 keys 14 us a step against 104 of the general kernel above, a prompt of 2000 tokens 165 against 1087; errors against 64
+// bits 2e-7 either way.
+template <int KB, int VB, int NW>
+__global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc,
+                                                          const float* __restrict__ vc, const int* __restrict__ bt, int bt_ld,
+                                                          int BSZ, const int* __restrict__ qstart, const int* __restrict__ qlen,
+                                                          const int* __restrict__ ctx, const int* __restrict__ tile_seq,
+                                                          const int* __restrict__ tile_tok0, const float* __restrict__ gate,
+                                                          long ldg, float* __restrict__ out, int H, int G, int d, int dv, int TQ,
+                                                          int win, int GV, int keep, float sink, int chunk, float cap,
+                                                          const float* __restrict__ sinks, long ldo,
+                                                          const float* __restrict__ slopes, int ghead) {
+  __shared__ __attribute__((aligned(16))) f32x4 Om[NW / 2][VB * 64];
+  __shared__ float ml[NW][2][16];
+  const int tile = gridDim.x - 1 - blockIdx.x;   // later tokens see more keys: start with the long rows
+  const int s = tile_seq[tile];
+  const int n = qlen[s], tok0 = tile_tok0[tile];
+  if (n <= 0 || tok0 >= n) return;               // the whole workgroup (padding tiles)
+  const int g = blockIdx.y, R = H / G;
+  const int r0 = blockIdx.z * GA_ROWS, Rh = min(GA_ROWS, R - r0);
+  const int nq = min(TQ, n - tok0), nrows = nq * Rh;
+  const int q0 = qstart[s], p0 = ctx[s] - n;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g4 = lane >> 4;
+  const bool row = lr < nrows;                   // rows past nrows are idle: they see no key and are not written
+  const long tok = q0 + tok0 + (row ? lr / Rh : 0);
+  const int h = g * R + r0 + (row ? lr % Rh : 0);
+  const int rpos = row ? p0 + tok0 + lr / Rh : -1, rlo = row ? oldest_key(rpos, win, chunk) : 0;
+  const float slp = slopes ? slopes[h] : 0.f;
+  f32x4 qf[KB];
+  const float* qp = q + (tok * H + h) * d;
+#pragma unroll
+  for (int b = 0; b < KB; ++b) {
+    const int i = 16 * b + 4 * g4;
+    qf[b] = i < d ? *reinterpret_cast<const f32x4*>(qp + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const int last = p0 + tok0 + nq - 1, first = oldest_key(p0 + tok0, win, chunk);   // the newest and oldest key any row sees
+  const int* btr = bt + (long)s * bt_ld;
+  const int gv = g / (G / GV);
+  f32x4 kf[KB], vf[VB], kn[KB], vn[VB];
+  auto fetch = [&](int k0, f32x4 (&k)[KB], f32x4 (&v)[VB]) {   // places past the widths are read at 0: q is 0 there, O is dropped
+    const long blk = btr[k0 / BSZ];
+    const int off = k0 % BSZ;
+    const float* kp = kc + ((blk * G + g) * BSZ + off + lr) * d;
+    const float* vp = vc + (blk * GV + gv) * dv * BSZ + off + 4 * g4;
+#pragma unroll
+    for (int b = 0; b < KB; ++b) k[b] = *reinterpret_cast<const f32x4*>(kp + (16 * b + 4 * g4 < d ? 16 * b + 4 * g4 : 0));
+#pragma unroll
+    for (int b = 0; b < VB; ++b) v[b] = *reinterpret_cast<const f32x4*>(vp + (long)(16 * b + lr < dv ? 16 * b + lr : 0) * BSZ);
+  };
+  // the wave's next page from k0 on (uniform in the wave): pages between the kept keys and the window are passed over
+  auto next = [&](int k0) {
+    while (k0 <= last && k0 >= keep && k0 + 16 <= first) k0 += 16 * NW;
+    return k0;
+  };
+  float m = -INFINITY, l = 0.f;
+  f32x4 O[VB];
+#pragma unroll
+  for (int b = 0; b < VB; ++b) O[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int k0 = next((keep > 0 ? 0 : first / 16 * 16) + 16 * w);
+  if (k0 <= last) fetch(k0, kn, vn);
+  while (k0 <= last) {
+    const int k1 = next(k0 + 16 * NW);
+#pragma unroll
+    for (int b = 0; b < KB; ++b) kf[b] = kn[b];
+#pragma unroll
+    for (int b = 0; b < VB; ++b) vf[b] = vn[b];
+    if (k1 <= last) fetch(k1, kn, vn);
+    f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KB; ++b)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) sc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][x], qf[b][x], sc, 0, 0, 0);
+    bool vis[4];
+    float mn = m;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int pk = k0 + 4 * g4 + x;
+      vis[x] = pk <= rpos && (pk >= rlo || pk < keep);
+      if (cap > 0.f) sc[x] = cap * tanhf(sc[x] / cap);
+      else if (slopes) sc[x] -= slp * (float)(rpos - pk);
+      if (vis[x]) mn = fmaxf(mn, sc[x]);
+    }
+    mn = fmaxf(mn, __shfl_xor(mn, 16));
+    mn = fmaxf(mn, __shfl_xor(mn, 32));
+    const float f = mn > -INFINITY ? expf(m - mn) : 1.f;   // before the first visible key: O and l are 0
+    f32x4 p;
+    l *= f;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      p[x] = vis[x] ? expf(sc[x] - mn) : 0.f;
+      l += p[x];
+    }
+    m = mn;
+    if (k0 + 15 > last) {   // values past the newest key are not of this sequence: whatever they hold, they count as 0
+#pragma unroll
+      for (int b = 0; b < VB; ++b)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) vf[b][x] = k0 + 4 * g4 + x <= last ? vf[b][x] : 0.f;
+    }
+#pragma unroll
+    for (int b = 0; b < VB; ++b) {
+      O[b] *= f;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) O[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][x], p[x], O[b], 0, 0, 0);
+    }
+    k0 = k1;
+  }
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (g4 == 0) {
+    ml[w][0][lr] = m;
+    ml[w][1][lr] = l;
+  }
+  __syncthreads();
+  float M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int x = 0; x < NW; ++x) M = fmaxf(M, ml[x][0][lr]);
+#pragma unroll
+  for (int x = 0; x < NW; ++x) L += ml[x][0][lr] > -INFINITY ? ml[x][1][lr] * expf(ml[x][0][lr] - M) : 0.f;
+  const float f = m > -INFINITY ? expf(m - M) : 0.f;
+#pragma unroll
+  for (int b = 0; b < VB; ++b) O[b] *= f;
+#pragma unroll
+  for (int half = NW / 2; half; half >>= 1) {
+    if (w >= half && w < 2 * half)
+#pragma unroll
+      for (int b = 0; b < VB; ++b) Om[w - half][b * 64 + lane] = O[b];
+    __syncthreads();
+    if (w < half)
+#pragma unroll
+      for (int b = 0; b < VB; ++b) O[b] += Om[w][b * 64 + lane];
+    __syncthreads();
+  }
+  if (w || !row) return;
+  const float inv = 1.f / (L + (sinks ? expf(sinks[h] - M) : sink > 0.f ? sink * expf(-M) : 0.f));
+  const float gh = gate && ghead ? 1.f / (1.f + expf(-gate[tok * ldg + h])) : 1.f;
+#pragma unroll
+  for (int b = 0; b < VB; ++b)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int j = 16 * b + 4 * g4 + x;
+      if (j >= dv) continue;
+      float o = O[b][x] * inv * gh;
+      if (gate && !ghead) o *= 1.f / (1.f + expf(-gate[tok * ldg + (long)h * dv + j]));
+      out[tok * ldo + (long)h * dv + j] = o;
+    }
 }
 
 // ---------------------------------------------------------------- bf16 on the matrix cores
@@ -954,6 +1115,28 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
       hipLaunchKernelGGL(gqa_combine_kernel, dim3(n_tiles, G, (rows + 3) / 4), dim3(256), 0, st, pp, splits, qstart, qlen,
                          tile_seq, tile_tok0, (const u16*)gate, ldg, (u16*)out, H, G, dv, TQ, out32, sink, sinks, ldo, ghead);
     }
+    return (int)hipGetLastError();
+  }
+  // f32, whole pages of 16 keys, key and query rows of whole 16-byte vectors: the matrix cores
+  if (f32 && BSZ % 16 == 0 && d % 4 == 0 && d <= 128 && dv <= 128 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0) {
+    const dim3 g3(n_tiles, G, (H / G + GA_ROWS - 1) / GA_ROWS);
+    const int tq = dllm_gqa_tile_tokens(H, G, 0);
+    const bool wide = (long)g3.x * g3.y * g3.z <= GQF_WIDE;
+#define GQF2(KB, VB, NW)                                                                                                     \
+  hipLaunchKernelGGL((gqa_f32_kernel<KB, VB, NW>), g3, dim3(64 * NW), 0, st, (const float*)q, (const float*)kc, (const float*)vc, bt, \
+                     bt_ld, BSZ, qstart, qlen, ctx, tile_seq, tile_tok0, (const float*)gate, ldg, (float*)out, H, G, d, dv, tq, win,  \
+                     GV, keep, sink, chunk, cap, sinks, ldo, slopes, ghead)
+#define GQF(KB, VB)                        \
+  do {                                     \
+    if (wide) GQF2(KB, VB, 8);             \
+    else GQF2(KB, VB, 4);                  \
+  } while (0)
+    if (d <= 64 && dv <= 64) GQF(4, 4);
+    else if (d <= 64 && dv <= 128) GQF(4, 8);
+    else if (d <= 128 && dv <= 64) GQF(8, 4);
+    else GQF(8, 8);
+#undef GQF
+#undef GQF2
     return (int)hipGetLastError();
   }
   int KT = 64;
