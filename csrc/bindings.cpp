@@ -74,6 +74,7 @@ int dllm_diff_combine(const float*, void*, int, long, int, int, int, float, floa
 int dllm_conv_silu(const void*, long, int, const float*, const float*, void*, const int*, const int*, const int*,
                    const int*, void*, int, int, int, int, int, int, hipStream_t);
 long dllm_scan_chunks_scratch(long, int, int, int);
+int dllm_scan_step_ok(long, int, int, const void*, const void*);
 int dllm_scan_chunks(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*, const void*, long,
                      float*, void*, int, const int*, const int*, const int*, const int*, void*, int, long, int, int, float*, hipStream_t);
 int dllm_selective_scan(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*,
@@ -1459,13 +1460,15 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
               "conv_state [slots, K - 1, C]");
   auto m = seq_meta(qstart, qlen, ctx, rows, ssm.size(0));
   const long ns = chunked ? dllm_scan_chunks_scratch(T, m.S, C, N) : 0;
-  if (ns > 0 && ns <= (1L << 30)) {      // chunk-parallel form (prompt portions)
-    auto sc = torch::empty({ns}, xc.options().dtype(torch::kFloat32));
+  const bool step = !chunked && dllm_scan_step_ok(T, m.S, N, ssm.data_ptr(), A.data_ptr());
+  if (step || (ns > 0 && ns <= (1L << 30))) {      // decode steps, or the chunk-parallel form (prompt portions)
+    torch::Tensor sc;
+    if (!step) sc = torch::empty({ns}, xc.options().dtype(torch::kFloat32));
     ok(dllm_scan_chunks(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(), dbc.data_ptr(),
                         dbc.stride(0), (int)dt_rank, D.data_ptr<float>(), xz.data_ptr(), xz.stride(0), ssm.data_ptr<float>(),
                         conv.data_ptr(), (int)conv.size(1), m.qstart, m.qlen, m.ctx, m.rows, out.data_ptr(), m.S, (long)T, C, N,
-                        sc.data_ptr<float>(), stream()),
-       "selective_scan (chunked)");
+                        step ? nullptr : sc.data_ptr<float>(), stream()),
+       step ? "selective_scan (step)" : "selective_scan (chunked)");
     return;
   }
   ok(dllm_selective_scan(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(),

@@ -114,10 +114,10 @@ def retention_step_lds(dim: int, vdim: int) -> int:
     return 4 * (dim * vdim + 8 * (2 * dim + 2 * vdim) + 2 * (256 // lj) * vdim)
 
 
-# average new tokens per sequence from which the chunk-parallel kernels run: about 25 us of launches against the serial
-# tokens of one workgroup per head (24 sequences of 8 tokens: 41 against 35 us for 8 heads of 64 x 128, 73 against 109
-# for 16 of 128 x 128; of 16 tokens: 44 against 62 and 80 against 204; 48 of 4: 57 against 23 and 117 against 95)
-RETENTION_CHUNK_MIN = 8
+# average new tokens per sequence from which the chunk-parallel kernels run (us token by token / in chunks for 8 heads of 64 x 128;
+# 16 of 128 x 128): one sequence of 8 tokens 26 / 27; 34 / 35, of 16 tokens 47 / 27; 62 / 36; 24 sequences of 8 tokens
+# 27 / 42; 43 / 79, of 16 tokens 48 / 43; 75 / 81
+RETENTION_CHUNK_MIN = 9
 
 
 def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen, ctx,

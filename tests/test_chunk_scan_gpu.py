@@ -190,3 +190,76 @@ def test_delta_rule(dt, case, H, G, d, dv, steep):
         errs.append((float((s32.double() - s64).norm() / s64.norm()), float((got.double() - want).norm() / want.norm())))
     # as exact as token by token, but for the inverse's own roundings: two of 2^-24 more
     assert errs[0][0] < 1.5 * errs[1][0] + 2.0 ** -23 and errs[0][1] < 1.5 * errs[1][1] + 2.0 ** -23
+
+
+STEPS = [([1] * 5, [3, 0, 64, 1, 7]), ([1, 0, 3, 2], [0, 5, 9, 0]), ([1], [400])]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", STEPS)
+@pytest.mark.parametrize("H,d,dv,rot", [(2, 64, 128, 64), (16, 128, 128, 0), (3, 20, 36, 10), (1, 256, 64, 32), (2, 5, 4, 0), (2, 64, 256, 6), (2, 33, 7, 32)])
+def test_retention_steps(dt, case, H, d, dv, rot):
+    """Few new tokens: 4 / 8 / 16 key rows a thread, columns that leave threads idle, widths that are no vectors (the LDS form)."""
+    torch.manual_seed(36)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, pos = batch(qlens, starts)
+    x = torch.randn(T, 2 * H * d + 2 * H * dv + 3, device=DEV)
+    # keys lean on their queries: a first token's output is (q . k) v to unit RMS, whose error is that of q . k over its size, without bound
+    # where the two are at right angles
+    x[:, H * d:2 * H * d] += x[:, :H * d]
+    x = x.to(dt)
+    table = ops.rope_cos_sin(512, max(rot, 2), 10000.0, DEV)
+    dec = torch.tensor([1.0 - 2.0 ** (-2 - 3 * (h % 4)) for h in range(H)], device=DEV)
+    st = torch.randn(len(qlens) + 1, H, d, dv, device=DEV)
+    q, k, v, g = x.double()[:, :2 * H * (d + dv)].split([H * d, H * d, H * dv, H * dv], 1)
+    q, k, h2 = q.view(T, H, d).clone(), k.view(T, H, d).clone(), rot // 2
+    c, s = (table[pos.long()].double()[:, None, i * h2:(i + 1) * h2] for i in range(2))
+    for z in (q, k):
+        a, b = z[..., :h2].clone(), z[..., h2:rot].clone()
+        z[..., :h2], z[..., h2:rot] = a * c - b * s, b * c + a * s
+    for form in ("retention", "lightning"):
+        s64, s32 = st.double(), st.clone()
+        if form == "retention":
+            got = seqmix.retention(x, H, d, dv, table, rot, dec, s32, 1e-6, pos, qstart, qlen, ctx, rows, chunked=False)
+            o = recur(q, k * d ** -0.5, v.reshape(T, H, dv), dec.double().expand(T, H), s64, qlens, starts, rows.tolist())
+            want = (o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-6)).reshape(T, -1) * F.silu(g)
+        else:
+            nw = torch.randn(H * dv, device=DEV)
+            got = seqmix.lightning_attention(x, H, d, dv, dec, s32, 1e-6, nw, qstart, qlen, ctx, rows, chunked=False)
+            y = F.silu(x.double()[:, :H * (2 * d + dv)])
+            o = recur(*(y[:, i * H * d:i * H * d + H * e].reshape(T, H, e) for i, e in ((0, d), (1, d), (2, dv))), dec.double().expand(T, H), s64,
+                      qlens, starts, rows.tolist()).reshape(T, -1)
+            want = o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-6) * nw.double() * torch.sigmoid(g)
+        close(got, want, 4e-6 if dt == torch.float32 else 4e-3)
+        close(s32, s64, 2e-6)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", STEPS)
+@pytest.mark.parametrize("C,N,R,K", [(2048, 16, 64, 4), (70, 4, 3, 2), (300, 32, 0, 1), (8, 20, 4, 9), (65, 8, 1, 3), (64, 6, 2, 4)])
+def test_scan_steps(dt, case, C, N, R, K):
+    """Few new tokens: a thread per channel, 8 / 16 / 32 states in registers, channels that fill no wave, 0 to 8 kept inputs (6 states: the
+    form of 16 lanes a channel)."""
+    torch.manual_seed(37)
+    qlens, starts = case
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    S = len(qlens)
+    xc, dtr = torch.randn(T, C, device=DEV).to(dt), torch.randn(T, C, device=DEV).to(dt)
+    dbc, xz = torch.randn(T, R + 2 * N + 1, device=DEV).to(dt), torch.randn(T, 2 * C + 3, device=DEV).to(dt)
+    dtb, A, D = torch.randn(C, device=DEV) - 2, -torch.rand(C, N, device=DEV) * 8, torch.randn(C, device=DEV)
+    st, cv = torch.randn(S + 1, C, N, device=DEV), torch.randn(S + 1, K - 1, C, device=DEV).to(dt)
+    step, want, s64, c2, t0 = F.softplus(dtr.double() + dtb.double(), threshold=40), torch.zeros(T, C, dtype=torch.float64, device=DEV), st.double(), cv.clone(), 0
+    for s, (n, a) in enumerate(zip(qlens, starts)):
+        h = s64[rows[s]].clone() if a else torch.zeros(C, N, dtype=torch.float64, device=DEV)
+        for t in range(t0, t0 + n):
+            h = torch.exp(step[t, :, None] * A.double()) * h + (step[t] * xc[t].double())[:, None] * dbc[t, R:R + N].double()
+            want[t] = (h * dbc[t, R + N:R + 2 * N].double()).sum(1) + D.double() * xc[t].double()
+        if n:
+            s64[rows[s]] = h
+            old = cv[rows[s]] if a else torch.zeros_like(cv[0])
+            c2[rows[s]] = torch.cat([old, xz[t0:t0 + n, :C]])[n:]
+        t0 += n
+    got = seqmix.selective_scan(xc, dtr, dtb, A, dbc, R, D, xz, st, cv, qstart, qlen, ctx, rows, chunked=False)
+    close(got, want * F.silu(xz[:, C:2 * C].double()), 4e-6 if dt == torch.float32 else 4e-3)
+    close(st, s64, 4e-6)
+    assert torch.equal(cv, c2)
