@@ -141,7 +141,8 @@ int dllm_car_vote(int, int*, void*, int*, hipStream_t);
 int dllm_tgemm(const void*, int, int, int, int, int, int, int, hipStream_t, int);
 int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
-                    int*, int*, int*, void*, void*, void*, int, const int*, hipStream_t);
+                    int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, hipStream_t);
+int dllm_moe_tail_ok(int, int);
 int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
                   float, hipStream_t);
@@ -921,21 +922,35 @@ void gemv_swiglu(torch::Tensor x, torch::Tensor w, torch::Tensor ssq, int64_t ss
 // grouped-tgemm MoE (csrc/kernels/moe.hip dllm_moe_ffn_tg): act_mode 0: w13 [E, 2I, H] interleaved per 16-row
 // group; 1: squared-ReLU experts, w13 [E, I, H]
 void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Tensor w13, torch::Tensor w2,
-                torch::Tensor out, std::vector<int64_t> plan, int64_t act_mode) {
+                c10::optional<torch::Tensor> out, std::vector<int64_t> plan, int64_t act_mode, c10::optional<torch::Tensor> norm_w,
+                double eps, c10::optional<torch::Tensor> xs, c10::optional<torch::Tensor> xl, int64_t groups) {
   check_bf16(x, "x");
   check_i32(ids, "ids");
   check_f32(wts, "wts");
   check_bf16(w13, "w13");
   check_bf16(w2, "w2");
-  check_bf16(out, "out");
-  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && out.is_contiguous(), "x rows 16-B aligned");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0, "x rows 16-B aligned");
   TORCH_CHECK(w13.dim() == 3 && w2.dim() == 3 && w13.is_contiguous() && w2.is_contiguous(), "w13/w2 [E, N, K]");
   const int64_t T = x.size(0), H = x.size(1), E = w13.size(0), I = w13.size(1) / (act_mode ? 1 : 2);
   TORCH_CHECK(w13.size(2) == H && w2.size(0) == E && w2.size(1) == H && w2.size(2) == I, "expert weight shapes");
   TORCH_CHECK(H % 64 == 0 && I % 64 == 0 && E <= 64, "H, I multiples of 64; E <= 64");
   TORCH_CHECK(ids.dim() == 2 && ids.size(0) == T && wts.sizes() == ids.sizes() && ids.is_contiguous() &&
                   wts.is_contiguous(), "ids/wts [T, k]");
-  TORCH_CHECK(out.size(0) == T && out.size(1) == H, "out shape");
+  if (xs) {   // the layer ends in the stream: xs += rmsnorm(sum) * norm_w, rounded copy in xl
+    check_f32(*xs, "xs");
+    TORCH_CHECK(norm_w.has_value() && xs->dim() == 2 && xs->is_contiguous() && xs->size(0) == T && xs->size(1) == H, "xs [T, H]");
+    check_f32(*norm_w, "norm weight");
+    TORCH_CHECK(norm_w->numel() == H && groups >= 1 && dllm_moe_tail_ok((int)H, (int)groups), "norm weight [H], parts of whole 256s");
+    TORCH_CHECK(((uintptr_t)xs->data_ptr() | (uintptr_t)norm_w->data_ptr()) % 16 == 0, "xs / norm weight 16-B aligned");
+    if (xl) {
+      check_bf16(*xl, "xl");
+      TORCH_CHECK(xl->is_contiguous() && xl->sizes() == xs->sizes() && (uintptr_t)xl->data_ptr() % 8 == 0, "xl [T, H]");
+    }
+  } else {
+    TORCH_CHECK(out.has_value(), "out");
+    check_bf16(*out, "out");
+    TORCH_CHECK(out->is_contiguous() && out->size(0) == T && out->size(1) == H, "out shape");
+  }
   TORCH_CHECK(act_mode == 0 || act_mode == 1, "act_mode 0 or 1");
   TORCH_CHECK(plan.size() == 9, "plan: bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2");
   const int bm = (int)plan[0];
@@ -960,7 +975,9 @@ void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Te
   for (int i = 0; i < 9; ++i) pl[i] = (int)plan[i];
   ok(dllm_moe_ffn_tg(x.data_ptr(), x.stride(0), T, (int)H, ids.data_ptr<int>(), wts.data_ptr<float>(), k, (int)E,
                      w13.data_ptr(), w2.data_ptr(), (int)I, perm.data_ptr<int>(), inv.data_ptr<int>(),
-                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), out.data_ptr(), (int)act_mode, pl, stream()),
+                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), xs ? nullptr : out->data_ptr(), (int)act_mode, pl,
+                     xs ? norm_w->data_ptr<float>() : nullptr, xs ? xs->data_ptr<float>() : nullptr,
+                     xs && xl ? xl->data_ptr() : nullptr, (float)eps, (int)groups, stream()),
      "moe_ffn_tg");
 }
 
@@ -2524,8 +2541,10 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("embed_ln", &embed_ln);
   m.def("moe_ffn", &moe_ffn, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
         py::arg("act_mode") = 0);
+  m.def("moe_tail_ok", [](int64_t H, int64_t groups) { return dllm_moe_tail_ok((int)H, (int)groups) != 0; });
   m.def("moe_ffn_tg", &moe_ffn_tg, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
-        py::arg("plan"), py::arg("act_mode") = 0);
+        py::arg("plan"), py::arg("act_mode") = 0, py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("xs") = py::none(),
+        py::arg("xl") = py::none(), py::arg("groups") = 1);
   m.def("tgemm", &tgemm);
   m.def("res_add_ssq", &res_add_ssq);
   m.def("qkv_post", &qkv_post, py::arg("y"), py::arg("ssq"), py::arg("ssq_n"), py::arg("scale"), py::arg("eps"),

@@ -29,6 +29,8 @@
 #include "common.h"
 #include "tgemm_args.h"
 
+extern "C" int dllm_moe_norm_resadd(const void* y, int f32, const int* inv, const float* wts, int k, const float* w, float* x, void* xl,
+                                    long T, int H, float eps, int groups, hipStream_t st);
 extern "C" int dllm_tgemm(const void* args, int bm, int bn, int stages, int ks, int nw, int wk, int epi,
                           hipStream_t stream, int nl);
 
@@ -43,26 +45,35 @@ __global__ void __launch_bounds__(1024) moe_route_kernel(const int* __restrict__
   // Pairs are placed in a stable order (pair index ascending within each expert): per chunk of
   // blockDim pairs, a pair's slot = expert base + pairs of its expert in earlier chunks + in earlier
   // waves of this chunk + lower lanes of its wave (ballot ranks), so the layout never depends on
-  // atomic arrival order.
-  __shared__ int cnt[64], off[65], cur[64], wcnt[16][64];
+  // atomic arrival order.  Few pairs take a block of few waves (24 tokens of 3: 5.0 us, with one thread laying out the tiles and
+  // 16 waves at every barrier 6.0).
+  __shared__ int cnt[64], off[64], toff[64], cur[64], wcnt[16][64], ntl;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwv = blockDim.x >> 6;
   if (tid < 64) { cnt[tid] = 0; cur[tid] = 0; }
   __syncthreads();
   for (int p = tid; p < P; p += blockDim.x) atomicAdd(&cnt[min(max(ids[p], 0), E - 1)], 1);  // order-free sum
   __syncthreads();
-  if (tid == 0) {
-    off[0] = 0;
-    for (int e = 0; e < E; ++e) off[e + 1] = off[e] + cnt[e];
-    int nt = 0;
-    for (int e = 0; e < E; ++e)
-      for (int r = 0; r < cnt[e] && nt < max_tiles; r += mt, ++nt) {
-        tile_e[nt] = e;
-        tile_r0[nt] = off[e] + r;
-        tile_n[nt] = min(mt, cnt[e] - r);
-      }
-    *n_tiles = nt;
+  if (tid < 64) {   // first pair and first tile of every expert: lane e of one wave
+    const int c = tid < E ? cnt[tid] : 0, nt = (c + mt - 1) / mt;
+    int po = c, to = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int a = __shfl_up(po, o), b = __shfl_up(to, o);
+      if (lane >= o) { po += a; to += b; }
+    }
+    off[tid] = po - c;
+    toff[tid] = to - nt;
+    if (tid == 63) *n_tiles = ntl = min(to, max_tiles);
   }
   __syncthreads();
+  for (int i = tid; i < ntl; i += blockDim.x) {
+    int e = 0;
+    for (int x = 1; x < E; ++x) e += toff[x] <= i;      // experts without tiles share the next one's start: the last of them owns it
+    const int r = (i - toff[e]) * mt;
+    tile_e[i] = e;
+    tile_r0[i] = off[e] + r;
+    tile_n[i] = min(mt, cnt[e] - r);
+  }
   for (int base = 0; base < P; base += blockDim.x) {  // uniform trip count: every wave ballots
     const int p = base + tid;
     const int e = p < P ? min(max(ids[p], 0), E - 1) : -1;
@@ -287,6 +298,7 @@ __global__ void moe_combine_kernel(const float* __restrict__ y, int k, int H, lo
     for (int j = 0; j < 4; ++j) o[j] = f2bf(s[j]);
   }
 }
+int route_threads(int P) { return P >= 1024 ? 1024 : (P + 63) / 64 * 64; }
 }  // namespace
 
 extern "C" int dllm_moe_max_tiles(int P, int E) { return (P + MT - 1) / MT + E; }
@@ -299,7 +311,7 @@ extern "C" int dllm_moe_ffn(const void* x, long x_stride, long T, int H, const i
   const int P = (int)(T * k);
   const int max_tiles = (P + MT - 1) / MT + E;
   int *te = tiles, *tr = tiles + max_tiles, *tn = tiles + 2 * max_tiles, *nt = tiles + 3 * max_tiles;
-  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt);
+  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(route_threads(P)), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt);
   if (act_mode)
     hipLaunchKernelGGL(moe_gemm13_kernel<1>, dim3(max_tiles, (I + 63) / 64), dim3(256), 0, stream, (const u16*)x,
                        x_stride, perm, k, te, tr, tn, nt, (const u16*)w13, (u16*)act, I, H);
@@ -320,17 +332,19 @@ extern "C" int dllm_moe_max_tiles_bm(int P, int E, int bm) { return (P + bm - 1)
 
 // plans: {bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2}; act_mode 0: w13 interleaved [E, 2I, H] (16 gate
 // rows, 16 up rows, ...), y bf16; 1: w13 [E, I, H], squared ReLU, y f32.  w2 [E, H, I]; scratch: perm/inv [P], tiles
-// [4 * max_tiles + 1], act [P, I], y [P, H].
+// [4 * max_tiles + 1], act [P, I], y [P, H].  xs (f32 [T, H]): instead of `out`, xs += rmsnorm(sum) * nw in `groups` parts, and its
+// rounded copy in xl (norm_resadd of seqmix.hip, in the combine's launch).
 extern "C" int dllm_moe_ffn_tg(const void* x, long x_stride, long T, int H, const int* ids, const float* wts, int k,
                                int E, const void* w13, const void* w2, int I, int* perm, int* inv, int* tiles,
-                               void* act, void* y, void* out, int act_mode, const int* plan, hipStream_t stream) {
+                               void* act, void* y, void* out, int act_mode, const int* plan, const float* nw, float* xs, void* xl,
+                               float eps, int groups, hipStream_t stream) {
   if (E < 1 || E > 64 || k < 1 || H % 64 != 0 || I % 64 != 0 || x_stride % 8) return -1;
   if (T == 0) return 0;
   const int bm = plan[0], NI = act_mode ? I : 2 * I;
   const int P = (int)(T * k);
   const int max_tiles = (P + bm - 1) / bm + E;
   int *te = tiles, *tr = tiles + max_tiles, *tn = tiles + 2 * max_tiles, *nt = tiles + 3 * max_tiles;
-  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt, bm,
+  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(route_threads(P)), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt, bm,
                      inv);
   dllm::GemmArgs g{};
   g.A = (const uint16_t*)x; g.lda = x_stride; g.W = (const uint16_t*)w13; g.Y = (uint16_t*)act; g.ldy = I;
@@ -344,6 +358,7 @@ extern "C" int dllm_moe_ffn_tg(const void* x, long x_stride, long T, int H, cons
   d.g_tiles = tiles; d.g_max = max_tiles; d.g_perm = nullptr; d.g_k = 1; d.g_wstride = (long)H * I;
   rc = dllm_tgemm(&d, bm, plan[5], plan[6], plan[7], plan[8], 1, act_mode ? dllm::EPI_F32 : dllm::EPI_PLAIN, stream, 0);
   if (rc) return 2000 + rc;
+  if (xs) return dllm_moe_norm_resadd(y, act_mode, inv, wts, k, nw, xs, xl, T, H, eps, groups, stream);   // the sum goes into the stream
   long n8 = T * (H / 8);
   long gr = (n8 + 255) / 256;
   if (gr > 4096) gr = 4096;

@@ -970,7 +970,7 @@ class HybridModel:
             a = seqmix.polynorm(z, L["act"], self.cfg.rms_eps) if f.act == "polynorm" else seqmix.gelu_erf(z)
         return _mm(a, L["down"])
 
-    def _experts_swiglu(self, L, f: MoESpec, x):
+    def _experts_swiglu(self, L, f: MoESpec, x, tail=None):
         """Sigmoid router in f32 with group-limited top-k, weights = the chosen scores; SwiGLU experts
         on the grouped MFMA kernels, or in the dense form (all experts' columns in two GEMMs, unused
         experts gated to zero) for f32 models and widths the grouped kernels do not take."""
@@ -978,7 +978,7 @@ class HybridModel:
         ids, w = seqmix.group_router(logits, f.top, f.group_count, f.group_keep)
         if f.scale != 1.0:
             w = w * f.scale
-        return self._swiglu_experts(L, f, x, ids, w)
+        return self._swiglu_experts(L, f, x, ids, w, tail)
 
     def _experts_terms(self, L, f: MoESpec, x) -> dict:
         """Softmax router in f32 whose choice (not its weights) sees a learned correction, group-limited
@@ -998,11 +998,11 @@ class HybridModel:
             out.update(y2=_mm(seqmix.glu_act(_mm(x, L["sh_up"])), L["sh_down"]), g2=logits[:, R] if f.shared_gate else None)
         return out
 
-    def _swiglu_experts(self, L, f: MoESpec, x, ids, w):
+    def _swiglu_experts(self, L, f: MoESpec, x, ids, w, tail=None):
         """sum_j w[t, j] expert_(ids[t, j])(x_t); ids beyond the experts (identity experts, whose weight
-        here is 0) add nothing."""
+        here is 0) add nothing.  ``tail`` as in ``_experts``."""
         if L.get("tg"):
-            return ops.moe_ffn_tg(x if x.stride(1) == 1 else x.contiguous(), ids, w, L["w1"], L["w2"])
+            return ops.moe_ffn_tg(x if x.stride(1) == 1 else x.contiguous(), ids, w, L["w1"], L["w2"], tail=tail)
         if "w2" in L and (not x.is_cuda or seqmix.moe_ffn_relu2_ok(x, L["w1"])):
             return ops.moe_ffn(x, ids, w, L["w1"], L["w2"])
         if "w2d" not in L:
@@ -1011,12 +1011,14 @@ class HybridModel:
         a = seqmix.swiglu_scale(_mm(x, L["w1"].view(f.experts * 2 * f.ff, -1)), g, f.ff)
         return _mm(a, L["w2d"])
 
-    def _experts(self, L, f: MoESpec, x):
+    def _experts(self, L, f: MoESpec, x, tail=None):
+        """``tail`` (ops.moe_ffn_tg): where the experts run on the grouped GEMM, their sum ends in the stream and None is
+        returned; elsewhere the caller adds what is returned."""
         if f.act == "swiglu":
-            return self._experts_swiglu(L, f, x)
+            return self._experts_swiglu(L, f, x, tail)
         if "shared_in" in L:
             ids, w = ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
-            return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"])
+            return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], tail)
         if f.experts > 64 or f.top > 8:      # beyond the router kernels' register budget: library top-k
             val, ids = torch.topk(torch.softmax(F.linear(x.float(), L["router"].float()), -1), f.top, -1)
             ids, w = ids.to(torch.int32), val / (val.sum(-1, keepdim=True) + 1e-20) * f.scale
@@ -1135,8 +1137,10 @@ class HybridModel:
                 seqmix.norm_resadd(y, L["norm1"], eps, x, xl, groups=ng, bias=L.get("ob"))
                 if S.mlp is not None:
                     hin = x if xl is None else xl
-                    y = self._dense(L, S.mlp, hin) if isinstance(S.mlp, DenseSpec) else self._experts(L, S.mlp, hin)
-                    seqmix.norm_resadd(y, L["norm2"], eps, x, xl, groups=ng)
+                    y = self._dense(L, S.mlp, hin) if isinstance(S.mlp, DenseSpec) else \
+                        self._experts(L, S.mlp, hin, (L["norm2"], eps, x, xl, ng))
+                    if y is not None:
+                        seqmix.norm_resadd(y, L["norm2"], eps, x, xl, groups=ng)
                 if X is not None:
                     x = seqmix.depth_mix(X, L["dwa"], i + 2)
                     if xl is not None:

@@ -455,21 +455,39 @@ def moe_plan(pairs: int) -> Tuple[int, ...]:
 
 
 def moe_ffn_tg(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torch.Tensor, w2: torch.Tensor,
-               plan: Optional[Tuple[int, ...]] = None) -> torch.Tensor:
+               plan: Optional[Tuple[int, ...]] = None, tail: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """Top-k expert FFN on the grouped LDS-tiled MFMA GEMM (csrc/kernels/moe.hip moe_ffn_tg):
     ``w13i`` [E, 2I, H] with gate/up rows interleaved in 16-row groups (models.llama.gate_up_order),
-    w2 [E, H, I].  Routing, both GEMMs and the weighted combine stay on the device."""
+    w2 [E, H, I].  Routing, both GEMMs and the weighted combine stay on the device.  ``tail`` =
+    (norm weight, eps, stream, rounded stream or None, groups): the sum ends in ``seqmix.norm_resadd``'s update of the
+    stream, in the combine's launch where the width allows; returns None then."""
     ext = _native(x)
     if ext is None:
         from ..models.llama import gate_up_order
         w13 = torch.empty_like(w13i)
         w13[:, gate_up_order(w13i.shape[1] // 2)] = w13i
-        return ref.moe_ffn(x, ids, wts, w13, w2)
-    out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
+        out = ref.moe_ffn(x, ids, wts, w13, w2)
+        return out if tail is None else moe_tail(out, tail)
     if plan is None:
         plan = moe_plan(x.shape[0] * ids.shape[1])
-    ext.moe_ffn_tg(x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, out, list(plan))
-    return out
+    return moe_run_tg(ext, x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, plan, 0, tail)
+
+
+def moe_tail(y: torch.Tensor, tail: tuple) -> None:
+    """``tail`` of ``moe_ffn_tg`` as a launch of its own."""
+    from . import seqmix
+    w, eps, x, xl, groups = tail
+    seqmix.norm_resadd(y, w, eps, x, xl, groups=groups)
+
+
+def moe_run_tg(ext, x, ids, wts, w1, w2, plan, act_mode: int, tail: Optional[tuple]) -> Optional[torch.Tensor]:
+    if tail is not None and ext.moe_tail_ok(x.shape[1], int(tail[4])):
+        w, eps, xs, xl, groups = tail
+        ext.moe_ffn_tg(x, ids, wts, w1, w2, None, list(plan), act_mode, w, float(eps), xs, xl, int(groups))
+        return None
+    out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
+    ext.moe_ffn_tg(x, ids, wts, w1, w2, out, list(plan), act_mode)
+    return out if tail is None else moe_tail(out, tail)
 
 
 # ----------------------------------------------------------------------------- sampling

@@ -46,3 +46,78 @@ def test_router_many_experts():
         val, idx = (x.double() @ wg.double().t()).topk(2, -1)
         assert torch.equal(ids.long(), idx)
         torch.testing.assert_close(w.double(), torch.softmax(val, -1), atol=1e-4, rtol=1e-4)
+
+
+def test_router_choice_of_ties_and_non_finite_logits():
+    """The lower expert first among equals; NaN is never chosen; expert 0 where nothing is left to choose."""
+    x = torch.zeros(4, 64, device=DEV).bfloat16()
+    x[:, 0], x[1, 1], x[2, 1], x[3, 1] = 1, 1, 1, 1
+    wg = torch.zeros(9, 64, device=DEV).bfloat16()
+    wg[:, 0] = torch.tensor([1, 3, 2, 3, 2, 3, 0, 1, 2]).bfloat16().to(DEV)
+    ids, w = ops.moe_router(x[:1], wg, 5)
+    assert ids.tolist() == [[1, 3, 5, 2, 4]]
+    torch.testing.assert_close(w[0].double(), torch.softmax(torch.tensor([3., 3, 3, 2, 2]).double(), 0).to(DEV), atol=1e-6, rtol=1e-6)
+    bad = wg.clone()
+    bad[1, 1], bad[5, 1] = float("nan"), float("-inf")
+    assert ops.moe_router(x[1:2], bad, 3)[0].tolist() == [[3, 2, 4]]
+    bad[:, 1] = float("-inf")
+    assert ops.moe_router(x[2:3], bad, 2)[0].tolist() == [[0, 0]]
+
+
+@pytest.mark.parametrize("E,top,T", [(1, 1, 1), (3, 2, 5), (64, 8, 16), (64, 8, 129), (8, 3, 700), (9, 1, 64), (40, 2, 2100)])
+@pytest.mark.parametrize("pairs", [1, 600, 1 << 20])      # the plans' tiles: 64, 128 and 256 rows
+def test_route_tiles(E, top, T, pairs):
+    """Pairs by expert in the order of their tokens, full and partial tiles; experts without pairs, one wave and many, more pairs than a
+    block: read off through experts that are multiples of the identity."""
+    torch.manual_seed(E)
+    H = 64
+    ids = torch.stack([torch.randperm(E, device=DEV)[:top] for _ in range(T)]).int()
+    ids = torch.where(ids % 5 == 2, ids // 2, ids)                      # some experts get nothing, some pairs repeat
+    wts = torch.rand(T, top, device=DEV)
+    x = torch.rand(T, H, device=DEV).bfloat16()
+    w1 = torch.eye(H, device=DEV).expand(E, H, H).bfloat16().contiguous()
+    w2 = (torch.eye(H, device=DEV)[None] * (1 + torch.arange(E, device=DEV))[:, None, None]).bfloat16()
+    out = torch.empty(T, H, device=DEV).bfloat16()
+    ops._native(x).moe_ffn_tg(x, ids, wts, w1, w2, out, list(ops.moe_plan(pairs)), 1)
+    want = (x.double() ** 2) * ((ids + 1).double() * wts.double()).sum(1, keepdim=True)
+    assert float((out.double() - want).norm() / want.norm()) < 2 ** -8
+
+
+@pytest.mark.parametrize("T,H,groups", [(1, 64, 1), (24, 1024, 4), (5, 1088, 1), (3, 2048, 8), (2, 4096, 16), (2, 8192, 2), (7, 320, 5), (2, 8256, 1)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_tail(T, H, groups, mode):
+    """The weighted sum, its norm and the residual add in one launch, and on widths that take their own launches (parts that are no whole
+    256s, rows past 8192)."""
+    torch.manual_seed(H)
+    E, top, I = 5, 3, 64
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    ids = torch.stack([torch.randperm(E, device=DEV)[:top] for _ in range(T)]).int()
+    wts, w, st = torch.rand(T, top, device=DEV), torch.randn(H, device=DEV), torch.randn(T, H, device=DEV)
+    w1, w2 = (torch.randn(E, a, b, device=DEV).div(b ** 0.5).bfloat16() for a, b in (((2 - mode) * I, H), (H, I)))
+    run = (lambda **kw: ops.moe_ffn_tg(x, ids, wts, w1, w2, **kw)) if mode == 0 else (lambda **kw: seqmix.moe_ffn_relu2(x, ids, wts, w1, w2, **kw))
+    y = run().double()
+    want = st.double() + (y.view(T, groups, -1) * torch.rsqrt(y.view(T, groups, -1).pow(2).mean(-1, keepdim=True) + 1e-6)).view(T, H) * w.double()
+    s2, xl = st.clone(), torch.empty_like(x)
+    assert run(tail=(w, 1e-6, s2, xl, groups)) is None
+    # y above was rounded to bf16 (2^-9 an element); the stream is f32
+    assert float((s2.double() - want).norm() / want.norm()) < 2 ** -8
+    assert torch.equal(xl, s2.bfloat16())
+    s3 = st.clone()
+    assert run(tail=(w, 1e-6, s3, None, groups)) is None
+    assert torch.equal(s2, s3)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,H,groups,pad", [(3, 1024, 4, 0), (2, 1020, 1, 4), (5, 64, 1, 0), (2, 2304, 9, 8), (1, 8192, 1, 0), (2, 6144, 3, 0), (2, 768, 6, 0), (3, 70, 1, 1)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_norm_resadd_widths(dt, T, H, groups, pad, bias):
+    """Rows in registers: 1 to 8 vectors a thread, rows that fill no workgroup, parts of whole 256s; other widths take the general form."""
+    torch.manual_seed(H)
+    y = torch.randn(T, H + pad, device=DEV).to(dt)[:, :H]
+    w, x, b = torch.randn(H, device=DEV), torch.randn(T, H, device=DEV), torch.randn(H, device=DEV) if bias else None
+    z = y.double() + (b.double() if bias else 0)
+    want = x.double() + (z.view(T, groups, -1) * torch.rsqrt(z.view(T, groups, -1).pow(2).mean(-1, keepdim=True) + 1e-5)).view(T, H) * w.double()
+    xl = torch.empty(T, H, device=DEV, dtype=dt)
+    seqmix.norm_resadd(y, w, 1e-5, x, xl, groups, b)
+    assert float((x.double() - want).norm() / want.norm()) < 1e-6
+    assert torch.equal(xl, x.to(dt))
