@@ -22,7 +22,7 @@ int dllm_embed(const int*, const void*, void*, long, int, long, long, float*, in
 int dllm_gemv(const void*, long, const void*, void*, long, int, int, int, int, int, const void*, void*, const void*,
               float, hipStream_t);
 int dllm_gelu(const void*, void*, long, hipStream_t);
-int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, hipStream_t);
+int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, const int*, int, hipStream_t);
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
 int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, hipStream_t);
 int dllm_scatter_pairs(int*, const int*, int, hipStream_t);
@@ -143,9 +143,9 @@ int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
                     int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, hipStream_t);
 int dllm_moe_tail_ok(int, int);
-int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, hipStream_t);
+int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, const int*, int, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
-                  float, hipStream_t);
+                  float, const int*, hipStream_t);
 int dllm_res_add_ssq(const void*, long, void*, long, float*, long, int, int, int, hipStream_t);
 int dllm_gemv_slots(int, int, int);
 void dllm_gemv_set_grid(int, int, int);
@@ -412,14 +412,22 @@ void gelu(torch::Tensor x, torch::Tensor y) {
   ok(dllm_gelu(x.data_ptr(), y.data_ptr(), x.numel(), stream()), "gelu");
 }
 
-void mean_pool_l2(torch::Tensor x, torch::Tensor lens, torch::Tensor out) {
+// x [B, S, H]; or, with starts (int32 [>= B], first row of each text), packed rows [T, H]
+void mean_pool_l2(torch::Tensor x, torch::Tensor lens, torch::Tensor out, c10::optional<torch::Tensor> starts) {
   check_bf16(x, "x");
   check_i32(lens, "lens");
   check_f32(out, "out");
-  TORCH_CHECK(x.dim() == 3 && x.is_contiguous(), "x [B, S, H]");
-  const int B = x.size(0), S = x.size(1), H = x.size(2);
-  TORCH_CHECK(lens.numel() == B && out.size(0) == B && out.size(1) == H, "shapes");
-  ok(dllm_mean_pool_l2(x.data_ptr(), lens.data_ptr<int>(), out.data_ptr<float>(), B, S, H, stream()), "mean_pool_l2");
+  TORCH_CHECK(x.dim() == (starts ? 2 : 3) && x.is_contiguous(), "x [B, S, H], packed [T, H]");
+  const int B = lens.numel(), S = starts ? 0 : x.size(1), H = x.size(x.dim() - 1), T = starts ? x.size(0) : 0;
+  if (starts) {
+    check_i32(*starts, "starts");
+    TORCH_CHECK(starts->is_contiguous() && starts->numel() >= B && lens.is_contiguous(), "starts [B]");
+  }
+  TORCH_CHECK((starts || x.size(0) == B) && out.size(0) == B && out.size(1) == H, "shapes");
+  if (B == 0) return;
+  ok(dllm_mean_pool_l2(x.data_ptr(), lens.data_ptr<int>(), out.data_ptr<float>(), B, S, H,
+                       starts ? starts->data_ptr<int>() : nullptr, T, stream()),
+     "mean_pool_l2");
 }
 
 void moe_gate(torch::Tensor logits, int64_t k, torch::Tensor ids, torch::Tensor w) {
@@ -1336,33 +1344,43 @@ int64_t res_add_ssq(c10::optional<torch::Tensor> h, torch::Tensor r, torch::Tens
 
 // router encoder (csrc/kernels/encoder.hip): bidirectional attention over a padded batch
 void encoder_attention(torch::Tensor qkv, torch::Tensor lens, torch::Tensor out, int64_t B, int64_t S, int64_t nh,
-                       int64_t d, double scale) {
+                       int64_t d, double scale, c10::optional<torch::Tensor> starts) {
   check_bf16(qkv, "qkv");
   check_bf16(out, "out");
   check_i32(lens, "lens");
   TORCH_CHECK(d == 32 || d == 64, "encoder attention: head_dim 32 or 64");
   TORCH_CHECK(S >= 1 && S <= 512, "encoder attention: 1 <= S <= 512");
-  TORCH_CHECK(qkv.is_contiguous() && qkv.dim() == 2 && qkv.size(0) == B * S && qkv.size(1) == 3 * nh * d,
+  const int64_t T = starts ? qkv.size(0) : B * S;      // packed: starts[b] is text b's first row, S the longest
+  TORCH_CHECK(qkv.is_contiguous() && qkv.dim() == 2 && qkv.size(0) == T && qkv.size(1) == 3 * nh * d,
               "qkv [B*S, 3 nh d]");
-  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == B * S && out.size(1) == nh * d, "out [B*S, nh d]");
+  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == T && out.size(1) == nh * d, "out [B*S, nh d]");
   TORCH_CHECK(lens.numel() >= B, "lens [B]");
-  ok(dllm_encoder_attention(qkv.data_ptr(), lens.data_ptr<int>(), out.data_ptr(), B, S, nh, d, (float)scale, stream()),
+  if (starts) {
+    check_i32(*starts, "starts");
+    TORCH_CHECK(starts->is_contiguous() && starts->numel() >= B && lens.is_contiguous(), "starts [B]");
+  }
+  ok(dllm_encoder_attention(qkv.data_ptr(), lens.data_ptr<int>(), out.data_ptr(), B, S, nh, d, (float)scale,
+                            starts ? starts->data_ptr<int>() : nullptr, (int)T, stream()),
      "encoder_attention");
 }
 
 void embed_ln(torch::Tensor ids, torch::Tensor word, torch::Tensor pos, torch::Tensor type0, torch::Tensor w,
-              torch::Tensor b, torch::Tensor out, int64_t S, double eps) {
+              torch::Tensor b, torch::Tensor out, int64_t S, double eps, c10::optional<torch::Tensor> at) {
   check_i32(ids, "ids");
+  if (at) {
+    check_i32(*at, "positions");
+    TORCH_CHECK(at->is_contiguous() && at->numel() == ids.numel(), "a position per id");
+  }
   for (auto* t : {&word, &pos, &type0, &w, &b, &out}) check_bf16(*t, "embed_ln operand");
   const int64_t T = ids.numel(), H = word.size(1);
   TORCH_CHECK(ids.is_contiguous() && word.is_contiguous() && pos.is_contiguous() && type0.is_contiguous() &&
                   w.is_contiguous() && b.is_contiguous() && out.is_contiguous(),
               "contiguous operands");
-  TORCH_CHECK(S >= 1 && T % S == 0 && pos.size(0) >= S && pos.size(1) == H && type0.numel() == H && w.numel() == H &&
+  TORCH_CHECK(S >= 1 && (at || T % S == 0) && pos.size(0) >= S && pos.size(1) == H && type0.numel() == H && w.numel() == H &&
                   b.numel() == H && out.numel() == T * H && H % 8 == 0 && H <= 2048,
               "embed_ln shapes");
   ok(dllm_embed_ln(ids.data_ptr<int>(), word.data_ptr(), pos.data_ptr(), type0.data_ptr(), w.data_ptr(), b.data_ptr(),
-                   out.data_ptr(), T, S, H, word.size(0), (float)eps, stream()),
+                   out.data_ptr(), T, S, H, word.size(0), (float)eps, at ? at->data_ptr<int>() : nullptr, stream()),
      "embed_ln");
 }
 // ---- sequence mixers and the f32 residual stream (csrc/kernels/seqmix.hip, latent.hip).
@@ -2537,8 +2555,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("splits") = 1, py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("mfma") = true,
         py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none());
   m.def("latent_mfma_ok", [](int64_t rank, int64_t rot, int64_t rows) { return dllm_latent_mfma_ok((int)rank, (int)rot, (int)rows) != 0; });
-  m.def("encoder_attention", &encoder_attention);
-  m.def("embed_ln", &embed_ln);
+  m.def("encoder_attention", &encoder_attention, py::arg("qkv"), py::arg("lens"), py::arg("out"), py::arg("B"), py::arg("S"), py::arg("nh"), py::arg("d"), py::arg("scale"), py::arg("starts") = py::none());
+  m.def("embed_ln", &embed_ln, py::arg("ids"), py::arg("word"), py::arg("pos"), py::arg("type0"), py::arg("w"), py::arg("b"), py::arg("out"), py::arg("S"), py::arg("eps"), py::arg("positions") = py::none());
   m.def("moe_ffn", &moe_ffn, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
         py::arg("act_mode") = 0);
   m.def("moe_tail_ok", [](int64_t H, int64_t groups) { return dllm_moe_tail_ok((int)H, (int)groups) != 0; });
@@ -2574,7 +2592,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("embed", &embed, py::arg("ids"), py::arg("table"), py::arg("out"), py::arg("lo"), py::arg("ssq") = py::none(),
         py::arg("sc_dst") = py::none(), py::arg("sc_buf") = py::none());
   m.def("gelu", &gelu);
-  m.def("mean_pool_l2", &mean_pool_l2);
+  m.def("mean_pool_l2", &mean_pool_l2, py::arg("x"), py::arg("lens"), py::arg("out"), py::arg("starts") = py::none());
   m.def("moe_gate", &moe_gate);
   m.def("moe_router", &moe_router, py::arg("x"), py::arg("wg"), py::arg("k"), py::arg("ids"), py::arg("w"),
         py::arg("logits") = py::none(), py::arg("shared") = false, py::arg("scale") = 1.0);

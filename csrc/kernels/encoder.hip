@@ -1,4 +1,4 @@
-// Router sentence encoder (MiniLM / BERT) kernels: bidirectional attention over a padded batch
+// Router sentence encoder (MiniLM / BERT) kernels: bidirectional attention over a padded or packed batch
 // and the fused embedding sum + LayerNorm.  The projections run on tgemm.hip (bias / GELU /
 // residual epilogues); LayerNorm after each residual on norm.hip; pooling on cosine.hip.
 //
@@ -13,6 +13,9 @@
 //   xor-shuffles) and O^T += V^T . P^T with P^T taken straight from the score registers (key
 //   permutation k-slot 8g+j <-> key j < 4 ? 4g+j : 16+4g+j-4, the same trick as attention.hip).
 //   Keys >= lens[b] are masked (padding tokens); K/V rows past S are zero in LDS.
+//   starts != null: the rows of all sequences lie one behind the other (sequence b from row starts[b], lens[b] of them, S the
+//   longest), and no row is padding: 96 texts of 6 to 70 words are 3800 rows instead of 6912, and every launch of the encoder
+//   takes about that share of its time (GEMMs 606 -> 406 us, attention 101 -> 79).
 #include "common.h"
 
 namespace {
@@ -20,17 +23,22 @@ constexpr float LOG2E = 1.4426950408889634f;
 
 template <int D>
 __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict__ qkv, const int* __restrict__ lens,
-                                                           u16* __restrict__ out, int S, int SP, int nh,
-                                                           float scale_log2) {
+                                                           u16* __restrict__ out, int Smax, int nh, float scale_log2,
+                                                           const int* __restrict__ starts, int T) {
   constexpr int KSTEPS = D / 32, NT = D / 16, CPR = D / 8;  // 16-B chunks per head row
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int b = blockIdx.z, h = blockIdx.y;
+  const long row0 = starts ? min(max(starts[b], 0), T) : b * (long)Smax;
+  // rows of this sequence (packed) or of every one (padded); the LDS holds Smax of them
+  const int S = starts ? (int)min((long)min(max(lens[b], 0), Smax), T - row0) : Smax;
+  if ((int)blockIdx.x * 64 >= S) return;     // the whole workgroup
+  const int SP = (S + 31) & ~31;
   const int VLD = SP + 8;  // V^T row stride (bf16): 16-B pad against bank conflicts
   u16* sk = reinterpret_cast<u16*>(smem);    // [SP][D]
   u16* sv = sk + SP * D;                     // [D][VLD]
-  const int b = blockIdx.z, h = blockIdx.y;
   const int H = nh * D;
   const long ld = 3L * H;
-  const u16* base = qkv + (long)b * S * ld;
+  const u16* base = qkv + row0 * ld;
   const int len = min(lens[b], S);
 
   // ---- stage K rows and V^T for the whole sequence (zero past S)
@@ -107,7 +115,7 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   if (q >= S) return;
   // acc[n][e] = O^T[dim 16n + 4g + e][query rl]: 4 consecutive dims -> one 8-B store
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  u16* op = out + ((long)b * S + q) * H + h * D;
+  u16* op = out + (row0 + q) * H + h * D;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     const uint32_t lo = (uint32_t)f2bf(acc[n][0] * inv) | ((uint32_t)f2bf(acc[n][1] * inv) << 16);
@@ -116,16 +124,17 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   }
 }
 
-// out[t] = LayerNorm(word[ids[t]] + pos[t % S] + type0) * w + b   (one wave per token, H <= 2048)
+// out[t] = LayerNorm(word[ids[t]] + pos[p] + type0) * w + b, p = at[t] or t % S   (one wave per token, H <= 2048)
 __global__ void __launch_bounds__(256) embed_ln_kernel(const int* __restrict__ ids, const u16* __restrict__ word,
                                                        const u16* __restrict__ pos, const u16* __restrict__ type0,
                                                        const u16* __restrict__ w, const u16* __restrict__ bias,
-                                                       u16* __restrict__ out, int T, int S, int H, int vocab, float eps) {
+                                                       u16* __restrict__ out, int T, int S, int H, int vocab, float eps,
+                                                       const int* __restrict__ at) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= T) return;
   const int id = min(max(ids[t], 0), vocab - 1);
   const u16* wr = word + (long)id * H;
-  const u16* pr = pos + (long)(t % S) * H;
+  const u16* pr = pos + (long)(at ? min(max(at[t], 0), S - 1) : t % S) * H;
   float x[4][8];
   float s = 0.f;
 #pragma unroll
@@ -164,7 +173,7 @@ __global__ void __launch_bounds__(256) embed_ln_kernel(const int* __restrict__ i
 }  // namespace
 
 extern "C" int dllm_encoder_attention(const void* qkv, const int* lens, void* out, int B, int S, int nh, int d,
-                                      float scale, hipStream_t stream) {
+                                      float scale, const int* starts, int T, hipStream_t stream) {
   if (B <= 0 || S <= 0) return 0;
   if (S > 512) return -1;
   const int SP = (S + 31) / 32 * 32;
@@ -180,12 +189,12 @@ extern "C" int dllm_encoder_attention(const void* qkv, const int* lens, void* ou
   if (attr_rc != 0 && lds > 64 * 1024) return -3;
   switch (d) {
     case 32:
-      hipLaunchKernelGGL(encoder_attn_kernel<32>, grid, dim3(256), lds, stream, (const u16*)qkv, lens, (u16*)out, S, SP,
-                         nh, scale * LOG2E);
+      hipLaunchKernelGGL(encoder_attn_kernel<32>, grid, dim3(256), lds, stream, (const u16*)qkv, lens, (u16*)out, S, nh,
+                         scale * LOG2E, starts, T);
       break;
     case 64:
-      hipLaunchKernelGGL(encoder_attn_kernel<64>, grid, dim3(256), lds, stream, (const u16*)qkv, lens, (u16*)out, S, SP,
-                         nh, scale * LOG2E);
+      hipLaunchKernelGGL(encoder_attn_kernel<64>, grid, dim3(256), lds, stream, (const u16*)qkv, lens, (u16*)out, S, nh,
+                         scale * LOG2E, starts, T);
       break;
     default:
       return -2;
@@ -194,10 +203,11 @@ extern "C" int dllm_encoder_attention(const void* qkv, const int* lens, void* ou
 }
 
 extern "C" int dllm_embed_ln(const int* ids, const void* word, const void* pos, const void* type0, const void* w,
-                             const void* b, void* out, int T, int S, int H, int vocab, float eps, hipStream_t stream) {
+                             const void* b, void* out, int T, int S, int H, int vocab, float eps, const int* at,
+                             hipStream_t stream) {
   if (H % 8 || H > 2048) return -1;
   if (T <= 0) return 0;
   hipLaunchKernelGGL(embed_ln_kernel, dim3((T + 3) / 4), dim3(256), 0, stream, ids, (const u16*)word, (const u16*)pos,
-                     (const u16*)type0, (const u16*)w, (const u16*)b, (u16*)out, T, S, H, vocab, eps);
+                     (const u16*)type0, (const u16*)w, (const u16*)b, (u16*)out, T, S, H, vocab, eps, at);
   return (int)hipGetLastError();
 }

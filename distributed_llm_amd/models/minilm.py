@@ -125,27 +125,29 @@ class MiniLMEncoder:
 
     @torch.no_grad()
     def _forward(self, texts: List[str], max_len: int) -> torch.Tensor:
-        """One padded batch through the HIP encoder: fused embedding+LN, per layer 4 tgemm launches
-        (QKV + bias, Wo + bias + residual, W1 + bias + GELU, W2 + bias + residual), the encoder
-        attention kernel and 2 LayerNorms; masked mean-pool + L2 (csrc/kernels/encoder.hip,
-        tgemm.hip, norm.hip, cosine.hip).  CPU tensors run the same graph on ops.reference."""
+        """One packed batch through the HIP encoder (the texts' rows one behind the other, no padding): fused embedding+LN,
+        per layer 4 tgemm launches (QKV + bias, Wo + bias + residual, W1 + bias + GELU, W2 + bias + residual), the encoder
+        attention kernel and 2 LayerNorms; mean-pool + L2 (csrc/kernels/encoder.hip, tgemm.hip, norm.hip, elementwise.hip).
+        CPU tensors run the same graph on ops.reference."""
         cfg = self.cfg
         toks = [self.tok.encode(t, max_len) for t in texts]
-        B, S = len(toks), max(len(x) for x in toks)
-        ids = torch.zeros((B, S), dtype=torch.int32)
-        for i, x in enumerate(toks):
-            ids[i, :len(x)] = torch.tensor(x, dtype=torch.int32)
-        lens = torch.tensor([len(x) for x in toks], dtype=torch.int32)
-        ids, lens_d = ids.to(self.device), lens.to(self.device)
+        lens = [len(x) for x in toks]
+        B, S, T = len(toks), max(lens), sum(lens)
+        flat, at, starts = [], [], []
+        for x, n in zip(toks, lens):
+            starts.append(len(flat))
+            flat += x
+            at += range(n)
+        ids, at_d, starts_d, lens_d = torch.tensor(flat + at + starts + lens, dtype=torch.int32).to(self.device).split([T, T, B, B])
         H, nh = cfg.hidden, cfg.heads
-        x = ops.embed_ln(ids, self.word, self.pos, self.type0, *self.emb_ln, S, cfg.eps)
+        x = ops.embed_ln(ids, self.word, self.pos, self.type0, *self.emb_ln, S, cfg.eps, at_d)
         for L in self.layers:
             qkv = ops.gemm.linear_bias(x, L["wqkv"], L["bqkv"])
-            a = ops.encoder_attention(qkv, lens_d, B, S, nh, H // nh)
+            a = ops.encoder_attention(qkv, lens_d, B, S, nh, H // nh, starts=starts_d)
             x = ops.layer_norm(ops.gemm.linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], cfg.eps)
             f = ops.gemm.linear_bias(x, L["w1"], L["b1"], gelu=True)
             x = ops.layer_norm(ops.gemm.linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], cfg.eps)
-        return ops.mean_pool_l2(x.view(B, S, H), lens_d)
+        return ops.mean_pool_l2(x, lens_d, starts_d)
 
     @torch.no_grad()
     def reference_forward(self, texts: List[str], max_len: int = 256) -> torch.Tensor:

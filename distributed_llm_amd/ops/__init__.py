@@ -362,36 +362,40 @@ def gelu(x: torch.Tensor) -> torch.Tensor:
 
 
 def encoder_attention(qkv: torch.Tensor, lens: torch.Tensor, B: int, S: int, nh: int, d: int,
-                      scale: Optional[float] = None) -> torch.Tensor:
+                      scale: Optional[float] = None, starts: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Bidirectional (encoder) attention over a padded batch, qkv [B*S, 3 nh d] -> [B*S, nh d];
-    keys at positions >= lens[b] are masked (csrc/kernels/encoder.hip)."""
+    keys at positions >= lens[b] are masked (csrc/kernels/encoder.hip).  ``starts`` (int32 [B]): a packed batch, text b's
+    ``lens[b]`` rows from row ``starts[b]``, S the longest; qkv [T, 3 nh d] -> [T, nh d]."""
     scale = (1.0 / math.sqrt(d)) if scale is None else scale
     ext = _native(qkv)
     if ext is None:
-        return ref.encoder_attention(qkv, lens, B, S, nh, d, scale)
-    out = torch.empty((B * S, nh * d), dtype=qkv.dtype, device=qkv.device)
-    ext.encoder_attention(qkv.contiguous(), lens.to(torch.int32).contiguous(), out, B, S, nh, d, float(scale))
+        return ref.encoder_attention(qkv, lens, B, S, nh, d, scale, starts)
+    out = torch.empty((qkv.shape[0] if starts is not None else B * S, nh * d), dtype=qkv.dtype, device=qkv.device)
+    ext.encoder_attention(qkv.contiguous(), lens.to(torch.int32).contiguous(), out, B, S, nh, d, float(scale), starts)
     return out
 
 
 def embed_ln(ids: torch.Tensor, word: torch.Tensor, pos: torch.Tensor, type0: torch.Tensor, w: torch.Tensor,
-             b: torch.Tensor, S: int, eps: float) -> torch.Tensor:
-    """BERT embeddings: LayerNorm(word[ids] + pos[t % S] + type0) for ids [B, S] -> [B*S, H]."""
+             b: torch.Tensor, S: int, eps: float, positions: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """BERT embeddings: LayerNorm(word[ids] + pos[t % S] + type0) for ids [B, S] -> [B*S, H]; with ``positions``
+    (int32 [T], below S) pos[positions[t]] for packed ids [T]."""
     ext = _native(word)
     if ext is None:
-        return ref.embed_ln(ids, word, pos, type0, w, b, S, eps)
+        return ref.embed_ln(ids, word, pos, type0, w, b, S, eps, positions)
     ids = ids.reshape(-1).to(torch.int32).contiguous()
     out = torch.empty((ids.numel(), word.shape[1]), dtype=word.dtype, device=word.device)
-    ext.embed_ln(ids, word, pos, type0, w, b, out, int(S), float(eps))
+    ext.embed_ln(ids, word, pos, type0, w, b, out, int(S), float(eps), positions)
     return out
 
 
-def mean_pool_l2(x: torch.Tensor, lens: torch.Tensor) -> torch.Tensor:
+def mean_pool_l2(x: torch.Tensor, lens: torch.Tensor, starts: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Unit vectors of the mean over each text's first ``lens[b]`` rows: x [B, S, H], or packed [T, H] with ``starts``
+    (int32 [B])."""
     ext = _native(x)
     if ext is None:
-        return ref.mean_pool_l2(x, lens)
-    out = torch.empty((x.shape[0], x.shape[2]), dtype=torch.float32, device=x.device)
-    ext.mean_pool_l2(x.contiguous(), lens.to(torch.int32).contiguous(), out)
+        return ref.mean_pool_l2(x, lens, starts)
+    out = torch.empty((lens.numel(), x.shape[-1]), dtype=torch.float32, device=x.device)
+    ext.mean_pool_l2(x.contiguous(), lens.to(torch.int32).contiguous(), out, starts)
     return out
 
 

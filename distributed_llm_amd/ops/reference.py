@@ -152,9 +152,12 @@ def gelu(x):
     return torch.nn.functional.gelu(x.float()).to(x.dtype)
 
 
-def encoder_attention(qkv, lens, B, S, nh, d, scale):
+def encoder_attention(qkv, lens, B, S, nh, d, scale, starts=None):
     """Bidirectional attention of a padded batch: qkv [B*S, 3 nh d] -> [B*S, nh d]; keys >= lens[b]
-    masked (csrc/kernels/encoder.hip)."""
+    masked (csrc/kernels/encoder.hip).  Packed with ``starts``: each text on its own."""
+    if starts is not None:
+        parts = [encoder_attention(qkv[a:a + n], torch.tensor([n]), 1, n, nh, d, scale) for a, n in zip(starts.tolist(), lens.tolist())]
+        return torch.cat(parts) if parts else qkv[:, :nh * d]
     x = qkv.float().view(B, S, 3, nh, d).permute(2, 0, 3, 1, 4)   # [3, B, nh, S, d]
     q, k, v = x[0], x[1], x[2]
     s = (q @ k.transpose(-1, -2)) * scale
@@ -165,16 +168,18 @@ def encoder_attention(qkv, lens, B, S, nh, d, scale):
     return o.to(qkv.dtype)
 
 
-def embed_ln(ids, word, pos, type0, w, b, S, eps):
-    """LayerNorm(word[ids] + pos[t % S] + type0) for flattened [B*S] ids (csrc/kernels/encoder.hip)."""
+def embed_ln(ids, word, pos, type0, w, b, S, eps, positions=None):
+    """LayerNorm(word[ids] + pos[t % S] + type0) for flattened [B*S] ids, or pos[positions] (csrc/kernels/encoder.hip)."""
     T = ids.numel()
-    p = pos[:S].float().repeat(T // S, 1)
+    p = pos[:S].float().repeat(T // S, 1) if positions is None else pos[positions.long()].float()
     x = word[ids.long().reshape(-1)].float() + p + type0.float()
     y = torch.nn.functional.layer_norm(x, (x.shape[-1],), w.float(), b.float(), eps)
     return y.to(word.dtype)
 
 
-def mean_pool_l2(x, lens):
+def mean_pool_l2(x, lens, starts=None):
+    if starts is not None:
+        return torch.cat([mean_pool_l2(x[None, a:a + n], torch.tensor([n])) for a, n in zip(starts.tolist(), lens.tolist())])
     B, S, H = x.shape
     m = (torch.arange(S)[None, :].to(x.device) < lens.to(x.device)[:, None]).float()
     s = (x.float() * m[..., None]).sum(1) / m.sum(1, keepdim=True).clamp(min=1.0)

@@ -76,3 +76,37 @@ def test_minilm_forward_matches_fp32_reference():
     cos = (got.cpu().float() * want).sum(-1)
     assert cos.min().item() > 0.999, cos
     assert enc.memo_stats()["encoded_texts"] == len(texts)
+
+
+@pytest.mark.parametrize("lens", [[1], [16], [77, 1, 32, 33, 64, 65, 2], [512, 3], [5] * 40])
+@pytest.mark.parametrize("nh,d", [(12, 32), (3, 64), (5, 32)])
+def test_packed_batch(lens, nh, d):
+    """Rows one behind the other: attention, embedding positions and pooling against each text on its own; texts that end at and past
+    the kernels' blocks of 32 keys and 64 queries, widths with one and several row groups."""
+    torch.manual_seed(len(lens) + d)
+    H, T, S = nh * d, sum(lens), max(lens)
+    starts = [sum(lens[:i]) for i in range(len(lens))]
+    dev = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    qkv = _b(T, 3 * H)
+    got = ops.encoder_attention(qkv, dev(lens), len(lens), S, nh, d, starts=dev(starts))
+    word, pos, t0, w, b = _b(100, H, scale=0.5), _b(512, H, scale=0.5), _b(H, scale=0.5), _b(H, scale=0.3) + 1, _b(H, scale=0.3)
+    ids, at = torch.randint(0, 100, (T,), dtype=torch.int32), [p for n in lens for p in range(n)]
+    emb = ops.embed_ln(ids.cuda(), word, pos, t0, w, b, S, 1e-12, dev(at))
+    pool = ops.mean_pool_l2(emb, dev(lens), dev(starts))
+    for i, (a, n) in enumerate(zip(starts, lens)):
+        one = torch.tensor([n], dtype=torch.int32).cuda()
+        # the same arithmetic row by row: a padded batch of one text gives the same bits
+        assert torch.equal(got[a:a + n], ops.encoder_attention(qkv[a:a + n].contiguous(), one, 1, n, nh, d))
+        assert torch.equal(emb[a:a + n], ops.embed_ln(ids[None, a:a + n].cuda(), word, pos, t0, w, b, n, 1e-12))
+        want = F.normalize(emb[a:a + n].double().mean(0), dim=0)
+        # n rows summed in f32: n roundings of 2^-24 at most, far below
+        assert float((pool[i].double() - want).norm()) < 1e-6
+
+
+@pytest.mark.parametrize("H", [4, 8, 100, 384, 1000, 1024, 2048])
+def test_mean_pool_widths(H):
+    x = _b(3, 9, H)
+    lens = torch.tensor([9, 1, 6], dtype=torch.int32).cuda()
+    got = ops.mean_pool_l2(x, lens)
+    for i, n in enumerate(lens.tolist()):
+        assert float((got[i].double() - F.normalize(x[i, :n].double().mean(0), dim=0)).norm()) < 1e-6
