@@ -141,12 +141,7 @@ class MiniLMEncoder:
         ids, at_d, starts_d, lens_d = torch.tensor(flat + at + starts + lens, dtype=torch.int32).to(self.device).split([T, T, B, B])
         H, nh = cfg.hidden, cfg.heads
         x = ops.embed_ln(ids, self.word, self.pos, self.type0, *self.emb_ln, S, cfg.eps, at_d)
-        for L in self.layers:
-            qkv = ops.gemm.linear_bias(x, L["wqkv"], L["bqkv"])
-            a = ops.encoder_attention(qkv, lens_d, B, S, nh, H // nh, starts=starts_d)
-            x = ops.layer_norm(ops.gemm.linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], cfg.eps)
-            f = ops.gemm.linear_bias(x, L["w1"], L["b1"], gelu=True)
-            x = ops.layer_norm(ops.gemm.linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], cfg.eps)
+        x = ops.gemm.encoder_layers(x, lens_d, starts_d, S, nh, H // nh, cfg.eps, self.layers)
         return ops.mean_pool_l2(x, lens_d, starts_d)
 
     @torch.no_grad()

@@ -626,6 +626,39 @@ def linear_bias_residual(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, r
     return residual
 
 
+def encoder_layers(x: torch.Tensor, lens: torch.Tensor, starts: torch.Tensor, S: int, nh: int, d: int, eps: float,
+                   layers) -> torch.Tensor:
+    """The sentence encoder's layers (dicts with wqkv, bqkv, wo, bo, ln1, w1, b1, w2, b2, ln2) over packed rows x [T, nh d], which
+    are overwritten: QKV, attention, output + residual, LayerNorm, up + GELU, down + residual, LayerNorm.  On the GPU one call
+    launches them all."""
+    from . import encoder_attention, layer_norm
+    T, H = x.shape
+    names = ("wqkv", "wo", "w1", "w2")
+    if T and layers and x.is_contiguous() and all(_enc_ok(x, L[n]) for L in layers for n in names):
+        shapes = [tuple(layers[0][n].shape) for n in names]
+        plans = [tg_plan(T, n, k) for n, k in shapes]
+        if all(tuple(L[n].shape) == s for L in layers for n, s in zip(names, shapes)) and not any(p[8:9] == (1,) for p in plans):
+            full, floats, tiles = [], 0, 0
+            for p, (n, k) in zip(plans, shapes):
+                p = p + (1, 4, 1, 0, 0, 64, 16, 0)[len(p) - 4:]
+                if k % (64 * p[4]):
+                    p = p[:4] + (1, p[5], 1) + p[7:]
+                if _tg_splits(k, p[3], p[4]) > 1:
+                    fl, ti = _need_tg(T, n, k, p[0], p[1], p[3], p[4])
+                    floats, tiles = max(floats, fl), max(tiles, ti)
+                full.append(list(p[:8] + p[9:]))
+            part, cnt = _P.workspace(x.device, floats, tiles) if tiles else (None, None)
+            return _native(x).encoder_layers(x, lens, starts, int(S), int(nh), int(d), float(eps),
+                                             [t for L in layers for t in (L["wqkv"], L["bqkv"], L["wo"], L["bo"], *L["ln1"], L["w1"], L["b1"],
+                                                                          L["w2"], L["b2"], *L["ln2"])], full, part, cnt)
+    for L in layers:
+        a = encoder_attention(linear_bias(x, L["wqkv"], L["bqkv"]), lens, lens.numel(), S, nh, d, starts=starts)
+        x = layer_norm(linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], eps)
+        f = linear_bias(x, L["w1"], L["b1"], gelu=True)
+        x = layer_norm(linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], eps)
+    return x
+
+
 def max_slots(N: int, M: int = 0) -> int:
     """Rows a partial-row-sum buffer needs for a residual producer of N columns: one per 64-column
     tgemm tile, at batch <= 8 one per fused-GEMV workgroup (N / 4 at R = 1), at batch <= 16 one

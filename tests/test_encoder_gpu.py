@@ -110,3 +110,24 @@ def test_mean_pool_widths(H):
     got = ops.mean_pool_l2(x, lens)
     for i, n in enumerate(lens.tolist()):
         assert float((got[i].double() - F.normalize(x[i, :n].double().mean(0), dim=0)).norm()) < 1e-6
+
+
+@pytest.mark.parametrize("lens", [[16], [3] * 30, [70, 30, 5, 64] * 8])
+@pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (4, 64, 512), (2, 32, 96), (3, 32, 256)])
+def test_layers_in_one_call(lens, nh, d, inter):
+    """The same launches with the same plans as one call per operation (widths that are no multiple of 64 take those): equal bits."""
+    torch.manual_seed(inter)
+    H, T, S = nh * d, sum(lens), max(lens)
+    layers = [dict(wqkv=_b(3 * H, H, scale=0.05), bqkv=_b(3 * H), wo=_b(H, H, scale=0.05), bo=_b(H), ln1=(_b(H) + 1, _b(H)), w1=_b(inter, H, scale=0.05),
+                   b1=_b(inter), w2=_b(H, inter, scale=0.05), b2=_b(H), ln2=(_b(H) + 1, _b(H))) for _ in range(2)]
+    x0 = _b(T, H)
+    dl = torch.tensor(lens, dtype=torch.int32).cuda()
+    ds = torch.tensor([sum(lens[:i]) for i in range(len(lens))], dtype=torch.int32).cuda()
+    got = ops.gemm.encoder_layers(x0.clone(), dl, ds, S, nh, d, 1e-12, layers)
+    x = x0.clone()
+    for L in layers:
+        a = ops.encoder_attention(ops.gemm.linear_bias(x, L["wqkv"], L["bqkv"]), dl, len(lens), S, nh, d, starts=ds)
+        x = ops.layer_norm(ops.gemm.linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], 1e-12)
+        f = ops.gemm.linear_bias(x, L["w1"], L["b1"], gelu=True)
+        x = ops.layer_norm(ops.gemm.linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], 1e-12)
+    assert torch.equal(got, x)
