@@ -143,6 +143,8 @@ int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
                     int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, hipStream_t);
 int dllm_moe_tail_ok(int, int);
+int dllm_enc_gemm_ok(int, int, int);
+int dllm_enc_gemm(const void*, long, const void*, const void*, void*, long, int, int, int, int, hipStream_t);
 int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, const int*, int, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
                   float, const int*, hipStream_t);
@@ -1364,6 +1366,26 @@ void encoder_attention(torch::Tensor qkv, torch::Tensor lens, torch::Tensor out,
      "encoder_attention");
 }
 
+// Projection of few rows with a bias (encoder.hip enc_gemm); false: not taken (rows, widths, alignment), nothing launched
+bool enc_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor bias, torch::Tensor y, int64_t epi) {
+  check_bf16(x, "x");
+  check_bf16(w, "w");
+  check_bf16(bias, "bias");
+  check_bf16(y, "y");
+  TORCH_CHECK(epi == 0 || epi == 1 || epi == 4, "epi: plain, residual or gelu");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 2 && w.is_contiguous() && w.size(1) == x.size(1) && bias.is_contiguous() &&
+                  bias.numel() == w.size(0) && y.dim() == 2 && y.stride(1) == 1 && y.size(0) == x.size(0) && y.size(1) == w.size(0),
+              "x [M, K], w [N, K], bias [N], y [M, N]");
+  const int64_t M = x.size(0), N = w.size(0), K = w.size(1);
+  const auto al = [](const torch::Tensor& t, uintptr_t b) { return ((uintptr_t)t.data_ptr() & (b - 1)) == 0; };
+  if (M > 64 || !dllm_enc_gemm_ok((int)M, (int)N, (int)K) || x.stride(0) % 8 || y.stride(0) % 4 || !al(x, 16) || !al(w, 16) || !al(y, 8) || !al(bias, 8))
+    return false;
+  ok(dllm_enc_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), bias.data_ptr(), y.data_ptr(), y.stride(0), (int)M, (int)N, (int)K, (int)epi,
+                   stream()),
+     "enc_gemm");
+  return true;
+}
+
 // All layers of the sentence encoder over packed rows, in one call: seven launches a layer back to back instead of seven calls
 // from the interpreter, whose 6 us each were most of a single text's 335 us.  weights: per layer QKV w, b, output w, b, norm w, b,
 // up w, b, down w, b, norm w, b.  plans (QKV, output, up, down): bm, bn, stages, splits, ks, waves, k-groups, loaders, k depth, mfma,
@@ -1383,7 +1405,7 @@ torch::Tensor encoder_layers(torch::Tensor x, torch::Tensor lens, torch::Tensor 
   const c10::optional<torch::Tensor> none;
   auto gemm = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& b, const torch::Tensor& out, int epi,
                   const std::vector<int64_t>& p) {
-    tgemm(in, w, out, epi, p[0], p[1], p[2], p[3], p[4], p[5], part, counters, none, 0, 0.0, 0.0, none, none, none, none, none, none,
+    if (!enc_gemm(in, w, b, out, epi)) tgemm(in, w, out, epi, p[0], p[1], p[2], p[3], p[4], p[5], part, counters, none, 0, 0.0, 0.0, none, none, none, none, none, none,
           none, 0, 0, 0, b, p[6], p[7], none, 0, none, p[8], p[9], p[10]);
   };
   for (size_t l = 0; l < weights.size(); l += 12) {
@@ -2591,6 +2613,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none());
   m.def("latent_mfma_ok", [](int64_t rank, int64_t rot, int64_t rows) { return dllm_latent_mfma_ok((int)rank, (int)rot, (int)rows) != 0; });
   m.def("encoder_layers", &encoder_layers);
+  m.def("enc_gemm", &enc_gemm);
   m.def("encoder_attention", &encoder_attention, py::arg("qkv"), py::arg("lens"), py::arg("out"), py::arg("B"), py::arg("S"), py::arg("nh"), py::arg("d"), py::arg("scale"), py::arg("starts") = py::none());
   m.def("embed_ln", &embed_ln, py::arg("ids"), py::arg("word"), py::arg("pos"), py::arg("type0"), py::arg("w"), py::arg("b"), py::arg("out"), py::arg("S"), py::arg("eps"), py::arg("positions") = py::none());
   m.def("moe_ffn", &moe_ffn, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),

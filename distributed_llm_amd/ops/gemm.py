@@ -609,8 +609,9 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, gelu: bool
         return ref.gelu(y) if gelu else y
     M, N, K = x.shape[0], w.shape[0], w.shape[1]
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    if M:
-        _tgemm(_native(x), x, w, EPI_GELU if gelu else EPI_PLAIN, tg_plan(M, N, K), y=y, bias=bias)
+    epi = EPI_GELU if gelu else EPI_PLAIN
+    if M and not _native(x).enc_gemm(x, w, bias, y, epi):      # few rows: straight to registers, else the tiled GEMM
+        _tgemm(_native(x), x, w, epi, tg_plan(M, N, K), y=y, bias=bias)
     return y
 
 
@@ -621,7 +622,7 @@ def linear_bias_residual(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor, r
         residual.copy_((F.linear(x, w, bias).float() + residual.float()).to(residual.dtype))
         return residual
     M, N, K = x.shape[0], w.shape[0], w.shape[1]
-    if M:
+    if M and not _native(x).enc_gemm(x, w, bias, residual, EPI_RESADD):
         _tgemm(_native(x), x, w, EPI_RESADD, tg_plan(M, N, K), y=residual, bias=bias)
     return residual
 

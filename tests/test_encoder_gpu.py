@@ -131,3 +131,19 @@ def test_layers_in_one_call(lens, nh, d, inter):
         f = ops.gemm.linear_bias(x, L["w1"], L["b1"], gelu=True)
         x = ops.layer_norm(ops.gemm.linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], 1e-12)
     assert torch.equal(got, x)
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 48, 63, 64])
+@pytest.mark.parametrize("N,K", [(16, 64), (48, 384), (1152, 320), (384, 1536), (64, 832), (32, 768)])
+def test_few_row_projections(M, N, K):
+    """Blocks of 16 rows full and not, waves without a step of K, partial groups of three steps, rows of a wider matrix."""
+    torch.manual_seed(M + N)
+    x, w, bias, y0 = _b(M, K + 8)[:, :K], _b(N, K, scale=K ** -0.5), _b(N, scale=0.5), _b(M, N)
+    ext = ops._native(x)
+    z = (x.double() @ w.double().t() + bias.double())
+    for epi, want in ((0, z), (1, z + y0.double()), (4, F.gelu(z))):
+        y = y0.clone()
+        assert ext.enc_gemm(x, w, bias, y, epi)
+        # two roundings to bf16 of at most 2^-9 each (the projection and the result)
+        assert float((y.double() - want).norm() / want.norm()) < 2 ** -8
+    assert not ext.enc_gemm(_b(65, K), w, bias, _b(65, N), 0) and not ext.enc_gemm(x, _b(N + 8, K), _b(N + 8), _b(M, N + 8), 0)
