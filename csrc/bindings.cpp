@@ -51,6 +51,8 @@ int dllm_moe_ffn(const void*, long, long, int, const int*, const float*, int, in
 int dllm_rms_rows(const void*, long, int, const float*, void*, long, int, int, int, float, int, hipStream_t);
 int dllm_norm_resadd(const void*, long, int, const float*, float*, void*, int, int, float, int, const float*, hipStream_t);
 int dllm_polynorm(const void*, long, int, const float*, void*, long, int, float, hipStream_t);
+int dllm_router_topk(const void*, long, const float*, int, int, float*, int, int, int, int, int, int, int, const float*, int, int*, float*, float*,
+                     hipStream_t);
 int dllm_route_topk(const float*, long, int, int, int, int, int, int, int, const float*, int, int*, float*, float*, hipStream_t);
 int dllm_ls_resadd_ln(const void*, long, int, const float*, const float*, const void*, long, const float*, long, const void*, long,
                       const float*, float*, const float*, const float*, void*, long, int, float, hipStream_t);
@@ -2268,6 +2270,44 @@ void route_topk(torch::Tensor logits, int64_t E, int64_t top, int64_t count, int
      "route_topk");
 }
 
+// f32 logits of x (bf16) against w [n, H] and route_topk over the first E of them in one launch (seqmix.hip router_topk)
+void router_topk(torch::Tensor x, torch::Tensor w, int64_t E, int64_t top, int64_t count, int64_t keep, int64_t smode, int64_t gmode,
+                 c10::optional<torch::Tensor> corr, int64_t real, torch::Tensor ids, torch::Tensor wts, torch::Tensor idw,
+                 c10::optional<torch::Tensor> logits) {
+  check_bf16(x, "x");
+  check_f32(w, "w");
+  check_i32(ids, "ids");
+  check_f32(wts, "wts");
+  check_f32(idw, "idw");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && (uintptr_t)x.data_ptr() % 16 == 0 && w.dim() == 2 &&
+                  w.is_contiguous() && (uintptr_t)w.data_ptr() % 16 == 0 && w.size(1) == x.size(1),
+              "x [T, H] of 16-byte rows, w [n, H]");
+  const int64_t T = x.size(0), H = x.size(1), n = w.size(0);
+  TORCH_CHECK(n >= 1 && n <= 256 && H % 8 == 0 && H <= 8192, "outputs <= 256, width a multiple of 8 up to 8192");
+  TORCH_CHECK(E >= 1 && E <= n && count >= 1 && E % count == 0 && keep >= 1 && keep <= count && top >= 1 &&
+                  top <= keep * (E / count) && real >= 0 && real <= E,
+              "groups divide the outputs, top fits the kept groups");
+  TORCH_CHECK((smode == 0 || smode == 1) && (gmode == 0 || gmode == 1), "score / group score mode");
+  TORCH_CHECK(ids.is_contiguous() && wts.is_contiguous() && ids.numel() == T * top && wts.numel() == T * top &&
+                  idw.is_contiguous() && idw.numel() == T,
+              "ids / wts [T, top], idw [T]");
+  const float* cp = nullptr;
+  if (corr) {
+    check_f32(*corr, "correction");
+    TORCH_CHECK(corr->is_contiguous() && corr->numel() == E, "correction [E]");
+    cp = corr->data_ptr<float>();
+  }
+  float* lp = nullptr;
+  if (logits) {
+    check_f32(*logits, "logits");
+    TORCH_CHECK(logits->is_contiguous() && logits->numel() == T * n, "logits [T, n]");
+    lp = logits->data_ptr<float>();
+  }
+  ok(dllm_router_topk(x.data_ptr(), x.stride(0), w.data_ptr<float>(), (int)n, (int)H, lp, (int)T, (int)E, (int)top, (int)count, (int)keep,
+                      (int)smode, (int)gmode, cp, (int)real, ids.data_ptr<int>(), wts.data_ptr<float>(), idw.data_ptr<float>(), stream()),
+     "router_topk");
+}
+
 void ls_resadd_ln(torch::Tensor x, torch::Tensor w, torch::Tensor b, double eps, torch::Tensor out,
                   c10::optional<torch::Tensor> y, c10::optional<torch::Tensor> ls, c10::optional<torch::Tensor> bias,
                   c10::optional<torch::Tensor> y2, c10::optional<torch::Tensor> g2, c10::optional<torch::Tensor> h,
@@ -2551,6 +2591,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("group_router", &group_router);
   m.def("swiglu_scale", &swiglu_scale);
   m.def("route_topk", &route_topk);
+  m.def("router_topk", &router_topk);
   m.def("ls_resadd_ln", &ls_resadd_ln);
   m.def("glu_act", &glu_act);
   m.def("proj_norm_prep", &proj_norm_prep, py::arg("proj"), py::arg("heads"), py::arg("kv_heads"), py::arg("dim"), py::arg("vdim"),

@@ -1085,21 +1085,16 @@ constexpr int ROUTER_MAX_E = 1024;
 // of its two best choice scores (gmode 0) or its best (1); the `top` best c inside the `keep` best
 // groups are chosen (ties: the lower index); weights are the scores s.  Outputs >= real are identity
 // experts: their weights leave summed in idw[t], and as 0 in wts.
-__global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict__ logits, long ld, int T, int E, int top,
-                                                         int count, int keep, int smode, int gmode,
-                                                         const float* __restrict__ corr, int real, int* __restrict__ ids,
-                                                         float* __restrict__ wts, float* __restrict__ idw) {
-  // per wave: scores [E], choice scores [E] (-inf: taken), group scores [E], kept-group flags [E bytes]
-  extern __shared__ float rsm[];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + wave;
-  if (t >= T) return;
-  const int per_wave = 3 * E + (E + 3) / 4;
-  float* sc = rsm + wave * per_wave;
+// one token's routing by one wave: z its logits, rsm the wave's patch of route_patch(E) floats
+__device__ __forceinline__ void route_one(const float* z, float* rsm, long t, int E, int top, int count, int keep, int smode, int gmode,
+                                          const float* __restrict__ corr, int real, int* __restrict__ ids,
+                                          float* __restrict__ wts, float* __restrict__ idw) {
+  // scores [E], choice scores [E] (-inf: taken), group scores [E], kept-group flags [E bytes]
+  const int lane = threadIdx.x & 63;
+  float* sc = rsm;
   float* ch = sc + E;
   float* gs = ch + E;
   unsigned char* ok = reinterpret_cast<unsigned char*>(gs + E);
-  const float* z = logits + (long)t * ld;
   if (smode == 0) {
     for (int e = lane; e < E; e += 64) sc[e] = 1.f / (1.f + expf(-z[e]));
   } else {
@@ -1159,6 +1154,66 @@ __global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict
     __builtin_amdgcn_wave_barrier();
   }
   if (lane == 0 && idw) idw[t] = isum;
+}
+
+__host__ __device__ constexpr int route_patch(int E) { return 3 * E + (E + 3) / 4; }
+
+__global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict__ logits, long ld, int T, int E, int top,
+                                                         int count, int keep, int smode, int gmode,
+                                                         const float* __restrict__ corr, int real, int* __restrict__ ids,
+                                                         float* __restrict__ wts, float* __restrict__ idw) {
+  extern __shared__ float rsm[];
+  const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+  if (t >= T) return;
+  route_one(logits + (long)t * ld, rsm + wave * route_patch(E), t, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw);
+}
+
+// The f32 router and the choice in one launch: a workgroup per token, EB rows of w [n, H] f32 a wave in flight, products summed
+// per lane and by a butterfly in a fixed order (a token's logits never depend on the batch), then one wave routes from LDS.
+// Bound by the rows' loads: 16 tokens, 8 outputs, width 1024: 6.2 us against 14.4 (the rounded rows made f32, a library
+// product and the choice in three launches).
+template <int XC>
+__global__ void __launch_bounds__(256) router_topk_kernel(const u16* __restrict__ x, long ldx, const float* __restrict__ w, int n, int H,
+                                                          float* __restrict__ logits, int E, int top, int count, int keep,
+                                                          int smode, int gmode, const float* __restrict__ corr, int real,
+                                                          int* __restrict__ ids, float* __restrict__ wts, float* __restrict__ idw) {
+  constexpr int EB = XC <= 4 ? 2 : 1;
+  extern __shared__ float rsm[];        // [n] logits, then route_one's patch
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nc = H >> 3;
+  const long t = blockIdx.x;
+  uint4 xr[XC];
+#pragma unroll
+  for (int c = 0; c < XC; ++c) xr[c] = lane + 64 * c < nc ? ld16(x + t * ldx + 8 * (lane + 64 * c)) : make_uint4(0u, 0u, 0u, 0u);
+  for (int e0 = wave * EB; e0 < n; e0 += 4 * EB) {
+    f32x4 a[EB][XC], b[EB][XC];
+#pragma unroll
+    for (int j = 0; j < EB; ++j)
+#pragma unroll
+      for (int c = 0; c < XC; ++c) {      // places past the row or the last output are read at 0: x is 0 there, or the sum is dropped
+        const float* p = w + (long)min(e0 + j, n - 1) * H + (lane + 64 * c < nc ? 8 * (lane + 64 * c) : 0);
+        a[j][c] = *reinterpret_cast<const f32x4*>(p);
+        b[j][c] = *reinterpret_cast<const f32x4*>(p + 4);
+      }
+#pragma unroll
+    for (int j = 0; j < EB; ++j) {
+      float s = 0.f;
+#pragma unroll
+      for (int c = 0; c < XC; ++c) {
+        if (lane + 64 * c >= nc) continue;
+        float f[8];
+        unpack8(xr[c], f);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += f[q] * a[j][c][q];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s += f[4 + q] * b[j][c][q];
+      }
+      s = wave_sum(s);
+      if (lane == 0 && e0 + j < n) rsm[e0 + j] = s;
+    }
+  }
+  __syncthreads();
+  if (logits && threadIdx.x < n) logits[t * n + threadIdx.x] = rsm[threadIdx.x];
+  if (wave == 0) route_one(rsm, rsm + n, t, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw);
 }
 
 // gu [rows, E 2 ff] (per expert: gate columns, then up columns) -> y [rows, E ff] = silu(gate) up gate[row, expert]
@@ -1701,6 +1756,24 @@ extern "C" int dllm_route_topk(const float* logits, long ld, int T, int E, int t
   ENSURE_LDS(route_topk_kernel, lds);
   hipLaunchKernelGGL(route_topk_kernel, dim3((T + 3) / 4), dim3(256), lds, st, logits, ld, T, E, top, count, keep, smode, gmode,
                      corr, real, ids, wts, idw);
+  return (int)hipGetLastError();
+}
+
+// logits = x [T, H] bf16 . w [n, H]^T in f32 and the routing of dllm_route_topk over the first E of them, in one launch; logits
+// [T, n] f32 may be null.  n <= 256 outputs, H <= 8192, rows of whole 16-byte vectors
+extern "C" int dllm_router_topk(const void* x, long ldx, const float* w, int n, int H, float* logits, int T, int E, int top, int count,
+                                int keep, int smode, int gmode, const float* corr, int real, int* ids, float* wts, float* idw,
+                                hipStream_t st) {
+  if (n < 1 || n > 256 || E < 1 || E > n || H % 8 || H > 8192 || ldx % 8 || top < 1 || count < 1 || E % count || keep < 1 ||
+      keep > count || top > keep * (E / count) || real < 0)
+    return -1;
+  if (T <= 0) return 0;
+  const size_t lds = 4UL * (n + route_patch(E));
+#define ROUT(XC)                                                                                                                \
+  hipLaunchKernelGGL(router_topk_kernel<XC>, dim3(T), dim3(256), lds, st, (const u16*)x, ldx, w, n, H, logits, E, top, count, keep, smode, \
+                     gmode, corr, real, ids, wts, idw)
+  if (H <= 1024) ROUT(2); else if (H <= 2048) ROUT(4); else if (H <= 4096) ROUT(8); else ROUT(16);
+#undef ROUT
   return (int)hipGetLastError();
 }
 

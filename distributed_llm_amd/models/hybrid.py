@@ -974,8 +974,7 @@ class HybridModel:
         """Sigmoid router in f32 with group-limited top-k, weights = the chosen scores; SwiGLU experts
         on the grouped MFMA kernels, or in the dense form (all experts' columns in two GEMMs, unused
         experts gated to zero) for f32 models and widths the grouped kernels do not take."""
-        logits = F.linear(x.float(), L["router"])
-        ids, w = seqmix.group_router(logits, f.top, f.group_count, f.group_keep)
+        ids, w, _, _ = seqmix.router_topk(x, L["router"], L["router"].shape[0], f.top, f.group_count, f.group_keep)
         if f.scale != 1.0:
             w = w * f.scale
         return self._swiglu_experts(L, f, x, ids, w, tail)
@@ -985,10 +984,9 @@ class HybridModel:
         top-k over experts and identity experts together, weights = the chosen scores; returns the
         terms of the residual launch (ops.seqmix.ls_resadd_ln): the routed experts' sum, the input
         times the identity experts' weights, the shared expert and its gate logit."""
-        logits = F.linear(x.float(), L["router"])      # [T, experts + identity (+ 1: the shared expert's gate)]
-        R = f.experts + f.identity
-        ids, w, idw = seqmix.route_topk(logits, R, f.top, f.group_count, f.group_keep, f.score, f.group_score,
-                                        L.get("corr"), f.experts)
+        R = f.experts + f.identity      # the router's rows: experts + identity (+ 1: the shared expert's gate)
+        ids, w, idw, logits = seqmix.router_topk(x, L["router"], R, f.top, f.group_count, f.group_keep, f.score, f.group_score,
+                                                 L.get("corr"), f.experts, want_logits=bool(f.shared_ff and f.shared_gate))
         if f.scale != 1.0:
             w, idw = w * f.scale, idw * f.scale
         out = dict(y=self._swiglu_experts(L, f, x, ids, w))

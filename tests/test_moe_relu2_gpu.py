@@ -121,3 +121,23 @@ def test_norm_resadd_widths(dt, T, H, groups, pad, bias):
     seqmix.norm_resadd(y, w, 1e-5, x, xl, groups, b)
     assert float((x.double() - want).norm() / want.norm()) < 1e-6
     assert torch.equal(xl, x.to(dt))
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (16, 1024), (5, 1032), (3, 2048), (2, 4096), (2, 8192)])
+@pytest.mark.parametrize("n,E,top,count,keep,score,gscore,real", [(8, 8, 2, 2, 1, "sigmoid", "top2", 8), (13, 12, 3, 4, 2, "softmax", "max", 10),
+                                                                  (256, 256, 8, 8, 4, "sigmoid", "top2", 256), (1, 1, 1, 1, 1, "softmax", "top2", 1)])
+def test_router_topk(T, H, n, E, top, count, keep, score, gscore, real):
+    """Logits, choice and weights of the one launch against f64 logits through the standalone routing; 1 to 16 vectors a lane, outputs
+    that fill no round of the waves, a column behind the routed ones."""
+    torch.manual_seed(n + H)
+    x = torch.randn(T, H + 8, device=DEV).bfloat16()[:, :H]
+    w, corr = torch.randn(n, H, device=DEV) / H ** 0.5, torch.randn(E, device=DEV) * 0.1
+    ids, wt, idw, lg = seqmix.router_topk(x, w, E, top, count, keep, score, gscore, corr, real, want_logits=True)
+    want = x.double() @ w.double().t()
+    assert float((lg.double() - want).abs().max()) < 2e-5          # H products of order H^-1/2 summed in f32
+    i2, w2, d2 = seqmix.route_topk(lg, E, top, count, keep, score, gscore, corr, real)
+    assert torch.equal(ids, i2) and torch.equal(wt, w2) and torch.equal(idw, d2)
+    i3, w3, d3, none = seqmix.router_topk(x, w, E, top, count, keep, score, gscore, corr, real)
+    assert none is None and torch.equal(ids, i3) and torch.equal(wt, w3) and torch.equal(idw, d3)
+    one = seqmix.router_topk(x[-1:], w, E, top, count, keep, score, gscore, corr, real, want_logits=True)
+    assert torch.equal(one[3], lg[-1:])                            # a token's logits do not depend on the batch
