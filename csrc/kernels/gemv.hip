@@ -384,6 +384,16 @@ void launch_gemv(const void* x, long ldx, const void* w, void* y, long ldy, int 
   // Llama-3-8B's, never slower; at batch 2 it is slower on the large shapes, so batch 1 only.
   if constexpr (M == 1 && !SW && !NORM) {
     const size_t lds_xg = EPI != GV_PLAIN ? (size_t)(M + 4 * R * M + 4 * M) * sizeof(float) : 0;
+    // Long rows on up to a workgroup per CU: a wave's whole rows (up to 12 loads a row) in flight, where 4 a trip wait out three
+    // latencies.  us with 12 / 4: 2048 x 5632 at R 2 6.5 / 7.6 (the best before, R 1: 7.0), 2048 x 4096 6.0 / 6.2, 1024 x 4096 at
+    // R 1 4.4 / 4.8; two workgroups a CU or four rows a wave lose (2048 x 5632 at R 1 7.9 / 7.0, 4096 x 4096 at R 2 10.2 / 8.5).
+    if constexpr (R <= 2) {
+      if (K > 2048 && K <= 6144 && gemv_blocks<R>(N) <= 256) {
+        hipLaunchKernelGGL((gemv_kernel<M, R, 12, SW, NORM, EPI, true>), dim3(gemv_blocks<R>(N)), dim3(256), lds_xg, stream,
+                           (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, N, K, na, ea);
+        return;
+      }
+    }
     hipLaunchKernelGGL((gemv_kernel<M, R, 4, SW, NORM, EPI, true>), dim3(gemv_blocks<R>(N)), dim3(256), lds_xg,
                        stream, (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, N, K, na, ea);
     return;

@@ -33,3 +33,16 @@ def test_results(N, K):
         y = G._run_plan(G._heuristic(M, N, K), x, w, False, None)
         want = x.double() @ w.double().t()
         assert float((y.double() - want).norm() / want.norm()) < 2 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K", [(1024, 2056), (1024, 4096), (2048, 5632), (2048, 6144), (100, 6152), (2052, 5632), (1028, 4096), (7, 2816)])
+@pytest.mark.parametrize("R", [1, 2, 4])
+def test_gemv_long_rows(N, K, R):
+    """One row on both sides of the line for whole rows in flight: 256 workgroups, 2048 < K <= 6144, the last load partly past K."""
+    torch.manual_seed(N + K)
+    x, w = torch.randn(1, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    y = torch.empty(1, N, device="cuda").bfloat16()
+    ops._native(x).gemv(x, w, y, R, False)
+    want = x.double() @ w.double().t()
+    assert float((y.double() - want).norm() / want.norm()) < 2 ** -8       # one rounding to bf16, f32 sums far below
