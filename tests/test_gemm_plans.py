@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from distributed_llm_amd import ops
 from distributed_llm_amd.ops import gemm as G
 
 SHAPES = [(1024, 1024), (1024, 2816), (5632, 1024), (4096, 1024), (4160, 64), (64, 4096), (2048, 8192), (1536, 768), (64, 64)]
