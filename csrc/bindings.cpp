@@ -24,7 +24,7 @@ int dllm_gemv(const void*, long, const void*, void*, long, int, int, int, int, i
 int dllm_gelu(const void*, void*, long, hipStream_t);
 int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, const int*, int, hipStream_t);
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
-int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, hipStream_t);
+int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, const void*, float, void*, hipStream_t);
 int dllm_scatter_pairs(int*, const int*, int, hipStream_t);
 int dllm_step_fetch(const int*, int*, int, int, int, int, const int*, const int*, int*, int, hipStream_t);
 int dllm_step_store(const int*, int*, int, hipStream_t);
@@ -143,7 +143,8 @@ int dllm_car_vote(int, int*, void*, int*, hipStream_t);
 int dllm_tgemm(const void*, int, int, int, int, int, int, int, hipStream_t, int);
 int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
-                    int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, hipStream_t);
+                    int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, void*, long, float*, long, int, hipStream_t);
+int dllm_moe_slice(int, int);
 int dllm_moe_tail_ok(int, int);
 int dllm_enc_gemm_ok(int, int, int);
 int dllm_enc_gemm(const void*, long, const void*, const void*, void*, long, int, int, int, int, hipStream_t);
@@ -446,9 +447,18 @@ void moe_gate(torch::Tensor logits, int64_t k, torch::Tensor ids, torch::Tensor 
 // fused router GEMV + top-k (batch-invariant): x [T, H] (row stride % 8), wg [E, H] -> ids/w [T, k]
 // scale multiplies the weights; with shared a token gets one more pair, (E, 1)
 void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids, torch::Tensor w,
-                c10::optional<torch::Tensor> logits, bool shared, double scale) {
+                c10::optional<torch::Tensor> logits, bool shared, double scale, c10::optional<torch::Tensor> norm_w, double eps,
+                c10::optional<torch::Tensor> xn) {
   check_bf16(x, "x");
   check_bf16(wg, "router weight");
+  if (norm_w) {      // x is the stream: xn receives its RMS norm, which is what is routed
+    check_bf16(*norm_w, "norm weight");
+    TORCH_CHECK(xn.has_value(), "xn");
+    check_bf16(*xn, "xn");
+    TORCH_CHECK(norm_w->is_contiguous() && norm_w->numel() == x.size(1) && xn->is_contiguous() && xn->sizes() == x.sizes() &&
+                    (((uintptr_t)norm_w->data_ptr() | (uintptr_t)xn->data_ptr()) & 15) == 0,
+                "norm weight [H], xn like x, 16-B aligned");
+  }
   check_i32(ids, "ids");
   check_f32(w, "weights");
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && wg.dim() == 2 && wg.is_contiguous() && wg.size(1) == x.size(1),
@@ -463,7 +473,8 @@ void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids,
     lp = logits->data_ptr<float>();
   }
   ok(dllm_moe_router(x.data_ptr(), x.stride(0), wg.data_ptr(), T, E, H, k, ids.data_ptr<int>(), w.data_ptr<float>(),
-                     lp, (int)shared, (float)scale, stream()),
+                     lp, (int)shared, (float)scale, norm_w ? norm_w->data_ptr() : nullptr, (float)eps,
+                     norm_w ? xn->data_ptr() : nullptr, stream()),
      "moe_router");
 }
 
@@ -933,9 +944,10 @@ void gemv_swiglu(torch::Tensor x, torch::Tensor w, torch::Tensor ssq, int64_t ss
 // caching allocator, so the call is graph-capturable.
 // grouped-tgemm MoE (csrc/kernels/moe.hip dllm_moe_ffn_tg): act_mode 0: w13 [E, 2I, H] interleaved per 16-row
 // group; 1: squared-ReLU experts, w13 [E, I, H]
-void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Tensor w13, torch::Tensor w2,
+int64_t moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Tensor w13, torch::Tensor w2,
                 c10::optional<torch::Tensor> out, std::vector<int64_t> plan, int64_t act_mode, c10::optional<torch::Tensor> norm_w,
-                double eps, c10::optional<torch::Tensor> xs, c10::optional<torch::Tensor> xl, int64_t groups) {
+                double eps, c10::optional<torch::Tensor> xs, c10::optional<torch::Tensor> xl, int64_t groups,
+                c10::optional<torch::Tensor> res, c10::optional<torch::Tensor> ssq) {
   check_bf16(x, "x");
   check_i32(ids, "ids");
   check_f32(wts, "wts");
@@ -958,6 +970,13 @@ void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Te
       check_bf16(*xl, "xl");
       TORCH_CHECK(xl->is_contiguous() && xl->sizes() == xs->sizes() && (uintptr_t)xl->data_ptr() % 8 == 0, "xl [T, H]");
     }
+  } else if (res) {   // the sum is added to the bf16 stream, squares per row and slice in ssq; returns the slices
+    check_bf16(*res, "res");
+    TORCH_CHECK(act_mode == 0 && ssq.has_value() && res->dim() == 2 && res->stride(1) == 1 && res->stride(0) % 8 == 0 &&
+                    (uintptr_t)res->data_ptr() % 16 == 0 && res->size(0) == T && res->size(1) == H,
+                "res [T, H] of 16-byte rows (SwiGLU experts), ssq");
+    check_f32(*ssq, "ssq");
+    TORCH_CHECK(ssq->dim() == 2 && ssq->size(0) >= 1 && ssq->size(1) >= T && ssq->stride(1) == 1, "ssq [slots, >= T]");
   } else {
     TORCH_CHECK(out.has_value(), "out");
     check_bf16(*out, "out");
@@ -987,10 +1006,15 @@ void moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Te
   for (int i = 0; i < 9; ++i) pl[i] = (int)plan[i];
   ok(dllm_moe_ffn_tg(x.data_ptr(), x.stride(0), T, (int)H, ids.data_ptr<int>(), wts.data_ptr<float>(), k, (int)E,
                      w13.data_ptr(), w2.data_ptr(), (int)I, perm.data_ptr<int>(), inv.data_ptr<int>(),
-                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), xs ? nullptr : out->data_ptr(), (int)act_mode, pl,
+                     tiles.data_ptr<int>(), act.data_ptr(), y.data_ptr(), xs || res ? nullptr : out->data_ptr(), (int)act_mode, pl,
                      xs ? norm_w->data_ptr<float>() : nullptr, xs ? xs->data_ptr<float>() : nullptr,
-                     xs && xl ? xl->data_ptr() : nullptr, (float)eps, (int)groups, stream()),
+                     xs && xl ? xl->data_ptr() : nullptr, (float)eps, (int)groups, res ? res->data_ptr() : nullptr,
+                     res ? res->stride(0) : 0, res ? ssq->data_ptr<float>() : nullptr, res ? ssq->stride(0) : 0,
+                     res ? (int)ssq->size(0) : 1, stream()),
      "moe_ffn_tg");
+  if (!res) return 0;
+  const int cw = dllm_moe_slice((int)H, (int)ssq->size(0));
+  return (H + cw - 1) / cw;
 }
 
 // act_mode 0: SwiGLU experts (w13 [E, 2I, H]); 1: squared-ReLU experts without a gate (w13 [E, I, H])
@@ -2662,7 +2686,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("moe_tail_ok", [](int64_t H, int64_t groups) { return dllm_moe_tail_ok((int)H, (int)groups) != 0; });
   m.def("moe_ffn_tg", &moe_ffn_tg, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
         py::arg("plan"), py::arg("act_mode") = 0, py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("xs") = py::none(),
-        py::arg("xl") = py::none(), py::arg("groups") = 1);
+        py::arg("xl") = py::none(), py::arg("groups") = 1, py::arg("res") = py::none(), py::arg("ssq") = py::none());
   m.def("tgemm", &tgemm);
   m.def("res_add_ssq", &res_add_ssq);
   m.def("qkv_post", &qkv_post, py::arg("y"), py::arg("ssq"), py::arg("ssq_n"), py::arg("scale"), py::arg("eps"),
@@ -2695,7 +2719,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("mean_pool_l2", &mean_pool_l2, py::arg("x"), py::arg("lens"), py::arg("out"), py::arg("starts") = py::none());
   m.def("moe_gate", &moe_gate);
   m.def("moe_router", &moe_router, py::arg("x"), py::arg("wg"), py::arg("k"), py::arg("ids"), py::arg("w"),
-        py::arg("logits") = py::none(), py::arg("shared") = false, py::arg("scale") = 1.0);
+        py::arg("logits") = py::none(), py::arg("shared") = false, py::arg("scale") = 1.0, py::arg("norm_w") = py::none(),
+        py::arg("eps") = 0.0, py::arg("xn") = py::none());
   m.def("argmax", &argmax);
   m.def("scatter_pairs", &scatter_pairs);
   m.def("step_fetch", &step_fetch);

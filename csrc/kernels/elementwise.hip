@@ -191,11 +191,13 @@ __global__ void moe_gate_kernel(const float* __restrict__ logits, int T, int E, 
 // Bound by latency: the rows' loads, one butterfly per expert (they overlap) and the choice.  Lane e holds expert e's logit and the
 // choice is a wave-wide maximum (a lane walking the logits in LDS with its choices in scratch took most of the launch): 8
 // experts, width 1024, 24 tokens 6.0 us against 10.0 (an empty launch shows 3).
-template <int XC, int EB>   // EB experts' rows in flight
+// NORM: x is the residual stream; the wave first norms its row, bf16(x / rms(x) * norm_w), leaves that in xn and routes it.
+template <int XC, int EB, bool NORM>   // EB experts' rows in flight
 __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__ x, long x_stride,
                                                          const u16* __restrict__ wg, int T, int E, int H, int k,
                                                          int* __restrict__ ids, float* __restrict__ w,
-                                                         float* __restrict__ logits, int shared, float scale) {
+                                                         float* __restrict__ logits, int shared, float scale,
+                                                         const u16* __restrict__ norm_w, float eps, u16* __restrict__ xn) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int t = blockIdx.x * 4 + wv;
   if (t >= T) return;  // whole wave; no block barrier below
@@ -205,6 +207,31 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
   for (int c = 0; c < XC; ++c) {
     const int ch = lane + 64 * c;
     xr[c] = ch < nc ? ld16(x + (long)t * x_stride + 8 * ch) : make_uint4(0u, 0u, 0u, 0u);
+  }
+  if constexpr (NORM) {
+    uint4 nw[XC];
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < XC; ++c) {
+      const int ch = lane + 64 * c;
+      nw[c] = ch < nc ? ld16(norm_w + 8 * ch) : make_uint4(0u, 0u, 0u, 0u);
+      float f[8];
+      unpack8(xr[c], f);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) s += f[q] * f[q];
+    }
+    const float rstd = rsqrtf(wave_sum(s) / H + eps);
+#pragma unroll
+    for (int c = 0; c < XC; ++c) {
+      const int ch = lane + 64 * c;
+      float f[8], g[8];
+      unpack8(xr[c], f);
+      unpack8(nw[c], g);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) f[q] = f[q] * rstd * g[q];
+      xr[c] = pack8(f);
+      if (ch < nc) st16(xn + (long)t * H + 8 * ch, xr[c]);
+    }
   }
   float lg = -INFINITY;   // lane e: expert e's logit
   for (int e0 = 0; e0 < E; e0 += EB) {
@@ -369,14 +396,21 @@ extern "C" int dllm_moe_gate(const float* logits, int T, int E, int k, int* ids,
 }
 
 extern "C" int dllm_moe_router(const void* x, long x_stride, const void* wg, int T, int E, int H, int k, int* ids,
-                               float* w, float* logits, int shared, float scale, hipStream_t stream) {
+                               float* w, float* logits, int shared, float scale, const void* norm_w, float eps, void* xn,
+                               hipStream_t stream) {
   if (E > 64 || k > 8 || k > E || H % 8 != 0 || H > 8192 || x_stride % 8 != 0) return -1;
   if (T == 0) return 0;
   const dim3 grid((T + 3) / 4), block(256);
   const int nc = H / 8;
 #define ROUTER(XC, EB)                                                                                                          \
-  hipLaunchKernelGGL((moe_router_kernel<XC, EB>), grid, block, 0, stream, (const u16*)x, x_stride, (const u16*)wg, T, E, H, k, ids, \
-                     w, logits, shared, scale)
+  do {                                                                                                                          \
+    if (norm_w)                                                                                                                 \
+      hipLaunchKernelGGL((moe_router_kernel<XC, EB, true>), grid, block, 0, stream, (const u16*)x, x_stride, (const u16*)wg, T, E, H, k, \
+                         ids, w, logits, shared, scale, (const u16*)norm_w, eps, (u16*)xn);                                     \
+    else                                                                                                                        \
+      hipLaunchKernelGGL((moe_router_kernel<XC, EB, false>), grid, block, 0, stream, (const u16*)x, x_stride, (const u16*)wg, T, E, H, k, \
+                         ids, w, logits, shared, scale, nullptr, 0.f, nullptr);                                                 \
+  } while (0)
   if (nc <= 128) ROUTER(2, 8);
   else if (nc <= 256) ROUTER(4, 4);
   else if (nc <= 512) ROUTER(8, 2);

@@ -127,6 +127,39 @@ __global__ void moe_combine_perm_kernel(const T_* __restrict__ y, const int* __r
   }
 }
 
+// The same sum rounded to bf16 and added to the residual stream, r = bf16(bf16(sum) + r), with the row's sums of squares per slice of
+// `cw` columns (res_add_ssq of tgemm.hip, bit for bit, in the combine's launch): a wave per row and slice.
+__global__ void __launch_bounds__(256) moe_combine_resadd_kernel(const u16* __restrict__ y, const int* __restrict__ inv,
+                                                                 const float* __restrict__ wts, int k, int H, int T,
+                                                                 u16* __restrict__ r, long ldr, float* __restrict__ ssq, long ssq_ld,
+                                                                 int cw) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= T) return;
+  u16* rr = r + (long)row * ldr;
+  const int c1 = min(H, (int)(blockIdx.y + 1) * cw);
+  float q = 0.f;
+  for (int c = blockIdx.y * cw + lane * 8; c < c1; c += 512) {
+    float v[8], s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    unpack8(ld16(rr + c), v);
+    for (int j = 0; j < k; ++j) {
+      const long p = (long)row * k + j;
+      float f[8];
+      ld8(y + (long)inv[p] * H + c, f);
+      const float w = wts[p];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] += w * f[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = bf2f(f2bf(v[e] + bf2f(f2bf(s[e]))));
+      q += v[e] * v[e];
+    }
+    st16(rr + c, pack8(v));
+  }
+  q = wave_sum(q);
+  if (lane == 0) ssq[(long)blockIdx.y * ssq_ld + row] = q;
+}
+
 __device__ __forceinline__ bf16x8 ld_or0(const u16* p, bool ok) {
   return __builtin_bit_cast(bf16x8, ok ? ld16(p) : make_uint4(0, 0, 0, 0));
 }
@@ -330,15 +363,20 @@ extern "C" int dllm_moe_ffn(const void* x, long x_stride, long T, int H, const i
 // Tile-list size for BM-row tiles: every expert may leave one partial tile.
 extern "C" int dllm_moe_max_tiles_bm(int P, int E, int bm) { return (P + bm - 1) / bm + E; }
 
+// columns of a slice when a row's squares go to `slices` slots: whole 512-column wave passes (as dllm_res_add_ssq)
+extern "C" int dllm_moe_slice(int H, int slices) { return ((H + slices - 1) / slices + 511) / 512 * 512; }
+
 // plans: {bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2}; act_mode 0: w13 interleaved [E, 2I, H] (16 gate
 // rows, 16 up rows, ...), y bf16; 1: w13 [E, I, H], squared ReLU, y f32.  w2 [E, H, I]; scratch: perm/inv [P], tiles
 // [4 * max_tiles + 1], act [P, I], y [P, H].  xs (f32 [T, H]): instead of `out`, xs += rmsnorm(sum) * nw in `groups` parts, and its
-// rounded copy in xl (norm_resadd of seqmix.hip, in the combine's launch).
+// rounded copy in xl (norm_resadd of seqmix.hip, in the combine's launch).  res (bf16 [T, H], act_mode 0): instead of `out`, added to the
+// residual stream with the rows' squares in ssq [slots][ssq_ld].
 extern "C" int dllm_moe_ffn_tg(const void* x, long x_stride, long T, int H, const int* ids, const float* wts, int k,
                                int E, const void* w13, const void* w2, int I, int* perm, int* inv, int* tiles,
                                void* act, void* y, void* out, int act_mode, const int* plan, const float* nw, float* xs, void* xl,
-                               float eps, int groups, hipStream_t stream) {
-  if (E < 1 || E > 64 || k < 1 || H % 64 != 0 || I % 64 != 0 || x_stride % 8) return -1;
+                               float eps, int groups, void* res, long ldr, float* ssq, long ssq_ld, int slices,
+                               hipStream_t stream) {
+  if (E < 1 || E > 64 || k < 1 || H % 64 != 0 || I % 64 != 0 || x_stride % 8 || (res && (act_mode || ldr % 8 || !ssq || slices < 1))) return -1;
   if (T == 0) return 0;
   const int bm = plan[0], NI = act_mode ? I : 2 * I;
   const int P = (int)(T * k);
@@ -358,6 +396,12 @@ extern "C" int dllm_moe_ffn_tg(const void* x, long x_stride, long T, int H, cons
   d.g_tiles = tiles; d.g_max = max_tiles; d.g_perm = nullptr; d.g_k = 1; d.g_wstride = (long)H * I;
   rc = dllm_tgemm(&d, bm, plan[5], plan[6], plan[7], plan[8], 1, act_mode ? dllm::EPI_F32 : dllm::EPI_PLAIN, stream, 0);
   if (rc) return 2000 + rc;
+  if (res) {                                                                                               // ... the bf16 one
+    const int cw = dllm_moe_slice(H, slices);
+    hipLaunchKernelGGL(moe_combine_resadd_kernel, dim3((unsigned)((T + 3) / 4), (H + cw - 1) / cw), dim3(256), 0, stream, (const u16*)y, inv,
+                       wts, k, H, (int)T, (u16*)res, ldr, ssq, ssq_ld, cw);
+    return (int)hipGetLastError();
+  }
   if (xs) return dllm_moe_norm_resadd(y, act_mode, inv, wts, k, nw, xs, xl, T, H, eps, groups, stream);   // the sum goes into the stream
   long n8 = T * (H / 8);
   long gr = (n8 + 255) / 256;

@@ -480,6 +480,10 @@ class LlamaModel:
                 else:
                     n = resadd(ops.linear(act, L["wd"], wp=L.get("wd_p")), r, ssq_a)
             else:
+                if not tp and self.moe_tg:      # norm and router, and combine and residual add, share a launch
+                    x, ids, w = ops.norm_moe_router(r, L["ln2"], eps, L["wgate"], cfg.experts_per_token)
+                    n = ops.moe_ffn_tg_resadd(x, ids, w, L["w13"], L["w2"], r, ssq_a)
+                    continue
                 x = ops.rms_norm(r, L["ln2"], eps)
                 if not tp:
                     n = ops.gemm.res_add_ssq(self._mlp(L, x), r, ssq_a)

@@ -432,6 +432,35 @@ def moe_router(x: torch.Tensor, wg: torch.Tensor, k: int, shared: bool = False,
     return ids, w
 
 
+def norm_moe_router(r: torch.Tensor, norm_w: torch.Tensor, eps: float, wg: torch.Tensor,
+                    k: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``x = rms_norm(r, norm_w, eps)`` and ``moe_router(x, wg, k)`` -> (x, ids, weights); bf16 rows of whole vectors take one
+    launch."""
+    ext = _native(r)
+    H = r.shape[1]
+    if (ext is None or r.dtype != torch.bfloat16 or H > 8192 or H % 8 or r.stride(1) != 1 or r.stride(0) % 8 or norm_w.dtype != r.dtype
+            or not norm_w.is_contiguous() or not wg.is_contiguous() or any(t.data_ptr() % 16 for t in (r, norm_w, wg))):
+        x = rms_norm(r, norm_w, eps)
+        return (x, *moe_router(x, wg, k))
+    x = torch.empty((r.shape[0], H), dtype=r.dtype, device=r.device)
+    ids = torch.empty((r.shape[0], k), dtype=torch.int32, device=r.device)
+    w = torch.empty((r.shape[0], k), dtype=torch.float32, device=r.device)
+    ext.moe_router(r, wg, k, ids, w, None, False, 1.0, norm_w, float(eps), x)
+    return x, ids, w
+
+
+def moe_ffn_tg_resadd(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torch.Tensor, w2: torch.Tensor, r: torch.Tensor,
+                      ssq: torch.Tensor) -> int:
+    """``gemm.res_add_ssq(moe_ffn_tg(...), r, ssq)`` with the residual add in the combine's launch; returns the slots of
+    ``ssq`` [slots, >= T] written."""
+    ext = _native(x)
+    if ext is None or r.stride(0) % 8 or r.data_ptr() % 16:
+        from . import gemm
+        return gemm.res_add_ssq(moe_ffn_tg(x, ids, wts, w13i, w2), r, ssq)
+    return int(ext.moe_ffn_tg(x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, None,
+                              list(moe_plan(x.shape[0] * ids.shape[1])), 0, res=r, ssq=ssq))
+
+
 def moe_ffn(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torch.Tensor,
             w2: torch.Tensor) -> torch.Tensor:
     """Top-k expert FFN (csrc/kernels/moe.hip): device-side routing + grouped MFMA GEMMs with the

@@ -141,3 +141,23 @@ def test_router_topk(T, H, n, E, top, count, keep, score, gscore, real):
     assert none is None and torch.equal(ids, i3) and torch.equal(wt, w3) and torch.equal(idw, d3)
     one = seqmix.router_topk(x[-1:], w, E, top, count, keep, score, gscore, corr, real, want_logits=True)
     assert torch.equal(one[3], lg[-1:])                            # a token's logits do not depend on the batch
+
+
+@pytest.mark.parametrize("T,H,E,top", [(1, 64, 4, 2), (12, 1024, 8, 2), (5, 1088, 8, 1), (9, 2048, 64, 8), (3, 4096, 8, 2), (2, 8192, 5, 3), (700, 512, 8, 2)])
+def test_norm_router_and_residual_combine(T, H, E, top):
+    """Norm + router and combine + residual add against the launches they replace: 1 to 16 vectors a lane, one and several slots."""
+    torch.manual_seed(H)
+    r = torch.randn(T, H + 8, device=DEV).bfloat16()[:, :H]
+    nw, wg = torch.randn(H, device=DEV).bfloat16(), torch.randn(E, H, device=DEV).bfloat16()
+    x, ids, w = ops.norm_moe_router(r, nw, 1e-5, wg, top)
+    z = r.double() * torch.rsqrt(r.double().pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    assert float((x.double() - z).norm() / z.norm()) < 2 ** -8          # one rounding to bf16
+    i2, w2 = ops.moe_router(x, wg, top)
+    assert torch.equal(ids, i2) and torch.equal(w, w2)                   # the rounded rows are what is routed
+    w13, w2d = torch.randn(E, 128, H, device=DEV).div(H ** 0.5).bfloat16(), torch.randn(E, H, 64, device=DEV).div(8).bfloat16()
+    for slots in (1, 3):
+        ra, rb = r.clone(), r.clone()
+        qa, qb = (torch.zeros(slots, T + 2, device=DEV) for _ in range(2))
+        na = ops.moe_ffn_tg_resadd(x, ids, w, w13, w2d, ra, qa)
+        nb = ops.gemm.res_add_ssq(ops.moe_ffn_tg(x, ids, w, w13, w2d), rb, qb)
+        assert na == nb and torch.equal(ra, rb) and torch.equal(qa, qb)
