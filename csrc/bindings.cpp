@@ -74,7 +74,8 @@ int dllm_qk_norm_prep(const void*, long, int, const float*, int, int, int, int, 
                       int, int, float, float, const int*, const int*, void*, void*, void*, long, int, hipStream_t);
 int dllm_diff_combine(const float*, void*, int, long, int, int, int, float, float, float, hipStream_t);
 int dllm_conv_silu(const void*, long, int, const float*, const float*, void*, const int*, const int*, const int*,
-                   const int*, void*, int, int, int, int, int, int, hipStream_t);
+                   const int*, void*, int, int, int, int, int, int, int, hipStream_t);
+int dllm_zero_free_rows(void*, int, long, int, const int*, const int*, int, hipStream_t);
 long dllm_scan_chunks_scratch(long, int, int, int);
 int dllm_scan_step_ok(long, int, int, const void*, const void*);
 int dllm_scan_chunks(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*, const void*, long,
@@ -84,7 +85,7 @@ int dllm_selective_scan(const void*, const void*, int, const float*, const float
                         int, int, hipStream_t);
 long dllm_retention_lds(int, int);
 int dllm_retention(const void*, long, int, int, int, int, const float*, int, int, const float*, float*, float,
-                   const int*, const int*, const int*, const int*, void*, int, int, float, float*, hipStream_t);
+                   const int*, const int*, const int*, const int*, void*, int, int, float, float*, long, hipStream_t);
 long dllm_retention_chunk_lds(int);
 int dllm_retention_chunked(const void*, long, int, int, int, int, const float*, int, int, const float*, float*, float,
                            const int*, const int*, const int*, const int*, float*, void*, int, long, int, float, int,
@@ -1529,7 +1530,7 @@ void norm_resadd(torch::Tensor y, torch::Tensor w, double eps, torch::Tensor x, 
 }
 
 void causal_conv_silu(torch::Tensor x, torch::Tensor w, torch::Tensor b, torch::Tensor state, torch::Tensor qstart,
-                      torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor y, bool refill, int64_t act) {
+                      torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor y, bool refill, int64_t act, bool zero) {
   const bool f = act_f32(x, "x");
   TORCH_CHECK(act == 0 || act == 1, "act: 0 (SiLU) or 1 (input plus convolution)");
   check_rows2d(x, "x");
@@ -1546,9 +1547,10 @@ void causal_conv_silu(torch::Tensor x, torch::Tensor w, torch::Tensor b, torch::
               "y [T, C]");
   TORCH_CHECK(y.data_ptr() != x.data_ptr() || (refill && x.stride(0) == C),
               "in place only for steps of single tokens (refill) over exactly the convolved columns");
+  TORCH_CHECK(!zero || y.data_ptr() != x.data_ptr(), "in place rows of no sequence keep their input");
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
   ok(dllm_conv_silu(x.data_ptr(), x.stride(0), f, w.data_ptr<float>(), b.data_ptr<float>(), state.data_ptr(), m.qstart,
-                    m.qlen, m.ctx, m.rows, y.data_ptr(), T, m.S, C, K, (int)refill, (int)act, stream()),
+                    m.qlen, m.ctx, m.rows, y.data_ptr(), T, m.S, C, K, (int)refill, (int)act, zero ? 1 : 0, stream()),
      "causal_conv_silu");
 }
 
@@ -1578,10 +1580,15 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
               "conv_state [slots, K - 1, C]");
   auto m = seq_meta(qstart, qlen, ctx, rows, ssm.size(0));
   const long ns = chunked ? dllm_scan_chunks_scratch(T, m.S, C, N) : 0;
-  const bool step = !chunked && dllm_scan_step_ok(T, m.S, N, ssm.data_ptr(), A.data_ptr());
+  // rows of no sequence become zeros: in the step kernel, else here
+  const auto clear = [&] { ok(dllm_zero_free_rows(out.data_ptr(), f ? 4 : 2, T, C, m.qstart, m.qlen, m.S, stream()), "zero_free_rows"); };
+  const bool step = m.S > 0 && !chunked && dllm_scan_step_ok(T, m.S, N, ssm.data_ptr(), A.data_ptr());
   if (step || (ns > 0 && ns <= (1L << 30))) {      // decode steps, or the chunk-parallel form (prompt portions)
     torch::Tensor sc;
-    if (!step) sc = torch::empty({ns}, xc.options().dtype(torch::kFloat32));
+    if (!step) {
+      clear();
+      sc = torch::empty({ns}, xc.options().dtype(torch::kFloat32));
+    }
     ok(dllm_scan_chunks(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(), dbc.data_ptr(),
                         dbc.stride(0), (int)dt_rank, D.data_ptr<float>(), xz.data_ptr(), xz.stride(0), ssm.data_ptr<float>(),
                         conv.data_ptr(), (int)conv.size(1), m.qstart, m.qlen, m.ctx, m.rows, out.data_ptr(), m.S, (long)T, C, N,
@@ -1589,6 +1596,7 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
        step ? "selective_scan (step)" : "selective_scan (chunked)");
     return;
   }
+  clear();
   ok(dllm_selective_scan(xc.data_ptr(), dt_raw.data_ptr(), f, dt_bias.data_ptr<float>(), A.data_ptr<float>(),
                          dbc.data_ptr(), dbc.stride(0), (int)dt_rank, D.data_ptr<float>(), xz.data_ptr(), xz.stride(0),
                          ssm.data_ptr<float>(), conv.data_ptr(), (int)conv.size(1), m.qstart, m.qlen, m.ctx, m.rows,
@@ -1629,6 +1637,7 @@ void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tens
     TORCH_CHECK(raw->numel() >= (int64_t)T * H * dv, "raw scratch [T, H, dv]");
     const auto sc = chunk_scratch(T, m.S, H, d, dv, qkvg);
     TORCH_CHECK(sc.defined() || dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
+    ok(dllm_zero_free_rows(out.data_ptr(), f ? 4 : 2, T, (int)(H * dv), m.qstart, m.qlen, m.S, stream()), "zero_free_rows");
     ok(dllm_retention_chunked(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, cos_sin.data_ptr<float>(),
                               (int)cos_sin.size(1), (int)rot, decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps,
                               m.qstart, m.qlen, m.ctx, m.rows, raw->data_ptr<float>(), out.data_ptr(), m.S, (long)T, 0,
@@ -1639,7 +1648,7 @@ void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tens
   TORCH_CHECK(dllm_retention_lds((int)d, (int)dv) <= 150 * 1024, "dim x vdim state does not fit the LDS");
   ok(dllm_retention(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, cos_sin.data_ptr<float>(),
                     (int)cos_sin.size(1), (int)rot, decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps, m.qstart,
-                    m.qlen, m.ctx, m.rows, out.data_ptr(), m.S, 0, 1.f / std::sqrt((float)d), nullptr, stream()),
+                    m.qlen, m.ctx, m.rows, out.data_ptr(), m.S, 0, 1.f / std::sqrt((float)d), nullptr, (long)T, stream()),
      "retention");
 }
 
@@ -1676,7 +1685,7 @@ void lightning_attention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, t
     TORCH_CHECK(dllm_retention_lds((int)d, (int)dv) <= 150 * 1024, "dim x vdim state does not fit the LDS");
     ok(dllm_retention(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, decay.data_ptr<float>(), 0, 0,
                       decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps, m.qstart, m.qlen, m.ctx, m.rows,
-                      out.data_ptr(), m.S, 1, 1.f, raw.data_ptr<float>(), stream()),
+                      out.data_ptr(), m.S, 1, 1.f, raw.data_ptr<float>(), (long)qkvg.size(0), stream()),
        "lightning attention");
   }
   ok(dllm_heads_norm_gate(raw.data_ptr<float>(), qkvg.data_ptr(), qkvg.stride(0), f, 2 * H * d + H * dv, (int)(H * dv),
@@ -2163,6 +2172,7 @@ void ssd_scan(torch::Tensor xbc, torch::Tensor proj, int64_t dt_col, int64_t H, 
               "state [slots, H, N, dv]");
   TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == xbc.size(0) && out.size(1) == H * dv, "out [T, H dv] f32");
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
+  ok(dllm_zero_free_rows(out.data_ptr(), 4, xbc.size(0), (int)(H * dv), m.qstart, m.qlen, m.S, stream()), "zero_free_rows");
   const auto sc = chunked ? chunk_scratch(xbc.size(0), m.S, H, N, dv, xbc) : torch::Tensor();
   if (sc.defined()) {
     const char* gates = (const char*)proj.data_ptr() + dt_col * proj.element_size();
@@ -2633,7 +2643,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("qk_norm_prep", &qk_norm_prep);
   m.def("diff_combine", &diff_combine);
   m.def("causal_conv_silu", &causal_conv_silu, py::arg("x"), py::arg("w"), py::arg("b"), py::arg("state"), py::arg("qstart"),
-        py::arg("qlen"), py::arg("ctx"), py::arg("rows"), py::arg("y"), py::arg("refill") = false, py::arg("act") = 0);
+        py::arg("qlen"), py::arg("ctx"), py::arg("rows"), py::arg("y"), py::arg("refill") = false, py::arg("act") = 0, py::arg("zero") = false);
   m.def("selective_scan", &selective_scan);
   m.def("retention", &retention, py::arg("qkvg"), py::arg("heads"), py::arg("dim"), py::arg("vdim"), py::arg("cos_sin"),
         py::arg("rot"), py::arg("decay"), py::arg("state"), py::arg("eps"), py::arg("positions"), py::arg("qstart"),

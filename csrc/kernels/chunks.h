@@ -42,4 +42,27 @@ template <int L> static __device__ __forceinline__ int chunks_before(const int* 
   return n;
 }
 
+// Clear the rows of `out` that belong to no sequence (the tokens a captured step is padded with): a wave asks for one row at a
+// time and writes only those.  part of parts: this workgroup's share, `waves` waves a workgroup.
+template <typename T>
+static __device__ __forceinline__ void zero_free_rows(T* out, long rows, int width, const int* qstart, const int* qlen, int S, long part,
+                                                      long parts, int waves) {
+  const int lane = threadIdx.x & 63;
+  for (long r = part * waves + (threadIdx.x >> 6); r < rows; r += parts * waves) {
+    bool in = false;
+    for (int s0 = lane; s0 < S; s0 += 256) {      // four sequences a lane in flight: a batch's slots cost one round trip
+      int a[4], n[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = qstart[min(s0 + 64 * u, S - 1)];
+        n[u] = qlen[min(s0 + 64 * u, S - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) in |= r >= a[u] && r < (long)a[u] + n[u];
+    }
+    if (__ballot(in)) continue;
+    for (int c = lane; c < width; c += 64) out[r * width + c] = T(0);
+  }
+}
+
 }  // namespace dllm

@@ -72,6 +72,7 @@ template <typename T> struct MambaArgs {
   T* out;
   int S, C, N, nchunks;
   float *ends, *steps;      // [chunks][N][C], [chunks][C]
+  long tokens;
 };
 
 // OUT = false: scan_sum, true: scan_out.  NP >= N states in registers (the padded ones stay zero).
@@ -192,6 +193,10 @@ template <typename T> __global__ void __launch_bounds__(256) scan_carry_kernel(M
 template <typename T, int NP> __global__ void __launch_bounds__(64) scan_step_kernel(MambaArgs<T> a) {
   __shared__ __attribute__((aligned(16))) float bc[2 * NP];
   const int s = blockIdx.y, lane = threadIdx.x;
+  if (s == a.S) {      // one more row of workgroups clears the rows of no sequence
+    dllm::zero_free_rows(a.out, a.tokens, a.C, a.qstart, a.qlen, a.S, blockIdx.x, gridDim.x, 1);
+    return;
+  }
   const int n = a.qlen[s];
   if (n <= 0) return;
   const int c0 = blockIdx.x * 64 + lane, c = c0 < a.C ? c0 : a.C - 1;   // lanes past the last channel shadow it and store nothing
@@ -266,9 +271,9 @@ int run(const void* xc, const void* dt_raw, const float* dt_bias, const float* A
         const float* D, const void* xz, long ldz, float* ssm, void* conv, int Km1, const int* qstart, const int* qlen,
         const int* ctx, const int* rows, void* out, int S, long tokens, int C, int N, float* scratch, hipStream_t st) {
   MambaArgs<T> a{(const T*)xc, (const T*)dt_raw, (const T*)dbc, (const T*)xz, ldd, ldz, dt_rank, dt_bias, A, D, ssm, (T*)conv,
-                 Km1, qstart, qlen, ctx, rows, (T*)out, S, C, N, (int)(tokens / SC_L) + S, scratch, nullptr};
+                 Km1, qstart, qlen, ctx, rows, (T*)out, S, C, N, (int)(tokens / SC_L) + S, scratch, nullptr, tokens};
   if (!scratch) {
-    const dim3 g((C + 63) / 64, S);
+    const dim3 g((C + 63) / 64, S + 1);
     if (N <= 8) hipLaunchKernelGGL((scan_step_kernel<T, 8>), g, dim3(64), 0, st, a);
     else if (N <= 16) hipLaunchKernelGGL((scan_step_kernel<T, 16>), g, dim3(64), 0, st, a);
     else hipLaunchKernelGGL((scan_step_kernel<T, 32>), g, dim3(64), 0, st, a);

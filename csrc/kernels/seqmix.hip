@@ -35,6 +35,7 @@
 // Sequence metadata: qstart / qlen / ctx / rows per sequence (int32); a sequence with qlen 0 is
 // skipped, one whose first new position (ctx - qlen) is 0 starts from a zero state.
 #include "common.h"
+#include "chunks.h"
 
 namespace {
 
@@ -411,9 +412,13 @@ __global__ void __launch_bounds__(256) conv_silu_kernel(const T* x, long ldx, co
                                                         const float* __restrict__ b, const T* state,
                                                         const int* __restrict__ qstart, const int* __restrict__ qlen,
                                                         const int* __restrict__ ctx, const int* __restrict__ rows,
-                                                        T* y, int C, int K, T* refill, int act) {
+                                                        T* y, int C, int K, T* refill, int act, int S, long tokens) {
   // act 0: y = silu(b + conv);  act 1: y = x + b + conv (an input convolution ahead of a mixer)
   const int s = blockIdx.y;
+  if (s == S) {      // one more row of workgroups (where asked for) clears the rows of no sequence
+    dllm::zero_free_rows(y, tokens, C, qstart, qlen, S, blockIdx.x + (long)gridDim.x * blockIdx.z, (long)gridDim.x * gridDim.z, 4);
+    return;
+  }
   const int n = qlen[s];
   if (n <= 0) return;
   const int c = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -727,9 +732,13 @@ __global__ void __launch_bounds__(256, NR <= 8 ? 4 : 3) retention_step_kernel(co
                                                              float eps, const int* __restrict__ qstart,
                                                              const int* __restrict__ qlen, const int* __restrict__ ctx,
                                                              const int* __restrict__ rows, T* __restrict__ out, int lq,
-                                                             int act, float kscale, float* __restrict__ raw) {
+                                                             int act, float kscale, float* __restrict__ raw, int S0, long tokens) {
   __shared__ __attribute__((aligned(16))) float qs[256], ks[256], part[256 * 4];
   const int h = blockIdx.x, s = blockIdx.y;
+  if (s == S0) {      // one more row of workgroups clears the rows of no sequence
+    dllm::zero_free_rows(out, tokens, H * dv, qstart, qlen, S0, blockIdx.x, gridDim.x, 4);
+    return;
+  }
   const int n = qlen[s];
   if (n <= 0) return;
   const int q0 = qstart[s], p0 = ctx[s] - n;
@@ -1417,6 +1426,24 @@ __global__ void __launch_bounds__(256) glu_act_kernel(const T* __restrict__ gu, 
 #define BY_T(f32, call_u16, call_f32) \
   if (f32) { call_f32; } else { call_u16; }
 
+namespace {
+template <typename T>
+__global__ void __launch_bounds__(256) zero_free_rows_kernel(T* __restrict__ out, long rows, int width, const int* __restrict__ qstart,
+                                                             const int* __restrict__ qlen, int S) {
+  dllm::zero_free_rows(out, rows, width, qstart, qlen, S, blockIdx.x, gridDim.x, 4);
+}
+}  // namespace
+
+// Clear the rows of out [rows, width] (esize 2 or 4 bytes) that belong to no sequence: kernels that write their sequences' rows only
+// leave the rest to this.  It writes nothing where every row is some sequence's, where a fill wrote the whole output.
+extern "C" int dllm_zero_free_rows(void* out, int esize, long rows, int width, const int* qstart, const int* qlen, int S, hipStream_t st) {
+  if (rows <= 0 || width <= 0) return 0;
+  const dim3 g((unsigned)((rows + 3) / 4 < 1024 ? (rows + 3) / 4 : 1024));
+  if (esize == 4) hipLaunchKernelGGL(zero_free_rows_kernel<uint32_t>, g, dim3(256), 0, st, (uint32_t*)out, rows, width, qstart, qlen, S);
+  else hipLaunchKernelGGL(zero_free_rows_kernel<u16>, g, dim3(256), 0, st, (u16*)out, rows, width, qstart, qlen, S);
+  return (int)hipGetLastError();
+}
+
 extern "C" int dllm_rms_rows(const void* x, long ldx, int x_f32, const float* w, void* y, long ldy, int y_f32, int rows,
                              int n, float eps, int groups, hipStream_t st) {
   if (rows <= 0 || n <= 0) return rows == 0 ? 0 : -1;
@@ -1556,12 +1583,17 @@ extern "C" int dllm_conv_refill(const void* x, long ldx, int f32, void* conv, in
 // refill != 0: a step of single tokens; the kernel also moves each token's input into its slot
 extern "C" int dllm_conv_silu(const void* x, long ldx, int f32, const float* w, const float* b, void* state,
                               const int* qstart, const int* qlen, const int* ctx, const int* rows, void* y, int T,
-                              int S, int C, int K, int refill, int act, hipStream_t st) {
-  if (T <= 0 || S <= 0) return 0;
+                              int S, int C, int K, int refill, int act, int zero, hipStream_t st) {
+  if (T <= 0) return 0;
+  if (S <= 0) return zero ? dllm_zero_free_rows(y, f32 ? 4 : 2, T, C, qstart, qlen, S, st) : 0;
   if (K < 1 || K > 9) return -1;
   // prompt portions of bf16 rows made of whole, aligned 16-byte vectors: the vector kernel
   if (!f32 && !refill && K <= 5 && T >= 4 * S && C % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 &&
       ((uintptr_t)y % 16) == 0 && ((uintptr_t)state % 16) == 0) {
+    if (zero) {
+      const int rc = dllm_zero_free_rows(y, 2, T, C, qstart, qlen, S, st);
+      if (rc) return rc;
+    }
     int gzv = (T + 4 * CV_RUN - 1) / (4 * CV_RUN);
     if (gzv > 256) gzv = 256;
     const dim3 gv((C / 8 + 63) / 64, S, gzv);
@@ -1580,10 +1612,10 @@ extern "C" int dllm_conv_silu(const void* x, long ldx, int f32, const float* w, 
   }
   int gz = (T + 31) / 32;
   if (gz > 128) gz = 128;
-  const dim3 g((C + 63) / 64, S, gz), blk(256);
+  const dim3 g((C + 63) / 64, S + (zero ? 1 : 0), gz), blk(256);
   BY_T(f32,
-       hipLaunchKernelGGL(conv_silu_kernel<u16>, g, blk, 0, st, (const u16*)x, ldx, w, b, (const u16*)state, qstart, qlen, ctx, rows, (u16*)y, C, K, refill ? (u16*)state : nullptr, act),
-       hipLaunchKernelGGL(conv_silu_kernel<float>, g, blk, 0, st, (const float*)x, ldx, w, b, (const float*)state, qstart, qlen, ctx, rows, (float*)y, C, K, refill ? (float*)state : nullptr, act))
+       hipLaunchKernelGGL(conv_silu_kernel<u16>, g, blk, 0, st, (const u16*)x, ldx, w, b, (const u16*)state, qstart, qlen, ctx, rows, (u16*)y, C, K, refill ? (u16*)state : nullptr, act, S, (long)T),
+       hipLaunchKernelGGL(conv_silu_kernel<float>, g, blk, 0, st, (const float*)x, ldx, w, b, (const float*)state, qstart, qlen, ctx, rows, (float*)y, C, K, refill ? (float*)state : nullptr, act, S, (long)T))
   return (int)hipGetLastError();
 }
 
@@ -1623,9 +1655,9 @@ extern "C" long dllm_retention_lds(int d, int dv) {
 
 extern "C" int dllm_retention(const void* qkvg, long ld, int f32, int H, int d, int dv, const float* cos_sin, int tab_w,
                               int rot, const float* decay, float* state, float eps, const int* qstart, const int* qlen,
-                              const int* ctx, const int* rows, void* out, int S, int act, float kscale, float* raw,
+                              const int* ctx, const int* rows, void* out, int S, int act, float kscale, float* raw, long T_,
                               hipStream_t st) {
-  if (S <= 0) return 0;
+  if (S <= 0) return raw ? 0 : dllm_zero_free_rows(out, f32 ? 4 : 2, T_, H * dv, qstart, qlen, S, st);
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w) return -1;
   const long lds = dllm_retention_lds(d, dv);
   if (lds > 150 * 1024) return -2;
@@ -1636,9 +1668,10 @@ extern "C" int dllm_retention(const void* qkvg, long ld, int f32, int H, int d, 
   while (4 << lq < dv) ++lq;
   const int nr = (d + (256 >> lq) - 1) / (256 >> lq);      // key rows a thread of the register form holds
   if (dv % 4 == 0 && dv <= 256 && d <= 256 && nr <= 16 && ((uintptr_t)state & 15) == 0) {
+    const dim3 gs(H, S + (raw ? 0 : 1));      // raw: the finish kernel writes every row
 #define RSTEP(T, NR)                                                                                                              \
-  hipLaunchKernelGGL((retention_step_kernel<T, NR>), g, dim3(256), 0, st, (const T*)qkvg, ld, H, d, dv, cos_sin, tab_w, rot, decay, \
-                     state, eps, qstart, qlen, ctx, rows, (T*)out, lq, act, kscale, raw)
+  hipLaunchKernelGGL((retention_step_kernel<T, NR>), gs, dim3(256), 0, st, (const T*)qkvg, ld, H, d, dv, cos_sin, tab_w, rot, decay, \
+                     state, eps, qstart, qlen, ctx, rows, (T*)out, lq, act, kscale, raw, S, T_)
 #define RSTEP2(T)                    \
   do {                               \
     if (nr <= 4) RSTEP(T, 4);        \
@@ -1649,6 +1682,10 @@ extern "C" int dllm_retention(const void* qkvg, long ld, int f32, int H, int d, 
 #undef RSTEP2
 #undef RSTEP
     return (int)hipGetLastError();
+  }
+  if (!raw) {
+    const int rc = dllm_zero_free_rows(out, f32 ? 4 : 2, T_, H * dv, qstart, qlen, S, st);
+    if (rc) return rc;
   }
   if (f32) {
     ENSURE_LDS(retention_kernel<float>, lds);

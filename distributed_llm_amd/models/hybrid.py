@@ -680,7 +680,8 @@ class HybridModel:
         conv_state, ssm_state = cache
         rows = meta.state_rows
         xz = _mm(x, L["in"])
-        xc = seqmix.causal_conv_silu(xz, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
+        xc = seqmix.causal_conv_silu(xz, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
+                                     all_rows=self._all_rows(xz, meta))
         dbc = _mm(xc, L["x"])
         dt_raw = _mm(dbc[:, :m.dt_rank], L["dt"])
         y = seqmix.selective_scan(xc, dt_raw, L["dt_b"], L["A"], dbc, m.dt_rank, L["D"], xz, ssm_state, conv_state,
@@ -753,7 +754,7 @@ class HybridModel:
         proj = _mm(x, L["proj"])                                        # q | k | v | gate | beta | decay logits
         single = meta.host_qlen is None      # a decode step: the convolution refills its slots itself
         qkv = seqmix.causal_conv_silu(proj, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
-                                      refill=single)
+                                      refill=single, all_rows=self._all_rows(proj, meta))
         if not single:
             seqmix.conv_state_refill(proj, conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
         o = seqmix.delta_rule(qkv, proj[:, c:], m.heads, m.kv_heads, m.dim, m.vdim, L["neg_a"], L["dt_b"], L["hnorm"],
@@ -946,7 +947,7 @@ class HybridModel:
         xbc_in = proj[:, inner:]
         single = meta.host_qlen is None      # a decode step: the convolution refills its slots itself
         xbc = seqmix.causal_conv_silu(xbc_in, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
-                                      refill=single)
+                                      refill=single, all_rows=self._all_rows(xbc_in, meta))
         if not single:
             seqmix.conv_state_refill(xbc_in, conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
         y = seqmix.ssd_scan(xbc, proj, 2 * inner + 2 * m.groups * m.state, m.heads, m.vdim, m.state, m.groups, L["dt_b"],

@@ -74,11 +74,11 @@ def causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, refill: bool 
             ref.conv_state_refill(x, conv_state, qstart, qlen, ctx, rows)
         return y
     if inplace and refill and x.is_contiguous() and x.shape[1] == w.shape[0]:
-        ext.causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, x, True, 0 if act == "silu" else 1)
+        ext.causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, x, True, 0 if act == "silu" else 1, False)
         return x
-    # rows of no sequence (graph padding) stay zero, never stale memory
-    y = (torch.empty if all_rows else torch.zeros)((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
-    ext.causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, y, bool(refill), 0 if act == "silu" else 1)
+    # rows of no sequence (graph padding) become zeros, never stale memory
+    y = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+    ext.causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, y, bool(refill), 0 if act == "silu" else 1, not all_rows)
     return y
 
 
@@ -98,7 +98,7 @@ def selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_
     if ext is None:
         return ref.selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_state, qstart, qlen,
                                   ctx, rows)
-    out = torch.zeros_like(xc)
+    out = torch.empty_like(xc)      # rows of no sequence become zeros
     if chunked is None:
         chunked = xc.shape[0] >= SCAN_CHUNK_MIN * qstart.numel()
     ext.selective_scan(xc, dt_raw, dt_bias, A, dbc, int(dt_rank), D, xz, ssm_state, conv_state, qstart, qlen, ctx,
@@ -128,7 +128,7 @@ def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, posi
     if ext is None:
         return ref.retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen,
                              ctx, rows)
-    out = torch.zeros((qkvg.shape[0], heads * vdim), dtype=qkvg.dtype, device=qkvg.device)
+    out = torch.empty((qkvg.shape[0], heads * vdim), dtype=qkvg.dtype, device=qkvg.device)      # rows of no sequence become zeros
     if chunked is None:
         chunked = qkvg.shape[0] >= RETENTION_CHUNK_MIN * qstart.numel()
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
@@ -465,7 +465,7 @@ def ssd_scan(xbc, proj, dt_col, heads, vdim, n_state, groups, dt_bias, neg_a, D,
     if ext is None:
         return ref.ssd_scan(xbc, proj, dt_col, heads, vdim, n_state, groups, dt_bias, neg_a, D, state, qstart, qlen, ctx,
                             rows)
-    out = torch.zeros((xbc.shape[0], heads * vdim), dtype=torch.float32, device=xbc.device)
+    out = torch.empty((xbc.shape[0], heads * vdim), dtype=torch.float32, device=xbc.device)      # rows of no sequence become zeros
     if chunked is None:
         chunked = xbc.shape[0] >= SSD_CHUNK_MIN * qstart.numel()
     ext.ssd_scan(xbc, proj, int(dt_col), int(heads), int(vdim), int(n_state), int(groups), dt_bias, neg_a, D, state,

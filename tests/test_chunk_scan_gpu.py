@@ -263,3 +263,48 @@ def test_scan_steps(dt, case, C, N, R, K):
     close(got, want * F.silu(xz[:, C:2 * C].double()), 4e-6 if dt == torch.float32 else 4e-3)
     close(st, s64, 4e-6)
     assert torch.equal(cv, c2)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 3, 70])
+@pytest.mark.parametrize("S", [0, 3, 130])
+def test_rows_of_no_sequence_are_zero(dt, n, S):
+    """Padding ahead of, between and behind the sequences, in the forms of a step, of few tokens and of chunks; stale memory under the
+    outputs is NaN.  S = 0: every row is padding."""
+    torch.manual_seed(38)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    T = S * (n + 1) + 5
+    qs, ql = i32([2 + s * (n + 1) for s in range(S)]), i32([n if s % 3 else 0 for s in range(S)])
+    cx, rw = ql + 4, i32(list(range(S)))
+    live = torch.zeros(T, dtype=torch.bool, device=DEV)
+    for a, m in zip(qs.tolist(), ql.tolist()):
+        live[a:a + m] = True
+
+    def check(f):
+        for w in (T * 70, T * 64, T * 256):          # blocks of these sizes come back from the allocator
+            for t in (torch.float32, torch.bfloat16):
+                x = torch.full((w,), float("nan"), device=DEV, dtype=t)
+                del x
+        y = f()
+        assert torch.isfinite(y).all() and not y[~live].any()
+        if S > 1:
+            assert y[live].any()
+
+    H, d, dv, C, N = 2, 16, 32, 64, 16
+    x = torch.randn(T, 2 * H * (d + dv), device=DEV).to(dt)
+    table, dec = ops.rope_cos_sin(512, 16, 10000.0, DEV), torch.full((H,), 0.9, device=DEV)
+    st = torch.randn(max(S, 1), H, d, dv, device=DEV)
+    pos = torch.zeros(T, dtype=torch.int32, device=DEV)
+    for c in (False, True):
+        check(lambda: seqmix.retention(x, H, d, dv, table, 16, dec, st, 1e-6, pos, qs, ql, cx, rw, chunked=c))
+    xc, dbc, xz = torch.randn(T, C, device=DEV).to(dt), torch.randn(T, 2 * N, device=DEV).to(dt), torch.randn(T, 2 * C, device=DEV).to(dt)
+    A, v, ss = -torch.rand(C, N, device=DEV), torch.zeros(C, device=DEV), torch.zeros(max(S, 1), C, N, device=DEV)
+    cv = torch.zeros(max(S, 1), 3, C, device=DEV).to(dt)
+    for c in (False, True):
+        check(lambda: seqmix.selective_scan(xc, xc, v, A, dbc, 0, v + 1, xz, ss, cv, qs, ql, cx, rw, chunked=c))
+        sd, pr = torch.zeros(max(S, 1), H, N, 32, device=DEV), torch.randn(T, H, device=DEV).to(dt)
+        check(lambda: seqmix.ssd_scan(torch.cat([xc, dbc], 1), pr, 0, H, 32, N, 1, dec, -dec, dec, sd, qs, ql, cx, rw, chunked=c))
+    w = torch.randn(C, 4, device=DEV)
+    check(lambda: seqmix.causal_conv_silu(xc, w, v, cv, qs, ql, cx, rw))
+    if n == 1:
+        check(lambda: seqmix.causal_conv_silu(xc, w, v, cv, qs, ql, cx, rw, refill=True))
