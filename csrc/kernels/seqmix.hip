@@ -66,6 +66,52 @@ __global__ void __launch_bounds__(256) rms_rows_kernel(const TI* __restrict__ x,
   for (int i = lane; i < n; i += 64) stf(yr + i, ldf(xr + i) * r * (w ? w[c0 + i] : 1.f));
 }
 
+// The same on whole, aligned vectors (parts of up to 256 NV entries): the part in its wave's registers, row and weights read once, side
+// by side.  Bound by one load's latency at decode: 24 rows of 1024 4.7 us against 12.4 element by element, twice.
+template <typename TI, typename TO, int NV>
+__global__ void __launch_bounds__(256) rms_rows_vec_kernel(const TI* __restrict__ x, long ldx, const float* __restrict__ w,
+                                                           TO* __restrict__ y, long ldy, int rows, int n, float eps, int groups) {
+  typedef TI vi_t __attribute__((ext_vector_type(4)));
+  typedef TO vo_t __attribute__((ext_vector_type(4)));
+  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (unit >= rows * groups) return;
+  const int row = unit / groups, c0 = (unit % groups) * n;
+  const TI* xr = x + (long)row * ldx + c0;
+  vi_t r[NV];
+  f32x4 g[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int c = 4 * lane + 256 * v;
+    r[v] = c < n ? *reinterpret_cast<const vi_t*>(xr + c) : vi_t(TI(0));
+    g[v] = w && c < n ? *reinterpret_cast<const f32x4*>(w + c0 + c) : f32x4{1.f, 1.f, 1.f, 1.f};
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const TI q = r[v][e];
+      const float f = ldf(&q);
+      s += f * f;
+    }
+  const float rs = 1.f / sqrtf(wave_sum(s) / (float)n + eps);
+  TO* yr = y + (long)row * ldy + c0;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int c = 4 * lane + 256 * v;
+    if (c >= n) continue;
+    vo_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const TI q = r[v][e];
+      TO z;
+      stf(&z, ldf(&q) * rs * g[v][e]);
+      o[e] = z;
+    }
+    *reinterpret_cast<vo_t*>(yr + c) = o;
+  }
+}
+
 // ---------------------------------------------------------------- norm_resadd
 template <typename T>
 __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ y, long ldy, const float* __restrict__ w,
@@ -1444,21 +1490,31 @@ extern "C" int dllm_zero_free_rows(void* out, int esize, long rows, int width, c
   return (int)hipGetLastError();
 }
 
+namespace {
+template <typename TI, typename TO>
+int rms_rows(const void* x, long ldx, const float* w, void* y, long ldy, int rows, int n, float eps, int groups, hipStream_t st) {
+  const dim3 g((rows * groups + 3) / 4), b(256);
+  const auto al = [](const void* p, size_t by) { return ((uintptr_t)p & (by - 1)) == 0; };
+  if (n % 4 == 0 && n <= 4096 && ldx % 4 == 0 && ldy % 4 == 0 && al(x, 4 * sizeof(TI)) && al(y, 4 * sizeof(TO)) && al(w, 16)) {
+#define RMSV(NV) hipLaunchKernelGGL((rms_rows_vec_kernel<TI, TO, NV>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups)
+    if (n <= 256) RMSV(1); else if (n <= 512) RMSV(2); else if (n <= 1024) RMSV(4); else if (n <= 2048) RMSV(8); else RMSV(16);
+#undef RMSV
+  } else {
+    hipLaunchKernelGGL((rms_rows_kernel<TI, TO>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups);
+  }
+  return (int)hipGetLastError();
+}
+}  // namespace
+
 extern "C" int dllm_rms_rows(const void* x, long ldx, int x_f32, const float* w, void* y, long ldy, int y_f32, int rows,
                              int n, float eps, int groups, hipStream_t st) {
   if (rows <= 0 || n <= 0) return rows == 0 ? 0 : -1;
   if (groups < 1 || n % groups) return -1;
   n /= groups;     // the kernel's rows are the parts
-  const dim3 g((rows * groups + 3) / 4), b(256);
-  if (x_f32 && y_f32)
-    hipLaunchKernelGGL((rms_rows_kernel<float, float>), g, b, 0, st, (const float*)x, ldx, w, (float*)y, ldy, rows, n, eps, groups);
-  else if (x_f32)
-    hipLaunchKernelGGL((rms_rows_kernel<float, u16>), g, b, 0, st, (const float*)x, ldx, w, (u16*)y, ldy, rows, n, eps, groups);
-  else if (y_f32)
-    hipLaunchKernelGGL((rms_rows_kernel<u16, float>), g, b, 0, st, (const u16*)x, ldx, w, (float*)y, ldy, rows, n, eps, groups);
-  else
-    hipLaunchKernelGGL((rms_rows_kernel<u16, u16>), g, b, 0, st, (const u16*)x, ldx, w, (u16*)y, ldy, rows, n, eps, groups);
-  return (int)hipGetLastError();
+  if (x_f32 && y_f32) return rms_rows<float, float>(x, ldx, w, y, ldy, rows, n, eps, groups, st);
+  if (x_f32) return rms_rows<float, u16>(x, ldx, w, y, ldy, rows, n, eps, groups, st);
+  if (y_f32) return rms_rows<u16, float>(x, ldx, w, y, ldy, rows, n, eps, groups, st);
+  return rms_rows<u16, u16>(x, ldx, w, y, ldy, rows, n, eps, groups, st);
 }
 
 namespace {

@@ -161,3 +161,20 @@ def test_norm_router_and_residual_combine(T, H, E, top):
         na = ops.moe_ffn_tg_resadd(x, ids, w, w13, w2d, ra, qa)
         nb = ops.gemm.res_add_ssq(ops.moe_ffn_tg(x, ids, w, w13, w2d), rb, qb)
         assert na == nb and torch.equal(ra, rb) and torch.equal(qa, qb)
+
+
+@pytest.mark.parametrize("ti", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("to", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,n,groups,pad", [(24, 1024, 1, 0), (5, 256, 1, 8), (3, 260, 1, 4), (7, 4, 1, 0), (2, 4096, 1, 0), (2, 4100, 1, 0), (3, 2048, 4, 0), (3, 70, 1, 0),
+                                            (3, 768, 3, 1), (1, 1536, 1, 0)])
+@pytest.mark.parametrize("weight", [False, True])
+def test_rms_rows_widths(ti, to, T, n, groups, pad, weight):
+    """Parts in registers: 1 to 16 vectors a lane, full and not; unaligned rows, odd widths and parts past 4096 take the other form."""
+    torch.manual_seed(n)
+    x = torch.randn(T, n + pad, device=DEV).to(ti)[:, :n]
+    w = torch.randn(n, device=DEV) if weight else None
+    z = x.double().reshape(T, groups, -1)
+    want = (z * torch.rsqrt(z.pow(2).mean(-1, keepdim=True) + 1e-6)).reshape(T, n) * (w.double() if weight else 1)
+    got = seqmix.rms_rows(x, w, 1e-6, to, groups)
+    # one rounding to the output's type (f32: the sum's and the root's few units of 2^-24 beside it)
+    assert float((got.double() - want).norm() / want.norm()) < (1e-6 if to == torch.float32 else 2 ** -9)
