@@ -246,6 +246,17 @@ def prefill_bucket(M: int) -> int:
     return PREFILL_MS[-1] if PREFILL_MS else M
 
 
+def next_batch_size(M: int) -> int:
+    """The smallest decode batch size the engine times plans for (1, 2, 4, 8, 16, 32, 48, 64, then every 32 to 256, then every 64)
+    that holds M rows.  A prompt of 57 tokens on TinyLlama: 1.37 ms of layer products with the plans
+    of 64 rows against 1.58 with the untimed rule of ``tg_plan``."""
+    for b in (1, 2, 4, 8, 16, 32, 48, 64):
+        if M <= b:
+            return b
+    step = 32 if M <= 256 else 64
+    return -(-M // step) * step
+
+
 def tg_plan(M: int, N: int, K: int) -> Tuple[int, ...]:
     """(bm, bn, stages, splits, ks, waves[, k-groups]) of the fused GEMM for this shape: tuned, else a
     heuristic sized so the grid covers the 256 CUs (bigger tiles first, split-K only for short
@@ -253,6 +264,8 @@ def tg_plan(M: int, N: int, K: int) -> Tuple[int, ...]:
     p = _P.tg_plans.get((M, N, K))
     if p is None and M > MAX_M and PREFILL_MS:
         p = _P.tg_plans.get((prefill_bucket(M), N, K))
+    if p is None and M <= MAX_M:      # rows between two timed batch sizes (a short prompt): what was timed for the next one
+        p = _P.tg_plans.get((next_batch_size(M), N, K))
     if p is not None:
         return tuple(p) + (1, 4)[len(p) - 4:] if len(p) < 6 else tuple(p)
     mt128, nt128 = -(-M // 128), -(-N // 128)

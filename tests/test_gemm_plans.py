@@ -47,3 +47,15 @@ def test_gemv_long_rows(N, K, R):
     ops._native(x).gemv(x, w, y, R, False)
     want = x.double() @ w.double().t()
     assert float((y.double() - want).norm() / want.norm()) < 2 ** -8       # one rounding to bf16, f32 sums far below
+
+
+def test_rows_between_batch_sizes_take_the_next_ones_plan(monkeypatch):
+    from distributed_llm_amd.engine.llm_engine import decode_buckets
+    ladder = decode_buckets(1024)
+    assert all(G.next_batch_size(m) == next(b for b in ladder if b >= m) for m in range(1, 1025))
+    timed = {(64, 256, 512): (64, 64, 3, 4, 2, 4), (96, 256, 512): (64, 128, 3, 2, 1, 4)}
+    monkeypatch.setattr(G._P, "tg_plans", timed)
+    assert G.tg_plan(57, 256, 512) == G.tg_plan(64, 256, 512) == (64, 64, 3, 4, 2, 4)
+    assert G.tg_plan(65, 256, 512) == (64, 128, 3, 2, 1, 4)
+    assert G.tg_plan(97, 256, 512)[:3] == G.tg_plan(48, 256, 512)[:3] == (64, 64, 3)      # no plan at 128 or 48 rows: the untimed rule
+    assert G.tg_slots(57, 256, 512) == 4 and G.tg_slots(70, 256, 512) == 2
