@@ -43,7 +43,7 @@ int dllm_sample_split_kmax();
 int dllm_skinny_epi(const void*, long, const void*, int, void*, long, int, int, int, int, int, int, float*, int*, void*,
                     long, float*, long, const float*, int, long, float, float, const int*, const float*, const int*,
                     void*, void*, void*, int, int, int, hipStream_t);
-int dllm_skinny_gemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, float*, int*,
+int dllm_skinny_gemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*,
                      hipStream_t);
 int dllm_moe_max_tiles(int, int);
 int dllm_moe_ffn(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int, int*,
@@ -702,7 +702,7 @@ void cache_write(std::vector<int64_t> srcs, std::vector<int64_t> slots, std::vec
 }
 // y[M, N] = x[M, K] . w[N, K]^T   (swiglu: x is [M, 2K] gate|up, silu(gate)*up computed on load)
 void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw, int64_t splits, bool swiglu,
-                 torch::Tensor part, torch::Tensor counters) {
+                 torch::Tensor part, torch::Tensor counters, int64_t vs) {
   check_bf16(x, "x");
   check_bf16(w, "w");
   check_bf16(y, "y");
@@ -716,6 +716,8 @@ void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw,
   TORCH_CHECK(y.size(0) == M && y.size(1) == N, "y shape");
   TORCH_CHECK(M >= 1 && M <= 128 && K % 32 == 0, "M in [1,128], K % 32 == 0");
   TORCH_CHECK(ntw == 1 || ntw == 2 || ntw == 4, "ntw in {1,2,4}");
+  TORCH_CHECK(vs == 1 || (!swiglu && ((vs == 4 && ntw == 1 && M <= 32) || (vs == 2 && ntw == 2 && M <= 64))),
+              "splits of a workgroup: 1, four of 16 columns (32 rows), two of 32 (64 rows)");
   // slab rows = the kernel's row-tile height (MT x 16, MT in {1, 2, 4, 8}), not ceil(M / 16) x 16
   const int nc = 16 * ntw, tiles = (N + nc - 1) / nc,
             mp = 16 * (M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8);
@@ -723,7 +725,7 @@ void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw,
     TORCH_CHECK(part.numel() >= (int64_t)splits * tiles * nc * mp, "split-K workspace too small");
     TORCH_CHECK(counters.numel() >= tiles, "counter buffer too small");
   }
-  ok(dllm_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), y.stride(0), M, N, K, ntw, splits, swiglu ? 1 : 0,
+  ok(dllm_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), y.stride(0), M, N, K, ntw, splits, (int)vs, swiglu ? 1 : 0,
         part.data_ptr<float>(), counters.data_ptr<int>(), stream()),
      "skinny_gemm");
 }
@@ -965,11 +967,11 @@ int64_t moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch:
     check_f32(*xs, "xs");
     TORCH_CHECK(norm_w.has_value() && xs->dim() == 2 && xs->is_contiguous() && xs->size(0) == T && xs->size(1) == H, "xs [T, H]");
     check_f32(*norm_w, "norm weight");
-    TORCH_CHECK(norm_w->numel() == H && groups >= 1 && dllm_moe_tail_ok((int)H, (int)groups), "norm weight [H], parts of whole 256s");
-    TORCH_CHECK(((uintptr_t)xs->data_ptr() | (uintptr_t)norm_w->data_ptr()) % 16 == 0, "xs / norm weight 16-B aligned");
+    TORCH_CHECK(norm_w->is_contiguous() && norm_w->numel() == H && groups >= 1 && dllm_moe_tail_ok((int)H, (int)groups),
+                "norm weight [H], a width the launch takes");
     if (xl) {
       check_bf16(*xl, "xl");
-      TORCH_CHECK(xl->is_contiguous() && xl->sizes() == xs->sizes() && (uintptr_t)xl->data_ptr() % 8 == 0, "xl [T, H]");
+      TORCH_CHECK(xl->is_contiguous() && xl->sizes() == xs->sizes(), "xl [T, H]");
     }
   } else if (res) {   // the sum is added to the bf16 stream, squares per row and slice in ssq; returns the slices
     check_bf16(*res, "res");
@@ -2746,7 +2748,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("cosine_scores", &cosine_scores);
   m.def("cache_scan", &cache_scan);
   m.def("cache_write", &cache_write);
-  m.def("skinny_gemm", &skinny_gemm);
+  m.def("skinny_gemm", &skinny_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("ntw"), py::arg("splits"), py::arg("swiglu"),
+        py::arg("part"), py::arg("counters"), py::arg("vs") = 1);
   m.def("skinny_epi", &skinny_epi);
   m.def("gemv", &gemv);
   m.def("gemv_norm", &gemv_norm);

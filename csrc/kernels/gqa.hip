@@ -17,7 +17,7 @@
 //               sum (one V read feeds four rows).  The output is multiplied by sigmoid(gate).
 //
 //   gqa_f32     the f32 form on the f32 matrix cores: a wave per 16-key page, no LDS until the waves of a
-//               workgroup meet (whole pages of 16 keys, widths up to 128; paged_gqa takes the rest).
+//               workgroup meet (whole pages of 16 keys, widths up to 128, a value head per key head; paged_gqa takes the rest).
 //
 //   paged_gqa_mfma  the bf16 form on the matrix cores: 64 rows per workgroup, 16 per wave, so a row's
 //               softmax never leaves its wave.  Q stays in registers as MFMA operands; a 64-key tile is
@@ -508,7 +508,7 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
                                                           const int* __restrict__ ctx, const int* __restrict__ tile_seq,
                                                           const int* __restrict__ tile_tok0, const float* __restrict__ gate,
                                                           long ldg, float* __restrict__ out, int H, int G, int d, int dv, int TQ,
-                                                          int win, int GV, int keep, float sink, int chunk, float cap,
+                                                          int win, int keep, float sink, int chunk, float cap,
                                                           const float* __restrict__ sinks, long ldo,
                                                           const float* __restrict__ slopes, int ghead) {
   __shared__ __attribute__((aligned(16))) f32x4 Om[NW / 2][VB * 64];
@@ -536,13 +536,12 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
   }
   const int last = p0 + tok0 + nq - 1, first = oldest_key(p0 + tok0, win, chunk);   // the newest and oldest key any row sees
   const int* btr = bt + (long)s * bt_ld;
-  const int gv = g / (G / GV);
   f32x4 kf[KB], vf[VB], kn[KB], vn[VB];
   auto fetch = [&](int k0, f32x4 (&k)[KB], f32x4 (&v)[VB]) {   // places past the widths are read at 0: q is 0 there, O is dropped
     const long blk = btr[k0 / BSZ];
     const int off = k0 % BSZ;
     const float* kp = kc + ((blk * G + g) * BSZ + off + lr) * d;
-    const float* vp = vc + (blk * GV + gv) * dv * BSZ + off + 4 * g4;
+    const float* vp = vc + (blk * G + g) * dv * BSZ + off + 4 * g4;
 #pragma unroll
     for (int b = 0; b < KB; ++b) k[b] = *reinterpret_cast<const f32x4*>(kp + (16 * b + 4 * g4 < d ? 16 * b + 4 * g4 : 0));
 #pragma unroll
@@ -1117,15 +1116,16 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
     }
     return (int)hipGetLastError();
   }
-  // f32, whole pages of 16 keys, key and query rows of whole 16-byte vectors: the matrix cores
-  if (f32 && BSZ % 16 == 0 && d % 4 == 0 && d <= 128 && dv <= 128 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0) {
+  // f32, whole pages of 16 keys, key and query rows of whole 16-byte vectors: the matrix cores.  Not where key heads share their
+  // values: those are the maps of differential attention, whose difference keeps the order of sums of paged_gqa
+  if (f32 && GV == G && BSZ % 16 == 0 && d % 4 == 0 && d <= 128 && dv <= 128 && (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15) == 0) {
     const dim3 g3(n_tiles, G, (H / G + GA_ROWS - 1) / GA_ROWS);
     const int tq = dllm_gqa_tile_tokens(H, G, 0);
     const bool wide = (long)g3.x * g3.y * g3.z <= GQF_WIDE;
 #define GQF2(KB, VB, NW)                                                                                                     \
   hipLaunchKernelGGL((gqa_f32_kernel<KB, VB, NW>), g3, dim3(64 * NW), 0, st, (const float*)q, (const float*)kc, (const float*)vc, bt, \
                      bt_ld, BSZ, qstart, qlen, ctx, tile_seq, tile_tok0, (const float*)gate, ldg, (float*)out, H, G, d, dv, tq, win,  \
-                     GV, keep, sink, chunk, cap, sinks, ldo, slopes, ghead)
+                     keep, sink, chunk, cap, sinks, ldo, slopes, ghead)
 #define GQF(KB, VB)                        \
   do {                                     \
     if (wide) GQF2(KB, VB, 8);             \

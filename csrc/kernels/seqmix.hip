@@ -66,50 +66,35 @@ __global__ void __launch_bounds__(256) rms_rows_kernel(const TI* __restrict__ x,
   for (int i = lane; i < n; i += 64) stf(yr + i, ldf(xr + i) * r * (w ? w[c0 + i] : 1.f));
 }
 
-// The same on whole, aligned vectors (parts of up to 256 NV entries): the part in its wave's registers, row and weights read once, side
-// by side.  Bound by one load's latency at decode: 24 rows of 1024 4.7 us against 12.4 element by element, twice.
-template <typename TI, typename TO, int NV>
-__global__ void __launch_bounds__(256) rms_rows_vec_kernel(const TI* __restrict__ x, long ldx, const float* __restrict__ w,
+// The same, bit for bit, with the part in its wave's registers: the same entries a lane and the same order of the sum, but every load
+// of the row and its weights in flight at once.  Bound by one load's latency at decode: 24 rows of 1024
+// 3.5 us against 6.6 in two passes; 8000 rows 9.0 against 11.2.
+template <typename TI, typename TO, int NE>
+__global__ void __launch_bounds__(256) rms_rows_reg_kernel(const TI* __restrict__ x, long ldx, const float* __restrict__ w,
                                                            TO* __restrict__ y, long ldy, int rows, int n, float eps, int groups) {
-  typedef TI vi_t __attribute__((ext_vector_type(4)));
-  typedef TO vo_t __attribute__((ext_vector_type(4)));
   const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (unit >= rows * groups) return;
   const int row = unit / groups, c0 = (unit % groups) * n;
   const TI* xr = x + (long)row * ldx + c0;
-  vi_t r[NV];
-  f32x4 g[NV];
+  TI v[NE];
+  float g[NE];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int c = 4 * lane + 256 * v;
-    r[v] = c < n ? *reinterpret_cast<const vi_t*>(xr + c) : vi_t(TI(0));
-    g[v] = w && c < n ? *reinterpret_cast<const f32x4*>(w + c0 + c) : f32x4{1.f, 1.f, 1.f, 1.f};
+  for (int j = 0; j < NE; ++j) {   // entries past the part are read at its last and dropped
+    const int i = min(lane + 64 * j, n - 1);
+    v[j] = xr[i];
+    g[j] = w ? w[c0 + i] : 1.f;
   }
   float s = 0.f;
 #pragma unroll
-  for (int v = 0; v < NV; ++v)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const TI q = r[v][e];
-      const float f = ldf(&q);
-      s += f * f;
-    }
-  const float rs = 1.f / sqrtf(wave_sum(s) / (float)n + eps);
+  for (int j = 0; j < NE; ++j) {
+    const float f = lane + 64 * j < n ? ldf(&v[j]) : 0.f;
+    s = fmaf(f, f, s);     // as the loop's sum is contracted
+  }
+  const float r = 1.f / sqrtf(wave_sum(s) / (float)n + eps);
   TO* yr = y + (long)row * ldy + c0;
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int c = 4 * lane + 256 * v;
-    if (c >= n) continue;
-    vo_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const TI q = r[v][e];
-      TO z;
-      stf(&z, ldf(&q) * rs * g[v][e]);
-      o[e] = z;
-    }
-    *reinterpret_cast<vo_t*>(yr + c) = o;
-  }
+  for (int j = 0; j < NE; ++j)
+    if (lane + 64 * j < n) stf(yr + lane + 64 * j, ldf(&v[j]) * r * g[j]);
 }
 
 // ---------------------------------------------------------------- norm_resadd
@@ -146,81 +131,78 @@ __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ 
   }
 }
 
-// The same on whole, aligned vectors: a row in the registers of its workgroup, four neighbours a thread, the stream and the weights
-// loaded beside y, one barrier.  A wave's 256 columns lie in one part (groups 1, or parts of whole 256s).  k > 0: y is the
-// weighted sum of a token's k expert rows (expert-sorted, TY), in the launch that uses it.  Bound by latency at decode: 24 rows of
-// 1024 4.6 us against 5.6 element by element with the stream read behind the sum; with the experts' sum 5.5 against 10.5 in two
-// launches.
-template <typename T, typename TY, int NV>
-__global__ void __launch_bounds__(256) norm_resadd_vec_kernel(const TY* __restrict__ y, long ldy, const float* __restrict__ w,
+// The same, bit for bit, with the row in registers: the same entries a thread (a lane, of parts) and the same order of the sum, but
+// the stream and the weights travel beside y and the row is read once.  k > 0: y is the weighted sum of a token's k expert rows
+// (expert-sorted, TY), in the launch that uses it; a sum of bf16 rows is rounded to bf16 first, as the combine of its own
+// writes it.  Bound by latency at decode: 24 rows of 1024 2.9 us against 3.4 in two passes (of 4096
+// 4.2 against 6.8), 8000 rows 17.5 against 21.2; with the experts' sum 0.9 us more than the combine whose place it takes.
+template <typename T, typename TY, int NE, bool PARTS>
+__global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restrict__ y, long ldy, const float* __restrict__ w,
                                                               float* __restrict__ x, T* __restrict__ xl, int H, float eps,
                                                               int groups, const float* __restrict__ bias,
                                                               const int* __restrict__ inv, const float* __restrict__ wts, int k) {
-  __shared__ float red[4 * NV];
-  typedef T vec_t __attribute__((ext_vector_type(4)));
-  typedef TY vecy_t __attribute__((ext_vector_type(4)));
+  __shared__ float red[4];
+  constexpr bool EARLY = NE <= 16;     // the stream and the weights in flight with the row, where the registers allow
+  constexpr int ST = PARTS ? 64 : 256;
   const long row = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  f32x4 a[NV], s[NV], g[NV];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, u = PARTS ? lane : (int)threadIdx.x;
+  const int n = H / groups;
+  float* xr = x + row * (long)H;
+  for (int p = PARTS ? wave : 0; p < groups; p += 4) {
+    const int c0 = p * n + u, c1 = p * n + n;     // this thread's entries: c0 + ST j below c1
+    float a[NE], s[EARLY ? NE : 1], g[EARLY ? NE : 1];
+    if constexpr (EARLY) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int c = 4 * tid + 1024 * v;
-    const bool in = c < H;
-    s[v] = in ? *reinterpret_cast<const f32x4*>(x + row * H + c) : f32x4{0.f, 0.f, 0.f, 0.f};
-    g[v] = in ? *reinterpret_cast<const f32x4*>(w + c) : f32x4{0.f, 0.f, 0.f, 0.f};
-    a[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (in && k == 0) {
-      const vecy_t r = *reinterpret_cast<const vecy_t*>(y + row * ldy + c);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const TY q = r[e];
-        a[v][e] = ldf(&q);
-      }
-      if (bias) a[v] += *reinterpret_cast<const f32x4*>(bias + c);
-    }
-  }
-  for (int j = 0; j < k; ++j) {
-    const TY* yr = y + (long)inv[row * k + j] * ldy;
-    const float wt = wts[row * k + j];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const int c = 4 * tid + 1024 * v;
-      if (c >= H) continue;
-      const vecy_t r = *reinterpret_cast<const vecy_t*>(yr + c);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const TY q = r[e];
-        a[v][e] += wt * ldf(&q);
+      for (int j = 0; j < NE; ++j) {
+        const int c = min(c0 + ST * j, c1 - 1);
+        s[j] = xr[c];
+        g[j] = w[c];
       }
     }
-  }
+    if (k == 0) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const float q = wave_sum(a[v][0] * a[v][0] + a[v][1] * a[v][1] + a[v][2] * a[v][2] + a[v][3] * a[v][3]);
-    if (lane == 0) red[4 * v + wave] = q;
-  }
-  __syncthreads();
-  const int n = H / groups, per = groups == 1 ? 4 * NV : n / 256;     // 256s of a part
+      for (int j = 0; j < NE; ++j) {
+        const int c = min(c0 + ST * j, c1 - 1);
+        a[j] = ldf(y + row * ldy + c) + (bias ? bias[c] : 0.f);
+      }
+    } else {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int c = 4 * tid + 1024 * v;
-    if (c >= H) continue;
-    const int first = (4 * v + wave) / per * per;
+      for (int j = 0; j < NE; ++j) a[j] = 0.f;
+      for (int e = 0; e < k; ++e) {
+        const TY* yr = y + (long)inv[row * k + e] * ldy;
+        const float wt = wts[row * k + e];
+#pragma unroll
+        for (int j = 0; j < NE; ++j) a[j] += wt * ldf(yr + min(c0 + ST * j, c1 - 1));
+      }
+      if constexpr (sizeof(TY) == 2) {
+#pragma unroll
+        for (int j = 0; j < NE; ++j) a[j] = bf2f(f2bf(a[j]));
+      }
+    }
     float q = 0.f;
-    for (int i = 0; i < per; ++i) q += red[first + i];
-    const float r = 1.f / sqrtf(q / (float)n + eps);
-    const f32x4 o = s[v] + a[v] * r * g[v];
-    *reinterpret_cast<f32x4*>(x + row * H + c) = o;
-    if (xl) {
-      vec_t b;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        T q;
-        stf(&q, o[e]);
-        b[e] = q;
-      }
-      *reinterpret_cast<vec_t*>(xl + row * H + c) = b;
+    for (int j = 0; j < NE; ++j) {
+      const float v = c0 + ST * j < c1 ? a[j] : 0.f;
+      q = fmaf(v, v, q);     // as the loop's sum is contracted
     }
+    q = wave_sum(q);
+    if constexpr (!PARTS) {
+      if (lane == 0) red[wave] = q;
+      __syncthreads();
+      q = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q += red[i];
+    }
+    const float r = 1.f / sqrtf(q / (float)n + eps);
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const int c = c0 + ST * j;
+      if (c >= c1) continue;
+      const float v = (EARLY ? s[EARLY ? j : 0] : xr[c]) + a[j] * r * (EARLY ? g[EARLY ? j : 0] : w[c]);
+      xr[c] = v;
+      if (xl) stf(xl + row * (long)H + c, v);
+    }
+    if constexpr (!PARTS) break;
   }
 }
 
@@ -1494,14 +1476,14 @@ namespace {
 template <typename TI, typename TO>
 int rms_rows(const void* x, long ldx, const float* w, void* y, long ldy, int rows, int n, float eps, int groups, hipStream_t st) {
   const dim3 g((rows * groups + 3) / 4), b(256);
-  const auto al = [](const void* p, size_t by) { return ((uintptr_t)p & (by - 1)) == 0; };
-  if (n % 4 == 0 && n <= 4096 && ldx % 4 == 0 && ldy % 4 == 0 && al(x, 4 * sizeof(TI)) && al(y, 4 * sizeof(TO)) && al(w, 16)) {
-#define RMSV(NV) hipLaunchKernelGGL((rms_rows_vec_kernel<TI, TO, NV>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups)
-    if (n <= 256) RMSV(1); else if (n <= 512) RMSV(2); else if (n <= 1024) RMSV(4); else if (n <= 2048) RMSV(8); else RMSV(16);
+#define RMSV(NE) hipLaunchKernelGGL((rms_rows_reg_kernel<TI, TO, NE>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups)
+  if (n <= 256) RMSV(4);
+  else if (n <= 512) RMSV(8);
+  else if (n <= 1024) RMSV(16);
+  else if (n <= 2048) RMSV(32);
+  else if (n <= 4096) RMSV(64);
+  else hipLaunchKernelGGL((rms_rows_kernel<TI, TO>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups);
 #undef RMSV
-  } else {
-    hipLaunchKernelGGL((rms_rows_kernel<TI, TO>), g, b, 0, st, (const TI*)x, ldx, w, (TO*)y, ldy, rows, n, eps, groups);
-  }
   return (int)hipGetLastError();
 }
 }  // namespace
@@ -1518,46 +1500,49 @@ extern "C" int dllm_rms_rows(const void* x, long ldx, int x_f32, const float* w,
 }
 
 namespace {
+// entries a thread holds: a workgroup on the row, or a wave on a part; 0: past the registers (rows of 8192, parts of 4096)
+int norm_resadd_entries(int H, int groups) {
+  const int e = groups == 1 ? (H + 255) / 256 : (H / groups + 63) / 64, most = groups == 1 ? 32 : 64;
+  return e > most ? 0 : e;
+}
 template <typename T, typename TY>
-int norm_resadd_vec(const void* y, long ldy, const float* w, float* x, void* xl, long rows, int H, float eps, int groups,
+int norm_resadd_reg(const void* y, long ldy, const float* w, float* x, void* xl, long rows, int H, float eps, int groups,
                     const float* bias, const int* inv, const float* wts, int k, hipStream_t st) {
-#define NRV(NV)                                                                                                            \
-  hipLaunchKernelGGL((norm_resadd_vec_kernel<T, TY, NV>), dim3((unsigned)rows), dim3(256), 0, st, (const TY*)y, ldy, w, x, (T*)xl, H, \
+  const int e = norm_resadd_entries(H, groups);
+#define NRV(NE, PARTS)                                                                                                                   \
+  hipLaunchKernelGGL((norm_resadd_reg_kernel<T, TY, NE, PARTS>), dim3((unsigned)rows), dim3(256), 0, st, (const TY*)y, ldy, w, x, (T*)xl, H, \
                      eps, groups, bias, inv, wts, k)
-  if (H <= 1024) NRV(1); else if (H <= 2048) NRV(2); else if (H <= 4096) NRV(4); else NRV(8);
+  if (groups == 1) {
+    if (e <= 4) NRV(4, false); else if (e <= 8) NRV(8, false); else if (e <= 16) NRV(16, false); else NRV(32, false);
+  } else {
+    if (e <= 4) NRV(4, true); else if (e <= 8) NRV(8, true); else if (e <= 16) NRV(16, true); else if (e <= 32) NRV(32, true); else NRV(64, true);
+  }
 #undef NRV
   return (int)hipGetLastError();
 }
-// rows of whole vectors whose parts are whole 256s; `ab`: bytes of a vector of activations
-bool norm_resadd_vec_ok(const void* y, long ldy, int yb, const float* w, const float* x, const void* xl, int ab, int H, int groups,
-                        const float* bias) {
-  const auto al = [](const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; };
-  return H % 4 == 0 && H <= 8192 && (groups == 1 || H / groups % 256 == 0) && ldy % 4 == 0 && al(y, yb) && al(w, 16) && al(x, 16) &&
-         al(bias, 16) && al(xl, ab);
-}
 }  // namespace
 
-// May a MoE layer end in one launch with its norm and residual add (the stream and the weights come 16-byte aligned)?
+// May a MoE layer end in one launch with its norm and residual add?
 extern "C" int dllm_moe_tail_ok(int H, int groups) {
-  return H % 4 == 0 && H <= 8192 && groups >= 1 && H % groups == 0 && (groups == 1 || H / groups % 256 == 0);
+  return groups >= 1 && H >= groups && H % groups == 0 && norm_resadd_entries(H, groups) > 0;
 }
 
 // x += rmsnorm(sum_j wts[t k + j] y[inv[t k + j]]) * w in `groups` parts; y [P, H] f32 or bf16, xl the rounded stream (bf16) or null
 extern "C" int dllm_moe_norm_resadd(const void* y, int f32, const int* inv, const float* wts, int k, const float* w, float* x, void* xl,
                                     long T, int H, float eps, int groups, hipStream_t st) {
   if (T <= 0) return T == 0 ? 0 : -1;
-  if (k < 1 || groups < 1 || H % groups || !norm_resadd_vec_ok(y, H, f32 ? 16 : 8, w, x, xl, 8, H, groups, nullptr)) return -2;
-  return f32 ? norm_resadd_vec<u16, float>(y, H, w, x, xl, T, H, eps, groups, nullptr, inv, wts, k, st)
-             : norm_resadd_vec<u16, u16>(y, H, w, x, xl, T, H, eps, groups, nullptr, inv, wts, k, st);
+  if (k < 1 || !dllm_moe_tail_ok(H, groups)) return -2;
+  return f32 ? norm_resadd_reg<u16, float>(y, H, w, x, xl, T, H, eps, groups, nullptr, inv, wts, k, st)
+             : norm_resadd_reg<u16, u16>(y, H, w, x, xl, T, H, eps, groups, nullptr, inv, wts, k, st);
 }
 
 extern "C" int dllm_norm_resadd(const void* y, long ldy, int f32, const float* w, float* x, void* xl, int rows, int H,
                                 float eps, int groups, const float* bias, hipStream_t st) {
   if (rows <= 0) return rows == 0 ? 0 : -1;
   if (groups < 1 || H % groups) return -1;
-  if (norm_resadd_vec_ok(y, ldy, f32 ? 16 : 8, w, x, xl, f32 ? 16 : 8, H, groups, bias))
-    return f32 ? norm_resadd_vec<float, float>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st)
-               : norm_resadd_vec<u16, u16>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st);
+  if (norm_resadd_entries(H, groups))
+    return f32 ? norm_resadd_reg<float, float>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st)
+               : norm_resadd_reg<u16, u16>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st);
   BY_T(f32,
        hipLaunchKernelGGL(norm_resadd_kernel<u16>, dim3(rows), dim3(256), 0, st, (const u16*)y, ldy, w, x, (u16*)xl, H, eps, groups, bias),
        hipLaunchKernelGGL(norm_resadd_kernel<float>, dim3(rows), dim3(256), 0, st, (const float*)y, ldy, w, x, (float*)xl, H, eps, groups, bias))

@@ -23,19 +23,22 @@
 
 namespace {
 
-template <int MT, int NTW, bool SWIGLU>
-__global__ void __launch_bounds__(256) skinny_gemm_kernel(const u16* __restrict__ X, long ldx,
+// VS splits of K share a workgroup, four waves each as if alone: the order of every sum is that of VS = 1 (a row's bits depend on the
+// splits only, never on the launch's shape), and up to VS splits meet in LDS instead of slabs and a ticket.
+template <int MT, int NTW, bool SWIGLU, int VS>
+__global__ void __launch_bounds__(256 * VS) skinny_gemm_kernel(const u16* __restrict__ X, long ldx,
                                                           const u16* __restrict__ W, u16* __restrict__ Y, long ldy,
-                                                          int M, int N, int K, int kchunk, float* __restrict__ part,
+                                                          int M, int N, int K, int kchunk, int S, float* __restrict__ part,
                                                           int* __restrict__ counters) {
   constexpr int NC = 16 * NTW;  // columns per workgroup
-  __shared__ float s_red[2][MT * 16][NC + 1];
+  __shared__ float s_all[VS][2][MT * 16][NC + 1];
   __shared__ int s_last;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = wv & 3, grp = wv >> 2;
   const int g = lane >> 4, r16 = lane & 15;
-  const int tile = blockIdx.x, split = blockIdx.y, S = gridDim.y;
+  const int tile = blockIdx.x, split = blockIdx.y * VS + grp;
+  float(*s_red)[MT * 16][NC + 1] = s_all[grp];
   const int col0 = tile * NC;
-  const int kbeg = split * kchunk;
+  const int kbeg = min(K, split * kchunk);      // a group past the last split has nothing
   const int kend = min(K, kbeg + kchunk);
   // contiguous K range of this wave (multiple of 32)
   const int klen = kend - kbeg;
@@ -67,7 +70,7 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(const u16* __restrict_
 
   // Software pipeline: the loads of block i+1 (U k-steps of W and X) are in flight while the
   // MFMAs of block i run (two register stages, ping-pong, fully unrolled -> static indexing).
-  constexpr int U = MT >= 8 ? 1 : (MT >= 4 ? 2 : 4);
+  constexpr int U = MT >= 8 ? 1 : (MT >= 4 || VS == 4 ? 2 : 4);     // (16 waves a workgroup: 128 registers)
   struct Stage {
     bf16x8 w[U][NTW];
     uint4 x[U][MT];
@@ -86,9 +89,10 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(const u16* __restrict_
         if constexpr (SWIGLU) st.xu[u][m] = ld16(xrow[m] + K + k0 + 32 * u);
       }
   };
-  auto compute = [&](const Stage& st) {
+  auto compute = [&](const Stage& st, int steps) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      if (u >= steps) break;
       bf16x8 xf[MT];
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
@@ -118,45 +122,31 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(const u16* __restrict_
     load(A, kb);
     for (int i = 0; i < nblk; i += 2) {
       if (i + 1 < nblk) load(B, kb + 32 * U);
-      compute(A);
+      compute(A, U);
       if (i + 1 < nblk) {
         if (i + 2 < nblk) load(A, kb + 64 * U);
-        compute(B);
+        compute(B, U);
       }
       kb += 64 * U;
     }
     kb = wk0 + nblk * 32 * U;
   }
-  for (; kb < wk1; kb += 32) {  // tail (< U k-steps)
+  if (kb < wk1) {  // tail (< U k-steps), its loads in flight together
     Stage T;
+    const int tail = (wk1 - kb) / 32;
 #pragma unroll
-    for (int n = 0; n < NTW; ++n) T.w[0][n] = ldnt_bf16x8(wrow[n] + kb);
+    for (int u = 0; u < U; ++u) {
+      if (u >= tail) break;
+      const int k = kb + 32 * u;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      T.x[0][m] = ld16(xrow[m] + kb);
-      if constexpr (SWIGLU) T.xu[0][m] = ld16(xrow[m] + K + kb);
-    }
-    // compute only u = 0
-    bf16x8 xf[MT];
+      for (int n = 0; n < NTW; ++n) T.w[u][n] = ldnt_bf16x8(wrow[n] + k);
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      uint4 v = T.x[0][m];
-      if constexpr (SWIGLU) {
-        float gt[8], up[8];
-        unpack8(v, gt);
-        unpack8(T.xu[0][m], up);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) gt[j] = gt[j] / (1.f + __expf(-gt[j])) * up[j];
-        v = pack8(gt);
+      for (int m = 0; m < MT; ++m) {
+        T.x[u][m] = ld16(xrow[m] + k);
+        if constexpr (SWIGLU) T.xu[u][m] = ld16(xrow[m] + K + k);
       }
-      if (!xok[m]) v = make_uint4(0, 0, 0, 0);
-      xf[m] = __builtin_bit_cast(bf16x8, v);
     }
-#pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int n = 0; n < NTW; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[m], T.w[0][n], acc[m][n], 0, 0, 0);
+    compute(T, tail);
   }
 
   // ---- reduce the 4 waves in a fixed order ((w0 + w2) + (w1 + w3)): bitwise reproducible.
@@ -190,23 +180,31 @@ __global__ void __launch_bounds__(256) skinny_gemm_kernel(const u16* __restrict_
 #undef DLLM_FOR_C
   __syncthreads();
   const int rows = min(M, MT * 16);
-  if (S == 1) {
-    for (int e = threadIdx.x; e < rows * NC; e += 256) {
+  if (S <= VS) {      // every split is here
+    for (int e = threadIdx.x; e < rows * NC; e += 256 * VS) {
       const int row = e / NC, c = e % NC;
-      if (col0 + c < N) Y[(long)row * ldy + col0 + c] = f2bf(s_red[1][row][c]);
+      float v = s_all[0][1][row][c];
+      if (S > 1) {
+        v += 0.f;      // as the slabs' sum begins
+#pragma unroll
+        for (int sp = 1; sp < VS; ++sp)
+          if (sp < S) v += s_all[sp][1][row][c];
+      }
+      if (col0 + c < N) Y[(long)row * ldy + col0 + c] = f2bf(v);
     }
     return;
   }
   // ---- split-K: write-through slab store, ticket; the last arriver reduces (sc1 loads)
   const long slab_elems = (long)(MT * 16) * NC;
-  const __amdgpu_buffer_rsrc_t pr = make_rsrc(part, (unsigned)min((long)gridDim.x * gridDim.y * slab_elems * 4, 0x7fffffffL));
+  const __amdgpu_buffer_rsrc_t pr = make_rsrc(part, (unsigned)min((long)gridDim.x * S * slab_elems * 4, 0x7fffffffL));
   const unsigned my_off = (unsigned)(((long)split * gridDim.x + tile) * slab_elems * 4);
-  for (int e = threadIdx.x * 4; e < rows * NC; e += 1024) {
-    const int row = e / NC, c = e % NC;
-    st_wt16(pr, my_off + e * 4, make_float4(s_red[1][row][c], s_red[1][row][c + 1], s_red[1][row][c + 2], s_red[1][row][c + 3]));
-  }
-  if (!ticket_last(&counters[tile], S, &s_last)) return;
-  for (int e = threadIdx.x * 4; e < rows * NC; e += 1024) {
+  if (split < S)
+    for (int e = (threadIdx.x & 255) * 4; e < rows * NC; e += 1024) {
+      const int row = e / NC, c = e % NC;
+      st_wt16(pr, my_off + e * 4, make_float4(s_red[1][row][c], s_red[1][row][c + 1], s_red[1][row][c + 2], s_red[1][row][c + 3]));
+    }
+  if (!ticket_last(&counters[tile], gridDim.y, &s_last)) return;
+  for (int e = threadIdx.x * 4; e < rows * NC; e += 1024 * VS) {
     const int row = e / NC, c = e % NC;
     float4 v = {0.f, 0.f, 0.f, 0.f};
     for (int sp = 0; sp < S; ++sp) {
@@ -488,47 +486,54 @@ int epi_by(int ntw, int epi, const void* X, long ldx, const void* W, void* Y, lo
   }
 }
 
-template <int MT, int NTW, bool SW>
+template <int MT, int NTW, bool SW, int VS>
 int launch(const void* X, long ldx, const void* W, void* Y, long ldy, int M, int N, int K, int splits, float* part,
            int* counters, hipStream_t st) {
   const int tiles = (N + 16 * NTW - 1) / (16 * NTW);
   int kchunk = (K + splits - 1) / splits;
   kchunk = (kchunk + 31) & ~31;
   const int S = (K + kchunk - 1) / kchunk;
-  hipLaunchKernelGGL((skinny_gemm_kernel<MT, NTW, SW>), dim3(tiles, S), dim3(256), 0, st, (const u16*)X, ldx,
-                     (const u16*)W, (u16*)Y, ldy, M, N, K, kchunk, part, counters);
+  hipLaunchKernelGGL((skinny_gemm_kernel<MT, NTW, SW, VS>), dim3(tiles, (S + VS - 1) / VS), dim3(256 * VS), 0, st, (const u16*)X, ldx,
+                     (const u16*)W, (u16*)Y, ldy, M, N, K, kchunk, S, part, counters);
   return (int)hipGetLastError();
 }
 
 template <int MT, bool SW>
-int by_ntw(int ntw, const void* X, long ldx, const void* W, void* Y, long ldy, int M, int N, int K, int splits,
+int by_ntw(int ntw, const void* X, long ldx, const void* W, void* Y, long ldy, int M, int N, int K, int splits, int vs,
            float* part, int* counters, hipStream_t st) {
+#define SKV(NTW, VS) return launch<MT, NTW, SW, VS>(X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st)
+  if constexpr (MT <= 4 && !SW)
+    if (ntw == 2 && vs == 2) SKV(2, 2);
+  if constexpr (MT <= 2 && !SW)
+    if (ntw == 1 && vs == 4) SKV(1, 4);
+  if (vs != 1) return -12;
   switch (ntw) {
-    case 1: return launch<MT, 1, SW>(X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
-    case 2: return launch<MT, 2, SW>(X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
-    case 4: return launch<MT, 4, SW>(X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
+    case 1: SKV(1, 1);
+    case 2: SKV(2, 1);
+    case 4: SKV(4, 1);
     default: return -10;
   }
+#undef SKV
 }
 
 template <bool SW>
-int by_mt(int M, int ntw, const void* X, long ldx, const void* W, void* Y, long ldy, int N, int K, int splits,
+int by_mt(int M, int ntw, const void* X, long ldx, const void* W, void* Y, long ldy, int N, int K, int splits, int vs,
           float* part, int* counters, hipStream_t st) {
-  if (M <= 16) return by_ntw<1, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
-  if (M <= 32) return by_ntw<2, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
-  if (M <= 64) return by_ntw<4, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
-  if (M <= 128 && ntw <= 2) return by_ntw<8, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, part, counters, st);
+  if (M <= 16) return by_ntw<1, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, vs, part, counters, st);
+  if (M <= 32) return by_ntw<2, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, vs, part, counters, st);
+  if (M <= 64) return by_ntw<4, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, vs, part, counters, st);
+  if (M <= 128 && ntw <= 2) return by_ntw<8, SW>(ntw, X, ldx, W, Y, ldy, M, N, K, splits, vs, part, counters, st);
   return -11;
 }
 }  // namespace
 
 // part: >= splits * ceil(N / (16 ntw)) * 16 * ceil(M/16) * 16 * ntw floats; counters: >= ceil(N/(16 ntw)) ints, zeroed.
 extern "C" int dllm_skinny_gemm(const void* X, long ldx, const void* W, void* Y, long ldy, int M, int N, int K, int ntw,
-                                int splits, int swiglu, float* part, int* counters, hipStream_t stream) {
+                                int splits, int vs, int swiglu, float* part, int* counters, hipStream_t stream) {
   if (K % 32 != 0 || M <= 0 || M > 128 || splits < 1) return -1;
   if (splits > 1 && (!part || !counters)) return -2;
-  return swiglu ? by_mt<true>(M, ntw, X, ldx, W, Y, ldy, N, K, splits, part, counters, stream)
-                : by_mt<false>(M, ntw, X, ldx, W, Y, ldy, N, K, splits, part, counters, stream);
+  return swiglu ? by_mt<true>(M, ntw, X, ldx, W, Y, ldy, N, K, splits, vs, part, counters, stream)
+                : by_mt<false>(M, ntw, X, ldx, W, Y, ldy, N, K, splits, vs, part, counters, stream);
 }
 
 // Small-batch MFMA GEMM with a fused decoder epilogue (skinny_epi_kernel): M <= 16, K % 64 == 0

@@ -974,8 +974,11 @@ class HybridModel:
     def _experts_swiglu(self, L, f: MoESpec, x, tail=None):
         """Sigmoid router in f32 with group-limited top-k, weights = the chosen scores; SwiGLU experts
         on the grouped MFMA kernels, or in the dense form (all experts' columns in two GEMMs, unused
-        experts gated to zero) for f32 models and widths the grouped kernels do not take."""
-        ids, w, _, _ = seqmix.router_topk(x, L["router"], L["router"].shape[0], f.top, f.group_count, f.group_keep)
+        experts gated to zero) for f32 models and widths the grouped kernels do not take.  The logits are the
+        vendor's f32 product: ``seqmix.router_topk`` sums in another order (16 rows 6 us instead of 14), and the mLSTM
+        layers of these models turn the last bit of a weight into tenths of a logit."""
+        logits = F.linear(x.float(), L["router"])
+        ids, w = seqmix.group_router(logits, f.top, f.group_count, f.group_keep)
         if f.scale != 1.0:
             w = w * f.scale
         return self._swiglu_experts(L, f, x, ids, w, tail)

@@ -185,29 +185,40 @@ def _need_tg(M: int, N: int, K: int, bm: int, bn: int, splits: int, ks: int = 1)
 
 # ----------------------------------------------------------------------------- plans
 
-def _heuristic(M: int, N: int, K: int) -> Tuple:
-    """Plan of a shape nothing timed.  A weight of a few MB is bounded by what one workgroup takes in and by the
-    launch (more waves a workgroup do not help), so: as many workgroups as the columns give, 16 each (32 past
-    4096 columns, or for more rows on a very long K), and K split over workgroups only where one would stream more
-    than 64 KB (32 KB past 16 rows, whose activations it re-reads too) or the rows keep it busy, since slabs
-    and ticket cost 1.3 us at two splits and 2.3 at four.  One or two rows, and four on few columns, take the
-    GEMV (4 columns a workgroup).  us at 1024 columns, this plan against 32
-    columns and up to 16 splits: K 1024: 1 row 2.9 / 6.2, 4 rows 3.9 / 6.3, 16 rows 4.8 / 6.4, 64 rows 7.8 / 9.0;
-    K 4096: 1 row 4.5 / 12.9, 16 rows 8.1 / 13.2, 64 rows 11.5 / 16.9."""
+def _heuristic(M: int, N: int, K: int, swiglu: bool = False) -> Tuple:
+    """Plan of a shape nothing timed.  The splits of K depend on N and K alone and every split sums in the same order
+    (skinny_gemm.hip), so up to 64 rows a row's bits depend neither on the batch nor on how the launch is cut: a design whose
+    heads divide by small sums (mLSTM) turns a last bit into tenths of a logit.  What is left to choose is the columns of a
+    workgroup (16 or 32) and ``_splits_together``.  K that is no whole 32s: the GEMV, which takes one, two and four rows."""
     if M > SKINNY_MAX_M:
         return ("blas",)
     if M > 64:
         tiles = (N + 15) // 16
         return ("skinny", 1, max(1, min(16, math.ceil(512 / tiles), K // 256)))
-    if K % 8 == 0 and (M in (1, 2) or (M == 4 and (N <= 1024 or (N <= 2048 and 2048 <= K <= 4096)))) and M * K * 2 <= 64 * 1024:
+    if K % 32 and K % 8 == 0 and M in (1, 2, 4) and M * K * 2 <= 64 * 1024:
         return ("gemv", 1)
-    ntw = 2 if N > 4096 or (M > 16 and K >= 8192) else 1
-    splits = 1
-    if K > 2048 or (K > 1024 and M > 16) or M > 32:
-        tiles = (N + 16 * ntw - 1) // (16 * ntw)
-        while splits < 4 and tiles * splits * 2 <= 256 and K >= 512 * splits:
-            splits *= 2
-    return ("skinny", ntw, splits)
+    splits = max(1, min(16, math.ceil(512 / ((N + 31) // 32)), K // 256))
+    narrow = N * K <= _NARROW if M <= 32 else N <= 2048 and splits <= 4
+    return ("skinny", 1 if narrow and not swiglu else 2, splits)
+
+
+# weights up to which 16 columns and four splits of K a workgroup (16 waves) beat 32 columns and two: past it the 16-wave workgroups,
+# one a CU, come in several rounds.  us at 8 rows / 24 rows, 16 x 4, 32 x 2, and 32 x 1 as nothing else would choose:
+# 1024 x 1024 4.2 / 5.1, 6.5 / 7.3, 6.1 / 6.7; 5632 x 1024 6.8 / 9.7, 8.6 / 11.9, 8.5 / 10.7; 1024 x 4096 11.4 / 12.7, 11.8 / 12.4,
+# 12.4 / 13.2; 8192 x 2048 10.9 / 16.0, 10.8 / 12.7, 12.7 / 14.8.  Past 32 rows a workgroup re-reads more rows than weights: 16
+# columns, a split each, where that is few workgroups (48 rows, 1024 x 1024: 7.1, 8.2, 8.5; 4096 x 1024 11.3, 8.9, 10.0).
+_NARROW = 8 << 20
+
+
+def _splits_together(M: int, plan: Tuple) -> int:
+    """Splits of K that share a workgroup of an untimed plan, meeting in LDS where they are all there (slabs and ticket cost 1.3 to 2.3
+    us).  Three splits of 32 columns stay apart: the pairs would leave a quarter of the waves idle."""
+    _, ntw, splits = plan
+    if M > 64 or splits == 1:
+        return 1
+    if ntw == 1:
+        return 4 if M <= 32 else 1
+    return 1 if splits == 3 else 2
 
 
 # Prefill-size buckets (M > MAX_M, PREFILL_TUNE): the fused ops' core is chosen per (bucket, N, K)
@@ -288,7 +299,7 @@ def tg_slots(M: int, N: int, K: int) -> int:
     return -(-N // tg_plan(M, N, K)[1])
 
 
-def _run_plan(plan, x, w, swiglu, out, wp=None):
+def _run_plan(plan, x, w, swiglu, out, wp=None, together=1):
     if plan[0] == "blas":
         if swiglu:
             x = ref_silu_mul(x)
@@ -309,7 +320,7 @@ def _run_plan(plan, x, w, swiglu, out, wp=None):
     y = out if out is not None else torch.empty((M, N), dtype=x.dtype, device=x.device)
     floats, tiles = _need(M, N, K, ntw, splits)
     part, cnt = _P.workspace(x.device, floats, tiles)
-    ext.skinny_gemm(x, w, y, ntw, splits, swiglu, part, cnt)
+    ext.skinny_gemm(x, w, y, ntw, splits, swiglu, part, cnt, together)
     return y
 
 
@@ -411,13 +422,15 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     """``x @ w.T`` on the shape's tuned plan; ``wp``: the panel copy a tgemm plan streams."""
     if not x.is_cuda or os.environ.get("DLLM_GEMM") == "blas":
         return F.linear(x, w) if out is None else torch.matmul(x, w.t(), out=out)
-    plan = _P.plans.get(_key(x, w, False))
+    plan, together = _P.plans.get(_key(x, w, False)), 1
     if plan is None:
         if x.shape[0] > MAX_M:
             plan = ("blas",)
         else:
             plan = _heuristic(x.shape[0], w.shape[0], w.shape[1])
-    return _run_plan(plan, x, w, False, out, wp)
+            if plan[0] == "skinny":
+                together = _splits_together(x.shape[0], plan)
+    return _run_plan(plan, x, w, False, out, wp, together)
 
 
 def norm_linear(h: torch.Tensor, residual: torch.Tensor, spare: torch.Tensor, norm_w: torch.Tensor, eps: float,
@@ -437,7 +450,7 @@ def linear_swiglu(gu: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if gu.shape[0] > MAX_M or os.environ.get("DLLM_GEMM") == "blas":
         from . import silu_mul
         return linear(silu_mul(gu), w)
-    plan = _P.plans.get(_key(gu, w, True)) or _heuristic(gu.shape[0], w.shape[0], w.shape[1])
+    plan = _P.plans.get(_key(gu, w, True)) or _heuristic(gu.shape[0], w.shape[0], w.shape[1], True)
     return _run_plan(plan, gu, w, True, None)
 
 
