@@ -24,11 +24,11 @@
 // padded by 4 floats: 16-byte reads over 16 rows and 4-byte reads over 4 rows x 16 columns both spread over all banks.
 //
 // Rows go to LDS in two steps, several loads a thread in flight before the first conversion (one at a time the
-// staging took half of either kernel), and SiLU is the hardware's exponential and reciprocal with a compensated argument.
+// staging took half of either kernel).
 //
 // What bounds it: 16 heads of 128 x 128 over 6 x 1400 tokens are 12 GFLOP of f32 MFMA a layer (80 us at 157 TFLOP/s) and
 // 0.5 GB of chunk states (100 us at 5.2 TB/s); chunks of 128 would halve the states and need twice the LDS.  Measured
-// there (bf16 rows): sums 108, carry 53, outputs 158 us (150, 53, 242 with rows staged one load at a time).  One
+// there (bf16 rows): sums 119, carry 53, outputs 175 us with SiLU on every row (expf and a division: 8 % of a layer).  One
 // prompt of 4096 tokens, with its norm and gate: retention with 8 heads of 64 x 128 about 80 us against 1900 us
 // for chunks in order (seqmix.hip); Mamba-2 with 32 heads of 128 x 64 about 150 us against 1390 us token by token
 // (outer_scan.hip).
@@ -63,14 +63,7 @@ struct ScanArgs {
   int vec, rotvec;            // rows, head offsets and widths allow four elements at a time; so do rotation and its table
 };
 
-// x sigmoid(x) within a few ulp, without expf's and the division's range handling: the product with log2 e in two
-// parts, the hardware's exponential and reciprocal.  Past the clamp the sigmoid is 1, or below 2^-125 times x.
-__device__ __forceinline__ float silu_f(float x) {
-  const float c = fminf(fmaxf(x, -87.f), 100.f);
-  const float hi = -1.44269504f * c, lo = fmaf(-1.44269504f, c, -hi) - 1.92596299e-8f * c;
-  const float e = __builtin_amdgcn_exp2f(hi);
-  return x * __builtin_amdgcn_rcpf(1.f + fmaf(e * lo, 0.693147181f, e));
-}
+__device__ __forceinline__ float silu_f(float x) { return x / (1.f + expf(-x)); }
 
 // four elements of a row as they lie in memory
 template <typename T> struct Quad;
