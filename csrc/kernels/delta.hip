@@ -223,7 +223,8 @@ constexpr int DT_W = 2 * DT_L + 8;  // floats delta_prep leaves per (token, head
 
 // A wave per (tile, head).  Operands come from the rows as they lie: lane lr of a matrix operand is token lr, and contraction
 // step x of lane group g4 stands for dim 16 b + 4 g4 + x, so a lane reads four neighbours.  The inverse is a forward
-// substitution with a column per lane (120 multiply-adds; A's columns broadcast from LDS).  8400 tokens of 16 heads of 128: 36 us (97 us with loads behind branches).
+// substitution with a column per lane (120 multiply-adds; A's columns broadcast from LDS).  8400 tokens of 16 heads of 128: 50 us
+// (36 with one chain of d for each dot product, 97 with loads behind branches).
 template <typename T, int NB, bool VL>
 __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ qkv, long ldq, const T* __restrict__ gba, long ldg,
                                                          int H, int G, int d, int dv, const float* __restrict__ neg_a,
@@ -295,16 +296,27 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ q
   sq += __shfl_xor(sq, 32);
   sk += __shfl_xor(sk, 32);
   const float fq = (1.f / sqrtf((float)d)) / sqrtf(sq + 1e-6f), fk = 1.f / sqrtf(sk + 1e-6f);
-  f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
+  // k . k and q . k as sixteen sums of at most eight dims, added pairwise: a chain of d roundings would be the largest error of the rule
+  const auto dots = [&](const f32x4(&a)[NB], const f32x4(&b)[NB]) {
+    f32x4 p[16];
+#pragma unroll
+    for (int x = 0; x < 16; ++x) p[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < NB; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[4 * (x & 3) + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x][e], b[x][e], p[4 * (x & 3) + e], 0, 0, 0);
+#pragma unroll
+    for (int o = 8; o; o >>= 1)
+#pragma unroll
+      for (int x = 0; x < o; ++x) p[x] += p[x + o];
+    return p[0];
+  };
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
-    const f32x4 a = k[b] * fk, z = q[b] * fq;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      kk = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], a[e], kk, 0, 0, 0);
-      qk = __builtin_amdgcn_mfma_f32_16x16x4f32(z[e], a[e], qk, 0, 0, 0);
-    }
+    k[b] *= fk;
+    q[b] *= fq;
   }
+  const f32x4 kk = dots(k, k), qk = dots(q, k);
   f32x4 av, pv;    // column lr, rows 4 g4 + e
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -351,10 +363,12 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ q
 // A workgroup owns 16 value columns of one (sequence, head); its four waves own a quarter of the key dims each, as the
 // accumulators of the last product, which are at once the right operand of S^T k and S^T q.  The waves' parts meet in LDS, a
 // thread sums one element of each, and U = (I + A)^-1 R comes out as the right operand of the state's update.  Serial over the
-// tiles, so the chain of one tile bounds it: two products, one exchange, two small products, the update.  bf16, 16 heads of 128 x 128: 6 sequences of 1400
-// tokens 349 us with the two launches beside it against 663 token by token, one of 4096 tokens 480 against 1224; errors against
-// 64 bits: state 3.1e-7 against 7.8e-7 over 385 tokens with slow decays, outputs 2.7e-7 against 2.9e-7 (steep decays: 1.3e-7
-// against 1.1e-7 and 2.2e-7 against 1.6e-7).
+// tiles, so the chain of one tile bounds it: two products, one exchange, two small products, the update.  Sums of more than four terms go in
+// parts that are added pairwise, or the largest last.  bf16, 16 heads of 128 x 128: 6 sequences of 1400 tokens 355 us with the two
+// launches beside it against 617 token by token, one of 4096 tokens 523 against 1219 (314 and 472 with one chain a sum, whose outputs
+// were up to 1.5 times as far off as token by token).  f32 errors against 64 bits over 385 tokens, state and outputs, token by token
+// in brackets: decays near 1 1.5e-7 (5.6e-7), 1.7e-7 (2.6e-7); a model's (0.01 to 0.3 a token) 1.2e-7 (1.9e-7), 1.6e-7 (1.7e-7); up
+// to 4 a token 1.0e-7 (1.05e-7), 1.53e-7 (1.49e-7).
 template <typename T, int NS, bool VL>
 __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ qkv, long ldq, int H, int G, int d, int dv,
                                                          float* __restrict__ state, const int* __restrict__ qstart,
@@ -454,20 +468,22 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
   for (int t0 = 0, buf = 0; t0 < n; t0 += DT_L, buf ^= 1) {
     const int nt = min(DT_L, n - t0);
     {
-      f32x4 tk = {0.f, 0.f, 0.f, 0.f}, tq = tk;
+      f32x4 tk[4], tq[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) tk[x] = tq[x] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const int i = lr * LD + 16 * (w * NB + b) + 4 * g4;
         const f32x4 a = *reinterpret_cast<const f32x4*>(ks[buf] + i), q = *reinterpret_cast<const f32x4*>(qs[buf] + i);
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-          tk = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], S[b][x], tk, 0, 0, 0);
-          tq = __builtin_amdgcn_mfma_f32_16x16x4f32(q[x], S[b][x], tq, 0, 0, 0);
+          tk[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], S[b][x], tk[x], 0, 0, 0);
+          tq[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[x], S[b][x], tq[x], 0, 0, 0);
         }
       }
       float* p = part + w * 2 * TP + lr * DT_P + 4 * g4;
-      *reinterpret_cast<f32x4*>(p) = tk;
-      *reinterpret_cast<f32x4*>(p + TP) = tq;
+      *reinterpret_cast<f32x4*>(p) = (tk[0] + tk[1]) + (tk[2] + tk[3]);
+      *reinterpret_cast<f32x4*>(p + TP) = (tq[0] + tq[1]) + (tq[2] + tq[3]);
     }
     __syncthreads();
     {   // token `row`, column lr
@@ -484,22 +500,33 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
     }
     __syncthreads();
     const f32x4 r = *reinterpret_cast<const f32x4*>(Rs + lr * DT_P + 4 * g4);
-    f32x4 u = {0.f, 0.f, 0.f, 0.f}, o = *reinterpret_cast<const f32x4*>(Os + lr * DT_P + 4 * g4);
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 u4[4];
+    // each of the small products as four sums: token i's own term, which steep decays leave alone, is then the last of sum i % 4 (of
+    // entry e = i % 4 of this lane's rows 4 g4 + e), and that sum is added last
     const f32x4 we = *reinterpret_cast<const f32x4*>(ws + 4 * g4);
     const float gam = last;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) u = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.inv[x], r[x], u, 0, 0, 0);
+    for (int x = 0; x < 4; ++x) u4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.inv[x], r[x], zero, 0, 0, 0);
+    f32x4 u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = (u4[e ^ 1][e] + (u4[e ^ 2][e] + u4[e ^ 3][e])) + u4[e][e];
     const f32x4 z = we * u;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const float* kp = ks[buf] + 4 * g4 * LD + 16 * (w * NB + b) + lr;
-      S[b] *= gam;
+      f32x4 s4[4];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) S[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kp[x * LD], z[x], S[b], 0, 0, 0);
+      for (int x = 0; x < 4; ++x) s4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kp[x * LD], z[x], zero, 0, 0, 0);
+      S[b] = ((gam * S[b] + (s4[0] + s4[1])) + s4[2]) + s4[3];      // the last tokens last
     }
     if (w == ((t0 >> 4) & 3)) {   // the waves take turns with the outputs
+      f32x4 o4[4];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) o = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x], u[x], o, 0, 0, 0);
+      for (int x = 0; x < 4; ++x) o4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x], u[x], zero, 0, 0, 0);
+      f32x4 o = *reinterpret_cast<const f32x4*>(Os + lr * DT_P + 4 * g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (o[e] + (o4[e ^ 1][e] + (o4[e ^ 2][e] + o4[e ^ 3][e]))) + o4[e][e];
 #pragma unroll
       for (int x = 0; x < 4; ++x)
         if (live && 4 * g4 + x < nt) raw[((long)(q0 + t0 + 4 * g4 + x) * H + h) * dv + j] = o[x];

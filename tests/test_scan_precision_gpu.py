@@ -56,3 +56,38 @@ def test_lightning(lo, hi):
         seqmix.lightning_attention(torch.cat([qk, v, v], 1), H, 1, dv, torch.full((H,), 0.9, device=DEV), s, 1e-6, torch.ones(H * dv, device=DEV),
                                    *one_token_each(S), chunked=chunked)
     assert torch.equal(st[0], st[1])                   # prompts and steps of one layer round alike
+
+
+@pytest.mark.parametrize("decay,more", [("slow", 0), ("model", 0), ("steep", 2)])
+@pytest.mark.parametrize("H,G,d,dv", [(16, 8, 128, 128), (4, 2, 64, 64)])
+def test_delta_tiles(decay, more, H, G, d, dv):
+    """Sixteen tokens at a time against token by token: no further from 64 bits with decays near 1 or a model's (A of 1 to 16, steps
+    of 0.001 to 0.1).  Where a token keeps a fiftieth of the state and a few roundings are all there is, two more (2^-24 / sqrt 3 root
+    mean square each): a token's update times its decay up to the tile's end, and the sum over the tile."""
+    torch.manual_seed(3)
+    T = 385
+    qkv, gba = torch.randn(T, 2 * G * d + H * dv, device=DEV), torch.randn(T, H * dv + 2 * H, device=DEV)
+    na, dtb, nw = -torch.rand(H, device=DEV) * {"slow": 0.05, "model": 0.0, "steep": 8.0}[decay], torch.randn(H, device=DEV), torch.randn(dv, device=DEV)
+    if decay == "model":
+        step = torch.exp(torch.rand(H, device=DEV) * 4.6 - 6.9)
+        na, dtb = -(1 + 15 * torch.rand(H, device=DEV)), step + torch.log(-torch.expm1(-step))
+    q, k, v = qkv.double().split([G * d, G * d, H * dv], 1)
+    q, k = (z.view(T, G, d) * torch.rsqrt((z.view(T, G, d) ** 2).sum(-1, keepdim=True) + 1e-6) for z in (q, k))
+    q, k = (q * d ** -0.5).repeat_interleave(H // G, 1), k.repeat_interleave(H // G, 1)
+    v, gate, beta, al = v.view(T, H, dv), *gba.double().split([H * dv, H, H], 1)
+    beta, g = torch.sigmoid(beta), torch.exp(na.double() * torch.nn.functional.softplus(al + dtb.double(), threshold=40))
+    M, o = torch.zeros(H, dv, d, dtype=torch.float64, device=DEV), []
+    for t in range(T):
+        M = g[t, :, None, None] * M
+        u = beta[t, :, None] * (v[t] - (M * k[t, :, None]).sum(-1))
+        M = M + u[:, :, None] * k[t, :, None]
+        o.append((M * q[t, :, None]).sum(-1))
+    o = torch.stack(o)
+    want = (o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-6) * nw.double()).reshape(T, -1) * torch.nn.functional.silu(gate)
+    i32 = lambda x: torch.tensor([x], dtype=torch.int32, device=DEV)  # noqa: E731
+    errs = []
+    for tiled in (True, False):
+        st = torch.zeros(1, H, dv, d, device=DEV)
+        y = seqmix.delta_rule(qkv, gba, H, G, d, dv, na, dtb, nw, 1e-6, st, i32(0), i32(T), i32(T), i32(0), tiled=tiled)
+        errs.append((float((y.double() - want).norm() / want.norm()), float((st[0].double() - M).norm() / M.norm())))
+    assert all(a * a <= b * b + more * 2.0 ** -48 / 3 for a, b in zip(*errs)), errs
