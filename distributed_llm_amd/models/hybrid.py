@@ -685,7 +685,7 @@ class HybridModel:
         dbc = _mm(xc, L["x"])
         dt_raw = _mm(dbc[:, :m.dt_rank], L["dt"])
         y = seqmix.selective_scan(xc, dt_raw, L["dt_b"], L["A"], dbc, m.dt_rank, L["D"], xz, ssm_state, conv_state,
-                                  meta.qstart, meta.qlen, meta.ctx, rows)
+                                  meta.qstart, meta.qlen, meta.ctx, rows, longest=self._longest(meta))
         return _mm(y, L["o"])
 
     def _retention(self, L, m: MixerSpec, x, positions, meta, cache):
@@ -693,7 +693,7 @@ class HybridModel:
         rot = m.rot.dims if m.rot is not None else 0
         table = self._table(m) if rot else self._any_table()
         o = seqmix.retention(qkvg, m.heads, m.dim, m.vdim, table, rot, L["decay"], cache[0], self.cfg.rms_eps,
-                             positions, meta.qstart, meta.qlen, meta.ctx, meta.state_rows)
+                             positions, meta.qstart, meta.qlen, meta.ctx, meta.state_rows, longest=self._longest(meta))
         return _mm(o, L["o"])
 
     def _any_table(self) -> torch.Tensor:
@@ -758,7 +758,7 @@ class HybridModel:
         if not single:
             seqmix.conv_state_refill(proj, conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
         o = seqmix.delta_rule(qkv, proj[:, c:], m.heads, m.kv_heads, m.dim, m.vdim, L["neg_a"], L["dt_b"], L["hnorm"],
-                              self.cfg.rms_eps, state, meta.qstart, meta.qlen, meta.ctx, rows)
+                              self.cfg.rms_eps, state, meta.qstart, meta.qlen, meta.ctx, rows, longest=self._longest(meta))
         return _mm(o, L["o"])
 
     def _parallel(self, L, m: MixerSpec, x, positions, meta, cache):
@@ -778,7 +778,7 @@ class HybridModel:
         lo = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
                                         gate, mfma, splits)
         ro = seqmix.lightning_attention(proj[:, nl:], b.heads, b.dim, b.vdim, L["decay"], state, eps, L["rnorm"],
-                                        meta.qstart, meta.qlen, meta.ctx, meta.state_rows)
+                                        meta.qstart, meta.qlen, meta.ctx, meta.state_rows, longest=self._longest(meta))
         return _mm(lo, L["lo"]), _mm(ro, L["ro"])
 
     def _diff_attention(self, L, m: MixerSpec, x, positions, meta, cache):
@@ -933,6 +933,11 @@ class HybridModel:
             if self.tap is not None:
                 self.tap.append(x.clone())
         return h if meta.all_last else h.index_select(0, meta.last_idx)
+
+    @staticmethod
+    def _longest(meta) -> int:
+        """New tokens of the step's longest portion; a decode step has single tokens."""
+        return 1 if not meta.host_qlen else max(int(n) for n in meta.host_qlen)
 
     @staticmethod
     def _all_rows(x, meta) -> bool:

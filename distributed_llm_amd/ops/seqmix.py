@@ -82,25 +82,33 @@ def causal_conv_silu(x, w, b, conv_state, qstart, qlen, ctx, rows, refill: bool 
     return y
 
 
-# average new tokens per sequence from which the chunk-parallel scan runs (2048 channels of 16 states): one sequence of
-# 128 tokens 40 against 30 us, 256 tokens 38 against 53; 24 sequences of 64 tokens 63 against 55, of 160 tokens 106
-# against 126; the two lines cross near 190 and 100 tokens
-SCAN_CHUNK_MIN = 160
+def longest_portion(T: int, S: int, longest: Optional[int]) -> float:
+    """New tokens of a step's longest portion, which is what a recurrence walked token by token takes its time from; where the
+    caller does not say, the average of T tokens over S sequences."""
+    return T / max(1, S) if longest is None else longest
+
+
+def scan_in_chunks(T: int, S: int, longest: Optional[int]) -> bool:
+    """Does the chunk-parallel scan run?  From portions of 160 tokens on; one such beside short ones has to pay for their chunks too.
+    2048 channels of 16 states, us token by token / in chunks: one sequence of 128 tokens 30 / 39, of 256 53 / 39; 24 of 64 53 / 64, of
+    192 132 / 121; 200 tokens beside 31 single ones 44 / 50, 2000 beside 23 of 20 436 / 81."""
+    n = longest_portion(T, S, longest)
+    return n >= 160 and (T >= 100 * S or n >= 160 + 2 * S)
 
 
 def selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_state, qstart, qlen, ctx,
-                   rows, chunked: Optional[bool] = None) -> torch.Tensor:
+                   rows, chunked: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
     """Mamba-1: S <- exp(dt A) S + dt x B, y = S C + D x, times silu(z), with dt = softplus(dt_raw + dt_bias), B and C
     behind the first ``dt_rank`` columns of dbc, z the second half of xz; also refills the convolution state.
-    ``chunked`` (GPU): the chunk-parallel kernels (N <= 32) or the token-by-token one; default by the step's
-    tokens per sequence."""
+    ``chunked`` (GPU): the chunk-parallel kernels (N <= 32) or the token-by-token one; default by the tokens of
+    the step's ``longest`` portion."""
     ext = _native(xc)
     if ext is None:
         return ref.selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_state, qstart, qlen,
                                   ctx, rows)
     out = torch.empty_like(xc)      # rows of no sequence become zeros
     if chunked is None:
-        chunked = xc.shape[0] >= SCAN_CHUNK_MIN * qstart.numel()
+        chunked = scan_in_chunks(xc.shape[0], qstart.numel(), longest)
     ext.selective_scan(xc, dt_raw, dt_bias, A, dbc, int(dt_rank), D, xz, ssm_state, conv_state, qstart, qlen, ctx,
                        rows, out, bool(chunked))
     return out
@@ -114,14 +122,17 @@ def retention_step_lds(dim: int, vdim: int) -> int:
     return 4 * (dim * vdim + 8 * (2 * dim + 2 * vdim) + 2 * (256 // lj) * vdim)
 
 
-# average new tokens per sequence from which the chunk-parallel kernels run (us token by token / in chunks for 8 heads of 64 x 128;
-# 16 of 128 x 128): one sequence of 8 tokens 26 / 27; 34 / 35, of 16 tokens 47 / 27; 62 / 36; 24 sequences of 8 tokens
-# 27 / 42; 43 / 79, of 16 tokens 48 / 43; 75 / 81
-RETENTION_CHUNK_MIN = 9
+def retention_in_chunks(T: int, S: int, heads: int, longest: Optional[int]) -> bool:
+    """Do the chunk-parallel kernels run?  Token by token a token costs 2.6 us of a chain that all sequences walk side by side; in chunks
+    three launches, and up to 0.1 us for every (sequence, head), whose last chunk is padded to 64 tokens, until the chip is as full
+    either way.  us token by token / in chunks, 8 heads of 64 x 128; 16 of 128 x 128: one sequence of 8 tokens 25 / 29; 31 / 41, of
+    16 47 / 29; 51 / 42; 24 sequences of 16 47 / 43; 63 / 85, of 32 90 / 54; 113 / 93; 64 of 24 75 / 86; 167 / 181, of 32 101 / 92;
+    214 / 186; 200 tokens beside 31 single ones 543 / 57; 602 / 125."""
+    return longest_portion(T, S, longest) >= min(28, 10 + S * heads / 24)
 
 
 def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen, ctx,
-              rows, chunked: Optional[bool] = None) -> torch.Tensor:
+              rows, chunked: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
     """``chunked`` (GPU): the chunk-parallel kernel (prompt portions) or the token-by-token one
     (decode steps); default by the step's tokens per sequence.  Same results either way."""
     ext = _native(qkvg)
@@ -130,7 +141,7 @@ def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, posi
                              ctx, rows)
     out = torch.empty((qkvg.shape[0], heads * vdim), dtype=qkvg.dtype, device=qkvg.device)      # rows of no sequence become zeros
     if chunked is None:
-        chunked = qkvg.shape[0] >= RETENTION_CHUNK_MIN * qstart.numel()
+        chunked = retention_in_chunks(qkvg.shape[0], qstart.numel(), heads, longest)
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
         chunked = True      # the token-by-token kernel keeps the whole [dim, vdim] state in LDS
     raw = torch.empty((qkvg.shape[0], heads, vdim), dtype=torch.float32, device=qkvg.device) if chunked else None
@@ -596,7 +607,7 @@ def softcap(x: torch.Tensor, cap: float) -> torch.Tensor:
 # ----------------------------------------------------------------------------- lightning attention, gated delta rule
 
 def lightning_attention(qkvg, heads, dim, vdim, decay, state, eps, norm_w, qstart, qlen, ctx, rows,
-                        chunked: Optional[bool] = None) -> torch.Tensor:
+                        chunked: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
     """Decayed linear attention over SiLU'd q, k, v (no rotation, no key scale); a token's heads are
     normed together and gated by a sigmoid.  Runs the retention kernels (token by token for decode
     steps, chunked for prompt portions) in their raw-output form, then one norm-and-gate launch."""
@@ -606,7 +617,7 @@ def lightning_attention(qkvg, heads, dim, vdim, decay, state, eps, norm_w, qstar
     T = qkvg.shape[0]
     out = torch.empty((T, heads * vdim), dtype=qkvg.dtype, device=qkvg.device)     # the finish kernel writes every row
     if chunked is None:
-        chunked = T >= RETENTION_CHUNK_MIN * qstart.numel()
+        chunked = retention_in_chunks(T, qstart.numel(), heads, longest)
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
         chunked = True
     raw = torch.empty((T, heads, vdim), dtype=torch.float32, device=qkvg.device)    # read for live tokens only
@@ -623,25 +634,25 @@ def conv_state_refill(x, conv_state, qstart, qlen, ctx, rows) -> None:
     ext.conv_state_refill(x, conv_state, qstart, qlen, ctx, rows)
 
 
-# average new tokens per sequence from which tiles of 16 tokens run (heads of 128 x 128, three launches against two): 24 sequences
-# of 32 tokens 54 against 66 us for 16 heads, 39 against 43 for 8; one sequence of 64 tokens 23 against 27, 256 tokens 45
-# against 80; below, a tile is mostly padding
+# tokens of the longest portion from which tiles of 16 tokens run (heads of 128 x 128, three launches against two; us token by token /
+# in tiles, 16 heads): one sequence of 32 tokens 17.7 / 19.4, of 64 27 / 23; 24 sequences of 8 tokens 35 / 35, of 32 63 / 55; 200 tokens
+# beside 31 single ones 78 / 47
 DELTA_TILE_MIN = 32
 
 
 def delta_rule(qkv, gba, heads, kv_heads, dim, vdim, neg_a, dt_bias, norm_w, eps, state, qstart, qlen, ctx,
-               rows, tiled: Optional[bool] = None) -> torch.Tensor:
+               rows, tiled: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
     """Gated delta rule over convolved q | k | v with the gate, beta and decay logits in ``gba``;
     unit q / k, decay, beta, the state [slots, heads, vdim, dim] and the per-head output norm in f32.
-    ``tiled`` (GPU): 16 tokens at a time (dim <= 128) or token by token; default by the step's tokens
-    per sequence."""
+    ``tiled`` (GPU): 16 tokens at a time (dim <= 128) or token by token; default by the tokens of the step's
+    ``longest`` portion."""
     ext = _native(qkv)
     if ext is None:
         return ref.delta_rule(qkv, gba, heads, kv_heads, dim, vdim, neg_a, dt_bias, norm_w, eps, state, qstart, qlen,
                               ctx, rows)
     out = torch.empty((qkv.shape[0], heads * vdim), dtype=qkv.dtype, device=qkv.device)     # the finish kernel writes every row
     if tiled is None:
-        tiled = qkv.shape[0] >= DELTA_TILE_MIN * qstart.numel()
+        tiled = longest_portion(qkv.shape[0], qstart.numel(), longest) >= DELTA_TILE_MIN
     ext.delta_rule(qkv, gba, int(heads), int(kv_heads), int(dim), int(vdim), neg_a, dt_bias, norm_w, float(eps), state,
                    qstart, qlen, ctx, rows, out, bool(tiled))
     return out

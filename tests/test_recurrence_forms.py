@@ -1,0 +1,62 @@
+"""Which form of a recurrence a step runs: a long portion is walked in chunks whatever single tokens share its step."""
+import types
+
+import torch
+
+from distributed_llm_amd.models.hybrid import HybridModel
+from distributed_llm_amd.ops import seqmix
+
+
+def forms(lens, heads=8):
+    T, S, n = sum(lens), len(lens), HybridModel._longest(types.SimpleNamespace(host_qlen=lens))
+    return seqmix.scan_in_chunks(T, S, n), seqmix.retention_in_chunks(T, S, heads, n), seqmix.longest_portion(T, S, n) >= seqmix.DELTA_TILE_MIN
+
+
+def test_mixed_steps():
+    assert forms([2000] + [20] * 23) == (True, True, True)
+    assert forms([200] + [1] * 31) == (False, True, True)          # a scan of 200 tokens costs less than the others' chunks
+    assert forms([200]) == (True, True, True)
+    assert forms([20] + [1] * 31, 16) == (False, False, False)
+    assert forms([160] * 24) == (True, True, True)
+
+
+def test_without_the_portions():
+    """A caller that does not say: the average.  No sequence, no new token: no chunks."""
+    assert seqmix.longest_portion(240, 24, None) == 10 and seqmix.longest_portion(0, 0, None) == 0
+    assert not seqmix.scan_in_chunks(2400, 24, None) and seqmix.scan_in_chunks(4800, 24, None)
+    assert HybridModel._longest(types.SimpleNamespace(host_qlen=None)) == 1 == HybridModel._longest(types.SimpleNamespace(host_qlen=[1, 0]))
+
+
+def test_layers_say_their_longest_portion(monkeypatch):
+    """Every recurrent mixer hands the step's longest portion to its op."""
+    seen = []
+
+    def op(name):
+        def f(*a, **k):
+            seen.append((name, k["longest"]))
+            raise StopIteration
+        return f
+
+    for name in ("selective_scan", "retention", "lightning_attention", "delta_rule"):
+        monkeypatch.setattr(seqmix, name, op(name))
+    for name in ("causal_conv_silu", "conv_state_refill", "paged_gqa_attention", "rope_prep", "attn_prep"):
+        monkeypatch.setattr(seqmix, name, lambda *a, **k: torch.zeros(33, 4096))
+    monkeypatch.setattr("distributed_llm_amd.models.hybrid._mm", lambda x, w: torch.zeros(33, 4096))
+    meta = types.SimpleNamespace(host_qlen=[31, 1, 1], qstart=None, qlen=None, ctx=None, state_rows=None)
+    model = HybridModel.__new__(HybridModel)
+    model.cfg = types.SimpleNamespace(rms_eps=1e-6)
+    model._any_table = lambda: None
+    m = types.SimpleNamespace(heads=2, kv_heads=2, dim=4, vdim=4, dt_rank=4, rot=None, inner=4, state=4)
+
+    class Any(dict):
+        def __missing__(self, k):
+            return torch.zeros(1)
+
+    for run in (lambda: model._mamba(Any(), m, torch.zeros(33, 8), meta, (None, None)),
+                lambda: model._retention(Any(), m, torch.zeros(33, 8), None, meta, (None,)),
+                lambda: model._delta(Any(), m, torch.zeros(33, 8), meta, (None, None))):
+        try:
+            run()
+        except StopIteration:
+            pass
+    assert seen == [("selective_scan", 31), ("retention", 31), ("delta_rule", 31)]
