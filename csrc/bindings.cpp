@@ -1585,7 +1585,7 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
   // rows of no sequence become zeros: in the step kernel, else here
   const auto clear = [&] { ok(dllm_zero_free_rows(out.data_ptr(), f ? 4 : 2, T, C, m.qstart, m.qlen, m.S, stream()), "zero_free_rows"); };
   const bool step = m.S > 0 && !chunked && dllm_scan_step_ok(T, m.S, N, ssm.data_ptr(), A.data_ptr());
-  if (step || (ns > 0 && ns <= (1L << 30))) {      // decode steps, or the chunk-parallel form (prompt portions)
+  if (step || ns > 0) {      // decode steps, or the chunk-parallel form (prompt portions)
     torch::Tensor sc;
     if (!step) {
       clear();
@@ -1607,7 +1607,7 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
 }
 
 // Chunk states of the chunk-parallel recurrences (chunk_scan.hip) for a step of T tokens and S sequences; undefined
-// where the key width is past 128 or the states would pass 4 GB (a step of several hundred thousand tokens).
+// where the key width is past 128, there is nothing to do, or one head's states would pass 4 GB (a step of millions of tokens).
 static torch::Tensor chunk_scratch(int64_t T, int S, int64_t H, int64_t d, int64_t dv, const torch::Tensor& like) {
   const long n = dllm_chunk_scan_scratch((long)T, S, (int)H, (int)d, (int)dv);
   if (n <= 0 || n > (1L << 30)) return {};

@@ -43,12 +43,15 @@ template <> __device__ __forceinline__ float ldf<float>(const float* p) { return
 
 constexpr int CS_L = 64;      // tokens per chunk
 constexpr int CS_VC = 128;    // value columns per workgroup, at most
+constexpr long CS_SCRATCH = 1L << 26;      // entries of chunk states (256 MB) up to which all heads go at once; else some at a time:
+                                           // 16 heads of 128 x 128 from 16000 tokens on, where one head's chunks fill the chip
 
 struct ScanArgs {
   const void *q, *k, *v;      // column 0 of the first head's q / k / v rows
   long ld, ldv;               // row strides of q and k, of v
   int kdiv;                   // heads per q / k head
   int H, d, dv, S;
+  int h0, HC;                 // first head of the launch, heads that the scratch holds
   // retention / lightning
   const float *cos_sin, *decay;
   int tab_w, rot, act;
@@ -58,7 +61,7 @@ struct ScanArgs {
   long ld_g;
   const float *dt_bias, *neg_a, *D;
   const int *qstart, *qlen, *ctx, *rows;
-  float *state, *chunks, *ends, *out;      // state slots; [chunks][H][d][dv], [chunks][H] A_end (ssd); out [T, H, dv]
+  float *state, *chunks, *ends, *out;      // state slots; [chunks][HC][d][dv], [chunks][HC] A_end (ssd); out [T, H, dv]
   int nchunks;
   int vec, rotvec;            // rows, head offsets and widths allow four elements at a time; so do rotation and its table
 };
@@ -220,7 +223,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
   __shared__ float wt[CS_L];
   int s, c;
   if (!dllm::find_chunk<CS_L>(a.qlen, a.S, blockIdx.x, s, c)) return;
-  const int h = blockIdx.y, v0 = blockIdx.z * CS_VC;
+  const int h = a.h0 + blockIdx.y, v0 = blockIdx.z * CS_VC;
   const int n = a.qlen[s], t0 = c * CS_L, nt = min(CS_L, n - t0), tok0 = a.qstart[s] + t0, p0 = a.ctx[s] - n + t0;
   float* Ks = sm;                    // [L][KS]: keys times their weight
   float* Vs = sm + CS_L * KS;        // [L][VS]
@@ -233,7 +236,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
       ssd_gates<T>(a, h, tok0, nt, dt, sum);
       const double end = __shfl(sum, 63);
       wt[lane] = dt * expf((float)(end - sum));
-      if (lane == 0 && v0 == 0) a.ends[(long)blockIdx.x * a.H + h] = expf((float)end);
+      if (lane == 0 && v0 == 0) a.ends[(long)blockIdx.x * a.HC + blockIdx.y] = expf((float)end);
     } else {
       wt[lane] = lane < nt ? powf(a.decay[h], (float)(nt - 1 - lane)) : 0.f;
     }
@@ -263,7 +266,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
         for (int j = 0; j < NC; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i], vb[j], acc[i][j], 0, 0, 0);
     }
   }
-  float* u = a.chunks + ((long)blockIdx.x * a.H + h) * a.d * a.dv;
+  float* u = a.chunks + ((long)blockIdx.x * a.HC + blockIdx.y) * a.d * a.dv;
 #pragma unroll
   for (int i = 0; i < NR; ++i)
 #pragma unroll
@@ -279,7 +282,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
 template <bool SSD, typename V>
 __global__ void __launch_bounds__(256) chunk_carry_kernel(ScanArgs a) {
   constexpr int W = sizeof(V) / 4, AHEAD = 4;
-  const int s = blockIdx.z, h = blockIdx.y;
+  const int s = blockIdx.z, hc = blockIdx.y, h = a.h0 + hc;
   const int n = a.qlen[s];
   if (n <= 0) return;
   const int first = dllm::chunks_before<CS_L>(a.qlen, s);
@@ -287,8 +290,8 @@ __global__ void __launch_bounds__(256) chunk_carry_kernel(ScanArgs a) {
   const long per = (long)a.d * a.dv, e = ((long)blockIdx.x * 256 + threadIdx.x) * W;
   if (e >= per) return;
   V* st = reinterpret_cast<V*>(a.state + ((long)a.rows[s] * a.H + h) * per + e);
-  V* u = reinterpret_cast<V*>(a.chunks + ((long)first * a.H + h) * per + e);
-  const long step = (long)a.H * per / W;
+  V* u = reinterpret_cast<V*>(a.chunks + ((long)first * a.HC + hc) * per + e);
+  const long step = (long)a.HC * per / W;
   const float dec = SSD ? 0.f : a.decay[h], full = SSD ? 0.f : powf(dec, (float)CS_L);
   V S = {};
   if (a.ctx[s] - n > 0) S = *st;
@@ -299,7 +302,7 @@ __global__ void __launch_bounds__(256) chunk_carry_kernel(ScanArgs a) {
     for (int j = 0; j < AHEAD; ++j) {
       const int c = min(c0 + j, nc - 1);
       x[j] = u[c * step];
-      if constexpr (SSD) g[j] = a.ends[(long)(first + c) * a.H + h];
+      if constexpr (SSD) g[j] = a.ends[(long)(first + c) * a.HC + hc];
       else g[j] = (c + 1) * CS_L <= n ? full : powf(dec, (float)(n - c * CS_L));
     }
 #pragma unroll
@@ -322,7 +325,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   __shared__ double lg[CS_L];          // ssd: sums of log decays
   int s, c;
   if (!dllm::find_chunk<CS_L>(a.qlen, a.S, blockIdx.x, s, c)) return;
-  const int h = blockIdx.y, v0 = blockIdx.z * CS_VC;
+  const int h = a.h0 + blockIdx.y, v0 = blockIdx.z * CS_VC;
   const int n = a.qlen[s], t0 = c * CS_L, nt = min(CS_L, n - t0), tok0 = a.qstart[s] + t0, p0 = a.ctx[s] - n + t0;
   float* Ks = sm;                      // [L][KS], then the state [KD][VS] from the start of sm
   float* Vs = sm + CS_L * KS;          // [L][VS]
@@ -399,7 +402,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   }
   if (c > 0 || p0 > 0) {      // (the same for the whole workgroup) a sequence starts from a zero state
     __syncthreads();
-    const float* st = a.chunks + ((long)blockIdx.x * a.H + h) * a.d * a.dv + v0;
+    const float* st = a.chunks + ((long)blockIdx.x * a.HC + blockIdx.y) * a.d * a.dv + v0;
     constexpr int IT = KD * NV / 64, U = IT < 8 ? IT : 8;
     if (a.dv % 4 == 0) {
       const int n = min(a.dv - v0, CS_VC);
@@ -449,7 +452,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   }
 }
 
-template <typename T, bool SSD, int KD, int NV> void launch_tiles(const ScanArgs& a, hipStream_t st) {
+template <typename T, bool SSD, int KD, int NV> void launch_tiles(ScanArgs a, hipStream_t st) {
   constexpr int lds = 4 * CS_L * (KD + 4 + 16 * NV + 4);
   static const bool set_ = [] {      // raised once: no attribute call inside a later stream capture
     (void)hipFuncSetAttribute((const void*)chunk_sum_kernel<T, KD, NV, SSD>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -457,14 +460,17 @@ template <typename T, bool SSD, int KD, int NV> void launch_tiles(const ScanArgs
     return true;
   }();
   (void)set_;
-  const dim3 g(a.nchunks, a.H, (a.dv + CS_VC - 1) / CS_VC);
-  hipLaunchKernelGGL((chunk_sum_kernel<T, KD, NV, SSD>), g, dim3(256), lds, st, a);
   const long per = (long)a.d * a.dv;
-  if (per % 4 == 0 && (uintptr_t)a.state % 16 == 0 && (uintptr_t)a.chunks % 16 == 0)
-    hipLaunchKernelGGL((chunk_carry_kernel<SSD, f32x4>), dim3((unsigned)((per / 4 + 255) / 256), a.H, a.S), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((chunk_carry_kernel<SSD, float>), dim3((unsigned)((per + 255) / 256), a.H, a.S), dim3(256), 0, st, a);
-  hipLaunchKernelGGL((chunk_out_kernel<T, KD, NV, SSD>), g, dim3(256), lds, st, a);
+  for (a.h0 = 0; a.h0 < a.H; a.h0 += a.HC) {      // the stream keeps one group's launches ahead of the next's writes
+    const int n = a.HC < a.H - a.h0 ? a.HC : a.H - a.h0;
+    const dim3 g(a.nchunks, n, (a.dv + CS_VC - 1) / CS_VC);
+    hipLaunchKernelGGL((chunk_sum_kernel<T, KD, NV, SSD>), g, dim3(256), lds, st, a);
+    if (per % 4 == 0 && (uintptr_t)a.state % 16 == 0 && (uintptr_t)a.chunks % 16 == 0)
+      hipLaunchKernelGGL((chunk_carry_kernel<SSD, f32x4>), dim3((unsigned)((per / 4 + 255) / 256), n, a.S), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((chunk_carry_kernel<SSD, float>), dim3((unsigned)((per + 255) / 256), n, a.S), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((chunk_out_kernel<T, KD, NV, SSD>), g, dim3(256), lds, st, a);
+  }
 }
 
 template <typename T, bool SSD> int launch_chunks(const ScanArgs& a, hipStream_t st) {
@@ -485,11 +491,17 @@ template <typename T> int vec_ok(const ScanArgs& a) {
          (uintptr_t)a.k % bytes == 0 && (uintptr_t)a.v % bytes == 0;
 }
 
+int heads_at_once(long nchunks, int H, int d, int dv) {
+  const long n = CS_SCRATCH / (nchunks * ((long)d * dv + 1));
+  return n < 1 ? 1 : n < H ? (int)n : H;
+}
+
 template <bool SSD> int run_chunks(ScanArgs& a, int f32, long T, float* scratch, hipStream_t st) {
   if (a.d < 1 || a.d > 128 || a.dv < 1 || a.S < 1 || T < 1) return -1;
   a.nchunks = (int)(T / CS_L) + a.S;
+  a.HC = heads_at_once(a.nchunks, a.H, a.d, a.dv);
   a.chunks = scratch;
-  a.ends = scratch + (long)a.nchunks * a.H * a.d * a.dv;
+  a.ends = scratch + (long)a.nchunks * a.HC * a.d * a.dv;
   a.rotvec = a.rot % 8 == 0 && a.tab_w % 4 == 0 && (uintptr_t)a.cos_sin % 16 == 0;
   if (f32) {
     a.vec = vec_ok<float>(a);
@@ -503,8 +515,9 @@ template <bool SSD> int run_chunks(ScanArgs& a, int f32, long T, float* scratch,
 
 // f32 entries of scratch for a step of T tokens and S sequences; 0: the width is not taken
 extern "C" long dllm_chunk_scan_scratch(long T, int S, int H, int d, int dv) {
-  if (d < 1 || d > 128) return 0;
-  return (T / CS_L + S) * (long)H * ((long)d * dv + 1);
+  if (d < 1 || d > 128 || T / CS_L + S < 1) return 0;
+  const long nc = T / CS_L + S;
+  return nc * heads_at_once(nc, H, d, dv) * ((long)d * dv + 1);
 }
 
 // qkvg [T, q | k | v | ..]: q and k rotated, k times kscale, or with act all three SiLU'd; out [T, H, dv] f32

@@ -59,6 +59,8 @@ __device__ __forceinline__ float silu_f(float z) { return z / (1.f + expf(-z)); 
 
 constexpr int SC_L = 32;      // tokens per chunk
 constexpr int SC_AHEAD = 8;   // tokens whose inputs are in flight
+constexpr long SC_SCRATCH = 1L << 26;     // entries of chunk ends (256 MB) up to which all channels go at once; else some at a time: 2048
+                                          // channels of 16 states from 61000 tokens on
 
 template <typename T> struct MambaArgs {
   const T *xc, *dt_raw, *dbc, *xz;
@@ -71,7 +73,8 @@ template <typename T> struct MambaArgs {
   const int *qstart, *qlen, *ctx, *rows;
   T* out;
   int S, C, N, nchunks;
-  float *ends, *steps;      // [chunks][N][C], [chunks][C]
+  int c0, CC;               // first channel of the launch, channels that the scratch holds
+  float *ends, *steps;      // [chunks][N][CC], [chunks][CC]
   long tokens;
 };
 
@@ -89,15 +92,15 @@ __global__ void __launch_bounds__(256) scan_chunk_kernel(MambaArgs<T> a) {
     bc[e] = t < nt && i < a.N ? ldf(a.dbc + (tok0 + t) * a.ldd + a.dt_rank + (k < NP ? 0 : a.N) + i) : 0.f;
   }
   __syncthreads();
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= a.C) return;
+  const int cc = blockIdx.x * 256 + threadIdx.x, c = a.c0 + cc;
+  if (cc >= a.CC || c >= a.C) return;
   float A[NP], S[NP];
-  float* ends = a.ends + (long)blockIdx.y * a.N * a.C + c;
+  float* ends = a.ends + (long)blockIdx.y * a.N * a.CC + cc;
   const bool carried = OUT && (ch > 0 || p0 > 0);
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
     A[i] = i < a.N ? Decay<T>::pre(a.A[(long)c * a.N + i]) : 0.f;
-    S[i] = carried && i < a.N ? ends[(long)i * a.C] : 0.f;
+    S[i] = carried && i < a.N ? ends[(long)i * a.CC] : 0.f;
   }
   const float dtb = a.dt_bias[c], skip = OUT ? a.D[c] : 0.f;
   float sum = 0.f;
@@ -138,8 +141,8 @@ __global__ void __launch_bounds__(256) scan_chunk_kernel(MambaArgs<T> a) {
   if constexpr (!OUT) {
 #pragma unroll
     for (int i = 0; i < NP; ++i)
-      if (i < a.N) ends[(long)i * a.C] = S[i];
-    a.steps[(long)blockIdx.y * a.C + c] = sum;
+      if (i < a.N) ends[(long)i * a.CC] = S[i];
+    a.steps[(long)blockIdx.y * a.CC + cc] = sum;
   } else if (t0 + nt == n && a.Km1 > 0) {
     // the last K-1 inputs of the sequence: new tokens where there are enough, else the slot's older ones
     T* cs = a.conv + (long)a.rows[s] * a.Km1 * a.C + c;
@@ -161,11 +164,11 @@ template <typename T> __global__ void __launch_bounds__(256) scan_carry_kernel(M
   if (n <= 0) return;
   const int first = dllm::chunks_before<SC_L>(a.qlen, s);
   const int nc = min((n + SC_L - 1) / SC_L, a.nchunks - first);
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= a.C) return;
+  const int cc = blockIdx.x * 256 + threadIdx.x, c = a.c0 + cc;
+  if (cc >= a.CC || c >= a.C) return;
   float* st = a.ssm + ((long)a.rows[s] * a.C + c) * a.N + i;
-  float* u = a.ends + ((long)first * a.N + i) * a.C + c;
-  const float* d = a.steps + (long)first * a.C + c;
+  float* u = a.ends + ((long)first * a.N + i) * a.CC + cc;
+  const float* d = a.steps + (long)first * a.CC + cc;
   const float A = a.A[(long)c * a.N + i];
   float S = a.ctx[s] - n > 0 ? *st : 0.f;
   for (int c0 = 0; c0 < nc; c0 += AHEAD) {
@@ -173,13 +176,13 @@ template <typename T> __global__ void __launch_bounds__(256) scan_carry_kernel(M
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
       const long k = min(c0 + j, nc - 1);
-      x[j] = u[k * a.N * a.C];
-      g[j] = d[k * a.C];
+      x[j] = u[k * a.N * a.CC];
+      g[j] = d[k * a.CC];
     }
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) {
       if (c0 + j >= nc) break;
-      u[(long)(c0 + j) * a.N * a.C] = S;
+      u[(long)(c0 + j) * a.N * a.CC] = S;
       S = expf(A * g[j]) * S + x[j];
     }
   }
@@ -259,11 +262,19 @@ template <typename T, int NP> __global__ void __launch_bounds__(64) scan_step_ke
     if (k < a.Km1) cs[(long)k * a.C] = cv[k];
 }
 
-template <typename T, int NP> void launch(const MambaArgs<T>& a, hipStream_t st) {
-  const dim3 g((a.C + 255) / 256, a.nchunks), b(256);
-  hipLaunchKernelGGL((scan_chunk_kernel<T, NP, false>), g, b, 0, st, a);
-  hipLaunchKernelGGL(scan_carry_kernel<T>, dim3((a.C + 255) / 256, a.N, a.S), b, 0, st, a);
-  hipLaunchKernelGGL((scan_chunk_kernel<T, NP, true>), g, b, 0, st, a);
+template <typename T, int NP> void launch(MambaArgs<T> a, hipStream_t st) {
+  for (a.c0 = 0; a.c0 < a.C; a.c0 += a.CC) {      // the stream keeps one group's launches ahead of the next's writes
+    const int n = ((a.CC < a.C - a.c0 ? a.CC : a.C - a.c0) + 255) / 256;
+    const dim3 g(n, a.nchunks), b(256);
+    hipLaunchKernelGGL((scan_chunk_kernel<T, NP, false>), g, b, 0, st, a);
+    hipLaunchKernelGGL(scan_carry_kernel<T>, dim3(n, a.N, a.S), b, 0, st, a);
+    hipLaunchKernelGGL((scan_chunk_kernel<T, NP, true>), g, b, 0, st, a);
+  }
+}
+
+int channels_at_once(long nchunks, int C, int N) {
+  const long n = SC_SCRATCH / (nchunks * (N + 1L)) / 256 * 256;
+  return n < 256 ? (C < 256 ? C : 256) : n < C ? (int)n : C;
 }
 
 template <typename T>
@@ -271,7 +282,7 @@ int run(const void* xc, const void* dt_raw, const float* dt_bias, const float* A
         const float* D, const void* xz, long ldz, float* ssm, void* conv, int Km1, const int* qstart, const int* qlen,
         const int* ctx, const int* rows, void* out, int S, long tokens, int C, int N, float* scratch, hipStream_t st) {
   MambaArgs<T> a{(const T*)xc, (const T*)dt_raw, (const T*)dbc, (const T*)xz, ldd, ldz, dt_rank, dt_bias, A, D, ssm, (T*)conv,
-                 Km1, qstart, qlen, ctx, rows, (T*)out, S, C, N, (int)(tokens / SC_L) + S, scratch, nullptr, tokens};
+                 Km1, qstart, qlen, ctx, rows, (T*)out, S, C, N, (int)(tokens / SC_L) + S, 0, C, scratch, nullptr, tokens};
   if (!scratch) {
     const dim3 g((C + 63) / 64, S + 1);
     if (N <= 8) hipLaunchKernelGGL((scan_step_kernel<T, 8>), g, dim3(64), 0, st, a);
@@ -279,7 +290,8 @@ int run(const void* xc, const void* dt_raw, const float* dt_bias, const float* A
     else hipLaunchKernelGGL((scan_step_kernel<T, 32>), g, dim3(64), 0, st, a);
     return (int)hipGetLastError();
   }
-  a.steps = scratch + (long)a.nchunks * N * C;
+  a.CC = channels_at_once(a.nchunks, C, N);
+  a.steps = scratch + (long)a.nchunks * N * a.CC;
   if (a.nchunks > 65535) return -3;
   if (N <= 8) launch<T, 8>(a, st);
   else if (N <= 16) launch<T, 16>(a, st);
@@ -293,7 +305,7 @@ int run(const void* xc, const void* dt_raw, const float* dt_bias, const float* A
 // chunks than a grid's second dimension)
 extern "C" long dllm_scan_chunks_scratch(long T, int S, int C, int N) {
   const long nc = T / SC_L + S;
-  return N < 1 || N > 32 || nc > 65535 ? 0 : nc * C * (N + 1L);
+  return N < 1 || N > 32 || nc < 1 || nc > 65535 ? 0 : nc * channels_at_once(nc, C, N) * (N + 1L);
 }
 
 // May the step kernel take it?  Steps of at most four tokens a sequence on average (2048 channels of 16 states, us with a thread /
