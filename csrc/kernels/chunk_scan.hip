@@ -515,7 +515,7 @@ template <bool SSD> int run_chunks(ScanArgs& a, int f32, long T, float* scratch,
 
 // f32 entries of scratch for a step of T tokens and S sequences; 0: the width is not taken
 extern "C" long dllm_chunk_scan_scratch(long T, int S, int H, int d, int dv) {
-  if (d < 1 || d > 128 || T / CS_L + S < 1) return 0;
+  if (d < 1 || d > 128 || dv < 1 || T < 1 || S < 1) return 0;
   const long nc = T / CS_L + S;
   return nc * heads_at_once(nc, H, d, dv) * ((long)d * dv + 1);
 }

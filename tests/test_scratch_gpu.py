@@ -58,3 +58,12 @@ def test_scan():
         z = seqmix.selective_scan(xc[:, c].contiguous(), raw[:, c].contiguous(), b[c], A[c], dbc, R, D[c],
                                   torch.cat([xz[:, c], xz[:, C + c0:C + c0 + 256]], 1), s1, v1, *m)
         assert torch.equal(z, y[:, c]) and torch.equal(s1, st[:, c]) and torch.equal(v1, cv[:, :, c])
+
+
+def test_no_sequence():
+    """Tokens of no sequence only: zeros, in chunks as token by token."""
+    n = torch.zeros(0, dtype=torch.int32, device=DEV)
+    H, dv, N = 2, 32, 16
+    xbc, proj, v = torch.randn(130, H * dv + 2 * N, device=DEV), torch.randn(130, H, device=DEV), torch.ones(H, device=DEV)
+    for chunked in (False, True):
+        assert not seqmix.ssd_scan(xbc, proj, 0, H, dv, N, 1, v, -v, v, torch.zeros(1, H, N, dv, device=DEV), n, n, n, n, chunked=chunked).any()
