@@ -111,9 +111,12 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
 
   constexpr int STEP = 512;  // K elements per wave-instruction
   constexpr int TRIP = STEP * UNR;
-  uint4 w[UNR][R], wn[UNR][R];
+  // XG of 12 loads a row: K is one trip and the grid every block, so there is no next trip to keep: with its registers (256 and
+  // AGPRs) a wave had a SIMD to itself, and two workgroups a CU lost what the loads gain; without (100 at R 1) four share one
+  constexpr bool ONE = XG && UNR == 12;
+  uint4 w[UNR][R], wn[ONE ? 1 : UNR][R];
   // XG (batch 1, plain X): X travels with W in every trip (L1/L2 hits, no LDS stage, no barrier)
-  uint4 xg[XG ? UNR : 1][XG ? M : 1], xgn[XG ? UNR : 1][XG ? M : 1];
+  uint4 xg[XG ? UNR : 1][XG ? M : 1], xgn[XG && !ONE ? UNR : 1][XG ? M : 1];
 #define DLLM_GEMV_LOAD(DST, XDST, KB, ROWS, ACT)                                                     \
   _Pragma("unroll") for (int u = 0; u < UNR; ++u) {                                                 \
     const int k_ = (KB) + u * STEP + 8 * lane;                                                      \
@@ -216,10 +219,12 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
     for (int r = 0; r < R; ++r) acc[m][r] = 0.f;
   for (int kb = 0; kb < K; kb += TRIP) {
     // next trip in flight during this one: this block's, else the next block's first
-    if (kb + TRIP < K) {
-      DLLM_GEMV_LOAD(wn, xgn, kb + TRIP, wr, active)
-    } else if (vn < nvb) {
-      DLLM_GEMV_LOAD(wn, xgn, 0, wrn, activen)
+    if constexpr (!ONE) {
+      if (kb + TRIP < K) {
+        DLLM_GEMV_LOAD(wn, xgn, kb + TRIP, wr, active)
+      } else if (vn < nvb) {
+        DLLM_GEMV_LOAD(wn, xgn, 0, wrn, activen)
+      }
     }
 #pragma unroll
     for (int u = 0; u < UNR; ++u) {
@@ -244,13 +249,16 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
         }
       }
     }
+    if constexpr (ONE) break;
+    else {
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
+      for (int u = 0; u < UNR; ++u) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) w[u][r] = wn[u][r];
-      if constexpr (XG) {
+        for (int r = 0; r < R; ++r) w[u][r] = wn[u][r];
+        if constexpr (XG) {
 #pragma unroll
-        for (int m = 0; m < M; ++m) xg[u][m] = xgn[u][m];
+          for (int m = 0; m < M; ++m) xg[u][m] = xgn[u][m];
+        }
       }
     }
   }
@@ -337,7 +345,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
     }
     if (vn < nvb) __syncthreads();  // s_ep is rewritten by the next block (uniform condition)
   }
-  if (vn >= nvb) break;
+  if (ONE || vn >= nvb) break;
   vb = vn;
   n0 = n0n;
   active = activen;
@@ -384,11 +392,11 @@ void launch_gemv(const void* x, long ldx, const void* w, void* y, long ldy, int 
   // Llama-3-8B's, never slower; at batch 2 it is slower on the large shapes, so batch 1 only.
   if constexpr (M == 1 && !SW && !NORM) {
     const size_t lds_xg = EPI != GV_PLAIN ? (size_t)(M + 4 * R * M + 4 * M) * sizeof(float) : 0;
-    // Long rows on up to a workgroup per CU: a wave's whole rows (up to 12 loads a row) in flight, where 4 a trip wait out three
-    // latencies.  us with 12 / 4: 2048 x 5632 at R 2 6.5 / 7.6 (the best before, R 1: 7.0), 2048 x 4096 6.0 / 6.2, 1024 x 4096 at
-    // R 1 4.4 / 4.8; two workgroups a CU or four rows a wave lose (2048 x 5632 at R 1 7.9 / 7.0, 4096 x 4096 at R 2 10.2 / 8.5).
+    // Long rows: a wave's whole rows (up to 12 loads a row) in flight, where 4 a trip wait out three latencies.  us with 12 / 4 at R 1;
+    // R 2: 1024 x 4096 4.0 / 4.4; 4.4 / 5.0, 2048 x 5632 6.6 / 7.7; 6.7 / 7.9, 4096 x 4096 8.1 / 8.5; 9.2 / 8.7 (the one loss of
+    // 13 shapes), 8192 x 2560 9.4 / 10.3; 10.0 / 10.8, 8192 x 5632 15.7 / 17.5; 16.2 / 17.4.  Four rows a wave do not fit the registers.
     if constexpr (R <= 2) {
-      if (K > 2048 && K <= 6144 && gemv_blocks<R>(N) <= 256) {
+      if (K > 2048 && K <= 6144) {
         hipLaunchKernelGGL((gemv_kernel<M, R, 12, SW, NORM, EPI, true>), dim3(gemv_blocks<R>(N)), dim3(256), lds_xg, stream,
                            (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, N, K, na, ea);
         return;
