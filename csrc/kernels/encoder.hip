@@ -1,9 +1,9 @@
 // Router sentence encoder (MiniLM / BERT) kernels: bidirectional attention over a padded or packed batch
-// and the fused embedding sum + LayerNorm.  The projections run on tgemm.hip (bias / GELU /
-// residual epilogues); LayerNorm after each residual on norm.hip; pooling on cosine.hip.
+// the fused embedding sum + LayerNorm, and the projections of up to 64 rows (enc_gemm; more rows run on tgemm.hip, with
+// the same bias / GELU / residual epilogues).  LayerNorm after each residual is in norm.hip, pooling in elementwise.hip.
 //
 // Reference parity: the reference encodes every query with sentence-transformers
-// all-MiniLM-L6-v2 on the host (/root/reference/src/query_router_engine.py:181,571).
+// all-MiniLM-L6-v2 on the host (src/query_router_engine.py:181,571).
 //
 // encoder_attn: qkv [B*S, 3H] (row b*S + s; q | k | v, head h at columns h*D), lens [B] -> out [B*S, H].
 //   Workgroup = (64-query slice, head, sequence), 4 waves x 16 queries.  The head's K and V^T for
