@@ -28,7 +28,7 @@
 //
 // What bounds it: 16 heads of 128 x 128 over 6 x 1400 tokens are 12 GFLOP of f32 MFMA a layer (80 us at 157 TFLOP/s) and
 // 0.5 GB of chunk states (100 us at 5.2 TB/s); chunks of 128 would halve the states and need twice the LDS.  Measured
-// there (bf16 rows): sums 119, carry 53, outputs 175 us with SiLU on every row (expf and a division: 8 % of a layer).  One
+// there (bf16 rows): sums 119, carry 53, outputs 179 us with SiLU on every row (expf and a division: 8 % of a layer).  One
 // prompt of 4096 tokens, with its norm and gate: retention with 8 heads of 64 x 128 about 80 us against 1900 us
 // for chunks in order (seqmix.hip); Mamba-2 with 32 heads of 128 x 64 about 150 us against 1390 us token by token
 // (outer_scan.hip).
@@ -168,9 +168,21 @@ __device__ __forceinline__ void stage_keys(const ScanArgs& a, float* Ks, const T
   }
 }
 
-// the chunk's values [L][16 NV + 4] from column 0 of vp, n of them in a row; rows past nt are zeros
+// Four of a token's values, rid of infinities and NaN; seen (one entry a token): 1, or NaN where the row had any.  The 4 NV threads of
+// a row are neighbours in a wave.
+template <int NV> __device__ __forceinline__ float4 finite4(float4 v, float* seen) {
+  constexpr unsigned long long row = (1ull << (4 * NV)) - 1;
+  const int lane = threadIdx.x & 63;
+  const unsigned long long bad = __ballot(!(fmaf(v.y, 0.f, v.x * 0.f) + fmaf(v.w, 0.f, v.z * 0.f) == 0.f));
+  if (lane % (4 * NV) == 0) *seen = (bad >> lane) & row ? __builtin_nanf("") : 1.f;
+  if (bad)
+    v = make_float4(v.x * 0.f == 0.f ? v.x : 0.f, v.y * 0.f == 0.f ? v.y : 0.f, v.z * 0.f == 0.f ? v.z : 0.f, v.w * 0.f == 0.f ? v.w : 0.f);
+  return v;
+}
+
+// the chunk's values [L][16 NV + 4] from column 0 of vp, n of them in a row; rows past nt are zeros.  seen: as in finite4, or null
 template <typename T, int NV>
-__device__ __forceinline__ void stage_values(const ScanArgs& a, float* Vs, const T* vp, int nt, int n) {
+__device__ __forceinline__ void stage_values(const ScanArgs& a, float* Vs, const T* vp, int nt, int n, float* seen) {
   constexpr int IT = CS_L * NV / 64, VS = 16 * NV + 4;
   if (a.vec) {
     Quad<T> x[IT];
@@ -184,14 +196,16 @@ __device__ __forceinline__ void stage_values(const ScanArgs& a, float* Vs, const
       const int e = threadIdx.x + 256 * it, t = e / (4 * NV), i = (e % (4 * NV)) * 4;
       float4 v = x[it].f();
       if (a.act) v = silu4(v);
-      *reinterpret_cast<float4*>(Vs + t * VS + i) = t < nt && i < n ? v : zero4();
+      v = t < nt && i < n ? v : zero4();
+      *reinterpret_cast<float4*>(Vs + t * VS + i) = seen ? finite4<NV>(v, seen + t) : v;
     }
   } else {
     for (int e = threadIdx.x; e < CS_L * NV * 4; e += 256) {
       const int t = e / (4 * NV), i = (e % (4 * NV)) * 4;
       float4 v = zero4();
       if (t < nt) v = ld4(vp + t * a.ldv, i, n);
-      *reinterpret_cast<float4*>(Vs + t * VS + i) = a.act ? silu4(v) : v;
+      if (a.act) v = silu4(v);
+      *reinterpret_cast<float4*>(Vs + t * VS + i) = seen ? finite4<NV>(v, seen + t) : v;
     }
   }
 }
@@ -241,7 +255,7 @@ __global__ void __launch_bounds__(256) chunk_sum_kernel(ScanArgs a) {
       wt[lane] = lane < nt ? powf(a.decay[h], (float)(nt - 1 - lane)) : 0.f;
     }
   }
-  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC));
+  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC), nullptr);
   __syncthreads();
   stage_keys<T, KD>(a, Ks, (const T*)a.k + (long)tok0 * a.ld + (long)(h / a.kdiv) * a.d, nt, p0, wt);
   __syncthreads();
@@ -323,6 +337,8 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   __shared__ float wt[CS_L + 1];       // retention: powers of the decay; ssd: steps
   __shared__ double lg[CS_L];          // ssd: sums of log decays
+  __shared__ float seen[CS_L];         // NaN: a value of the token is infinite or NaN.  It must not reach the tokens before it, whose
+                                       // zero weights it would meet, so it reaches those behind as a weight
   int s, c;
   if (!dllm::find_chunk<CS_L>(a.qlen, a.S, blockIdx.x, s, c)) return;
   const int h = a.h0 + blockIdx.y, v0 = blockIdx.z * CS_VC;
@@ -345,7 +361,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
   }
   const long kh = (long)tok0 * a.ld + (long)(h / a.kdiv) * a.d;
   stage_keys<T, KD>(a, Ks, (const T*)a.k + kh, nt, p0, nullptr);
-  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC));
+  stage_values<T, NV>(a, Vs, (const T*)a.v + (long)tok0 * a.ldv + (long)h * a.dv + v0, nt, min(a.dv - v0, CS_VC), seen);
   // the wave's queries: row lr, dims 16 b + 4 g4 ..
   const int tq = 16 * wave + lr, tl = min(tq, nt - 1);
   float4 q[NB];
@@ -390,7 +406,7 @@ __global__ void __launch_bounds__(256) chunk_out_kernel(ScanArgs a) {
     for (int x = 0; x < 4; ++x) {
       const int k = 16 * b + 4 * g4 + x;
       float w = 0.f;
-      if (k <= tq) w = SSD ? wt[k] * expf((float)(lq - lg[k])) : wt[tq - k];
+      if (k <= tq) w = (SSD ? wt[k] * expf((float)(lq - lg[k])) : wt[tq - k]) * seen[k];
       p[x] = k <= tq ? p[x] * w : 0.f;
     }
 #pragma unroll
