@@ -364,9 +364,9 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ q
 // accumulators of the last product, which are at once the right operand of S^T k and S^T q.  The waves' parts meet in LDS, a
 // thread sums one element of each, and U = (I + A)^-1 R comes out as the right operand of the state's update.  Serial over the
 // tiles, so the chain of one tile bounds it: two products, one exchange, two small products, the update.  Sums of more than four terms go in
-// parts that are added pairwise, or the largest last.  bf16, 16 heads of 128 x 128: 6 sequences of 1400 tokens 355 us with the two
-// launches beside it against 617 token by token, one of 4096 tokens 523 against 1219 (314 and 472 with one chain a sum, whose outputs
-// were up to 1.5 times as far off as token by token).  f32 errors against 64 bits over 385 tokens, state and outputs, token by token
+// parts that are added pairwise, or the largest last.  bf16, 16 heads of 128 x 128: 6 sequences of 1400 tokens 363 us with the two
+// launches beside it against 617 token by token, one of 4096 tokens 536 against 1219 (358 and 520 without the look for infinities and
+// NaN; before that, with one chain a sum, 314 and 472, with outputs up to 1.5 times as far off as token by token).  f32 errors against 64 bits over 385 tokens, state and outputs, token by token
 // in brackets: decays near 1 1.5e-7 (5.6e-7), 1.7e-7 (2.6e-7); a model's (0.01 to 0.3 a token) 1.2e-7 (1.9e-7), 1.6e-7 (1.7e-7); up
 // to 4 a token 1.0e-7 (1.05e-7), 1.53e-7 (1.49e-7).
 template <typename T, int NS, bool VL>
@@ -499,7 +499,21 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
       fetch_keys(t0 + 2 * DT_L);
     }
     __syncthreads();
-    const f32x4 r = *reinterpret_cast<const f32x4*>(Rs + lr * DT_P + 4 * g4);
+    f32x4 r = *reinterpret_cast<const f32x4*>(Rs + lr * DT_P + 4 * g4);
+    // An infinity or NaN of a token must not reach those before it, whose zeros in (I + A)^-1 and P it would meet: it leaves the
+    // products, and the column is NaN from its first such row on.
+    int lost = DT_L;
+    const bool bad = __ballot(!(fmaf(r[1], 0.f, r[0] * 0.f) + fmaf(r[3], 0.f, r[2] * 0.f) == 0.f));
+    if (bad) {
+#pragma unroll
+      for (int e = 3; e >= 0; --e)
+        if (!(r[e] * 0.f == 0.f)) {
+          lost = 4 * g4 + e;
+          r[e] = 0.f;
+        }
+      lost = min(lost, __shfl_xor(lost, 16));
+      lost = min(lost, __shfl_xor(lost, 32));
+    }
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 u4[4];
     // each of the small products as four sums: token i's own term, which steep decays leave alone, is then the last of sum i % 4 (of
@@ -511,7 +525,14 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
     f32x4 u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) u[e] = (u4[e ^ 1][e] + (u4[e ^ 2][e] + u4[e ^ 3][e])) + u4[e][e];
-    const f32x4 z = we * u;
+    f32x4 z = we * u;
+    if (bad) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        z[e] = 4 * g4 + e < lost ? z[e] : __builtin_nanf("");
+        u[e] = 4 * g4 + e < lost ? u[e] : 0.f;
+      }
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const float* kp = ks[buf] + 4 * g4 * LD + 16 * (w * NB + b) + lr;
@@ -527,6 +548,9 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
       f32x4 o = *reinterpret_cast<const f32x4*>(Os + lr * DT_P + 4 * g4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = (o[e] + (o4[e ^ 1][e] + (o4[e ^ 2][e] + o4[e ^ 3][e]))) + o4[e][e];
+      if (bad)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = 4 * g4 + e < lost ? o[e] : __builtin_nanf("");
 #pragma unroll
       for (int x = 0; x < 4; ++x)
         if (live && 4 * g4 + x < nt) raw[((long)(q0 + t0 + 4 * g4 + x) * H + h) * dv + j] = o[x];

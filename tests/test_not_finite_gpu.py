@@ -43,3 +43,24 @@ def test_chunks(act, where, value):
             return seqmix.lightning_attention(x, H, d, dv, dec, st.clone(), 1e-5, nw, qstart, qlen, ctx, rows, chunked=True)
         return seqmix.retention(x, H, d, dv, table, d, dec, st.clone(), 1e-6, pos, qstart, qlen, ctx, rows, chunked=True)
     same_before(run, x, {"q": 5, "k": H * d + 5, "v": 2 * H * d + 21}[where], value)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "beta", "decay"])
+def test_tiles(where, value):
+    torch.manual_seed(72)
+    H, G, d, dv = 2, 2, 128, 128
+    T, qstart, qlen, ctx, rows, _ = batch(QLENS, STARTS)
+    n = G * d
+    x = torch.randn(T, 2 * n + H * dv + H * dv + 2 * H, device=DEV)
+    split = 2 * n + H * dv
+    na, dtb, nw = torch.tensor([-0.1, -0.3], device=DEV), torch.zeros(H, device=DEV), torch.ones(dv, device=DEV)
+    st = torch.randn(2, H, dv, d, device=DEV)
+
+    def run(x):
+        return seqmix.delta_rule(x[:, :split].contiguous(), x[:, split:].contiguous(), H, G, d, dv, na, dtb, nw, 1e-6, st.clone(), qstart, qlen,
+                                 ctx, rows, tiled=True)
+    gba = split + H * dv
+    if where in ("beta", "decay"):
+        value = float("nan")      # infinite logits are a gate of 0 or 1
+    same_before(run, x, {"q": 5, "k": n + 5, "v": 2 * n + 21, "beta": gba, "decay": gba + H}[where], value)
