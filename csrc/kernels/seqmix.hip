@@ -7,12 +7,14 @@
 //                    the inputs before a sequence's first new token come from its state slot
 //   scan             Mamba-1 selective scan: 16 lanes per channel share its states, tokens in order;
 //                    softplus, decay, state and the output gate in f32; refills the convolution state
+//                    (short portions; decode steps and long portions run scan_chunk.hip)
 //   retention        decayed linear attention: one workgroup per (sequence, head), the [dim x vdim]
-//                    state in LDS, rotate-half positions applied while q / k are staged, unit-RMS
-//                    heads and the SiLU gate in the same launch
-//   retention_chunk  the same recurrence for prompt portions in its chunked form (32 tokens at a time:
+//                    state in registers (retention_step; in LDS for widths that are no vectors),
+//                    rotate-half positions applied while q / k are staged, unit-RMS heads and the SiLU
+//                    gate in the same launch
+//   retention_chunk  the same recurrence for prompt portions with dim > 128 (32 tokens at a time:
 //                    scores inside the chunk + the carried state), one workgroup per (head, 32 value
-//                    columns, sequence); retention_finish norms and gates
+//                    columns, sequence); other dims run chunk_scan.hip; retention_finish norms and gates
 //   resadd_norm      x (f32) += rmsnorm(y) * w with y one branch or the normed average of two, plus the
 //                    next sublayer's normed input; depth_mix: a weighted sum over the f32 stack of
 //                    layer results, plus the normed input of the next layer; gelu_erf; conv_refill
@@ -29,7 +31,8 @@
 //   glu_act          gated activations of a fused gate | up projection: SiLU gate, or clamped with
 //                    g sigmoid(alpha g) (u + 1)
 //   route_topk       group-limited top-k routing with sigmoid or softmax scores, a correction on the
-//                    choice and identity experts (group_router is its sigmoid / two-best form)
+//                    choice and identity experts (group_router is its sigmoid / two-best form);
+//                    router_topk: the f32 logits of bf16 rows and the choice in one launch
 //
 // Activations are bf16 or f32 (template T = u16 / float); every sum, state, norm and gate is f32.
 // Sequence metadata: qstart / qlen / ctx / rows per sequence (int32); a sequence with qlen 0 is

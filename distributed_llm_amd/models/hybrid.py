@@ -52,8 +52,8 @@ they do not take and for f32 models), everything between them on the HIP kernels
              alone) -> attention inside a sliding window that also keeps the first tokens, with one
              more term of score 0 in the softmax denominator -> out-proj
   clamped    one fused gate | up projection -> biases, clamps, g sigmoid(1.702 g) (u + 1) -> down-proj
-  experts    (softmax scores + a correction for the choice, identity experts) one f32 GEMM for the
-             router logits and the shared expert's gate logit -> group-limited top-k -> SwiGLU experts;
+  experts    (softmax scores + a correction for the choice, identity experts) f32 logits of the
+             router and the shared expert's gate and the group-limited top-k in one launch -> SwiGLU experts;
              identity experts, the gated shared expert and the layer scale ride in the residual launch
   gated_attn (mixer and feed-forward side by side) one fused projection q | k | v | gate | up -> rotation
              (YaRN frequencies), k and v to their pages, relu(up)^2, in one launch -> attention inside
