@@ -77,7 +77,7 @@ int dllm_conv_silu(const void*, long, int, const float*, const float*, void*, co
                    const int*, void*, int, int, int, int, int, int, int, hipStream_t);
 int dllm_zero_free_rows(void*, int, long, int, const int*, const int*, int, hipStream_t);
 long dllm_scan_chunks_scratch(long, int, int, int);
-int dllm_scan_step_ok(long, int, int, const void*, const void*);
+int dllm_scan_step_ok(int, const void*, const void*);
 int dllm_scan_chunks(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*, const void*, long,
                      float*, void*, int, const int*, const int*, const int*, const int*, void*, int, long, int, int, float*, hipStream_t);
 int dllm_selective_scan(const void*, const void*, int, const float*, const float*, const void*, long, int, const float*,
@@ -1559,7 +1559,7 @@ void causal_conv_silu(torch::Tensor x, torch::Tensor w, torch::Tensor b, torch::
 void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bias, torch::Tensor A, torch::Tensor dbc,
                     int64_t dt_rank, torch::Tensor D, torch::Tensor xz, torch::Tensor ssm, torch::Tensor conv,
                     torch::Tensor qstart, torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out,
-                    bool chunked) {
+                    bool chunked, bool few) {
   const bool f = act_f32(xc, "xc");
   for (auto* t : {&dt_raw, &dbc, &xz, &out, &conv})
     TORCH_CHECK(t->is_cuda() && t->scalar_type() == xc.scalar_type(), "activations share one dtype");
@@ -1584,7 +1584,7 @@ void selective_scan(torch::Tensor xc, torch::Tensor dt_raw, torch::Tensor dt_bia
   const long ns = chunked ? dllm_scan_chunks_scratch(T, m.S, C, N) : 0;
   // rows of no sequence become zeros: in the step kernel, else here
   const auto clear = [&] { ok(dllm_zero_free_rows(out.data_ptr(), f ? 4 : 2, T, C, m.qstart, m.qlen, m.S, stream()), "zero_free_rows"); };
-  const bool step = m.S > 0 && !chunked && dllm_scan_step_ok(T, m.S, N, ssm.data_ptr(), A.data_ptr());
+  const bool step = m.S > 0 && !chunked && few && dllm_scan_step_ok(N, ssm.data_ptr(), A.data_ptr());
   if (step || ns > 0) {      // decode steps, or the chunk-parallel form (prompt portions)
     torch::Tensor sc;
     if (!step) {

@@ -308,11 +308,9 @@ extern "C" long dllm_scan_chunks_scratch(long T, int S, int C, int N) {
   return N < 1 || N > 32 || nc < 1 || nc > 65535 ? 0 : nc * channels_at_once(nc, C, N) * (N + 1L);
 }
 
-// May the step kernel take it?  Steps of at most four tokens a sequence on average (2048 channels of 16 states, us with a thread /
-// 16 lanes a channel: one sequence of 1 token 4.9 / 6.3, of 4 6.4 / 6.5, of 8 8.3 / 7.0; 24 of 1 6.9 / 14.0, of 4 8.5 / 14.2).
-// Whole, aligned vectors of states.
-extern "C" int dllm_scan_step_ok(long T, int S, int N, const void* ssm, const void* A) {
-  return T <= 4L * S && N % 4 == 0 && N <= 32 && (((uintptr_t)ssm | (uintptr_t)A) & 15) == 0;
+// May the step kernel take it?  Whole, aligned vectors of states.
+extern "C" int dllm_scan_step_ok(int N, const void* ssm, const void* A) {
+  return N % 4 == 0 && N <= 32 && (((uintptr_t)ssm | (uintptr_t)A) & 15) == 0;
 }
 
 // the arguments of dllm_selective_scan, and the scratch; without scratch the step kernel (dllm_scan_step_ok)

@@ -96,6 +96,12 @@ def scan_in_chunks(T: int, S: int, longest: Optional[int]) -> bool:
     return n >= 160 and (T >= 100 * S or n >= 160 + 2 * S)
 
 
+# tokens of the longest portion up to which a thread takes a channel, past it 16 lanes (us, 2048 channels of 16 states): one sequence of 1
+# token 4.9 / 6.3, of 4 6.4 / 6.5, of 8 8.3 / 7.0; 24 of 1 6.9 / 14.0, of 4 8.5 / 14.2; 16 tokens beside 7 single ones 12.3 / 8.9, 150
+# beside 63 90 / 36
+SCAN_STEP_MAX = 4
+
+
 def selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_state, qstart, qlen, ctx,
                    rows, chunked: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
     """Mamba-1: S <- exp(dt A) S + dt x B, y = S C + D x, times silu(z), with dt = softplus(dt_raw + dt_bias), B and C
@@ -110,7 +116,7 @@ def selective_scan(xc, dt_raw, dt_bias, A, dbc, dt_rank, D, xz, ssm_state, conv_
     if chunked is None:
         chunked = scan_in_chunks(xc.shape[0], qstart.numel(), longest)
     ext.selective_scan(xc, dt_raw, dt_bias, A, dbc, int(dt_rank), D, xz, ssm_state, conv_state, qstart, qlen, ctx,
-                       rows, out, bool(chunked))
+                       rows, out, bool(chunked), longest_portion(xc.shape[0], qstart.numel(), longest) <= SCAN_STEP_MAX)
     return out
 
 

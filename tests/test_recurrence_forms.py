@@ -60,3 +60,13 @@ def test_layers_say_their_longest_portion(monkeypatch):
         except StopIteration:
             pass
     assert seen == [("selective_scan", 31), ("retention", 31), ("delta_rule", 31)]
+
+
+def test_scan_steps(monkeypatch):
+    """A thread takes a channel where no sequence brings more than four tokens, whatever the average."""
+    seen = []
+    monkeypatch.setattr(seqmix, "_native", lambda x: types.SimpleNamespace(selective_scan=lambda *a: seen.append(a[-2:])))
+    for lens in ([1] * 24, [4, 1], [150] + [1] * 63, [16] + [1] * 7, [2000]):
+        x, q = torch.zeros(sum(lens), 8), torch.zeros(len(lens), dtype=torch.int32)
+        seqmix.selective_scan(x, x, None, None, None, 4, None, None, None, None, q, q, q, q, longest=max(lens))
+    assert seen == [(False, True), (False, True), (False, False), (False, False), (True, False)]
