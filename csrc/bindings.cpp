@@ -1617,7 +1617,7 @@ static torch::Tensor chunk_scratch(int64_t T, int S, int64_t H, int64_t d, int64
 void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tensor cos_sin, int64_t rot,
                torch::Tensor decay, torch::Tensor state, double eps, torch::Tensor pos, torch::Tensor qstart,
                torch::Tensor qlen, torch::Tensor ctx, torch::Tensor rows, torch::Tensor out,
-               c10::optional<torch::Tensor> raw) {
+               c10::optional<torch::Tensor> raw, bool in_order) {
   const bool f = act_f32(qkvg, "qkvg");
   check_rows2d(qkvg, "qkvg");
   check_f32(cos_sin, "cos_sin");
@@ -1637,7 +1637,7 @@ void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tens
   if (raw) {   // chunked form (prompt portions): f32 scratch [T, H, dv]
     check_f32(*raw, "raw");
     TORCH_CHECK(raw->numel() >= (int64_t)T * H * dv, "raw scratch [T, H, dv]");
-    const auto sc = chunk_scratch(T, m.S, H, d, dv, qkvg);
+    const auto sc = in_order ? torch::Tensor() : chunk_scratch(T, m.S, H, d, dv, qkvg);
     TORCH_CHECK(sc.defined() || dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
     ok(dllm_zero_free_rows(out.data_ptr(), f ? 4 : 2, T, (int)(H * dv), m.qstart, m.qlen, m.S, stream()), "zero_free_rows");
     ok(dllm_retention_chunked(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, cos_sin.data_ptr<float>(),
@@ -1658,7 +1658,7 @@ void retention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tens
 // outputs [T, H, dv]; then the heads of a token are normed together and gated by a sigmoid.
 void lightning_attention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, torch::Tensor decay, torch::Tensor state,
                          double eps, torch::Tensor norm_w, torch::Tensor qstart, torch::Tensor qlen, torch::Tensor ctx,
-                         torch::Tensor rows, torch::Tensor out, torch::Tensor raw, bool chunked) {
+                         torch::Tensor rows, torch::Tensor out, torch::Tensor raw, bool chunked, bool in_order) {
   const bool f = act_f32(qkvg, "qkvg");
   check_rows2d(qkvg, "qkvg");
   check_f32(decay, "decay");
@@ -1676,7 +1676,7 @@ void lightning_attention(torch::Tensor qkvg, int64_t H, int64_t d, int64_t dv, t
   TORCH_CHECK(raw.numel() >= (int64_t)T * H * dv, "raw scratch [T, H, dv]");
   auto m = seq_meta(qstart, qlen, ctx, rows, state.size(0));
   if (chunked) {
-    const auto sc = chunk_scratch(T, m.S, H, d, dv, qkvg);
+    const auto sc = in_order ? torch::Tensor() : chunk_scratch(T, m.S, H, d, dv, qkvg);
     TORCH_CHECK(sc.defined() || dllm_retention_chunk_lds((int)d) <= 150 * 1024, "dim does not fit the LDS");
     ok(dllm_retention_chunked(qkvg.data_ptr(), qkvg.stride(0), f, (int)H, (int)d, (int)dv, decay.data_ptr<float>(), 0, 0,
                               decay.data_ptr<float>(), state.data_ptr<float>(), (float)eps, m.qstart, m.qlen, m.ctx, m.rows,
@@ -2649,7 +2649,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("selective_scan", &selective_scan);
   m.def("retention", &retention, py::arg("qkvg"), py::arg("heads"), py::arg("dim"), py::arg("vdim"), py::arg("cos_sin"),
         py::arg("rot"), py::arg("decay"), py::arg("state"), py::arg("eps"), py::arg("positions"), py::arg("qstart"),
-        py::arg("qlen"), py::arg("ctx"), py::arg("rows"), py::arg("out"), py::arg("raw") = py::none());
+        py::arg("qlen"), py::arg("ctx"), py::arg("rows"), py::arg("out"), py::arg("raw") = py::none(), py::arg("in_order") = false);
   m.def("relu2_scale", &relu2_scale);
   m.def("dense_gate", &dense_gate);
   m.def("lightning_attention", &lightning_attention);

@@ -129,7 +129,7 @@ def retention_step_lds(dim: int, vdim: int) -> int:
 
 
 def retention_in_chunks(T: int, S: int, heads: int, longest: Optional[int]) -> bool:
-    """Do the chunk-parallel kernels run?  Token by token a token costs 2.6 us of a chain that all sequences walk side by side; in chunks
+    """Do the chunk-parallel kernels run where chunks in order have too many workgroups?  Token by token a token costs 2.6 us of a chain that all sequences walk side by side; in chunks
     three launches, and up to 0.1 us for every (sequence, head), whose last chunk is padded to 64 tokens, until the chip is as full
     either way.  us token by token / in chunks, 8 heads of 64 x 128; 16 of 128 x 128: one sequence of 8 tokens 25 / 29; 31 / 41, of
     16 47 / 29; 51 / 42; 24 sequences of 16 47 / 43; 63 / 85, of 32 90 / 54; 113 / 93; 64 of 24 75 / 86; 167 / 181, of 32 101 / 92;
@@ -137,22 +137,41 @@ def retention_in_chunks(T: int, S: int, heads: int, longest: Optional[int]) -> b
     return longest_portion(T, S, longest) >= min(28, 10 + S * heads / 24)
 
 
+def retention_form(T: int, S: int, heads: int, dim: int, vdim: int, longest: Optional[int]) -> Tuple[bool, bool]:
+    """(chunked, in order) of a step.  Between single tokens and long prompts the chunks of 32 tokens in order win: one launch
+    of S heads vdim / 32 workgroups, of which the chip holds two to a CU at heads of 128 and four below (``fill`` of that; past 2 the rule
+    of ``retention_in_chunks``).  us token by token / in order / in parallel: 8 heads of 64 x 128, one sequence of 5 tokens 17 / 17 / 32,
+    of 16 36 / 19 / 32, of 64 - / 34 / 40, of 96 - / 47 / 40; 24 of 8 26 / 27 / 45, of 16 41 / 30 / 46, of 64 - / 54 / 62; 16 of
+    128 x 128: one of 8 32 / 26 / 42, of 64 - / 50 / 54; 8 of 8 33 / 34 / 58; 16 of 16 60 / 67 / 77, of 24 84 / 73 / 83, of 48
+    - / 111 / 91; 4 of 32 x 32: one of 4 13.5 / 12.1 / 18.6, of 32 66 / 17 / 20, of 48 - / 23 / 21; 16 of 64 x 64: of 32 61 / 22 / 28,
+    of 64 - / 35 / 31."""
+    n = longest_portion(T, S, longest)
+    fill = S * heads * -(-vdim // 32) / (256 if dim > 128 else 512 if dim > 64 else 1024)
+    line = (3.5 if dim <= 32 else 5) + 4 * fill * max(1.0, fill)
+    if dim > 128:      # the chunk-parallel kernels do not take it
+        return n >= min(28, line), True
+    if fill > 2:
+        return retention_in_chunks(T, S, heads, longest), False
+    return n >= line, n <= (64 if dim * vdim > 4096 and fill <= 1 else 32)
+
+
 def retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen, ctx,
               rows, chunked: Optional[bool] = None, longest: Optional[int] = None) -> torch.Tensor:
-    """``chunked`` (GPU): the chunk-parallel kernel (prompt portions) or the token-by-token one
-    (decode steps); default by the step's tokens per sequence.  Same results either way."""
+    """``chunked`` (GPU): the chunk-parallel kernels (prompt portions) or the token-by-token one
+    (decode steps); default by the step's ``longest`` portion, with chunks in order between the two.  Same results either way."""
     ext = _native(qkvg)
     if ext is None:
         return ref.retention(qkvg, heads, dim, vdim, cos_sin, rot_dims, decay, state, eps, positions, qstart, qlen,
                              ctx, rows)
     out = torch.empty((qkvg.shape[0], heads * vdim), dtype=qkvg.dtype, device=qkvg.device)      # rows of no sequence become zeros
+    in_order = False
     if chunked is None:
-        chunked = retention_in_chunks(qkvg.shape[0], qstart.numel(), heads, longest)
+        chunked, in_order = retention_form(qkvg.shape[0], qstart.numel(), heads, dim, vdim, longest)
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
         chunked = True      # the token-by-token kernel keeps the whole [dim, vdim] state in LDS
     raw = torch.empty((qkvg.shape[0], heads, vdim), dtype=torch.float32, device=qkvg.device) if chunked else None
     ext.retention(qkvg, int(heads), int(dim), int(vdim), cos_sin, int(rot_dims), decay, state, float(eps), positions,
-                  qstart, qlen, ctx, rows, out, raw)
+                  qstart, qlen, ctx, rows, out, raw, in_order)
     return out
 
 
@@ -623,12 +642,13 @@ def lightning_attention(qkvg, heads, dim, vdim, decay, state, eps, norm_w, qstar
     T = qkvg.shape[0]
     out = torch.empty((T, heads * vdim), dtype=qkvg.dtype, device=qkvg.device)     # the finish kernel writes every row
     if chunked is None:
-        chunked = retention_in_chunks(T, qstart.numel(), heads, longest)
+        chunked, in_order = retention_form(T, qstart.numel(), heads, dim, vdim, longest)
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
+    in_order = False
         chunked = True
     raw = torch.empty((T, heads, vdim), dtype=torch.float32, device=qkvg.device)    # read for live tokens only
     ext.lightning_attention(qkvg, int(heads), int(dim), int(vdim), decay, state, float(eps), norm_w, qstart, qlen, ctx,
-                            rows, out, raw, bool(chunked))
+                            rows, out, raw, bool(chunked), in_order)
     return out
 
 

@@ -62,6 +62,20 @@ def test_layers_say_their_longest_portion(monkeypatch):
     assert seen == [("selective_scan", 31), ("retention", 31), ("delta_rule", 31)]
 
 
+def test_chunks_in_order_between():
+    """Portions of a few to 64 tokens on few heads: chunks in order, neither token by token nor in parallel."""
+    def form(lens, heads, dim, vdim):
+        return seqmix.retention_form(sum(lens), len(lens), heads, dim, vdim, max(lens))
+
+    for lens, heads, dim, vdim in (([8], 8, 64, 128), ([16] * 24, 8, 64, 128), ([64], 16, 128, 128), ([8] * 24, 4, 32, 32), ([16] + [1] * 7, 16, 128, 128)):
+        assert form(lens, heads, dim, vdim) == (True, True)
+    for lens, heads, dim, vdim in (([200], 8, 64, 128), ([96], 16, 128, 128), ([48], 4, 32, 32), ([64] * 24, 16, 128, 128), ([1000] + [1] * 31, 8, 64, 128)):
+        assert form(lens, heads, dim, vdim) == (True, False)
+    for lens, heads, dim, vdim in (([4], 8, 64, 128), ([1] * 64, 16, 128, 128), ([16] * 24, 16, 128, 128), ([8] * 48, 8, 64, 128), ([], 8, 64, 128)):
+        assert not seqmix.retention_form(sum(lens), len(lens), heads, dim, vdim, max(lens, default=None))[0]
+    assert form([40], 4, 256, 64) == (True, True)      # widths only the chunks in order take
+
+
 def test_scan_steps(monkeypatch):
     """A thread takes a channel where no sequence brings more than four tokens, whatever the average."""
     seen = []
