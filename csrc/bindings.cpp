@@ -52,7 +52,7 @@ int dllm_rms_rows(const void*, long, int, const float*, void*, long, int, int, i
 int dllm_norm_resadd(const void*, long, int, const float*, float*, void*, int, int, float, int, const float*, hipStream_t);
 int dllm_polynorm(const void*, long, int, const float*, void*, long, int, float, hipStream_t);
 int dllm_router_topk(const void*, long, const float*, int, int, float*, int, int, int, int, int, int, int, const float*, int, int*, float*, float*,
-                     hipStream_t);
+                     int, hipStream_t);
 int dllm_route_topk(const float*, long, int, int, int, int, int, int, int, const float*, int, int*, float*, float*, hipStream_t);
 int dllm_ls_resadd_ln(const void*, long, int, const float*, const float*, const void*, long, const float*, long, const void*, long,
                       const float*, float*, const float*, const float*, void*, long, int, float, hipStream_t);
@@ -2309,7 +2309,8 @@ void route_topk(torch::Tensor logits, int64_t E, int64_t top, int64_t count, int
 // f32 logits of x (bf16) against w [n, H] and route_topk over the first E of them in one launch (seqmix.hip router_topk)
 void router_topk(torch::Tensor x, torch::Tensor w, int64_t E, int64_t top, int64_t count, int64_t keep, int64_t smode, int64_t gmode,
                  c10::optional<torch::Tensor> corr, int64_t real, torch::Tensor ids, torch::Tensor wts, torch::Tensor idw,
-                 c10::optional<torch::Tensor> logits) {
+                 c10::optional<torch::Tensor> logits, bool apart) {
+  TORCH_CHECK(!apart || logits, "two launches pass the logits on");
   check_bf16(x, "x");
   check_f32(w, "w");
   check_i32(ids, "ids");
@@ -2340,7 +2341,7 @@ void router_topk(torch::Tensor x, torch::Tensor w, int64_t E, int64_t top, int64
     lp = logits->data_ptr<float>();
   }
   ok(dllm_router_topk(x.data_ptr(), x.stride(0), w.data_ptr<float>(), (int)n, (int)H, lp, (int)T, (int)E, (int)top, (int)count, (int)keep,
-                      (int)smode, (int)gmode, cp, (int)real, ids.data_ptr<int>(), wts.data_ptr<float>(), idw.data_ptr<float>(), stream()),
+                      (int)smode, (int)gmode, cp, (int)real, ids.data_ptr<int>(), wts.data_ptr<float>(), idw.data_ptr<float>(), apart ? 1 : 0, stream()),
      "router_topk");
 }
 

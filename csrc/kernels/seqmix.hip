@@ -1208,23 +1208,17 @@ __global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict
   route_one(logits + (long)t * ld, rsm + wave * route_patch(E), t, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw);
 }
 
-// The f32 router and the choice in one launch: a workgroup per token, EB rows of w [n, H] f32 a wave in flight, products summed
-// per lane and by a butterfly in a fixed order (a token's logits never depend on the batch), then one wave routes from LDS.
-// Bound by the rows' loads: 16 tokens, 8 outputs, width 1024: 6.2 us against 14.4 (the rounded rows made f32, a library
-// product and the choice in three launches).
+// f32 products of token t with outputs e0, e0 + step .. of w [n, H], EB rows of w a wave in flight, summed per lane and by a butterfly in a
+// fixed order: a token's logits depend neither on the batch nor on which launch makes them
 template <int XC>
-__global__ void __launch_bounds__(256) router_topk_kernel(const u16* __restrict__ x, long ldx, const float* __restrict__ w, int n, int H,
-                                                          float* __restrict__ logits, int E, int top, int count, int keep,
-                                                          int smode, int gmode, const float* __restrict__ corr, int real,
-                                                          int* __restrict__ ids, float* __restrict__ wts, float* __restrict__ idw) {
+__device__ __forceinline__ void router_dots(const u16* __restrict__ x, const float* __restrict__ w, int n, int H, int e0, int end, int step,
+                                            float* z) {
   constexpr int EB = XC <= 4 ? 2 : 1;
-  extern __shared__ float rsm[];        // [n] logits, then route_one's patch
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nc = H >> 3;
-  const long t = blockIdx.x;
+  const int lane = threadIdx.x & 63, nc = H >> 3;
   uint4 xr[XC];
 #pragma unroll
-  for (int c = 0; c < XC; ++c) xr[c] = lane + 64 * c < nc ? ld16(x + t * ldx + 8 * (lane + 64 * c)) : make_uint4(0u, 0u, 0u, 0u);
-  for (int e0 = wave * EB; e0 < n; e0 += 4 * EB) {
+  for (int c = 0; c < XC; ++c) xr[c] = lane + 64 * c < nc ? ld16(x + 8 * (lane + 64 * c)) : make_uint4(0u, 0u, 0u, 0u);
+  for (; e0 < end; e0 += step) {
     f32x4 a[EB][XC], b[EB][XC];
 #pragma unroll
     for (int j = 0; j < EB; ++j)
@@ -1248,12 +1242,37 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const u16* __restrict_
         for (int q = 0; q < 4; ++q) s += f[4 + q] * b[j][c][q];
       }
       s = wave_sum(s);
-      if (lane == 0 && e0 + j < n) rsm[e0 + j] = s;
+      if (lane == 0 && e0 + j < n) z[e0 + j] = s;
     }
   }
+}
+
+// The f32 router and the choice in one launch: a workgroup per token, then one wave routes from LDS.  Bound by the rows' loads: 16 tokens,
+// 8 outputs, width 1024: 6.2 us against 14.4 (the rounded rows made f32, a library product and the choice in three launches).
+template <int XC>
+__global__ void __launch_bounds__(256) router_topk_kernel(const u16* __restrict__ x, long ldx, const float* __restrict__ w, int n, int H,
+                                                          float* __restrict__ logits, int E, int top, int count, int keep,
+                                                          int smode, int gmode, const float* __restrict__ corr, int real,
+                                                          int* __restrict__ ids, float* __restrict__ wts, float* __restrict__ idw) {
+  constexpr int EB = XC <= 4 ? 2 : 1;
+  extern __shared__ float rsm[];        // [n] logits, then route_one's patch
+  const int wave = threadIdx.x >> 6;
+  const long t = blockIdx.x;
+  router_dots<XC>(x + t * ldx, w, n, H, wave * EB, n, 4 * EB, rsm);
   __syncthreads();
   if (logits && threadIdx.x < n) logits[t * n + threadIdx.x] = rsm[threadIdx.x];
   if (wave == 0) route_one(rsm, rsm + n, t, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw);
+}
+
+// The logits alone, a wave per EB outputs of a token: for weights that one workgroup takes in too slowly (16 tokens, 256 outputs of width
+// 1024: 28 us in one launch)
+template <int XC>
+__global__ void __launch_bounds__(256) router_logits_kernel(const u16* __restrict__ x, long ldx, const float* __restrict__ w, int n, int H,
+                                                            float* __restrict__ logits) {
+  constexpr int EB = XC <= 4 ? 2 : 1;
+  const int e0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * EB;
+  const long t = blockIdx.x;
+  router_dots<XC>(x + t * ldx, w, n, H, e0, min(n, e0 + EB), EB, logits + t * n);
 }
 
 // gu [rows, E 2 ff] (per expert: gate columns, then up columns) -> y [rows, E ff] = silu(gate) up gate[row, expert]
@@ -1840,11 +1859,11 @@ extern "C" int dllm_route_topk(const float* logits, long ld, int T, int E, int t
   return (int)hipGetLastError();
 }
 
-// logits = x [T, H] bf16 . w [n, H]^T in f32 and the routing of dllm_route_topk over the first E of them, in one launch; logits
-// [T, n] f32 may be null.  n <= 256 outputs, H <= 8192, rows of whole 16-byte vectors
+// logits = x [T, H] bf16 . w [n, H]^T in f32 and the routing of dllm_route_topk over the first E of them, in one launch, or with `apart`
+// in two (the same bits); logits [T, n] f32 may be null in one.  n <= 256 outputs, H <= 8192, rows of whole 16-byte vectors
 extern "C" int dllm_router_topk(const void* x, long ldx, const float* w, int n, int H, float* logits, int T, int E, int top, int count,
                                 int keep, int smode, int gmode, const float* corr, int real, int* ids, float* wts, float* idw,
-                                hipStream_t st) {
+                                int apart, hipStream_t st) {
   if (n < 1 || n > 256 || E < 1 || E > n || H % 8 || H > 8192 || ldx % 8 || top < 1 || count < 1 || E % count || keep < 1 ||
       keep > count || top > keep * (E / count) || real < 0)
     return -1;
@@ -1852,6 +1871,16 @@ extern "C" int dllm_router_topk(const void* x, long ldx, const float* w, int n, 
   const size_t lds = 4UL * (n + route_patch(E));
 #define ROUT(XC)                                                                                                                \
   hipLaunchKernelGGL(router_topk_kernel<XC>, dim3(T), dim3(256), lds, st, (const u16*)x, ldx, w, n, H, logits, E, top, count, keep, smode, \
+  if (apart) {
+    if (!logits) return -2;
+#define RLOG(XC)                                                                                                                          \
+  hipLaunchKernelGGL(router_logits_kernel<XC>, dim3(T, (n + 4 * (XC <= 4 ? 2 : 1) - 1) / (4 * (XC <= 4 ? 2 : 1))), dim3(256), 0, st,       \
+                     (const u16*)x, ldx, w, n, H, logits)
+    if (H <= 1024) RLOG(2); else if (H <= 2048) RLOG(4); else if (H <= 4096) RLOG(8); else RLOG(16);
+#undef RLOG
+    const int rc = (int)hipGetLastError();
+    return rc ? rc : dllm_route_topk(logits, n, T, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw, st);
+  }
                      gmode, corr, real, ids, wts, idw)
   if (H <= 1024) ROUT(2); else if (H <= 2048) ROUT(4); else if (H <= 4096) ROUT(8); else ROUT(16);
 #undef ROUT

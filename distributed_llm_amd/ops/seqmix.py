@@ -576,28 +576,31 @@ def route_topk(logits: torch.Tensor, n_out: int, top: int, count: int = 1, keep:
 
 # rows times outputs up to which the router's product and choice are one launch: a workgroup per token reads the router's weights
 # again, the library's product does not (us, one launch / three, width 2048: 8 outputs, 16 rows 6.6 / 15.0, 4096 rows 20 / 31, 8192
-# rows 36 / 40; 64 outputs, 16 rows 15 / 17, 256 rows 16 / 19, 1024 rows 29 / 22)
-ROUTER_WORK = 1 << 15
+# rows 36 / 40; 64 outputs, 16 rows 15 / 17, 256 rows 16 / 19, 1024 rows 29 / 22); outputs and weights up to which a workgroup alone reads
+# them in that time, and f32 read in all (rows x weights) up to which the logits are a launch of many workgroups instead (us, one launch
+# / three: 16 rows, 64 outputs of width 8192 28 / 23; 256 of 1024 28 / 16, of 8192 91 / 25)
+ROUTER_WORK, ROUTER_OUT, ROUTER_WEIGHTS, ROUTER_READ = 1 << 15, 64, 1 << 17, 1 << 23
 
 
 def router_topk(x: torch.Tensor, w: torch.Tensor, n_out: int, top: int, count: int = 1, keep: int = 1, score: str = "sigmoid",
                 group_score: str = "top2", correction: Optional[torch.Tensor] = None, real: Optional[int] = None,
                 want_logits: bool = False):
     """``route_topk`` of the f32 logits x . w^T (w [n, H] f32): ids, weights, identity weights and, on request, the logits
-    [T, n] (else None).  bf16 rows of whole vectors take one launch."""
+    [T, n] (else None).  bf16 rows of whole vectors take one launch, or two where the weights are many."""
     ext = _native(x)
     T, H = x.shape
-    if (ext is None or x.dtype != torch.bfloat16 or T * w.shape[0] > ROUTER_WORK or H % 8 or H > 8192 or w.shape[0] > 256 or x.stride(1) != 1
-            or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous()):
+    one = T * w.shape[0] <= ROUTER_WORK and w.shape[0] <= ROUTER_OUT and w.numel() <= ROUTER_WEIGHTS
+    if (ext is None or x.dtype != torch.bfloat16 or not (one or T * w.numel() <= ROUTER_READ) or w.shape[0] > 256 or H % 8 or H > 8192
+            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16 or w.data_ptr() % 16 or not w.is_contiguous()):
         logits = torch.nn.functional.linear(x.float(), w)
         return (*route_topk(logits, n_out, top, count, keep, score, group_score, correction, real), logits)
     ids = torch.empty((T, top), dtype=torch.int32, device=x.device)
     wts = torch.empty((T, top), dtype=torch.float32, device=x.device)
     idw = torch.empty((T,), dtype=torch.float32, device=x.device)
-    logits = torch.empty((T, w.shape[0]), dtype=torch.float32, device=x.device) if want_logits else None
+    logits = torch.empty((T, w.shape[0]), dtype=torch.float32, device=x.device) if want_logits or not one else None
     ext.router_topk(x, w, int(n_out), int(top), int(count), int(keep), 0 if score == "sigmoid" else 1, 0 if group_score == "top2" else 1,
-                    correction, int(n_out if real is None else real), ids, wts, idw, logits)
-    return ids, wts, idw, logits
+                    correction, int(n_out if real is None else real), ids, wts, idw, logits, not one)
+    return ids, wts, idw, logits if want_logits else None
 
 
 def group_router(logits: torch.Tensor, top: int, count: int, keep: int) -> Tuple[torch.Tensor, torch.Tensor]:
