@@ -131,11 +131,12 @@ __global__ void __launch_bounds__(256 * VS) skinny_gemm_kernel(const u16* __rest
     }
     kb = wk0 + nblk * 32 * U;
   }
-  if (kb < wk1) {  // tail (< U k-steps), its loads in flight together
+  constexpr int TU = SWIGLU ? 1 : U;      // tail (< U k-steps), its loads in flight together; one at a time where a step's code is long
+  for (; kb < wk1; kb += 32 * TU) {
     Stage T;
-    const int tail = (wk1 - kb) / 32;
+    const int tail = TU == 1 ? 1 : (wk1 - kb) / 32;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < TU; ++u) {
       if (u >= tail) break;
       const int k = kb + 32 * u;
 #pragma unroll
