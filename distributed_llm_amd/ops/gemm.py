@@ -199,7 +199,7 @@ def _heuristic(M: int, N: int, K: int, swiglu: bool = False) -> Tuple:
         return ("gemv", 1)
     splits = max(1, min(16, math.ceil(512 / ((N + 31) // 32)), K // 256))
     narrow = N * K <= _NARROW if M <= 32 else N <= 2048 and splits <= 4
-    return ("skinny", 1 if narrow and not swiglu else 2, splits)
+    return ("skinny", 2 if swiglu else _apart(M, N, K, splits) or (1 if narrow else 2), splits)
 
 
 # weights up to which 16 columns and four splits of K a workgroup (16 waves) beat 32 columns and two: past it the 16-wave workgroups,
@@ -207,14 +207,31 @@ def _heuristic(M: int, N: int, K: int, swiglu: bool = False) -> Tuple:
 # 1024 x 1024 4.2 / 5.1, 6.5 / 7.3, 6.1 / 6.7; 5632 x 1024 6.8 / 9.7, 8.6 / 11.9, 8.5 / 10.7; 1024 x 4096 11.4 / 12.7, 11.8 / 12.4,
 # 12.4 / 13.2; 8192 x 2048 10.9 / 16.0, 10.8 / 12.7, 12.7 / 14.8.  Past 32 rows a workgroup re-reads more rows than weights: 16
 # columns, a split each, where that is few workgroups (48 rows, 1024 x 1024: 7.1, 8.2, 8.5; 4096 x 1024 11.3, 8.9, 10.0).
-_NARROW = 8 << 20
+_NARROW = 6 << 20
 
 
-def _splits_together(M: int, plan: Tuple) -> int:
+def _apart(M: int, N: int, K: int, splits: int) -> int:
+    """Columns (in 16s) of a workgroup where more than four splits stay in workgroups of their own, else 0: few columns, whose joint
+    workgroups are too few, and numbers of splits that leave a joint workgroup half empty.  us apart / together: 128 x 2048 8 rows 6.3 / 7.0,
+    32 rows 7.2 / 8.8; 512 x 2048 8 rows 8.2 / 8.3, 32 rows 8.6 / 9.7, 64 rows 9.2 / 10.5; 256 x 8192 8 rows 11.0 (32 columns; 16 12.0) / 12.3; six splits:
+    3000 x 1536 8 rows equal, 32 rows 11.0 / 12.6, 3000 x 4096 8 rows (32 columns) 11.5 / 13.1, 3000 x 8192 64 rows, 32 columns 32.9,
+    16 38.2."""
+    if splits <= 4:
+        return 0
+    if N <= 256 and splits > 8 and N > 128 and M <= 32:
+        return 2
+    if N <= 128 or (N <= 512 and M > 16):
+        return 1
+    if splits % 4 in (1, 2) and (M > 16 or N * K > _NARROW):
+        return 1 if M > 16 and N * K <= 2 * _NARROW else 2
+    return 0
+
+
+def _splits_together(M: int, N: int, K: int, plan: Tuple) -> int:
     """Splits of K that share a workgroup of an untimed plan, meeting in LDS where they are all there (slabs and ticket cost 1.3 to 2.3
     us).  Three splits of 32 columns stay apart: the pairs would leave a quarter of the waves idle."""
     _, ntw, splits = plan
-    if M > 64 or splits == 1:
+    if M > 64 or splits == 1 or _apart(M, N, K, splits):
         return 1
     if ntw == 1:
         return 4 if M <= 32 else 1
@@ -429,7 +446,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
         else:
             plan = _heuristic(x.shape[0], w.shape[0], w.shape[1])
             if plan[0] == "skinny":
-                together = _splits_together(x.shape[0], plan)
+                together = _splits_together(x.shape[0], w.shape[0], w.shape[1], plan)
     return _run_plan(plan, x, w, False, out, wp, together)
 
 
