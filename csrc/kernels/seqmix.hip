@@ -1562,7 +1562,10 @@ extern "C" int dllm_norm_resadd(const void* y, long ldy, int f32, const float* w
                                 float eps, int groups, const float* bias, hipStream_t st) {
   if (rows <= 0) return rows == 0 ? 0 : -1;
   if (groups < 1 || H % groups) return -1;
-  if (norm_resadd_entries(H, groups))
+  // f32 rows of 8192 (parts of 2048) hold 32 entries a thread, and many of them stream better in two passes of more waves: 4000 x 8192
+  // 151 us in registers, 126 in two passes; 300 rows 11.9, 15.4
+  const int e = norm_resadd_entries(H, groups);
+  if (e && !(f32 && e > 16 && rows > 1024))
     return f32 ? norm_resadd_reg<float, float>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st)
                : norm_resadd_reg<u16, u16>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st);
   BY_T(f32,
