@@ -295,7 +295,7 @@ template <> struct vec4<u16> {
 // sum over depth are read four vectors ahead.  Bound by memory: n slots are n
 // rows of f32 a token in and two out.  8k tokens of width 2048, the 18 launches of 12 layers whose sums take 2 to 13
 // slots (7.4 GB, 1.4 ms at 5.2 TB/s): 3.8 ms entry by entry, 1.7 ms here.
-template <typename T, int NV, bool TWO>
+template <typename T, int NV, bool TWO, bool DEPTH>
 __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restrict__ a, long lda, const T* __restrict__ b, long ldb,
                                                               const float* __restrict__ wa, const float* __restrict__ wb,
                                                               const float* __restrict__ w_post, float* __restrict__ x,
@@ -352,7 +352,7 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
       const float4 g = *reinterpret_cast<const float4*>(w_post + c);
       v[j].x += y[j].x * ry * g.x; v[j].y += y[j].y * ry * g.y; v[j].z += y[j].z * ry * g.z; v[j].w += y[j].w * ry * g.w;
       *reinterpret_cast<float4*>(xr + c) = v[j];
-      if (dw) {     // the layer's weighted sum over slots 0 .. dn - 1 of the stack, the last of them being this row
+      if constexpr (DEPTH) {     // the layer's weighted sum over slots 0 .. dn - 1 of the stack, the last of them being this row
         const float* p0 = xr + c - (long)(dn - 1) * TH;
         float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
         auto add = [&](float w, const float4& q) { s.x += w * q.x; s.y += w * q.y; s.z += w * q.z; s.w += w * q.w; };
@@ -1587,10 +1587,10 @@ extern "C" int dllm_resadd_norm(const void* a, long lda, const void* b, long ldb
   if (H % 4 == 0 && H <= 8192 && lda % 4 == 0 && (uintptr_t)a % ab == 0 && f16(x) && f16(w_post) && (!xn || (uintptr_t)xn % ab == 0) &&
       f16(w_next) && f16(bias) && (!b || (ldb % 4 == 0 && (uintptr_t)b % ab == 0 && f16(wa) && f16(wb)))) {
     const int nv = (H + 1023) / 1024;
-#define RN(T, NV, TWO)                                                                                                        \
-  hipLaunchKernelGGL((resadd_norm_vec_kernel<T, NV, TWO>), dim3(rows), dim3(256), 0, st, (const T*)a, lda, (const T*)b, ldb, wa, wb, \
+#define RN(T, NV, TWO, DEPTH)                                                                                                 \
+  hipLaunchKernelGGL((resadd_norm_vec_kernel<T, NV, TWO, DEPTH>), dim3(rows), dim3(256), 0, st, (const T*)a, lda, (const T*)b, ldb, wa, wb, \
                      w_post, x, w_next, (T*)xn, H, eps, bias, dw, dn, (long)rows * H)
-#define RNB(T, NV) do { if (b) RN(T, NV, true); else RN(T, NV, false); } while (0)
+#define RNB(T, NV) do { if (dw) { if (b) RN(T, NV, true, true); else RN(T, NV, false, true); } else { if (b) RN(T, NV, true, false); else RN(T, NV, false, false); } } while (0)
 #define RNT(T) do { if (nv <= 1) RNB(T, 1); else if (nv <= 2) RNB(T, 2); else if (nv <= 4) RNB(T, 4); else RNB(T, 8); } while (0)
     if (f32) RNT(float); else RNT(u16);
 #undef RNT
