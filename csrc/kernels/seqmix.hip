@@ -1871,9 +1871,6 @@ extern "C" int dllm_router_topk(const void* x, long ldx, const float* w, int n, 
       keep > count || top > keep * (E / count) || real < 0)
     return -1;
   if (T <= 0) return 0;
-  const size_t lds = 4UL * (n + route_patch(E));
-#define ROUT(XC)                                                                                                                \
-  hipLaunchKernelGGL(router_topk_kernel<XC>, dim3(T), dim3(256), lds, st, (const u16*)x, ldx, w, n, H, logits, E, top, count, keep, smode, \
   if (apart) {
     if (!logits) return -2;
 #define RLOG(XC)                                                                                                                          \
@@ -1884,6 +1881,9 @@ extern "C" int dllm_router_topk(const void* x, long ldx, const float* w, int n, 
     const int rc = (int)hipGetLastError();
     return rc ? rc : dllm_route_topk(logits, n, T, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw, st);
   }
+  const size_t lds = 4UL * (n + route_patch(E));
+#define ROUT(XC)                                                                                                                \
+  hipLaunchKernelGGL(router_topk_kernel<XC>, dim3(T), dim3(256), lds, st, (const u16*)x, ldx, w, n, H, logits, E, top, count, keep, smode, \
                      gmode, corr, real, ids, wts, idw)
   if (H <= 1024) ROUT(2); else if (H <= 2048) ROUT(4); else if (H <= 4096) ROUT(8); else ROUT(16);
 #undef ROUT

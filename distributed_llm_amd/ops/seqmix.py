@@ -644,10 +644,10 @@ def lightning_attention(qkvg, heads, dim, vdim, decay, state, eps, norm_w, qstar
         return ref.lightning_attention(qkvg, heads, dim, vdim, decay, state, eps, norm_w, qstart, qlen, ctx, rows)
     T = qkvg.shape[0]
     out = torch.empty((T, heads * vdim), dtype=qkvg.dtype, device=qkvg.device)     # the finish kernel writes every row
+    in_order = False
     if chunked is None:
         chunked, in_order = retention_form(T, qstart.numel(), heads, dim, vdim, longest)
     if not chunked and retention_step_lds(dim, vdim) > 150 * 1024:
-    in_order = False
         chunked = True
     raw = torch.empty((T, heads, vdim), dtype=torch.float32, device=qkvg.device)    # read for live tokens only
     ext.lightning_attention(qkvg, int(heads), int(dim), int(vdim), decay, state, float(eps), norm_w, qstart, qlen, ctx,
