@@ -12,9 +12,9 @@
 //                    state in registers (retention_step; in LDS for widths that are no vectors),
 //                    rotate-half positions applied while q / k are staged, unit-RMS heads and the SiLU
 //                    gate in the same launch
-//   retention_chunk  the same recurrence for prompt portions with dim > 128 (32 tokens at a time:
+//   retention_chunk  the same recurrence for short portions and for dim > 128 (32 tokens at a time:
 //                    scores inside the chunk + the carried state), one workgroup per (head, 32 value
-//                    columns, sequence); other dims run chunk_scan.hip; retention_finish norms and gates
+//                    columns, sequence); longer portions run chunk_scan.hip; retention_finish norms and gates
 //   resadd_norm      x (f32) += rmsnorm(y) * w with y one branch or the normed average of two, plus the
 //                    next sublayer's normed input; depth_mix: a weighted sum over the f32 stack of
 //                    layer results, plus the normed input of the next layer; gelu_erf; conv_refill
@@ -32,7 +32,7 @@
 //                    g sigmoid(alpha g) (u + 1)
 //   route_topk       group-limited top-k routing with sigmoid or softmax scores, a correction on the
 //                    choice and identity experts (group_router is its sigmoid / two-best form);
-//                    router_topk: the f32 logits of bf16 rows and the choice in one launch
+//                    router_topk: the f32 logits of bf16 rows and the choice in one launch, or two
 //
 // Activations are bf16 or f32 (template T = u16 / float); every sum, state, norm and gate is f32.
 // Sequence metadata: qstart / qlen / ctx / rows per sequence (int32); a sequence with qlen 0 is
@@ -864,7 +864,7 @@ __global__ void __launch_bounds__(256, NR <= 8 ? 4 : 3) retention_step_kernel(co
   }
 }
 
-// ---------------------------------------------------------------- retention, chunked (prompt portions with d > 128)
+// ---------------------------------------------------------------- retention, chunked (short portions, and d > 128)
 // One workgroup per (head, 32-column slice of the value dim, sequence); tokens in chunks of 32.
 // With the chunk's rotated q / k (k scaled) and v slice in LDS and g = decay:
 //   A[t][s] = g^(t-s) q_t . k_s  (s <= t)            scores inside the chunk, f32
@@ -1773,7 +1773,7 @@ extern "C" int dllm_retention_chunks(const void*, long, int, int, int, int, cons
                                      const int*, const int*, const int*, float*, int, long, int, float, float*, hipStream_t);
 
 // Chunked form for prompt portions: `raw` is an f32 scratch [T, H, dv].  `scratch` (dllm_chunk_scan_scratch entries): the
-// chunk-parallel kernels of chunk_scan.hip; null (widths they do not take): chunks in order, one workgroup per
+// chunk-parallel kernels of chunk_scan.hip; null (short portions, or widths they do not take): chunks in order, one workgroup per
 // (head, 32 value columns, sequence).
 extern "C" int dllm_retention_chunked(const void* qkvg, long ld, int f32, int H, int d, int dv, const float* cos_sin,
                                       int tab_w, int rot, const float* decay, float* state, float eps, const int* qstart,

@@ -129,9 +129,9 @@ def retention_step_lds(dim: int, vdim: int) -> int:
 
 
 def retention_in_chunks(T: int, S: int, heads: int, longest: Optional[int]) -> bool:
-    """Do the chunk-parallel kernels run where chunks in order have too many workgroups?  Token by token a token costs 2.6 us of a chain that all sequences walk side by side; in chunks
-    three launches, and up to 0.1 us for every (sequence, head), whose last chunk is padded to 64 tokens, until the chip is as full
-    either way.  us token by token / in chunks, 8 heads of 64 x 128; 16 of 128 x 128: one sequence of 8 tokens 25 / 29; 31 / 41, of
+    """Do the chunk-parallel kernels run where chunks in order have too many workgroups?  Token by token a token costs 2.6 us of a chain
+    that all sequences walk side by side; in chunks three launches, and up to 0.1 us for every (sequence, head), whose last chunk is
+    padded to 64 tokens, until the chip is as full either way.  us token by token / in chunks, 8 heads of 64 x 128; 16 of 128 x 128: one sequence of 8 tokens 25 / 29; 31 / 41, of
     16 47 / 29; 51 / 42; 24 sequences of 16 47 / 43; 63 / 85, of 32 90 / 54; 113 / 93; 64 of 24 75 / 86; 167 / 181, of 32 101 / 92;
     214 / 186; 200 tokens beside 31 single ones 543 / 57; 602 / 125."""
     return longest_portion(T, S, longest) >= min(28, 10 + S * heads / 24)
