@@ -43,6 +43,8 @@ int dllm_sample_split_kmax();
 int dllm_skinny_epi(const void*, long, const void*, int, void*, long, int, int, int, int, int, int, float*, int*, void*,
                     long, float*, long, const float*, int, long, float, float, const int*, const float*, const int*,
                     void*, void*, void*, int, int, int, hipStream_t);
+int dllm_dgemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*, void*, long, float*, long,
+               float, float, const int*, const float*, const int*, void*, void*, void*, void*, long, int, int, int, hipStream_t);
 int dllm_skinny_gemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*,
                      hipStream_t);
 int dllm_moe_max_tiles(int, int);
@@ -729,6 +731,96 @@ void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw,
         part.data_ptr<float>(), counters.data_ptr<int>(), stream()),
      "skinny_gemm");
 }
+// Decode GEMM on fragment-major weights (csrc/kernels/decode_gemm.hip), M <= 64: x [M, K], w [ceil(N / 16), K / 32, 64, 8]
+// (ops.gemm.frag_weight; paired for epi 2 and 3), epi 0 plain (y [M, N]), 1 residual add (res in place, per-tile row sums of squares ->
+// ssq_out), 2 QKV (row scale, RoPE, q_out, paged K, V^T or v_rows), 3 SwiGLU (row scale, y = act [M, N / 2]).  nt 16-column tiles a
+// workgroup, splits of K, vs of them a workgroup.  Returns the row-sum slots written (epi 1) or 0.
+int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int64_t nt, int64_t vs, int64_t splits,
+              c10::optional<torch::Tensor> y, c10::optional<torch::Tensor> part, c10::optional<torch::Tensor> counters,
+              c10::optional<torch::Tensor> res, c10::optional<torch::Tensor> ssq_out, double scale, double eps,
+              c10::optional<torch::Tensor> pos, c10::optional<torch::Tensor> cos_sin, c10::optional<torch::Tensor> slots,
+              c10::optional<torch::Tensor> q_out, c10::optional<torch::Tensor> kc, c10::optional<torch::Tensor> vc,
+              c10::optional<torch::Tensor> v_rows, int64_t nq, int64_t nkv, int64_t d) {
+  check_bf16(x, "x");
+  check_bf16(w, "w");
+  const int64_t M = x.size(0), K = x.dim() == 2 ? x.size(1) : 0, N = n_cols;
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) <= (1 << 24) && (uintptr_t)x.data_ptr() % 16 == 0, "x [M, K], 16-B rows");
+  TORCH_CHECK(M >= 1 && M <= 64 && K >= 32 && K % 32 == 0 && x.stride(0) >= (M > 1 ? K : 0), "M in [1, 64], K % 32 == 0");
+  TORCH_CHECK(w.dim() == 4 && w.is_contiguous() && w.size(0) == (N + 15) / 16 && w.size(1) == K / 32 && w.size(2) == 64 && w.size(3) == 8 && N >= 1,
+              "w: [ceil(N / 16), K / 32, 64, 8]");
+  TORCH_CHECK(epi >= 0 && epi <= 3 && nt >= 1 && nt <= 3 && (vs == 1 || vs == 2 || (vs == 4 && nt == 1 && M <= 32 && epi == 0)) && splits >= 1 && splits <= 64,
+              "no such plan");
+  const int64_t tiles = (N + 16 * nt - 1) / (16 * nt), kchunk = ((K + splits - 1) / splits + 31) / 32 * 32;
+  const int64_t S = (K + kchunk - 1) / kchunk, gy = (S + vs - 1) / vs, mr = (M + 15) / 16 * 16;
+  float* pp = nullptr;
+  int* cp = nullptr;
+  if (gy > 1) {
+    TORCH_CHECK(part.has_value() && counters.has_value(), "splits over workgroups need a workspace");
+    check_f32(*part, "part");
+    check_i32(*counters, "counters");
+    TORCH_CHECK(part->numel() >= gy * vs * tiles * mr * (16 * nt + 1) && gy * vs * tiles * mr * (16 * nt + 1) * 4 < 0x7fffffffL, "split-K workspace too small");
+    TORCH_CHECK(counters->numel() >= tiles, "counter buffer too small");
+    pp = part->data_ptr<float>();
+    cp = counters->data_ptr<int>();
+  }
+  void *yp = nullptr, *rp = nullptr, *qo = nullptr, *kp = nullptr, *vp = nullptr, *vr = nullptr;
+  long ldy = 0, ldr = 0, so_ld = 0, v_ld = 0;
+  float* so = nullptr;
+  const int *pos_p = nullptr, *sl = nullptr;
+  const float* cs = nullptr;
+  if (epi == 0 || epi == 3) {
+    TORCH_CHECK(y.has_value(), "y required");
+    check_bf16(*y, "y");
+    TORCH_CHECK(y->dim() == 2 && y->stride(1) == 1 && y->size(0) == M && y->size(1) == (epi == 3 ? N / 2 : N), "y shape");
+    TORCH_CHECK((uintptr_t)y->data_ptr() % 8 == 0 && (epi == 0 || (N % 32 == 0 && y->stride(0) % 4 == 0)), "y rows of 8 bytes");
+    yp = y->data_ptr();
+    ldy = y->stride(0);
+  }
+  if (epi == 1) {
+    TORCH_CHECK(res.has_value() && ssq_out.has_value(), "residual epilogue: res and ssq_out");
+    check_bf16(*res, "res");
+    check_f32(*ssq_out, "ssq_out");
+    TORCH_CHECK(res->dim() == 2 && res->stride(1) == 1 && res->size(0) == M && res->size(1) == N && N % 4 == 0 && res->stride(0) % 4 == 0 &&
+                    (uintptr_t)res->data_ptr() % 8 == 0, "res [M, N], 8-B rows");
+    TORCH_CHECK(ssq_out->dim() == 2 && ssq_out->size(0) >= tiles && ssq_out->size(1) >= M && ssq_out->stride(1) == 1, "ssq_out [>= tiles, >= M]");
+    rp = res->data_ptr();
+    ldr = res->stride(0);
+    so = ssq_out->data_ptr<float>();
+    so_ld = ssq_out->stride(0);
+  }
+  if (epi == 2) {
+    TORCH_CHECK(pos.has_value() && cos_sin.has_value() && slots.has_value() && q_out.has_value() && kc.has_value() && vc.has_value(), "QKV operands");
+    check_i32(*pos, "pos");
+    check_i32(*slots, "slots");
+    check_f32(*cos_sin, "cos_sin");
+    check_bf16(*q_out, "q_out");
+    check_bf16(*kc, "k_cache");
+    check_bf16(*vc, "v_cache");
+    TORCH_CHECK(d >= 32 && d % 32 == 0 && N == (nq + 2 * nkv) * d, "q | k | v columns");
+    TORCH_CHECK(pos->numel() >= M && slots->numel() >= M && cos_sin->dim() == 2 && cos_sin->size(1) == d && cos_sin->is_contiguous(), "pos / slots / cos_sin");
+    TORCH_CHECK(q_out->is_contiguous() && q_out->numel() == M * nq * d && kc->is_contiguous() && vc->is_contiguous(), "q_out / caches");
+    TORCH_CHECK(kc->dim() == 4 && kc->size(1) == nkv && kc->size(2) == 16 && kc->size(3) == d, "k_cache [blocks, nkv, 16, d]");
+    TORCH_CHECK(vc->dim() == 4 && vc->size(1) == nkv && vc->size(2) == d && vc->size(3) == 16, "v_cache [blocks, nkv, d, 16]");
+    pos_p = pos->data_ptr<int>();
+    sl = slots->data_ptr<int>();
+    cs = cos_sin->data_ptr<float>();
+    qo = q_out->data_ptr();
+    kp = kc->data_ptr();
+    vp = vc->data_ptr();
+    if (v_rows.has_value()) {
+      check_bf16(*v_rows, "v_rows");
+      TORCH_CHECK(v_rows->dim() == 2 && v_rows->size(0) == M && v_rows->size(1) == nkv * d && v_rows->stride(1) == 1 && v_rows->stride(0) % 4 == 0 &&
+                      (uintptr_t)v_rows->data_ptr() % 8 == 0, "v_rows [M, nkv d]");
+      vr = v_rows->data_ptr();
+      v_ld = v_rows->stride(0);
+    }
+  }
+  ok(dllm_dgemm(x.data_ptr(), M > 1 ? x.stride(0) : K, w.data_ptr(), yp, ldy, (int)M, (int)N, (int)K, (int)nt, (int)vs, (int)splits, (int)epi, pp, cp,
+                rp, ldr, so, so_ld, (float)scale, (float)eps, pos_p, cs, sl, qo, kp, vp, vr, v_ld, (int)nq, (int)nkv, (int)d, stream()),
+     "dgemm");
+  return epi == 1 ? tiles : 0;
+}
+
 // Small-batch (M <= 16) MFMA GEMM with a fused decoder epilogue (csrc/kernels/skinny_gemm.hip
 // skinny_epi_kernel): epi 0 plain (y), 1 residual add (res in place + per-tile row sums -> ssq_out),
 // 2 QKV (RoPE, q_out, paged K / V^T), 3 SwiGLU (y = act [M, N/2]).  w: [N, K] or the panel copy
@@ -2752,6 +2844,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("skinny_gemm", &skinny_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("ntw"), py::arg("splits"), py::arg("swiglu"),
         py::arg("part"), py::arg("counters"), py::arg("vs") = 1);
   m.def("skinny_epi", &skinny_epi);
+  m.def("dgemm", &dgemm);
   m.def("gemv", &gemv);
   m.def("gemv_norm", &gemv_norm);
   m.def("gemv_slots", &gemv_slots);

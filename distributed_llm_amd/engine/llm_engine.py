@@ -346,7 +346,8 @@ class LLMEngine:
             if big:
                 with ops.gemm.workspace_owner(self._ws_owner):
                     ops.gemm_autotune(big, [b for b in self.buckets if b <= ops.gemm.MAX_M], self.device,
-                                      verbose=os.environ.get("DLLM_VERBOSE") == "1")
+                                      verbose=os.environ.get("DLLM_VERBOSE") == "1",
+                                      frag=[] if m.lm_head_r is None else [b[:2] for b in big])
                     ops.gemm.reserve(self.device)
             return
         shapes = set()
@@ -363,7 +364,9 @@ class LLMEngine:
             ops.gemm_autotune(sorted(shapes), [b for b in self.buckets if b <= ops.gemm.MAX_M], self.device,
                               verbose=os.environ.get("DLLM_VERBOSE") == "1", fused=fused,
                               qkv_dims=(m.nq, m.nkv, m.d) if fused else None,
-                              qkv_cache=self.kv_caches[0] if fused else None)
+                              qkv_cache=self.kv_caches[0] if fused else None,
+                              frag=[tuple(w.shape) for n, w in [*L.items(), ("lm_head", m.lm_head)]
+                                    if n + "_r" in L or (n == "lm_head" and m.lm_head_r is not None)])
             ops.gemm.reserve(self.device)
 
     # Decode attention split-K.  Default: a static split count sized to the batch (_splits_for),

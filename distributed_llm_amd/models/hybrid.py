@@ -95,13 +95,24 @@ from ..parallel.comm import SINGLE, ParallelContext
 from .configs import DenseSpec, HybridConfig, LayerSpec, MixerSpec, MoESpec, QTempSpec, RopeSpec
 
 
-def _mm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM."""
+# projections that get a fragment-major copy (ops.gemm.frag_weight) for steps of up to 64 rows, named with "_r" behind
+_PROJECTIONS = ("proj", "out", "dqkv", "uq", "o", "up", "down", "in", "x", "dt", "qkvg", "lo", "ro", "sh_up", "sh_down")
+
+
+def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
+    """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy."""
+    if wf is not None and ops.gemm.dg_takes(x):
+        return ops.linear(x, w, wf=wf, keep_order=keep_order)
     if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1
             and x.shape[1] % 64 == 0 and w.shape[0] % 64 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and w.is_contiguous()):
         return ops.linear(x, w)
     return F.linear(x, w)
+
+
+def _pm(x: torch.Tensor, L: Dict[str, torch.Tensor], name: str) -> torch.Tensor:
+    wf = L.get(name + "_r")
+    return _mm(x, L[name]) if wf is None else _mm(x, L[name], wf, L["order_kept"])
 
 
 class HybridModel:
@@ -143,6 +154,7 @@ class HybridModel:
         self._max_pos = 0
         raw = self._load(weights) if weights else self._random(seed, init_std)
         self._place(raw)
+        self._place_fragments()
         self.ensure_positions(2048)
 
     # ------------------------------------------------------------------ weights
@@ -515,6 +527,29 @@ class HybridModel:
                     assert D["sh_down"].shape[1] == f.shared_ff
             self.layers.append(D)
 
+    @property
+    def order_kept(self) -> bool:
+        """Small products keep the order of their sums: an mLSTM head divides by sums of a few thousandths of their terms, and a last
+        bit ahead of it becomes tenths of a logit."""
+        return any(m.kind == "mlstm" for L in self.cfg.layers for m in L.mixer.parts)
+
+    def _place_fragments(self) -> None:
+        """Fragment-major copies of the projections and the head for the decode GEMM (ops.gemm.frag_weight), while they fit in a
+        quarter of the memory still free.  Where the order of sums is kept, of those alone that ops.linear multiplies anyway."""
+        self.lm_head_r: Optional[torch.Tensor] = None
+        if self.dtype != torch.bfloat16 or self.device.type != "cuda" or not ops.native_available():
+            return
+        takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
+        todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
+        extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
+        if extra > 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+            return
+        for L, n in todo:
+            L[n + "_r"] = ops.gemm.frag_weight(L[n])
+            L["order_kept"] = self.order_kept
+        if takes(self.lm_head):
+            self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
+
     def _fuse(self, parts: List[torch.Tensor], put) -> Tuple[torch.Tensor, int]:
         """One projection for several that read the same input, and its rows; bf16 models on the GPU get
         zero rows behind them up to a multiple of 64, the output tile of the tuned GEMMs."""
@@ -551,8 +586,7 @@ class HybridModel:
         """(out, in) of the large bf16 weights that run on the tuned GEMMs (the engine times their plans)."""
         if self.dtype != torch.bfloat16:
             return []
-        names = ("proj", "out", "dqkv", "uq", "o", "up", "down", "in", "x", "dt", "qkvg", "lo", "ro", "sh_up", "sh_down")
-        ws = [L[k] for L in self.layers for k in names if k in L] + [self.lm_head] + \
+        ws = [L[k] for L in self.layers for k in _PROJECTIONS if k in L] + [self.lm_head] + \
             ([self.loop_in] if self.cfg.loop is not None else [])
         return sorted({tuple(w.shape) for w in ws if w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and w.numel() >= 1 << 22})
 
@@ -561,7 +595,8 @@ class HybridModel:
         if self.cfg.loop is not None:
             n += sum(x.numel() * x.element_size() for x in (self.loop_in, self.loop_step))
         n += 0 if self.cfg.tied_head else self.lm_head.numel() * self.lm_head.element_size()
-        return n + sum(x.numel() * x.element_size() for L in self.layers for x in L.values() if torch.is_tensor(x))
+        return n + sum(x.numel() * x.element_size() for L in self.layers for k, x in L.items()
+                       if torch.is_tensor(x) and not k.endswith("_r"))
 
     def decode_read_bytes(self, top_only: bool = True) -> int:
         """Weight bytes one decode token reads (routed experts: ``top`` of them)."""
@@ -571,7 +606,7 @@ class HybridModel:
         for i, _ in self.cfg.runs:      # a looped layer is read in every pass
             L, S = self.layers[i], self.cfg.layers[i]
             for k, x in L.items():
-                if not torch.is_tensor(x) or k == "uv":      # (prompt steps read that layout of uvT)
+                if not torch.is_tensor(x) or k == "uv" or k.endswith("_r"):      # (prompt steps read that layout of uvT; copies)
                     continue
                 b = x.numel() * x.element_size()
                 if k in ("w1", "w2", "w2d") and top_only and isinstance(S.mlp, MoESpec):
@@ -679,22 +714,22 @@ class HybridModel:
     def _mamba(self, L, m: MixerSpec, x, meta, cache):
         conv_state, ssm_state = cache
         rows = meta.state_rows
-        xz = _mm(x, L["in"])
+        xz = _pm(x, L, "in")
         xc = seqmix.causal_conv_silu(xz, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
                                      all_rows=self._all_rows(xz, meta))
-        dbc = _mm(xc, L["x"])
-        dt_raw = _mm(dbc[:, :m.dt_rank], L["dt"])
+        dbc = _pm(xc, L, "x")
+        dt_raw = _pm(dbc[:, :m.dt_rank], L, "dt")
         y = seqmix.selective_scan(xc, dt_raw, L["dt_b"], L["A"], dbc, m.dt_rank, L["D"], xz, ssm_state, conv_state,
                                   meta.qstart, meta.qlen, meta.ctx, rows, longest=self._longest(meta))
-        return _mm(y, L["o"])
+        return _pm(y, L, "o")
 
     def _retention(self, L, m: MixerSpec, x, positions, meta, cache):
-        qkvg = _mm(x, L["qkvg"])
+        qkvg = _pm(x, L, "qkvg")
         rot = m.rot.dims if m.rot is not None else 0
         table = self._table(m) if rot else self._any_table()
         o = seqmix.retention(qkvg, m.heads, m.dim, m.vdim, table, rot, L["decay"], cache[0], self.cfg.rms_eps,
                              positions, meta.qstart, meta.qlen, meta.ctx, meta.state_rows, longest=self._longest(meta))
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     def _any_table(self) -> torch.Tensor:
         if not self._rot:
@@ -705,7 +740,7 @@ class HybridModel:
         """Latent attention behind a query latent: on the cached latents (absorbed form), or for steps of
         longer prompt portions on keys and values made from them."""
         T, H, eps, rd = x.shape[0], m.heads, self.cfg.rms_eps, m.rot_dim
-        down = _mm(x, L["dqkv"])                    # query latent | latent | rotated key part (| head gates)
+        down = _pm(x, L, "dqkv")                    # query latent | latent | rotated key part (| head gates)
         g0 = m.q_rank + m.kv_rank + rd
         gate = down[:, g0:g0 + H] if m.head_gate else None
         table = self._table(m) if rd else self._any_table()
@@ -717,7 +752,7 @@ class HybridModel:
         lat = None if expand else torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)
         cq = seqmix.latent_kv_write(down[:, m.q_rank:g0], m.kv_rank, L["dkv_norm"], eps, positions, table, meta.slots,
                                     cache[0], m.rot_half, down[:, :m.q_rank], L["dq_norm"], None if all_rows else lat)
-        q = _mm(cq, L["uq"])                                            # [T, H (dim + rot)]
+        q = _pm(cq, L, "uq")                                            # [T, H (dim + rot)]
         if expand:
             q = seqmix.latent_q_prep(q, H, m.dim, rd, positions, table, m.scale, m.rot_half)
             k, v, pages = seqmix.latent_expand(cache[0], meta.block_tables, meta.ctx, L["uk"], L["uv"])
@@ -726,7 +761,7 @@ class HybridModel:
             splits = seqmix.gqa_splits(int(ts.numel()), H, meta.max_ctx) if mfma else 1
             o = seqmix.paged_gqa_attention(q, k, v, pages, meta.qstart, meta.qlen, meta.ctx, ts, tt, gate, mfma, splits,
                                            all_rows=True, sinks=L.get("sink"))
-            return _mm(o, L["o"])
+            return _pm(o, L, "o")
         qn = q.view(T, H, m.dim + rd)[:, :, :m.dim].transpose(0, 1)
         qa = torch.bmm(qn, L["uk"])                                     # key up-projection absorbed: [H, T, rank]
         rows = (seqmix.LAT_ROWS if meta.host_qlen is None else
@@ -740,7 +775,7 @@ class HybridModel:
             o = seqmix.gate_heads(o, gate, torch.empty((T, H * m.vdim), dtype=x.dtype, device=x.device))
         else:
             o = o.transpose(0, 1).reshape(T, H * m.vdim)
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     @staticmethod
     def _left_cols(a: MixerSpec) -> int:
@@ -751,7 +786,7 @@ class HybridModel:
         conv_state, state = cache
         rows = meta.state_rows
         c = 2 * m.kv_heads * m.dim + m.heads * m.vdim
-        proj = _mm(x, L["proj"])                                        # q | k | v | gate | beta | decay logits
+        proj = _pm(x, L, "proj")                                        # q | k | v | gate | beta | decay logits
         single = meta.host_qlen is None      # a decode step: the convolution refills its slots itself
         qkv = seqmix.causal_conv_silu(proj, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
                                       refill=single, all_rows=self._all_rows(proj, meta))
@@ -759,13 +794,13 @@ class HybridModel:
             seqmix.conv_state_refill(proj, conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
         o = seqmix.delta_rule(qkv, proj[:, c:], m.heads, m.kv_heads, m.dim, m.vdim, L["neg_a"], L["dt_b"], L["hnorm"],
                               self.cfg.rms_eps, state, meta.qstart, meta.qlen, meta.ctx, rows, longest=self._longest(meta))
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     def _parallel(self, L, m: MixerSpec, x, positions, meta, cache):
         """Both sides' outputs, un-normed: the caller's residual launch norms and averages them."""
         a, b, eps = m.left, m.right, self.cfg.rms_eps
         k_cache, v_cache, state = cache
-        proj = _mm(x, L["proj"])
+        proj = _pm(x, L, "proj")
         nl = self._left_cols(a)
         rot = a.rot.dims if a.rot is not None else 0
         table = self._table(a) if rot else self._any_table()
@@ -779,14 +814,14 @@ class HybridModel:
                                         gate, mfma, splits)
         ro = seqmix.lightning_attention(proj[:, nl:], b.heads, b.dim, b.vdim, L["decay"], state, eps, L["rnorm"],
                                         meta.qstart, meta.qlen, meta.ctx, meta.state_rows, longest=self._longest(meta))
-        return _mm(lo, L["lo"]), _mm(ro, L["ro"])
+        return _pm(lo, L, "lo"), _pm(ro, L, "ro")
 
     def _diff_attention(self, L, m: MixerSpec, x, positions, meta, cache):
         """Both maps of every head run as rows of one grouped-query attention over 2 kv_heads key
         heads and kv_heads shared value heads; the maps are combined afterwards."""
         k_cache, v_cache = cache
         own = m.kv_from is None
-        proj = _mm(x, L["proj"])
+        proj = _pm(x, L, "proj")
         rot = m.rot.dims if m.rot is not None else 0
         table = self._table(m) if rot else self._any_table()
         q = seqmix.qk_norm_prep(proj, L["bias"], m.heads, m.kv_heads, 2, m.dim, m.vdim, L["qnorm"], L["knorm"], table, rot,
@@ -799,7 +834,7 @@ class HybridModel:
         a = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
                                        None, mfma, splits, window=m.window, out_f32=True)
         o = seqmix.diff_combine(a, m.heads, m.kv_heads, m.vdim, L["lam"], self.cfg.rms_eps, 1.0 - m.diff, self.dtype)
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     def _input_conv(self, L, h, meta, state):
         """h + a short causal convolution of h over time (per channel, no activation); the slot keeps
@@ -815,7 +850,7 @@ class HybridModel:
     def _sink_attention(self, L, m: MixerSpec, x, positions, meta, cache):
         k_cache, v_cache = cache[0], cache[1]
         own = m.kv_from is None
-        proj = _mm(x, L["proj"])                                        # q | k | v, or q alone
+        proj = _pm(x, L, "proj")                                        # q | k | v, or q alone
         rot = m.rot.dims if m.rot is not None else 0
         table = self._table(m) if rot else self._any_table()
         # a step with padding rows (decode graphs): the prep launch clears the attention output's rows
@@ -829,11 +864,11 @@ class HybridModel:
         o = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
                                        None, mfma, splits, window=m.window, keep_first=m.keep_first, sink=m.sink,
                                        all_rows=self._all_rows(x, meta), out=out)
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     def _biased_attention(self, L, m: MixerSpec, x, positions, meta, cache):
         k_cache, v_cache = cache[0], cache[1]
-        proj = _mm(x, L["proj"])                                        # q | k | v (| head gates)
+        proj = _pm(x, L, "proj")                                        # q | k | v (| head gates)
         n = (m.heads + m.kv_heads) * m.dim + m.kv_heads * m.vdim
         gate = proj[:, n:n + m.heads] if m.head_gate else None
         all_rows = self._all_rows(x, meta)      # else the prep launch clears the attention output's padding rows
@@ -846,14 +881,14 @@ class HybridModel:
         splits = seqmix.gqa_splits(int(ts.numel()), m.kv_heads, meta.max_ctx, m.window) if mfma else 1
         o = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
                                        gate, mfma, splits, window=m.window, all_rows=all_rows, out=out, slopes=L["slopes"])
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     # ------------------------------------------------------------------ mixer and feed-forward side by side
     def _gated_attention_ff(self, L, m: MixerSpec, f: Optional[DenseSpec], x, positions, meta, cache):
         """mixer(x) + ff(x): one projection in, one out; the heads and the activations meet in one buffer."""
         k_cache, v_cache = cache[0], cache[1]
         T, hv = x.shape[0], m.heads * m.vdim
-        proj = _mm(x, L["proj"])                                        # q | k | v | gate | up
+        proj = _pm(x, L, "proj")                                        # q | k | v | gate | up
         g0 = (m.heads + m.kv_heads) * m.dim + m.kv_heads * m.vdim
         both = torch.empty((T, hv + (f.ff if f is not None else 0)), dtype=x.dtype, device=x.device)
         o = both[:, :hv]
@@ -867,13 +902,13 @@ class HybridModel:
         splits = seqmix.gqa_splits(int(ts.numel()), m.kv_heads, meta.max_ctx, chunk=m.chunk) if mfma else 1
         seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
                                    proj[:, g0:g0 + hv], mfma, splits, out=o, chunk=m.chunk, softcap=m.softcap, sinks=L["sink"])
-        return _mm(both, L["out"])
+        return _pm(both, L, "out")
 
     def _latent_ff(self, L, m: MixerSpec, f: Optional[DenseSpec], x, positions, meta, cache):
         """mixer(x) + ff(x) with latent attention (direct queries, gated heads): on the cached latents
         (absorbed form), or for steps of longer prompt portions on keys and values made from them."""
         T, H, hv = x.shape[0], m.heads, m.heads * m.vdim
-        proj = _mm(x, L["proj"])                                        # q | latent | gate | up
+        proj = _pm(x, L, "proj")                                        # q | latent | gate | up
         c0 = H * m.dim
         g0 = c0 + m.kv_rank
         both = torch.empty((T, hv + (f.ff if f is not None else 0)), dtype=x.dtype, device=x.device)
@@ -888,7 +923,7 @@ class HybridModel:
             splits = seqmix.gqa_splits(int(ts.numel()), H, meta.max_ctx) if mfma else 1
             seqmix.paged_gqa_attention(q, k, v, table, meta.qstart, meta.qlen, meta.ctx, ts, tt, proj[:, g0:g0 + hv], mfma, splits,
                                        out=both[:, :hv])
-            return _mm(both, L["out"])
+            return _pm(both, L, "out")
         lat = torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)     # padding rows cleared by the prep launch
         seqmix.latent_prep(proj, c0, L["dkv_norm"], self.cfg.rms_eps, meta.slots, cache[0], g0 + hv, act, zero=lat)
         q = proj[:, :c0]
@@ -899,7 +934,7 @@ class HybridModel:
         lat = seqmix.latent_attention(qa, q, m.dim, 0, positions, self._any_table(), cache[0], meta.block_tables, meta.qstart,
                                       meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat)
         seqmix.gate_heads(torch.bmm(lat, L["uvT"]), proj[:, g0:g0 + hv], both[:, :hv])
-        return _mm(both, L["out"])
+        return _pm(both, L, "out")
 
     def _hidden_parallel(self, x, xl, positions, meta, kv_caches):
         """The layer loop of ``parallel_ff`` models on the f32 stream x [T, width] (the embedding output):
@@ -948,7 +983,7 @@ class HybridModel:
         conv_state, state = cache
         rows = meta.state_rows
         inner = m.heads * m.vdim
-        proj = _mm(x, L["in"])                                          # z | x | B | C | dt
+        proj = _pm(x, L, "in")                                          # z | x | B | C | dt
         xbc_in = proj[:, inner:]
         single = meta.host_qlen is None      # a decode step: the convolution refills its slots itself
         xbc = seqmix.causal_conv_silu(xbc_in, L["conv"], L["conv_b"], conv_state, meta.qstart, meta.qlen, meta.ctx, rows,
@@ -957,24 +992,24 @@ class HybridModel:
             seqmix.conv_state_refill(xbc_in, conv_state, meta.qstart, meta.qlen, meta.ctx, rows)
         y = seqmix.ssd_scan(xbc, proj, 2 * inner + 2 * m.groups * m.state, m.heads, m.vdim, m.state, m.groups, L["dt_b"],
                             L["neg_a"], L["D"], state, meta.qstart, meta.qlen, meta.ctx, rows)
-        return _mm(seqmix.gated_group_norm(y, proj, L["gnorm"], m.norm_groups, self.cfg.rms_eps, self.dtype), L["o"])
+        return _pm(seqmix.gated_group_norm(y, proj, L["gnorm"], m.norm_groups, self.cfg.rms_eps, self.dtype), L, "o")
 
     def _mlstm(self, L, m: MixerSpec, x, meta, cache):
         state, nm = cache
-        proj = _mm(x, L["proj"])                                        # q | k | v | gate | input gate | forget gate
+        proj = _pm(x, L, "proj")                                        # q | k | v | gate | input gate | forget gate
         o = seqmix.mlstm(proj, m.heads, m.dim, m.vdim, L["gate_b"], m.gate_cap, state, nm, self.cfg.rms_eps, L["hnorm"],
                          meta.qstart, meta.qlen, meta.ctx, meta.state_rows)
-        return _mm(o, L["o"])
+        return _pm(o, L, "o")
 
     def _dense(self, L, f: DenseSpec, x):
-        z = _mm(x, L["up"])
+        z = _pm(x, L, "up")
         if f.act == "clamped_glu":      # the down projection's bias rides in the residual launch
             a = seqmix.glu_act(z, L.get("up_b"), "clamped", f.limit, 1.702)
         elif f.act == "gelu_glu":       # likewise
             a = seqmix.glu_act(z, L.get("up_b"), "gelu_tanh")
         else:
             a = seqmix.polynorm(z, L["act"], self.cfg.rms_eps) if f.act == "polynorm" else seqmix.gelu_erf(z)
-        return _mm(a, L["down"])
+        return _pm(a, L, "down")
 
     def _experts_swiglu(self, L, f: MoESpec, x, tail=None):
         """Sigmoid router in f32 with group-limited top-k, weights = the chosen scores; SwiGLU experts
@@ -1002,7 +1037,7 @@ class HybridModel:
         if f.identity:
             out.update(h=x, hw=idw)
         if f.shared_ff:
-            out.update(y2=_mm(seqmix.glu_act(_mm(x, L["sh_up"])), L["sh_down"]), g2=logits[:, R] if f.shared_gate else None)
+            out.update(y2=_pm(seqmix.glu_act(_pm(x, L, "sh_up")), L, "sh_down"), g2=logits[:, R] if f.shared_gate else None)
         return out
 
     def _swiglu_experts(self, L, f: MoESpec, x, ids, w, tail=None):
@@ -1016,7 +1051,7 @@ class HybridModel:
             L["w2d"] = L["w2"].permute(1, 0, 2).reshape(x.shape[1], -1).contiguous()
         g = seqmix.dense_gate(ids, w, f.experts)
         a = seqmix.swiglu_scale(_mm(x, L["w1"].view(f.experts * 2 * f.ff, -1)), g, f.ff)
-        return _mm(a, L["w2d"])
+        return _pm(a, L, "w2d")
 
     def _experts(self, L, f: MoESpec, x, tail=None):
         """``tail`` (ops.moe_ffn_tg): where the experts run on the grouped GEMM, their sum ends in the stream and None is
@@ -1041,9 +1076,9 @@ class HybridModel:
                 L["w2d"] = L["w2"].permute(1, 0, 2).reshape(x.shape[1], -1).contiguous()
             g = seqmix.dense_gate(ids, w, f.experts)
             a = seqmix.relu2_scale(_mm(x, L["w1"].view(f.experts * f.ff, -1)), g, f.ff)
-            y = _mm(a, L["w2d"])
+            y = _pm(a, L, "w2d")
         if f.shared_ff:
-            y = y + _mm(seqmix.relu2_scale(_mm(x, L["sh_up"])), L["sh_down"])
+            y = y + _pm(seqmix.relu2_scale(_pm(x, L, "sh_up")), L, "sh_down")
         return y
 
     # ------------------------------------------------------------------ forward
@@ -1160,13 +1195,13 @@ class HybridModel:
         return seqmix.rms_rows(sel, self.final_norm, eps, out_dtype=self.dtype, groups=cfg.norm_groups)
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        lg = _mm(hidden, self.lm_head)
+        lg = _mm(hidden, self.lm_head, self.lm_head_r)
         if self.cfg.logit_softcap > 0:
             return seqmix.softcap(lg, self.cfg.logit_softcap).to(lg.dtype)
         return lg if self.cfg.logit_scale == 1.0 else lg * self.cfg.logit_scale
 
     def logits_f32(self, hidden: torch.Tensor) -> torch.Tensor:
-        lg = _mm(hidden, self.lm_head)
+        lg = _mm(hidden, self.lm_head, self.lm_head_r)
         if self.cfg.logit_softcap > 0:
             return seqmix.softcap(lg, self.cfg.logit_softcap)
         return lg.float() * self.cfg.logit_scale

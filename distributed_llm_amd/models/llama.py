@@ -167,6 +167,7 @@ class LlamaModel:
         if weights:
             self.load_safetensors(weights)
         self.cos_sin = ops.rope_cos_sin(cfg.max_position, self.d, cfg.rope_theta, self.device, cfg.rope_scaling)
+        self.lm_head_r: Optional[torch.Tensor] = None       # fragment-major copy
         self.fused = self._fusable()
         if self.fused:
             self._fuse_weights()
@@ -212,6 +213,16 @@ class LlamaModel:
         for L in self.layers:
             for n in names:
                 L[n + "_p"] = ops.gemm.panel_weight(L[n])
+        # the decode GEMM's fragment-major copies, under the same rule (of what is then left)
+        extra += self.lm_head.numel() * self.lm_head.element_size()
+        free, _ = torch.cuda.mem_get_info(self.device)
+        if extra > 0.25 * free:
+            return
+        for L in self.layers:
+            for n in names:
+                L[n + "_r"] = ops.gemm.frag_weight(L[n], paired=n in ("wqkv_f", "wgu_f"))
+        if self.lm_head.shape[1] % 32 == 0:
+            self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
 
     def reference_layers(self) -> List[Dict[str, torch.Tensor]]:
         """Layer weights in the plain (unfused) layout, e.g. for a CPU reference forward."""
@@ -219,7 +230,7 @@ class LlamaModel:
             return self.layers
         out = []
         for L in self.layers:
-            R = {k: v for k, v in L.items() if k not in ("wqkv_f", "wgu_f") and not k.endswith("_p")}
+            R = {k: v for k, v in L.items() if k not in ("wqkv_f", "wgu_f") and not k.endswith(("_p", "_r"))}
             if "wqkv_f" in L:
                 R["wqkv"] = unfuse_qkv_weight(L["wqkv_f"], L["ln1"], self.nq, self.nkv, self.d)
             if "wgu_f" in L:
@@ -336,8 +347,8 @@ class LlamaModel:
 
     def weight_bytes(self) -> int:
         n = self.embed.numel() + (0 if self.lm_head is self.embed else self.lm_head.numel()) + self.final_norm.numel()
-        for L in self.layers:   # one copy of each matrix: the K-panel copies ("_p") duplicate bytes, not reads
-            n += sum(t.numel() for k, t in L.items() if not k.endswith("_p"))
+        for L in self.layers:   # one copy of each matrix: the K-panel ("_p") and fragment ("_r") copies duplicate bytes, not reads
+            n += sum(t.numel() for k, t in L.items() if not k.endswith(("_p", "_r")))
         return n * self.embed.element_size()
 
     # ------------------------------------------------------------------ forward
@@ -464,21 +475,21 @@ class LlamaModel:
             kc, vc = kv_caches[li]
             # column-parallel QKV (this rank's heads) with RMSNorm folded + RoPE + paged K/V write
             q = ops.gemm.qkv_rope_cache(r, L["wqkv_f"], ssq_a, n, eps, positions, self.cos_sin, meta.slots, kc, vc,
-                                        self.nq, self.nkv, self.d, wp=L.get("wqkv_f_p"), v_new=vn)
+                                        self.nq, self.nkv, self.d, wp=L.get("wqkv_f_p"), v_new=vn, wf=L.get("wqkv_f_r"))
             v_new = None
             if vn is not None:
                 q, v_new = q
             o = self._attention(q, kc, vc, meta, v_new=v_new)
             if not tp:
-                nb = ops.gemm.matmul_resadd(o.view(T, -1), L["wo"], r, ssq_b, wp=L.get("wo_p"))
+                nb = ops.gemm.matmul_resadd(o.view(T, -1), L["wo"], r, ssq_b, wp=L.get("wo_p"), wf=L.get("wo_r"))
             else:   # row-parallel o_proj: partial sums -> all-reduce + residual add + row statistics
-                nb = resadd(ops.linear(o.view(T, -1), L["wo"], wp=L.get("wo_p")), r, ssq_b)
+                nb = resadd(ops.linear(o.view(T, -1), L["wo"], wp=L.get("wo_p"), wf=L.get("wo_r")), r, ssq_b)
             if not cfg.is_moe:
-                act = ops.gemm.swiglu_matmul(r, L["wgu_f"], ssq_b, nb, eps, wp=L.get("wgu_f_p"))
+                act = ops.gemm.swiglu_matmul(r, L["wgu_f"], ssq_b, nb, eps, wp=L.get("wgu_f_p"), wf=L.get("wgu_f_r"))
                 if not tp:
-                    n = ops.gemm.matmul_resadd(act, L["wd"], r, ssq_a, wp=L.get("wd_p"))
+                    n = ops.gemm.matmul_resadd(act, L["wd"], r, ssq_a, wp=L.get("wd_p"), wf=L.get("wd_r"))
                 else:
-                    n = resadd(ops.linear(act, L["wd"], wp=L.get("wd_p")), r, ssq_a)
+                    n = resadd(ops.linear(act, L["wd"], wp=L.get("wd_p"), wf=L.get("wd_r")), r, ssq_a)
             else:
                 if not tp and self.moe_tg:      # norm and router, and combine and residual add, share a launch
                     x, ids, w = ops.norm_moe_router(r, L["ln2"], eps, L["wgate"], cfg.experts_per_token)
@@ -529,7 +540,7 @@ class LlamaModel:
 
     def logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """This rank's vocab shard of the logits: [S, V / tp] (bf16)."""
-        return ops.linear(hidden, self.lm_head)
+        return ops.linear(hidden, self.lm_head, wf=self.lm_head_r)
 
     def greedy(self, hidden: torch.Tensor) -> torch.Tensor:
         """Distributed arg-max over the vocab-parallel LM head -> token ids [S] int32."""

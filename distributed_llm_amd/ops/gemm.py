@@ -8,8 +8,9 @@ Kernels (csrc/kernels):
     block order, optional in-launch split-K) with the transformer epilogues used by the fused
     decoder layer (models/llama.py): QKV + RoPE + paged-KV write, residual add + row sums of
     squares (RMSNorm folded into the next GEMM), SwiGLU.  Any M (decode buckets and prefill).
+  * ``decode_gemm.hip`` (M <= 64): decode GEMMs with the same epilogues on fragment-major weight copies (``frag_weight``).
   * ``gemv.hip`` (M <= 8), ``skinny_gemm.hip`` (M <= 128): register-streaming decode GEMMs without
-    LDS tiling.
+    LDS tiling, on row-major weights.
   * hipBLASLt via ``F.linear`` stays a candidate, so a custom kernel is used only where it wins.
 
 Plans are measured once per (M, N, K) OUTSIDE graph capture (``autotune``, called by the engine
@@ -108,6 +109,25 @@ def panel_weight(w: torch.Tensor) -> torch.Tensor:
     return w.view(N, K // 64, 64).transpose(0, 1).contiguous()
 
 
+# Fragment-major weight copies of the decode GEMM (csrc/kernels/decode_gemm.hip): a wave's load of a weight fragment is one contiguous
+# 1 KB instead of 16 rows of 64 bytes.
+DG_MAX_M = 64
+_PAIR_ROWS = [*range(8), *range(16, 24), *range(8, 16), *range(24, 32)]
+
+
+def frag_weight(w: torch.Tensor, paired: bool = False) -> torch.Tensor:
+    """[N, K] -> [ceil(N / 16), K / 32, 64, 8]: of a 16-column tile and 32 k, lane 16 g + r holds W[16 t + r][32 s + 8 g ...+ 7]; rows past
+    N are zeros.  ``paired`` (the QKV and gate|up weights of models.llama, pairs 16 rows apart in groups of 32): pairs 8 rows apart."""
+    N, K = w.shape
+    if K % 32 or (paired and N % 32):
+        raise ValueError(f"frag_weight: {N} x {K}")
+    if paired:
+        w = w.view(N // 32, 32, K)[:, _PAIR_ROWS].reshape(N, K)
+    elif N % 16:
+        w = torch.cat([w, w.new_zeros(16 - N % 16, K)])
+    return w.view(-1, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).reshape(-1, K // 32, 64, 8).contiguous()
+
+
 def _nk(w: torch.Tensor) -> Tuple[int, int]:
     """(N, K) of a row-major [N, K] or panel [K / 64, N, 64] weight."""
     return (w.shape[1], w.shape[0] * 64) if w.dim() == 3 else (w.shape[0], w.shape[1])
@@ -129,7 +149,8 @@ class _Planner:
     def __init__(self):
         self.plans: Dict[Tuple[int, int, int, bool], Tuple] = {}     # best overall, for linear()
         self.tg_plans: Dict[Tuple[int, int, int], Tuple] = {}        # best tgemm tile, for the fused ops
-        self.fused_core: Dict[Tuple[int, int, int], str] = {}        # "tg" | "lin" | "gemvR" per tuned shape
+        self.dg_plans: Dict[Tuple[int, int, int], Tuple] = {}        # decode GEMM (nt, vs, splits), where it beats plans[...]
+        self.fused_core: Dict[Tuple[int, int, int], str] = {}        # "tg" | "lin" | "gemvR" | "skES" | "dgN.V.S" per tuned shape
         self.fused_opts: Dict[Tuple[int, int, int], Dict[str, float]] = {}   # measured us per core choice
         self.ws: Dict[Tuple, Tuple[torch.Tensor, torch.Tensor]] = {}
         self.sk_tables: Dict[Tuple, Tuple[torch.Tensor, int]] = {}   # stream-K segment lists per shape
@@ -434,19 +455,51 @@ def _key(x, w, swiglu):
     return (x.shape[0], w.shape[0], w.shape[1], bool(swiglu))
 
 
+def dgemm(x: torch.Tensor, wf: torch.Tensor, n: int, epi: int, plan: Tuple[int, int, int], y=None, res=None, ssq_out=None,
+          scale: float = 0.0, eps: float = 0.0, pos=None, cos_sin=None, slots=None, q_out=None, kc=None, vc=None, v_rows=None,
+          nq: int = 0, nkv: int = 0, d: int = 0) -> int:
+    """One launch of the decode GEMM on ``wf`` = frag_weight of an [n, K] weight; ``plan`` = (16-column tiles a workgroup, splits a
+    workgroup, splits of K)."""
+    nt, vs, splits = plan
+    M, K = x.shape
+    kchunk = (-(-K // splits) + 31) // 32 * 32
+    gy, tiles = -(-(-(-K // kchunk)) // vs), -(-n // (16 * nt))
+    part = cnt = None
+    if gy > 1:
+        part, cnt = _P.workspace(x.device, gy * vs * tiles * -(-M // 16) * 16 * (16 * nt + 1), tiles)
+    return int(_native(x).dgemm(x, wf, n, int(epi), nt, vs, splits, y, part, cnt, res, ssq_out, float(scale), float(eps), pos, cos_sin,
+                                slots, q_out, kc, vc, v_rows, int(nq), int(nkv), int(d)))
+
+
+def dg_takes(x: torch.Tensor) -> bool:
+    """The decode GEMM reads these rows: up to 64, 16-byte aligned."""
+    return 0 < x.shape[0] <= DG_MAX_M and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
+        (x.shape[0] == 1 or x.stride(0) >= x.shape[1]) and x.data_ptr() % 16 == 0
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
-           wp: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``x @ w.T`` on the shape's tuned plan; ``wp``: the panel copy a tgemm plan streams."""
+           wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
+    """``x @ w.T`` on the shape's tuned plan; ``wp``: the panel copy a tgemm plan streams, ``wf``: the fragment-major copy of the
+    decode GEMM, which takes the untimed products of up to 64 rows with the splits and the order of sums they have without it, and
+    timed ones where it was faster, or with ``keep_order`` where the plan is a skinny one, whose sums it keeps."""
     if not x.is_cuda or os.environ.get("DLLM_GEMM") == "blas":
         return F.linear(x, w) if out is None else torch.matmul(x, w.t(), out=out)
+    M, (N, K) = x.shape[0], w.shape
     plan, together = _P.plans.get(_key(x, w, False)), 1
-    if plan is None:
-        if x.shape[0] > MAX_M:
-            plan = ("blas",)
-        else:
-            plan = _heuristic(x.shape[0], w.shape[0], w.shape[1])
-            if plan[0] == "skinny":
-                together = _splits_together(x.shape[0], w.shape[0], w.shape[1], plan)
+    dg = _P.dg_plans.get((M, N, K)) if wf is not None and not keep_order else None
+    timed = plan is not None
+    if not timed:
+        plan = _heuristic(M, N, K) if M <= MAX_M else ("blas",)
+    if plan[0] == "skinny" and (wf is not None or not timed):
+        same = ("skinny", min(plan[1], 2), plan[2])
+        together = _splits_together(M, N, K, same)
+        if wf is not None and dg is None:
+            dg = (same[1], together, same[2])
+        together = 1 if timed else together
+    if dg is not None and dg_takes(x):
+        y = out if out is not None else torch.empty((M, N), dtype=x.dtype, device=x.device)
+        dgemm(x, wf, N, EPI_PLAIN, dg, y=y)
+        return y
     return _run_plan(plan, x, w, False, out, wp, together)
 
 
@@ -544,6 +597,17 @@ def skinny_epi(x: torch.Tensor, w: torch.Tensor, epi: int, splits: int, y=None, 
                                      int(d)))
 
 
+def fused_dg(x: torch.Tensor, N: int, K: int, wf: Optional[torch.Tensor]) -> Optional[Tuple[int, int, int]]:
+    """Plan of the decode GEMM (csrc/kernels/decode_gemm.hip) if the autotuner picked it for this fused op's shape (``fused_core`` =
+    ``dg<nt>.<vs>.<splits>``) and the caller keeps its weight copy, else None."""
+    if wf is None:
+        return None
+    c = os.environ.get("DLLM_FUSED_CORE") or _P.fused_core.get((x.shape[0], N, K))
+    if not c or not c.startswith("dg") or not dg_takes(x):
+        return None
+    return tuple(int(v) for v in c[2:].split("."))
+
+
 def _core(x: torch.Tensor, w: torch.Tensor, wp: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Plain product for the split (core + epilogue) form of a fused op: the tuned plan of this
     shape (M <= MAX_M), hipBLASLt above."""
@@ -552,7 +616,7 @@ def _core(x: torch.Tensor, w: torch.Tensor, wp: Optional[torch.Tensor] = None) -
 def qkv_rope_cache(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: int, eps: float,
                    positions: torch.Tensor, cos_sin: torch.Tensor, slots: torch.Tensor, k_cache: torch.Tensor,
                    v_cache: torch.Tensor, nq: int, nkv: int, d: int, wp: Optional[torch.Tensor] = None,
-                   v_new: Optional[torch.Tensor] = None):
+                   v_new: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None):
     """q [T, nq, d] of ``rope(rmsnorm(r) . Wqkv^T)``, K/V written to the paged caches, one launch.
 
     ``w`` is the folded/permuted weight of models.llama.fuse_qkv_weight; ``ssq[:ssq_n]`` holds
@@ -568,6 +632,11 @@ def qkv_rope_cache(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: i
     if T == 0:
         return q if v_new is None else (q, None)
     out = (lambda used: q if v_new is None else (q, v_new if used else None))
+    dg = fused_dg(r, w.shape[0], H, wf)
+    if dg:
+        dgemm(r, wf, w.shape[0], EPI_QKV, dg, scale=1.0 / H, eps=eps, pos=positions, cos_sin=cos_sin, slots=slots, q_out=q, kc=k_cache,
+              vc=v_cache, v_rows=v_new, nq=nq, nkv=nkv, d=d)
+        return out(True)
     R = fused_gemv_r(r, w.shape[0])
     if R:
         _native(r).gemv_qkv(r, w, ssq, int(ssq_n), 1.0 / H, float(eps), positions, cos_sin, slots, q, k_cache,
@@ -590,10 +659,13 @@ def qkv_rope_cache(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: i
 
 
 def matmul_resadd(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, ssq_out: torch.Tensor,
-                  wp: Optional[torch.Tensor] = None) -> int:
+                  wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None) -> int:
     """``residual += x . w^T`` (bf16 rounding as ``rms_norm``'s residual add) and the partial row
     sums of the new residual's squares into ``ssq_out[:slots]``; returns ``slots``."""
     M, N, K = x.shape[0], w.shape[0], w.shape[1]
+    dg = fused_dg(x, N, K, wf) if M else None
+    if dg:
+        return dgemm(x, wf, N, EPI_RESADD, dg, res=residual, ssq_out=ssq_out)
     R = fused_gemv_r(x, N) if M else 0
     if R:
         return int(_native(x).gemv_resadd(x, w, residual, ssq_out, R))
@@ -609,11 +681,15 @@ def matmul_resadd(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, ssq_
 
 
 def swiglu_matmul(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: int, eps: float,
-                  wp: Optional[torch.Tensor] = None) -> torch.Tensor:
+                  wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``silu(g) * u`` with ``[g | u] = rmsnorm(r) . Wgu^T`` (interleaved rows, models.llama
     .fuse_gate_up_weight) -> [T, I]."""
     T, H = r.shape
     act = torch.empty((T, w.shape[0] // 2), dtype=r.dtype, device=r.device)
+    dg = fused_dg(r, w.shape[0], H, wf) if T else None
+    if dg:
+        dgemm(r, wf, w.shape[0], EPI_SWIGLU, dg, y=act, scale=1.0 / H, eps=eps)
+        return act
     R = fused_gemv_r(r, w.shape[0]) if T else 0
     if R:
         _native(r).gemv_swiglu(r, w, ssq, int(ssq_n), 1.0 / H, float(eps), act, R)
@@ -705,11 +781,11 @@ def encoder_layers(x: torch.Tensor, lens: torch.Tensor, starts: torch.Tensor, S:
 
 def max_slots(N: int, M: int = 0) -> int:
     """Rows a partial-row-sum buffer needs for a residual producer of N columns: one per 64-column
-    tgemm tile, at batch <= 8 one per fused-GEMV workgroup (N / 4 at R = 1), at batch <= 16 one
-    per 32-column small-batch MFMA tile (skinny_epi)."""
+    tgemm tile, at batch <= 8 one per fused-GEMV workgroup (N / 4 at R = 1), at batch <= 64 one
+    per 16-column tile of the decode GEMM."""
     if 0 < M <= max(_GEMV_MS):
         return -(-N // 4)
-    return -(-N // 32) if 0 < M <= SKE_MAX_M else -(-N // 64)
+    return -(-N // 16) if 0 < M <= DG_MAX_M else -(-N // 64)
 
 
 # ----------------------------------------------------------------------------- autotuning
@@ -758,7 +834,8 @@ def _plan_key(k) -> str:
 
 
 def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device, verbose: bool = False,
-             fused: Iterable[Tuple[int, int]] = (), prefill: bool = False, qkv_dims=None, qkv_cache=None) -> None:
+             fused: Iterable[Tuple[int, int]] = (), prefill: bool = False, qkv_dims=None, qkv_cache=None,
+             frag: Iterable[Tuple[int, int]] = ()) -> None:
     """Measure every candidate plan for each (M, N, K, swiglu) and keep the fastest.
 
     ``fused``: the (N, K) shapes of one decoder layer's fused ops (QKV, Wo, gate|up, down); a
@@ -766,7 +843,8 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     (``_couple_gemv_choices``).  Their fused-op cores are timed through the fused ops themselves
     (``_retime_fused``); ``qkv_dims`` = (nq, nkv, d) of the QKV op (None: QKV keeps the stand-in
     timings); ``qkv_cache`` = one layer's (K, V^T) caches of the engine, which the QKV timing writes
-    into at scattered free blocks (the TLB reach of a whole serving pool, not of a small buffer)."""
+    into at scattered free blocks (the TLB reach of a whole serving pool, not of a small buffer); ``frag`` =
+    the (N, K) shapes whose weights have fragment-major copies (the decode GEMM is then a candidate)."""
     dev = torch.device(device)
     if dev.type != "cuda" or os.environ.get("DLLM_GEMM") == "blas":
         return
@@ -779,6 +857,8 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
                 parts = k.split(",")
                 if parts[0] == "t":
                     _P.tg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
+                elif parts[0] == "d":
+                    _P.dg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
                 elif parts[0] == "c":
                     _P.fused_core[(int(parts[1]), int(parts[2]), int(parts[3]))] = v
                 else:
@@ -787,11 +867,10 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     fused = list(fused)
     # the fused ops' tgemm plans stream the panel weight copies: time them in that layout
     roles = {}
-    if len(fused) == 4:   # (QKV, Wo, gate|up, down) of a dense layer
-        roles = {tuple(fused[0]): "qkv", tuple(fused[1]): "resadd", tuple(fused[2]): "swiglu",
-                 tuple(fused[3]): "resadd"}
+    if len(fused) in (2, 4):   # (QKV, Wo[, gate|up, down]) of a layer
+        roles = dict(zip((tuple(f) for f in fused), ("qkv", "resadd", "swiglu", "resadd")))
     _autotune(shapes, list(ms), dev, verbose, {tuple(f) for f in fused} if W_PANEL else set(), roles, qkv_dims,
-              qkv_cache)
+              qkv_cache, {tuple(f) for f in frag})
     _couple_gemv_choices(fused, list(ms), verbose)
     if PREFILL_TUNE or prefill:
         _autotune_prefill(fused, dev, verbose)
@@ -800,6 +879,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
         d = {_plan_key(k): list(v) for k, v in _P.plans.items()}
         d.update({_plan_key(k): list(v) for k, v in _P.tg_plans.items()})
         d.update({"c,%d,%d,%d" % k: v for k, v in _P.fused_core.items()})
+        d.update({"d,%d,%d,%d" % k: list(v) for k, v in _P.dg_plans.items()})
         if os.path.dirname(cache):
             os.makedirs(os.path.dirname(cache), exist_ok=True)
         with open(cache, "w") as f:
@@ -852,12 +932,12 @@ def _couple_gemv_choices(fused, ms, verbose: bool) -> None:
         for prod, cons in pairs:
             kp, kc = (M,) + tuple(prod), (M,) + tuple(cons)
             cp, cc = _P.fused_core.get(kp), _P.fused_core.get(kc)
-            if cp is None or not cp.startswith("gemv") or (cc is not None and cc.startswith(("gemv", "skE"))):
+            if cp is None or not cp.startswith(("gemv", "dg1.")) or (cc is not None and cc.startswith(("gemv", "skE", "dg"))):
                 continue
-            opts = {c: t for c, t in _P.fused_opts.get(kp, {}).items() if not c.startswith("gemv")}
+            opts = {c: t for c, t in _P.fused_opts.get(kp, {}).items() if not c.startswith(("gemv", "dg1."))}
             _P.fused_core[kp] = min(opts, key=opts.get) if opts else "lin"
             if verbose:
-                print(f"gemm M={M} N={kp[1]} K={kp[2]}: fused GEMV dropped (its consumer N={kc[1]} K={kc[2]} "
+                print(f"gemm M={M} N={kp[1]} K={kp[2]}: {cp} dropped (its consumer N={kc[1]} K={kc[2]} "
                       f"runs {cc}, which would walk the per-workgroup row sums) -> core {_P.fused_core[kp]}",
                       flush=True)
 
@@ -917,7 +997,26 @@ def _tg_cands(M: int, N: int, K: int):
     return [c for c in out if tg_built(c)]
 
 
-def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None):
+def _dg_cands(M: int, N: int, K: int):
+    """(nt, vs, splits) of the decode GEMM worth timing: a wave walks at least 64 k, the grid is no more than eight workgroups a CU and
+    not under a quarter of the CUs."""
+    out = []
+    if M > DG_MAX_M or K % 32:
+        return out
+    for nt in (1, 2, 3):
+        for vs in (1, 2):
+            for gy in (1, 2, 4) if nt < 3 else (1,):      # three tiles a workgroup: where the weight is wide
+                s, tiles = vs * gy, -(-N // (16 * nt))
+                kchunk = (-(-K // s) + 31) // 32 * 32
+                if -(-K // kchunk) != s or K // (4 * s) < 64 or not 64 <= tiles * gy <= 2048 or (gy > 1 and tiles * gy > 1024):
+                    continue
+                if gy > 1 and s * tiles * 64 * (16 * nt + 1) > WS_FLOATS:
+                    continue
+                out.append((nt, vs, s))
+    return out
+
+
+def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, wfs=None):
     """Time every fused-core option of a decoder-layer shape through the fused op itself: its real
     epilogue and its row-scale prologue over the producer's partial row sums.  The stand-in timings
     (PLAIN tgemm, RESADD GEMV / skinny_epi) missed those: gate|up at batch 4 chose a tgemm timed at
@@ -925,14 +1024,17 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None):
     M, N, K = tkey
     copies = len(ws)
     wsrc = lambda i: (ws[i % copies], wps[i % copies] if wps is not None else None)
+    wf = lambda i: wfs[i % copies] if wfs is not None else None
+    if wfs is not None:
+        opts = dict(opts, **{"dg%d.%d.%d" % p: 0.0 for p in _dg_cands(M, N, K)})
     slots_in = -(-K // 32)   # the producer's partial row sums (as many as a skinny_epi producer leaves)
     ssq = torch.rand(slots_in, M, device=dev) + 1.0
     if role == "resadd":
         res = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
         so = torch.empty(max_slots(N, M), M, dtype=torch.float32, device=dev)
-        fn = lambda i: matmul_resadd(x, wsrc(i)[0], res, so, wp=wsrc(i)[1])
+        fn = lambda i: matmul_resadd(x, wsrc(i)[0], res, so, wp=wsrc(i)[1], wf=wf(i))
     elif role == "swiglu":
-        fn = lambda i: swiglu_matmul(x, wsrc(i)[0], ssq, slots_in, 1e-5, wp=wsrc(i)[1])
+        fn = lambda i: swiglu_matmul(x, wsrc(i)[0], ssq, slots_in, 1e-5, wp=wsrc(i)[1], wf=wf(i))
     elif role == "qkv" and qkv_dims is not None:
         nq, nkv, d = qkv_dims
         if (nq + 2 * nkv) * d != N:
@@ -955,7 +1057,7 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None):
         # the strided V^T cache writes)
         vn = torch.empty(M, nkv * d, dtype=torch.bfloat16, device=dev) if d == 64 else None
         fn = lambda i: qkv_rope_cache(x, wsrc(i)[0], ssq, slots_in, 1e-5, pos, cs, sl, kc, vc, nq, nkv, d,
-                                      wp=wsrc(i)[1], v_new=vn)
+                                      wp=wsrc(i)[1], v_new=vn, wf=wf(i))
     else:
         return None
     saved = _P.fused_core.get(tkey)
@@ -978,12 +1080,13 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None):
 
 
 def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=None, qkv_dims=None,
-              qkv_cache=None) -> None:
+              qkv_cache=None, frag_shapes=frozenset()) -> None:
     use_tg = True
     for (N, K, sw) in shapes:
         copies = max(2, min(64, math.ceil((768 << 20) / (N * K * 2))))
         ws = [(torch.randn(N, K, device=dev) * 0.02).to(torch.bfloat16) for _ in range(copies)]
         wps = [panel_weight(w) for w in ws] if (N, K) in panel_shapes and K % 64 == 0 and not sw else None
+        wfs = [frag_weight(w) for w in ws] if (N, K) in frag_shapes and K % 32 == 0 and not sw else None
         for M in ms:
             if M > MAX_M:
                 continue
@@ -1017,6 +1120,14 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
             if need_plain:
                 _P.plans[key] = best
                 _P.timings[key] = {str(c): round(t, 2) for c, t in res.items()}
+                dg = {}
+                if wfs is not None:
+                    y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+                    dg = {p: _time(lambda i: dgemm(x, wfs[i % copies], N, EPI_PLAIN, p, y=y)) for p in _dg_cands(M, N, K)}
+                best_dg = min(dg, key=dg.get, default=None)
+                if best_dg is not None and dg[best_dg] < res[best]:
+                    _P.dg_plans[tkey] = best_dg
+                    _P.timings[key]["dg"] = round(dg[best_dg], 2)
             tgc = [c for c in res if c[0] == "tg"]
             post = None
             if need_tg and tgc:
@@ -1037,7 +1148,7 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                         opts["gemv%d" % c[1]] = _time(lambda i: ext.gemv_resadd(x, ws[i % copies], rr, sq, c[1]))
                 # small-batch MFMA GEMM with the epilogue fused (one launch), timed in its RESADD form
                 # on the weight layout the fused ops stream (the panel copy where the model keeps one)
-                if M <= SKE_MAX_M and N % 32 == 0 and K % 64 == 0:
+                if M <= SKE_MAX_M and N % 32 == 0 and K % 64 == 0 and wfs is None:
                     rr = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
                     sq = torch.empty(max_slots(N, M), M, dtype=torch.float32, device=dev)
                     src = wps if wps is not None else ws
@@ -1051,7 +1162,7 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                             pass
                 role = (roles or {}).get((N, K))
                 if FUSED_INSITU and role is not None and M <= MAX_M and os.environ.get("DLLM_FUSED_CORE") is None:
-                    insitu = _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache)
+                    insitu = _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
                     if insitu:
                         opts = insitu
                 core = min(opts, key=opts.get)
@@ -1073,10 +1184,11 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                 print(f"gemm M={M} N={N} K={K} swiglu={sw}: best={best} {res[best]:.1f}us "
                       f"({N * K * 2 / res[best] / 1e3:.0f} GB/s, {2 * M * N * K / res[best] / 1e6:.0f} TF/s; "
                       f"blas {res[('blas',)]:.1f}us; {extra})", flush=True)
-        del ws, wps
+        del ws, wps, wfs
 
 
 def plans() -> Dict:
     d = {str(k): v for k, v in _P.plans.items()}
     d.update({"tg" + str(k): v for k, v in _P.tg_plans.items()})
+    d.update({"dg" + str(k): v for k, v in _P.dg_plans.items()})
     return d
