@@ -146,7 +146,7 @@ int dllm_car_vote(int, int*, void*, int*, hipStream_t);
 int dllm_tgemm(const void*, int, int, int, int, int, int, int, hipStream_t, int);
 int dllm_moe_max_tiles_bm(int, int, int);
 int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int,
-                    int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, void*, long, float*, long, int, hipStream_t);
+                    int*, int*, int*, void*, void*, void*, int, const int*, const float*, float*, void*, float, int, void*, long, float*, long, int, const void*, const void*, int, hipStream_t);
 int dllm_moe_slice(int, int);
 int dllm_moe_tail_ok(int, int);
 int dllm_enc_gemm_ok(int, int, int);
@@ -1042,7 +1042,8 @@ void gemv_swiglu(torch::Tensor x, torch::Tensor w, torch::Tensor ssq, int64_t ss
 int64_t moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch::Tensor w13, torch::Tensor w2,
                 c10::optional<torch::Tensor> out, std::vector<int64_t> plan, int64_t act_mode, c10::optional<torch::Tensor> norm_w,
                 double eps, c10::optional<torch::Tensor> xs, c10::optional<torch::Tensor> xl, int64_t groups,
-                c10::optional<torch::Tensor> res, c10::optional<torch::Tensor> ssq) {
+                c10::optional<torch::Tensor> res, c10::optional<torch::Tensor> ssq, c10::optional<torch::Tensor> w13f,
+                c10::optional<torch::Tensor> w2f, int64_t few_ks) {
   check_bf16(x, "x");
   check_i32(ids, "ids");
   check_f32(wts, "wts");
@@ -1091,9 +1092,17 @@ int64_t moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch:
   }
   const int k = ids.size(1);
   auto iopt = ids.options();
-  const int P = (int)(T * k), mt = dllm_moe_max_tiles_bm(P, (int)E, bm);
-  auto perm = torch::empty({std::max(P, 1)}, iopt);
-  auto inv = torch::empty({std::max(P, 1)}, iopt);
+  const bool few = w13f.has_value();      // a decode step on the fragment-major copies
+  if (few) {
+    check_bf16(*w13f, "w13f");
+    TORCH_CHECK(w2f.has_value() && T * k <= 256, "w2f, at most 256 pairs");
+    check_bf16(*w2f, "w2f");
+    TORCH_CHECK(w13f->is_contiguous() && w13f->numel() == w13.numel() && w2f->is_contiguous() && w2f->numel() == w2.numel() &&
+                    (uintptr_t)x.data_ptr() % 16 == 0, "fragment-major copies of w13 and w2");
+  }
+  const int P = (int)(T * k), mt = few ? 0 : dllm_moe_max_tiles_bm(P, (int)E, bm);
+  auto perm = torch::empty({few ? 1 : std::max(P, 1)}, iopt);
+  auto inv = torch::empty({few ? 1 : std::max(P, 1)}, iopt);
   auto tiles = torch::empty({4 * mt + 1}, iopt);
   auto act = torch::empty({std::max(P, 1), I}, x.options());
   auto y = torch::empty({std::max(P, 1), H}, act_mode ? wts.options() : x.options());
@@ -1105,7 +1114,7 @@ int64_t moe_ffn_tg(torch::Tensor x, torch::Tensor ids, torch::Tensor wts, torch:
                      xs ? norm_w->data_ptr<float>() : nullptr, xs ? xs->data_ptr<float>() : nullptr,
                      xs && xl ? xl->data_ptr() : nullptr, (float)eps, (int)groups, res ? res->data_ptr() : nullptr,
                      res ? res->stride(0) : 0, res ? ssq->data_ptr<float>() : nullptr, res ? ssq->stride(0) : 0,
-                     res ? (int)ssq->size(0) : 1, stream()),
+                     res ? (int)ssq->size(0) : 1, few ? w13f->data_ptr() : nullptr, few ? w2f->data_ptr() : nullptr, few_ks == 1 ? 1 : 4, stream()),
      "moe_ffn_tg");
   if (!res) return 0;
   const int cw = dllm_moe_slice((int)H, (int)ssq->size(0));
@@ -2791,7 +2800,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("moe_tail_ok", [](int64_t H, int64_t groups) { return dllm_moe_tail_ok((int)H, (int)groups) != 0; });
   m.def("moe_ffn_tg", &moe_ffn_tg, py::arg("x"), py::arg("ids"), py::arg("wts"), py::arg("w13"), py::arg("w2"), py::arg("out"),
         py::arg("plan"), py::arg("act_mode") = 0, py::arg("norm_w") = py::none(), py::arg("eps") = 0.0, py::arg("xs") = py::none(),
-        py::arg("xl") = py::none(), py::arg("groups") = 1, py::arg("res") = py::none(), py::arg("ssq") = py::none());
+        py::arg("xl") = py::none(), py::arg("groups") = 1, py::arg("res") = py::none(), py::arg("ssq") = py::none(), py::arg("w13f") = py::none(),
+        py::arg("w2f") = py::none(), py::arg("few_ks") = 1);
   m.def("tgemm", &tgemm);
   m.def("res_add_ssq", &res_add_ssq);
   m.def("qkv_post", &qkv_post, py::arg("y"), py::arg("ssq"), py::arg("ssq_n"), py::arg("scale"), py::arg("eps"),

@@ -31,6 +31,8 @@
 
 extern "C" int dllm_moe_norm_resadd(const void* y, int f32, const int* inv, const float* wts, int k, const float* w, float* x, void* xl,
                                     long T, int H, float eps, int groups, hipStream_t st);
+extern "C" int dllm_moe_decode(const void* x, long ldx, int div, const int* ids, int P, int E, const void* w, int N, int K, int act,
+                               int ks, void* out, long ldo, hipStream_t st);
 extern "C" int dllm_tgemm(const void* args, int bm, int bn, int stages, int ks, int nw, int wk, int epi,
                           hipStream_t stream, int nl);
 
@@ -118,7 +120,7 @@ __global__ void moe_combine_perm_kernel(const T_* __restrict__ y, const int* __r
     for (int j = 0; j < k; ++j) {
       const long p = t * k + j;
       float f[8];
-      ld8(y + (long)inv[p] * H + h, f);
+      ld8(y + (inv ? (long)inv[p] : p) * H + h, f);
       const float w = wts[p];
 #pragma unroll
       for (int q = 0; q < 8; ++q) s[q] += w * f[q];
@@ -144,7 +146,7 @@ __global__ void __launch_bounds__(256) moe_combine_resadd_kernel(const u16* __re
     for (int j = 0; j < k; ++j) {
       const long p = (long)row * k + j;
       float f[8];
-      ld8(y + (long)inv[p] * H + c, f);
+      ld8(y + (inv ? (long)inv[p] : p) * H + c, f);
       const float w = wts[p];
 #pragma unroll
       for (int e = 0; e < 8; ++e) s[e] += w * f[e];
@@ -370,32 +372,41 @@ extern "C" int dllm_moe_slice(int H, int slices) { return ((H + slices - 1) / sl
 // rows, 16 up rows, ...), y bf16; 1: w13 [E, I, H], squared ReLU, y f32.  w2 [E, H, I]; scratch: perm/inv [P], tiles
 // [4 * max_tiles + 1], act [P, I], y [P, H].  xs (f32 [T, H]): instead of `out`, xs += rmsnorm(sum) * nw in `groups` parts, and its
 // rounded copy in xl (norm_resadd of seqmix.hip, in the combine's launch).  res (bf16 [T, H], act_mode 0): instead of `out`, added to the
-// residual stream with the rows' squares in ssq [slots][ssq_ld].
+// residual stream with the rows' squares in ssq [slots][ssq_ld].  w13f / w2f (P <= 256): the decode step's kernels on their
+// fragment-major copies instead, few_ks waves a tile (perm, inv and tiles are then not read).
 extern "C" int dllm_moe_ffn_tg(const void* x, long x_stride, long T, int H, const int* ids, const float* wts, int k,
                                int E, const void* w13, const void* w2, int I, int* perm, int* inv, int* tiles,
                                void* act, void* y, void* out, int act_mode, const int* plan, const float* nw, float* xs, void* xl,
-                               float eps, int groups, void* res, long ldr, float* ssq, long ssq_ld, int slices,
-                               hipStream_t stream) {
+                               float eps, int groups, void* res, long ldr, float* ssq, long ssq_ld, int slices, const void* w13f,
+                               const void* w2f, int few_ks, hipStream_t stream) {
   if (E < 1 || E > 64 || k < 1 || H % 64 != 0 || I % 64 != 0 || x_stride % 8 || (res && (act_mode || ldr % 8 || !ssq || slices < 1))) return -1;
   if (T == 0) return 0;
   const int bm = plan[0], NI = act_mode ? I : 2 * I;
   const int P = (int)(T * k);
   const int max_tiles = (P + bm - 1) / bm + E;
-  int *te = tiles, *tr = tiles + max_tiles, *tn = tiles + 2 * max_tiles, *nt = tiles + 3 * max_tiles;
-  hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(route_threads(P)), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt, bm,
-                     inv);
-  dllm::GemmArgs g{};
-  g.A = (const uint16_t*)x; g.lda = x_stride; g.W = (const uint16_t*)w13; g.Y = (uint16_t*)act; g.ldy = I;
-  g.M = max_tiles * bm; g.N = NI; g.K = H; g.kchunk = H; g.splits = 1;
-  g.g_tiles = tiles; g.g_max = max_tiles; g.g_perm = perm; g.g_k = k; g.g_wstride = (long)NI * H;
-  int rc = dllm_tgemm(&g, bm, plan[1], plan[2], plan[3], plan[4], 1, act_mode ? dllm::EPI_RELU2 : dllm::EPI_SWIGLU, stream, 0);
-  if (rc) return 1000 + rc;
-  dllm::GemmArgs d{};
-  d.A = (const uint16_t*)act; d.lda = I; d.W = (const uint16_t*)w2; d.Y = (uint16_t*)y; d.ldy = H;
-  d.M = max_tiles * bm; d.N = H; d.K = I; d.kchunk = I; d.splits = 1;
-  d.g_tiles = tiles; d.g_max = max_tiles; d.g_perm = nullptr; d.g_k = 1; d.g_wstride = (long)H * I;
-  rc = dllm_tgemm(&d, bm, plan[5], plan[6], plan[7], plan[8], 1, act_mode ? dllm::EPI_F32 : dllm::EPI_PLAIN, stream, 0);
-  if (rc) return 2000 + rc;
+  if (w13f) {      // a decode step on fragment-major weights: rows stay in pair order (moe_decode.hip)
+    int rc = dllm_moe_decode(x, x_stride, k, ids, P, E, w13f, NI, H, act_mode ? 1 : 0, few_ks, act, I, stream);
+    if (rc) return 3000 + rc;
+    rc = dllm_moe_decode(act, I, 1, ids, P, E, w2f, H, I, act_mode ? 3 : 2, few_ks, y, H, stream);
+    if (rc) return 4000 + rc;
+    inv = nullptr;
+  } else {
+    int *te = tiles, *tr = tiles + max_tiles, *tn = tiles + 2 * max_tiles, *nt = tiles + 3 * max_tiles;
+    hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(route_threads(P)), 0, stream, ids, P, E, max_tiles, perm, te, tr, tn, nt, bm,
+                       inv);
+    dllm::GemmArgs g{};
+    g.A = (const uint16_t*)x; g.lda = x_stride; g.W = (const uint16_t*)w13; g.Y = (uint16_t*)act; g.ldy = I;
+    g.M = max_tiles * bm; g.N = NI; g.K = H; g.kchunk = H; g.splits = 1;
+    g.g_tiles = tiles; g.g_max = max_tiles; g.g_perm = perm; g.g_k = k; g.g_wstride = (long)NI * H;
+    int rc = dllm_tgemm(&g, bm, plan[1], plan[2], plan[3], plan[4], 1, act_mode ? dllm::EPI_RELU2 : dllm::EPI_SWIGLU, stream, 0);
+    if (rc) return 1000 + rc;
+    dllm::GemmArgs d{};
+    d.A = (const uint16_t*)act; d.lda = I; d.W = (const uint16_t*)w2; d.Y = (uint16_t*)y; d.ldy = H;
+    d.M = max_tiles * bm; d.N = H; d.K = I; d.kchunk = I; d.splits = 1;
+    d.g_tiles = tiles; d.g_max = max_tiles; d.g_perm = nullptr; d.g_k = 1; d.g_wstride = (long)H * I;
+    rc = dllm_tgemm(&d, bm, plan[5], plan[6], plan[7], plan[8], 1, act_mode ? dllm::EPI_F32 : dllm::EPI_PLAIN, stream, 0);
+    if (rc) return 2000 + rc;
+  }
   if (res) {                                                                                               // ... the bf16 one
     const int cw = dllm_moe_slice(H, slices);
     hipLaunchKernelGGL(moe_combine_resadd_kernel, dim3((unsigned)((T + 3) / 4), (H + cw - 1) / cw), dim3(256), 0, stream, (const u16*)y, inv,

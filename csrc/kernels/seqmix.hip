@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restri
 #pragma unroll
       for (int j = 0; j < NE; ++j) a[j] = 0.f;
       for (int e = 0; e < k; ++e) {
-        const TY* yr = y + (long)inv[row * k + e] * ldy;
+        const TY* yr = y + (inv ? (long)inv[row * k + e] : row * k + e) * ldy;
         const float wt = wts[row * k + e];
 #pragma unroll
         for (int j = 0; j < NE; ++j) a[j] += wt * ldf(yr + min(c0 + ST * j, c1 - 1));
@@ -1549,7 +1549,7 @@ extern "C" int dllm_moe_tail_ok(int H, int groups) {
   return groups >= 1 && H >= groups && H % groups == 0 && norm_resadd_entries(H, groups) > 0;
 }
 
-// x += rmsnorm(sum_j wts[t k + j] y[inv[t k + j]]) * w in `groups` parts; y [P, H] f32 or bf16, xl the rounded stream (bf16) or null
+// x += rmsnorm(sum_j wts[t k + j] y[inv[t k + j]]) * w in `groups` parts; y [P, H] f32 or bf16 (inv null: in pair order), xl the rounded stream (bf16) or null
 extern "C" int dllm_moe_norm_resadd(const void* y, int f32, const int* inv, const float* wts, int k, const float* w, float* x, void* xl,
                                     long T, int H, float eps, int groups, hipStream_t st) {
   if (T <= 0) return T == 0 ? 0 : -1;

@@ -547,6 +547,13 @@ class HybridModel:
         for L, n in todo:
             L[n + "_r"] = ops.gemm.frag_weight(L[n])
             L["order_kept"] = self.order_kept
+        ex = [(L, S.mlp) for L, S in zip(self.layers, self.cfg.layers)
+              if isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
+              and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
+        extra = sum(L[n].numel() * L[n].element_size() for L, _ in ex for n in ("w1", "w2"))
+        if extra <= 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+            for L, f in ex:
+                L["experts_r"] = (ops.frag_experts(L["w1"], paired=f.act == "swiglu"), ops.frag_experts(L["w2"]), self.order_kept)
         if takes(self.lm_head):
             self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
 
@@ -1044,7 +1051,7 @@ class HybridModel:
         """sum_j w[t, j] expert_(ids[t, j])(x_t); ids beyond the experts (identity experts, whose weight
         here is 0) add nothing.  ``tail`` as in ``_experts``."""
         if L.get("tg"):
-            return ops.moe_ffn_tg(x if x.stride(1) == 1 else x.contiguous(), ids, w, L["w1"], L["w2"], tail=tail)
+            return ops.moe_ffn_tg(x if x.stride(1) == 1 else x.contiguous(), ids, w, L["w1"], L["w2"], tail=tail, frag=L.get("experts_r"))
         if "w2" in L and (not x.is_cuda or seqmix.moe_ffn_relu2_ok(x, L["w1"])):
             return ops.moe_ffn(x, ids, w, L["w1"], L["w2"])
         if "w2d" not in L:
@@ -1060,7 +1067,7 @@ class HybridModel:
             return self._experts_swiglu(L, f, x, tail)
         if "shared_in" in L:
             ids, w = ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
-            return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], tail)
+            return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], tail, L.get("experts_r"))
         if f.experts > 64 or f.top > 8:      # beyond the router kernels' register budget: library top-k
             val, ids = torch.topk(torch.softmax(F.linear(x.float(), L["router"].float()), -1), f.top, -1)
             ids, w = ids.to(torch.int32), val / (val.sum(-1, keepdim=True) + 1e-20) * f.scale
@@ -1070,7 +1077,7 @@ class HybridModel:
             ids, w = ops.moe_gate(F.linear(x.float(), L["router"].float()), f.top)
             w = w * f.scale
         if "w2" in L and (not x.is_cuda or seqmix.moe_ffn_relu2_ok(x, L["w1"])):
-            y = seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"])
+            y = seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], frag=L.get("experts_r"))
         else:
             if "w2d" not in L:
                 L["w2d"] = L["w2"].permute(1, 0, 2).reshape(x.shape[1], -1).contiguous()

@@ -179,6 +179,10 @@ class LlamaModel:
             idx = gate_up_order(self.I).to(self.device)
             for L in self.layers:
                 L["w13"] = L["w13"].index_select(1, idx).contiguous()
+            extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in ("w13", "w2"))
+            if self.fused and extra <= 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+                for L in self.layers:     # the decode step's fragment-major copies (ops.frag_experts)
+                    L["w13_r"], L["w2_r"] = ops.frag_experts(L["w13"], paired=True), ops.frag_experts(L["w2"])
 
     # ------------------------------------------------------------------ fused layout
     def _fusable(self) -> bool:
@@ -370,8 +374,12 @@ class LlamaModel:
         the partial sums."""
         ids, w = ops.moe_router(x, L["wgate"], self.cfg.experts_per_token)
         if self.moe_tg:
-            return ops.moe_ffn_tg(x, ids, w, L["w13"], L["w2"])
+            return ops.moe_ffn_tg(x, ids, w, L["w13"], L["w2"], frag=self._experts_r(L))
         return ops.moe_ffn(x, ids, w, L["w13"], L["w2"])
+
+    @staticmethod
+    def _experts_r(L):
+        return (L["w13_r"], L["w2_r"]) if "w13_r" in L else None
 
     def use_ep(self, T: int) -> bool:
         """Expert-parallel MoE for this batch: EP mode, a prefill-size batch, not inside a graph
@@ -493,7 +501,7 @@ class LlamaModel:
             else:
                 if not tp and self.moe_tg:      # norm and router, and combine and residual add, share a launch
                     x, ids, w = ops.norm_moe_router(r, L["ln2"], eps, L["wgate"], cfg.experts_per_token)
-                    n = ops.moe_ffn_tg_resadd(x, ids, w, L["w13"], L["w2"], r, ssq_a)
+                    n = ops.moe_ffn_tg_resadd(x, ids, w, L["w13"], L["w2"], r, ssq_a, frag=self._experts_r(L))
                     continue
                 x = ops.rms_norm(r, L["ln2"], eps)
                 if not tp:

@@ -450,15 +450,15 @@ def norm_moe_router(r: torch.Tensor, norm_w: torch.Tensor, eps: float, wg: torch
 
 
 def moe_ffn_tg_resadd(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torch.Tensor, w2: torch.Tensor, r: torch.Tensor,
-                      ssq: torch.Tensor) -> int:
+                      ssq: torch.Tensor, frag: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> int:
     """``gemm.res_add_ssq(moe_ffn_tg(...), r, ssq)`` with the residual add in the combine's launch; returns the slots of
     ``ssq`` [slots, >= T] written."""
     ext = _native(x)
     if ext is None or r.stride(0) % 8 or r.data_ptr() % 16:
         from . import gemm
-        return gemm.res_add_ssq(moe_ffn_tg(x, ids, wts, w13i, w2), r, ssq)
+        return gemm.res_add_ssq(moe_ffn_tg(x, ids, wts, w13i, w2, frag=frag), r, ssq)
     return int(ext.moe_ffn_tg(x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, None,
-                              list(moe_plan(x.shape[0] * ids.shape[1])), 0, res=r, ssq=ssq))
+                              list(moe_plan(x.shape[0] * ids.shape[1])), 0, res=r, ssq=ssq, **moe_few(x, ids, frag)))
 
 
 def moe_ffn(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torch.Tensor,
@@ -483,17 +483,38 @@ MOE_PLANS = {  # (bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2) by rou
 }
 
 
+# tokens and routed pairs up to which the experts run on their fragment-major copies (csrc/kernels/moe_decode.hip, whose pair list ends
+# at 256).  Routing, both products and the sum, us grouped / here: 8 experts of 1024 x 1024 (SwiGLU, top 2) 1 token 28 / 15, 12 32 / 23,
+# 64 32 / 27; with a shared expert (squared ReLU) 1 token 26 / 15, 24 28 / 21, 42 28.7 / 28.9, 48 33.6 / 30.1, 64 34.4 / 33.9, 85 34 / 51.
+MOE_FEW, MOE_FEW_TOKENS = 256, 64
+
+
+def frag_experts(w: torch.Tensor, paired: bool = False) -> torch.Tensor:
+    """[E, N, K] expert weights fragment-major (gemm.frag_weight) for the decode step's kernels."""
+    return torch.stack([gemm.frag_weight(e, paired) for e in w])
+
+
+def moe_few(x: torch.Tensor, ids: torch.Tensor, frag) -> dict:
+    """The launch's fragment-major weights where the pairs are few, else nothing.  ``frag`` = (w13, w2[, order kept]): with the order of
+    the grouped GEMM's sums one wave walks all of K, else four share it."""
+    if frag is None or not 0 < ids.numel() <= MOE_FEW or x.shape[0] > MOE_FEW_TOKENS or x.data_ptr() % 16:
+        return {}
+    return dict(w13f=frag[0], w2f=frag[1], few_ks=1 if len(frag) > 2 and frag[2] else 4)
+
+
 def moe_plan(pairs: int) -> Tuple[int, ...]:
     return MOE_PLANS["decode" if pairs <= 128 else "mid" if pairs <= 1024 else "prefill"]
 
 
 def moe_ffn_tg(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torch.Tensor, w2: torch.Tensor,
-               plan: Optional[Tuple[int, ...]] = None, tail: Optional[tuple] = None) -> Optional[torch.Tensor]:
+               plan: Optional[Tuple[int, ...]] = None, tail: Optional[tuple] = None,
+               frag: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> Optional[torch.Tensor]:
     """Top-k expert FFN on the grouped LDS-tiled MFMA GEMM (csrc/kernels/moe.hip moe_ffn_tg):
     ``w13i`` [E, 2I, H] with gate/up rows interleaved in 16-row groups (models.llama.gate_up_order),
     w2 [E, H, I].  Routing, both GEMMs and the weighted combine stay on the device.  ``tail`` =
     (norm weight, eps, stream, rounded stream or None, groups): the sum ends in ``seqmix.norm_resadd``'s update of the
-    stream, in the combine's launch where the width allows; returns None then."""
+    stream, in the combine's launch where the width allows; returns None then.  ``frag``: ``frag_experts`` of both weights (w13i
+    paired), for steps of few pairs."""
     ext = _native(x)
     if ext is None:
         from ..models.llama import gate_up_order
@@ -503,7 +524,7 @@ def moe_ffn_tg(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torc
         return out if tail is None else moe_tail(out, tail)
     if plan is None:
         plan = moe_plan(x.shape[0] * ids.shape[1])
-    return moe_run_tg(ext, x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, plan, 0, tail)
+    return moe_run_tg(ext, x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, plan, 0, tail, frag)
 
 
 def moe_tail(y: torch.Tensor, tail: tuple) -> None:
@@ -513,13 +534,14 @@ def moe_tail(y: torch.Tensor, tail: tuple) -> None:
     seqmix.norm_resadd(y, w, eps, x, xl, groups=groups)
 
 
-def moe_run_tg(ext, x, ids, wts, w1, w2, plan, act_mode: int, tail: Optional[tuple]) -> Optional[torch.Tensor]:
+def moe_run_tg(ext, x, ids, wts, w1, w2, plan, act_mode: int, tail: Optional[tuple], frag=None) -> Optional[torch.Tensor]:
+    few = moe_few(x, ids, frag)
     if tail is not None and ext.moe_tail_ok(x.shape[1], int(tail[4])):
         w, eps, xs, xl, groups = tail
-        ext.moe_ffn_tg(x, ids, wts, w1, w2, None, list(plan), act_mode, w, float(eps), xs, xl, int(groups))
+        ext.moe_ffn_tg(x, ids, wts, w1, w2, None, list(plan), act_mode, w, float(eps), xs, xl, int(groups), **few)
         return None
     out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
-    ext.moe_ffn_tg(x, ids, wts, w1, w2, out, list(plan), act_mode)
+    ext.moe_ffn_tg(x, ids, wts, w1, w2, out, list(plan), act_mode, **few)
     return out if tail is None else moe_tail(out, tail)
 
 

@@ -265,10 +265,10 @@ def relu2_scale(x: torch.Tensor, gate: Optional[torch.Tensor] = None, ff: int = 
     return y
 
 
-def moe_ffn_relu2(x, ids, wts, w1, w2, tail: Optional[tuple] = None) -> Optional[torch.Tensor]:
+def moe_ffn_relu2(x, ids, wts, w1, w2, tail: Optional[tuple] = None, frag=None) -> Optional[torch.Tensor]:
     """Top-k experts with a squared-ReLU activation and no gate projection (csrc/kernels/moe.hip, activation
     mode 1): on the LDS-tiled grouped GEMM where it takes the widths (multiples of 64), else on the
-    32-row grouped kernels.  ``tail`` as in ``ops.moe_ffn_tg``."""
+    32-row grouped kernels.  ``tail`` and ``frag`` as in ``ops.moe_ffn_tg``."""
     from . import moe_run_tg, moe_tail
     ext = _native(x)
     if ext is None:
@@ -276,7 +276,7 @@ def moe_ffn_relu2(x, ids, wts, w1, w2, tail: Optional[tuple] = None) -> Optional
         return out if tail is None else moe_tail(out, tail)
     ids, wts = ids.to(torch.int32).contiguous(), wts.float().contiguous()
     if moe_ffn_relu2_tg_ok(x, w1):
-        return moe_run_tg(ext, x, ids, wts, w1, w2, moe_plan(x.shape[0] * ids.shape[1]), 1, tail)
+        return moe_run_tg(ext, x, ids, wts, w1, w2, moe_plan(x.shape[0] * ids.shape[1]), 1, tail, frag)
     out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
     ext.moe_ffn(x, ids, wts, w1, w2, out, 1)
     return out if tail is None else moe_tail(out, tail)
