@@ -1,15 +1,50 @@
-// pybind11 module `_runtime`: Python binding of the native paged-KV block manager
-// (core in block_manager.h).
+// pybind11 module `_runtime`: Python bindings of the native paged-KV block manager (core in block_manager.h) and of the sentence
+// encoder's word tokenizer (word_tokenizer.h).
+#include <pybind11/numpy.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
 #include "block_manager.h"
+#include "word_tokenizer.h"
 
 namespace py = pybind11;
 using dllm::BlockManager;
 
+// A batch of texts as one int32 array: the token ids one text behind the other, each token's place in its text, each text's first
+// token, its number of tokens.  Texts that are not ASCII are tokenised by `other(text)`.  Returns (array, tokens, longest text).
+static py::tuple pack_words(const py::list& texts, int64_t max_len, int64_t vocab, const py::function& other) {
+  if (max_len < 2 || vocab <= 1000) throw py::value_error("pack_words: max_len of at least 2, vocab past 1000");
+  dllm::WordHasher hash(vocab);
+  std::vector<int32_t> ids, starts;
+  for (const py::handle t : texts) {
+    if (!PyUnicode_Check(t.ptr())) throw py::type_error("pack_words: texts are str");
+    starts.push_back((int32_t)ids.size());
+    Py_ssize_t n = 0;
+    const char* s = PyUnicode_IS_ASCII(t.ptr()) ? PyUnicode_AsUTF8AndSize(t.ptr(), &n) : nullptr;
+    if (!s || !hash.append(s, (size_t)n, max_len, ids)) {
+      PyErr_Clear();
+      for (const py::handle v : other(t)) ids.push_back(v.cast<int32_t>());
+    }
+  }
+  hash.flush(ids);
+  const size_t T = ids.size(), B = starts.size();
+  py::array_t<int32_t> out((py::ssize_t)(2 * T + 2 * B));
+  int32_t* o = out.mutable_data();
+  int32_t longest = 0;
+  std::copy(ids.begin(), ids.end(), o);
+  for (size_t b = 0; b < B; ++b) {
+    const int32_t n = (int32_t)(b + 1 < B ? starts[b + 1] : T) - starts[b];
+    for (int32_t i = 0; i < n; ++i) o[T + starts[b] + i] = i;
+    o[2 * T + b] = starts[b];
+    o[2 * T + B + b] = n;
+    longest = std::max(longest, n);
+  }
+  return py::make_tuple(out, (int64_t)T, longest);
+}
+
 PYBIND11_MODULE(_runtime, m) {
-  m.doc() = "distributed_llm_amd native serving runtime (paged-KV block manager)";
+  m.doc() = "distributed_llm_amd native serving runtime (paged-KV block manager, word tokenizer)";
+  m.def("pack_words", &pack_words, py::arg("texts"), py::arg("max_len"), py::arg("vocab"), py::arg("other"));
   py::class_<BlockManager>(m, "BlockManager")
       .def(py::init<int, int, bool, int>(), py::arg("num_blocks"), py::arg("block_size") = 16,
            py::arg("prefix_cache") = true, py::arg("placement") = 2)

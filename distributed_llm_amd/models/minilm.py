@@ -19,12 +19,17 @@ import re
 import threading
 from collections import OrderedDict
 from dataclasses import dataclass
-from typing import Dict, List, Optional
+from typing import Dict, List, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
 
 from .. import ops
+
+try:
+    from ..engine import _runtime
+except ImportError:      # not built: word by word in Python
+    _runtime = None
 
 _WORD = re.compile(r"[a-z0-9]+|[^\sa-z0-9]")
 
@@ -54,6 +59,24 @@ class _HashWordTokenizer:
         ids = ids[:max_len - 1] + [self.SEP]
         return ids
 
+    def pack(self, texts: List[str], max_len: int) -> Tuple[torch.Tensor, int, int]:
+        """``_pack`` of every text's ``encode`` in one native call (csrc/runtime/word_tokenizer.h)."""
+        if _runtime is None or max_len < 2 or not all(type(t) is str for t in texts):
+            return _pack([self.encode(t, max_len) for t in texts])
+        a, T, S = _runtime.pack_words(texts, max_len, self.vocab, lambda t: self.encode(t, max_len))
+        return torch.from_numpy(a), T, S
+
+
+def _pack(toks: List[List[int]]) -> Tuple[torch.Tensor, int, int]:
+    """(token ids one text behind the other | their places | first tokens | lengths, tokens, longest)."""
+    lens = [len(x) for x in toks]
+    flat, at, starts = [], [], []
+    for x, n in zip(toks, lens):
+        starts.append(len(flat))
+        flat += x
+        at += range(n)
+    return torch.tensor(flat + at + starts + lens, dtype=torch.int32), len(flat), max(lens)
+
 
 class _WordPiece:
     def __init__(self, vocab_file: str):
@@ -63,6 +86,9 @@ class _WordPiece:
     def encode(self, text: str, max_len: int) -> List[int]:
         ids = self.tok.encode(text).ids
         return ids[:max_len - 1] + ids[-1:] if len(ids) > max_len else ids
+
+    def pack(self, texts: List[str], max_len: int) -> Tuple[torch.Tensor, int, int]:
+        return _pack([self.encode(t, max_len) for t in texts])
 
 
 class MiniLMEncoder:
@@ -130,15 +156,9 @@ class MiniLMEncoder:
         attention kernel and 2 LayerNorms; mean-pool + L2 (csrc/kernels/encoder.hip, tgemm.hip, norm.hip, elementwise.hip).
         CPU tensors run the same graph on ops.reference."""
         cfg = self.cfg
-        toks = [self.tok.encode(t, max_len) for t in texts]
-        lens = [len(x) for x in toks]
-        B, S, T = len(toks), max(lens), sum(lens)
-        flat, at, starts = [], [], []
-        for x, n in zip(toks, lens):
-            starts.append(len(flat))
-            flat += x
-            at += range(n)
-        ids, at_d, starts_d, lens_d = torch.tensor(flat + at + starts + lens, dtype=torch.int32).to(self.device).split([T, T, B, B])
+        packed, T, S = self.tok.pack(texts, max_len)
+        B = len(texts)
+        ids, at_d, starts_d, lens_d = packed.to(self.device).split([T, T, B, B])
         H, nh = cfg.hidden, cfg.heads
         x = ops.embed_ln(ids, self.word, self.pos, self.type0, *self.emb_ln, S, cfg.eps, at_d)
         x = ops.gemm.encoder_layers(x, lens_d, starts_d, S, nh, H // nh, cfg.eps, self.layers)
@@ -196,6 +216,14 @@ class MiniLMEncoder:
 
     def encode(self, texts: List[str], max_len: int = 256) -> torch.Tensor:
         """[n, 384] f32 unit vectors on the device; memoised per text."""
+        if texts and not self._memo_size and len(set(texts)) == len(texts):      # nothing kept: the forward's rows as they are
+            with self._lock:
+                fresh = not any(t in self._scope for t in texts)
+                if fresh:
+                    self.memo_misses += len(texts)
+                    self.encoded_texts += len(texts)
+            if fresh:
+                return self._forward(list(texts), max_len)
         out = self.encode_rows(texts, max_len)
         return torch.stack(out) if out else torch.zeros((0, self.cfg.hidden), device=self.device)
 
