@@ -602,7 +602,8 @@ def fused_dg(x: torch.Tensor, N: int, K: int, wf: Optional[torch.Tensor]) -> Opt
     ``dg<nt>.<vs>.<splits>``) and the caller keeps its weight copy, else None."""
     if wf is None:
         return None
-    c = os.environ.get("DLLM_FUSED_CORE") or _P.fused_core.get((x.shape[0], N, K))
+    M = x.shape[0]      # rows between two timed batch sizes (a short prompt): what was timed for the next one
+    c = os.environ.get("DLLM_FUSED_CORE") or _P.fused_core.get((M, N, K)) or _P.fused_core.get((next_batch_size(M), N, K))
     if not c or not c.startswith("dg") or not dg_takes(x):
         return None
     return tuple(int(v) for v in c[2:].split("."))
