@@ -201,7 +201,8 @@ class LLMEngine:
             self._autotune()      # DLLM_AUTOTUNE=0: heuristic GEMM plans (multi-process tests on one GPU)
         self._graphs: Dict[int, torch.cuda.CUDAGraph] = {}
         self._graph_pool = None
-        self.d_logits: Optional[torch.Tensor] = None    # [max bucket, vocab] f32, kept by feed()
+        self.d_logits: Optional[torch.Tensor] = None    # [max bucket, vocab] f32, of a feed() step
+        self._feeding = False                           # (under the lock) the step being run is feed()'s
         self._streams: Dict[object, _Seq] = {}           # forced-token requests by caller key (feed)
         self.collective_trips = 0
         self.trip_steps: List[int] = []   # decode-step counter at each collective trip
@@ -1327,8 +1328,9 @@ class LLMEngine:
 
     def _gkey(self, bs: int, p: int):
         # with step I/O kernels the staging buffer's address is baked into the graph: one graph
-        # per bucket and buffer parity
-        return (bs, p) if self._gio else bs
+        # per bucket and buffer parity; a feed step's graph ends in the logits, any other in the sampled tokens
+        key = (bs, p) if self._gio else bs
+        return ("feed", key) if self._feeding else key
 
     def _read_out(self, B: int, p: int, bs: int) -> "torch.cuda.Event":
         if not self._gio:           # else the step's last kernel (ops.step_store) wrote _out_bufs[p]
@@ -1704,7 +1706,7 @@ class LLMEngine:
             items = (self._items_bufs[p][0], self.items_dev) if self.attn_worklist else (None, None)
             ops.step_fetch(self._dec_bufs[p][0], self.dec_dev, o[0], o[9], mb, self.d_out, *items)
         self._decode_body(bs)
-        if self._gio:
+        if self._gio and not self._feeding:
             ops.step_store(self.d_out, self._out_bufs[p], bs + 1)
 
     def _decode_body(self, bs: int) -> None:
@@ -1712,9 +1714,13 @@ class LLMEngine:
         # embedding launch)
         hid = self.model.hidden_states(self.d_ids[:bs], self.d_pos[:bs], self._decode_meta(bs), self.kv_caches,
                                        scatter=(self.bt_dev, self.d_upd))
-        if self.d_logits is not None:      # forced-token replay: the step's logits stay on the device
+        if self._feeding:      # given tokens: the step ends in its logits, nothing is sampled
             lf = getattr(self.model, "logits_f32", None)
-            self.d_logits[:bs].copy_(lf(hid) if lf is not None else self.model.logits(hid).float())
+            if lf is None or self.model.plain_logits:
+                self.d_logits[:bs].copy_(self.model.logits(hid))      # (rounded logits; the copy widens them)
+            else:
+                self.d_logits[:bs].copy_(lf(hid))
+            return
         if self.fused_sampler:
             self.model.sample(hid, self.d_temp[:bs], self.d_topp[:bs], self.d_topk[:bs], self.d_seed,
                               self.d_out[:bs])
@@ -1855,15 +1861,18 @@ class LLMEngine:
         if decode:
             if self.d_logits is None:
                 self.d_logits = torch.zeros((self.buckets[-1], self.cfg.vocab), dtype=torch.float32, device=self.device)
-                self._graphs.clear()        # graphs captured before did not keep the logits
             B = len(seqs)
             lens = np.fromiter((s.length for s in seqs), dtype=np.int64, count=B)
             last = np.fromiter((s.prompt[-1] for s in seqs), dtype=np.int64, count=B)
             bs = self._prep_decode(seqs, lens, last, 0)
-            if self.use_graphs:
-                self._replay(bs, 0)
-            else:
-                self._decode_forward(bs, 0)
+            self._feeding = True
+            try:
+                if self.use_graphs:
+                    self._replay(bs, 0)
+                else:
+                    self._decode_forward(bs, 0)
+            finally:
+                self._feeding = False
             self.steps["decode"] += 1
             self.steps["decode_tokens"] += B
             rows = [i for i, (_, _, w) in enumerate(entries) for _ in w]

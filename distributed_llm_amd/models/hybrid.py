@@ -1207,6 +1207,11 @@ class HybridModel:
             return seqmix.softcap(lg, self.cfg.logit_softcap).to(lg.dtype)
         return lg if self.cfg.logit_scale == 1.0 else lg * self.cfg.logit_scale
 
+    @property
+    def plain_logits(self) -> bool:
+        """``logits_f32`` is the head's product widened, nothing else."""
+        return self.cfg.logit_softcap <= 0 and self.cfg.logit_scale == 1.0
+
     def logits_f32(self, hidden: torch.Tensor) -> torch.Tensor:
         lg = _mm(hidden, self.lm_head, self.lm_head_r)
         if self.cfg.logit_softcap > 0:
