@@ -170,25 +170,16 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
     }
   }
 
-  // ---- QKV row metadata: the positions and cache slots of this lane's output rows are loaded
-  // with the row-scale partials, before the ring (they retire at its first wait), so the epilogue
-  // starts with them in registers: its RoPE table reads are then ONE round trip, not two dependent
-  // ones (pos -> cos/sin), and the K copy-out reads its slots from LDS.  Decode-sized tiles only
-  // (FM <= 2): 2 FM*4 live registers across the ring spill the large prefill tiles
-  constexpr bool QPF = EPI == EPI_QKV && FM <= 2 && MF == 16;
-  constexpr int QR = QPF ? FM * 4 : 1;
+  // ---- QKV row metadata: one thread a row loads its position and cache slot with the row-scale partials, before the ring (they
+  // retire at its first wait); the epilogue finds them in LDS, so its RoPE table reads are one round trip
+  constexpr int QR = EPI == EPI_QKV ? (BM + NT - 1) / NT : 1;
   int q_pos[QR], q_slot[QR];
-  if constexpr (QPF) {
-    if (!loader) {
-      const int rlq = wm * WM + 4 * (lane >> 4);
+  if constexpr (EPI == EPI_QKV) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int mm = min(m0 + rlq + 16 * i + e, M - 1);
-          q_pos[4 * i + e] = a.pos[mm];
-          q_slot[4 * i + e] = a.slots[mm];
-        }
+    for (int i = 0; i < QR; ++i) {
+      const int mm = min(m0 + min((int)threadIdx.x + i * NT, BM - 1), M - 1);
+      q_pos[i] = a.pos[mm];
+      q_slot[i] = a.slots[mm];
     }
   }
 
@@ -653,31 +644,8 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
             ri = rsqrtf(sum * a.norm_scale + a.eps);
           }
           if constexpr (EPI == EPI_QKV) {
-            const int d = a.d, hd = d / 2, nkv = a.nkv, qcols = a.nq * d, kcols = nkv * d;
-            const int m = m0 + rl, mq = min(m, M - 1);
-            const int slot = a.slots[mq];
-            if (wn == 0 && lc == 0) reinterpret_cast<int*>(s_red)[rl] = slot;
-            const float* cs = a.cos_sin + (long)a.pos[mq] * d;
 #pragma unroll
-            for (int j = 0; j < FN32; ++j) {
-              const int cb = wn * WN + 32 * j, nb = n0 + cb;
-              const float xs = bfr(acc32[i][j][v] * ri);
-              const float xp = __shfl_xor(xs, 16, 64);
-              if (nb >= N) continue;   // wave-uniform
-              if (nb < qcols + kcols) {
-                const int cc = nb < qcols ? nb : nb - qcols;
-                const int d1 = 16 * ((cc % d) >> 5) + c16;
-                const float co = cs[d1], si = cs[hd + d1];
-                // first half (x1 = own, x2 = partner): x1 co - x2 si; second half: x2 co + x1 si
-                so[rl * OLD + cb + lc] = f2bf(hi ? xs * co + xp * si : xs * co - xp * si);
-              } else if (a.v_rows != nullptr) {
-                so[rl * OLD + cb + lc] = f2bf(xs);
-              } else if (m < M && slot >= 0) {
-                const int cc = nb - qcols - kcols;
-                u16* vo = a.vc + (((long)(slot >> 4) * nkv + cc / d) * d) * 16 + (slot & 15);
-                vo[(long)(cc % d + lc) * 16] = f2bf(xs);
-              }
-            }
+            for (int j = 0; j < FN32; ++j) so[rl * OLD + wn * WN + 32 * j + lc] = f2bf(acc32[i][j][v] * ri);
           } else if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
             for (int j = 0; j < FN32; ++j) {
@@ -698,71 +666,86 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
   }
 
   if constexpr (EPI == EPI_QKV) {
-    // RoPE in registers (pairs in adjacent fragments of one lane), V written straight from the
-    // registers (transposed cache layout: no row vectors to form), q/k staged.
+    // The tile is staged row-scaled and rounded; the copy-out rotates row vectors of eight pairs.  (Rotated in registers every lane
+    // waited for the table rows of its FM x 4 output rows one after the other, and V went out in 2-byte stores 32 B apart: of a
+    // 256 x 128 tile's 54 us at 2100 rows that was 21.)
     const int d = a.d, hd = d / 2, nq = a.nq, nkv = a.nkv;
-    const int qcols = nq * d, kcols = nkv * d;
-    int* s_slot = reinterpret_cast<int*>(s_red);   // [BM] cache slot per tile row (copy-out)
+    const int qcols = nq * d, kcols = nkv * d, vcol0 = qcols + kcols;
+    int* s_slot = reinterpret_cast<int*>(s_red);   // [BM] cache slot, [BM] position per tile row
+    int* s_pos = s_slot + BM;
+#pragma unroll
+    for (int i = 0; i < QR; ++i) {
+      const int r = threadIdx.x + i * NT;
+      if (r < BM) { s_slot[r] = q_slot[i]; s_pos[r] = q_pos[i]; }
+    }
     if (fw && MF == 16) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int rl = rl0 + 16 * i + e, m = m0 + rl;
-        const int mq = min(m, M - 1);
-        const int slot = QPF ? q_slot[(4 * i + e) % QR] : a.slots[mq];
-        if (wn == 0 && cl == 0) s_slot[rl] = slot;
-        const float* cs = a.cos_sin + (long)(QPF ? q_pos[(4 * i + e) % QR] : a.pos[mq]) * d;
-        const long blk = slot >> 4, off = slot & 15;
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int jp = 0; jp < FN / 2; ++jp) {
-          const int cb = wn * WN + 32 * jp;  // tile column of this 32-aligned group
-          const int nb = n0 + cb;
-          if (nb >= N) continue;
-          const float x1 = bfr(acc[i][2 * jp][e] * rinv[i][e]), x2 = bfr(acc[i][2 * jp + 1][e] * rinv[i][e]);
-          if (nb < qcols + kcols) {
-            const int cc = nb < qcols ? nb : nb - qcols;
-            const int d1 = 16 * ((cc % d) >> 5) + cl;
-            const float co = cs[d1], si = cs[hd + d1];
-            so[rl * OLD + cb + cl] = f2bf(x1 * co - x2 * si);
-            so[rl * OLD + cb + 16 + cl] = f2bf(x2 * co + x1 * si);
-          } else if (a.v_rows != nullptr) {
-            // V staged like q/k and copied out as 16-B row vectors (natural dim order)
-            so[rl * OLD + cb + cl] = f2bf(x1);
-            so[rl * OLD + cb + 16 + cl] = f2bf(x2);
-          } else if (m < M && slot >= 0) {
-            // V^T cache directly: 2-byte stores 32 B apart (the slow form: a workgroup holding
-            // V columns takes several us longer than its q/k neighbours at decode batch sizes)
-            const int cc = nb - qcols - kcols;
-            const int head = cc / d, dim = cc % d + cl;
-            u16* vo = a.vc + ((blk * nkv + head) * d) * 16 + off;
-            vo[(long)dim * 16] = f2bf(x1);
-            vo[(long)(dim + 16) * 16] = f2bf(x2);
-          }
-        }
-      }
+          for (int j = 0; j < FN; ++j) so[(rl0 + 16 * i + e) * OLD + wn * WN + 16 * j + cl] = f2bf(acc[i][j][e] * rinv[i][e]);
     }
     __syncthreads();
-    // copy-out of q/k: an 8-column chunk of a 16-column half-group is 8 consecutive natural dims
-    for (int e = threadIdx.x; e < BM * (BN / 8); e += NT) {
-      const int rl = e / (BN / 8), c0 = (e % (BN / 8)) * 8;
+    for (int e = threadIdx.x; e < BM * (BN / 16); e += NT) {
+      const int rl = e / (BN / 16), u = e % (BN / 16), c0 = 32 * (u >> 1) + 8 * (u & 1);
       const int m = m0 + rl, n = n0 + c0;
-      if (m >= M || n >= N) continue;
-      if (n >= qcols + kcols) {
-        if (a.v_rows != nullptr) st16(a.v_rows + (long)m * a.v_ld + (n - qcols - kcols), *reinterpret_cast<const uint4*>(so + rl * OLD + c0));
-        continue;
-      }
+      if (m >= M || n >= vcol0 || n >= N) continue;
       const bool isq = n < qcols;
-      const int cc = isq ? n : n - qcols;
-      const int head = cc / d, o = cc % d;
-      const int dim = ((o & 31) >> 4) * hd + 16 * (o >> 5) + (o & 15);
-      const uint4 v = *reinterpret_cast<const uint4*>(so + rl * OLD + c0);
-      if (isq) {
-        st16(a.q_out + ((long)m * nq + head) * d + dim, v);
-      } else {
-        const int slot = s_slot[rl];
-        if (slot >= 0) st16(a.kc + (((long)(slot >> 4) * nkv + head) * 16 + (slot & 15)) * d + dim, v);
+      const int cc = isq ? n : n - qcols, head = cc / d, o = cc % d, d1 = 16 * (o >> 5) + (o & 15);
+      const float* cs = a.cos_sin + (long)s_pos[rl] * d + d1;
+      float co[8], si[8], x1[8], x2[8], r1[8], r2[8];
+      *(float4*)&co[0] = *(const float4*)cs;
+      *(float4*)&co[4] = *(const float4*)(cs + 4);
+      *(float4*)&si[0] = *(const float4*)(cs + hd);
+      *(float4*)&si[4] = *(const float4*)(cs + hd + 4);
+      unpack8(*reinterpret_cast<const uint4*>(so + rl * OLD + c0), x1);
+      unpack8(*reinterpret_cast<const uint4*>(so + rl * OLD + c0 + 16), x2);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        r1[j] = x1[j] * co[j] - x2[j] * si[j];
+        r2[j] = x2[j] * co[j] + x1[j] * si[j];
       }
+      const int slot = s_slot[rl];
+      u16* dst = isq ? a.q_out + ((long)m * nq + head) * d
+                     : (slot >= 0 ? a.kc + (((long)(slot >> 4) * nkv + head) * 16 + (slot & 15)) * d : nullptr);
+      if (dst) {
+        st16(dst + d1, pack8(r1));
+        st16(dst + hd + d1, pack8(r2));
+      }
+    }
+    if (n0 + BN <= vcol0) return;      // (block-uniform)
+    const int v0 = max(0, vcol0 - n0), nv = min(BN, N - n0) - v0;      // this tile's V columns
+    if (a.v_rows != nullptr) {
+      for (int e = threadIdx.x; e < BM * (nv / 8); e += NT) {
+        const int rl = e / (nv / 8), c = v0 + (e % (nv / 8)) * 8;
+        if (m0 + rl < M) st16(a.v_rows + (long)(m0 + rl) * a.v_ld + (n0 + c - vcol0), *reinterpret_cast<const uint4*>(so + rl * OLD + c));
+      }
+      return;
+    }
+    // V^T cache [block][head][dim][16]: eight rows in eight consecutive slots of half a block (a prompt's) are one 16-byte store per
+    // dim, written by the first of them; rows outside such a run store their two bytes
+    int* s_run = reinterpret_cast<int*>(s_rsp);      // [BM] 0 alone, 1 in a run, 2 a run's first (the row scales are in registers)
+    for (int r = threadIdx.x; r < BM; r += NT) {
+      const int sl = s_slot[r], st = r - (sl & 7);
+      bool run = sl >= 0 && st >= 0 && st + 7 < BM && m0 + st + 7 < M;
+      if (run)
+        for (int j = 0; j < 8; ++j) run = run && s_slot[st + j] == (sl & ~7) + j;
+      s_run[r] = run ? 1 + (st == r) : 0;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < BM * nv; e += NT) {
+      const int rl = e / nv, c = v0 + e % nv, run = s_run[rl], slot = s_slot[rl];
+      if (m0 + rl >= M || slot < 0 || run == 1) continue;
+      const int cc = n0 + c - vcol0;
+      u16* vo = a.vc + (((long)(slot >> 4) * nkv + cc / d) * d + cc % d) * 16 + (slot & 15);
+      if (run == 2) {
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          w[j] = (uint32_t)so[(rl + 2 * j) * OLD + c] | ((uint32_t)so[(rl + 2 * j + 1) * OLD + c] << 16);
+        st16(vo, make_uint4(w[0], w[1], w[2], w[3]));
+      } else *vo = so[rl * OLD + c];
     }
     return;
   } else {
