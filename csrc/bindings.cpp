@@ -188,6 +188,12 @@ void check_f32(const torch::Tensor& t, const char* name) {
   check_dev(t, name);
   TORCH_CHECK(t.scalar_type() == torch::kFloat32 && t.is_contiguous(), name, " must be contiguous f32");
 }
+// row sums of squares [slots, >= M], a range of rows of a larger buffer among them
+void check_slots(const torch::Tensor& t, int64_t slots, int64_t M, const char* name) {
+  check_dev(t, name);
+  TORCH_CHECK(t.scalar_type() == torch::kFloat32 && t.dim() == 2 && t.size(0) >= slots && t.size(1) >= M && (t.stride(1) == 1 || M <= 1) &&
+                  (t.stride(0) >= M || t.size(0) <= 1), name, ": f32 [slots, >= M]");
+}
 void ok(int rc, const char* what) { TORCH_CHECK(rc == 0, what, " launch failed, code ", rc); }
 
 // y = norm(x (+ residual)) * w (+ b); residual (if given) is updated in place to x + residual.
@@ -1331,13 +1337,12 @@ void tgemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> y, int
     a.counters = counters->data_ptr<int>();
   }
   if (ssq_in.has_value()) {
-    check_f32(*ssq_in, "ssq_in");
-    TORCH_CHECK(ssq_in->dim() == 2 && ssq_in->size(1) >= M && ssq_in_n >= 1 && ssq_in_n <= ssq_in->size(0),
-                "ssq_in [slots, >= M]");
+    TORCH_CHECK(ssq_in_n >= 1, "ssq_in_n");
+    check_slots(*ssq_in, ssq_in_n, M, "ssq_in");
     TORCH_CHECK(epi != 1, "residual epilogue takes no row scale");
     a.ssq_in = ssq_in->data_ptr<float>();
     a.ssq_in_n = ssq_in_n;
-    a.ssq_in_ld = ssq_in->size(1);
+    a.ssq_in_ld = ssq_in->stride(0);
     a.norm_scale = (float)norm_scale;
     a.eps = (float)eps;
   }
@@ -1356,11 +1361,9 @@ void tgemm(torch::Tensor x, torch::Tensor w, c10::optional<torch::Tensor> y, int
     a.ldy = y->stride(0);
   }
   if (epi == 1 && ssq_out.has_value()) {
-    check_f32(*ssq_out, "ssq_out");
-    TORCH_CHECK(ssq_out->dim() == 2 && ssq_out->size(0) >= (N + bn - 1) / bn && ssq_out->size(1) >= M,
-                "ssq_out [>= n_tiles, >= M]");
+    check_slots(*ssq_out, (N + bn - 1) / bn, M, "ssq_out");
     a.ssq_out = ssq_out->data_ptr<float>();
-    a.ssq_out_ld = ssq_out->size(1);
+    a.ssq_out_ld = ssq_out->stride(0);
   }
   if (epi == 3) TORCH_CHECK(N % 32 == 0, "swiglu: N % 32 == 0");
   if (epi == 2) {
@@ -1410,14 +1413,14 @@ void qkv_post(torch::Tensor y, torch::Tensor ssq, int64_t ssq_n, double scale, d
               torch::Tensor cos_sin, torch::Tensor slots, torch::Tensor q_out, torch::Tensor kc, torch::Tensor vc,
               int64_t nq, int64_t nkv, int64_t d, c10::optional<torch::Tensor> v_rows) {
   check_bf16(y, "y");
-  check_f32(ssq, "ssq");
   check_i32(pos, "positions");
   check_i32(slots, "slots");
   check_f32(cos_sin, "cos_sin");
   for (auto* t : {&q_out, &kc, &vc}) check_bf16(*t, "qkv outputs");
   const int M = y.size(0);
   TORCH_CHECK(y.dim() == 2 && y.stride(1) == 1 && y.size(1) == (nq + 2 * nkv) * d && d % 32 == 0, "y [M, (nq+2nkv) d]");
-  TORCH_CHECK(ssq.dim() == 2 && ssq.size(1) >= M && ssq_n >= 1 && ssq_n <= ssq.size(0), "ssq [slots, >= M]");
+  TORCH_CHECK(ssq_n >= 1, "ssq_n");
+  check_slots(ssq, ssq_n, M, "ssq");
   TORCH_CHECK(pos.numel() >= M && slots.numel() >= M && cos_sin.size(1) == d, "positions/slots/cos_sin");
   TORCH_CHECK(q_out.is_contiguous() && q_out.numel() >= (int64_t)M * nq * d, "q_out");
   TORCH_CHECK(kc.is_contiguous() && vc.is_contiguous() && kc.size(1) == nkv && kc.size(2) == 16 && kc.size(3) == d &&
@@ -1429,7 +1432,7 @@ void qkv_post(torch::Tensor y, torch::Tensor ssq, int64_t ssq_n, double scale, d
     TORCH_CHECK(v_rows->is_contiguous() && v_rows->numel() >= (int64_t)M * nkv * d, "v_rows [M, nkv d]");
     vr = v_rows->data_ptr();
   }
-  ok(dllm_qkv_post(y.data_ptr(), y.stride(0), ssq.data_ptr<float>(), ssq_n, ssq.size(1), (float)scale, (float)eps,
+  ok(dllm_qkv_post(y.data_ptr(), y.stride(0), ssq.data_ptr<float>(), ssq_n, ssq.stride(0), (float)scale, (float)eps,
                    pos.data_ptr<int>(), cos_sin.data_ptr<float>(), slots.data_ptr<int>(), q_out.data_ptr(), kc.data_ptr(),
                    vc.data_ptr(), vr, M, nq, nkv, d, stream()),
      "qkv_post");
@@ -1437,13 +1440,13 @@ void qkv_post(torch::Tensor y, torch::Tensor ssq, int64_t ssq_n, double scale, d
 
 void swiglu_post(torch::Tensor y, torch::Tensor ssq, int64_t ssq_n, double scale, double eps, torch::Tensor act) {
   check_bf16(y, "y");
-  check_f32(ssq, "ssq");
   check_bf16(act, "act");
   const int M = y.size(0), N = y.size(1);
   TORCH_CHECK(y.dim() == 2 && y.stride(1) == 1 && N % 32 == 0, "y [M, 2I]");
   TORCH_CHECK(act.dim() == 2 && act.stride(1) == 1 && act.size(0) == M && act.size(1) == N / 2, "act [M, I]");
-  TORCH_CHECK(ssq.dim() == 2 && ssq.size(1) >= M && ssq_n >= 1 && ssq_n <= ssq.size(0), "ssq [slots, >= M]");
-  ok(dllm_swiglu_post(y.data_ptr(), y.stride(0), ssq.data_ptr<float>(), ssq_n, ssq.size(1), (float)scale, (float)eps,
+  TORCH_CHECK(ssq_n >= 1, "ssq_n");
+  check_slots(ssq, ssq_n, M, "ssq");
+  ok(dllm_swiglu_post(y.data_ptr(), y.stride(0), ssq.data_ptr<float>(), ssq_n, ssq.stride(0), (float)scale, (float)eps,
                       act.data_ptr(), act.stride(0), M, N, stream()),
      "swiglu_post");
 }

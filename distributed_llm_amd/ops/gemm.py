@@ -152,6 +152,9 @@ class _Planner:
         self.dg_plans: Dict[Tuple[int, int, int], Tuple] = {}        # decode GEMM (nt, vs, splits), where it beats plans[...]
         self.fused_core: Dict[Tuple[int, int, int], str] = {}        # "tg" | "lin" | "gemvR" | "skES" | "dgN.V.S" per tuned shape
         self.fused_opts: Dict[Tuple[int, int, int], Dict[str, float]] = {}   # measured us per core choice
+        self.pf_times: Dict[Tuple[int, int], list] = {}      # (N, K) of prompts: [(plan, rows, us)]
+        self.pf_small: Dict[Tuple[int, int, int], Tuple] = {}        # (rows of PF_SMALL_MS, N, K): (fastest plan, its us)
+        self.pf_parts: Dict[Tuple[int, int, int], Tuple] = {}        # prompt_parts' answers
         self.ws: Dict[Tuple, Tuple[torch.Tensor, torch.Tensor]] = {}
         self.sk_tables: Dict[Tuple, Tuple[torch.Tensor, int]] = {}   # stream-K segment lists per shape
         self.timings: Dict[Tuple[int, int, int, bool], Dict[str, float]] = {}
@@ -288,6 +291,80 @@ _PF_PLANS = ((256, 256, 2, 1, 1, 8), (256, 128, 3, 1, 1, 8), (192, 128, 3, 1, 1,
              (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 8))
 
 
+# Row counts between the decode buckets and the prefill buckets, whose plans are timed once too: a short prompt's products, and what
+# prompt_parts leaves behind whole rounds of large tiles.
+PF_SMALL_MS = (128, 256, 384, 512, 768, 1024)
+_PF_SMALL = ((64, 64, 3, 1, 1, 4), (64, 64, 3, 2, 1, 4), (64, 64, 4, 1, 1, 4, 1, 8), (64, 128, 3, 1, 1, 8), (128, 64, 4, 1, 1, 4, 1, 8),
+             (128, 128, 3, 1, 1, 8), (160, 128, 3, 1, 1, 8, 1, 6), (192, 128, 3, 1, 1, 8), (256, 128, 3, 1, 1, 8, 1, 8))
+_PART_US = 4.0            # a second launch of a product, and the clearing of row-sum slots it does not write
+_PART_GAIN = 0.95         # another plan than the bucket's, or a second launch, where the rounds make it that much shorter: they are
+#                           within 5 % of what is measured
+
+
+def _small(m: int, N: int, K: int):
+    """(fastest plan, its us) timed for the next of PF_SMALL_MS, or None."""
+    b = next((b for b in PF_SMALL_MS if m <= b), None)
+    return None if b is None else _P.pf_small.get((b, N, K))
+
+
+def _rounds(tiles: int, cus: int) -> float:
+    """Rounds that tiles take on the CUs: one that is part full is hardly shorter (TinyLlama's down, 256 x 128 and 192 x 128 tiles, 2100
+    rows: 77 and 83 us with 144 and 176 of 256 CUs, 86 and 88 with all)."""
+    full, rest = divmod(tiles, cus)
+    return full + (0.8 + 0.2 * rest / cus if rest else 0.0)
+
+
+def _round_us(N: int, K: int, cus: int = 256):
+    """us a round of each timed prompt plan, from the largest size it was timed at."""
+    out = {}
+    for plan, m, t in sorted(_P.pf_times.get((N, K), ()), key=lambda e: e[1]):
+        out[plan] = t / _rounds(-(-m // plan[0]) * -(-N // plan[1]), cus)
+    return out
+
+
+def prompt_parts(M: int, N: int, K: int, cus: int = 256) -> Optional[Tuple]:
+    """How the one-launch form of a fused product of a prompt's M > MAX_M rows runs: ((rows, plan), ...) one behind the other, or None
+    where nothing was timed.  A large tile costs by rounds over the CUs: 8928 rows of 2048 columns are 280 tiles of 256 x 256, two
+    rounds of which the second holds 24, so the last 736 rows go to a launch of small tiles.  us, one launch / here, TinyLlama: Wo
+    4500 rows 72 / 56, 8928 rows 140 / 94; gate|up 1500 rows 107 / 92, 3000 rows 196 / 157, 4500 rows 261 / 224."""
+    key = (M, N, K)
+    if key in _P.pf_parts:
+        return _P.pf_parts[key]
+    best, parts = float("inf"), None
+    rounds, usual = _round_us(N, K, cus), tg_plan(M, N, K)
+    tiles = lambda rows, plan: -(-rows // plan[0]) * -(-N // plan[1])
+    if usual in rounds:
+        best, parts = _PART_GAIN * _rounds(tiles(M, usual), cus) * rounds[usual], ((M, usual),)
+    for plan, u in rounds.items():
+        t = _rounds(tiles(M, plan), cus) * u
+        if t < best:
+            best, parts = t, ((M, plan),)
+        for k in range(1, -(-tiles(M, plan) // cus)):      # k rounds of it, and the rows they leave
+            rows = k * cus // -(-N // plan[1]) * plan[0]
+            tail = _small(M - rows, N, K) if 0 < rows < M else None
+            if tail is not None:
+                t = _rounds(tiles(rows, plan), cus) * u + tail[1] + _PART_US
+                if t < best:
+                    best, parts = t, ((rows, plan), (M - rows, tail[0]))
+    if parts is not None:
+        if len(_P.pf_parts) > 4096:
+            _P.pf_parts.clear()
+        _P.pf_parts[key] = parts
+    return parts
+
+
+def _row_parts(M: int, N: int, K: int) -> list:
+    """[(first row, end, plan or "lin")]: a fused product's launches."""
+    if use_vendor_core(M, N, K):
+        return [(0, M, "lin")]
+    parts = prompt_parts(M, N, K) if M > MAX_M and PREFILL_MS and not os.environ.get("DLLM_FUSED_CORE") else None
+    out, lo = [], 0
+    for rows, plan in parts or ((M, tg_plan(M, N, K)),):
+        out.append((lo, lo + rows, plan))
+        lo += rows
+    return out
+
+
 def prefill_bucket(M: int) -> int:
     for b in PREFILL_MS:
         if M <= b:
@@ -315,6 +392,8 @@ def tg_plan(M: int, N: int, K: int) -> Tuple[int, ...]:
         p = _P.tg_plans.get((prefill_bucket(M), N, K))
     if p is None and M <= MAX_M:      # rows between two timed batch sizes (a short prompt): what was timed for the next one
         p = _P.tg_plans.get((next_batch_size(M), N, K))
+        if p is None and M > DG_MAX_M:
+            p = (_small(M, N, K) or (None,))[0]
     if p is not None:
         return tuple(p) + (1, 4)[len(p) - 4:] if len(p) < 6 else tuple(p)
     mt128, nt128 = -(-M // 128), -(-N // 128)
@@ -648,15 +727,19 @@ def qkv_rope_cache(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: i
         skinny_epi(r, wp if wp is not None else w, EPI_QKV, sp, ssq_in=ssq, ssq_n=ssq_n, scale=1.0 / H, eps=eps,
                    pos=positions, cos_sin=cos_sin, slots=slots, q_out=q, kc=k_cache, vc=v_cache, nq=nq, nkv=nkv, d=d)
         return out(False)
-    if use_vendor_core(T, w.shape[0], H):
-        vr = v_new if QKV_POST_VROWS else None
-        _native(r).qkv_post(_core(r, w, wp), ssq, int(ssq_n), 1.0 / H, float(eps), positions, cos_sin, slots, q,
-                            k_cache, v_cache, nq, nkv, d, vr)
-        return out(vr is not None)
-    _tgemm(_native(r), r, wp if wp is not None else w, EPI_QKV, tg_plan(T, w.shape[0], H), ssq_in=ssq, ssq_n=ssq_n, norm_scale=1.0 / H,
-           eps=eps, pos=positions, cos_sin=cos_sin, slots=slots, q_out=q, kc=k_cache, vc=v_cache, nq=nq, nkv=nkv,
-           d=d, v_rows=v_new)
-    return out(True)
+    for lo, hi, plan in _row_parts(T, w.shape[0], H):
+        rows, sq = (r, ssq) if hi - lo == T else (r[lo:hi], ssq[:, lo:hi])
+        if plan == "lin":
+            vr = v_new if QKV_POST_VROWS else None
+            _native(r).qkv_post(_core(rows, w, wp), sq, int(ssq_n), 1.0 / H, float(eps), positions[lo:hi], cos_sin, slots[lo:hi], q[lo:hi],
+                                k_cache, v_cache, nq, nkv, d, vr)      # (all rows)
+            used = vr is not None
+        else:
+            _tgemm(_native(r), rows, wp if wp is not None else w, EPI_QKV, plan, ssq_in=sq, ssq_n=ssq_n, norm_scale=1.0 / H,
+                   eps=eps, pos=positions[lo:hi], cos_sin=cos_sin, slots=slots[lo:hi], q_out=q[lo:hi], kc=k_cache, vc=v_cache, nq=nq,
+                   nkv=nkv, d=d, v_rows=v_new if v_new is None else v_new[lo:hi])
+            used = True
+    return out(used)
 
 
 def matmul_resadd(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, ssq_out: torch.Tensor,
@@ -673,12 +756,20 @@ def matmul_resadd(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, ssq_
     sp = fused_ske(x, N, K) if M else 0
     if sp:
         return skinny_epi(x, wp if wp is not None else w, EPI_RESADD, sp, res=residual, ssq_out=ssq_out)
-    if M and use_vendor_core(M, N, K):
+    if not M:
+        return -(-N // tg_plan(M, N, K)[1])
+    parts = _row_parts(M, N, K)
+    if parts[0][2] == "lin":
         return int(_native(x).res_add_ssq(_core(x, w, wp), residual, ssq_out))
-    plan = tg_plan(M, N, K)
-    if M:
-        _tgemm(_native(x), x, wp if wp is not None else w, EPI_RESADD, plan, y=residual, ssq_out=ssq_out)
-    return -(-N // plan[1])
+    n = max(-(-N // p[1]) for _, _, p in parts)
+    for lo, hi, plan in parts:
+        mine, whole = -(-N // plan[1]), hi - lo == M
+        so = ssq_out if whole else ssq_out[:, lo:hi]
+        _tgemm(_native(x), x if whole else x[lo:hi], wp if wp is not None else w, EPI_RESADD, plan, y=residual if whole else residual[lo:hi],
+               ssq_out=so)
+        if mine < n:
+            so[mine:n].zero_()
+    return n
 
 
 def swiglu_matmul(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: int, eps: float,
@@ -700,12 +791,15 @@ def swiglu_matmul(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: in
         skinny_epi(r, wp if wp is not None else w, EPI_SWIGLU, sp, y=act, ssq_in=ssq, ssq_n=ssq_n, scale=1.0 / H,
                    eps=eps)
         return act
-    if T and use_vendor_core(T, w.shape[0], H):
-        _native(r).swiglu_post(_core(r, w, wp), ssq, int(ssq_n), 1.0 / H, float(eps), act)
+    if not T:
         return act
-    if T:
-        _tgemm(_native(r), r, wp if wp is not None else w, EPI_SWIGLU, tg_plan(T, w.shape[0], H), y=act, ssq_in=ssq, ssq_n=ssq_n,
-               norm_scale=1.0 / H, eps=eps)
+    for lo, hi, plan in _row_parts(T, w.shape[0], H):
+        rows, sq = (r, ssq) if hi - lo == T else (r[lo:hi], ssq[:, lo:hi])
+        if plan == "lin":
+            _native(r).swiglu_post(_core(rows, w, wp), sq, int(ssq_n), 1.0 / H, float(eps), act[lo:hi])
+        else:
+            _tgemm(_native(r), rows, wp if wp is not None else w, EPI_SWIGLU, plan, y=act[lo:hi], ssq_in=sq, ssq_n=ssq_n, norm_scale=1.0 / H,
+                   eps=eps)
     return act
 
 
@@ -858,6 +952,10 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
                 parts = k.split(",")
                 if parts[0] == "t":
                     _P.tg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
+                elif parts[0] == "s":
+                    _P.pf_small[tuple(int(q) for q in parts[1:])] = (tuple(v[0]), v[1])
+                elif parts[0] == "p":
+                    _P.pf_times[(int(parts[1]), int(parts[2]))] = [(tuple(q), m, t) for q, m, t in v]
                 elif parts[0] == "d":
                     _P.dg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
                 elif parts[0] == "c":
@@ -874,23 +972,27 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
               qkv_cache, {tuple(f) for f in frag})
     _couple_gemv_choices(fused, list(ms), verbose)
     if PREFILL_TUNE or prefill:
-        _autotune_prefill(fused, dev, verbose)
+        _autotune_prefill(fused, dev, verbose, roles, qkv_dims)
     if cache:
         import json
         d = {_plan_key(k): list(v) for k, v in _P.plans.items()}
         d.update({_plan_key(k): list(v) for k, v in _P.tg_plans.items()})
         d.update({"c,%d,%d,%d" % k: v for k, v in _P.fused_core.items()})
         d.update({"d,%d,%d,%d" % k: list(v) for k, v in _P.dg_plans.items()})
+        d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
+        d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
         if os.path.dirname(cache):
             os.makedirs(os.path.dirname(cache), exist_ok=True)
         with open(cache, "w") as f:
             json.dump(d, f)
 
 
-def _autotune_prefill(fused, dev, verbose: bool) -> None:
+def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> None:
     """Fused-op core at the prefill buckets: one tgemm launch with the epilogue fused (PLAIN timed,
     the fused epilogues write the same tile or less) against hipBLASLt + the standalone epilogue
-    kernel; the tgemm plans stream the K-panel weight copy the model keeps (W_PANEL)."""
+    kernel; the tgemm plans stream the K-panel weight copy the model keeps (W_PANEL).  Among the tgemm plans
+    ``prompt_parts`` chooses by times with the epilogue; plans of the sizes below the buckets are timed too."""
+    roles = roles or {}
     for (N, K) in {tuple(f) for f in fused}:
         todo = [M for M in PREFILL_MS if (M, N, K) not in _P.fused_core]
         if not todo or K % 64:
@@ -904,6 +1006,8 @@ def _autotune_prefill(fused, dev, verbose: bool) -> None:
             ext = _native(x)
             lin = _time(lambda i: torch.matmul(x, ws[i % copies].t(), out=y), iters=8) + _post_us(M, N, dev)
             best, best_t = None, float("inf")
+            times = _P.pf_times.setdefault((N, K), [])
+            whole = _fused_call(roles.get((N, K)), x, ws, wps, qkv_dims, dev)
             for p in _PF_PLANS:
                 try:
                     t = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
@@ -911,6 +1015,13 @@ def _autotune_prefill(fused, dev, verbose: bool) -> None:
                     continue
                 if t < best_t:
                     best, best_t = p, t
+                if whole is not None:      # with its epilogue: what choosing among the plans goes by
+                    _P.pf_parts[(M, N, K)] = ((M, p),)
+                    saved, _P.fused_core[(M, N, K)] = _P.fused_core.get((M, N, K)), "tg"
+                    t = _time(whole, iters=8)
+                    if saved is None:
+                        del _P.fused_core[(M, N, K)]
+                times.append((p, M, t))
             if best is not None:
                 _P.tg_plans[(M, N, K)] = best
             _P.fused_core[(M, N, K)] = "tg" if best is not None and best_t < lin else "lin"
@@ -918,6 +1029,18 @@ def _autotune_prefill(fused, dev, verbose: bool) -> None:
                 print(f"gemm prefill M={M} N={N} K={K}: blas+post {lin:.1f}us, tgemm {best} {best_t:.1f}us "
                       f"-> {_P.fused_core[(M, N, K)]}", flush=True)
             del x, y
+        for M in PF_SMALL_MS:
+            x, y = torch.randn(M, K, device=dev).to(torch.bfloat16), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+            ext, res = _native(x), {}
+            for p in _PF_SMALL:
+                if p[0] > max(64, M) or (p[3] > 1 and _need_tg(M, N, K, p[0], p[1], p[3])[0] > WS_FLOATS) or _tg_splits(K, p[3]) != p[3]:
+                    continue
+                res[p] = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
+            best = min(res, key=res.get)
+            _P.pf_small[(M, N, K)] = (best, res[best])
+            if verbose:
+                print(f"gemm rows M={M} N={N} K={K}: {best} {res[best]:.1f}us", flush=True)
+        _P.pf_parts.clear()
         del ws, wps
 
 
@@ -1017,18 +1140,16 @@ def _dg_cands(M: int, N: int, K: int):
     return out
 
 
-def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, wfs=None):
-    """Time every fused-core option of a decoder-layer shape through the fused op itself: its real
-    epilogue and its row-scale prologue over the producer's partial row sums.  The stand-in timings
-    (PLAIN tgemm, RESADD GEMV / skinny_epi) missed those: gate|up at batch 4 chose a tgemm timed at
-    13.6 us that ran 17.3 us inside the step graph (profiles/r6_small_batch.md)."""
-    M, N, K = tkey
+def _fused_call(role, x, ws, wps, qkv_dims, dev, qkv_cache=None, wfs=None):
+    """fn(i): the fused op of a layer's weight (``role`` qkv, resadd or swiglu) on rows x and the i-th copy of its weights, or None."""
+    if role is None:
+        return None
+    M, N, K = x.shape[0], ws[0].shape[0], ws[0].shape[1]
     copies = len(ws)
     wsrc = lambda i: (ws[i % copies], wps[i % copies] if wps is not None else None)
     wf = lambda i: wfs[i % copies] if wfs is not None else None
-    if wfs is not None:
-        opts = dict(opts, **{"dg%d.%d.%d" % p: 0.0 for p in _dg_cands(M, N, K)})
-    slots_in = -(-K // 32)   # the producer's partial row sums (as many as a skinny_epi producer leaves)
+    prompt = M > MAX_M
+    slots_in = -(-K // (128 if prompt else 32))   # the producer's partial row sums (as many as a skinny_epi producer leaves)
     ssq = torch.rand(slots_in, M, device=dev) + 1.0
     if role == "resadd":
         res = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
@@ -1052,14 +1173,31 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, w
             kc = torch.zeros(nblk, nkv, 16, d, dtype=torch.bfloat16, device=dev)
             vc = torch.zeros(nblk, nkv, d, 16, dtype=torch.bfloat16, device=dev)
         pos = torch.randint(100, 4000, (M,), dtype=torch.int32, device=dev)
-        sl = (torch.randperm(nblk, device=dev)[:M] * 16 + torch.randint(0, 16, (M,), device=dev)).to(torch.int32)
+        if prompt:      # one sequence's rows, one behind the other
+            sl = torch.arange(M, dtype=torch.int32, device=dev)
+        else:
+            sl = (torch.randperm(nblk, device=dev)[:M] * 16 + torch.randint(0, 16, (M,), device=dev)).to(torch.int32)
         cs = torch.rand(4096, d, device=dev)
         # (d = 64 decode hands V over row-major, as models.llama does: the one-launch cores then skip
         # the strided V^T cache writes)
-        vn = torch.empty(M, nkv * d, dtype=torch.bfloat16, device=dev) if d == 64 else None
+        vn = torch.empty(M, nkv * d, dtype=torch.bfloat16, device=dev) if d == 64 and not prompt else None
         fn = lambda i: qkv_rope_cache(x, wsrc(i)[0], ssq, slots_in, 1e-5, pos, cs, sl, kc, vc, nq, nkv, d,
                                       wp=wsrc(i)[1], v_new=vn, wf=wf(i))
     else:
+        return None
+    return fn
+
+
+def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, wfs=None):
+    """Time every fused-core option of a decoder-layer shape through the fused op itself: its real
+    epilogue and its row-scale prologue over the producer's partial row sums.  The stand-in timings
+    (PLAIN tgemm, RESADD GEMV / skinny_epi) missed those: gate|up at batch 4 chose a tgemm timed at
+    13.6 us that ran 17.3 us inside the step graph (profiles/r6_small_batch.md)."""
+    M, N, K = tkey
+    if wfs is not None:
+        opts = dict(opts, **{"dg%d.%d.%d" % p: 0.0 for p in _dg_cands(M, N, K)})
+    fn = _fused_call(role, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
+    if fn is None:
         return None
     saved = _P.fused_core.get(tkey)
     out = {}

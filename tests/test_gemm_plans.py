@@ -59,3 +59,70 @@ def test_rows_between_batch_sizes_take_the_next_ones_plan(monkeypatch):
     assert G.tg_plan(65, 256, 512) == (64, 128, 3, 2, 1, 4)
     assert G.tg_plan(97, 256, 512)[:3] == G.tg_plan(48, 256, 512)[:3] == (64, 64, 3)      # no plan at 128 or 48 rows: the untimed rule
     assert G.tg_slots(57, 256, 512) == 4 and G.tg_slots(70, 256, 512) == 2
+
+
+def _timed(monkeypatch, N, K, us, small):
+    """Tables as the autotuner leaves them: a round of 256 tiles of 256 x 256 and of 256 x 128, and plans of small tiles."""
+    big, half = (256, 256, 2, 1, 1, 8), (256, 128, 3, 1, 1, 8)
+    times = [(p, m, u * -(-(-(-m // 256) * -(-N // p[1])) // 256)) for p, u in ((big, us), (half, 0.6 * us)) for m in (2048, 4096, 8192)]
+    monkeypatch.setattr(G._P, "pf_times", {(N, K): times})
+    monkeypatch.setattr(G._P, "pf_small", {(m, N, K): ((128, 128, 3, 1, 1, 8), small) for m in G.PF_SMALL_MS})
+    monkeypatch.setattr(G._P, "pf_parts", {})
+    monkeypatch.setattr(G._P, "tg_plans", {(m, N, K): big for m in (2048, 4096, 8192)})
+    return big, half
+
+
+@pytest.mark.parametrize("N,us,small", [(2048, 90.0, 15.0), (2560, 90.0, 15.0), (11264, 70.0, 20.0), (96, 50.0, 10.0), (2048, 20.0, 60.0)])
+def test_prompt_parts(monkeypatch, N, us, small):
+    big, half = _timed(monkeypatch, N, 256, us, small)
+    for M in list(range(1025, 12000, 331)) + [8192, 8928, 9000, 40000]:
+        parts = G.prompt_parts(M, N, 256)
+        assert sum(r for r, _ in parts) == M and len(parts) <= 2 and all(r > 0 for r, _ in parts)
+        (rows, plan) = parts[0]
+        assert plan in (big, half)
+        if len(parts) == 2:      # whole rounds of large tiles, then rows the small plans were timed for
+            assert rows % plan[0] == 0 and parts[1][0] <= G.PF_SMALL_MS[-1]
+            tiles, every = rows // plan[0] * -(-N // plan[1]), -(-M // plan[0]) * -(-N // plan[1])
+            assert -(-tiles // 256) < -(-every // 256)
+    if (N, us) == (2048, 90.0):
+        assert G.prompt_parts(8928, N, 256) == ((8192, big), (736, (128, 128, 3, 1, 1, 8)))
+        assert G.prompt_parts(8192, N, 256) == ((8192, big),)
+    monkeypatch.setattr(G._P, "pf_times", {})
+    monkeypatch.setattr(G._P, "pf_parts", {})
+    assert G.prompt_parts(8928, N, 256) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("panel", [False, True])
+def test_parts_are_the_whole(monkeypatch, panel):
+    """Each fused product in two parts against one launch: every row's chain over K is the same, so are its bits."""
+    torch.manual_seed(1)
+    M, H, I, nq, nkv, d = 1300, 256, 512, 4, 2, 64
+    N = (nq + 2 * nkv) * d
+    rnd = lambda *s: (torch.randn(*s, device="cuda") * s[-1] ** -0.5).bfloat16()  # noqa: E731
+    r, w_qkv, w_gu, w_d, res = rnd(M, H), rnd(N, H), rnd(2 * I, H), rnd(H, I), rnd(M, H)
+    ssq = torch.rand(1, M, device="cuda") + 1.0      # (several partial sums are added in an order that depends on the tile)
+    pos = torch.randint(0, 2000, (M,), device="cuda", dtype=torch.int32)
+    slots = torch.randperm(1600, device="cuda")[:M].to(torch.int32)
+    cs = ops.rope_cos_sin(2048, d, 10000.0, "cuda")
+    wp = G.panel_weight if panel else (lambda w: None)
+
+    def run():
+        kc, vc = torch.zeros(100, nkv, 16, d, device="cuda").bfloat16(), torch.zeros(100, nkv, d, 16, device="cuda").bfloat16()
+        q = G.qkv_rope_cache(r, w_qkv, ssq, 1, 1e-5, pos, cs, slots, kc, vc, nq, nkv, d, wp=wp(w_qkv))
+        act = G.swiglu_matmul(r, w_gu, ssq, 1, 1e-5, wp=wp(w_gu))
+        x, so = res.clone(), torch.full((G.max_slots(H, M), M), float("nan"), device="cuda")
+        n = G.matmul_resadd(act, w_d, x, so, wp=wp(w_d))
+        return q, kc, vc, act, x, so[:n].sum(0)
+
+    big, small = (256, 256, 2, 1, 1, 8), (64, 128, 3, 1, 1, 8)
+    monkeypatch.setattr(G, "use_vendor_core", lambda M, N, K: False)
+    monkeypatch.setattr(G, "prompt_parts", lambda M, N, K: ((M, big),))
+    one = run()
+    monkeypatch.setattr(G, "prompt_parts", lambda M, N, K: ((1024, big), (M - 1024, small)))
+    two = run()
+    assert all(torch.equal(a, b) for a, b in zip(one[:5], two[:5]))
+    torch.testing.assert_close(one[5], two[5], rtol=1e-5, atol=1e-6)
+    monkeypatch.setattr(G, "use_vendor_core", lambda M, N, K: True)
+    for a, b in zip(one, run()):
+        torch.testing.assert_close(a.float(), b.float(), rtol=2e-2, atol=2e-2)
