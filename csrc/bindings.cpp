@@ -44,7 +44,8 @@ int dllm_skinny_epi(const void*, long, const void*, int, void*, long, int, int, 
                     long, float*, long, const float*, int, long, float, float, const int*, const float*, const int*,
                     void*, void*, void*, int, int, int, hipStream_t);
 int dllm_dgemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*, void*, long, float*, long,
-               float, float, const int*, const float*, const int*, void*, void*, void*, void*, long, int, int, int, hipStream_t);
+               float, float, const int*, const float*, const int*, void*, void*, void*, void*, long, int, int, int, const float*, int, float,
+               float, hipStream_t);
 int dllm_skinny_gemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*,
                      hipStream_t);
 int dllm_moe_max_tiles(int, int);
@@ -738,15 +739,16 @@ void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw,
      "skinny_gemm");
 }
 // Decode GEMM on fragment-major weights (csrc/kernels/decode_gemm.hip), M <= 64: x [M, K], w [ceil(N / 16), K / 32, 64, 8]
-// (ops.gemm.frag_weight; paired for epi 2 and 3), epi 0 plain (y [M, N]), 1 residual add (res in place, per-tile row sums of squares ->
-// ssq_out), 2 QKV (row scale, RoPE, q_out, paged K, V^T or v_rows), 3 SwiGLU (row scale, y = act [M, N / 2]).  nt 16-column tiles a
-// workgroup, splits of K, vs of them a workgroup.  Returns the row-sum slots written (epi 1) or 0.
+// (ops.gemm.frag_weight; paired for epi 2, 3 and 4), epi 0 plain (y [M, N]), 1 residual add (res in place, per-tile row sums of squares ->
+// ssq_out), 2 QKV (row scale, RoPE, q_out, paged K, V^T or v_rows), 3 SwiGLU (row scale, y = act [M, N / 2]), 4 gated activation `mode` of glu_act with
+// bias (y [M, N / 2]), 5 erf GELU.  nt 16-column tiles a workgroup, splits of K, vs of them a workgroup.  Returns the row-sum slots written (epi 1) or 0.
 int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int64_t nt, int64_t vs, int64_t splits,
               c10::optional<torch::Tensor> y, c10::optional<torch::Tensor> part, c10::optional<torch::Tensor> counters,
               c10::optional<torch::Tensor> res, c10::optional<torch::Tensor> ssq_out, double scale, double eps,
               c10::optional<torch::Tensor> pos, c10::optional<torch::Tensor> cos_sin, c10::optional<torch::Tensor> slots,
               c10::optional<torch::Tensor> q_out, c10::optional<torch::Tensor> kc, c10::optional<torch::Tensor> vc,
-              c10::optional<torch::Tensor> v_rows, int64_t nq, int64_t nkv, int64_t d) {
+              c10::optional<torch::Tensor> v_rows, int64_t nq, int64_t nkv, int64_t d, c10::optional<torch::Tensor> bias, int64_t mode,
+              double limit, double alpha) {
   check_bf16(x, "x");
   check_bf16(w, "w");
   const int64_t M = x.size(0), K = x.dim() == 2 ? x.size(1) : 0, N = n_cols;
@@ -754,7 +756,7 @@ int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int
   TORCH_CHECK(M >= 1 && M <= 64 && K >= 32 && K % 32 == 0 && x.stride(0) >= (M > 1 ? K : 0), "M in [1, 64], K % 32 == 0");
   TORCH_CHECK(w.dim() == 4 && w.is_contiguous() && w.size(0) == (N + 15) / 16 && w.size(1) == K / 32 && w.size(2) == 64 && w.size(3) == 8 && N >= 1,
               "w: [ceil(N / 16), K / 32, 64, 8]");
-  TORCH_CHECK(epi >= 0 && epi <= 3 && nt >= 1 && nt <= 3 && (vs == 1 || vs == 2 || (vs == 4 && nt == 1 && M <= 32 && epi == 0)) && splits >= 1 && splits <= 64,
+  TORCH_CHECK(epi >= 0 && epi <= 5 && nt >= 1 && nt <= 3 && (vs == 1 || vs == 2 || (vs == 4 && nt == 1 && M <= 32 && (epi == 0 || epi >= 4))) && splits >= 1 && splits <= 64,
               "no such plan");
   const int64_t tiles = (N + 16 * nt - 1) / (16 * nt), kchunk = ((K + splits - 1) / splits + 31) / 32 * 32;
   const int64_t S = (K + kchunk - 1) / kchunk, gy = (S + vs - 1) / vs, mr = (M + 15) / 16 * 16;
@@ -774,11 +776,19 @@ int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int
   float* so = nullptr;
   const int *pos_p = nullptr, *sl = nullptr;
   const float* cs = nullptr;
-  if (epi == 0 || epi == 3) {
+  const bool half = epi == 3 || epi == 4;
+  const float* bp = nullptr;
+  if (epi == 0 || epi >= 3) {
     TORCH_CHECK(y.has_value(), "y required");
     check_bf16(*y, "y");
-    TORCH_CHECK(y->dim() == 2 && y->stride(1) == 1 && y->size(0) == M && y->size(1) == (epi == 3 ? N / 2 : N), "y shape");
-    TORCH_CHECK((uintptr_t)y->data_ptr() % 8 == 0 && (epi == 0 || (N % 32 == 0 && y->stride(0) % 4 == 0)), "y rows of 8 bytes");
+    TORCH_CHECK(y->dim() == 2 && y->stride(1) == 1 && y->size(0) == M && y->size(1) == (half ? N / 2 : N), "y shape");
+    TORCH_CHECK((uintptr_t)y->data_ptr() % 8 == 0 && (!half || (N % (epi == 3 ? 32 : 16) == 0 && y->stride(0) % 4 == 0)), "y rows of 8 bytes");
+    if (epi == 4 && bias.has_value()) {
+      check_f32(*bias, "bias");
+      TORCH_CHECK(bias->numel() == N && (uintptr_t)bias->data_ptr() % 16 == 0 && (N / 2) % 4 == 0, "bias [N]");
+      bp = bias->data_ptr<float>();
+    }
+    TORCH_CHECK(mode >= 0 && mode <= 2, "mode 0, 1 or 2");
     yp = y->data_ptr();
     ldy = y->stride(0);
   }
@@ -822,7 +832,8 @@ int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int
     }
   }
   ok(dllm_dgemm(x.data_ptr(), M > 1 ? x.stride(0) : K, w.data_ptr(), yp, ldy, (int)M, (int)N, (int)K, (int)nt, (int)vs, (int)splits, (int)epi, pp, cp,
-                rp, ldr, so, so_ld, (float)scale, (float)eps, pos_p, cs, sl, qo, kp, vp, vr, v_ld, (int)nq, (int)nkv, (int)d, stream()),
+                rp, ldr, so, so_ld, (float)scale, (float)eps, pos_p, cs, sl, qo, kp, vp, vr, v_ld, (int)nq, (int)nkv, (int)d, bp, (int)mode,
+                (float)limit, (float)alpha, stream()),
      "dgemm");
   return epi == 1 ? tiles : 0;
 }

@@ -18,11 +18,12 @@
 // scale, RoPE, q and paged K / V writes); SWIGLU (row scale, silu(g) u).  What an epilogue reads (residual, positions, slots, cos /
 // sin) is loaded at the kernel's start.  The row scale of a folded RMSNorm needs no partial sums from the producer: every wave has
 // all of its K range of X in fragments, and X . X^T's diagonal, one more MFMA per fragment, is the rows' sums of squares.
-// QKV and SWIGLU weights are stored with the halves of a pair 8 columns apart in one tile (frag_weight(paired = True)).
+// GLU and GELU are the activations of layer-list feed-forwards, on the rounded product as their own launches do them (a launch of its
+// own: 3.4 us and the gap before it).  QKV, SWIGLU and GLU weights are stored with the halves of a pair 8 columns apart in one tile (frag_weight).
 #include "common.h"
 
 namespace {
-enum { DG_PLAIN = 0, DG_RESADD = 1, DG_QKV = 2, DG_SWIGLU = 3 };
+enum { DG_PLAIN = 0, DG_RESADD = 1, DG_QKV = 2, DG_SWIGLU = 3, DG_GLU = 4, DG_GELU = 5 };
 
 struct DgArgs {
   const u16* X;
@@ -47,6 +48,9 @@ struct DgArgs {
   u16* v_rows;        // V row-major [M, v_ld] instead of the V^T cache
   long v_ld;
   int nq, nkv, d;
+  const float* bias;  // GLU: over the gate columns, then the up columns (null: none)
+  int mode;           // GLU: 0 silu, 1 clamped, 2 tanh GELU (glu_act of seqmix.hip)
+  float limit, alpha;
 };
 
 __device__ __forceinline__ uint4 ldb16(__amdgpu_buffer_rsrc_t r, unsigned off) {
@@ -56,23 +60,23 @@ __device__ __forceinline__ uint4 ldb16(__amdgpu_buffer_rsrc_t r, unsigned off) {
 template <int MT, int NT, int VS, int EPI>
 struct Dg {
   static constexpr int WV = 4 * VS, T = 64 * WV, NC = 16 * NT, MR = 16 * MT, LD = NC + 4;
-  static constexpr bool XL = MT >= 2, PAIR = EPI == DG_QKV || EPI == DG_SWIGLU;
+  static constexpr bool XL = MT >= 2, SQ = EPI == DG_QKV || EPI == DG_SWIGLU, PAIR = SQ || EPI == DG_GLU;
   // k-steps of 32 in flight per stage (two stages): registers of 16 waves, or of many fragments, hold two
   static constexpr int U = VS == 4 || NT + MT > 4 ? 2 : 4;
   static constexpr int PX = 64 * U + 16;      // bytes of a staged row
   static constexpr int REG = (XL && MR * PX > MR * LD * 4) ? MR * PX : MR * LD * 4;   // a wave's piece of LDS
   static constexpr int ITEMS = MR * NC / (PAIR ? 8 : 4), NI = (ITEMS + T - 1) / T;
-  static constexpr int LDS = WV * REG + (PAIR ? WV * MR * 4 : MR * (NC / 4) * 4) + 16;
+  static constexpr int LDS = WV * REG + (SQ ? WV * MR * 4 : MR * (NC / 4) * 4) + 16;
 };
 
 template <int MT, int NT, int VS, int EPI>
 __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   using C = Dg<MT, NT, VS, EPI>;
   constexpr int NC = C::NC, MR = C::MR, LD = C::LD, U = C::U, WV = C::WV, T = C::T, NI = C::NI, PX = C::PX;
-  constexpr bool XL = C::XL, PAIR = C::PAIR;
+  constexpr bool XL = C::XL, PAIR = C::PAIR, SQ = C::SQ;
   extern __shared__ __attribute__((aligned(16))) unsigned char dg_smem[];
   float* s_tail = reinterpret_cast<float*>(dg_smem + WV * C::REG);      // row sums: [WV][MR] of X, or [MR][NC / 4] of the result
-  int* s_last = reinterpret_cast<int*>(s_tail + (PAIR ? WV * MR : MR * (NC / 4)));
+  int* s_last = reinterpret_cast<int*>(s_tail + (SQ ? WV * MR : MR * (NC / 4)));
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wv = wave & 3, grp = wave >> 2;
   const int g = lane >> 4, r16 = lane & 15;
   const int tile = blockIdx.x, split = blockIdx.y * VS + grp, col0 = tile * NC;
@@ -94,12 +98,22 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     }
   }
 
-  f32x4 acc[MT][NT], sq[PAIR ? MT : 1];
+  f32x4 e_bg[EPI == DG_GLU ? NI : 1], e_bu[EPI == DG_GLU ? NI : 1];
+  if constexpr (EPI == DG_GLU) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int q = (threadIdx.x + i * T) % IPR, c = min(8 * (tile * NT + q / 2) + 4 * (q & 1), N / 2 - 4);
+      e_bg[i] = a.bias ? *reinterpret_cast<const f32x4*>(a.bias + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+      e_bu[i] = a.bias ? *reinterpret_cast<const f32x4*>(a.bias + N / 2 + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+
+  f32x4 acc[MT][NT], sq[SQ ? MT : 1];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (PAIR) sq[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (SQ) sq[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int nt16 = (N + 15) >> 4;
   const u16* wt[NT];      // wave-uniform: the lane's 16 bytes are a 32-bit offset of the load
@@ -146,7 +160,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
           else xf = __builtin_bit_cast(bf16x8, st.x[u]);
 #pragma unroll
           for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, st.w[u][n], acc[m][n], 0, 0, 0);
-          if constexpr (PAIR) sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, xf, sq[m], 0, 0, 0);
+          if constexpr (SQ) sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, xf, sq[m], 0, 0, 0);
         }
       }
   };
@@ -190,7 +204,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     for (int n = 0; n < NT; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) pt[(16 * m + 4 * g + r) * LD + 16 * n + r16] = acc[m][n][r];
-    if constexpr (PAIR) {
+    if constexpr (SQ) {
       const float dg = r16 & 2 ? (r16 & 1 ? sq[m][3] : sq[m][2]) : (r16 & 1 ? sq[m][1] : sq[m][0]);
       if ((r16 >> 2) == g) s_tail[wave * MR + 16 * m + r16] = dg;
     }
@@ -217,10 +231,10 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     return s;
   };
   f32x4 x1[NI], x2[PAIR ? NI : 1];
-  float rs[PAIR ? NI : 1];
+  float rs[SQ ? NI : 1];
   if (gridDim.y > 1) {
     // write-through slabs, one a split (results, then the rows' sums), ticket; the last arriver adds them in split order
-    constexpr int slab = MR * NC + (PAIR ? MR : 0);
+    constexpr int slab = MR * NC + (SQ ? MR : 0);
     const int S = gridDim.y * VS;
     const __amdgpu_buffer_rsrc_t pr = make_rsrc(a.part, (unsigned)min((long)gridDim.x * S * slab * 4, 0x7fffffffL));
     auto slab_at = [&](int sp) { return (unsigned)(((long)sp * gridDim.x + tile) * slab * 4); };
@@ -231,7 +245,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
         const f32x4 v = group_part(gr, e / NC, e % NC);
         st_wt16(pr, my + e * 4, make_float4(v[0], v[1], v[2], v[3]));
       }
-      if constexpr (PAIR)
+      if constexpr (SQ)
         if (threadIdx.x < MR / 4) {
           const int m = threadIdx.x * 4;
           st_wt16(pr, my + (MR * NC + m) * 4, make_float4(row_sum(4 * gr, 4, m), row_sum(4 * gr, 4, m + 1), row_sum(4 * gr, 4, m + 2), row_sum(4 * gr, 4, m + 3)));
@@ -247,7 +261,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
       }
       return v;
     };
-    if constexpr (PAIR) {
+    if constexpr (SQ) {
       if (threadIdx.x < MR / 4) *reinterpret_cast<f32x4*>(s_tail + threadIdx.x * 4) = all_slabs(MR * NC + threadIdx.x * 4);
     }
 #pragma unroll
@@ -259,7 +273,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
         x2[i] = all_slabs(row * NC + q / 2 * 16 + 8 + 4 * (q & 1));
       } else x1[i] = all_slabs(row * NC + 4 * q);
     }
-    if constexpr (PAIR) {
+    if constexpr (SQ) {
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < NI; ++i) rs[i] = s_tail[min((int)(threadIdx.x + i * T) / IPR, MR - 1)];
@@ -272,7 +286,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
       if constexpr (PAIR) {
         x1[i] = group_sum(row, q / 2 * 16 + 4 * (q & 1));
         x2[i] = group_sum(row, q / 2 * 16 + 8 + 4 * (q & 1));
-        rs[i] = row_sum(0, WV, row);
+        if constexpr (SQ) rs[i] = row_sum(0, WV, row);
       } else x1[i] = group_sum(row, 4 * q);
     }
     if constexpr (EPI == DG_RESADD) __syncthreads();
@@ -283,10 +297,16 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     const int it = threadIdx.x + i * T, m = it / IPR, q = it % IPR;
     if (m >= M) continue;
     u16x4 o;
-    if constexpr (EPI == DG_PLAIN) {
+    if constexpr (EPI == DG_PLAIN || EPI == DG_GELU) {
       const int c = col0 + 4 * q;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o.v[j] = f2bf(x1[i][j]);
+      for (int j = 0; j < 4; ++j) {
+        o.v[j] = f2bf(x1[i][j]);
+        if constexpr (EPI == DG_GELU) {
+          const float v = bf2f(o.v[j]);
+          o.v[j] = f2bf(0.5f * v * (1.f + erff(v * 0.70710678118654752f)));
+        }
+      }
       u16* y = a.Y + (long)m * a.ldy + c;
       if (c + 4 <= N && (a.ldy & 3) == 0) *reinterpret_cast<u16x4*>(y) = o;
       else
@@ -304,6 +324,23 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
       }
       if (c < N) *reinterpret_cast<u16x4*>(a.res + (long)m * a.ldr + c) = o;
       s_tail[m * (NC / 4) + q] = c < N ? ss : 0.f;
+    } else if constexpr (EPI == DG_GLU) {
+      // the product's rounding, then glu_act's steps (seqmix.hip) on it
+      const int c = 8 * (tile * NT + q / 2) + 4 * (q & 1);
+      if (2 * c >= N) continue;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float g = bf2f(f2bf(x1[i][j])) + e_bg[i][j], u = bf2f(f2bf(x2[i][j])) + e_bu[i][j], al = 1.f;
+        if (a.mode == 1) {
+          g = fminf(g, a.limit);
+          u = fminf(fmaxf(u, -a.limit), a.limit) + 1.f;
+          al = a.alpha;
+        } else if (a.mode == 2) {
+          al = 1.5957691216057308f * (1.f + 0.044715f * g * g);
+        }
+        o.v[j] = f2bf(g * __builtin_amdgcn_rcpf(1.f + __expf(-al * g)) * u);
+      }
+      *reinterpret_cast<u16x4*>(a.Y + (long)m * a.ldy + c) = o;
     } else {
       const float ri = rsqrtf(rs[i] * a.scale + a.eps);
       const int t16 = tile * NT + q / 2, h8 = 8 * (t16 & 1) + 4 * (q & 1), cb = (t16 >> 1) * 32;
@@ -387,7 +424,7 @@ int by_shape(const DgArgs& a, int nt, int vs, int gy, hipStream_t st) {
     if (nt == 2) return launch<MT, 2, 2, EPI>(a, gy, st);
     if (nt == 3) return launch<MT, 3, 2, EPI>(a, gy, st);
   } else if (vs == 4) {
-    if constexpr (MT <= 2 && EPI == DG_PLAIN)
+    if constexpr (MT <= 2 && (EPI == DG_PLAIN || EPI >= DG_GLU))
       if (nt == 1) return launch<MT, 1, 4, EPI>(a, gy, st);
   }
   return -10;
@@ -408,14 +445,15 @@ int by_rows(const DgArgs& a, int nt, int vs, int gy, hipStream_t st) {
 extern "C" int dllm_dgemm(const void* X, long ldx, const void* W, void* Y, long ldy, int M, int N, int K, int nt, int vs, int splits,
                           int epi, float* part, int* counters, void* res, long ldr, float* ssq_out, long ssq_ld, float scale, float eps,
                           const int* pos, const float* cos_sin, const int* slots, void* q_out, void* kc, void* vc, void* v_rows,
-                          long v_ld, int nq, int nkv, int d, hipStream_t stream) {
+                          long v_ld, int nq, int nkv, int d, const float* bias, int mode, float limit, float alpha, hipStream_t stream) {
   if (M < 1 || M > 64 || ldx < K || ldx > (1 << 24) || N < 1 || K < 32 || K % 32 || splits < 1 || nt < 1 || vs < 1) return -1;
   int kchunk = (K + splits - 1) / splits;
   kchunk = (kchunk + 31) & ~31;
   const int S = (K + kchunk - 1) / kchunk, gy = (S + vs - 1) / vs;
   if (gy > 1 && (!part || !counters)) return -2;
   const DgArgs a{(const u16*)X, ldx, (const u16*)W, (u16*)Y, ldy, M, N, K, kchunk, S, part, counters, (u16*)res, ldr, ssq_out, ssq_ld,
-                 scale, eps, pos, cos_sin, slots, (u16*)q_out, (u16*)kc, (u16*)vc, (u16*)v_rows, v_ld, nq, nkv, d};
+                 scale, eps, pos, cos_sin, slots, (u16*)q_out, (u16*)kc, (u16*)vc, (u16*)v_rows, v_ld, nq, nkv, d,
+                 bias, mode, limit, alpha};
   switch (epi) {
     case DG_PLAIN: return Y ? by_rows<DG_PLAIN>(a, nt, vs, gy, stream) : -3;
     case DG_RESADD: return res && ssq_out && N % 4 == 0 && ldr % 4 == 0 ? by_rows<DG_RESADD>(a, nt, vs, gy, stream) : -4;
@@ -423,6 +461,8 @@ extern "C" int dllm_dgemm(const void* X, long ldx, const void* W, void* Y, long 
       if (d < 32 || d % 32 || N != (nq + 2 * nkv) * d || !q_out || !kc || !vc || !pos || !cos_sin || !slots || (v_rows && v_ld % 4)) return -5;
       return by_rows<DG_QKV>(a, nt, vs, gy, stream);
     case DG_SWIGLU: return Y && N % 32 == 0 && ldy % 4 == 0 ? by_rows<DG_SWIGLU>(a, nt, vs, gy, stream) : -6;
+    case DG_GLU: return Y && N % 16 == 0 && ldy % 4 == 0 && mode >= 0 && mode <= 2 ? by_rows<DG_GLU>(a, nt, vs, gy, stream) : -8;
+    case DG_GELU: return Y ? by_rows<DG_GELU>(a, nt, vs, gy, stream) : -3;
     default: return -7;
   }
 }

@@ -530,8 +530,9 @@ class HybridModel:
     @property
     def order_kept(self) -> bool:
         """Small products keep the order of their sums: an mLSTM head divides by sums of a few thousandths of their terms, and a last
-        bit ahead of it becomes tenths of a logit."""
-        return any(m.kind == "mlstm" for L in self.cfg.layers for m in L.mixer.parts)
+        bit ahead of it becomes tenths of a logit.  Behind a norm ahead of every sublayer it does not: another order moves Figotar's
+        logits by 0.004 and leaves them as far from 64 bits (0.0116, five batches) as they were."""
+        return not self.cfg.pre_norm and any(m.kind == "mlstm" for L in self.cfg.layers for m in L.mixer.parts)
 
     def _place_fragments(self) -> None:
         """Fragment-major copies of the projections and the head for the decode GEMM (ops.gemm.frag_weight), while they fit in a
@@ -544,9 +545,16 @@ class HybridModel:
         extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
         if extra > 0.25 * torch.cuda.mem_get_info(self.device)[0]:
             return
+        for L, S in zip(self.layers, self.cfg.layers):
+            f = S.mlp
+            act = self._act_args(f) if isinstance(f, DenseSpec) and not self.cfg.parallel_ff else None
+            # an up projection with its activation: that copy alone (its plain product runs where no decode GEMM does)
+            if act is not None and any(l is L and n == "up" for l, n in todo) and (act[0] == "gelu" or f.ff % 8 == 0):
+                L["up_act_r"], L["order_kept"] = ops.gemm.frag_weight(L["up"], paired=False if act[0] == "gelu" else "glu"), self.order_kept
         for L, n in todo:
-            L[n + "_r"] = ops.gemm.frag_weight(L[n])
-            L["order_kept"] = self.order_kept
+            if n != "up" or "up_act_r" not in L:
+                L[n + "_r"] = ops.gemm.frag_weight(L[n])
+                L["order_kept"] = self.order_kept
         ex = [(L, S.mlp) for L, S in zip(self.layers, self.cfg.layers)
               if isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
               and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
@@ -1008,14 +1016,22 @@ class HybridModel:
                          meta.qstart, meta.qlen, meta.ctx, meta.state_rows)
         return _pm(o, L, "o")
 
+    # an activation that the decode GEMM ends in: (ops.gemm.linear_act's name, limit, alpha); a down projection's bias rides in the
+    # residual launch
+    @staticmethod
+    def _act_args(f) -> tuple:
+        return {"clamped_glu": ("clamped", f.limit, 1.702), "gelu_glu": ("gelu_tanh", 0.0, 1.0), "polynorm": None}.get(f.act, ("gelu", 0.0, 1.0))
+
     def _dense(self, L, f: DenseSpec, x):
-        z = _pm(x, L, "up")
-        if f.act == "clamped_glu":      # the down projection's bias rides in the residual launch
-            a = seqmix.glu_act(z, L.get("up_b"), "clamped", f.limit, 1.702)
-        elif f.act == "gelu_glu":       # likewise
-            a = seqmix.glu_act(z, L.get("up_b"), "gelu_tanh")
-        else:
-            a = seqmix.polynorm(z, L["act"], self.cfg.rms_eps) if f.act == "polynorm" else seqmix.gelu_erf(z)
+        act, a = self._act_args(f), None
+        if "up_act_r" in L:
+            a = ops.gemm.linear_act(x, L["up"], L["up_act_r"], act[0], L.get("up_b"), act[1], act[2], L["order_kept"])
+        if a is None:
+            z = _pm(x, L, "up")
+            if act is None:
+                a = seqmix.polynorm(z, L["act"], self.cfg.rms_eps)
+            else:
+                a = seqmix.gelu_erf(z) if act[0] == "gelu" else seqmix.glu_act(z, L.get("up_b"), *act)
         return _pm(a, L, "down")
 
     def _experts_swiglu(self, L, f: MoESpec, x, tail=None):

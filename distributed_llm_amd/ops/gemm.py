@@ -95,6 +95,7 @@ WS_FLOATS = 16 << 20      # 64 MiB of f32 split-K slabs per (device, owner)
 WS_COUNTERS = 1 << 16
 
 EPI_PLAIN, EPI_RESADD, EPI_QKV, EPI_SWIGLU, EPI_GELU = 0, 1, 2, 3, 4
+DG_GLU, DG_GELU = 4, 5      # of the decode GEMM alone
 
 # K-panel-major weight copies for the fused decoder GEMMs (GemmArgs.w_panel): every tgemm ring fill
 # of the weight operand is one contiguous 1 KB instead of eight 128-B row pieces 4-11 KB apart
@@ -115,10 +116,14 @@ DG_MAX_M = 64
 _PAIR_ROWS = [*range(8), *range(16, 24), *range(8, 16), *range(24, 32)]
 
 
-def frag_weight(w: torch.Tensor, paired: bool = False) -> torch.Tensor:
+def frag_weight(w: torch.Tensor, paired=False) -> torch.Tensor:
     """[N, K] -> [ceil(N / 16), K / 32, 64, 8]: of a 16-column tile and 32 k, lane 16 g + r holds W[16 t + r][32 s + 8 g ...+ 7]; rows past
-    N are zeros.  ``paired`` (the QKV and gate|up weights of models.llama, pairs 16 rows apart in groups of 32): pairs 8 rows apart."""
+    N are zeros.  ``paired`` (the QKV and gate|up weights of models.llama, pairs 16 rows apart in groups of 32): pairs 8 rows apart; "glu": gate rows, then up rows, likewise."""
     N, K = w.shape
+    if paired == "glu":
+        if K % 32 or N % 16:
+            raise ValueError(f"frag_weight: {N} x {K}")
+        return frag_weight(w.view(2, N // 16, 8, K).transpose(0, 1).reshape(N, K))
     if K % 32 or (paired and N % 32):
         raise ValueError(f"frag_weight: {N} x {K}")
     if paired:
@@ -536,7 +541,7 @@ def _key(x, w, swiglu):
 
 def dgemm(x: torch.Tensor, wf: torch.Tensor, n: int, epi: int, plan: Tuple[int, int, int], y=None, res=None, ssq_out=None,
           scale: float = 0.0, eps: float = 0.0, pos=None, cos_sin=None, slots=None, q_out=None, kc=None, vc=None, v_rows=None,
-          nq: int = 0, nkv: int = 0, d: int = 0) -> int:
+          nq: int = 0, nkv: int = 0, d: int = 0, bias=None, mode: int = 0, limit: float = 0.0, alpha: float = 1.0) -> int:
     """One launch of the decode GEMM on ``wf`` = frag_weight of an [n, K] weight; ``plan`` = (16-column tiles a workgroup, splits a
     workgroup, splits of K)."""
     nt, vs, splits = plan
@@ -547,13 +552,49 @@ def dgemm(x: torch.Tensor, wf: torch.Tensor, n: int, epi: int, plan: Tuple[int, 
     if gy > 1:
         part, cnt = _P.workspace(x.device, gy * vs * tiles * -(-M // 16) * 16 * (16 * nt + 1), tiles)
     return int(_native(x).dgemm(x, wf, n, int(epi), nt, vs, splits, y, part, cnt, res, ssq_out, float(scale), float(eps), pos, cos_sin,
-                                slots, q_out, kc, vc, v_rows, int(nq), int(nkv), int(d)))
+                                slots, q_out, kc, vc, v_rows, int(nq), int(nkv), int(d), bias, int(mode), float(limit), float(alpha)))
 
 
 def dg_takes(x: torch.Tensor) -> bool:
     """The decode GEMM reads these rows: up to 64, 16-byte aligned."""
     return 0 < x.shape[0] <= DG_MAX_M and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
         (x.shape[0] == 1 or x.stride(0) >= x.shape[1]) and x.data_ptr() % 16 == 0
+
+
+def _linear_plan(x: torch.Tensor, w: torch.Tensor, frag: bool, keep_order: bool):
+    """(plan on the row-major weight, splits a workgroup, decode GEMM's plan or None) of ``linear``."""
+    M, (N, K) = x.shape[0], w.shape
+    plan, together = _P.plans.get(_key(x, w, False)), 1
+    dg = _P.dg_plans.get((M, N, K)) if frag and not keep_order else None
+    timed = plan is not None
+    if not timed:
+        plan = _heuristic(M, N, K) if M <= MAX_M else ("blas",)
+    if plan[0] == "skinny" and (frag or not timed):
+        same = ("skinny", min(plan[1], 2), plan[2])
+        together = _splits_together(M, N, K, same)
+        if frag and dg is None:
+            dg = (same[1], together, same[2])
+        together = 1 if timed else together
+    return plan, together, dg
+
+
+def linear_act(x: torch.Tensor, w: torch.Tensor, wf: torch.Tensor, act: str, bias: Optional[torch.Tensor] = None, limit: float = 0.0,
+               alpha: float = 1.0, keep_order: bool = False) -> Optional[torch.Tensor]:
+    """``seqmix.gelu_erf(linear(x, w))`` (act "gelu") or ``seqmix.glu_act(linear(x, w), bias, act, limit, alpha)`` in the launch of the
+    decode GEMM, where it takes the product; else None.  ``wf``: frag_weight(w), paired = "glu" for the gated ones."""
+    if not dg_takes(x) or os.environ.get("DLLM_GEMM") == "blas":
+        return None
+    dg = _linear_plan(x, w, True, keep_order)[2]
+    if dg is None:
+        return None
+    N = w.shape[0]
+    y = torch.empty((x.shape[0], N if act == "gelu" else N // 2), dtype=x.dtype, device=x.device)
+    if act == "gelu":
+        dgemm(x, wf, N, DG_GELU, dg, y=y)
+    else:
+        from .seqmix import GLU_MODES
+        dgemm(x, wf, N, DG_GLU, dg, y=y, bias=bias, mode=GLU_MODES[act], limit=limit, alpha=alpha)
+    return y
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -563,21 +604,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
     timed ones where it was faster, or with ``keep_order`` where the plan is a skinny one, whose sums it keeps."""
     if not x.is_cuda or os.environ.get("DLLM_GEMM") == "blas":
         return F.linear(x, w) if out is None else torch.matmul(x, w.t(), out=out)
-    M, (N, K) = x.shape[0], w.shape
-    plan, together = _P.plans.get(_key(x, w, False)), 1
-    dg = _P.dg_plans.get((M, N, K)) if wf is not None and not keep_order else None
-    timed = plan is not None
-    if not timed:
-        plan = _heuristic(M, N, K) if M <= MAX_M else ("blas",)
-    if plan[0] == "skinny" and (wf is not None or not timed):
-        same = ("skinny", min(plan[1], 2), plan[2])
-        together = _splits_together(M, N, K, same)
-        if wf is not None and dg is None:
-            dg = (same[1], together, same[2])
-        together = 1 if timed else together
+    plan, together, dg = _linear_plan(x, w, wf is not None, keep_order)
     if dg is not None and dg_takes(x):
-        y = out if out is not None else torch.empty((M, N), dtype=x.dtype, device=x.device)
-        dgemm(x, wf, N, EPI_PLAIN, dg, y=y)
+        y = out if out is not None else torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+        dgemm(x, wf, w.shape[0], EPI_PLAIN, dg, y=y)
         return y
     return _run_plan(plan, x, w, False, out, wp, together)
 

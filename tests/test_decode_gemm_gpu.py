@@ -133,3 +133,20 @@ def test_swiglu(M, plan, H, I):
     want = ref.silu_mul(gu).float()
     # each factor to 2^-6 of the largest (as test_qkv), the product of two
     torch.testing.assert_close(act.cpu().float(), want, atol=2.0 ** -6 * gu.float().abs().max().item() * 2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("M", [1, 4, 17, 48, 64])
+@pytest.mark.parametrize("act,limit,alpha,bias", [("gelu", 0.0, 1.0, False), ("swiglu", 0.0, 1.0, False), ("clamped", 1.5, 1.702, True),
+                                                  ("gelu_tanh", 0.0, 1.0, True), ("gelu_tanh", 0.0, 1.0, False)])
+@pytest.mark.parametrize("N,K", [(5632, 1024), (4096, 1024), (144, 96), (1024, 4096)])
+def test_activations(M, act, limit, alpha, bias, N, K):
+    """The activation in the product's launch: the bits of the two launches."""
+    from distributed_llm_amd.ops import seqmix
+    torch.manual_seed(M + N)
+    G.reserve(DEV)
+    x, w = _rnd(M, K), _rnd(N, K, scale=2 * K ** -0.5)
+    b = torch.randn(N, device=DEV) if bias else None
+    got = G.linear_act(x, w, G.frag_weight(w, paired=False if act == "gelu" else "glu"), act, b, limit, alpha)
+    z = G.linear(x, w, wf=G.frag_weight(w))
+    want = seqmix.gelu_erf(z) if act == "gelu" else seqmix.glu_act(z, b, act, limit, alpha)
+    assert torch.equal(got, want)
