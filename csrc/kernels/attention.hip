@@ -205,16 +205,16 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       float mloc = -INFINITY;
 #pragma unroll
       for (int j = 0; j < 8; ++j) mloc = fmaxf(mloc, p[j]);
-      mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-      mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+      mloc = lane_max(mloc, 16);
+      mloc = lane_max(mloc, 32);
       const float m_new = fmaxf(m_run, mloc);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
       const float alpha = exp2f(m_run - m_safe);
       float lsum = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) { p[j] = exp2f(p[j] - m_safe); lsum += p[j]; }
-      lsum += __shfl_xor(lsum, 16, 64);
-      lsum += __shfl_xor(lsum, 32, 64);
+      lsum = lane_add(lsum, 16);
+      lsum = lane_add(lsum, 32);
       l_run = l_run * alpha + lsum;
       m_run = m_new;
       const bf16x8 pf = __builtin_bit_cast(bf16x8, pack8(p));

@@ -291,10 +291,10 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ q
       sq += q[b][e] * q[b][e];
       sk += k[b][e] * k[b][e];
     }
-  sq += __shfl_xor(sq, 16);
-  sk += __shfl_xor(sk, 16);
-  sq += __shfl_xor(sq, 32);
-  sk += __shfl_xor(sk, 32);
+  sq = lane_add(sq, 16);
+  sk = lane_add(sk, 16);
+  sq = lane_add(sq, 32);
+  sk = lane_add(sk, 32);
   const float fq = (1.f / sqrtf((float)d)) / sqrtf(sq + 1e-6f), fk = 1.f / sqrtf(sk + 1e-6f);
   // k . k and q . k as sixteen sums of at most eight dims, added pairwise: a chain of d roundings would be the largest error of the rule
   const auto dots = [&](const f32x4(&a)[NB], const f32x4(&b)[NB]) {
@@ -511,8 +511,8 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
           lost = 4 * g4 + e;
           r[e] = 0.f;
         }
-      lost = min(lost, __shfl_xor(lost, 16));
-      lost = min(lost, __shfl_xor(lost, 32));
+      lost = min(lost, lane_xor(lost, 16));
+      lost = min(lost, lane_xor(lost, 32));
     }
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 u4[4];
@@ -609,7 +609,7 @@ __global__ void __launch_bounds__(256) delta_finish_kernel(const float* __restri
     for (int x = 0; x < W; ++x) ss += v[x] * v[x];
   }
 #pragma unroll
-  for (int x = LPR >> 1; x; x >>= 1) ss += __shfl_xor(ss, x);
+  for (int x = LPR >> 1; x; x >>= 1) ss = lane_add(ss, x);
   const float rs = 1.f / sqrtf(ss / (float)dv + eps);
   if (rr >= rows_total) return;
   for (int j = lane * W; j < dv; j += LPR * W) {

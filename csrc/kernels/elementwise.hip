@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1)
 #pragma unroll
-      for (int x = 0; x < EB; ++x) s[x] += __shfl_xor(s[x], m);
+      for (int x = 0; x < EB; ++x) s[x] = lane_add(s[x], m);
 #pragma unroll
     for (int x = 0; x < EB; ++x) lg = lane == e0 + x ? s[x] : lg;
   }
@@ -272,8 +272,8 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
     int bi = lane;
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) {
-      const float ov = __shfl_xor(best, m);
-      const int oi = __shfl_xor(bi, m);
+      const float ov = lane_xor(best, m);
+      const int oi = lane_xor(bi, m);
       if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
     }
     if (!(best > -INFINITY)) bi = 0;

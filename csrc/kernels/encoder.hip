@@ -91,15 +91,15 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
     float mloc = p[0];
 #pragma unroll
     for (int j = 1; j < 8; ++j) mloc = fmaxf(mloc, p[j]);
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = lane_max(mloc, 16);
+    mloc = lane_max(mloc, 32);
     const float m_new = fmaxf(m_run, mloc);  // finite: key kc < len is always valid
     const float alpha = exp2f(m_run - m_new);
     float lsum = 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) { p[j] = exp2f(p[j] - m_new); lsum += p[j]; }
-    lsum += __shfl_xor(lsum, 16, 64);
-    lsum += __shfl_xor(lsum, 32, 64);
+    lsum = lane_add(lsum, 16);
+    lsum = lane_add(lsum, 32);
     l_run = l_run * alpha + lsum;
     m_run = m_new;
     const bf16x8 pf = __builtin_bit_cast(bf16x8, pack8(p));

@@ -270,7 +270,7 @@ __global__ void __launch_bounds__(512, MINW) flash_prefill_kernel(FlashArgs a) {
     for (int i = 1; i < 16; ++i) mloc = fmaxf(mloc, sc[0][i]);
 #pragma unroll
     for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[1][i]);
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+    mloc = lane_max(mloc, 32);
     const float m_new = fmaxf(m_run, mloc);
     if constexpr (PIPE) {  // P.V of the previous chunk (never the context's tail), previous max frame
       pv_chunk<D, NB, false>(acc, vprev, pf_prev, 0, 0, rl, h);
@@ -314,7 +314,7 @@ __global__ void __launch_bounds__(512, MINW) flash_prefill_kernel(FlashArgs a) {
   }
 
   // acc[n][i] = O^T[dim 32 n + 8 (i >> 2) + 4 h + (i & 3)][row rl]
-  float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  float l_tot = lane_add(l_run, 32);
   if (SPLIT && n_split > 1) {
     // split-KV: publish this split's unnormalised O and (m, l) write-through, take the ticket
     const long unit = (long)(tile * a.nkv + kvh);

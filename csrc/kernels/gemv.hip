@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
         for (int j = 0; j < 8; ++j) ss[m] += a[j] * a[j];
       }
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) ss[m] += __shfl_xor(ss[m], o, 64);
+      for (int o = 32; o >= 1; o >>= 1) ss[m] = lane_add(ss[m], o);
       if (lane == 0) red[wave * M + m] = ss[m];
     }
     __syncthreads();
@@ -268,7 +268,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
     for (int r = 0; r < R; ++r) {
       float v = acc[m][r];
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+      for (int o = 32; o >= 1; o >>= 1) v = lane_add(v, o);
       acc[m][r] = v;
     }
   if constexpr (EPI == GV_PLAIN) {
@@ -356,7 +356,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
   if constexpr (EPI == GV_RESADD) {
     // this workgroup's partial row sums of r^2 over all its blocks: one slot per workgroup
 #pragma unroll
-    for (int o = 1; o < R; o <<= 1) v2sum += __shfl_xor(v2sum, o, 64);  // the R lanes of a row (aligned groups)
+    for (int o = 1; o < R; o <<= 1) v2sum = lane_add(v2sum, o);  // the R lanes of a row (aligned groups)
     if (lane < M * R && lane % R == 0) s_red[wave * M + lane / R] = v2sum;  // inactive waves store zeros
     __syncthreads();
     if (threadIdx.x < M) {

@@ -580,8 +580,8 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
       else if (slopes) sc[x] -= slp * (float)(rpos - pk);
       if (vis[x]) mn = fmaxf(mn, sc[x]);
     }
-    mn = fmaxf(mn, __shfl_xor(mn, 16));
-    mn = fmaxf(mn, __shfl_xor(mn, 32));
+    mn = lane_max(mn, 16);
+    mn = lane_max(mn, 32);
     const float f = mn > -INFINITY ? expf(m - mn) : 1.f;   // before the first visible key: O and l are 0
     f32x4 p;
     l *= f;
@@ -605,8 +605,8 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
     }
     k0 = k1;
   }
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = lane_add(l, 16);
+  l = lane_add(l, 32);
   if (g4 == 0) {
     ml[w][0][lr] = m;
     ml[w][1][lr] = l;

@@ -95,7 +95,7 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float u = ACT == 0 ? __shfl_xor(acc[m][r], 8, 64) : 0.f;
+      const float u = ACT == 0 ? lane_xor(acc[m][r], 8) : 0.f;
       if (ACT != 0 || r16 < 8) put(row0 + 16 * m + 4 * g + r, r16, acc[m][r], u);
     }
 }

@@ -46,8 +46,8 @@ __global__ void __launch_bounds__(256) argmax_kernel(const void* __restrict__ lo
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    float ov = __shfl_xor(bv, o, 64);
-    int oi = __shfl_xor(bi, o, 64);
+    float ov = lane_xor(bv, o);
+    int oi = lane_xor(bi, o);
     better(bv, bi, ov, oi);
   }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -442,7 +442,7 @@ static __device__ __forceinline__ int draw_rank(const SrShared& sh, int kk, floa
     if (r < kk && pre + c4[q] >= tp) cut = min(cut, r + 1);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) cut = min(cut, __shfl_xor(cut, o, 64));
+  for (int o = 32; o > 0; o >>= 1) cut = min(cut, lane_xor(cut, o));
   const int last = cut - 1;
   const float mass = __shfl(pre + c4[last & 3], last >> 2, 64);
   const float target = row_uniform(seed, row) * mass;
@@ -453,7 +453,7 @@ static __device__ __forceinline__ int draw_rank(const SrShared& sh, int kk, floa
     if (r < cut && pre + c4[q] > target) pick = min(pick, r);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) pick = min(pick, __shfl_xor(pick, o, 64));
+  for (int o = 32; o > 0; o >>= 1) pick = min(pick, lane_xor(pick, o));
   return pick;
 }
 
@@ -481,8 +481,8 @@ __global__ void __launch_bounds__(SR_THREADS) sample_rows_kernel(const u16* __re
     for (int i = (nv << 3) + tid; i < V; i += SR_THREADS) better(bv, bi, bf2f(l[i]), i);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
+      const float ov = lane_xor(bv, o);
+      const int oi = lane_xor(bi, o);
       better(bv, bi, ov, oi);
     }
     if (lane == 0) { sh.sv[wid] = bv; sh.si[wid] = bi; }
@@ -625,8 +625,8 @@ __global__ void __launch_bounds__(SR_THREADS) sample_split_kernel(const u16* __r
     for (int i = (nv << 3) + tid; i < len; i += SR_THREADS) better(bv, bi, bf2f(l[i]), start + i);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
+      const float ov = lane_xor(bv, o);
+      const int oi = lane_xor(bi, o);
       better(bv, bi, ov, oi);
     }
     if (lane == 0) { sh.sv[wid] = bv; sh.si[wid] = bi; }

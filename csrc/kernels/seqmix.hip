@@ -1112,8 +1112,8 @@ __global__ void __launch_bounds__(256) polynorm_kernel(const T* __restrict__ z, 
 __device__ __forceinline__ void wave_argmax(float& v, int& idx) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, 64);
-    const int oi = __shfl_xor(idx, o, 64);
+    const float ov = lane_xor(v, o);
+    const int oi = lane_xor(idx, o);
     if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
   }
 }

@@ -650,7 +650,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
 #pragma unroll
             for (int j = 0; j < FN32; ++j) {
               const float xs = bfr(acc32[i][j][v] * ri);
-              const float xp = __shfl_xor(xs, 16, 64);
+              const float xp = lane_xor(xs, 16);
               if (!hi) so[rl * OLD + (wn * WN + 32 * j) / 2 + c16] = f2bf(silu(xs) * xp);
             }
           } else {
@@ -807,7 +807,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
         st16(yp, pack8(r));
       }
 #pragma unroll
-      for (int o = 1; o < CPR; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      for (int o = 1; o < CPR; o <<= 1) ss = lane_add(ss, o);
       if (a.ssq_out != nullptr && threadIdx.x % CPR == 0 && m < M) a.ssq_out[(long)n_tile * a.ssq_out_ld + m] = ss;
     }
   } else {
