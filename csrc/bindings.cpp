@@ -151,6 +151,9 @@ int dllm_moe_ffn_tg(const void*, long, long, int, const int*, const float*, int,
 int dllm_moe_slice(int, int);
 int dllm_moe_tail_ok(int, int);
 int dllm_enc_gemm_ok(int, int, int);
+int dllm_enc_few_ok(int, int, int, int, int);
+int dllm_enc_few_layer(void*, void*, void*, void*, void*, const void* const*, const void*, const void*, int, int, int, int, float, float,
+                       const int*, const int*, int, int, hipStream_t);
 int dllm_enc_gemm(const void*, long, const void*, const void*, void*, long, int, int, int, int, hipStream_t);
 int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, const int*, int, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
@@ -1530,7 +1533,7 @@ bool enc_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor bias, torch::Tenso
   return true;
 }
 
-// All layers of the sentence encoder over packed rows, in one call: seven launches a layer back to back instead of seven calls
+// All layers of the sentence encoder over packed rows, in one call: seven launches a layer (four at up to 16 rows) back to back instead of seven calls
 // from the interpreter, whose 6 us each were most of a single text's 335 us.  weights: per layer QKV w, b, output w, b, norm w, b,
 // up w, b, down w, b, norm w, b.  plans (QKV, output, up, down): bm, bn, stages, splits, ks, waves, k-groups, loaders, k depth, mfma,
 // raster.  x [T, H] is overwritten; returns the last layer's rows.
@@ -1547,6 +1550,33 @@ torch::Tensor encoder_layers(torch::Tensor x, torch::Tensor lens, torch::Tensor 
   auto qkv = torch::empty({T, 3 * H}, x.options()), a = torch::empty({T, H}, x.options()), f = torch::empty({T, I}, x.options()),
        y = torch::empty({T, H}, x.options());
   const c10::optional<torch::Tensor> none;
+  const double scale = 1.0 / std::sqrt((double)d);
+  // up to 16 rows: four launches a layer (encoder.hip), if every weight is as those kernels read it
+  bool few = T <= 16 && dllm_enc_few_ok((int)T, (int)nh, (int)d, (int)I, (int)B) && S >= 1 && starts.numel() >= B && lens.is_contiguous() &&
+             starts.is_contiguous() && lens.scalar_type() == torch::kInt32 && starts.scalar_type() == torch::kInt32 && lens.is_cuda() &&
+             starts.is_cuda() && ((uintptr_t)x.data_ptr() & 15) == 0;
+  const int64_t rows[12] = {3 * H, 3 * H, H, H, H, H, I, I, H, H, H, H};
+  for (size_t i = 0; few && i < weights.size(); ++i) {
+    const auto& w = weights[i];
+    const int64_t k = i % 12, c = k == 0 || k == 2 || k == 6 ? H : k == 8 ? I : 0;
+    few = w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.is_contiguous() && ((uintptr_t)w.data_ptr() & 15) == 0 &&
+          (c ? w.dim() == 2 && w.size(0) == rows[k] && w.size(1) == c : w.numel() == rows[k]);
+  }
+  if (few) {
+    auto vt = torch::empty({H, 16}, x.options());
+    const void *ln_w = nullptr, *ln_b = nullptr;
+    for (size_t l = 0; l < weights.size(); l += 12) {
+      const void* w[10];
+      for (int i = 0; i < 10; ++i) w[i] = weights[l + i].data_ptr();
+      ok(dllm_enc_few_layer(x.data_ptr(), y.data_ptr(), qkv.data_ptr(), vt.data_ptr(), f.data_ptr(), w, ln_w, ln_b, (int)T, (int)nh, (int)d,
+                            (int)I, (float)eps, (float)scale, starts.data_ptr<int>(), lens.data_ptr<int>(), (int)B, (int)S, stream()),
+         "encoder layer");
+      ln_w = weights[l + 10].data_ptr();
+      ln_b = weights[l + 11].data_ptr();
+    }
+    norm(y, none, weights[weights.size() - 2], weights.back(), x, eps, true);
+    return x;
+  }
   auto gemm = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& b, const torch::Tensor& out, int epi,
                   const std::vector<int64_t>& p) {
     if (!enc_gemm(in, w, b, out, epi)) tgemm(in, w, out, epi, p[0], p[1], p[2], p[3], p[4], p[5], part, counters, none, 0, 0.0, 0.0, none, none, none, none, none, none,
@@ -1555,7 +1585,7 @@ torch::Tensor encoder_layers(torch::Tensor x, torch::Tensor lens, torch::Tensor 
   for (size_t l = 0; l < weights.size(); l += 12) {
     const torch::Tensor* w = &weights[l];
     gemm(x, w[0], w[1], qkv, 0, plans[0]);
-    encoder_attention(qkv, lens, a, B, S, nh, d, 1.0 / std::sqrt((double)d), starts);
+    encoder_attention(qkv, lens, a, B, S, nh, d, scale, starts);
     gemm(a, w[2], w[3], x, 1, plans[1]);
     norm(x, none, w[4], w[5], y, eps, true);
     gemm(y, w[6], w[7], f, 4, plans[2]);

@@ -1,6 +1,7 @@
 // Router sentence encoder (MiniLM / BERT) kernels: bidirectional attention over a padded or packed batch
 // the fused embedding sum + LayerNorm, and the projections of up to 64 rows (enc_gemm; more rows run on tgemm.hip, with
-// the same bias / GELU / residual epilogues).  LayerNorm after each residual is in norm.hip, pooling in elementwise.hip.
+// the same bias / GELU / residual epilogues) and whole layers of up to 16 (enc_rows, attn_out; LayerNorm after each residual of more
+// rows is in norm.hip), pooling in elementwise.hip.
 //
 // Reference parity: the reference encodes every query with sentence-transformers
 // all-MiniLM-L6-v2 on the host (src/query_router_engine.py:181,571).
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
 // rows come straight to registers (a weight is used by one workgroup, the rows are a few KB in L2).  Bound by one load's latency,
 // the launch and the exchange; the LDS-tiled GEMM adds a ring's fill and, for long K, a split's exchange through memory: 16 rows,
 // 384 -> 1152 / 384 -> 384 / 384 -> 1536 / 1536 -> 384 columns 2.9 / 3.5 / 3.5 / 5.4 us against 5.4 / 5.6 / 7.7 / 9.4.
-enum { ENC_PLAIN = 0, ENC_RESADD = 1, ENC_GELU = 4 };
+enum { ENC_PLAIN = 0, ENC_RESADD = 1, ENC_QKV = 2, ENC_GELU = 4 };
 template <int MT, int NW, int EPI>
 __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict__ X, long ldx, const u16* __restrict__ W,
                                                            const u16* __restrict__ bias, u16* __restrict__ Y, long ldy, int M, int N,
@@ -191,6 +192,173 @@ int launch_enc_gemm(const u16* x, long ldx, const u16* w, const u16* bias, u16* 
   else if (epi == ENC_GELU) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_GELU>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
   else return -1;
   return (int)hipGetLastError();
+}
+
+// ---- whole layers of up to 16 rows (H <= 384) in four launches instead of seven: [LayerNorm +] QKV, attention + output + residual,
+// LayerNorm + up + GELU, down + residual (enc_gemm).  A launch of this size costs 3 to 4 us whatever it does, so a workgroup
+// recomputes what passed between two of them for all rows (16 rows x 384 columns are a few KB in L2) and multiplies it with its 16
+// columns of the next product.  All waves share the first part, a row or a head each; what they leave in LDS as bf16 rows one wave
+// multiplies, in enc_gemm's four partial sums, which makes its bits.  Six layers of 384 / 1536 on 16 rows: 154 -> 135 us.  More rows
+// repeat too much: with as many row tiles a workgroup, 32 rows took 185 us against 171, 64 299 against 214.
+constexpr int FEW_M = 16, FEW_K = 384, FEW_LD = FEW_K + 8;      // most rows and columns; LDS rows 16 bytes apart in the banks
+struct FewW {
+  bf16x8 f[4][3];
+  __device__ __forceinline__ void load(const u16* __restrict__ wr, int steps) {
+    const int per = (steps + 3) / 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int u = 0; u < 3; ++u) f[j][u] = __builtin_bit_cast(bf16x8, ld16(wr + 32 * min(j * per + min(u, per - 1), steps - 1)));
+  }
+  __device__ __forceinline__ f32x4 mul(const u16* a, int steps) const {     // a: this lane's row and columns in LDS
+    const int per = (steps + 3) / 4;
+    f32x4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int s = j * per + u;
+        if (u < per && s < steps)
+          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a + 32 * s)), f[j][u], acc[j], 0, 0, 0);
+      }
+    return ((acc[0] + acc[1]) + acc[2]) + acc[3];
+  }
+};
+
+// EPI ENC_QKV: columns of q and k as they are, to Y; those of v transposed, to Vt [H][16], zero from row M on, as attn_out reads them.
+// ENC_GELU as in enc_gemm.  LN: X is the sum that a LayerNorm takes (norm.hip's arithmetic, a wave a row); the first workgroup stores
+// its rows to Xn for the residual sum that follows.
+template <int EPI, bool LN>
+__global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ X, const u16* __restrict__ W, const u16* __restrict__ bias,
+                                                        u16* __restrict__ Y, int M, int N, int K, const u16* __restrict__ lnw,
+                                                        const u16* __restrict__ lnb, float eps, u16* __restrict__ Xn, u16* __restrict__ Vt) {
+  __shared__ __attribute__((aligned(16))) u16 sx[FEW_M * FEW_LD];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g = lane >> 4;
+  const int col0 = blockIdx.x * 16, steps = K / 32, c = 8 * lane;
+  uint4 xv = {}, gw = {}, gb = {};
+  FewW wf;
+  float b = 0.f;
+  if (c < K) {
+    xv = ld16(X + (long)min(w, M - 1) * K + c);        // rows past M repeat the last and are dropped
+    if (LN) { gw = ld16(lnw + c); gb = ld16(lnb + c); }
+  }
+  if (w == 0) {
+    wf.load(W + (long)(col0 + lr) * K + 8 * g, steps);
+    b = bf2f(bias[col0 + lr]);
+  }
+  if (LN) {
+    float v[8], s = 0.f, q = 0.f, ga[8], be[8];
+    unpack8(xv, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += v[j];
+    const float mean = wave_sum(s) / K;
+    if (c < K)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { const float d = v[j] - mean; q += d * d; }
+    const float rstd = rsqrtf(wave_sum(q) / K + eps);
+    unpack8(gw, ga);
+    unpack8(gb, be);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (v[j] - mean) * rstd * ga[j] + be[j];
+    xv = pack8(v);
+    if (blockIdx.x == 0 && w < M && c < K) st16(Xn + (long)w * K + c, xv);
+  }
+  if (c < K) st16(sx + w * FEW_LD + c, xv);
+  __syncthreads();
+  if (w > 0) return;
+  const f32x4 v = wf.mul(sx + lr * FEW_LD + 8 * g, steps);       // column lr of rows 4g..4g + 3
+  if (EPI == ENC_QKV && 3 * col0 >= 2 * N) {          // N = 3 H, and H in whole tiles of 16
+    u16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.v[i] = 4 * g + i < M ? f2bf(v[i] + b) : 0;
+    *reinterpret_cast<u16x4*>(Vt + (long)(col0 - N / 3 * 2 + lr) * FEW_M + 4 * g) = o;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * g + i < M) {
+      const float z = bf2f(f2bf(v[i] + b));
+      Y[(long)(4 * g + i) * N + col0 + lr] = f2bf(EPI == ENC_GELU ? 0.5f * z * (1.f + erff(z * 0.70710678118654752f)) : z);
+    }
+}
+
+// y += attention(qkv) . w^T + bias.  A wave takes a head, all queries and keys.  S^T = K . Q^T leaves a query's scores in one lane
+// column and P^T feeds O^T = V^T . P^T as in encoder_attn, in its key order (keys 16 to 31 of a step are zero).  Rows of other texts
+// are masked by the text's bounds.
+template <int D>
+__global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __restrict__ qkv, const u16* __restrict__ Vt,
+                                                                  const u16* __restrict__ W, const u16* __restrict__ bias,
+                                                                  u16* __restrict__ Y, int M, int nh, float scale_log2,
+                                                                  const int* __restrict__ starts, const int* __restrict__ lens, int B,
+                                                                  int Smax) {
+  constexpr int KST = D / 32, NT = D / 16;
+  __shared__ __attribute__((aligned(16))) u16 so[FEW_M * FEW_LD];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g = lane >> 4;
+  const int col0 = blockIdx.x * 16, H = nh * D, steps = H / 32;
+  const u16* qp = qkv + (long)min(lr, M - 1) * (3 * H) + w * D + 8 * g;
+  bf16x8 qf[KST], kf[KST], vf[NT];
+#pragma unroll
+  for (int u = 0; u < KST; ++u) {
+    qf[u] = __builtin_bit_cast(bf16x8, ld16(qp + 32 * u));
+    kf[u] = __builtin_bit_cast(bf16x8, ld16(qp + H + 32 * u));
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const uint2 x = *reinterpret_cast<const uint2*>(Vt + (long)(w * D + 16 * n + lr) * FEW_M + 4 * g);
+    vf[n] = __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, 0, 0));
+  }
+  int ts = 0, tn = 0;                  // text `lane`: first row, rows
+  if (lane < B) {
+    ts = min(max(starts[lane], 0), M);
+    tn = min(min(max(lens[lane], 0), Smax), M - ts);
+  }
+  FewW wf;
+  float b = 0.f, r[4] = {};
+  if (w == 0) {
+    wf.load(W + (long)(col0 + lr) * H + 8 * g, steps);
+    b = bf2f(bias[col0 + lr]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = bf2f(Y[(long)min(4 * g + i, M - 1) * H + col0 + lr]);
+  }
+  int q0 = 0, q1 = 0;                  // the keys of this lane's query
+  for (int t = 0; t < B; ++t) {
+    const int a = __builtin_amdgcn_readlane(ts, t), e = a + __builtin_amdgcn_readlane(tn, t);
+    if (lr >= a && lr < e) q0 = a, q1 = e;
+  }
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < KST; ++u) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u], qf[u], s, 0, 0, 0);
+  float p[8] = {}, mx = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    p[i] = 4 * g + i >= q0 && 4 * g + i < q1 ? s[i] * scale_log2 : -INFINITY;
+    mx = fmaxf(mx, p[i]);
+  }
+  mx = lane_max(mx, 16);
+  mx = lane_max(mx, 32);
+  if (mx == -INFINITY) mx = 0.f;       // a row of no text (or past M): every weight 0
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { p[i] = exp2f(p[i] - mx); l += p[i]; }
+  l = lane_add(l, 16);
+  l = lane_add(l, 32);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const bf16x8 pf = __builtin_bit_cast(bf16x8, pack8(p));
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const f32x4 o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[n], pf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    u16x4 z;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) z.v[i] = f2bf(o[i] * inv);
+    *reinterpret_cast<u16x4*>(so + lr * FEW_LD + w * D + 16 * n + 4 * g) = z;
+  }
+  __syncthreads();
+  if (w > 0) return;
+  const f32x4 v = wf.mul(so + lr * FEW_LD + 8 * g, steps);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (4 * g + i < M) Y[(long)(4 * g + i) * H + col0 + lr] = f2bf(bf2f(f2bf(v[i] + b)) + r[i]);
 }
 
 // out[t] = LayerNorm(word[ids[t]] + pos[p] + type0) * w + b, p = at[t] or t % S   (one wave per token, H <= 2048)
@@ -297,4 +465,29 @@ extern "C" int dllm_enc_gemm(const void* x, long ldx, const void* w, const void*
   if (M <= 48) ENCG(3);
   ENCG(4);
 #undef ENCG
+}
+
+// May a whole layer take dllm_enc_few_layer?  (16 rows: above at enc_rows)
+extern "C" int dllm_enc_few_ok(int M, int nh, int d, int I, int B) {
+  return M >= 1 && M <= FEW_M && B >= 1 && B <= 64 && (d == 32 || d == 64) && nh >= 1 && nh * d <= FEW_K && I >= 32 && I % 32 == 0;
+}
+
+// One layer on M packed rows.  x [M, H]: the rows, or (ln0w) where they go: they are the LayerNorm of the sums in y.  Leaves the next
+// sums in y.  w: QKV w, b, output w, b, norm w, b, up w, b, down w, b.  qkv [M, 3H], vt [H, 16], f [M, I].  Operands 16-byte aligned,
+// rows contiguous.
+extern "C" int dllm_enc_few_layer(void* x, void* y, void* qkv, void* vt, void* f, const void* const* w, const void* ln0w, const void* ln0b,
+                                  int M, int nh, int d, int I, float eps, float scale, const int* starts, const int* lens, int B, int S,
+                                  hipStream_t st) {
+  if (!dllm_enc_few_ok(M, nh, d, I, B)) return -1;
+  u16 *X = (u16*)x, *Y = (u16*)y, *Q = (u16*)qkv, *V = (u16*)vt, *F = (u16*)f;
+  const u16* const* W = reinterpret_cast<const u16* const*>(w);
+  const int H = nh * d;
+  const dim3 rows(64 * FEW_M), heads(64 * nh);
+  if (ln0w) hipLaunchKernelGGL((enc_rows_kernel<ENC_QKV, true>), dim3(3 * H / 16), rows, 0, st, Y, W[0], W[1], Q, M, 3 * H, H, (const u16*)ln0w, (const u16*)ln0b, eps, X, V);
+  else hipLaunchKernelGGL((enc_rows_kernel<ENC_QKV, false>), dim3(3 * H / 16), rows, 0, st, X, W[0], W[1], Q, M, 3 * H, H, nullptr, nullptr, eps, nullptr, V);
+  if (d == 32) hipLaunchKernelGGL(attn_out_kernel<32>, dim3(H / 16), heads, 0, st, Q, V, W[2], W[3], X, M, nh, scale * LOG2E, starts, lens, B, S);
+  else hipLaunchKernelGGL(attn_out_kernel<64>, dim3(H / 16), heads, 0, st, Q, V, W[2], W[3], X, M, nh, scale * LOG2E, starts, lens, B, S);
+  hipLaunchKernelGGL((enc_rows_kernel<ENC_GELU, true>), dim3(I / 16), rows, 0, st, X, W[6], W[7], F, M, I, H, W[4], W[5], eps, Y, nullptr);
+  const int rc = (int)hipGetLastError();
+  return rc ? rc : dllm_enc_gemm(F, I, W[8], W[9], Y, H, M, H, I, ENC_RESADD, st);
 }

@@ -147,3 +147,36 @@ def test_few_row_projections(M, N, K):
         # two roundings to bf16 of at most 2^-9 each (the projection and the result)
         assert float((y.double() - want).norm() / want.norm()) < 2 ** -8
     assert not ext.enc_gemm(_b(65, K), w, bias, _b(65, N), 0) and not ext.enc_gemm(x, _b(N + 8, K), _b(N + 8), _b(M, N + 8), 0)
+
+
+@pytest.mark.parametrize("lens", [[1], [15], [16], [17], [9, 7], [1] * 16, [1, 0, 12]])
+@pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (6, 64, 320), (3, 64, 96), (1, 32, 32), (5, 32, 64)])
+def test_layers_of_few_rows(lens, nh, d, inter):
+    """Four launches a layer against one per operation.  A single text meets the same sums in the same order: equal bits.
+    Among several, a text's keys lie in other lanes and its sums take another order: rows then lie no further from a
+    double's than the separate launches' do, give or take a tenth (root mean square over at least 416 numbers; most of either error is
+    the roundings both share)."""
+    torch.manual_seed(sum(lens) + inter)
+    H, T, S = nh * d, sum(lens), max(lens)
+    layers = [dict(wqkv=_b(3 * H, H, scale=0.05), bqkv=_b(3 * H), wo=_b(H, H, scale=0.05), bo=_b(H), ln1=(_b(H) + 1, _b(H)), w1=_b(inter, H, scale=0.05),
+                   b1=_b(inter), w2=_b(H, inter, scale=0.05), b2=_b(H), ln2=(_b(H) + 1, _b(H))) for _ in range(2)]
+    x0 = _b(T, H)
+    starts = [sum(lens[:i]) for i in range(len(lens))]
+    dl, ds = (torch.tensor(v, dtype=torch.int32).cuda() for v in (lens, starts))
+    got = ops.gemm.encoder_layers(x0.clone(), dl, ds, S, nh, d, 1e-12, layers)
+    x, y = x0.clone(), x0.double().cpu()
+    for L in layers:
+        a = ops.encoder_attention(ops.gemm.linear_bias(x, L["wqkv"], L["bqkv"]), dl, len(lens), S, nh, d, starts=ds)
+        x = ops.layer_norm(ops.gemm.linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], 1e-12)
+        f = ops.gemm.linear_bias(x, L["w1"], L["b1"], gelu=True)
+        x = ops.layer_norm(ops.gemm.linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], 1e-12)
+        D = {k: tuple(t.double().cpu() for t in v) if isinstance(v, tuple) else v.double().cpu() for k, v in L.items()}
+        q, k, v = F.linear(y, D["wqkv"], D["bqkv"]).view(T, 3, nh, d).unbind(1)
+        a = torch.cat([F.scaled_dot_product_attention(*(t[s:s + n].transpose(0, 1) for t in (q, k, v))).transpose(0, 1).reshape(n, H)
+                       for s, n in zip(starts, lens) if n])
+        y = F.layer_norm(y + F.linear(a, D["wo"], D["bo"]), (H,), *D["ln1"], 1e-12)
+        y = F.layer_norm(y + F.linear(F.gelu(F.linear(y, D["w1"], D["b1"])), D["w2"], D["b2"]), (H,), *D["ln2"], 1e-12)
+    if len(lens) == 1:
+        assert torch.equal(got, x)
+    rms = lambda t: float((t.cpu().double() - y).square().mean().sqrt())  # noqa: E731
+    assert rms(got) <= 1.1 * rms(x) + 1e-9, (rms(got), rms(x))
