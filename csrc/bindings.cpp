@@ -43,6 +43,7 @@ int dllm_sample_split_kmax();
 int dllm_skinny_epi(const void*, long, const void*, int, void*, long, int, int, int, int, int, int, float*, int*, void*,
                     long, float*, long, const float*, int, long, float, float, const int*, const float*, const int*,
                     void*, void*, void*, int, int, int, hipStream_t);
+int dllm_f32_gemm(const float*, long, const float*, float*, long, int, int, int, int, hipStream_t);
 int dllm_dgemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*, void*, long, float*, long,
                float, float, const int*, const float*, const int*, void*, void*, void*, void*, long, int, int, int, const float*, int, float,
                float, hipStream_t);
@@ -741,6 +742,24 @@ void skinny_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t ntw,
         part.data_ptr<float>(), counters.data_ptr<int>(), stream()),
      "skinny_gemm");
 }
+
+// Projection of up to 16 f32 rows on a fragment-major weight (f32_gemm.hip); epi 0 plain, 5 erf-GELU
+void f32_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor y, int64_t epi) {
+  for (auto* t : {&x, &w, &y}) {
+    check_dev(*t, "f32_gemm operand");
+    TORCH_CHECK(t->scalar_type() == torch::kFloat32, "f32 operands");
+  }
+  TORCH_CHECK(x.dim() == 2 && y.dim() == 2 && x.size(0) >= 1 && x.size(0) <= 16 && y.size(0) == x.size(0) && x.stride(1) == 1 && y.stride(1) == 1,
+              "x [M, K], y [M, N], up to 16 rows of unit column stride");
+  const int64_t M = x.size(0), K = x.size(1), N = y.size(1);
+  TORCH_CHECK(w.dim() == 4 && w.is_contiguous() && w.size(0) == (N + 15) / 16 && w.size(1) * 16 == K && w.size(2) == 64 && w.size(3) == 4,
+              "w [ceil(N / 16), K / 16, 64, 4]");
+  TORCH_CHECK(epi == 0 || epi == 5, "epi: plain or gelu");
+  ok(dllm_f32_gemm(x.data_ptr<float>(), M > 1 ? x.stride(0) : K, w.data_ptr<float>(), y.data_ptr<float>(), M > 1 ? y.stride(0) : N, (int)M, (int)N,
+                   (int)K, (int)epi, stream()),
+     "f32_gemm");
+}
+
 // Decode GEMM on fragment-major weights (csrc/kernels/decode_gemm.hip), M <= 64: x [M, K], w [ceil(N / 16), K / 32, 64, 8]
 // (ops.gemm.frag_weight; paired for epi 2, 3 and 4), epi 0 plain (y [M, N]), 1 residual add (res in place, per-tile row sums of squares ->
 // ssq_out), 2 QKV (row scale, RoPE, q_out, paged K, V^T or v_rows), 3 SwiGLU (row scale, y = act [M, N / 2]), 4 gated activation `mode` of glu_act with
@@ -2898,6 +2917,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("skinny_gemm", &skinny_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("ntw"), py::arg("splits"), py::arg("swiglu"),
         py::arg("part"), py::arg("counters"), py::arg("vs") = 1);
   m.def("skinny_epi", &skinny_epi);
+  m.def("f32_gemm", &f32_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("epi") = 0);
   m.def("dgemm", &dgemm);
   m.def("gemv", &gemv);
   m.def("gemv_norm", &gemv_norm);

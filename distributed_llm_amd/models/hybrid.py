@@ -103,6 +103,8 @@ def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, kee
     """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy."""
     if wf is not None and ops.gemm.dg_takes(x):
         return ops.linear(x, w, wf=wf, keep_order=keep_order)
+    if wf is not None and ops.gemm.fg_takes(x):
+        return ops.gemm.f32_linear(x, wf, w.shape[0])
     if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1
             and x.shape[1] % 64 == 0 and w.shape[0] % 64 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and w.is_contiguous()):
@@ -536,11 +538,16 @@ class HybridModel:
 
     def _place_fragments(self) -> None:
         """Fragment-major copies of the projections and the head for the decode GEMM (ops.gemm.frag_weight), while they fit in a
-        quarter of the memory still free.  Where the order of sums is kept, of those alone that ops.linear multiplies anyway."""
+        quarter of the memory still free.  Where the order of sums is kept, of those alone that ops.linear multiplies anyway: of an f32
+        model, whose products are the vendor's, none."""
         self.lm_head_r: Optional[torch.Tensor] = None
-        if self.dtype != torch.bfloat16 or self.device.type != "cuda" or not ops.native_available():
+        f32 = self.dtype == torch.float32
+        if self.device.type != "cuda" or not ops.native_available() or (f32 and self.order_kept):
             return
-        takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
+        if f32:
+            takes = lambda w: w.shape[1] % 16 == 0 and w.shape[1] <= ops.gemm.FG_MAX_K
+        else:
+            takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
         todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
         extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
         if extra > 0.25 * torch.cuda.mem_get_info(self.device)[0]:
@@ -549,14 +556,14 @@ class HybridModel:
             f = S.mlp
             act = self._act_args(f) if isinstance(f, DenseSpec) and not self.cfg.parallel_ff else None
             # an up projection with its activation: that copy alone (its plain product runs where no decode GEMM does)
-            if act is not None and any(l is L and n == "up" for l, n in todo) and (act[0] == "gelu" or f.ff % 8 == 0):
+            if not f32 and act is not None and any(l is L and n == "up" for l, n in todo) and (act[0] == "gelu" or f.ff % 8 == 0):
                 L["up_act_r"], L["order_kept"] = ops.gemm.frag_weight(L["up"], paired=False if act[0] == "gelu" else "glu"), self.order_kept
         for L, n in todo:
             if n != "up" or "up_act_r" not in L:
                 L[n + "_r"] = ops.gemm.frag_weight(L[n])
                 L["order_kept"] = self.order_kept
         ex = [(L, S.mlp) for L, S in zip(self.layers, self.cfg.layers)
-              if isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
+              if not f32 and isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
               and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
         extra = sum(L[n].numel() * L[n].element_size() for L, _ in ex for n in ("w1", "w2"))
         if extra <= 0.25 * torch.cuda.mem_get_info(self.device)[0]:
@@ -1026,6 +1033,8 @@ class HybridModel:
         act, a = self._act_args(f), None
         if "up_act_r" in L:
             a = ops.gemm.linear_act(x, L["up"], L["up_act_r"], act[0], L.get("up_b"), act[1], act[2], L["order_kept"])
+        elif "up_r" in L and act is not None and act[0] == "gelu" and ops.gemm.fg_takes(x):
+            a = ops.gemm.f32_linear(x, L["up_r"], L["up"].shape[0], gelu=True)
         if a is None:
             z = _pm(x, L, "up")
             if act is None:

@@ -118,8 +118,14 @@ _PAIR_ROWS = [*range(8), *range(16, 24), *range(8, 16), *range(24, 32)]
 
 def frag_weight(w: torch.Tensor, paired=False) -> torch.Tensor:
     """[N, K] -> [ceil(N / 16), K / 32, 64, 8]: of a 16-column tile and 32 k, lane 16 g + r holds W[16 t + r][32 s + 8 g ...+ 7]; rows past
-    N are zeros.  ``paired`` (the QKV and gate|up weights of models.llama, pairs 16 rows apart in groups of 32): pairs 8 rows apart; "glu": gate rows, then up rows, likewise."""
+    N are zeros.  ``paired`` (the QKV and gate|up weights of models.llama, pairs 16 rows apart in groups of 32): pairs 8 rows apart; "glu": gate rows, then up rows, likewise.
+    f32: [ceil(N / 16), K / 16, 64, 4], lane 16 g + r holds W[16 t + r][16 s + 4 g ...+ 3] (f32_gemm)."""
     N, K = w.shape
+    if w.dtype == torch.float32:
+        if K % 16 or paired:
+            raise ValueError(f"frag_weight: {N} x {K}")
+        w = torch.cat([w, w.new_zeros(-N % 16, K)])
+        return w.view(-1, 16, K // 16, 4, 4).permute(0, 2, 3, 1, 4).reshape(-1, K // 16, 64, 4).contiguous()
     if paired == "glu":
         if K % 32 or N % 16:
             raise ValueError(f"frag_weight: {N} x {K}")
@@ -559,6 +565,22 @@ def dg_takes(x: torch.Tensor) -> bool:
     """The decode GEMM reads these rows: up to 64, 16-byte aligned."""
     return 0 < x.shape[0] <= DG_MAX_M and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and \
         (x.shape[0] == 1 or x.stride(0) >= x.shape[1]) and x.data_ptr() % 16 == 0
+
+
+FG_MAX_M, FG_MAX_K = 16, 2048      # f32_gemm.hip: past them the vendor GEMM is as fast
+
+
+def fg_takes(x: torch.Tensor) -> bool:
+    """The f32 decode product reads these rows: up to 16, 16-byte aligned."""
+    return 0 < x.shape[0] <= FG_MAX_M and x.dtype == torch.float32 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 4 == 0 and \
+        (x.shape[0] == 1 or x.stride(0) >= x.shape[1]) and x.data_ptr() % 16 == 0 and os.environ.get("DLLM_GEMM") != "blas"
+
+
+def f32_linear(x: torch.Tensor, wf: torch.Tensor, N: int, gelu: bool = False) -> torch.Tensor:
+    """``x @ w.T`` [-> erf-GELU] of up to 16 f32 rows on the weight's fragment-major copy (csrc/kernels/f32_gemm.hip)."""
+    y = torch.empty((x.shape[0], N), dtype=torch.float32, device=x.device)
+    _native(x).f32_gemm(x, wf, y, DG_GELU if gelu else EPI_PLAIN)
+    return y
 
 
 def _linear_plan(x: torch.Tensor, w: torch.Tensor, frag: bool, keep_order: bool):

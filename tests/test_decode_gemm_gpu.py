@@ -150,3 +150,20 @@ def test_activations(M, act, limit, alpha, bias, N, K):
     z = G.linear(x, w, wf=G.frag_weight(w))
     want = seqmix.gelu_erf(z) if act == "gelu" else seqmix.glu_act(z, b, act, limit, alpha)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M", [1, 2, 15, 16])
+@pytest.mark.parametrize("N,K", [(16, 16), (90, 48), (515, 512), (1000, 1040), (256, 2048)])
+def test_f32_rows(M, N, K):
+    """The f32 product: waves without a step, partial groups of steps, columns past N, rows of a wider matrix; against a double's.  A sum is
+    at most K / 8 + 15 terms in a row and eight of those: that many roundings of 2^-24 of the absolute sum; erf-GELU (slope at most
+    1.13) adds four of its own of a value or of 1."""
+    x, w = torch.randn(M, K + 4, device=DEV)[:, :K], torch.randn(N, K, device=DEV)
+    assert G.fg_takes(x) and not G.fg_takes(torch.randn(17, K, device=DEV)) and not G.fg_takes(torch.randn(M + 1, K + 1, device=DEV)[:, 1:])
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    wf = G.frag_weight(w)
+    err = (G.f32_linear(x, wf, N).double() - want).abs()
+    bound = (K / 8 + 24) * 2.0 ** -24 * size
+    assert (err <= bound).all()
+    got = G.f32_linear(x, wf, N, gelu=True).double()
+    assert ((got - torch.nn.functional.gelu(want)).abs() <= 1.13 * bound + 4 * 2.0 ** -24 * (want.abs() + 1)).all()
