@@ -114,6 +114,88 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(const T* __restrict__ pr
   }
 }
 
+// The same in 16-byte vectors (bf16): D / 8 lanes a head, a wave 512 / D heads of a token and four tokens with every load in flight; a
+// workgroup covers 16 tokens (blockIdx.x) and one such group of heads, or (the last blockIdx.y) 512 value entries, turned in LDS so that
+// the 16 tokens of an entry, which lie side by side in V^T's page, are stored by neighbouring lanes.  Element by element it is bound by
+// 2-byte accesses, made twice, and by a sector for each value: 7300 tokens, 32 + 8 heads of 64 and as many values 123 us, here 32 (the
+// bytes alone: 15); a decode step's six tokens 5.2, here 4.9.
+// A lane's eight squares are added in the order that the wave's exchanges have there (D = 64: the same bits).
+constexpr int APV_T = 16, APV_V = 512;
+template <int D>
+__global__ void __launch_bounds__(256) attn_prep_vec_kernel(const u16* __restrict__ proj, long ld, int H, int G, int dv,
+                                                            const float* __restrict__ cos_sin, int tab_w, int rot, float eps,
+                                                            const float* __restrict__ qscale, const int* __restrict__ pos,
+                                                            const int* __restrict__ slots, u16* __restrict__ kc, u16* __restrict__ vc,
+                                                            u16* __restrict__ q, int BSZ, int T, int ny) {
+  constexpr int LPH = D / 8, TW = APV_T / 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t0 = blockIdx.x * APV_T;
+  if ((int)blockIdx.y < ny) {
+    const int hh = (blockIdx.y * 64 + lane) / LPH, c = lane % LPH * 8, half = rot >> 1;
+    const int hx = min(hh, H + G - 1), f = c < half ? c : c - half;
+    const bool is_q = hh < H, turn = c < rot;
+    const float qs = qscale[min(hh, H - 1)];
+    uint4 x[TW], p[TW];
+    f32x4 cs[TW][2], sn[TW][2];
+    int slot[TW];
+#pragma unroll
+    for (int k = 0; k < TW; ++k) {
+      const int tok = min(t0 + wave + 4 * k, T - 1);
+      const u16* r = proj + tok * ld + hx * D;
+      x[k] = ld16(r + c);
+      slot[k] = slots[tok];
+      if (turn) {
+        p[k] = ld16(r + (c < half ? c + half : c - half));
+        const float* cp = cos_sin + (long)pos[tok] * tab_w + f;
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+          cs[k][y] = *reinterpret_cast<const f32x4*>(cp + 4 * y);
+          sn[k][y] = *reinterpret_cast<const f32x4*>(cp + half + 4 * y);
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < TW; ++k) {
+      const int tok = t0 + wave + 4 * k;
+      float v[8], w[8], e[8];
+      unpack8(x[k], v);
+      if (turn) {
+        unpack8(p[k], w);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float co = cs[k][j / 4][j % 4], si = sn[k][j / 4][j % 4];
+          v[j] = c < half ? v[j] * co - w[j] * si : v[j] * co + w[j] * si;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) e[j] = v[j] * v[j];
+#pragma unroll
+      for (int o = LPH / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = lane_add(e[j], o);
+      const float ss = ((e[0] + e[4]) + (e[2] + e[6])) + ((e[1] + e[5]) + (e[3] + e[7]));
+      const float sc = (is_q ? qs : 1.f) / sqrtf(ss / (float)D + eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] *= sc;
+      if (tok >= T || hh >= H + G || (!is_q && slot[k] < 0)) continue;
+      u16* dst = is_q ? q + ((long)tok * H + hh) * D : kc + (((long)(slot[k] / BSZ) * G + (hh - H)) * BSZ + slot[k] % BSZ) * D;
+      st16(dst + c, pack8(v));
+    }
+    return;
+  }
+  __shared__ __attribute__((aligned(16))) u16 sv[APV_T][APV_V + 8];
+  const int e0 = (blockIdx.y - ny) * APV_V, ne = min(APV_V, G * dv - e0);      // whole vectors of 8
+  for (int i = threadIdx.x; i < APV_T * (APV_V / 8); i += 256) {
+    const int t = i / (APV_V / 8), c = i % (APV_V / 8) * 8;
+    if (t0 + t < T && c < ne) st16(&sv[t][c], ld16(proj + (t0 + t) * ld + (long)(H + G) * D + e0 + c));
+  }
+  const int t = lane % APV_T, slot = t0 + t < T ? slots[t0 + t] : -1;
+  __syncthreads();
+  if (slot < 0) return;
+  const long blk = slot / BSZ;
+  u16* vp = vc + blk * G * dv * BSZ + slot % BSZ;
+  for (int i = threadIdx.x / APV_T; i < ne; i += 256 / APV_T) vp[(long)(e0 + i) * BSZ] = sv[t][i];
+}
+
 // One wave per q / k vector (head, map): bias, weighted RMS norm over d, rotate-half positions on the
 // first `rot` dims, q times `qscale`.  Query unit (h, m) of key/value head g = h / R leaves as row
 // g M R + m R + h % R of q [T, H M, d]; key unit (g, m) goes to key head g M + m of the page.
@@ -1046,6 +1128,21 @@ extern "C" int dllm_attn_prep(const void* proj, long ld, int f32, int H, int G, 
                               void* vc, void* q, long T, int BSZ, hipStream_t st) {
   if (T <= 0) return 0;
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w) return -1;
+  // whole vectors: heads of 32 to 256, halves of the rotation and values in eights, 16-byte aligned rows
+  if (!f32 && (d == 32 || d == 64 || d == 128 || d == 256) && dv % 8 == 0 && rot % 16 == 0 && ld % 8 == 0 && tab_w % 4 == 0 && T < (1 << 20) &&
+      (((uintptr_t)proj | (uintptr_t)cos_sin | (uintptr_t)kc | (uintptr_t)q) & 15) == 0) {
+    const int ny = ((H + G) * (d / 8) + 63) / 64;
+    const dim3 g(((unsigned)T + APV_T - 1) / APV_T, ny + (G * dv + APV_V - 1) / APV_V);
+#define APV(D)                                                                                                                     \
+  hipLaunchKernelGGL(attn_prep_vec_kernel<D>, g, dim3(256), 0, st, (const u16*)proj, ld, H, G, dv, cos_sin, tab_w, rot, eps, qscale, pos, \
+                     slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ, (int)T, ny)
+    if (d == 32) APV(32);
+    else if (d == 64) APV(64);
+    else if (d == 128) APV(128);
+    else APV(256);
+#undef APV
+    return (int)hipGetLastError();
+  }
   const dim3 grid((unsigned)T, (H + G + 3) / 4);
   if (f32)
     hipLaunchKernelGGL(attn_prep_kernel<float>, grid, dim3(256), 0, st, (const float*)proj, ld, H, G, d, dv, cos_sin, tab_w, rot,

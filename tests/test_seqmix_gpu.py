@@ -842,3 +842,51 @@ def test_biased_attention_kernels(dt, case, H, G, d, dv, win):
             torch.testing.assert_close(got.float(), want, **tol(dt))
     with pytest.raises(RuntimeError):      # a cap on the scores has no form beside slopes
         seqmix.paged_gqa_attention(q2, kc2, vc2, bt, qstart, qlen, ctx, ts, tt, None, mfma, 1, softcap=3.0, slopes=slopes)
+
+
+@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130])])
+@pytest.mark.parametrize("H,G,d,dv,rot", [(32, 8, 64, 64, 32), (4, 2, 32, 32, 32), (6, 2, 128, 200, 64), (3, 3, 256, 8, 256), (5, 1, 64, 520, 0), (33, 1, 32, 64, 16)])
+def test_attn_prep_in_vectors(case, H, G, d, dv, rot):
+    """bf16 rows of whole vectors: groups of heads and of tokens full and not, a value block of 512 that ends inside, rows without a slot;
+    against the element-by-element form of the same rows at an odd offset (a rounding apart: a head's sum of squares may be added in
+    another order)."""
+    torch.manual_seed(6)
+    dt = torch.bfloat16
+    T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
+    n = (H + G) * d + G * dv
+    proj = torch.randn(T, n + 8, device=DEV).to(dt)
+    odd = torch.empty(T, n + 9, dtype=dt, device=DEV)
+    odd[:, :n] = proj[:, :n]
+    table = ops.rope_cos_sin(256, max(rot, 4), 100.0, DEV)
+    qscale = torch.rand(H, device=DEV) * 2 + 0.5
+    slots[T // 2] = -1
+    kc2, vc2 = kc.clone(), vc.clone()
+    q1 = seqmix.attn_prep(proj, H, G, d, dv, table, rot, 1e-5, qscale, pos, slots, kc, vc)
+    q2 = seqmix.attn_prep(odd, H, G, d, dv, table, rot, 1e-5, qscale, pos, slots, kc2, vc2)
+    torch.testing.assert_close(q1.float(), q2.float(), atol=1e-6, rtol=2.0 ** -7)
+    torch.testing.assert_close(kc.float(), kc2.float(), atol=1e-6, rtol=2.0 ** -7)
+    assert torch.equal(vc, vc2)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,dv", [(1, 8), (2, 256), (8, 256), (9, 256), (5, 100)])
+def test_joint_head_norm(dt, H, dv):
+    """Heads of a token normed together and gated: entries in one, several and all eight of a thread's places, and past them; rows of no sequence."""
+    torch.manual_seed(7)
+    d = 8
+    T, qstart, qlen, ctx, rows, pos = batch([1, 1, 0, 1], [4, 0, 33, 2])
+    qkvg = torch.randn(T + 2, 2 * H * d + 2 * H * dv, device=DEV).to(dt)
+    decay, w = torch.rand(H, device=DEV), torch.randn(H * dv, device=DEV)
+    st = torch.randn(5, H, d, dv, device=DEV)
+    s2 = st.clone()
+    o1 = seqmix.lightning_attention(qkvg, H, d, dv, decay, st, 1e-6, w, qstart, qlen, ctx, rows)
+    o2 = ref.lightning_attention(qkvg, H, d, dv, decay, s2, 1e-6, w, qstart, qlen, ctx, rows)
+    torch.testing.assert_close(o1.float(), o2.float(), **tol(dt))
+    assert not o1[T:].any()
+
+
+@pytest.mark.parametrize("n", [8, 2048, 2056, 8 * 256 * 8192 + 8])
+def test_gelu_in_vectors(n):
+    """Bits of the element-by-element form (an odd offset), one vector, a block of them and more than the grid holds."""
+    x = (torch.randn(n + 1, device=DEV) * 3).bfloat16()
+    assert torch.equal(seqmix.gelu_erf(x[1:].clone()), seqmix.gelu_erf(x)[1:])
