@@ -687,3 +687,26 @@ def test_gemv_norm(M, N, K):
     ops._load().gemv_norm(h, res, spare, nw, 1e-5, w, y, 2)
     assert torch.equal(spare, res_ref)
     torch.testing.assert_close(y.float(), want, atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (2, 2), (5, 2), (64, 3)])
+@pytest.mark.parametrize("T", [1, 21, 32, 64, 65, 341, 1025, 4099, 16385])
+def test_routing_places_every_pair(T, E, k):
+    """Waves with and without pairs, runs of 64 full and not, more pairs than a wave keeps in flight, experts without a pair and one with
+    all; against the same rows by expert (ids past the experts count as the last).  Each pair's row is its own: 2^-8 of the largest
+    product for the bf16 roundings of activation and sum, of which there are k."""
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    H, I = 64, 64
+    x = torch.randn(T, H, device="cuda", generator=g).bfloat16()
+    w13 = (torch.randn(E, 2 * I, H, device="cuda", generator=g) * 0.1).bfloat16()
+    w2 = (torch.randn(E, H, I, device="cuda", generator=g) * 0.1).bfloat16()
+    w = torch.rand(T, k, device="cuda", generator=g)
+    for skew in (False, True):
+        ids = torch.randint(0, E + 1, (T, k), device="cuda", generator=g, dtype=torch.int32)
+        if skew:
+            ids[:] = max(0, E - 2)
+        got, want = ops.moe_ffn(x, ids, w, w13, w2).double(), torch.zeros(T, H, dtype=torch.float64, device="cuda")
+        for e in range(E):
+            y = torch.nn.functional.silu(x.float() @ w13[e, :I].float().t()) * (x.float() @ w13[e, I:].float().t())
+            want += ((ids.clamp(max=E - 1) == e) * w).sum(1, keepdim=True).double() * (y @ w2[e].float().t()).double()
+        assert float((got - want).abs().max()) <= 2.0 ** -8 * (k + 1) * max(1.0, float(want.abs().max()))
