@@ -565,24 +565,55 @@ static inline MfmaLds mfma_lds(int rank, int rot, int KT, int rows = LROWS) {
   return L;
 }
 
-// A key tile's rows into registers: wave w takes rows w, w + 4, ..., a lane 16 bytes of a row (two per
-// row cover up to 1024 entries); rows past `kend` and lanes past the row's end get zeros.
+// A key tile's rows into registers: wave w takes the KT / 4 rows from KT / 4 w on, which lie in one page (`page`, the wave's own), a
+// lane 16 bytes of a row (two per row cover up to 1024 entries); rows past `kend` and lanes past the row's end get zeros.
 template <int KT>
-__device__ __forceinline__ void fetch_tile(uint4 (&pf)[KT / 4][2], const u16* __restrict__ cache,
-                                           const int* __restrict__ btr, int k0, int kend, int Dp, int lane, int wave) {
-  const int nk = min(KT, kend - k0);
-  const int pg0 = k0 >> 4, npg = ((k0 + nk - 1) >> 4) - pg0 + 1;
-  const int pg = lane < npg ? btr[pg0 + lane] : 0;
+__device__ __forceinline__ void fetch_tile(uint4 (&pf)[KT / 4][2], const u16* __restrict__ cache, int page, int k0, int kend, int Dp,
+                                           int lane, int wave) {
+  const int kk = k0 + KT / 4 * wave;
+  const u16* src = cache + ((long)page * 16 + (kk & 15)) * Dp + 8 * lane;
 #pragma unroll
-  for (int r = 0; r < KT / 4; ++r) {
-    const int kk = wave + 4 * r, kidx = k0 + kk;
-    const bool live = kk < nk;
-    const long page = __shfl(pg, live ? (kidx >> 4) - pg0 : 0);
-    const uint4* src = reinterpret_cast<const uint4*>(cache + (page * 16 + (kidx & 15)) * Dp);
+  for (int r = 0; r < KT / 4; ++r)
+    pf[r][0] = kk + r < kend && lane < (Dp >> 3) ? ld16(src + r * Dp) : make_uint4(0u, 0u, 0u, 0u);
+  if (Dp > 512) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c8 = lane + 64 * j;
-      pf[r][j] = (live && c8 < (Dp >> 3)) ? src[c8] : make_uint4(0u, 0u, 0u, 0u);
+    for (int r = 0; r < KT / 4; ++r)
+      pf[r][1] = kk + r < kend && lane + 64 < (Dp >> 3) ? ld16(src + r * Dp + 512) : make_uint4(0u, 0u, 0u, 0u);
+  }
+}
+
+// The fetched rows to LDS: as they are, and the latent part transposed ([dim][key], 8-key groups swapped about by the dim's vector so
+// that the lanes' stores spread over the banks).  A lane holds 8 dims of KT / 4 consecutive keys: the turn is a byte permutation of
+// its registers (through 2-byte reads of the rows in LDS it was a third of the launch, 2.2 us a 64-key tile, and a barrier).
+__device__ __forceinline__ int turn_at(int dim, int kg, int KT) { return 8 * (kg ^ ((dim >> 3) & (KT / 8 - 1))); }
+template <int KT>
+__device__ __forceinline__ void put_tile(const uint4 (&pf)[KT / 4][2], u16* __restrict__ ksh, u16* __restrict__ ktr, int Dp, int ndim,
+                                         int qstr, int ktstr, int lane, int wave) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int c = 8 * (lane + 64 * j);
+    if (j == 1 && Dp <= 512) break;
+    if (c >= Dp) continue;
+#pragma unroll
+    for (int r = 0; r < KT / 4; ++r) st16(ksh + (KT / 4 * wave + r) * qstr + c, pf[r][j]);
+    if (c >= ndim) continue;
+#pragma unroll
+    for (int r = 0; r < KT / 4; r += 8) {
+      const int kg = (KT / 4 * wave + r) >> 3;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        uint32_t lo[4], hi[4];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const uint4 e = pf[r + 2 * y][j], o = pf[r + 2 * y + 1][j];
+          const uint32_t ex = x == 0 ? e.x : x == 1 ? e.y : x == 2 ? e.z : e.w, ox = x == 0 ? o.x : x == 1 ? o.y : x == 2 ? o.z : o.w;
+          lo[y] = __builtin_amdgcn_perm(ox, ex, 0x05040100u);
+          hi[y] = __builtin_amdgcn_perm(ox, ex, 0x07060302u);
+        }
+        u16* t = ktr + (c + 2 * x) * ktstr + turn_at(c, kg, KT);
+        st16(t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        st16(t + ktstr, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+      }
     }
   }
 }
@@ -590,6 +621,10 @@ __device__ __forceinline__ void fetch_tile(uint4 (&pf)[KT / 4][2], const u16* __
 // LR: 16-row blocks per workgroup (1: decode steps and short portions; 2: prompt portions, where the
 // tile's staging, transposition and barriers then serve 32 rows and every wave has a score task at
 // 32-key tiles).  Score tasks (row block, 16 keys) are dealt to the waves round-robin.
+// Decode is bound by the launch and its chain of trips to memory (step metadata, page numbers, rows), then by the steps of a tile one
+// behind the other, not by bytes: four sequences, 16 heads, rank 256, 16 splits, with the merging launch: 1000 keys (a tile each) 20.2 -> 13.4
+// us, 1300 (two) 27.0 -> 17.0; one of 4000 (four) 40.5 -> 24.1.  Of that the turn of the rows in registers is 2 us a tile, scalar page
+// numbers (a shuffle through LDS for each row before) and the queries' loads ahead of them 3 us a launch.
 template <int CB, int KT, int LR>
 __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
     const u16* __restrict__ qa, const u16* __restrict__ q, long ldq, int H, int dim, int rot, int rank, long Ttot,
@@ -620,35 +655,9 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
   u16* phi = ktr + RB * 16 * ktstr;                     // [RPB][pstr]
   u16* plo = phi + RPB * pstr;
   float* wred = reinterpret_cast<float*>(plo + RPB * pstr);   // [4][RPB]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, g = lane >> 4;
   const int half = rot >> 1;
-  // queries: the latent part as 16-byte vectors where rows allow it, the rest (rotated part, padding) alone
-  const int cs0 = (rank & 7) == 0 ? rank : 0;
-  for (int e = tid; e < RPB * (cs0 >> 3); e += 256) {
-    const int rr = e / (cs0 >> 3), c = 8 * (e - rr * (cs0 >> 3)), row = row0 + rr;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (row < nrows) v = ld16(qa + ((long)(row % H) * Ttot + q0 + tok0 + row / H) * rank + c);
-    st16(qsh + rr * qstr + c, v);
-  }
-  const int nrest = Dpad - cs0;
-  for (int e = tid; e < RPB * nrest; e += 256) {
-    const int rr = e / nrest, c = cs0 + e - rr * nrest, row = row0 + rr;
-    float v = 0.f;
-    if (row < nrows && c < Dp) {
-      const int tl = tok0 + row / H, h = row % H;
-      const long tok = q0 + tl;
-      if (c < rank) {
-        v = bf2f(qa[((long)h * Ttot + tok) * rank + c]);
-      } else {
-        v = rotated(q + tok * ldq + (long)h * (dim + rot) + dim, c - rank, half, hf, cos_sin + (long)(p0 + tl) * tab_w);
-      }
-    }
-    qsh[rr * qstr + c] = f2bf(v);
-  }
-  // zero what no staging pass writes: the key rows' padded dims
-  const int npad = Dpad - Dp;
-  for (int e = tid; e < KT * npad; e += 256) ksh[(e / npad) * qstr + Dp + e % npad] = 0;
   const int last_row = min(row0 + RPB, nrows) - 1;
   const int kmax = p0 + tok0 + last_row / H + 1;
   int rpos[LR][4];
@@ -672,26 +681,68 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
   const int ntiles = (kmax + KT - 1) / KT;
   const int kbeg = (int)((long)ntiles * blockIdx.z / splits) * KT;
   const int kend = min(kmax, (int)((long)ntiles * (blockIdx.z + 1) / splits) * KT);
+  if (splits > 1 && kbeg >= kend) {        // more splits than tiles: nothing to leave but that (decode grids have them for the longest context)
+    if (tid < RPB) {
+      const long pr = (((long)entry * gridDim.x + blockIdx.x) * RPB + tid) * splits + blockIdx.z;
+      part_ml[2 * pr] = -INFINITY;
+      part_ml[2 * pr + 1] = 0.f;
+    }
+    return;
+  }
   // rows of a multiple of 8 entries (and at most 1024) move as 16-byte vectors, one tile ahead
   const bool pre = (Dp & 7) == 0 && Dp <= 1024;
   uint4 pf[KT / 4][2];
-  if (pre && kbeg < kend) fetch_tile<KT>(pf, cache, btr, kbeg, kend, Dp, lane, wave);
+  // The page of the wave's rows of a tile; 0 past the last key.  Then the queries' latent part and the first tile's rows, so that what the
+  // staging waits for is all on its way.
+  auto page_of = [&](int k0) { return pre && k0 + KT / 4 * wave < kend ? btr[(k0 + KT / 4 * wave) >> 4] : 0; };
+  int page = page_of(kbeg);
+  constexpr int NQ = 2 * LR;
+  const int cs0 = (rank & 7) == 0 ? rank : 0;
+  auto query = [&](int e) {
+    const int rr = e / (cs0 >> 3), c = 8 * (e - rr * (cs0 >> 3)), row = row0 + rr;
+    return row < nrows ? ld16(qa + ((long)(row % H) * Ttot + q0 + tok0 + row / H) * rank + c) : make_uint4(0u, 0u, 0u, 0u);
+  };
+  uint4 qv[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i)
+    if (tid + 256 * i < RPB * (cs0 >> 3)) qv[i] = query(tid + 256 * i);
+  if (pre && kbeg < kend) fetch_tile<KT>(pf, cache, page, kbeg, kend, Dp, lane, wave);
+  page = page_of(kbeg + KT);
+  // queries: the latent part as 16-byte vectors where rows allow it, the rest (rotated part, padding) alone
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int e = tid + 256 * i;
+    if (e < RPB * (cs0 >> 3)) st16(qsh + e / (cs0 >> 3) * qstr + 8 * (e % (cs0 >> 3)), qv[i]);
+  }
+  for (int e = tid + 256 * NQ; e < RPB * (cs0 >> 3); e += 256) st16(qsh + e / (cs0 >> 3) * qstr + 8 * (e % (cs0 >> 3)), query(e));
+  const int nrest = Dpad - cs0;
+#pragma unroll 2
+  for (int e = tid; e < RPB * nrest; e += 256) {
+    const int rr = e / nrest, c = cs0 + e - rr * nrest, row = row0 + rr;
+    float v = 0.f;
+    if (row < nrows && c < Dp) {
+      const int tl = tok0 + row / H, h = row % H;
+      const long tok = q0 + tl;
+      if (c < rank) {
+        v = bf2f(qa[((long)h * Ttot + tok) * rank + c]);
+      } else {
+        v = rotated(q + tok * ldq + (long)h * (dim + rot) + dim, c - rank, half, hf, cos_sin + (long)(p0 + tl) * tab_w);
+      }
+    }
+    qsh[rr * qstr + c] = f2bf(v);
+  }
+  // zero what no staging pass writes: the key rows' padded dims
+  const int npad = Dpad - Dp;
+  for (int e = tid; e < KT * npad; e += 256) ksh[(e / npad) * qstr + Dp + e % npad] = 0;
   for (int k0 = kbeg; k0 < kend; k0 += KT) {
     const int nk = min(KT, kend - k0);
     __syncthreads();
     if (pre) {
       // this tile's rows were fetched into registers while the previous tile was computed; put them
       // in LDS and start the next tile's fetch, which the products below then hide
-#pragma unroll
-      for (int r = 0; r < KT / 4; ++r) {
-        const int kk = wave + 4 * r;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int c8 = lane + 64 * j;
-          if (c8 < (Dp >> 3)) *reinterpret_cast<uint4*>(ksh + kk * qstr + 8 * c8) = pf[r][j];
-        }
-      }
-      if (k0 + KT < kend) fetch_tile<KT>(pf, cache, btr, k0 + KT, kend, Dp, lane, wave);
+      put_tile<KT>(pf, ksh, ktr, Dp, RB * 16, qstr, ktstr, lane, wave);
+      if (k0 + KT < kend) fetch_tile<KT>(pf, cache, page, k0 + KT, kend, Dp, lane, wave);
+      page = page_of(k0 + 2 * KT);
     } else {
       const int pg0 = k0 >> 4, npg = ((k0 + nk - 1) >> 4) - pg0 + 1;
       const int pg = lane < npg ? btr[pg0 + lane] : 0;
@@ -706,11 +757,9 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
           *reinterpret_cast<uint32_t*>(ksh + kk * qstr + 2 * c2) = w;
         }
       }
-    }
-    __syncthreads();
-    // the latent part once more, transposed ([dim][key]): threads along the dims read 8 keys' entries
-    // (2-byte reads of consecutive halfwords) and write them as one 16-byte vector
-    {
+      __syncthreads();
+      // the latent part once more, transposed: threads along the dims read 8 keys' entries (2-byte reads of consecutive
+      // halfwords) and write them as one 16-byte vector
       const int ndim = RB * 16;
       for (int e = tid; e < ndim * (KT / 8); e += 256) {
         const int kg = e / ndim, c = e - kg * ndim;
@@ -721,7 +770,7 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
           for (int x = 0; x < 4; ++x)
             w4[x] = (uint32_t)col[(2 * x) * qstr] | ((uint32_t)col[(2 * x + 1) * qstr] << 16);
         }
-        *reinterpret_cast<uint4*>(ktr + c * ktstr + 8 * kg) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+        *reinterpret_cast<uint4*>(ktr + c * ktstr + turn_at(c, kg, KT)) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
       }
     }
     __syncthreads();
@@ -742,6 +791,7 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
       if (on) {
         const u16* ap = qsh + (16 * rb + lr) * qstr + 8 * g;
         const u16* bp = ksh + (16 * kb + lr) * qstr + 8 * g;
+#pragma unroll 3
         for (int st = 0; st < Dpad; st += 32) {
           const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(ap + st));
           const bf16x8 b = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(bp + st));
@@ -811,9 +861,10 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
         for (int b = 0; b < LR; ++b)
 #pragma unroll
           for (int i = 0; i < 4; ++i) acc[j][b][i] *= alpha[b][i];
-        const u16* bp = ktr + (cb * 16 + lr) * ktstr + 8 * g;
+        const u16* bp = ktr + (cb * 16 + lr) * ktstr;
+#pragma unroll
         for (int ks = 0; ks < KT; ks += 32) {
-          const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(bp + ks));
+          const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(bp + turn_at(cb * 16 + lr, (ks >> 3) + g, KT)));
 #pragma unroll
           for (int b = 0; b < LR; ++b) {
             const int ro = (16 * b + lr) * pstr + ks + 8 * g;
@@ -877,34 +928,49 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
                                                              const int* __restrict__ tile_tok0, int tpe,
                                                              T* __restrict__ out, int rpb,
                                                              const float* __restrict__ sinks) {
+  // the partials are asked for before it is known that the row is one (every row has its place), and with their weights: this is bound
+  // by trips to memory one behind the other (four users, 16 heads, 16 splits: 7.9 -> 4.9 us)
+  constexpr int NZ = 16;
   const long r = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
+  const float* ml = part_ml + 2 * r * splits;
+  const float* po = part_o + r * splits * rank;
+  const float mz = lane < splits ? ml[2 * lane] : -INFINITY, lz = lane < splits ? ml[2 * lane + 1] : 0.f;
+  float first[NZ];
+#pragma unroll
+  for (int z = 0; z < NZ; ++z) first[z] = z < splits && tid < rank ? po[(long)z * rank + tid] : 0.f;
   const int rl = (int)(r % rpb);
   const long eb = r / rpb;
   const int bx = (int)(eb % gx), entry = (int)(eb / gx);
   const int s = tile_seq[entry];
-  const int n = qlen[s], tok0 = tile_tok0[entry];
+  const int n = qlen[s], tok0 = tile_tok0[entry], q0 = qstart[s];
   if (n <= 0 || tok0 >= n) return;
   const int row = bx * rpb + rl;
   if (row >= min(tpe, n - tok0) * H) return;
-  const float* ml = part_ml + 2 * r * splits;
-  const float mz = lane < splits ? ml[2 * lane] : -INFINITY, lz = lane < splits ? ml[2 * lane + 1] : 0.f;
   const float M = wave_max(mz);
   const float ez = mz > -INFINITY ? expf(mz - M) : 0.f;
   float L = wave_sum(lz * ez);
   if (sinks && L > 0.f) L += expf(sinks[row % H] - M);
   const float wz = L > 0.f ? ez / L : 0.f;
-  const long tok = qstart[s] + tok0 + row / H;
+  const long tok = q0 + tok0 + row / H;
   const int h = row % H;
-  const float* po = part_o + r * splits * rank;
   for (int c0 = 0; c0 < rank; c0 += 256) {     // every lane stays in the loop: the shuffles read all lanes
     const int c = c0 + tid;
     const bool on = c < rank;
     float o = 0.f;
+    int z0 = 0;
+    if (c0 == 0) {
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) {
+        const float w = __shfl(wz, z, 64);
+        if (w != 0.f) o += first[z] * w;       // a split that saw no key left nothing to read
+      }
+      z0 = min(splits, NZ);
+    }
 #pragma unroll 8
-    for (int z = 0; z < splits; ++z) {
+    for (int z = z0; z < splits; ++z) {
       const float w = __shfl(wz, z, 64);
-      if (on && w != 0.f) o += po[(long)z * rank + c] * w;     // a split that saw no key left nothing to read
+      if (on && w != 0.f) o += po[(long)z * rank + c] * w;
     }
     if (on) stf(out + ((long)h * Ttot + tok) * rank + c, o);
   }
