@@ -114,7 +114,7 @@ int dllm_gqa_tile_tokens(int, int, int);
 int dllm_gqa_mfma_ok(int, int, int, int, int, int);
 int dllm_paged_gqa(const void*, const void*, const void*, int, const int*, int, int, const int*, const int*, const int*,
                    const int*, const int*, int, const void*, long, void*, int, int, int, int, int, int, float*, int, int, int,
-                   int, float, int, float, const float*, long, const float*, int, hipStream_t);
+                   int, float, int, float, const float*, long, const float*, int, long, hipStream_t);
 int dllm_rope_prep(const void*, long, int, int, int, int, int, const float*, int, int, float, const int*, const int*, void*, void*,
                    void*, long, int, int, int, void*, long, void*, long, int, const float*, const float*, hipStream_t);
 int dllm_latent_prep(const void*, long, int, int, int, const float*, float, const int*, void*, int, int, void*, long, void*, int,
@@ -2089,7 +2089,7 @@ void paged_gqa_attention(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, to
                                 tile_seq.data_ptr<int>(), tile_tok0.data_ptr<int>(), (int)tile_seq.numel(), gp, ldg,
                                 out.data_ptr(), (int)H, (int)G, (int)d, (int)dv, (int)mfma, (int)splits, pptr, (int)window,
                                 (int)GV, (int)of32, (int)keep_first, (float)sink, (int)chunk, (float)cap, sk,
-                                (long)out.stride(0), sl, (int)ghead, stream());
+                                (long)out.stride(0), sl, (int)ghead, (long)T, stream());
   TORCH_CHECK(rc != -2, "head widths do not fit the LDS");
   ok(rc, "paged_gqa_attention");
 }

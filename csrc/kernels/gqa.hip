@@ -1043,6 +1043,188 @@ __global__ void __launch_bounds__(256) paged_gqa_mfma_kernel(const u16* __restri
   }
 }
 
+// The same for few rows a tile (decode steps: a token's R <= 16 heads): there paged_gqa_mfma has one wave of four with live rows, which
+// walks every tile of its split behind two barriers (3 us a tile).  Here each wave takes 32-key chunks of its own and keeps its own
+// maximum, sum and O^T; keys and values come from the pages straight to registers, the next chunk's while this one is multiplied, and
+// no barrier stands before the waves meet at the end.  S^T = K . Q^T leaves a head's scores in one lane column, P^T feeds
+// O^T = V^T . P^T with the key order 8 g + j <-> j < 4 ? 4 g + j : 16 + 4 g + j - 4 (two 8-byte loads of V^T's pages); p = hi + lo as
+// above.  With splits 16, merge included: four sequences of 1300, 8 heads of 64 with slopes 19 -> 13 us; six of 2600, 8 splits 28 -> 19.
+// More than 16 rows (a tile of a short portion) are walked 16 at a time.
+template <int KD, int VD, bool CAP, bool DIST>
+__global__ void __launch_bounds__(256) gqa_few_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
+                                                      const int* __restrict__ bt, int bt_ld, const int* __restrict__ qstart,
+                                                      const int* __restrict__ qlen, const int* __restrict__ ctx,
+                                                      const int* __restrict__ tile_seq, const int* __restrict__ tile_tok0,
+                                                      const u16* __restrict__ gate, long ldg, u16* __restrict__ out, int H, int G, int d,
+                                                      int dv, int TQ, int splits, float* __restrict__ part, int win, int keep,
+                                                      float sink, int chunk, float cap, const float* __restrict__ sinks, long ldo,
+                                                      const float* __restrict__ slopes, int ghead) {
+  constexpr int KU = KD / 32, VB = VD / 16;
+  __shared__ __attribute__((aligned(16))) f32x4 Om[4][VB * 64];
+  __shared__ float ml[4][2][16];
+  const int g = blockIdx.x % G, tile = blockIdx.x / G;
+  const int s = tile_seq[tile], tok0 = tile_tok0[tile];
+  const int n = qlen[s], q0 = qstart[s], p0 = ctx[s] - n;
+  if (n <= 0 || tok0 >= n) return;   // the whole workgroup (padding tiles)
+  const int R = H / G, nq = min(TQ, n - tok0), nrows = nq * R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g4 = lane >> 4;
+  const int last = p0 + tok0 + nq - 1;   // the newest key any row sees
+  const int* btr = bt + (long)s * bt_ld;
+  const float cap2 = cap > 0.f ? (CAP ? 2.88539008f : 2.f) / cap : 0.f, capl = 1.44269504f * cap;
+  // the walk over tiles of 64 keys and its splits: as in paged_gqa_mfma
+  const int tfirst = oldest_key(p0 + tok0, win, chunk) / GM_KT, nkeep = min(tfirst, (keep + GM_KT - 1) / GM_KT);
+  const int ntiles = last / GM_KT + 1 - tfirst + nkeep;
+  const int vbeg = (int)((long)ntiles * blockIdx.z / splits), nch = 2 * ((int)((long)ntiles * (blockIdx.z + 1) / splits) - vbeg);
+  auto key0 = [&](int c) { const int v = vbeg + (c >> 1); return (v < nkeep ? v : tfirst + v - nkeep) * GM_KT + 32 * (c & 1); };
+  struct Pages { int a, b; };
+  auto pages = [&](int c) {
+    Pages pg{0, 0};
+    if (c < nch) {
+      const int k0 = key0(c);
+      if (k0 <= last) pg.a = btr[k0 >> 4];
+      if (k0 + 16 <= last) pg.b = btr[(k0 >> 4) + 1];
+    }
+    return pg;
+  };
+  const u16* kl = kc + ((long)g * GM_BS + lr) * d + 8 * g4;
+  const u16* vl = vc + ((long)g * dv + lr) * GM_BS + 4 * g4;
+  const long kpage = (long)G * GM_BS * d, vpage = (long)G * dv * GM_BS;
+  struct Keys { uint4 k[2][KU]; uint2 v[2][VB]; };
+  auto load = [&](Keys& x, int c, Pages pg) {      // pages past the last key read as zeros
+    const int k0 = key0(c);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bool on = k0 + 16 * t <= last;
+      const long page = t ? pg.b : pg.a;
+#pragma unroll
+      for (int u = 0; u < KU; ++u) x.k[t][u] = on && 32 * u + 8 * g4 < d ? ld16(kl + page * kpage + 32 * u) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int b = 0; b < VB; ++b)
+        x.v[t][b] = on && 16 * b + lr < dv ? *reinterpret_cast<const uint2*>(vl + page * vpage + 16 * b * GM_BS) : make_uint2(0u, 0u);
+    }
+  };
+  for (int rb = 0; rb < nrows; rb += 16) {
+    const int row = rb + lr;
+    const bool live = row < nrows;
+    const int tl = live ? row / R : 0, h = g * R + (live ? row % R : 0);
+    const int rpos = live ? p0 + tok0 + tl : -1, rlo = live ? oldest_key(rpos, win, chunk) : 0;
+    const float slp = DIST && live ? slopes[h] : 0.f;
+    const long tok = q0 + tok0 + tl;
+    Pages pg = pages(wave);
+    bf16x8 qf[KU];
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+      qf[u] = __builtin_bit_cast(bf16x8, live && 32 * u + 8 * g4 < d ? ld16(q + (tok * H + h) * d + 32 * u + 8 * g4) : make_uint4(0u, 0u, 0u, 0u));
+    float m = CAP ? 0.f : -INFINITY, l = 0.f;
+    f32x4 O[VB];
+#pragma unroll
+    for (int b = 0; b < VB; ++b) O[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Keys cur, nxt;
+    if (wave < nch) load(cur, wave, pg);
+    pg = pages(wave + 4);
+    for (int c = wave; c < nch; c += 4) {
+      if (c + 4 < nch) load(nxt, c + 4, pg);
+      pg = pages(c + 8);
+      const int k0 = key0(c);
+      float p[8];
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (DIST)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[i] = slp * (float)(k0 + 16 * t + 4 * g4 + i - rpos);
+#pragma unroll
+        for (int u = 0; u < KU; ++u) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, cur.k[t][u]), qf[u], sc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v = sc[i];
+          if (!CAP && !DIST && cap > 0.f) v = cap_fast(v, cap, cap2);
+          if constexpr (CAP) v = capl - 2.f * capl * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap2) + 1.f);
+          const int key = k0 + 16 * t + 4 * g4 + i;
+          const bool vis = (key <= rpos) & ((key >= rlo) | (key < keep));
+          v = vis ? v : -INFINITY;
+          p[4 * t + i] = v;
+          mx = fmaxf(mx, v);
+        }
+      }
+      float alpha = 1.f;
+      if constexpr (CAP) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(p[j]);   // 0 for masked keys
+      } else {
+        mx = lane_max(mx, 16);
+        mx = lane_max(mx, 32);
+        const float mn = fmaxf(m, mx);
+        const bool any = mn > -INFINITY;
+        alpha = any ? __expf(m - mn) : 1.f;   // m = -inf before the first visible key: 0, and O, l are 0
+        m = mn;
+        l *= alpha;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = any ? __expf(p[j] - mn) : 0.f;
+#pragma unroll
+        for (int b = 0; b < VB; ++b) O[b] *= alpha;
+      }
+      float lo[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        l += p[j];
+        lo[j] = p[j] - bf2f(f2bf(p[j]));
+      }
+      const bf16x8 ph = __builtin_bit_cast(bf16x8, pack8(p)), pl = __builtin_bit_cast(bf16x8, pack8(lo));
+#pragma unroll
+      for (int b = 0; b < VB; ++b) {
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, make_uint4(cur.v[0][b].x, cur.v[0][b].y, cur.v[1][b].x, cur.v[1][b].y));
+        O[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, ph, O[b], 0, 0, 0);
+        O[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, O[b], 0, 0, 0);
+      }
+      cur = nxt;
+    }
+    l = lane_add(l, 16);
+    l = lane_add(l, 32);
+    if (g4 == 0) { ml[wave][0][lr] = m; ml[wave][1][lr] = l; }
+#pragma unroll
+    for (int b = 0; b < VB; ++b) Om[wave][b * 64 + lane] = O[b];
+    __syncthreads();
+    float M = ml[0][0][lr], L = 0.f, f[4];
+#pragma unroll
+    for (int x = 1; x < 4; ++x) M = fmaxf(M, ml[x][0][lr]);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      f[x] = CAP ? 1.f : ml[x][0][lr] > -INFINITY ? __expf(ml[x][0][lr] - M) : 0.f;
+      L += ml[x][1][lr] * f[x];
+    }
+    if (live) {
+      float* pr = part ? part + ((((long)tile * G + g) * splits + blockIdx.z) * GM_ROWS + row) * (dv + 2) : nullptr;
+      if (pr && wave == 0 && g4 == 0) { pr[0] = M; pr[1] = L; }
+      float inv = 1.f;
+      if (!pr) {
+        inv = 1.f / (L + (sinks ? __expf(sinks[h] - M) : sink > 0.f ? sink * __expf(-M) : 0.f));
+        if (gate && ghead) inv *= 1.f / (1.f + expf(-bf2f(gate[tok * ldg + h])));
+      }
+#pragma unroll
+      for (int y = 0; y < (VB + 3) / 4; ++y) {
+        const int b = wave + 4 * y;
+        if (b >= VB) break;
+        const f32x4 o = (Om[0][b * 64 + lane] * f[0] + Om[1][b * 64 + lane] * f[1]) + (Om[2][b * 64 + lane] * f[2] + Om[3][b * 64 + lane] * f[3]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = 16 * b + 4 * g4 + i;
+          if (j >= dv) continue;
+          if (pr) {
+            pr[2 + j] = o[i];
+            continue;
+          }
+          float v = o[i] * inv;
+          if (gate && !ghead) v *= 1.f / (1.f + expf(-bf2f(gate[tok * ldg + (long)h * dv + j])));
+          out[tok * ldo + (long)h * dv + j] = f2bf(v);
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // merge the key splits of paged_gqa_mfma: one wave per (tile, kv head, row)
 __global__ void __launch_bounds__(256) gqa_combine_kernel(const float* __restrict__ part, int splits,
                                                           const int* __restrict__ qstart, const int* __restrict__ qlen,
@@ -1194,7 +1376,7 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
                               const int* qstart, const int* qlen, const int* ctx, const int* tile_seq, const int* tile_tok0,
                               int n_tiles, const void* gate, long ldg, void* out, int H, int G, int d, int dv, int mfma,
                               int splits, float* part, int win, int GV, int out_f32, int keep, float sink, int chunk, float cap,
-                              const float* sinks, long ldo, const float* slopes, int ghead, hipStream_t st) {
+                              const float* sinks, long ldo, const float* slopes, int ghead, long T, hipStream_t st) {
   if (n_tiles <= 0) return 0;
   if (slopes && cap > 0.f) return -1;
   if (chunk < 0 || (chunk > 0 && win > 0) || cap < 0.f || ldo < (long)H * dv) return -1;
@@ -1207,7 +1389,7 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
     const dim3 grid((unsigned)n_tiles * G, 1, splits);
     const int TQ = dllm_gqa_tile_tokens(H, G, 1);
     float* pp = splits > 1 ? part : nullptr;
-#define GQM(KD, VD, CAP, DIST)                                                                                           \
+#define GQT(KD, VD, CAP, DIST)                                                                                           \
   do {                                                                                                                   \
     const long lds = gqa_mfma_lds(KD, VD);                                                                               \
     ENSURE_LDS((paged_gqa_mfma_kernel<KD, VD, CAP, DIST>), lds);                                                         \
@@ -1220,17 +1402,34 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
     // of their own, so that the extra dims do not widen the value side
 #define GQZ(CAP, DIST)                                                                                                   \
   do {                                                                                                                   \
-    if (d <= 64 && dv <= 64) GQM(64, 64, CAP, DIST);                                                                     \
-    else if (d <= 96 && dv <= 64) GQM(96, 64, CAP, DIST);                                                                \
-    else if (d <= 128 && dv <= 128) GQM(128, 128, CAP, DIST);                                                            \
-    else if (d <= 192 && dv <= 128) GQM(192, 128, CAP, DIST);                                                            \
-    else GQM(256, 256, CAP, DIST);                                                                                       \
+    if (d <= 64 && dv <= 64) GQT(64, 64, CAP, DIST);                                                                     \
+    else if (d <= 96 && dv <= 64) GQT(96, 64, CAP, DIST);                                                                \
+    else if (d <= 128 && dv <= 128) GQT(128, 128, CAP, DIST);                                                            \
+    else if (d <= 192 && dv <= 128) GQT(192, 128, CAP, DIST);                                                            \
+    else GQT(256, 256, CAP, DIST);                                                                                       \
   } while (0)
-    if (cap > 0.f && cap <= CAP_MAX) GQZ(true, false);
+    // at most 16 rows a tile on average: decode steps.  Not where key heads share their values or the result is f32: those are the maps
+    // of differential attention, whose difference keeps the order of sums of paged_gqa_mfma
+    if (GV == G && !out32 && d <= 128 && dv <= 128 && T * (H / G) <= 16L * n_tiles) {
+#define GQM(KD, VD, CAP, DIST)                                                                                                   \
+  hipLaunchKernelGGL((gqa_few_kernel<KD, VD, CAP, DIST>), grid, dim3(256), 0, st, (const u16*)q, (const u16*)kc, (const u16*)vc, bt, \
+                     bt_ld, qstart, qlen, ctx, tile_seq, tile_tok0, (const u16*)gate, ldg, (u16*)out, H, G, d, dv, TQ, splits, pp, win, keep, \
+                     sink, chunk, cap, sinks, ldo, slopes, ghead)
+#define GQF(CAP, DIST)                                 \
+  do {                                                 \
+    if (d <= 64 && dv <= 64) GQM(64, 64, CAP, DIST);   \
+    else GQM(128, 128, CAP, DIST);                     \
+  } while (0)
+      if (cap > 0.f && cap <= CAP_MAX) GQF(true, false);
+      else if (slopes) GQF(false, true);
+      else GQF(false, false);
+#undef GQF
+#undef GQM
+    } else if (cap > 0.f && cap <= CAP_MAX) GQZ(true, false);
     else if (slopes) GQZ(false, true);
     else GQZ(false, false);
 #undef GQZ
-#undef GQM
+#undef GQT
     if (pp) {
       const int rows = (TQ * (H / G) < GM_ROWS ? TQ * (H / G) : GM_ROWS);
       hipLaunchKernelGGL(gqa_combine_kernel, dim3(n_tiles, G, (rows + 3) / 4), dim3(256), 0, st, pp, splits, qstart, qlen,

@@ -890,3 +890,35 @@ def test_gelu_in_vectors(n):
     """Bits of the element-by-element form (an odd offset), one vector, a block of them and more than the grid holds."""
     x = (torch.randn(n + 1, device=DEV) * 3).bfloat16()
     assert torch.equal(seqmix.gelu_erf(x[1:].clone()), seqmix.gelu_erf(x)[1:])
+
+
+@pytest.mark.parametrize("splits", [1, 3, 16])
+@pytest.mark.parametrize("H,G,d,dv", [(4, 4, 64, 64), (16, 1, 64, 64), (24, 2, 96, 64), (8, 2, 128, 128), (6, 3, 40, 72)])
+@pytest.mark.parametrize("opts", [{}, {"window": 40}, {"window": 100, "keep_first": 20, "sink": 0.5}, {"chunk": 64}, {"softcap": 5.0},
+                                  {"softcap": 200.0}, {"slopes": True}, {"sinks": True, "gate": True}, {"gate": "head"}])
+def test_gqa_of_few_rows(H, G, d, dv, splits, opts):
+    """Decode steps (the form that keeps keys and values in registers) against the tile form, which f32 results take: contexts that end at
+    and around pages, chunks and tiles, one tile of two tokens (more than 16 rows at 12 heads a group), heads past 16-wide blocks, splits without keys.  Both sum
+    hi + lo weights in f32, in another order: 2^-8 of a value for the rounding to bf16 and 2^-14 of the largest for the sums and the
+    exponentials' last bits."""
+    from distributed_llm_amd.models.llama import AttnMeta
+    torch.manual_seed(8)
+    dt = torch.bfloat16
+    case = ([1] * 10 + [1 if H // G == 16 else 2], [0, 14, 15, 16, 30, 31, 63, 64, 95, 299, 127])
+    T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
+    q = (torch.randn(T, H, d, device=DEV) * 0.5).to(dt)
+    kw = dict(opts)
+    gate = kw.pop("gate", None)
+    if gate is not None:
+        gate = torch.randn(T, H if gate == "head" else H * dv, device=DEV).to(dt)
+    for name in ("slopes", "sinks"):
+        if kw.pop(name, None):
+            kw[name] = torch.rand(H, device=DEV) + 0.1
+    meta = AttnMeta(slots=None, block_tables=bt, qstart=qstart, qlen=qlen, ctx=ctx, tile_seq=None, tile_tok0=None,
+                    last_idx=None, host_qlen=case[0])
+    ts, tt = meta.latent_tiles(1, DEV, seqmix.gqa_tokens_per_tile(H, G, True))
+    assert T * (H // G) <= 16 * ts.numel()
+    run = lambda f32: seqmix.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, ts, tt, gate, True, splits, out_f32=f32, **kw).float()  # noqa: E731
+    got, want = run(False), run(True)
+    assert torch.isfinite(want).all()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * want.abs().max()).all()
