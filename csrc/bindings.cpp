@@ -118,7 +118,7 @@ int dllm_paged_gqa(const void*, const void*, const void*, int, const int*, int, 
 int dllm_rope_prep(const void*, long, int, int, int, int, int, const float*, int, int, float, const int*, const int*, void*, void*,
                    void*, long, int, int, int, void*, long, void*, long, int, const float*, const float*, hipStream_t);
 int dllm_latent_prep(const void*, long, int, int, int, const float*, float, const int*, void*, int, int, void*, long, void*, int,
-                     float, void*, int, long, hipStream_t);
+                     float, void*, int, int, long, long, long, hipStream_t);
 int dllm_latent_expand_ok(int, int, int, int);
 int dllm_latent_expand(const void*, const int*, int, int, int, int, const int*, int, int, int, int, const void*, const void*, void*,
                        void*, int, hipStream_t);
@@ -128,10 +128,10 @@ int dllm_scaled_resadd_rms(const void*, long, int, float, int, const float*, flo
 int dllm_relu2_scale(const void*, int, const float*, int, int, void*, long, int, hipStream_t);
 int dllm_dense_gate(const int*, const float*, float*, long, int, int, hipStream_t);
 int dllm_latent_kv_write(const void*, long, int, int, int, const float*, float, const int*, const float*, int, const int*,
-                         void*, int, int, const void*, long, int, const float*, void*, void*, int, hipStream_t);
+                         void*, int, int, const void*, long, int, const float*, void*, void*, int, int, long, long, hipStream_t);
 int dllm_latent_attention(const void*, const void*, long, int, int, int, int, int, long, const float*, int, const void*,
                           const int*, int, const int*, const int*, const int*, const int*, const int*, int, float, void*,
-                          int, float*, float*, int, int, int, const float*, hipStream_t);
+                          int, float*, float*, int, int, int, const float*, const void*, int, const void*, long, int, void*, long, hipStream_t);
 int dllm_latent_mfma_ok(int, int, int);
 int dllm_car_alloc(long, void**);
 int dllm_car_get_handle(void*, char*);
@@ -2188,17 +2188,20 @@ void latent_prep(torch::Tensor proj, int64_t ccol, torch::Tensor w, double eps, 
     qp = q->data_ptr();
   }
   void* zp = nullptr;
-  int64_t zh = 0;
+  int64_t zh = 0, zc = 0, zn = 0, zt = 0;
   if (zero) {
-    TORCH_CHECK(zero->is_cuda() && zero->scalar_type() == proj.scalar_type() && zero->is_contiguous() && zero->dim() == 3 &&
-                    zero->size(1) == T && zero->size(2) == rank,
-                "zero [H, T, rank] in the activations' dtype");
+    TORCH_CHECK(zero->is_cuda() && zero->scalar_type() == proj.scalar_type() && zero->dim() == 3 && zero->size(1) == T &&
+                    zero->stride(2) == 1 && zero->size(0) * zero->size(2) < (1 << 30),
+                "zero [n, T, c] of unit column stride in the activations' dtype");
     zh = zero->size(0);
+    zc = zero->size(2);
+    zn = zero->stride(0);
+    zt = zero->stride(1);
     zp = zero->data_ptr();
   }
   ok(dllm_latent_prep(proj.data_ptr(), proj.stride(0), f, (int)ccol, (int)rank, w.data_ptr<float>(), (float)eps,
                       slots.data_ptr<int>(), cache.data_ptr(), (int)ucol, (int)ff, ap, lda, qp, (int)nq, (float)qscale, zp, (int)zh,
-                      (long)T, stream()),
+                      (int)zc, (long)zn, (long)zt, (long)T, stream()),
      "latent_prep");
 }
 
@@ -2690,7 +2693,7 @@ void latent_kv_write(torch::Tensor ckv, int64_t rank, torch::Tensor w, double ep
   const float* qw = nullptr;
   void *qd = nullptr, *zp = nullptr;
   long ldqs = 0;
-  int64_t qn = 0, zh = 0;
+  int64_t qn = 0, zh = 0, zc = 0, zn = 0, zt = 0;
   if (q_src) {
     TORCH_CHECK(q_norm && q_out, "a query latent needs its norm weight and its output");
     qn = q_src->size(1);
@@ -2704,15 +2707,18 @@ void latent_kv_write(torch::Tensor ckv, int64_t rank, torch::Tensor w, double ep
     qd = q_out->data_ptr();
   }
   if (zero) {
-    TORCH_CHECK(zero->is_cuda() && zero->scalar_type() == ckv.scalar_type() && zero->is_contiguous() && zero->dim() == 3 &&
-                    zero->size(1) == T && zero->size(2) == rank,
-                "zero [H, T, rank] in the activations' dtype");
+    TORCH_CHECK(zero->is_cuda() && zero->scalar_type() == ckv.scalar_type() && zero->dim() == 3 && zero->size(1) == T &&
+                    zero->stride(2) == 1 && zero->size(0) * zero->size(2) < (1 << 30),
+                "zero [n, T, c] of unit column stride in the activations' dtype");
     zh = zero->size(0);
+    zc = zero->size(2);
+    zn = zero->stride(0);
+    zt = zero->stride(1);
     zp = zero->data_ptr();
   }
   ok(dllm_latent_kv_write(ckv.data_ptr(), ckv.stride(0), f, (int)rank, (int)rot, w.data_ptr<float>(), (float)eps,
                           pos.data_ptr<int>(), cos_sin.data_ptr<float>(), (int)cos_sin.size(1), slots.data_ptr<int>(),
-                          cache.data_ptr(), T, (int)half, qs, ldqs, (int)qn, qw, qd, zp, (int)zh, stream()),
+                          cache.data_ptr(), T, (int)half, qs, ldqs, (int)qn, qw, qd, zp, (int)zh, (int)zc, (long)zn, (long)zt, stream()),
      "latent_kv_write");
 }
 
@@ -2736,7 +2742,8 @@ void latent_attention(torch::Tensor qa, torch::Tensor q, int64_t dim, int64_t ro
                       torch::Tensor cache, torch::Tensor bt, torch::Tensor qstart, torch::Tensor qlen, torch::Tensor ctx,
                       torch::Tensor tile_seq, torch::Tensor tile_tok0, double scale, torch::Tensor out, int64_t splits,
                       c10::optional<torch::Tensor> part_o, c10::optional<torch::Tensor> part_ml, bool mfma,
-                      int64_t rows, bool half, c10::optional<torch::Tensor> sinks) {
+                      int64_t rows, bool half, c10::optional<torch::Tensor> sinks, c10::optional<torch::Tensor> up_w,
+                      c10::optional<torch::Tensor> gate, c10::optional<torch::Tensor> up_out) {
   const bool f = act_f32(qa, "qa");
   TORCH_CHECK(rows == 16 || (rows == 32 && mfma && !f && dllm_latent_mfma_ok((int)qa.size(2), (int)rot, 32)),
               "rows per workgroup: 16, or 32 where the matrix-core kernel takes the shape");
@@ -2775,11 +2782,31 @@ void latent_attention(torch::Tensor qa, torch::Tensor q, int64_t dim, int64_t ro
     po = part_o->data_ptr<float>();
     pml = part_ml->data_ptr<float>();
   }
+  // value up-projection and gate in the merging launch: up_w [H, rank, dv], gate [T, H dv] or [T, H], up_out [T, H dv] instead of out
+  const void* gp = nullptr;
+  long ldg = 0;
+  int64_t dv = 0;
+  if (up_w) {
+    TORCH_CHECK(!f && mfma && splits > 1 && up_out, "value up-projection: bf16, matrix-core kernel, key splits, an output");
+    check_bf16(*up_w, "up_w");
+    check_bf16(*up_out, "up_out");
+    TORCH_CHECK(up_w->dim() == 3 && up_w->is_contiguous() && up_w->size(0) == H && up_w->size(1) == rank, "up_w [H, rank, dv]");
+    dv = up_w->size(2);
+    TORCH_CHECK(up_out->dim() == 2 && up_out->stride(1) == 1 && up_out->size(0) == T && up_out->size(1) == H * dv, "up_out [T, H dv]");
+    if (gate) {
+      check_bf16(*gate, "gate");
+      TORCH_CHECK(gate->dim() == 2 && gate->size(0) == T && gate->stride(1) == 1 && (gate->size(1) == H * dv || gate->size(1) == H), "gate [T, H dv] or [T, H]");
+      gp = gate->data_ptr();
+      ldg = gate->stride(0);
+    }
+  }
   ok(dllm_latent_attention(qa.data_ptr(), q.data_ptr(), q.stride(0), f, (int)H, (int)dim, (int)rot, (int)rank, T,
                            cos_sin.data_ptr<float>(), (int)cos_sin.size(1), cache.data_ptr(), bt.data_ptr<int>(),
                            (int)bt.size(1), qstart.data_ptr<int>(), qlen.data_ptr<int>(), ctx.data_ptr<int>(),
                            tile_seq.data_ptr<int>(), tile_tok0.data_ptr<int>(), (int)tile_seq.numel(), (float)scale,
-                           out.data_ptr(), (int)splits, po, pml, mfma ? 1 : 0, (int)rows, (int)half, sk, stream()),
+                           out.data_ptr(), (int)splits, po, pml, mfma ? 1 : 0, (int)rows, (int)half, sk,
+                           up_w ? up_w->data_ptr() : nullptr, (int)dv, gp, ldg, gate && gate->size(1) == H && dv != 1, up_w ? up_out->data_ptr() : nullptr,
+                           up_w ? (long)up_out->stride(0) : 0, stream()),
      "latent_attention");
 }
 }  // namespace
@@ -2852,7 +2879,8 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("positions"), py::arg("cos_sin"), py::arg("cache"), py::arg("block_tables"), py::arg("qstart"),
         py::arg("qlen"), py::arg("ctx"), py::arg("tile_seq"), py::arg("tile_tok0"), py::arg("scale"), py::arg("out"),
         py::arg("splits") = 1, py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("mfma") = true,
-        py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none());
+        py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none(), py::arg("up_w") = py::none(),
+        py::arg("gate") = py::none(), py::arg("up_out") = py::none());
   m.def("latent_mfma_ok", [](int64_t rank, int64_t rot, int64_t rows) { return dllm_latent_mfma_ok((int)rank, (int)rot, (int)rows) != 0; });
   m.def("encoder_layers", &encoder_layers);
   m.def("enc_gemm", &enc_gemm);

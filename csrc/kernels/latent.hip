@@ -65,13 +65,13 @@ __global__ void __launch_bounds__(256) latent_kv_write_kernel(const T* __restric
                                                               const int* __restrict__ slots, T* __restrict__ cache, int hf,
                                                               const T* __restrict__ qsrc, long ldqs, int qn,
                                                               const float* __restrict__ qw, T* __restrict__ qdst,
-                                                              T* __restrict__ zl, int zh) {
+                                                              T* __restrict__ zl, int zh, int zc, long zn, long zt) {
   constexpr int NR = 8;      // values a lane keeps
   __shared__ float red[3];
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int slot = slots[t];
   if (zl && slot < 0)
-    for (int i = threadIdx.x; i < zh * rank; i += blockDim.x) stf(zl + ((long)(i / rank) * gridDim.x + t) * rank + i % rank, 0.f);
+    for (int i = threadIdx.x; i < zh * zc; i += blockDim.x) stf(zl + i / zc * zn + t * zt + i % zc, 0.f);
   const bool is_q = wave > 0;
   const T* r = is_q ? qsrc + (long)t * ldqs : ckv + (long)t * ld;
   const int n = is_q ? qn : rank, i0 = is_q ? threadIdx.x - 64 : lane, step = is_q ? 192 : 64;
@@ -159,16 +159,16 @@ __global__ void __launch_bounds__(256) latent_prep_kernel(const T* __restrict__ 
                                                           const float* __restrict__ w, float eps,
                                                           const int* __restrict__ slots, T* __restrict__ cache, int ucol,
                                                           int ff, T* __restrict__ act, long lda, int vec,
-                                                          T* __restrict__ q, int nq, float qscale, T* __restrict__ zl, int zh) {
+                                                          T* __restrict__ q, int nq, float qscale, T* __restrict__ zl, int zh, int zc,
+                                                          long zn, long zt) {
   // q (optional): the row's first nq columns times qscale, as rows of a matrix of their own
   const long tok = blockIdx.x;
   const int tid = threadIdx.x;
   const T* row = proj + tok * ld;
   const int slot = slots[tok];
-  // zl (optional, [H, T, rank]): a padding token's rows, which no attention tile writes, are cleared
+  // zl (optional, [zh, T, zc], strides zn, zt): a padding token's rows, which no attention tile writes, are cleared
   if (zl && slot < 0)
-    for (int i = blockIdx.y * 256 + tid; i < zh * rank; i += gridDim.y * 256)
-      stf(zl + ((long)(i / rank) * gridDim.x + tok) * rank + i % rank, 0.f);
+    for (int i = blockIdx.y * 256 + tid; i < zh * zc; i += gridDim.y * 256) stf(zl + i / zc * zn + tok * zt + i % zc, 0.f);
   if (blockIdx.y == 0 && tid < 64 && slot >= 0) {
     const T* r = row + ccol;
     float s = 0.f;
@@ -976,21 +976,109 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
   }
 }
 
+// latent_combine, the head's value up-projection and its gate in one launch, for steps of few tokens: a workgroup merges a (token,
+// head) row's splits, rounds it to bf16 and multiplies it with the head's W [rank, 8 NV], a thread NV-th of the columns and some of
+// the ranks; weights, partials and gate are all asked for at the start.  As launches of their own the batched product of the vendor's
+// library and the gate cost 5 and 4.6 us beside the merge's 4.9 (four tokens, 16 heads, 256 -> 64): Filevik's
+// batch of 24 10.3 -> 9.85 ms, Figotar's of four 12.6 -> 12.4.  Past 64 tokens the
+// re-read weights (32 KB a row) weigh more than the launches.
+struct LatUp { const u16 *w, *gate; long ldg; int dv, ghead; u16* out; long ldo; };      // w null: none
+template <int NV>
+__global__ void __launch_bounds__(256) latent_up_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, int splits,
+                                                        int gx, int H, int rank, const int* __restrict__ qstart,
+                                                        const int* __restrict__ qlen, const int* __restrict__ tile_seq,
+                                                        const int* __restrict__ tile_tok0, int tpe, int rpb,
+                                                        const float* __restrict__ sinks, const u16* __restrict__ W,
+                                                        const u16* __restrict__ gate, long ldg, int ghead, u16* __restrict__ out,
+                                                        long ldo) {
+  constexpr int NZ = 16, DV = 8 * NV, NG = 256 / NV, NW = 8;     // NG ranks at a time
+  __shared__ float lat[512], red[4][DV];
+  const long r = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const long eb = r / rpb;
+  const int bx = (int)(eb % gx), entry = (int)(eb / gx), row = bx * rpb + (int)(r % rpb), h = row % H;
+  const float* ml = part_ml + 2 * r * splits;
+  const float* po = part_o + r * splits * rank;
+  const float mz = lane < splits ? ml[2 * lane] : -INFINITY, lz = lane < splits ? ml[2 * lane + 1] : 0.f;
+  float first[NZ];
+#pragma unroll
+  for (int z = 0; z < NZ; ++z) first[z] = z < splits && tid < rank ? po[(long)z * rank + tid] : 0.f;
+  const u16* wp = W + (long)h * rank * DV + tid % NV * 8;
+  const int k0 = tid / NV;
+  uint4 wv[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) wv[i] = k0 + NG * i < rank ? ld16(wp + (long)(k0 + NG * i) * DV) : make_uint4(0, 0, 0, 0);
+  const int s = tile_seq[entry];
+  const int n = qlen[s], tok0 = tile_tok0[entry], q0 = qstart[s];
+  if (n <= 0 || tok0 >= n || row >= min(tpe, n - tok0) * H) return;      // the whole workgroup
+  const long tok = q0 + tok0 + row / H;
+  const float gv = gate && tid < DV ? bf2f(gate[tok * ldg + (ghead ? h : h * DV + tid)]) : 0.f;
+  const float M = wave_max(mz);
+  const float ez = mz > -INFINITY ? expf(mz - M) : 0.f;
+  float L = wave_sum(lz * ez);
+  if (sinks && L > 0.f) L += expf(sinks[h] - M);
+  const float wz = L > 0.f ? ez / L : 0.f;
+  for (int c0 = 0; c0 < rank; c0 += 256) {     // every lane stays in the loop: the shuffles read all lanes
+    const int c = c0 + tid;
+    float o = 0.f;
+    int z0 = 0;
+    if (c0 == 0) {
+#pragma unroll
+      for (int z = 0; z < NZ; ++z) {
+        const float w = __shfl(wz, z, 64);
+        if (w != 0.f) o += first[z] * w;       // a split that saw no key left nothing to read
+      }
+      z0 = min(splits, NZ);
+    }
+#pragma unroll 8
+    for (int z = z0; z < splits; ++z) {
+      const float w = __shfl(wz, z, 64);
+      if (c < rank && w != 0.f) o += po[(long)z * rank + c] * w;
+    }
+    if (c < rank) lat[c] = bf2f(f2bf(o));
+  }
+  __syncthreads();
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto add = [&](uint4 w, int k) {
+    float f[8];
+    unpack8(w, f);
+    const float x = lat[k];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += x * f[j];
+  };
+#pragma unroll
+  for (int i = 0; i < NW; ++i)
+    if (k0 + NG * i < rank) add(wv[i], k0 + NG * i);
+  for (int k = k0 + NG * NW; k < rank; k += NG) add(ld16(wp + (long)k * DV), k);
+#pragma unroll
+  for (int o = 32; o >= NV; o >>= 1)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = lane_add(acc[j], o);
+  if (lane < NV)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) red[tid >> 6][8 * lane + j] = acc[j];
+  __syncthreads();
+  if (tid >= DV) return;
+  float v = bf2f(f2bf((red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid])));
+  if (gate) v *= ghead ? 1.f / (1.f + __expf(-gv)) : __builtin_amdgcn_rcpf(1.f + __expf(-gv));      // gate_heads' arithmetic
+  out[tok * ldo + (long)h * DV + tid] = f2bf(v);
+}
+
 }  // namespace
 
 extern "C" int dllm_latent_kv_write(const void* ckv, long ld, int f32, int rank, int rot, const float* w, float eps,
                                     const int* pos, const float* cos_sin, int tab_w, const int* slots, void* cache,
                                     int T, int hf, const void* qsrc, long ldqs, int qn, const float* qw, void* qdst, void* zl,
-                                    int zh, hipStream_t st) {
+                                    int zh, int zc, long zn, long zt, hipStream_t st) {
   if (T <= 0) return 0;
   if (rot < 0 || (rot & 1) || rot > tab_w || rank < 1 || (qsrc && (qn < 1 || !qw || !qdst))) return -1;
   const dim3 block(qsrc ? 256 : 64);
   if (f32)
     hipLaunchKernelGGL(latent_kv_write_kernel<float>, dim3(T), block, 0, st, (const float*)ckv, ld, rank, rot, w, eps, pos,
-                       cos_sin, tab_w, slots, (float*)cache, hf, (const float*)qsrc, ldqs, qn, qw, (float*)qdst, (float*)zl, zh);
+                       cos_sin, tab_w, slots, (float*)cache, hf, (const float*)qsrc, ldqs, qn, qw, (float*)qdst, (float*)zl, zh, zc, zn, zt);
   else
     hipLaunchKernelGGL(latent_kv_write_kernel<u16>, dim3(T), block, 0, st, (const u16*)ckv, ld, rank, rot, w, eps, pos,
-                       cos_sin, tab_w, slots, (u16*)cache, hf, (const u16*)qsrc, ldqs, qn, qw, (u16*)qdst, (u16*)zl, zh);
+                       cos_sin, tab_w, slots, (u16*)cache, hf, (const u16*)qsrc, ldqs, qn, qw, (u16*)qdst, (u16*)zl, zh, zc, zn, zt);
   return (int)hipGetLastError();
 }
 
@@ -1049,7 +1137,7 @@ int launch_latent_mfma(dim3 g, hipStream_t st, const u16* qa, const u16* q, long
                        long Ttot, const float* cos_sin, int tab_w, const u16* cache, const int* bt, int bt_w,
                        const int* qstart, const int* qlen, const int* ctx, const int* tile_seq, const int* tile_tok0,
                        float scale, u16* out, int KT, int tpe, int splits, float* part_o, float* part_ml, int rows, int hf,
-                       const float* sinks) {
+                       const float* sinks, const LatUp& up) {
   const MfmaLds L = mfma_lds(rank, rot, KT, rows);
   const int cbs = (L.RB + 3) / 4;
 #define LATM3(CB, KTC, LRC)                                                                                                 \
@@ -1078,7 +1166,15 @@ int launch_latent_mfma(dim3 g, hipStream_t st, const u16* qa, const u16* q, long
 #undef LATM3
   if (splits > 1) {
     const long n_rows = (long)g.y * g.x * rows;
-    hipLaunchKernelGGL(latent_combine_kernel<u16>, dim3((unsigned)n_rows), dim3(256), 0, st, part_o, part_ml, splits, (int)g.x, H,
+#define LATU(NV)                                                                                                               \
+  hipLaunchKernelGGL(latent_up_kernel<NV>, dim3((unsigned)n_rows), dim3(256), 0, st, part_o, part_ml, splits, (int)g.x, H, rank, qstart, \
+                     qlen, tile_seq, tile_tok0, tpe, rows, sinks, up.w, up.gate, up.ldg, up.ghead, up.out, up.ldo)
+    if (up.w && up.dv == 32) LATU(4);
+    else if (up.w && up.dv == 64) LATU(8);
+    else if (up.w) LATU(16);
+    else
+#undef LATU
+      hipLaunchKernelGGL(latent_combine_kernel<u16>, dim3((unsigned)n_rows), dim3(256), 0, st, part_o, part_ml, splits, (int)g.x, H,
                        rank, Ttot, qstart, qlen, tile_seq, tile_tok0, tpe, out, rows, sinks);
   }
   return (int)hipGetLastError();
@@ -1097,8 +1193,13 @@ extern "C" int dllm_latent_attention(const void* qa, const void* q, long ldq, in
                                      int bt_w, const int* qstart, const int* qlen, const int* ctx, const int* tile_seq,
                                      const int* tile_tok0, int n_entries, float scale, void* out, int splits,
                                      float* part_o, float* part_ml, int mfma, int rows, int hf, const float* sinks,
+                                     const void* up_w, int up_dv, const void* gate, long ldg, int ghead, void* up_out, long ldo,
                                      hipStream_t st) {
   if (n_entries <= 0 || Ttot <= 0) return 0;
+  const LatUp up{(const u16*)up_w, (const u16*)gate, ldg, up_dv, ghead, (u16*)up_out, ldo};
+  if (up_w && (!mfma || f32 || splits < 2 || !dllm_latent_mfma_ok(rank, rot, rows) || (up_dv != 32 && up_dv != 64 && up_dv != 128) ||
+               ((uintptr_t)up_w & 15)))
+    return -5;
   if (rank < 1 || rank > 512 || rot < 0 || (rot & 1) || rot > tab_w || H < 1) return -1;
   if (splits < 1 || (splits > 1 && (!part_o || !part_ml))) return -3;
   if (mfma && !f32 && dllm_latent_mfma_ok(rank, rot, rows)) {
@@ -1107,7 +1208,7 @@ extern "C" int dllm_latent_attention(const void* qa, const void* q, long ldq, in
     const dim3 gm((tpe_m * H + rows - 1) / rows, n_entries, splits);
     return launch_latent_mfma(gm, st, (const u16*)qa, (const u16*)q, ldq, H, dim, rot, rank, Ttot, cos_sin, tab_w,
                               (const u16*)cache, bt, bt_w, qstart, qlen, ctx, tile_seq, tile_tok0, scale, (u16*)out, KTm,
-                              tpe_m, splits, part_o, part_ml, rows, hf, sinks);
+                              tpe_m, splits, part_o, part_ml, rows, hf, sinks, up);
   }
   if (rows != LROWS) return -4;   // only the matrix-core kernel has the 32-row form
   // key rows in LDS: an odd stride for 4-byte reads; when the row length is a multiple of 4 a stride
@@ -1133,7 +1234,7 @@ extern "C" int dllm_latent_attention(const void* qa, const void* q, long ldq, in
 
 extern "C" int dllm_latent_prep(const void* proj, long ld, int f32, int ccol, int rank, const float* w, float eps,
                                 const int* slots, void* cache, int ucol, int ff, void* act, long lda, void* q, int nq,
-                                float qscale, void* zl, int zh, long T, hipStream_t st) {
+                                float qscale, void* zl, int zh, int zc, long zn, long zt, long T, hipStream_t st) {
   if (T <= 0) return 0;
   if (rank < 1 || (act && ff < 1)) return -1;
   const dim3 grid((unsigned)T, act ? (ff + 2047) / 2048 : 1);
@@ -1141,10 +1242,10 @@ extern "C" int dllm_latent_prep(const void* proj, long ld, int f32, int ccol, in
                   (uintptr_t)act % 16 == 0;
   if (f32)
     hipLaunchKernelGGL(latent_prep_kernel<float>, grid, dim3(256), 0, st, (const float*)proj, ld, ccol, rank, w, eps, slots,
-                       (float*)cache, ucol, ff, (float*)act, lda, vec, (float*)q, nq, qscale, (float*)zl, zh);
+                       (float*)cache, ucol, ff, (float*)act, lda, vec, (float*)q, nq, qscale, (float*)zl, zh, zc, zn, zt);
   else
     hipLaunchKernelGGL(latent_prep_kernel<u16>, grid, dim3(256), 0, st, (const u16*)proj, ld, ccol, rank, w, eps, slots,
-                       (u16*)cache, ucol, ff, (u16*)act, lda, vec, (u16*)q, nq, qscale, (u16*)zl, zh);
+                       (u16*)cache, ucol, ff, (u16*)act, lda, vec, (u16*)q, nq, qscale, (u16*)zl, zh, zc, zn, zt);
   return (int)hipGetLastError();
 }
 

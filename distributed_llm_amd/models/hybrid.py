@@ -770,10 +770,20 @@ class HybridModel:
         S = 0 if meta.host_qlen is None else len(meta.host_qlen)
         expand = bool(S) and all_rows and seqmix.latent_expand_wanted(cache[0], H, m.dim, m.vdim, T, S,
                                                                        meta.block_tables.numel(), rd)
-        # absorbed form: padding rows of the attention output are cleared by the write launch
-        lat = None if expand else torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)
+        # absorbed form: padding rows of the attention output (behind the up-projection, where its launch makes that) are cleared by the
+        # write launch
+        lat = up = zero = None
+        if not expand:
+            rows = (seqmix.LAT_ROWS if meta.host_qlen is None else
+                    seqmix.latent_rows(x, m.kv_rank, m.rot_dim, T, len(meta.host_qlen)))
+            ts, tr = meta.latent_tiles(H, self.device, rows)
+            if not self.order_kept and seqmix.latent_up_ok(x, H, T, int(ts.numel()), m.kv_rank, rd, L["uvT"], rows):
+                up = (L["uvT"], gate, torch.empty((T, H * m.vdim), dtype=x.dtype, device=x.device))
+                zero = up[2][None]
+            else:
+                zero = lat = torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)
         cq = seqmix.latent_kv_write(down[:, m.q_rank:g0], m.kv_rank, L["dkv_norm"], eps, positions, table, meta.slots,
-                                    cache[0], m.rot_half, down[:, :m.q_rank], L["dq_norm"], None if all_rows else lat)
+                                    cache[0], m.rot_half, down[:, :m.q_rank], L["dq_norm"], None if all_rows else zero)
         q = _pm(cq, L, "uq")                                            # [T, H (dim + rot)]
         if expand:
             q = seqmix.latent_q_prep(q, H, m.dim, rd, positions, table, m.scale, m.rot_half)
@@ -786,12 +796,11 @@ class HybridModel:
             return _pm(o, L, "o")
         qn = q.view(T, H, m.dim + rd)[:, :, :m.dim].transpose(0, 1)
         qa = torch.bmm(qn, L["uk"])                                     # key up-projection absorbed: [H, T, rank]
-        rows = (seqmix.LAT_ROWS if meta.host_qlen is None else
-                seqmix.latent_rows(x, m.kv_rank, m.rot_dim, T, len(meta.host_qlen)))
-        ts, tr = meta.latent_tiles(H, self.device, rows)
         lat = seqmix.latent_attention(qa, q, m.dim, rd, positions, table, cache[0], meta.block_tables, meta.qstart,
                                       meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat, half=m.rot_half,
-                                      sinks=L.get("sink"))
+                                      sinks=L.get("sink"), up=up)
+        if up is not None:
+            return _pm(lat, L, "o")
         o = torch.bmm(lat, L["uvT"])                                    # [H, T, vdim]
         if gate is not None:
             o = seqmix.gate_heads(o, gate, torch.empty((T, H * m.vdim), dtype=x.dtype, device=x.device))
@@ -946,16 +955,23 @@ class HybridModel:
             seqmix.paged_gqa_attention(q, k, v, table, meta.qstart, meta.qlen, meta.ctx, ts, tt, proj[:, g0:g0 + hv], mfma, splits,
                                        out=both[:, :hv])
             return _pm(both, L, "out")
-        lat = torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)     # padding rows cleared by the prep launch
-        seqmix.latent_prep(proj, c0, L["dkv_norm"], self.cfg.rms_eps, meta.slots, cache[0], g0 + hv, act, zero=lat)
-        q = proj[:, :c0]
-        qa = torch.bmm(q.unflatten(1, (H, m.dim)).transpose(0, 1), L["uk"])     # key up-projection absorbed: [H, T, rank]
         rows = (seqmix.LAT_ROWS if meta.host_qlen is None else
                 seqmix.latent_rows(x, m.kv_rank, 0, T, len(meta.host_qlen)))
         ts, tr = meta.latent_tiles(H, self.device, rows)
+        lat = up = None
+        if not self.order_kept and seqmix.latent_up_ok(x, H, T, int(ts.numel()), m.kv_rank, 0, L["uvT"], rows):
+            up = (L["uvT"], proj[:, g0:g0 + hv], both[:, :hv])
+        else:
+            lat = torch.empty((H, T, m.kv_rank), dtype=x.dtype, device=x.device)
+        # padding rows of the attention output, or of what the up-projection's launch makes of it, cleared by the prep launch
+        seqmix.latent_prep(proj, c0, L["dkv_norm"], self.cfg.rms_eps, meta.slots, cache[0], g0 + hv, act,
+                           zero=lat if up is None else both[:, :hv][None])
+        q = proj[:, :c0]
+        qa = torch.bmm(q.unflatten(1, (H, m.dim)).transpose(0, 1), L["uk"])     # key up-projection absorbed: [H, T, rank]
         lat = seqmix.latent_attention(qa, q, m.dim, 0, positions, self._any_table(), cache[0], meta.block_tables, meta.qstart,
-                                      meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat)
-        seqmix.gate_heads(torch.bmm(lat, L["uvT"]), proj[:, g0:g0 + hv], both[:, :hv])
+                                      meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat, up=up)
+        if up is None:
+            seqmix.gate_heads(torch.bmm(lat, L["uvT"]), proj[:, g0:g0 + hv], both[:, :hv])
         return _pm(both, L, "out")
 
     def _hidden_parallel(self, x, xl, positions, meta, kv_caches):

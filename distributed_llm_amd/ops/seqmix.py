@@ -180,7 +180,7 @@ def latent_kv_write(ckv, rank, norm_w, eps, positions, cos_sin, slots, cache, ha
                     zero: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """A token's latent (RMS norm, weight ``norm_w``) and its rotated key part (pairs (2i, 2i + 1), with
     ``half`` (i, i + rot / 2)) into its cache slot.  ``q_src`` [T, n]: the query latent made by the same
-    projection; returns rmsnorm(q_src) * q_norm from the same launch.  ``zero`` [heads, T, rank]: the
+    projection; returns rmsnorm(q_src) * q_norm from the same launch.  ``zero`` [n, T, c] (unit column stride): the
     rows of tokens without a slot (padding) are cleared."""
     ext = _native(ckv)
     if ext is None:
@@ -226,21 +226,36 @@ def latent_rows(x: torch.Tensor, rank: int, rot_dim: int, tokens: int, seqs: int
     return 32 if ext is not None and ext.latent_mfma_ok(int(rank), int(rot_dim), 32) else LAT_ROWS
 
 
+LAT_UP_TOKENS = 64     # latent_up_kernel: past it the batched product reads the weights less often
+
+
+def latent_up_ok(x: torch.Tensor, heads: int, tokens: int, entries: int, rank: int, rot_dim: int, uv: torch.Tensor, rows: int) -> bool:
+    """Does a latent attention launch over ``entries`` tiles merge its splits together with the value up-projection ``uv``
+    [heads, rank, vdim] (``latent_attention``'s ``up``)?"""
+    if not x.is_cuda or x.dtype != torch.bfloat16 or tokens > LAT_UP_TOKENS or os.environ.get("DLLM_LATENT_MFMA", "1") != "1":
+        return False
+    ext = _native(x)
+    return (ext is not None and uv.shape[2] in (32, 64, 128) and uv.is_contiguous() and uv.data_ptr() % 16 == 0 and
+            latent_splits(entries, heads, rows) > 1 and bool(ext.latent_mfma_ok(int(rank), int(rot_dim), int(rows))))
+
+
 def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_tables, qstart, qlen, ctx, tile_seq,
                      tile_tok0, scale, splits: Optional[int] = None, mfma: Optional[bool] = None,
                      rows: int = LAT_ROWS, out: Optional[torch.Tensor] = None, half: bool = False,
-                     sinks: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     sinks: Optional[torch.Tensor] = None, up: Optional[tuple] = None) -> torch.Tensor:
     """``out``: a prepared output like qa (its padding rows already cleared).  ``mfma`` (GPU, bf16): the
     matrix-core kernel (default where the shape fits it; ``DLLM_LATENT_MFMA=0`` or ``mfma=False``
     keeps the vector-ALU kernel that f32 models run).  ``half``: layout of the rotary pairs as in
     ``latent_kv_write``.  ``sinks`` [heads] f32: one more term of that score per head (not scaled) in the
-    denominator, with no value."""
+    denominator, with no value.  ``up`` (where ``latent_up_ok``) = (uv [heads, rank, vdim], gate [T, heads vdim] or [T, heads] or None,
+    result [T, heads vdim], its padding rows already cleared): the merging launch goes on to the value up-projection and the gate,
+    and the result is returned."""
     ext = _native(qa)
     if ext is None:
         return ref.latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_tables, qstart, qlen, ctx,
                                     scale, half, sinks)
     if out is None:
-        out = torch.zeros_like(qa)
+        out = torch.zeros_like(qa) if up is None else qa      # with splits and an up-projection nothing is written there
     H, n_entries = qa.shape[0], int(tile_seq.numel())
     sp = latent_splits(n_entries, H, rows) if splits is None else int(splits)
     po = pml = None
@@ -252,8 +267,8 @@ def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_table
     if mfma is None:
         mfma = os.environ.get("DLLM_LATENT_MFMA", "1") == "1"
     ext.latent_attention(qa, q, int(dim), int(rot_dim), positions, cos_sin, cache, block_tables, qstart, qlen, ctx,
-                         tile_seq, tile_tok0, float(scale), out, sp, po, pml, bool(mfma), int(rows), bool(half), sinks)
-    return out
+                         tile_seq, tile_tok0, float(scale), out, sp, po, pml, bool(mfma), int(rows), bool(half), sinks, *(up or ()))
+    return out if up is None else up[2]
 
 
 def relu2_scale(x: torch.Tensor, gate: Optional[torch.Tensor] = None, ff: int = 0) -> torch.Tensor:
@@ -825,7 +840,7 @@ def latent_prep(proj, ccol, norm_w, eps, slots, cache, ucol: int = 0, act: Optio
     """``latent_kv_write`` for a latent without a rotated part inside a wider projection: cache [blocks,
     block, rank] receives rmsnorm(proj[:, ccol : ccol + rank]) * norm_w at the tokens' slots; ``act``
     as in ``rope_prep``; ``q`` [T, ...] (contiguous) receives the first columns of proj times ``qscale``;
-    ``zero`` [heads, T, rank]: the rows of tokens without a slot (padding) are cleared."""
+    ``zero`` [n, T, c] (unit column stride): the rows of tokens without a slot (padding) are cleared."""
     ext = _native(proj)
     if ext is None:
         return ref.latent_prep(proj, ccol, norm_w, eps, slots, cache, ucol, act, q, qscale, zero)

@@ -922,3 +922,42 @@ def test_gqa_of_few_rows(H, G, d, dv, splits, opts):
     got, want = run(False), run(True)
     assert torch.isfinite(want).all()
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("splits", [2, 5, 16, 20])
+@pytest.mark.parametrize("H,rank,vdim", [(16, 256, 64), (3, 40, 32), (20, 128, 128), (2, 512, 64), (16, 72, 128)])
+@pytest.mark.parametrize("gate", [None, "head", "entry"])
+def test_latent_up_projection(H, rank, vdim, splits, gate):
+    """Merge, value up-projection and gate in one launch against the launches of their own: the same latents, rounded alike, whose product
+    is added in another order (2^-8 of a value for its rounding to bf16, and 2^-16 of the absolute sum's largest); padding rows are left
+    alone; splits without keys and more of them than are fetched at once; ranks past a round of the threads and past the first eight."""
+    from distributed_llm_amd.models.llama import AttnMeta
+    torch.manual_seed(9)
+    dt, dim, rot = torch.bfloat16, 32, 16
+    qlens, starts = [1, 1, 2, 1], [0, 14, 300, 63]
+    T, qstart, qlen, ctx, rows, pos = batch(qlens, starts)
+    S, nblk = len(qlens), 20
+    table = ops.rope_cos_sin(512, rot, 10000.0, DEV)
+    bt = torch.randperm(S * nblk, device=DEV).to(torch.int32).view(S, nblk)
+    cache = torch.randn(S * nblk, 16, rank + rot, device=DEV).to(dt)
+    qa = (torch.randn(H, T + 2, rank, device=DEV) * 0.3).to(dt)
+    q = torch.randn(T + 2, H * (dim + rot), device=DEV).to(dt)
+    pos = torch.cat([pos, i32([0, 0])])
+    uv = (torch.randn(H, rank, vdim, device=DEV) * 0.2).to(dt)
+    gt = None if gate is None else torch.randn(T + 2, H if gate == "head" else H * vdim, device=DEV).to(dt)
+    meta = AttnMeta(slots=None, block_tables=bt, qstart=qstart, qlen=qlen, ctx=ctx, tile_seq=None, tile_tok0=None,
+                    last_idx=None, host_qlen=qlens)
+    ts, tt = meta.latent_tiles(H, DEV, 16)
+    assert seqmix.latent_up_ok(q, H, T + 2, int(ts.numel()), rank, rot, uv, 16)
+    run = lambda up: seqmix.latent_attention(qa, q, dim, rot, pos, table, cache, bt, qstart, qlen, ctx, ts, tt, 0.2, splits=splits, up=up)  # noqa: E731
+    wide = torch.full((T + 2, H * vdim + 8), 7.0, dtype=dt, device=DEV)
+    got = run((uv, gt, wide[:, :H * vdim]))
+    lat = run(None)
+    o = torch.stack([lat[h].float() @ uv[h].float() for h in range(H)])
+    mag = torch.stack([lat[h].float().abs() @ uv[h].float().abs() for h in range(H)]).max()
+    want = o.transpose(0, 1).reshape(T + 2, H * vdim)
+    if gate is not None:
+        want = want * torch.sigmoid(gt.float() if gate == "entry" else gt.float().repeat_interleave(vdim, 1))
+    # two roundings with a gate: the product's and the result's
+    assert ((got[:T].float() - want[:T]).abs() <= 2.0 ** -7 * want[:T].abs() + 2.0 ** -16 * mag).all()
+    assert (wide[T:] == 7).all() and (wide[:, H * vdim:] == 7).all()
