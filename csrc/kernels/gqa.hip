@@ -1172,6 +1172,15 @@ __global__ void __launch_bounds__(256) gqa_few_kernel(const u16* __restrict__ q,
         lo[j] = p[j] - bf2f(f2bf(p[j]));
       }
       const bf16x8 ph = __builtin_bit_cast(bf16x8, pack8(p)), pl = __builtin_bit_cast(bf16x8, pack8(lo));
+      if (k0 + 31 > last) {      // values behind the last key: whatever an earlier sequence left, and 0 times an infinity is NaN
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int left = last + 1 - (k0 + 16 * t + 4 * g4);      // of this lane's four keys
+          const unsigned x = left >= 2 ? ~0u : left == 1 ? 0xffffu : 0u, y = left >= 4 ? ~0u : left == 3 ? 0xffffu : 0u;
+#pragma unroll
+          for (int b = 0; b < VB; ++b) { cur.v[t][b].x &= x; cur.v[t][b].y &= y; }
+        }
+      }
 #pragma unroll
       for (int b = 0; b < VB; ++b) {
         const bf16x8 vf = __builtin_bit_cast(bf16x8, make_uint4(cur.v[0][b].x, cur.v[0][b].y, cur.v[1][b].x, cur.v[1][b].y));
