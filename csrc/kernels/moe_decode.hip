@@ -6,7 +6,11 @@
 // rows touch 16 lines for the bytes of 8 (15 + 10 us a layer of 8 experts of 1024 x 1024).  Here a wave owns one 16-column tile of one
 // expert and the whole of K, streams it as contiguous kilobytes, and finds the expert's pairs itself: 64 ids are a ballot.
 // One wave a tile (KS 1): its sum over K is the chain of the grouped GEMM (ascending, one accumulator, same operand order), the same
-// bits, for models that need them.  KS 4: four waves of a tile share K and meet in LDS, a quarter of the chain.
+// bits, for models that need them.  KS 4: four waves of a tile share K and meet in LDS, a quarter of the chain.  A layer of 8 or 9 experts is
+// 512 to 1152 workgroups, so what a wave keeps in registers decides whether they run side by side: with three stages and row blocks of
+// 64 (180 registers, two workgroups a CU, the rest in a second round) both products of 8 experts took 20.5 us at 12 tokens and 21.0 at
+// 24, with two stages and rows by 32 (105 registers, four a CU) 15.9 and 17.2; 9 squared-ReLU experts 18.6 -> 14.8 at 12, 21.5 -> 18.3
+// at 24 tokens.
 //
 //   moe_decode_kernel<ACT 0>  act[pair] = silu(g) u of x[pair / k], weights paired 8 columns apart
 //                    <ACT 1>  act[pair] = relu(x . w)^2
@@ -21,7 +25,7 @@ constexpr int MD_TILES = 2;      // column tiles a workgroup of KS 1: the 64 x 9
 template <int ACT, int MT, int KS>
 __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx, int div, const u16* __restrict__ wt, int kb, int K,
                                             const int* list, int row0, int n, int c0, void* __restrict__ out, long ldo,
-                                            const bf16x8 (&w0)[4], float (*s_acc)[64][17]) {      // k in [kb, K)
+                                            const bf16x8 (&w0)[4], float (*s_acc)[KS > 1 ? 32 : 1][17]) {      // k in [kb, K)
   const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
   const u16* xr[MT];
   bool ok[MT];
@@ -30,7 +34,7 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
     ok[m] = row0 + 16 * m + r16 < n;
     xr[m] = x + (long)(list[min(row0 + 16 * m + r16, n - 1)] / div) * ldx + 8 * g;
   }
-  constexpr int U = MT > 2 ? 2 : 4;
+  constexpr int U = MT > 2 || (KS > 1 && MT > 1) ? 2 : 4;
   struct Stage { bf16x8 w[U]; uint4 x[U][MT]; };
   auto load = [&](Stage& st, int k0, bool first) {
 #pragma unroll
@@ -53,16 +57,26 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
         acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, st.x[u][m]), st.w[u], acc[m], 0, 0, 0);
     }
   };
-  Stage A, B, C;      // two stages ahead of the one that is multiplied
+  Stage A, B;
   load(A, kb, true);
   load(B, kb + 32 * U, false);
-  for (int k0 = kb; k0 < K; k0 += 96 * U) {
-    load(C, k0 + 64 * U, false);
-    compute(A, k0);
-    load(A, k0 + 96 * U, false);
-    compute(B, k0 + 32 * U);
-    load(B, k0 + 128 * U, false);
-    compute(C, k0 + 64 * U);
+  if constexpr (KS > 1) {      // a quarter of K is two stages or little more
+    for (int k0 = kb; k0 < K; k0 += 64 * U) {
+      compute(A, k0);
+      load(A, k0 + 64 * U, false);
+      compute(B, k0 + 32 * U);
+      load(B, k0 + 96 * U, false);
+    }
+  } else {
+    Stage C;      // two stages ahead of the one that is multiplied
+    for (int k0 = kb; k0 < K; k0 += 96 * U) {
+      load(C, k0 + 64 * U, false);
+      compute(A, k0);
+      load(A, k0 + 96 * U, false);
+      compute(B, k0 + 32 * U);
+      load(B, k0 + 128 * U, false);
+      compute(C, k0 + 64 * U);
+    }
   }
   auto put = [&](int row, int c, float a, float u) {
     if (row >= n) return;
@@ -101,12 +115,12 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
 }
 
 template <int ACT, int KS>
-__global__ void __launch_bounds__(KS > 1 ? 64 * KS : 64 * MD_TILES) moe_decode_kernel(const u16* __restrict__ x, long ldx, int div, const int* __restrict__ ids, int P,
+__global__ void __launch_bounds__(KS > 1 ? 64 * KS : 64 * MD_TILES, KS > 1 ? 4 : 1) moe_decode_kernel(const u16* __restrict__ x, long ldx, int div, const int* __restrict__ ids, int P,
                                                                    int E, const u16* __restrict__ w, int N, int K, void* __restrict__ out,
                                                                    long ldo) {
   constexpr int WV = KS > 1 ? KS : MD_TILES;
   __shared__ int s_list[WV][MD_PAIRS];
-  __shared__ float s_acc[KS > 1 ? KS : 1][64][17];
+  __shared__ float s_acc[KS > 1 ? KS : 1][KS > 1 ? 32 : 1][17];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int e = blockIdx.y, tile = KS > 1 ? blockIdx.x : blockIdx.x * MD_TILES + wave;
   if (tile * 16 >= N) return;      // (KS 1: no barrier below)
@@ -130,6 +144,8 @@ __global__ void __launch_bounds__(KS > 1 ? 64 * KS : 64 * MD_TILES) moe_decode_k
   __builtin_amdgcn_wave_barrier();
   if (n <= 16) expert_rows<ACT, 1, KS>(x, ldx, div, wt, kb, ke, list, 0, n, tile * 16, out, ldo, w0, s_acc);
   else if (n <= 32) expert_rows<ACT, 2, KS>(x, ldx, div, wt, kb, ke, list, 0, n, tile * 16, out, ldo, w0, s_acc);
+  else if constexpr (KS > 1)
+    for (int r = 0; r < n; r += 32) expert_rows<ACT, 2, KS>(x, ldx, div, wt, kb, ke, list, r, n, tile * 16, out, ldo, w0, s_acc);
   else
     for (int r = 0; r < n; r += 64) expert_rows<ACT, 4, KS>(x, ldx, div, wt, kb, ke, list, r, n, tile * 16, out, ldo, w0, s_acc);
 }
