@@ -484,14 +484,15 @@ MOE_PLANS = {  # (bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2) by rou
 
 
 # tokens and routed pairs up to which the experts run on their fragment-major copies (csrc/kernels/moe_decode.hip, whose pair list ends
-# at 256).  Routing, both products and the sum, us grouped / here: 8 experts of 1024 x 1024 (SwiGLU, top 2) 1 token 28 / 15, 12 32 / 23,
-# 64 32 / 27; with a shared expert (squared ReLU) 1 token 26 / 15, 24 28 / 21, 42 28.7 / 28.9, 48 33.6 / 30.1, 64 34.4 / 33.9, 85 34 / 51.
+# at 256).  Routing, both products and the sum, us grouped / here: 8 experts of 1024 x 1024 (SwiGLU, top 2) 1 token 28 / 12, 12 31 / 16,
+# 64 32 / 24; with a shared expert (squared ReLU) 1 token 27 / 12, 24 28 / 18, 42 29 / 23, 48 34 / 24, 64 34 / 28.
 MOE_FEW, MOE_FEW_TOKENS = 256, 64
 
 
 def frag_experts(w: torch.Tensor, paired: bool = False) -> torch.Tensor:
     """[E, N, K] expert weights fragment-major (gemm.frag_weight) for the decode step's kernels."""
-    return torch.stack([gemm.frag_weight(e, paired) for e in w])
+    from .gemm import frag_weight
+    return torch.stack([frag_weight(e, paired) for e in w])
 
 
 def moe_few(x: torch.Tensor, ids: torch.Tensor, frag) -> dict:
