@@ -758,8 +758,10 @@ typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 // 4 g4 .. 4 g4 + 3 of column lr.
 constexpr float CAP_MAX = 64.f;
 // DIST: the scores fall with the distance (`slopes`); the score accumulators start at -slope * distance.
+// Up to 64-wide heads four workgroups fit a CU's LDS, and its registers if a wave keeps to 128 (6 sequences of 7300 tokens, 32 / 8 heads:
+// 266 us with three, 232 with four).
 template <int KD, int VD, bool CAP, bool DIST>
-__global__ void __launch_bounds__(256) paged_gqa_mfma_kernel(const u16* __restrict__ q, const u16* __restrict__ kc,
+__global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(const u16* __restrict__ q, const u16* __restrict__ kc,
                                                              const u16* __restrict__ vc, const int* __restrict__ bt,
                                                              int bt_ld, const int* __restrict__ qstart,
                                                              const int* __restrict__ qlen, const int* __restrict__ ctx,
@@ -839,7 +841,7 @@ __global__ void __launch_bounds__(256) paged_gqa_mfma_kernel(const u16* __restri
   uint4 pk_[NFK], pv_[NFV];
   // A thread moves the same (key, chunk) and (dim, page, half) of every tile (tiles start at multiples
   // of 64 keys), so only the page ids change from tile to tile: offsets inside a page are kept.
-  long koff[NFK], voff[NFV];
+  int koff[NFK], voff[NFV];      // inside a page
   int kkey[NFK], vpg[NFV];
   bool kon[NFK], von[NFV];
   const long kpage = (long)G * GM_BS * d, vpage = (long)GV * dv * GM_BS;
@@ -850,7 +852,7 @@ __global__ void __launch_bounds__(256) paged_gqa_mfma_kernel(const u16* __restri
     const int kk = e / KCH, c = (e % KCH) * 8;
     kkey[f] = kk;
     kon[f] = c < d;
-    koff[f] = ((long)g * GM_BS + (kk & 15)) * d + c;
+    koff[f] = (g * GM_BS + (kk & 15)) * d + c;
   }
 #pragma unroll
   for (int f = 0; f < NFV; ++f) {
@@ -858,7 +860,7 @@ __global__ void __launch_bounds__(256) paged_gqa_mfma_kernel(const u16* __restri
     const int j = e / (GM_KT / 8), cc = e % (GM_KT / 8);
     vpg[f] = cc >> 1;
     von[f] = j < dv;
-    voff[f] = ((long)gv * dv + j) * GM_BS + 8 * (cc & 1);
+    voff[f] = (gv * dv + j) * GM_BS + 8 * (cc & 1);
   }
   auto fetch = [&](int k0) {
     const int nk = min(GM_KT, last + 1 - k0);
