@@ -5,8 +5,8 @@ attention, differential sliding-window attention, Mamba-2, mLSTM) and an optiona
 
 The residual stream lives in f32; each sublayer reads its rounding to the model dtype and adds
 ``rmsnorm(sublayer(x)) * w`` (ops.seqmix.norm_resadd: the f32 add, the norm and the rounded copy in
-one launch).  Projections run on the framework's GEMMs (ops.linear; the vendor GEMM for shapes
-they do not take and for f32 models), everything between them on the HIP kernels of ops.seqmix:
+one launch).  Projections run on the framework's GEMMs (ops.linear, ops.gemm.f32_linear for
+up to 16 rows of an f32 model; the vendor GEMM for shapes they do not take and longer f32 steps), everything between them on the HIP kernels of ops.seqmix:
 
   mamba1     in-proj -> causal conv + SiLU (reads the slot's last inputs) -> x-proj -> dt-proj ->
              selective scan (f32 state per slot, softplus / decay / gate in f32; refills the
