@@ -206,6 +206,14 @@ def _need(M: int, N: int, K: int, ntw: int, splits: int) -> Tuple[int, int]:
     return (S * tiles * nc * mp if S > 1 else 0), tiles
 
 
+def _need_dg(M: int, N: int, K: int, plan: Tuple[int, int, int]) -> Tuple[int, int]:
+    """Floats and tickets of a decode GEMM ``plan``; (0, 0) where one workgroup has all of a tile's splits."""
+    nt, vs, splits = plan
+    kchunk = (-(-K // splits) + 31) // 32 * 32
+    gy, tiles = -(-(-(-K // kchunk)) // vs), -(-N // (16 * nt))
+    return (gy * vs * tiles * -(-M // 16) * 16 * (16 * nt + 1), tiles) if gy > 1 else (0, 0)
+
+
 def _tg_splits(K: int, splits: int, ks: int = 1) -> int:
     q = 64 * ks
     kchunk = ((K + splits - 1) // splits + q - 1) // q * q
@@ -551,12 +559,8 @@ def dgemm(x: torch.Tensor, wf: torch.Tensor, n: int, epi: int, plan: Tuple[int, 
     """One launch of the decode GEMM on ``wf`` = frag_weight of an [n, K] weight; ``plan`` = (16-column tiles a workgroup, splits a
     workgroup, splits of K)."""
     nt, vs, splits = plan
-    M, K = x.shape
-    kchunk = (-(-K // splits) + 31) // 32 * 32
-    gy, tiles = -(-(-(-K // kchunk)) // vs), -(-n // (16 * nt))
-    part = cnt = None
-    if gy > 1:
-        part, cnt = _P.workspace(x.device, gy * vs * tiles * -(-M // 16) * 16 * (16 * nt + 1), tiles)
+    floats, tiles = _need_dg(x.shape[0], n, x.shape[1], plan)
+    part, cnt = _P.workspace(x.device, floats, tiles) if floats else (None, None)
     return int(_native(x).dgemm(x, wf, n, int(epi), nt, vs, splits, y, part, cnt, res, ssq_out, float(scale), float(eps), pos, cos_sin,
                                 slots, q_out, kc, vc, v_rows, int(nq), int(nkv), int(d), bias, int(mode), float(limit), float(alpha)))
 
@@ -583,20 +587,25 @@ def f32_linear(x: torch.Tensor, wf: torch.Tensor, N: int, gelu: bool = False) ->
     return y
 
 
-def _linear_plan(x: torch.Tensor, w: torch.Tensor, frag: bool, keep_order: bool):
-    """(plan on the row-major weight, splits a workgroup, decode GEMM's plan or None) of ``linear``."""
+def _linear_plan(x: torch.Tensor, w: torch.Tensor, frag: bool, keep_order: bool, ends: bool = False):
+    """(plan on the row-major weight, splits a workgroup, decode GEMM's plan or None) of ``linear``; ``ends``: the decode GEMM would end in
+    the activation, a launch (3.4 us) that the plan it is timed against has yet to make."""
     M, (N, K) = x.shape[0], w.shape
     plan, together = _P.plans.get(_key(x, w, False)), 1
     dg = _P.dg_plans.get((M, N, K)) if frag and not keep_order else None
     timed = plan is not None
     if not timed:
         plan = _heuristic(M, N, K) if M <= MAX_M else ("blas",)
-    if plan[0] == "skinny" and (frag or not timed):
+    if plan[0] == "skinny":
         same = ("skinny", min(plan[1], 2), plan[2])
-        together = _splits_together(M, N, K, same)
-        if frag and dg is None:
-            dg = (same[1], together, same[2])
-        together = 1 if timed else together
+        as_one = _splits_together(M, N, K, same)
+        if not timed:
+            together = as_one
+        if frag and dg is None and (not timed or keep_order or ends):
+            dg = (same[1], as_one, same[2])
+            floats, tiles = _need_dg(M, N, K, dg)
+            if M > DG_MAX_M or floats > WS_FLOATS or tiles > WS_COUNTERS:      # (a slab is a column wider than the skinny plan's)
+                dg = None
     return plan, together, dg
 
 
@@ -606,7 +615,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, wf: torch.Tensor, act: str, bia
     decode GEMM, where it takes the product; else None.  ``wf``: frag_weight(w), paired = "glu" for the gated ones."""
     if not dg_takes(x) or os.environ.get("DLLM_GEMM") == "blas":
         return None
-    dg = _linear_plan(x, w, True, keep_order)[2]
+    dg = _linear_plan(x, w, True, keep_order, ends=True)[2]
     if dg is None:
         return None
     N = w.shape[0]
@@ -1186,7 +1195,7 @@ def _dg_cands(M: int, N: int, K: int):
                 kchunk = (-(-K // s) + 31) // 32 * 32
                 if -(-K // kchunk) != s or K // (4 * s) < 64 or not 64 <= tiles * gy <= 2048 or (gy > 1 and tiles * gy > 1024):
                     continue
-                if gy > 1 and s * tiles * 64 * (16 * nt + 1) > WS_FLOATS:
+                if _need_dg(M, N, K, (nt, vs, s))[0] > WS_FLOATS:
                     continue
                 out.append((nt, vs, s))
     return out

@@ -126,3 +126,27 @@ def test_parts_are_the_whole(monkeypatch, panel):
     monkeypatch.setattr(G, "use_vendor_core", lambda M, N, K: True)
     for a, b in zip(one, run()):
         torch.testing.assert_close(a.float(), b.float(), rtol=2e-2, atol=2e-2)
+
+
+def test_decode_gemm_in_place_of_a_skinny_plan(monkeypatch):
+    """A timed plan runs as timed, unless the decode GEMM was faster, has to keep the order of its sums or saves the activation's launch; and
+    only where its slabs, one column of a tile wider than the skinny plan's, fit the workspace."""
+    monkeypatch.setattr(G._P, "plans", {(16, 2048, 2048, False): ("skinny", 2, 8), (64, 32000, 2048, False): ("skinny", 2, 8),
+                                        (8, 2048, 2048, False): ("tg", 64, 64, 3, 1, 1, 4), (4, 2048, 2048, False): ("skinny", 4, 2)})
+    monkeypatch.setattr(G._P, "dg_plans", {(8, 2048, 2048): (1, 2, 4)})
+    of = lambda M, N, K, *a, **k: G._linear_plan(torch.empty(M, K), torch.empty(N, K), *a, **k)  # noqa: E731
+    assert of(16, 2048, 2048, True, False) == (("skinny", 2, 8), 1, None)
+    assert of(16, 2048, 2048, True, True)[2] == of(16, 2048, 2048, True, False, ends=True)[2] == (2, 2, 8)
+    assert of(4, 2048, 2048, True, True)[2] == (2, 2, 2) and of(4, 2048, 2048, True, False)[2] is None
+    assert of(8, 2048, 2048, True, False)[2] == (1, 2, 4) and of(8, 2048, 2048, True, True)[2] is None
+    assert G._need(64, 32000, 2048, 2, 8)[0] <= G.WS_FLOATS < G._need_dg(64, 32000, 2048, (2, 2, 8))[0]
+    for keep in (False, True):
+        assert of(64, 32000, 2048, True, keep, ends=True) == (("skinny", 2, 8), 1, None)
+    # nothing timed: the rule's plan, its splits together, with and without copies
+    plan = G._heuristic(16, 1024, 1024)
+    assert of(16, 1024, 1024, False, False) == (plan, G._splits_together(16, 1024, 1024, plan), None)
+    assert of(16, 1024, 1024, True, False)[2] == (plan[1], G._splits_together(16, 1024, 1024, plan), plan[2])
+    for M in range(1, 65):
+        for N, K in SHAPES:
+            dg = of(M, N, K, True, False)[2]
+            assert dg is None or G._need_dg(M, N, K, dg)[0] <= G.WS_FLOATS
