@@ -28,6 +28,7 @@ from __future__ import annotations
 
 import contextlib
 import contextvars
+import json
 import math
 import os
 from typing import Dict, Iterable, Optional, Tuple
@@ -160,8 +161,12 @@ class _Planner:
     def __init__(self):
         self.plans: Dict[Tuple[int, int, int, bool], Tuple] = {}     # best overall, for linear()
         self.tg_plans: Dict[Tuple[int, int, int], Tuple] = {}        # best tgemm tile, for the fused ops
-        self.dg_plans: Dict[Tuple[int, int, int], Tuple] = {}        # decode GEMM (nt, vs, splits), where it beats plans[...]
-        self.fused_core: Dict[Tuple[int, int, int], str] = {}        # "tg" | "lin" | "gemvR" | "skES" | "dgN.V.S" per tuned shape
+        # decode GEMM (nt, vs, splits) where it beats plans[...], None where it was timed and does not
+        self.dg_plans: Dict[Tuple[int, int, int], Optional[Tuple]] = {}
+        self.fused_core: Dict[Tuple[int, int, int], str] = {}        # "tg" | "lin" | "gemvR" | "skES" per tuned shape
+        # the same with "dgN.V.S" among the choices, for weights that have fragment-major copies: whether a model has them is decided by
+        # the memory that is free when it is made, so both kinds may run in one process or load one plan file
+        self.frag_core: Dict[Tuple[int, int, int], str] = {}
         self.fused_opts: Dict[Tuple[int, int, int], Dict[str, float]] = {}   # measured us per core choice
         self.pf_times: Dict[Tuple[int, int], list] = {}      # (N, K) of prompts: [(plan, rows, us)]
         self.pf_small: Dict[Tuple[int, int, int], Tuple] = {}        # (rows of PF_SMALL_MS, N, K): (fastest plan, its us)
@@ -372,9 +377,9 @@ def prompt_parts(M: int, N: int, K: int, cus: int = 256) -> Optional[Tuple]:
     return parts
 
 
-def _row_parts(M: int, N: int, K: int) -> list:
+def _row_parts(M: int, N: int, K: int, frag: bool = False) -> list:
     """[(first row, end, plan or "lin")]: a fused product's launches."""
-    if use_vendor_core(M, N, K):
+    if use_vendor_core(M, N, K, True) if frag else use_vendor_core(M, N, K):
         return [(0, M, "lin")]
     parts = prompt_parts(M, N, K) if M > MAX_M and PREFILL_MS and not os.environ.get("DLLM_FUSED_CORE") else None
     out, lo = [], 0
@@ -675,14 +680,21 @@ def linear_swiglu(gu: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 POST_US = 3.0
 
 
-def use_vendor_core(M: int, N: int, K: int) -> bool:
+def _core_of(M: int, N: int, K: int, frag: bool) -> Optional[str]:
+    """The timed core of a fused op whose weight has (``frag``) or has no fragment-major copy; a decode GEMM is ``fused_dg``'s to take,
+    rows it does not read get what was chosen without it."""
+    c = _P.frag_core.get((M, N, K)) if frag else None
+    return _P.fused_core.get((M, N, K)) if c is None or c.startswith("dg") else c
+
+
+def use_vendor_core(M: int, N: int, K: int, frag: bool = False) -> bool:
     """True: run the fused op as ``linear()`` (the shape's best plain plan — GEMV / skinny /
     hipBLASLt / plain tgemm) followed by the standalone epilogue kernel; False: one tgemm launch
     with the epilogue fused.  (A ``gemvR`` choice is taken before this by ``fused_gemv_r``.)"""
     env = os.environ.get("DLLM_FUSED_CORE")
     if env in ("tg", "blas", "lin"):
         return env != "tg"
-    c = _P.fused_core.get((M, N, K))
+    c = _core_of(M, N, K, frag)
     if c is None and M > MAX_M and PREFILL_MS:
         c = _P.fused_core.get((prefill_bucket(M), N, K))
     if c is not None:
@@ -690,7 +702,7 @@ def use_vendor_core(M: int, N: int, K: int) -> bool:
     return M > MAX_M
 
 
-def fused_gemv_r(x: torch.Tensor, N: int) -> int:
+def fused_gemv_r(x: torch.Tensor, N: int, frag: bool = False) -> int:
     """R (output rows per wave) of the fused-epilogue GEMV (csrc/kernels/gemv.hip EPI) if the
     autotuner picked it for this fused op's shape (``fused_core`` = ``gemvR``; forced by
     ``DLLM_FUSED_CORE=gemvR``), else 0.  Batch <= 8 only: it replaces GEMV/skinny + a standalone
@@ -699,13 +711,13 @@ def fused_gemv_r(x: torch.Tensor, N: int) -> int:
     if M not in _GEMV_MS or K % 8 or M * K * 2 > 64 * 1024 or x.stride(1) != 1 or x.stride(0) % 8 or N % 32:
         return 0
     env = os.environ.get("DLLM_FUSED_CORE")
-    c = env if env else _P.fused_core.get((M, N, K))
+    c = env if env else _core_of(M, N, K, frag)
     if isinstance(c, str) and c.startswith("gemv") and c[4:] in ("1", "2", "4"):
         return int(c[4:])
     return 0
 
 
-def fused_ske(x: torch.Tensor, N: int, K: int) -> int:
+def fused_ske(x: torch.Tensor, N: int, K: int, frag: bool = False) -> int:
     """Split count of the small-batch fused-epilogue MFMA GEMM (skinny_epi, 32-column tiles) if the
     autotuner picked it for this fused op's shape (``fused_core`` = ``skE<splits>``; forced by
     ``DLLM_FUSED_CORE=skE<splits>``), else 0."""
@@ -713,7 +725,7 @@ def fused_ske(x: torch.Tensor, N: int, K: int) -> int:
     if not (0 < M <= SKE_MAX_M) or K % 64 or N % 32 or x.stride(1) != 1 or x.stride(0) % 8:
         return 0
     env = os.environ.get("DLLM_FUSED_CORE")
-    c = env if env and env.startswith("skE") else _P.fused_core.get((M, N, K))
+    c = env if env and env.startswith("skE") else _core_of(M, N, K, frag)
     if isinstance(c, str) and c.startswith("skE") and c[3:].isdigit():
         return int(c[3:])
     return 0
@@ -738,12 +750,12 @@ def skinny_epi(x: torch.Tensor, w: torch.Tensor, epi: int, splits: int, y=None, 
 
 
 def fused_dg(x: torch.Tensor, N: int, K: int, wf: Optional[torch.Tensor]) -> Optional[Tuple[int, int, int]]:
-    """Plan of the decode GEMM (csrc/kernels/decode_gemm.hip) if the autotuner picked it for this fused op's shape (``fused_core`` =
+    """Plan of the decode GEMM (csrc/kernels/decode_gemm.hip) if the autotuner picked it for this fused op's shape (``frag_core`` =
     ``dg<nt>.<vs>.<splits>``) and the caller keeps its weight copy, else None."""
     if wf is None:
         return None
     M = x.shape[0]      # rows between two timed batch sizes (a short prompt): what was timed for the next one
-    c = os.environ.get("DLLM_FUSED_CORE") or _P.fused_core.get((M, N, K)) or _P.fused_core.get((next_batch_size(M), N, K))
+    c = os.environ.get("DLLM_FUSED_CORE") or _P.frag_core.get((M, N, K)) or _P.frag_core.get((next_batch_size(M), N, K))
     if not c or not c.startswith("dg") or not dg_takes(x):
         return None
     return tuple(int(v) for v in c[2:].split("."))
@@ -778,17 +790,17 @@ def qkv_rope_cache(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: i
         dgemm(r, wf, w.shape[0], EPI_QKV, dg, scale=1.0 / H, eps=eps, pos=positions, cos_sin=cos_sin, slots=slots, q_out=q, kc=k_cache,
               vc=v_cache, v_rows=v_new, nq=nq, nkv=nkv, d=d)
         return out(True)
-    R = fused_gemv_r(r, w.shape[0])
+    R = fused_gemv_r(r, w.shape[0], wf is not None)
     if R:
         _native(r).gemv_qkv(r, w, ssq, int(ssq_n), 1.0 / H, float(eps), positions, cos_sin, slots, q, k_cache,
                             v_cache, nq, nkv, d, R)
         return out(False)
-    sp = fused_ske(r, w.shape[0], H)
+    sp = fused_ske(r, w.shape[0], H, wf is not None)
     if sp:
         skinny_epi(r, wp if wp is not None else w, EPI_QKV, sp, ssq_in=ssq, ssq_n=ssq_n, scale=1.0 / H, eps=eps,
                    pos=positions, cos_sin=cos_sin, slots=slots, q_out=q, kc=k_cache, vc=v_cache, nq=nq, nkv=nkv, d=d)
         return out(False)
-    for lo, hi, plan in _row_parts(T, w.shape[0], H):
+    for lo, hi, plan in _row_parts(T, w.shape[0], H, wf is not None):
         rows, sq = (r, ssq) if hi - lo == T else (r[lo:hi], ssq[:, lo:hi])
         if plan == "lin":
             vr = v_new if QKV_POST_VROWS else None
@@ -811,15 +823,15 @@ def matmul_resadd(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, ssq_
     dg = fused_dg(x, N, K, wf) if M else None
     if dg:
         return dgemm(x, wf, N, EPI_RESADD, dg, res=residual, ssq_out=ssq_out)
-    R = fused_gemv_r(x, N) if M else 0
+    R = fused_gemv_r(x, N, wf is not None) if M else 0
     if R:
         return int(_native(x).gemv_resadd(x, w, residual, ssq_out, R))
-    sp = fused_ske(x, N, K) if M else 0
+    sp = fused_ske(x, N, K, wf is not None) if M else 0
     if sp:
         return skinny_epi(x, wp if wp is not None else w, EPI_RESADD, sp, res=residual, ssq_out=ssq_out)
     if not M:
         return -(-N // tg_plan(M, N, K)[1])
-    parts = _row_parts(M, N, K)
+    parts = _row_parts(M, N, K, wf is not None)
     if parts[0][2] == "lin":
         return int(_native(x).res_add_ssq(_core(x, w, wp), residual, ssq_out))
     n = max(-(-N // p[1]) for _, _, p in parts)
@@ -843,18 +855,18 @@ def swiglu_matmul(r: torch.Tensor, w: torch.Tensor, ssq: torch.Tensor, ssq_n: in
     if dg:
         dgemm(r, wf, w.shape[0], EPI_SWIGLU, dg, y=act, scale=1.0 / H, eps=eps)
         return act
-    R = fused_gemv_r(r, w.shape[0]) if T else 0
+    R = fused_gemv_r(r, w.shape[0], wf is not None) if T else 0
     if R:
         _native(r).gemv_swiglu(r, w, ssq, int(ssq_n), 1.0 / H, float(eps), act, R)
         return act
-    sp = fused_ske(r, w.shape[0], H) if T else 0
+    sp = fused_ske(r, w.shape[0], H, wf is not None) if T else 0
     if sp:
         skinny_epi(r, wp if wp is not None else w, EPI_SWIGLU, sp, y=act, ssq_in=ssq, ssq_n=ssq_n, scale=1.0 / H,
                    eps=eps)
         return act
     if not T:
         return act
-    for lo, hi, plan in _row_parts(T, w.shape[0], H):
+    for lo, hi, plan in _row_parts(T, w.shape[0], H, wf is not None):
         rows, sq = (r, ssq) if hi - lo == T else (r[lo:hi], ssq[:, lo:hi])
         if plan == "lin":
             _native(r).swiglu_post(_core(rows, w, wp), sq, int(ssq_n), 1.0 / H, float(eps), act[lo:hi])
@@ -989,6 +1001,41 @@ def _plan_key(k) -> str:
     return "%d,%d,%d,%d" % (k[0], k[1], k[2], int(k[3]))
 
 
+def _load_plans(path: str) -> None:
+    with open(path) as f:
+        for k, v in json.load(f).items():
+            kind, *at = k.split(",")
+            if kind == "t":
+                _P.tg_plans[tuple(map(int, at))] = tuple(v)
+            elif kind == "s":
+                _P.pf_small[tuple(map(int, at))] = (tuple(v[0]), v[1])
+            elif kind == "p":
+                _P.pf_times[tuple(map(int, at))] = [(tuple(q), m, t) for q, m, t in v]
+            elif kind == "d":
+                _P.dg_plans[tuple(map(int, at))] = v and tuple(v)
+            elif kind == "r":
+                _P.frag_core[tuple(map(int, at))] = v
+            elif kind == "c":
+                if not v.startswith("dg"):      # (files that kept one choice for weights with and without copies: timed again)
+                    _P.fused_core[tuple(map(int, at))] = v
+            else:
+                _P.plans[(int(kind), int(at[0]), int(at[1]), at[2] == "1")] = tuple(v)
+
+
+def _save_plans(path: str) -> None:
+    d = {_plan_key(k): list(v) for k, v in _P.plans.items()}
+    d.update({_plan_key(k): list(v) for k, v in _P.tg_plans.items()})
+    d.update({"c,%d,%d,%d" % k: v for k, v in _P.fused_core.items()})
+    d.update({"r,%d,%d,%d" % k: v for k, v in _P.frag_core.items()})
+    d.update({"d,%d,%d,%d" % k: v and list(v) for k, v in _P.dg_plans.items()})
+    d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
+    d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
+    if os.path.dirname(path):
+        os.makedirs(os.path.dirname(path), exist_ok=True)
+    with open(path, "w") as f:
+        json.dump(d, f)
+
+
 def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device, verbose: bool = False,
              fused: Iterable[Tuple[int, int]] = (), prefill: bool = False, qkv_dims=None, qkv_cache=None,
              frag: Iterable[Tuple[int, int]] = ()) -> None:
@@ -1007,22 +1054,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     reserve(dev)
     cache = os.environ.get("DLLM_GEMM_PLANS")  # JSON plan cache: re-use a previous run's choices
     if cache and os.path.exists(cache):
-        import json
-        with open(cache) as f:
-            for k, v in json.load(f).items():
-                parts = k.split(",")
-                if parts[0] == "t":
-                    _P.tg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
-                elif parts[0] == "s":
-                    _P.pf_small[tuple(int(q) for q in parts[1:])] = (tuple(v[0]), v[1])
-                elif parts[0] == "p":
-                    _P.pf_times[(int(parts[1]), int(parts[2]))] = [(tuple(q), m, t) for q, m, t in v]
-                elif parts[0] == "d":
-                    _P.dg_plans[(int(parts[1]), int(parts[2]), int(parts[3]))] = tuple(v)
-                elif parts[0] == "c":
-                    _P.fused_core[(int(parts[1]), int(parts[2]), int(parts[3]))] = v
-                else:
-                    _P.plans[(int(parts[0]), int(parts[1]), int(parts[2]), parts[3] == "1")] = tuple(v)
+        _load_plans(cache)
     shapes = list(shapes)
     fused = list(fused)
     # the fused ops' tgemm plans stream the panel weight copies: time them in that layout
@@ -1035,17 +1067,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     if PREFILL_TUNE or prefill:
         _autotune_prefill(fused, dev, verbose, roles, qkv_dims)
     if cache:
-        import json
-        d = {_plan_key(k): list(v) for k, v in _P.plans.items()}
-        d.update({_plan_key(k): list(v) for k, v in _P.tg_plans.items()})
-        d.update({"c,%d,%d,%d" % k: v for k, v in _P.fused_core.items()})
-        d.update({"d,%d,%d,%d" % k: list(v) for k, v in _P.dg_plans.items()})
-        d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
-        d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
-        if os.path.dirname(cache):
-            os.makedirs(os.path.dirname(cache), exist_ok=True)
-        with open(cache, "w") as f:
-            json.dump(d, f)
+        _save_plans(cache)
 
 
 def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> None:
@@ -1113,18 +1135,21 @@ def _couple_gemv_choices(fused, ms, verbose: bool) -> None:
     (MoE layers pass (QKV, Wo): their producers feed standalone norms, no constraint)."""
     fused = list(fused)
     pairs = [(fused[1], fused[2]), (fused[3], fused[0])] if len(fused) == 4 else []
-    for M in ms:
-        for prod, cons in pairs:
-            kp, kc = (M,) + tuple(prod), (M,) + tuple(cons)
-            cp, cc = _P.fused_core.get(kp), _P.fused_core.get(kc)
-            if cp is None or not cp.startswith(("gemv", "dg1.")) or (cc is not None and cc.startswith(("gemv", "skE", "dg"))):
-                continue
-            opts = {c: t for c, t in _P.fused_opts.get(kp, {}).items() if not c.startswith(("gemv", "dg1."))}
-            _P.fused_core[kp] = min(opts, key=opts.get) if opts else "lin"
-            if verbose:
-                print(f"gemm M={M} N={kp[1]} K={kp[2]}: {cp} dropped (its consumer N={kc[1]} K={kc[2]} "
-                      f"runs {cc}, which would walk the per-workgroup row sums) -> core {_P.fused_core[kp]}",
-                      flush=True)
+    # the decode GEMM's narrowest tiles leave a slot per 16 columns; as a consumer it takes the row sums from its own operands
+    for cores, many, fits, out in ((_P.fused_core, ("gemv",), ("gemv", "skE"), ("gemv", "dg")),
+                                   (_P.frag_core, ("gemv", "dg1."), ("gemv", "skE", "dg"), ("gemv", "dg1."))):
+        for M in ms:
+            for prod, cons in pairs:
+                kp, kc = (M,) + tuple(prod), (M,) + tuple(cons)
+                cp, cc = cores.get(kp), cores.get(kc, _P.fused_core.get(kc))
+                if cp is None or not cp.startswith(many) or (cc is not None and cc.startswith(fits)):
+                    continue
+                opts = {c: t for c, t in _P.fused_opts.get(kp, {}).items() if not c.startswith(out)}
+                cores[kp] = min(opts, key=opts.get) if opts else "lin"
+                if verbose:
+                    print(f"gemm M={M} N={kp[1]} K={kp[2]}: {cp} dropped (its consumer N={kc[1]} K={kc[2]} "
+                          f"runs {cc}, which would walk the per-workgroup row sums) -> core {cores[kp]}",
+                          flush=True)
 
 
 def _tg_cands(M: int, N: int, K: int):
@@ -1260,12 +1285,13 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, w
     fn = _fused_call(role, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
     if fn is None:
         return None
-    saved = _P.fused_core.get(tkey)
+    cores = _P.fused_core if wfs is None else _P.frag_core
+    saved = cores.get(tkey)
     out = {}
     try:
         for _ in range(2):   # two interleaved passes, the faster of each option's two times
             for opt in opts:
-                _P.fused_core[tkey] = opt
+                cores[tkey] = opt
                 try:
                     t = _time(fn)
                 except Exception:  # noqa: BLE001 - option not runnable for this shape
@@ -1273,10 +1299,37 @@ def _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache=None, w
                 out[opt] = min(out.get(opt, float("inf")), t)
     finally:
         if saved is None:
-            _P.fused_core.pop(tkey, None)
+            cores.pop(tkey, None)
         else:
-            _P.fused_core[tkey] = saved
+            cores[tkey] = saved
     return out
+
+
+def _best_core(opts: Dict[str, float]) -> str:
+    core = min(opts, key=opts.get)
+    one = {c: t for c, t in opts.items() if c != "lin"}
+    if core == "lin" and one and min(one.values()) <= SPLIT_MARGIN * opts["lin"]:
+        core = min(one, key=one.get)
+    return core
+
+
+def _time_dg(tkey, us: float, x, wfs) -> None:
+    """Time the decode GEMM's candidates on the copies ``wfs`` of a shape's weights; ``us``: the plan to beat."""
+    M, N, K = tkey
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    t = {p: _time(lambda i: dgemm(x, wfs[i % len(wfs)], N, EPI_PLAIN, p, y=y)) for p in _dg_cands(M, N, K)}
+    best = min(t, key=t.get, default=None)
+    _P.dg_plans[tkey] = best if best is not None and t[best] < us else None
+    if _P.dg_plans[tkey]:
+        _P.timings.setdefault((M, N, K, False), {})["dg"] = round(t[best], 2)
+
+
+def _time_frag_core(tkey, role, x, ws, wps, qkv_dims, dev, qkv_cache, wfs) -> None:
+    """The decode GEMM against the core that was chosen where there were no copies."""
+    opts = _retime_fused(tkey, role, {_P.fused_core[tkey]: 0.0}, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
+    if opts:
+        _P.fused_opts.setdefault(tkey, {}).update(opts)
+        _P.frag_core[tkey] = _best_core(opts)
 
 
 def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=None, qkv_dims=None,
@@ -1294,9 +1347,20 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
             tkey = (M, N, K)
             need_plain = key not in _P.plans
             need_tg = use_tg and not sw and (tkey not in _P.tg_plans or tkey not in _P.fused_core) and K % 64 == 0
-            if not (need_plain or need_tg):
+            role = (roles or {}).get((N, K)) if FUSED_INSITU and M <= MAX_M and os.environ.get("DLLM_FUSED_CORE") is None else None
+            # with copies there is more to choose from; what was chosen without them stands
+            need_dg = wfs is not None and M <= DG_MAX_M and tkey not in _P.dg_plans
+            need_frag = wfs is not None and M <= DG_MAX_M and role is not None and K % 64 == 0 and tkey not in _P.frag_core
+            if not (need_plain or need_tg or need_dg or need_frag):
                 continue
             x = torch.randn(M, 2 * K if sw else K, device=dev).to(torch.bfloat16)
+            plain = lambda c: _time(lambda i: _run_plan(c, x, ws[i % copies], sw, None, wps[i % copies] if wps is not None else None))  # noqa: E731
+            if not (need_plain or need_tg):
+                if need_dg:
+                    _time_dg(tkey, plain(_P.plans[key]), x, wfs)
+                if need_frag:
+                    _time_frag_core(tkey, role, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
+                continue
             cands = [("blas",)]
             if M in _GEMV_MS and K % 8 == 0 and M * K * 2 <= 64 * 1024:
                 cands.extend(("gemv", r) for r in _GEMV_RS)
@@ -1312,22 +1376,13 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                     cands.append(("skinny", ntw, s))
             if use_tg and not sw:
                 cands.extend(("tg",) + c for c in _tg_cands(M, N, K))
-            res = {}
-            for c in cands:
-                res[c] = _time(lambda i: _run_plan(c, x, ws[i % copies], sw, None,
-                                                   wps[i % copies] if wps is not None else None))
+            res = {c: plain(c) for c in cands}
             best = min(res, key=res.get)
             if need_plain:
                 _P.plans[key] = best
                 _P.timings[key] = {str(c): round(t, 2) for c, t in res.items()}
-                dg = {}
-                if wfs is not None:
-                    y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
-                    dg = {p: _time(lambda i: dgemm(x, wfs[i % copies], N, EPI_PLAIN, p, y=y)) for p in _dg_cands(M, N, K)}
-                best_dg = min(dg, key=dg.get, default=None)
-                if best_dg is not None and dg[best_dg] < res[best]:
-                    _P.dg_plans[tkey] = best_dg
-                    _P.timings[key]["dg"] = round(dg[best_dg], 2)
+            if need_dg:
+                _time_dg(tkey, res[_P.plans[key]] if _P.plans[key] in res else res[best], x, wfs)
             tgc = [c for c in res if c[0] == "tg"]
             post = None
             if need_tg and tgc:
@@ -1348,7 +1403,7 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                         opts["gemv%d" % c[1]] = _time(lambda i: ext.gemv_resadd(x, ws[i % copies], rr, sq, c[1]))
                 # small-batch MFMA GEMM with the epilogue fused (one launch), timed in its RESADD form
                 # on the weight layout the fused ops stream (the panel copy where the model keeps one)
-                if M <= SKE_MAX_M and N % 32 == 0 and K % 64 == 0 and wfs is None:
+                if M <= SKE_MAX_M and N % 32 == 0 and K % 64 == 0:
                     rr = torch.zeros(M, N, dtype=torch.bfloat16, device=dev)
                     sq = torch.empty(max_slots(N, M), M, dtype=torch.float32, device=dev)
                     src = wps if wps is not None else ws
@@ -1360,17 +1415,16 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                                                                              ssq_out=sq))
                         except Exception:  # noqa: BLE001 - workspace / shape refused
                             pass
-                role = (roles or {}).get((N, K))
-                if FUSED_INSITU and role is not None and M <= MAX_M and os.environ.get("DLLM_FUSED_CORE") is None:
-                    insitu = _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
+                if role is not None:
+                    insitu = _retime_fused(tkey, role, opts, x, ws, wps, qkv_dims, dev, qkv_cache, wfs if M <= DG_MAX_M else None)
                     if insitu:
                         opts = insitu
-                core = min(opts, key=opts.get)
-                one = {c: t for c, t in opts.items() if c != "lin"}
-                if core == "lin" and one and min(one.values()) <= SPLIT_MARGIN * opts["lin"]:
-                    core = min(one, key=one.get)
-                _P.fused_core[tkey] = core
+                        if wfs is not None and M <= DG_MAX_M:
+                            _P.frag_core[tkey] = _best_core(opts)
+                _P.fused_core[tkey] = _best_core({c: t for c, t in opts.items() if not c.startswith("dg")})
                 _P.fused_opts[tkey] = opts
+            elif need_frag and tkey in _P.fused_core:
+                _time_frag_core(tkey, role, x, ws, wps, qkv_dims, dev, qkv_cache, wfs)
             if verbose:
                 bk = {k: min((c for c in res if c[0] == k), key=res.get, default=None)
                       for k in ("gemv", "skinny", "tg")}
@@ -1380,7 +1434,7 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
                 if post is not None:
                     extra += (f" | post {post:.1f}us | fused " +
                               " ".join(f"{k}:{v:.1f}" for k, v in _P.fused_opts[tkey].items()) +
-                              f" -> core {_P.fused_core[tkey]}")
+                              f" -> core {_P.fused_core[tkey]}, with copies {_P.frag_core.get(tkey)}")
                 print(f"gemm M={M} N={N} K={K} swiglu={sw}: best={best} {res[best]:.1f}us "
                       f"({N * K * 2 / res[best] / 1e3:.0f} GB/s, {2 * M * N * K / res[best] / 1e6:.0f} TF/s; "
                       f"blas {res[('blas',)]:.1f}us; {extra})", flush=True)
@@ -1390,5 +1444,5 @@ def _autotune(shapes, ms, dev, verbose: bool, panel_shapes=frozenset(), roles=No
 def plans() -> Dict:
     d = {str(k): v for k, v in _P.plans.items()}
     d.update({"tg" + str(k): v for k, v in _P.tg_plans.items()})
-    d.update({"dg" + str(k): v for k, v in _P.dg_plans.items()})
+    d.update({"dg" + str(k): v for k, v in _P.dg_plans.items() if v})
     return d

@@ -150,3 +150,82 @@ def test_decode_gemm_in_place_of_a_skinny_plan(monkeypatch):
         for N, K in SHAPES:
             dg = of(M, N, K, True, False)[2]
             assert dg is None or G._need_dg(M, N, K, dg)[0] <= G.WS_FLOATS
+
+
+def _none_timed(monkeypatch):
+    for name in ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "fused_opts", "pf_times", "pf_small", "pf_parts"):
+        monkeypatch.setattr(G._P, name, {})
+
+
+def test_cores_with_and_without_copies(monkeypatch):
+    """One process serves models with and without fragment-major copies of the same shapes: the decode GEMM runs where there is a copy and
+    the rows are as it reads them; everything else gets what was chosen without it."""
+    monkeypatch.delenv("DLLM_FUSED_CORE", raising=False)
+    _none_timed(monkeypatch)
+    N, K = 2048, 2048
+    rows = lambda M: torch.zeros(M, K + 8, dtype=torch.bfloat16)[:, :K]  # noqa: E731
+    odd = torch.zeros(2, K + 4, dtype=torch.bfloat16)[:, :K]
+    G._P.fused_core.update({(1, N, K): "gemv2", (2, N, K): "lin", (16, N, K): "skE4", (64, N, K): "tg", (32, N, K): "tg"})
+    G._P.frag_core.update({(1, N, K): "dg1.2.2", (2, N, K): "dg1.1.4", (16, N, K): "dg2.2.2", (64, N, K): "dg1.1.2", (32, N, K): "lin"})
+    wf = torch.zeros(1)
+    assert [G.fused_dg(rows(M), N, K, wf) for M in (1, 2, 16, 32, 57, 64)] == [(1, 2, 2), (1, 1, 4), (2, 2, 2), None, (1, 1, 2), (1, 1, 2)]
+    assert all(G.fused_dg(rows(M), N, K, None) is None for M in (1, 2, 16, 32, 57, 64))
+    assert G.fused_dg(odd, N, K, wf) is None and G.use_vendor_core(2, N, K, True)
+    for frag in (False, True):      # (with copies: rows that the decode GEMM does not read)
+        assert G.fused_gemv_r(rows(1), N, frag) == 2 and G.fused_ske(rows(16), N, K, frag) == 4 and not G.use_vendor_core(64, N, K, frag)
+    assert G.use_vendor_core(32, N, K, True) and not G.use_vendor_core(32, N, K)
+    G._P.frag_core[(1, N, K)] = "skE2"      # chosen among more: not what is chosen without
+    assert G.fused_ske(rows(1), N, K, True) == 2 and G.fused_gemv_r(rows(1), N, True) == 0 and G.fused_gemv_r(rows(1), N) == 2
+
+
+def test_narrow_producers_and_their_consumers(monkeypatch):
+    _none_timed(monkeypatch)
+    shapes = [(2560, 2048), (2048, 2048), (11264, 2048), (2048, 5632)]
+    prod, cons = [(M,) + shapes[1] for M in (1, 4, 8)], [(M,) + shapes[2] for M in (1, 4, 8)]
+    G._P.fused_core.update({prod[0]: "gemv2", cons[0]: "tg", prod[1]: "lin", cons[1]: "tg", prod[2]: "gemv1", cons[2]: "skE2"})
+    G._P.frag_core.update({prod[0]: "gemv2", cons[0]: "dg2.1.1", prod[1]: "dg1.2.2", prod[2]: "dg1.1.4", cons[2]: "tg"})
+    for k in prod:
+        G._P.fused_opts[k] = {"gemv2": 3.0, "gemv1": 3.1, "dg1.2.2": 3.2, "dg1.1.4": 3.3, "dg2.1.1": 4.0, "lin": 5.0}
+    G._couple_gemv_choices(shapes, [1, 4, 8], verbose=False)
+    assert [G._P.fused_core[k] for k in prod] == ["lin", "lin", "gemv1"]
+    assert [G._P.frag_core[k] for k in prod] == ["gemv2", "dg2.1.1", "dg2.1.1"]      # a consumer timed without copies counts, too
+
+
+def test_plan_file(monkeypatch, tmp_path):
+    """What was timed comes back; a file that kept one choice for weights with and without copies has its decode GEMMs timed again."""
+    import json
+    _none_timed(monkeypatch)
+    k = (16, 2048, 2048)
+    G._P.plans[k + (False,)] = ("skinny", 2, 4)
+    G._P.tg_plans[k], G._P.fused_core[k], G._P.frag_core[k] = (64, 64, 3, 1, 1, 4), "skE4", "dg1.2.2"
+    G._P.dg_plans.update({k: (1, 2, 4), (8, 2048, 2048): None})
+    G._P.pf_times[2048, 2048], G._P.pf_small[128, 2048, 2048] = [((256, 256, 2, 1, 1, 8), 2048, 50.0)], ((64, 64, 3, 1, 1, 4), 9.0)
+    tables = ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "pf_times", "pf_small")
+    want = {n: dict(getattr(G._P, n)) for n in tables}
+    G._save_plans(str(tmp_path / "sub" / "plans.json"))
+    _none_timed(monkeypatch)
+    G._load_plans(str(tmp_path / "sub" / "plans.json"))
+    assert {n: getattr(G._P, n) for n in tables} == want
+    _none_timed(monkeypatch)
+    with open(tmp_path / "old.json", "w") as f:
+        json.dump({"c,16,2048,2048": "dg1.2.2", "c,8,2048,2048": "tg", "d,8,2048,2048": [1, 2, 4]}, f)
+    G._load_plans(str(tmp_path / "old.json"))
+    assert G._P.fused_core == {(8, 2048, 2048): "tg"} and G._P.dg_plans == {(8, 2048, 2048): (1, 2, 4)} and not G._P.frag_core
+
+
+@pytest.mark.gpu
+def test_copies_are_timed_when_they_come_second(monkeypatch):
+    """Shapes timed for a model without copies, then for one with them: the decode GEMM is timed, the earlier choices stand."""
+    _none_timed(monkeypatch)
+    monkeypatch.delenv("DLLM_FUSED_CORE", raising=False)
+    monkeypatch.delenv("DLLM_GEMM_PLANS", raising=False)
+    monkeypatch.setattr(G, "PREFILL_TUNE", False)
+    fused = [(1024, 1024), (1024, 768), (2816, 1024), (1024, 1408)]
+    tune = lambda frag: G.autotune([(n, k, False) for n, k in fused], [4, 96], "cuda", fused=fused, qkv_dims=(12, 2, 64), frag=frag)  # noqa: E731
+    tune([])
+    assert not G._P.frag_core and not G._P.dg_plans and all(not c.startswith("dg") for c in G._P.fused_core.values())
+    kept = dict(G._P.fused_core), dict(G._P.plans), dict(G._P.tg_plans)
+    tune(fused)
+    assert (G._P.fused_core, G._P.plans, G._P.tg_plans) == kept
+    assert set(G._P.dg_plans) == set(G._P.frag_core) == {(4,) + f for f in fused}
+    assert all(any(c.startswith("dg") for c in G._P.fused_opts[(4,) + f]) for f in fused)
