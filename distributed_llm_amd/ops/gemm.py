@@ -1093,18 +1093,18 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
             whole = _fused_call(roles.get((N, K)), x, ws, wps, qkv_dims, dev)
             for p in _PF_PLANS:
                 try:
-                    t = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
+                    t = t_whole = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
+                    if whole is not None:      # with its epilogue: what choosing among the plans goes by
+                        _P.pf_parts[(M, N, K)], _P.fused_core[(M, N, K)] = ((M, p),), "tg"
+                        t_whole = _time(whole, iters=8)
                 except Exception:  # noqa: BLE001 - plan refused for this shape
                     continue
+                finally:
+                    _P.pf_parts.pop((M, N, K), None)
+                    _P.fused_core.pop((M, N, K), None)      # (not timed yet: ``todo``)
                 if t < best_t:
                     best, best_t = p, t
-                if whole is not None:      # with its epilogue: what choosing among the plans goes by
-                    _P.pf_parts[(M, N, K)] = ((M, p),)
-                    saved, _P.fused_core[(M, N, K)] = _P.fused_core.get((M, N, K)), "tg"
-                    t = _time(whole, iters=8)
-                    if saved is None:
-                        del _P.fused_core[(M, N, K)]
-                times.append((p, M, t))
+                times.append((p, M, t_whole))
             if best is not None:
                 _P.tg_plans[(M, N, K)] = best
             _P.fused_core[(M, N, K)] = "tg" if best is not None and best_t < lin else "lin"
@@ -1118,10 +1118,14 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
             for p in _PF_SMALL:
                 if p[0] > max(64, M) or (p[3] > 1 and _need_tg(M, N, K, p[0], p[1], p[3])[0] > WS_FLOATS) or _tg_splits(K, p[3]) != p[3]:
                     continue
-                res[p] = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
-            best = min(res, key=res.get)
-            _P.pf_small[(M, N, K)] = (best, res[best])
-            if verbose:
+                try:
+                    res[p] = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
+                except Exception:  # noqa: BLE001 - plan refused for this shape
+                    continue
+            best = min(res, key=res.get, default=None)
+            if best is not None:
+                _P.pf_small[(M, N, K)] = (best, res[best])
+            if verbose and best is not None:
                 print(f"gemm rows M={M} N={N} K={K}: {best} {res[best]:.1f}us", flush=True)
         _P.pf_parts.clear()
         del ws, wps

@@ -229,3 +229,42 @@ def test_copies_are_timed_when_they_come_second(monkeypatch):
     assert (G._P.fused_core, G._P.plans, G._P.tg_plans) == kept
     assert set(G._P.dg_plans) == set(G._P.frag_core) == {(4,) + f for f in fused}
     assert all(any(c.startswith("dg") for c in G._P.fused_opts[(4,) + f]) for f in fused)
+
+
+@pytest.mark.parametrize("role", ["resadd", None])
+def test_refused_prompt_plans(monkeypatch, role):
+    """A plan that the product takes and its epilogue refuses, one that both refuse and small plans that are refused: left out, and nothing
+    that timing forced for them stays behind."""
+    _none_timed(monkeypatch)
+    N, K = 128, 64
+    monkeypatch.setattr(G, "PREFILL_MS", (2048, 4096))
+    monkeypatch.setattr(G, "_native", lambda x: None)
+    monkeypatch.setattr(G, "_post_us", lambda *a: 3.0)
+    us = {p: 50.0 + i for i, p in enumerate(dict.fromkeys(G._PF_PLANS + G._PF_SMALL))}
+    us[G._PF_PLANS[3]] = 10.0      # the fastest product: its epilogue is refused
+    ran = []
+
+    def tgemm(ext, x, w, epi, plan, **kw):
+        M = x.shape[0]
+        if M == 256 or (plan != G._PF_SMALL[0] if M in G.PF_SMALL_MS else plan == G._PF_PLANS[1]):
+            raise RuntimeError("no such plan")
+        ran.append(us[plan])
+
+    def whole(i):
+        (_, plan), = G.prompt_parts(ran_rows[-1], N, K)
+        assert not G.use_vendor_core(ran_rows[-1], N, K)
+        if plan == G._PF_PLANS[3]:
+            raise RuntimeError("no such epilogue")
+        ran.append(us[plan] + 5.0)
+
+    ran_rows = []
+    monkeypatch.setattr(G, "_fused_call", lambda role, x, *a: ran_rows.append(x.shape[0]) or (whole if role else None))
+    monkeypatch.setattr(G, "_tgemm", tgemm)
+    monkeypatch.setattr(G, "_time", lambda fn, iters=24: (ran.append(1e3), fn(0), ran[-1])[-1])
+    G._autotune_prefill([(N, K)], torch.device("cpu"), False, {(N, K): role} if role else {})
+    out = {G._PF_PLANS[1]} | ({G._PF_PLANS[3]} if role else set())
+    extra = 5.0 if role else 0.0
+    assert G._P.pf_times[N, K] == [(p, M, us[p] + extra) for M in (2048, 4096) for p in G._PF_PLANS if p not in out]
+    assert G._P.tg_plans == {(M, N, K): G._PF_PLANS[0 if role else 3] for M in (2048, 4096)}
+    assert set(G._P.fused_core) == {(2048, N, K), (4096, N, K)} and not G._P.pf_parts
+    assert set(G._P.pf_small) == {(M, N, K) for M in G.PF_SMALL_MS if M != 256}
