@@ -171,6 +171,7 @@ class _Planner:
         self.pf_times: Dict[Tuple[int, int], list] = {}      # (N, K) of prompts: [(plan, rows, us)]
         self.pf_small: Dict[Tuple[int, int, int], Tuple] = {}        # (rows of PF_SMALL_MS, N, K): (fastest plan, its us)
         self.pf_parts: Dict[Tuple[int, int, int], Tuple] = {}        # prompt_parts' answers
+        self.cus = 256            # CUs of the device the prompt plans were timed on
         self.ws: Dict[Tuple, Tuple[torch.Tensor, torch.Tensor]] = {}
         self.sk_tables: Dict[Tuple, Tuple[torch.Tensor, int]] = {}   # stream-K segment lists per shape
         self.timings: Dict[Tuple[int, int, int, bool], Dict[str, float]] = {}
@@ -338,15 +339,15 @@ def _rounds(tiles: int, cus: int) -> float:
     return full + (0.8 + 0.2 * rest / cus if rest else 0.0)
 
 
-def _round_us(N: int, K: int, cus: int = 256):
+def _round_us(N: int, K: int):
     """us a round of each timed prompt plan, from the largest size it was timed at."""
     out = {}
     for plan, m, t in sorted(_P.pf_times.get((N, K), ()), key=lambda e: e[1]):
-        out[plan] = t / _rounds(-(-m // plan[0]) * -(-N // plan[1]), cus)
+        out[plan] = t / _rounds(-(-m // plan[0]) * -(-N // plan[1]), _P.cus)
     return out
 
 
-def prompt_parts(M: int, N: int, K: int, cus: int = 256) -> Optional[Tuple]:
+def prompt_parts(M: int, N: int, K: int) -> Optional[Tuple]:
     """How the one-launch form of a fused product of a prompt's M > MAX_M rows runs: ((rows, plan), ...) one behind the other, or None
     where nothing was timed.  A large tile costs by rounds over the CUs: 8928 rows of 2048 columns are 280 tiles of 256 x 256, two
     rounds of which the second holds 24, so the last 736 rows go to a launch of small tiles.  us, one launch / here, TinyLlama: Wo
@@ -354,8 +355,8 @@ def prompt_parts(M: int, N: int, K: int, cus: int = 256) -> Optional[Tuple]:
     key = (M, N, K)
     if key in _P.pf_parts:
         return _P.pf_parts[key]
-    best, parts = float("inf"), None
-    rounds, usual = _round_us(N, K, cus), tg_plan(M, N, K)
+    best, parts, cus = float("inf"), None, _P.cus
+    rounds, usual = _round_us(N, K), tg_plan(M, N, K)
     tiles = lambda rows, plan: -(-rows // plan[0]) * -(-N // plan[1])
     if usual in rounds:
         best, parts = _PART_GAIN * _rounds(tiles(M, usual), cus) * rounds[usual], ((M, usual),)
@@ -1052,6 +1053,9 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     if dev.type != "cuda" or os.environ.get("DLLM_GEMM") == "blas":
         return
     reserve(dev)
+    if _P.cus != _sk_grid(dev):
+        _P.cus = _sk_grid(dev)
+        _P.pf_parts.clear()
     cache = os.environ.get("DLLM_GEMM_PLANS")  # JSON plan cache: re-use a previous run's choices
     if cache and os.path.exists(cache):
         _load_plans(cache)

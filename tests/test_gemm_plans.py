@@ -268,3 +268,29 @@ def test_refused_prompt_plans(monkeypatch, role):
     assert G._P.tg_plans == {(M, N, K): G._PF_PLANS[0 if role else 3] for M in (2048, 4096)}
     assert set(G._P.fused_core) == {(2048, N, K), (4096, N, K)} and not G._P.pf_parts
     assert set(G._P.pf_small) == {(M, N, K) for M in G.PF_SMALL_MS if M != 256}
+
+
+@pytest.mark.parametrize("cus", [64, 128, 256, 304])
+def test_prompt_parts_by_the_devices_cus(monkeypatch, cus):
+    """Rounds are over the CUs of the device at hand: two rounds and an eighth of one more become two, and a launch of small tiles."""
+    N, big, small = 2048, (256, 256, 2, 1, 1, 8), (128, 128, 3, 1, 1, 8)
+    monkeypatch.setattr(G._P, "cus", cus)
+    rows = lambda rounds: int(rounds * cus) // 8 * 256  # noqa: E731
+    monkeypatch.setattr(G._P, "pf_times", {(N, 256): [(big, rows(2), 180.0)]})
+    monkeypatch.setattr(G._P, "pf_small", {(m, N, 256): (small, 10.0) for m in G.PF_SMALL_MS})
+    monkeypatch.setattr(G._P, "tg_plans", {(m, N, 256): big for m in G.PREFILL_MS})
+    monkeypatch.setattr(G._P, "pf_parts", {})
+    tail = rows(2.125) - rows(2)
+    assert G.prompt_parts(rows(2), N, 256) == ((rows(2), big),)
+    assert tail > G.PF_SMALL_MS[-1] or G.prompt_parts(rows(2) + tail, N, 256) == ((rows(2), big), (tail, small))
+    if cus == 256:
+        assert tail <= G.PF_SMALL_MS[-1]
+
+
+@pytest.mark.gpu
+def test_rounds_count_this_devices_cus(monkeypatch):
+    monkeypatch.setattr(G._P, "cus", 7)
+    monkeypatch.setattr(G._P, "pf_parts", {(2000, 64, 64): ((2000, (64, 64, 3, 1, 1, 4)),)})
+    monkeypatch.delenv("DLLM_GEMM_PLANS", raising=False)
+    G.autotune([], [], "cuda")
+    assert G._P.cus == torch.cuda.get_device_properties(0).multi_processor_count and not G._P.pf_parts
