@@ -550,7 +550,7 @@ class HybridModel:
             takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
         todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
         extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
-        if extra > 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+        if not ops.gemm.copies_fit(extra, self.device):
             return
         for L, S in zip(self.layers, self.cfg.layers):
             f = S.mlp
@@ -566,7 +566,7 @@ class HybridModel:
               if not f32 and isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
               and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
         extra = sum(L[n].numel() * L[n].element_size() for L, _ in ex for n in ("w1", "w2"))
-        if extra <= 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+        if ops.gemm.copies_fit(extra, self.device):
             for L, f in ex:
                 L["experts_r"] = (ops.frag_experts(L["w1"], paired=f.act == "swiglu"), ops.frag_experts(L["w2"]), self.order_kept)
         if takes(self.lm_head):

@@ -180,7 +180,7 @@ class LlamaModel:
             for L in self.layers:
                 L["w13"] = L["w13"].index_select(1, idx).contiguous()
             extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in ("w13", "w2"))
-            if self.fused and extra <= 0.25 * torch.cuda.mem_get_info(self.device)[0]:
+            if self.fused and ops.gemm.copies_fit(extra, self.device):
                 for L in self.layers:     # the decode step's fragment-major copies (ops.frag_experts)
                     L["w13_r"], L["w2_r"] = ops.frag_experts(L["w13"], paired=True), ops.frag_experts(L["w2"])
 
@@ -202,25 +202,19 @@ class LlamaModel:
             if "wgu" in L:
                 L["wgu_f"] = fuse_gate_up_weight(L.pop("wgu"), L["ln2"])
         # K-panel-major copies of the fused decoder GEMM weights (ops.gemm.panel_weight): the tgemm
-        # plans stream them; the row-major weights stay for the GEMV / skinny / hipBLASLt paths.  Kept
-        # only while the copies fit in a quarter of the device memory still FREE (e.g. not
-        # Llama-3-70B at TP=1: 141 GB of weights on a 288 GB part; co-located engines and processes
-        # sharing the GPU each see what the others left), and never in the one-GPU multi-rank
-        # rehearsal (N processes would each add a copy on one card)
-        if not ops.gemm.W_PANEL or self.device.type != "cuda" or os.environ.get("DLLM_REHEARSE_ONE_GPU") == "1":
+        # plans stream them; the row-major weights stay for the GEMV / skinny / hipBLASLt paths
+        if not ops.gemm.W_PANEL or self.device.type != "cuda":
             return
         names = [n for n in self.PANEL_NAMES if n in self.layers[0] and self.layers[0][n].shape[1] % 64 == 0]
         extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in names)
-        free, _ = torch.cuda.mem_get_info(self.device)
-        if extra > 0.25 * free:
+        if not ops.gemm.copies_fit(extra, self.device):
             return
         for L in self.layers:
             for n in names:
                 L[n + "_p"] = ops.gemm.panel_weight(L[n])
         # the decode GEMM's fragment-major copies, under the same rule (of what is then left)
         extra += self.lm_head.numel() * self.lm_head.element_size()
-        free, _ = torch.cuda.mem_get_info(self.device)
-        if extra > 0.25 * free:
+        if not ops.gemm.copies_fit(extra, self.device):
             return
         for L in self.layers:
             for n in names:
