@@ -150,7 +150,7 @@ class LLMEngine:
         self.par = par
         if dtype != torch.bfloat16 and not isinstance(self.cfg, HybridConfig):
             raise ValueError(f"{self.cfg.name}: this model class serves bfloat16 only")
-        self.model = build_model(self.cfg, device=self.device, dtype=dtype, par=par, seed=seed, weights=weights)
+        self.model = build_model(self.cfg, device=self.device, dtype=dtype, par=par, seed=seed, weights=weights, fragments=False)
         self.tok = get_tokenizer(self.cfg.vocab, self.cfg.bos_id, self.cfg.eos_id, tokenizer)
         if max_model_len is None and isinstance(self.cfg, HybridConfig):
             max_model_len = 8192           # the design itself has no position limit
@@ -167,6 +167,8 @@ class LLMEngine:
         self.max_prefill_tokens = max_prefill_tokens
         self.max_blocks = (self.max_model_len + BS - 1) // BS
         self._alloc_kv(kv_cache_gb, num_kv_blocks)
+        # behind the pool: copies that only make steps faster take neither blocks from it nor of the reserve beside it
+        self.model.place_fragments(int(KV_RESERVE_GB * 2**30))
         self.bm = _need_runtime().BlockManager(self.num_blocks, BS, prefix_cache, int(self.KV_PLACEMENT))
         self._ids = itertools.count()
         self._lock = threading.Lock()          # held by the thread currently driving the step loop

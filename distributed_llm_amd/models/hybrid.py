@@ -123,7 +123,7 @@ class HybridModel:
     attn_geometry = None               # no softmax-attention split-K workspace
 
     def __init__(self, cfg: HybridConfig, device="cuda", dtype=torch.bfloat16, par: ParallelContext = SINGLE,
-                 seed: int = 0, weights: Optional[str] = None, init_std: float = 0.02):
+                 seed: int = 0, weights: Optional[str] = None, init_std: float = 0.02, fragments: bool = True):
         if par.tp_size > 1:
             raise ValueError(f"{cfg.name}: layer-list models run on one GPU (no tensor parallelism)")
         if dtype not in (torch.bfloat16, torch.float32):
@@ -156,7 +156,9 @@ class HybridModel:
         self._max_pos = 0
         raw = self._load(weights) if weights else self._random(seed, init_std)
         self._place(raw)
-        self._place_fragments()
+        self.lm_head_r: Optional[torch.Tensor] = None
+        if fragments:
+            self.place_fragments()
         self.ensure_positions(2048)
 
     # ------------------------------------------------------------------ weights
@@ -536,11 +538,10 @@ class HybridModel:
         logits by 0.004 and leaves them as far from 64 bits (0.0116, five batches) as they were."""
         return not self.cfg.pre_norm and any(m.kind == "mlstm" for L in self.cfg.layers for m in L.mixer.parts)
 
-    def _place_fragments(self) -> None:
-        """Fragment-major copies of the projections and the head for the decode GEMM (ops.gemm.frag_weight), while they fit in a
-        quarter of the memory still free.  Where the order of sums is kept, of those alone that ops.linear multiplies anyway: of an f32
-        model, whose products are the vendor's, none."""
-        self.lm_head_r: Optional[torch.Tensor] = None
+    def place_fragments(self, spare: int = 0) -> None:
+        """Fragment-major copies of the projections and the head for the decode GEMM (ops.gemm.frag_weight) and of the experts, while
+        they fit in a quarter of the memory then free beyond ``spare`` bytes.  Where the order of sums is kept, of those alone that
+        ops.linear multiplies anyway: of an f32 model, whose products are the vendor's, none."""
         f32 = self.dtype == torch.float32
         if self.device.type != "cuda" or not ops.native_available() or (f32 and self.order_kept):
             return
@@ -550,7 +551,7 @@ class HybridModel:
             takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
         todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
         extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
-        if not ops.gemm.copies_fit(extra, self.device):
+        if not ops.gemm.copies_fit(extra, self.device, spare):
             return
         for L, S in zip(self.layers, self.cfg.layers):
             f = S.mlp
@@ -566,7 +567,7 @@ class HybridModel:
               if not f32 and isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
               and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
         extra = sum(L[n].numel() * L[n].element_size() for L, _ in ex for n in ("w1", "w2"))
-        if ops.gemm.copies_fit(extra, self.device):
+        if ops.gemm.copies_fit(extra, self.device, spare):
             for L, f in ex:
                 L["experts_r"] = (ops.frag_experts(L["w1"], paired=f.act == "swiglu"), ops.frag_experts(L["w2"]), self.order_kept)
         if takes(self.lm_head):

@@ -137,7 +137,7 @@ def unfuse_gate_up_weight(wf: torch.Tensor, ln: torch.Tensor) -> torch.Tensor:
 
 class LlamaModel:
     def __init__(self, cfg: ModelConfig, device="cuda", dtype=torch.bfloat16, par: ParallelContext = SINGLE,
-                 seed: int = 0, weights: Optional[str] = None, init_std: float = 0.02):
+                 seed: int = 0, weights: Optional[str] = None, init_std: float = 0.02, fragments: bool = True):
         self.cfg = cfg
         self.device = torch.device(device)
         self.dtype = dtype
@@ -179,10 +179,8 @@ class LlamaModel:
             idx = gate_up_order(self.I).to(self.device)
             for L in self.layers:
                 L["w13"] = L["w13"].index_select(1, idx).contiguous()
-            extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in ("w13", "w2"))
-            if self.fused and ops.gemm.copies_fit(extra, self.device):
-                for L in self.layers:     # the decode step's fragment-major copies (ops.frag_experts)
-                    L["w13_r"], L["w2_r"] = ops.frag_experts(L["w13"], paired=True), ops.frag_experts(L["w2"])
+        if fragments:
+            self.place_fragments()
 
     # ------------------------------------------------------------------ fused layout
     def _fusable(self) -> bool:
@@ -212,15 +210,25 @@ class LlamaModel:
         for L in self.layers:
             for n in names:
                 L[n + "_p"] = ops.gemm.panel_weight(L[n])
-        # the decode GEMM's fragment-major copies, under the same rule (of what is then left)
-        extra += self.lm_head.numel() * self.lm_head.element_size()
-        if not ops.gemm.copies_fit(extra, self.device):
+
+    def place_fragments(self, spare: int = 0) -> None:
+        """The decode kernels' fragment-major copies (ops.gemm.frag_weight, ops.frag_experts), each kind where it fits in a quarter of the
+        memory then free beyond ``spare`` bytes; the projections' only beside their panel copies."""
+        if not self.fused:
             return
-        for L in self.layers:
-            for n in names:
-                L[n + "_r"] = ops.gemm.frag_weight(L[n], paired=n in ("wqkv_f", "wgu_f"))
-        if self.lm_head.shape[1] % 32 == 0:
-            self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
+        names = [n for n in self.PANEL_NAMES if n + "_p" in self.layers[0]]
+        extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in names) + self.lm_head.numel() * self.lm_head.element_size()
+        if names and ops.gemm.copies_fit(extra, self.device, spare):
+            for L in self.layers:
+                for n in names:
+                    L[n + "_r"] = ops.gemm.frag_weight(L[n], paired=n in ("wqkv_f", "wgu_f"))
+            if self.lm_head.shape[1] % 32 == 0:
+                self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
+        if self.moe_tg:
+            extra = sum(L[n].numel() * L[n].element_size() for L in self.layers for n in ("w13", "w2"))
+            if ops.gemm.copies_fit(extra, self.device, spare):
+                for L in self.layers:
+                    L["w13_r"], L["w2_r"] = ops.frag_experts(L["w13"], paired=True), ops.frag_experts(L["w2"])
 
     def reference_layers(self) -> List[Dict[str, torch.Tensor]]:
         """Layer weights in the plain (unfused) layout, e.g. for a CPU reference forward."""

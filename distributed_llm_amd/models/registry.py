@@ -20,5 +20,7 @@ def model_class(cfg):
 
 
 def build_model(cfg, device="cuda", dtype=torch.bfloat16, par: ParallelContext = SINGLE, seed: int = 0,
-                weights: Optional[str] = None):
-    return model_class(cfg)(cfg, device=device, dtype=dtype, par=par, seed=seed, weights=weights)
+                weights: Optional[str] = None, fragments: bool = True):
+    """``fragments``: lay out the decode kernels' weight copies at once, where they fit; False leaves that to a later
+    ``place_fragments`` (the engine's: behind its KV pool)."""
+    return model_class(cfg)(cfg, device=device, dtype=dtype, par=par, seed=seed, weights=weights, fragments=fragments)

@@ -111,11 +111,11 @@ def panel_weight(w: torch.Tensor) -> torch.Tensor:
     return w.view(N, K // 64, 64).transpose(0, 1).contiguous()
 
 
-def copies_fit(extra: int, device) -> bool:
-    """May a model lay out ``extra`` bytes of further weight copies?  While they fit in a quarter of the device memory still free (e.g. not
-    Llama-3-70B at TP=1: 141 GB of weights on a 288 GB part; co-located engines and processes sharing the GPU each see what the others
-    left), and never in the one-GPU multi-rank rehearsal (N processes would each add a copy on one card)."""
-    return os.environ.get("DLLM_REHEARSE_ONE_GPU") != "1" and extra <= 0.25 * torch.cuda.mem_get_info(device)[0]
+def copies_fit(extra: int, device, spare: int = 0) -> bool:
+    """May a model lay out ``extra`` bytes of further weight copies?  While they fit in a quarter of the device memory still free beyond
+    ``spare`` bytes (e.g. not Llama-3-70B at TP=1: 141 GB of weights on a 288 GB part; co-located engines and processes sharing the GPU
+    each see what the others left), and never in the one-GPU multi-rank rehearsal (N processes would each add a copy on one card)."""
+    return os.environ.get("DLLM_REHEARSE_ONE_GPU") != "1" and extra <= 0.25 * (torch.cuda.mem_get_info(device)[0] - spare)
 
 
 # Fragment-major weight copies of the decode GEMM (csrc/kernels/decode_gemm.hip): a wave's load of a weight fragment is one contiguous

@@ -23,6 +23,7 @@ def test_a_quarter_of_what_is_free(monkeypatch):
     monkeypatch.delenv("DLLM_REHEARSE_ONE_GPU", raising=False)
     monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d: (4000, 10000))
     assert G.copies_fit(1000, "cuda") and not G.copies_fit(1001, "cuda")
+    assert G.copies_fit(500, "cuda", 2000) and not G.copies_fit(501, "cuda", 2000) and not G.copies_fit(1, "cuda", 4000)
     monkeypatch.setenv("DLLM_REHEARSE_ONE_GPU", "1")
     assert not G.copies_fit(1, "cuda")
 
@@ -38,3 +39,36 @@ def test_none_where_ranks_share_a_gpu(monkeypatch, cfg, some):
     assert some <= set(_copies(build_model(cfg)))
     monkeypatch.setenv("DLLM_REHEARSE_ONE_GPU", "1")
     assert _copies(build_model(cfg)) == []
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg,some", MODELS, ids=lambda c: getattr(c, "name", None))
+def test_the_pool_comes_first(monkeypatch, cfg, some):
+    """Fragment-major copies are laid out behind the paged pool, out of what neither it nor the reserve beside it takes; an engine that has
+    no room for them serves without."""
+    from distributed_llm_amd.engine import llm_engine as E
+    monkeypatch.delenv("DLLM_REHEARSE_ONE_GPU", raising=False)
+    seen, alloc, info = [], E.LLMEngine._alloc_kv, torch.cuda.mem_get_info
+
+    def alloc_kv(self, *a):
+        seen.append([k for k in _copies(self.model) if not k.endswith("_p")])
+        alloc(self, *a)
+
+    monkeypatch.setattr(E.LLMEngine, "_alloc_kv", alloc_kv)
+    make = lambda **kw: E.LLMEngine(cfg, device="cuda", max_num_seqs=4, max_model_len=256, prefix_cache=False, **kw)  # noqa: E731
+    prompts = [[5, 9, 13], [7] * 20]
+    steps = lambda e: [e.feed([(k, p, [len(p) - 1]) for k, p in enumerate(prompts)])] + [  # noqa: E731
+        e.feed([(k, [11 + k + i], [0]) for k in range(2)]) for i in range(3)]
+    with_copies = make(num_kv_blocks=300)
+    assert seen == [[]] and with_copies.num_blocks == 300 and some <= set(_copies(with_copies.model))
+    want = torch.cat(steps(with_copies))
+    # a device with no more than the reserve free beside the pool that was asked for
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (int((E.KV_RESERVE_GB + 1) * 2 ** 30), info(d)[1]))
+    without = make(kv_cache_gb=8.0)
+    assert without.kv_cache_gb == 1.0
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (int(E.KV_RESERVE_GB * 2 ** 30), info(d)[1]))
+    without = make(num_kv_blocks=300)
+    assert not [k for k in _copies(without.model) if not k.endswith("_p")]
+    got = torch.cat(steps(without))
+    # other plans: bf16 roundings of a few layers
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -5
