@@ -965,3 +965,51 @@ def test_latent_up_projection(H, rank, vdim, splits, gate):
     # two roundings with a gate: the product's and the result's
     assert ((got[:T].float() - want[:T]).abs() <= 2.0 ** -7 * want[:T].abs() + 2.0 ** -16 * mag).all()
     assert (wide[T:] == 7).all() and (wide[:, H * vdim:] == 7).all()
+
+
+@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130])])
+@pytest.mark.parametrize("H,G,d,dv,rot", [(32, 8, 64, 64, 32), (4, 2, 32, 32, 32), (6, 2, 128, 200, 64), (3, 3, 256, 8, 256), (5, 1, 64, 520, 0), (33, 1, 32, 64, 16)])
+def test_attn_prep_in_vectors_against_f32(case, H, G, d, dv, rot):
+    """The same rows and places against the f32 reference on f32 pages: one rounding to bf16 (2^-8 of a value at most) of f32 sums of at
+    most 256 squares (2^-15 of a value is far more than they leave); values as they were."""
+    torch.manual_seed(16)
+    dt = torch.bfloat16
+    T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
+    proj = torch.randn(T, (H + G) * d + G * dv + 8, device=DEV).to(dt)
+    table, qscale = ops.rope_cos_sin(256, max(rot, 4), 100.0, DEV), torch.rand(H, device=DEV) * 2 + 0.5
+    slots[T // 2] = -1
+    kw, vw = kc.float(), vc.float()
+    want = ref.attn_prep(proj.float(), H, G, d, dv, table, rot, 1e-5, qscale, pos, slots, kw, vw)
+    got = seqmix.attn_prep(proj, H, G, d, dv, table, rot, 1e-5, qscale, pos, slots, kc, vc)
+    near = lambda a, b: ((a.float() - b).abs() <= (2.0 ** -8 + 2.0 ** -15) * b.abs() + 1e-6).all()  # noqa: E731
+    assert near(got, want) and near(kc, kw) and torch.equal(vc.float(), vw)
+
+
+@pytest.mark.parametrize("splits", [1, 3, 16])
+@pytest.mark.parametrize("H,G,d,dv", [(4, 4, 64, 64), (16, 1, 64, 64), (24, 2, 96, 64), (8, 2, 128, 128), (6, 3, 40, 72)])
+@pytest.mark.parametrize("opts", [{}, {"window": 40}, {"window": 100, "keep_first": 20, "sink": 0.5}, {"chunk": 64}, {"softcap": 5.0},
+                                  {"softcap": 200.0}, {"slopes": True}, {"sinks": True, "gate": True}, {"gate": "head"}])
+def test_gqa_of_few_rows_against_f32(H, G, d, dv, splits, opts):
+    """The decode form against plain f32 softmax attention: 2^-8 of a value for its rounding to bf16, 2^-13 of the largest for f32 sums in
+    another order, weights as bf16 hi + lo (2^-16 of a weight) and the fast exponentials' last bits."""
+    from distributed_llm_amd.models.llama import AttnMeta
+    torch.manual_seed(18)
+    dt = torch.bfloat16
+    case = ([1] * 10 + [1 if H // G == 16 else 2], [0, 14, 15, 16, 30, 31, 63, 64, 95, 299, 127])
+    T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
+    q = (torch.randn(T, H, d, device=DEV) * 0.5).to(dt)
+    kw = dict(opts)
+    gate = kw.pop("gate", None)
+    if gate is not None:
+        gate = torch.randn(T, H if gate == "head" else H * dv, device=DEV).to(dt)
+    for name in ("slopes", "sinks"):
+        if kw.pop(name, None):
+            kw[name] = torch.rand(H, device=DEV) + 0.1
+    meta = AttnMeta(slots=None, block_tables=bt, qstart=qstart, qlen=qlen, ctx=ctx, tile_seq=None, tile_tok0=None,
+                    last_idx=None, host_qlen=case[0])
+    ts, tt = meta.latent_tiles(1, DEV, seqmix.gqa_tokens_per_tile(H, G, True))
+    assert T * (H // G) <= 16 * ts.numel()
+    want = ref.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, gate, out_f32=True, **kw)
+    got = seqmix.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, ts, tt, gate, True, splits, **kw).float()
+    assert torch.isfinite(want).all()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all()
