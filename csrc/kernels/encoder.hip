@@ -198,7 +198,7 @@ int launch_enc_gemm(const u16* x, long ldx, const u16* w, const u16* bias, u16* 
 // LayerNorm + up + GELU, down + residual (enc_gemm).  A launch of this size costs 3 to 4 us whatever it does, so a workgroup
 // recomputes what passed between two of them for all rows (16 rows x 384 columns are a few KB in L2) and multiplies it with its 16
 // columns of the next product.  All waves share the first part, a row or a head each; what they leave in LDS as bf16 rows one wave
-// multiplies, in enc_gemm's four partial sums, which makes its bits.  Six layers of 384 / 1536 on 16 rows: 154 -> 135 us.  More rows
+// multiplies, in enc_gemm's four partial sums, which makes its bits.  Six layers of 384 / 1536 on 16 rows, in a captured graph: 144 -> 124 us.  More rows
 // repeat too much: with as many row tiles a workgroup, 32 rows took 185 us against 171, 64 299 against 214.
 constexpr int FEW_M = 16, FEW_K = 384, FEW_LD = FEW_K + 8;      // most rows and columns; LDS rows 16 bytes apart in the banks
 struct FewW {
