@@ -286,7 +286,7 @@ __global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ 
 
 // y += attention(qkv) . w^T + bias.  A wave takes a head, all queries and keys.  S^T = K . Q^T leaves a query's scores in one lane
 // column and P^T feeds O^T = V^T . P^T as in encoder_attn, in its key order (keys 16 to 31 of a step are zero).  Rows of other texts
-// are masked by the text's bounds.
+// are masked by the text's bounds; where a head's values are not all finite (0 times one is NaN) each text is multiplied by itself.
 template <int D>
 __global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __restrict__ qkv, const u16* __restrict__ Vt,
                                                                   const u16* __restrict__ W, const u16* __restrict__ bias,
@@ -345,9 +345,27 @@ __global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __r
   l = lane_add(l, 32);
   const float inv = l > 0.f ? 1.f / l : 0.f;
   const bf16x8 pf = __builtin_bit_cast(bf16x8, pack8(p));
+  bool lost = false;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
-    const f32x4 o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[n], pf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    const uint4 x = __builtin_bit_cast(uint4, vf[n]);
+    const unsigned e = 0x7f80u;      // an exponent of ones: an infinity or NaN
+    lost |= (x.x & e) == e || (x.x >> 16 & e) == e || (x.y & e) == e || (x.y >> 16 & e) == e;
+  }
+  const bool apart = __any(lost);
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    if (!apart) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[n], pf, o, 0, 0, 0);
+    else
+      for (int t = 0; t < B; ++t) {
+        const int a = __builtin_amdgcn_readlane(ts, t), e = a + __builtin_amdgcn_readlane(tn, t), k = 4 * g;
+        uint4 v = __builtin_bit_cast(uint4, vf[n]);
+        v.x &= (k >= a && k < e ? 0xffffu : 0u) | (k + 1 >= a && k + 1 < e ? 0xffff0000u : 0u);
+        v.y &= (k + 2 >= a && k + 2 < e ? 0xffffu : 0u) | (k + 3 >= a && k + 3 < e ? 0xffff0000u : 0u);
+        const f32x4 mine = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v), pf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (lr >= a && lr < e) o = mine;
+      }
     u16x4 z;
 #pragma unroll
     for (int i = 0; i < 4; ++i) z.v[i] = f2bf(o[i] * inv);

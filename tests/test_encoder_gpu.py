@@ -150,7 +150,8 @@ def test_few_row_projections(M, N, K):
 
 
 @pytest.mark.parametrize("lens", [[1], [15], [16], [17], [9, 7], [1] * 16, [1, 0, 12]])
-@pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (6, 64, 320), (3, 64, 96), (1, 32, 32), (5, 32, 64)])
+@pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (6, 64, 320), (3, 64, 96), (1, 32, 32), (5, 32, 64), (3, 64, 128), (2, 32, 64), (10, 32, 704),
+                                        (1, 64, 64)])      # (widths that are no whole 64s take one launch an operation)
 def test_layers_of_few_rows(lens, nh, d, inter):
     """Four launches a layer against one per operation.  A single text meets the same sums in the same order: equal bits.
     Among several, a text's keys lie in other lanes and its sums take another order: rows then lie no further from a
@@ -180,3 +181,22 @@ def test_layers_of_few_rows(lens, nh, d, inter):
         assert torch.equal(got, x)
     rms = lambda t: float((t.cpu().double() - y).square().mean().sqrt())  # noqa: E731
     assert rms(got) <= 1.1 * rms(x) + 1e-9, (rms(got), rms(x))
+
+
+@pytest.mark.parametrize("lens,bad", [([9, 7], 0), ([9, 7], 1), ([1] * 16, 5), ([3, 1, 0, 4, 8], 3), ([16], 0), ([5, 0, 2], 2)])
+@pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (6, 64, 320), (3, 64, 128), (5, 32, 64)])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_not_finite_rows_of_few_stay_in_their_text(lens, bad, nh, d, inter, value):
+    """One row of one text is not finite: that text's rows are lost, every other text's are the bits they are without it."""
+    torch.manual_seed(sum(lens) + inter)
+    H, T, S = nh * d, sum(lens), max(lens)
+    layers = [dict(wqkv=_b(3 * H, H, scale=0.05), bqkv=_b(3 * H), wo=_b(H, H, scale=0.05), bo=_b(H), ln1=(_b(H) + 1, _b(H)), w1=_b(inter, H, scale=0.05),
+                   b1=_b(inter), w2=_b(H, inter, scale=0.05), b2=_b(H), ln2=(_b(H) + 1, _b(H))) for _ in range(2)]
+    x, starts = _b(T, H), [sum(lens[:i]) for i in range(len(lens))]
+    dl, ds = (torch.tensor(v, dtype=torch.int32).cuda() for v in (lens, starts))
+    want = ops.gemm.encoder_layers(x.clone(), dl, ds, S, nh, d, 1e-12, layers)
+    x[starts[bad] + lens[bad] - 1, 7] = value
+    got = ops.gemm.encoder_layers(x.clone(), dl, ds, S, nh, d, 1e-12, layers)
+    mine = torch.zeros(T, dtype=torch.bool, device="cuda")
+    mine[starts[bad]:starts[bad] + lens[bad]] = True
+    assert torch.isfinite(want).all() and got[mine].isnan().all() and torch.equal(got[~mine], want[~mine])
