@@ -1423,7 +1423,8 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
     else if (d <= 192 && dv <= 128) GQT(192, 128, CAP, DIST);                                                            \
     else GQT(256, 256, CAP, DIST);                                                                                       \
   } while (0)
-    // at most 16 rows a tile on average: decode steps.  Not where key heads share their values or the result is f32: those are the maps
+    // at most 16 rows a tile on average: decode steps.  (Heads of a group of one with fewer than 100 keys take up to 1.6 us longer than as tiles,
+    // 64 sequences of 64 8.0 / 9.6; 200 keys 16.6 / 12.7.)  Not where key heads share their values or the result is f32: those are the maps
     // of differential attention, whose difference keeps the order of sums of paged_gqa_mfma
     if (GV == G && !out32 && d <= 128 && dv <= 128 && T * (H / G) <= 16L * n_tiles) {
 #define GQM(KD, VD, CAP, DIST)                                                                                                   \
@@ -1446,8 +1447,12 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
 #undef GQZ
 #undef GQT
     if (pp) {
-      const int rows = (TQ * (H / G) < GM_ROWS ? TQ * (H / G) : GM_ROWS);
-      hipLaunchKernelGGL(gqa_combine_kernel, dim3(n_tiles, G, (rows + 3) / 4), dim3(256), 0, st, pp, splits, qstart, qlen,
+      // a wave asks for its row's partials before it knows that there is such a row, so the launch has waves for four times the rows that
+      // tiles have on average (all of a decode step's) and goes round where a tile has more.  With waves for every row a tile could
+      // have, their loads cost more than they hide: 64 sequences of 100 keys, 16 heads of 64 on 4, two splits 14.9 us, here 11.8
+      const int R = H / G, full = TQ * R < GM_ROWS ? TQ * R : GM_ROWS;
+      const long rows = T <= n_tiles ? R : 4 * ((T * R + n_tiles - 1) / n_tiles);
+      hipLaunchKernelGGL(gqa_combine_kernel, dim3(n_tiles, G, (unsigned)((rows < full ? rows : full) + 3) / 4), dim3(256), 0, st, pp, splits, qstart, qlen,
                          tile_seq, tile_tok0, (const u16*)gate, ldg, (u16*)out, H, G, dv, TQ, out32, sink, sinks, ldo, ghead);
     }
     return (int)hipGetLastError();

@@ -1013,3 +1013,25 @@ def test_gqa_of_few_rows_against_f32(H, G, d, dv, splits, opts):
     got = seqmix.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, ts, tt, gate, True, splits, **kw).float()
     assert torch.isfinite(want).all()
     assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("splits", [2, 5, 16])
+@pytest.mark.parametrize("qlens,starts,padding", [([16] + [1] * 20, [30] + [7 * i for i in range(20)], 0), ([2, 1, 1], [100, 5, 40], 6), ([3] * 5, [1, 2, 3, 64, 200], 0),
+                                                  ([1] * 9, [50 * i for i in range(9)], 7), ([40, 1], [0, 9], 0)])
+@pytest.mark.parametrize("H,G,d,dv", [(8, 2, 64, 64), (4, 4, 32, 32), (24, 2, 64, 64), (4, 1, 256, 200)])
+def test_merge_of_key_splits_goes_round(H, G, d, dv, qlens, starts, padding, splits):
+    """The merging launch has waves for a multiple of the rows that tiles have on average: a tile of many rows beside tiles of one, tiles of
+    no row (decode steps are padded with an empty sequence's), more tiles than tokens.  Against plain f32 attention, as above."""
+    from distributed_llm_amd.models.llama import AttnMeta
+    torch.manual_seed(20)
+    dt = torch.bfloat16
+    qlens, starts = qlens + [0], starts + [0]
+    T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages((qlens, starts), G, d, dv, dt)
+    q = (torch.randn(T, H, d, device=DEV) * 0.5).to(dt)
+    meta = AttnMeta(slots=None, block_tables=bt, qstart=qstart, qlen=qlen, ctx=ctx, tile_seq=None, tile_tok0=None,
+                    last_idx=None, host_qlen=qlens)
+    ts, tt = meta.latent_tiles(1, DEV, seqmix.gqa_tokens_per_tile(H, G, True))
+    ts, tt = torch.cat([ts, i32([len(qlens) - 1] * padding)]), torch.cat([tt, i32([0] * padding)])
+    want = ref.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, out_f32=True)
+    got = seqmix.paged_gqa_attention(q, kc, vc, bt, qstart, qlen, ctx, ts, tt, None, True, splits).float()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all()
