@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(const T* __restrict__ pr
 // workgroup covers 16 tokens (blockIdx.x) and one such group of heads, or (the last blockIdx.y) 512 value entries, turned in LDS so that
 // the 16 tokens of an entry, which lie side by side in V^T's page, are stored by neighbouring lanes.  Element by element it is bound by
 // 2-byte accesses, made twice, and by a sector for each value: 7300 tokens, 32 + 8 heads of 64 and as many values 123 us, here 32 (the
-// bytes alone: 15); a decode step's six tokens 5.2, here 4.9.
+// bytes alone: 15).  Where it begins: dllm_attn_prep.
 // A lane's eight squares are added in the order that the wave's exchanges have there (D = 64: the same bits).
 constexpr int APV_T = 16, APV_V = 512;
 template <int D>
@@ -1350,8 +1350,11 @@ extern "C" int dllm_attn_prep(const void* proj, long ld, int f32, int H, int G, 
                               void* vc, void* q, long T, int BSZ, hipStream_t st) {
   if (T <= 0) return 0;
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w) return -1;
-  // whole vectors: heads of 32 to 256, halves of the rotation and values in eights, 16-byte aligned rows
-  if (!f32 && (d == 32 || d == 64 || d == 128 || d == 256) && dv % 8 == 0 && rot % 16 == 0 && ld % 8 == 0 && tab_w % 4 == 0 && T < (1 << 20) &&
+  // whole vectors: heads of 32 to 256, halves of the rotation and values in eights, 16-byte aligned rows; and enough of them: 16 tokens a
+  // workgroup leave few steps' worth of waves, of which each waits for all its loads (element by element / here, us, heads + key heads
+  // x width: 40 x 64, 6 tokens 3.2 / 4.0, 64 3.8 / 5.8, 192 5.4 / 5.9, 256 6.3 / 6.0; 20 x 64, 384 5.4 / 5.9, 512 6.4 / 6.0; 5 x 256, 700 6.0 / 6.3,
+  // 1500 9.3 / 7.9; 32 x 128, 128 4.5 / 5.0, 192 5.4 / 5.2)
+  if (T * (H + G) * (d + 128) >= 2000000 && !f32 && (d == 32 || d == 64 || d == 128 || d == 256) && dv % 8 == 0 && rot % 16 == 0 && ld % 8 == 0 && tab_w % 4 == 0 && T < (1 << 20) &&
       (((uintptr_t)proj | (uintptr_t)cos_sin | (uintptr_t)kc | (uintptr_t)q) & 15) == 0) {
     const int ny = ((H + G) * (d / 8) + 63) / 64;
     const dim3 g(((unsigned)T + APV_T - 1) / APV_T, ny + (G * dv + APV_V - 1) / APV_V);

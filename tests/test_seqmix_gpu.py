@@ -844,20 +844,26 @@ def test_biased_attention_kernels(dt, case, H, G, d, dv, win):
         seqmix.paged_gqa_attention(q2, kc2, vc2, bt, qstart, qlen, ctx, ts, tt, None, mfma, 1, softcap=3.0, slopes=slopes)
 
 
-@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130])])
+def _enough_for_vectors(H, G, d, odd):
+    """Portions of as many tokens as the vector form of attn_prep asks for (csrc/kernels/gqa.hip dllm_attn_prep), and ``odd`` more."""
+    return [-(-2000000 // ((H + G) * (d + 128))) + odd - 5, 5], [0, 90]
+
+
+@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130]), 0, 1, 15])
 @pytest.mark.parametrize("H,G,d,dv,rot", [(32, 8, 64, 64, 32), (4, 2, 32, 32, 32), (6, 2, 128, 200, 64), (3, 3, 256, 8, 256), (5, 1, 64, 520, 0), (33, 1, 32, 64, 16)])
 def test_attn_prep_in_vectors(case, H, G, d, dv, rot):
     """bf16 rows of whole vectors: groups of heads and of tokens full and not, a value block of 512 that ends inside, rows without a slot;
     against the element-by-element form of the same rows at an odd offset (a rounding apart: a head's sum of squares may be added in
-    another order)."""
+    another order).  Steps of few tokens take the element-by-element form either way."""
     torch.manual_seed(6)
     dt = torch.bfloat16
+    case = _enough_for_vectors(H, G, d, case) if isinstance(case, int) else case
     T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
     n = (H + G) * d + G * dv
     proj = torch.randn(T, n + 8, device=DEV).to(dt)
     odd = torch.empty(T, n + 9, dtype=dt, device=DEV)
     odd[:, :n] = proj[:, :n]
-    table = ops.rope_cos_sin(256, max(rot, 4), 100.0, DEV)
+    table = ops.rope_cos_sin(4096, max(rot, 4), 100.0, DEV)
     qscale = torch.rand(H, device=DEV) * 2 + 0.5
     slots[T // 2] = -1
     kc2, vc2 = kc.clone(), vc.clone()
@@ -885,9 +891,9 @@ def test_joint_head_norm(dt, H, dv):
     assert not o1[T:].any()
 
 
-@pytest.mark.parametrize("n", [8, 2048, 2056, 8 * 256 * 8192 + 8])
+@pytest.mark.parametrize("n", [8, 2048, 2056, (1 << 19) - 8, 1 << 19, (1 << 19) + 8, 8 * 256 * 8192 + 8])
 def test_gelu_in_vectors(n):
-    """Bits of the element-by-element form (an odd offset), one vector, a block of them and more than the grid holds."""
+    """Bits of the element-by-element form (an odd offset) on both sides of the line, at whole blocks and not, and past what the grid holds."""
     x = (torch.randn(n + 1, device=DEV) * 3).bfloat16()
     assert torch.equal(seqmix.gelu_erf(x[1:].clone()), seqmix.gelu_erf(x)[1:])
 
@@ -967,16 +973,17 @@ def test_latent_up_projection(H, rank, vdim, splits, gate):
     assert (wide[T:] == 7).all() and (wide[:, H * vdim:] == 7).all()
 
 
-@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130])])
+@pytest.mark.parametrize("case", CASES + [([40, 3], [90, 130]), 0, 1, 15])
 @pytest.mark.parametrize("H,G,d,dv,rot", [(32, 8, 64, 64, 32), (4, 2, 32, 32, 32), (6, 2, 128, 200, 64), (3, 3, 256, 8, 256), (5, 1, 64, 520, 0), (33, 1, 32, 64, 16)])
 def test_attn_prep_in_vectors_against_f32(case, H, G, d, dv, rot):
     """The same rows and places against the f32 reference on f32 pages: one rounding to bf16 (2^-8 of a value at most) of f32 sums of at
     most 256 squares (2^-15 of a value is far more than they leave); values as they were."""
     torch.manual_seed(16)
     dt = torch.bfloat16
+    case = _enough_for_vectors(H, G, d, case) if isinstance(case, int) else case
     T, qstart, qlen, ctx, pos, bt, kc, vc, slots = _pages(case, G, d, dv, dt)
     proj = torch.randn(T, (H + G) * d + G * dv + 8, device=DEV).to(dt)
-    table, qscale = ops.rope_cos_sin(256, max(rot, 4), 100.0, DEV), torch.rand(H, device=DEV) * 2 + 0.5
+    table, qscale = ops.rope_cos_sin(4096, max(rot, 4), 100.0, DEV), torch.rand(H, device=DEV) * 2 + 0.5
     slots[T // 2] = -1
     kw, vw = kc.float(), vc.float()
     want = ref.attn_prep(proj.float(), H, G, d, dv, table, rot, 1e-5, qscale, pos, slots, kw, vw)
