@@ -1654,7 +1654,8 @@ extern "C" int dllm_depth_mix(float* X, const float* w, int n, long T, int H, co
 
 extern "C" int dllm_gelu_erf(const void* x, void* y, int f32, long n, hipStream_t st) {
   if (n <= 0) return 0;
-  if (!f32 && n % 8 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0) {
+  // (a vector a lane from half a million entries: 2^18 2.6 / 3.0 us, 2^19 3.1 / 3.0, 2^21 6.2 / 4.4; fewer leave CUs idle)
+  if (!f32 && n >= 1 << 19 && n % 8 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0) {
     const long g = (n / 8 + 255) / 256;
     hipLaunchKernelGGL(gelu_erf_vec_kernel, dim3((unsigned)(g > 8192 ? 8192 : g)), dim3(256), 0, st, (const uint4*)x, (uint4*)y, n / 8);
     return (int)hipGetLastError();
