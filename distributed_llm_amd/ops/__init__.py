@@ -487,6 +487,11 @@ MOE_PLANS = {  # (bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2) by rou
 # at 256).  Routing, both products and the sum, us grouped / here: 8 experts of 1024 x 1024 (SwiGLU, top 2) 1 token 28 / 12, 12 31 / 16,
 # 64 32 / 24; with a shared expert (squared ReLU) 1 token 27 / 12, 24 28 / 18, 42 29 / 23, 48 34 / 24, 64 34 / 28.
 MOE_FEW, MOE_FEW_TOKENS = 256, 64
+# Weights beyond the Infinity Cache (entries of both): the grouped GEMM, whose tiles hold the rows, then streams as fast, and here every column
+# tile reads its expert's rows once more.  Pairs an expert up to which this is the faster one: 8 experts of 4096 x 7168 10 pairs 275 / 267 us,
+# 12 265 / 279, 16 267 / 325; 4096 x 3584 12 152 / 145, 16 152 / 169; 2048 x 2816 12 62 / 55, 16 62 / 66; 4 of 4096 x 3584 16 98 / 87, 20 95 / 99.
+# One wave a tile: 2 to 4 experts of 1024 x 1024 24 pairs 26 / 19, 32 26 / 26, 64 26 / 29.
+MOE_FEW_CACHED, MOE_FEW_ROWS, MOE_FEW_ROWS_IN_ORDER = 128 << 20, 10, 24
 
 
 def frag_experts(w: torch.Tensor, paired: bool = False) -> torch.Tensor:
@@ -500,7 +505,14 @@ def moe_few(x: torch.Tensor, ids: torch.Tensor, frag) -> dict:
     the grouped GEMM's sums one wave walks all of K, else four share it."""
     if frag is None or not 0 < ids.numel() <= MOE_FEW or x.shape[0] > MOE_FEW_TOKENS or x.data_ptr() % 16:
         return {}
-    return dict(w13f=frag[0], w2f=frag[1], few_ks=1 if len(frag) > 2 and frag[2] else 4)
+    in_order = len(frag) > 2 and frag[2]
+    if frag[0].numel() + frag[1].numel() > MOE_FEW_CACHED:
+        most = MOE_FEW_ROWS
+    else:
+        most = MOE_FEW_ROWS_IN_ORDER if in_order else MOE_FEW
+    if ids.numel() > most * frag[0].shape[0]:
+        return {}
+    return dict(w13f=frag[0], w2f=frag[1], few_ks=1 if in_order else 4)
 
 
 def moe_plan(pairs: int) -> Tuple[int, ...]:

@@ -6,7 +6,6 @@ import torch
 from distributed_llm_amd import ops
 from distributed_llm_amd.ops import seqmix
 
-pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
@@ -29,6 +28,7 @@ def all_sizes(monkeypatch):
     monkeypatch.setattr(ops, "MOE_FEW_TOKENS", 256)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("T,E,k,H,I", [(1, 8, 2, 1024, 1024), (5, 3, 2, 64, 192), (12, 8, 2, 1024, 1024), (17, 4, 3, 320, 64), (33, 9, 3, 1024, 512),
                                        (64, 8, 2, 128, 256), (64, 64, 4, 192, 128), (85, 2, 3, 64, 64)])
@@ -46,6 +46,7 @@ def test_bits_of_the_grouped_gemm(mode, T, E, k, H, I, same):
         assert torch.equal(got, want)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("T,groups", [(1, 1), (24, 4), (40, 1)])
 def test_sum_ends_in_the_stream(mode, T, groups):
@@ -59,6 +60,7 @@ def test_sum_ends_in_the_stream(mode, T, groups):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 12, 64])
 def test_sum_added_to_the_residual(T):
     x, ids, wts, w1, w2, frag, _ = _case(T, 8, 2, 1024, 256, 0, False)
@@ -68,3 +70,20 @@ def test_sum_added_to_the_residual(T):
         n = ops.moe_ffn_tg_resadd(x, ids, wts, w1, w2, r, ssq, frag=f)
         out.append((r, ssq[:n]))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+class _Fragments:
+    """frag_experts' shape of weights, without the weights."""
+    def __init__(self, E, N, K):
+        self.shape, self.numel = (E, N // 16, K // 32, 64, 8), lambda: E * N * K
+
+
+@pytest.mark.parametrize("E,k,H,I,order,tokens", [(8, 2, 1024, 1024, False, 64), (8, 2, 1024, 1024, True, 64), (8, 2, 4096, 3584, False, 40), (8, 2, 4096, 3584, True, 40),
+                                                  (2, 2, 1024, 1024, False, 64), (2, 2, 1024, 1024, True, 24), (64, 4, 2048, 1408, False, 64),
+                                                  (4, 2, 4096, 3584, False, 20), (1, 1, 512, 512, True, 24), (8, 8, 256, 256, False, 32)])
+def test_how_many_are_few(monkeypatch, E, k, H, I, order, tokens):
+    """The most tokens that run on the fragment-major copies: of large experts, and of one wave a tile, by the pairs an expert has."""
+    monkeypatch.setattr(ops, "MOE_FEW_TOKENS", 64)
+    frag = (_Fragments(E, 2 * I, H), _Fragments(E, H, I)) + ((True,) if order else ())
+    few = lambda T: ops.moe_few(torch.zeros(T, 8, dtype=torch.bfloat16), torch.zeros(T, k, dtype=torch.int32), frag)  # noqa: E731
+    assert few(1)["few_ks"] == few(tokens)["few_ks"] == (1 if order else 4) and few(tokens + 1) == {} and few(0) == {}
