@@ -103,7 +103,7 @@ def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, kee
     """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy."""
     if wf is not None and ops.gemm.dg_takes(x):
         return ops.linear(x, w, wf=wf, keep_order=keep_order)
-    if wf is not None and ops.gemm.fg_takes(x):
+    if wf is not None and ops.gemm.fg_takes(x, w.shape[0]):
         return ops.gemm.f32_linear(x, wf, w.shape[0])
     if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1
             and x.shape[1] % 64 == 0 and w.shape[0] % 64 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
@@ -1050,7 +1050,7 @@ class HybridModel:
         act, a = self._act_args(f), None
         if "up_act_r" in L:
             a = ops.gemm.linear_act(x, L["up"], L["up_act_r"], act[0], L.get("up_b"), act[1], act[2], L["order_kept"])
-        elif "up_r" in L and act is not None and act[0] == "gelu" and ops.gemm.fg_takes(x):
+        elif "up_r" in L and act is not None and act[0] == "gelu" and ops.gemm.fg_takes(x, L["up"].shape[0]):
             a = ops.gemm.f32_linear(x, L["up_r"], L["up"].shape[0], gelu=True)
         if a is None:
             z = _pm(x, L, "up")

@@ -294,3 +294,14 @@ def test_rounds_count_this_devices_cus(monkeypatch):
     monkeypatch.delenv("DLLM_GEMM_PLANS", raising=False)
     G.autotune([], [], "cuda")
     assert G._P.cus == torch.cuda.get_device_properties(0).multi_processor_count and not G._P.pf_parts
+
+
+def test_which_f32_products_are_taken(monkeypatch):
+    monkeypatch.delenv("DLLM_GEMM", raising=False)
+    rows = lambda M, K: torch.zeros(M, K)  # noqa: E731
+    for M in range(1, 9):
+        assert all(G.fg_takes(rows(M, K), N) for N in (16, 8192, 32000) for K in (512, 2048))
+    for M, K, N, yes in [(9, 1024, 32000, True), (12, 1024, 32000, True), (13, 1024, 32000, False), (16, 1024, 16384, True), (16, 1024, 16, True),
+                         (16, 2048, 128, False), (9, 2048, 8192, False), (16, 2048, 512, True), (16, 2048, 4096, True), (17, 512, 512, False)]:
+        assert G.fg_takes(rows(M, K), N) == yes and G.fg_takes(rows(M, K)) == (M <= 16)
+    assert not G.fg_takes(torch.zeros(4, 520)[:, 1:513], 512) and not G.fg_takes(rows(4, 512).bfloat16(), 512)
