@@ -119,8 +119,8 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   u16* op = out + (row0 + q) * H + h * D;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
-    const uint32_t lo = (uint32_t)f2bf(acc[n][0] * inv) | ((uint32_t)f2bf(acc[n][1] * inv) << 16);
-    const uint32_t hi = (uint32_t)f2bf(acc[n][2] * inv) | ((uint32_t)f2bf(acc[n][3] * inv) << 16);
+    const uint32_t lo = f2bf2(acc[n][0] * inv, acc[n][1] * inv);
+    const uint32_t hi = f2bf2(acc[n][2] * inv, acc[n][3] * inv);
     *reinterpret_cast<uint2*>(op + 16 * n + 4 * g) = make_uint2(lo, hi);
   }
 }

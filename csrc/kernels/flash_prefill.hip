@@ -368,8 +368,8 @@ __global__ void __launch_bounds__(512, MINW) flash_prefill_kernel(FlashArgs a) {
   for (int n = 0; n < NB; ++n)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const uint32_t lo = (uint32_t)f2bf(acc[n][4 * g] * inv) | ((uint32_t)f2bf(acc[n][4 * g + 1] * inv) << 16);
-      const uint32_t hi = (uint32_t)f2bf(acc[n][4 * g + 2] * inv) | ((uint32_t)f2bf(acc[n][4 * g + 3] * inv) << 16);
+      const uint32_t lo = f2bf2(acc[n][4 * g] * inv, acc[n][4 * g + 1] * inv);
+      const uint32_t hi = f2bf2(acc[n][4 * g + 2] * inv, acc[n][4 * g + 3] * inv);
       *reinterpret_cast<uint2*>(o + 32 * n + 8 * g) = make_uint2(lo, hi);
     }
 }

@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(256) latent_expand_kernel(const u16* __restric
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const f32x4 a = acc[t][b];
-        const uint2 v = make_uint2((uint32_t)f2bf(a[0]) | ((uint32_t)f2bf(a[1]) << 16), (uint32_t)f2bf(a[2]) | ((uint32_t)f2bf(a[3]) << 16));
+        const uint2 v = make_uint2(f2bf2(a[0], a[1]), f2bf2(a[2], a[3]));
         const int c0 = (b0 + b) * 16;
         if (key) {
           if (c0 + 4 * g4 < d) *reinterpret_cast<uint2*>(kc + (page * 16 + lr) * kd + c0 + 4 * g4) = v;

@@ -286,8 +286,8 @@ template <> struct vec4<u16> {
                        __uint_as_float(w.y & 0xffff0000u));
   }
   static __device__ __forceinline__ void st(u16* p, float4 v) {
-    *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f2bf(v.x) | ((uint32_t)f2bf(v.y) << 16),
-                                              (uint32_t)f2bf(v.z) | ((uint32_t)f2bf(v.w) << 16));
+    *reinterpret_cast<uint2*>(p) = make_uint2(f2bf2(v.x, v.y),
+                                              f2bf2(v.z, v.w));
   }
 };
 
