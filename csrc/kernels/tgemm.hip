@@ -34,7 +34,7 @@
 // m-tiles / k-splits) share one XCD's L2.  Optional split-K over k with the in-launch
 // last-arriver combine (write-through f32 slabs + relaxed ticket, Guideline 16 R1).
 #include "common.h"
-#include "tgemm_args.h"
+#include "tgemm_shared.h"
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -47,6 +47,7 @@ using dllm::EPI_SWIGLU;
 using dllm::EPI_GELU;
 using dllm::EPI_RELU2;
 using dllm::EPI_F32;
+using dllm::qkv_copy_out;
 constexpr int BK = 64;
 constexpr int ROWB = BK * 2;  // 128 bytes per staged row
 
@@ -666,11 +667,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
   }
 
   if constexpr (EPI == EPI_QKV) {
-    // The tile is staged row-scaled and rounded; the copy-out rotates row vectors of eight pairs.  (Rotated in registers every lane
-    // waited for the table rows of its FM x 4 output rows one after the other, and V went out in 2-byte stores 32 B apart: of a
-    // 256 x 128 tile's 54 us at 2100 rows that was 21.)
-    const int d = a.d, hd = d / 2, nq = a.nq, nkv = a.nkv;
-    const int qcols = nq * d, kcols = nkv * d, vcol0 = qcols + kcols;
+    // the tile is staged row-scaled and rounded; the copy-out rotates row vectors of eight pairs
     int* s_slot = reinterpret_cast<int*>(s_red);   // [BM] cache slot, [BM] position per tile row
     int* s_pos = s_slot + BM;
 #pragma unroll
@@ -687,69 +684,8 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
           for (int j = 0; j < FN; ++j) so[(rl0 + 16 * i + e) * OLD + wn * WN + 16 * j + cl] = f2bf(acc[i][j][e] * rinv[i][e]);
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < BM * (BN / 16); e += NT) {
-      const int rl = e / (BN / 16), u = e % (BN / 16), c0 = 32 * (u >> 1) + 8 * (u & 1);
-      const int m = m0 + rl, n = n0 + c0;
-      if (m >= M || n >= vcol0 || n >= N) continue;
-      const bool isq = n < qcols;
-      const int cc = isq ? n : n - qcols, head = cc / d, o = cc % d, d1 = 16 * (o >> 5) + (o & 15);
-      const float* cs = a.cos_sin + (long)s_pos[rl] * d + d1;
-      float co[8], si[8], x1[8], x2[8], r1[8], r2[8];
-      *(float4*)&co[0] = *(const float4*)cs;
-      *(float4*)&co[4] = *(const float4*)(cs + 4);
-      *(float4*)&si[0] = *(const float4*)(cs + hd);
-      *(float4*)&si[4] = *(const float4*)(cs + hd + 4);
-      unpack8(*reinterpret_cast<const uint4*>(so + rl * OLD + c0), x1);
-      unpack8(*reinterpret_cast<const uint4*>(so + rl * OLD + c0 + 16), x2);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        r1[j] = x1[j] * co[j] - x2[j] * si[j];
-        r2[j] = x2[j] * co[j] + x1[j] * si[j];
-      }
-      const int slot = s_slot[rl];
-      u16* dst = isq ? a.q_out + ((long)m * nq + head) * d
-                     : (slot >= 0 ? a.kc + (((long)(slot >> 4) * nkv + head) * 16 + (slot & 15)) * d : nullptr);
-      if (dst) {
-        st16(dst + d1, pack8(r1));
-        st16(dst + hd + d1, pack8(r2));
-      }
-    }
-    if (n0 + BN <= vcol0) return;      // (block-uniform)
-    const int v0 = max(0, vcol0 - n0), nv = min(BN, N - n0) - v0;      // this tile's V columns
-    if (a.v_rows != nullptr) {
-      for (int e = threadIdx.x; e < BM * (nv / 8); e += NT) {
-        const int rl = e / (nv / 8), c = v0 + (e % (nv / 8)) * 8;
-        if (m0 + rl < M) st16(a.v_rows + (long)(m0 + rl) * a.v_ld + (n0 + c - vcol0), *reinterpret_cast<const uint4*>(so + rl * OLD + c));
-      }
-      return;
-    }
-    // V^T cache [block][head][dim][16]: eight rows in eight consecutive slots of half a block (a prompt's) are one 16-byte store per
-    // dim, written by the first of them; rows outside such a run store their two bytes.  Rows and columns by the tile's constants: divisions
-    // by the tile's number of V columns and by d made a decode step's tiles slower than stores from registers (96 rows, 6144 columns
-    // of 128: 25.5 from registers, 27.9, here 25.7 us)
-    int* s_run = reinterpret_cast<int*>(s_rsp);      // [BM] 0 alone, 1 in a run, 2 a run's first (the row scales are in registers)
-    for (int r = threadIdx.x; r < BM; r += NT) {
-      const int sl = s_slot[r], st = r - (sl & 7);
-      bool run = sl >= 0 && st >= 0 && st + 7 < BM && m0 + st + 7 < M;
-      if (run)
-        for (int j = 0; j < 8; ++j) run = run && s_slot[st + j] == (sl & ~7) + j;
-      s_run[r] = run ? 1 + (st == r) : 0;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < BM * BN; e += NT) {
-      const int rl = e / BN, c = e % BN;
-      if (c < v0 || c >= v0 + nv || m0 + rl >= M) continue;
-      const int run = s_run[rl], slot = s_slot[rl];
-      if (slot < 0 || run == 1) continue;
-      u16* vo = a.vc + ((long)(slot >> 4) * nkv * d + (n0 + c - vcol0)) * 16 + (slot & 15);      // (head, dim: the column itself)
-      if (run == 2) {
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          w[j] = (uint32_t)so[(rl + 2 * j) * OLD + c] | ((uint32_t)so[(rl + 2 * j + 1) * OLD + c] << 16);
-        st16(vo, make_uint4(w[0], w[1], w[2], w[3]));
-      } else *vo = so[rl * OLD + c];
-    }
+    // (the runs lie over the row scales, which are in registers)
+    qkv_copy_out<BM, BN, OLD, NT>(a, so, s_slot, s_pos, reinterpret_cast<int*>(s_rsp), M, m0, n0);
     return;
   } else {
     // bias (encoder layers): one value per lane column, hoisted out of the row loop
@@ -1052,6 +988,7 @@ int by_tile(int bm, int bn, int stages, int ks, int nw, int wk, const GemmArgs& 
     if (bm == 64 && bn == 128) return by_pipe_deep<64, 128, EPI, 4>(stages, ks, a, st);
     if (bm == 128 && bn == 64) return by_pipe_deep<128, 64, EPI, 4>(stages, ks, a, st);
     if (bm == 128 && bn == 128) return by_pipe_deep<128, 128, EPI, 4>(stages, ks, a, st);
+    if (bm == 256 && bn == 256 && stages == 2 && ks == 1) return dllm::wide_gemm(a, EPI, st);
   } else if (nw == 8) {
     if (bm == 64 && bn == 128) return by_pipe_deep<64, 128, EPI, 8>(stages, ks, a, st);
     if (bm == 128 && bn == 128) return by_pipe_deep<128, 128, EPI, 8>(stages, ks, a, st);
@@ -1069,6 +1006,7 @@ int by_tile_grouped(int bm, int bn, int stages, int ks, int nw, const GemmArgs& 
   if (bm == 64 && bn == 128 && stages == 3 && nw == 4) return launch_fit<64, 128, EPI, 3, 1, 4>(a, st);
   if (bm == 64 && bn == 64 && stages == 6 && nw == 4) return launch_fit<64, 64, EPI, 6, 1, 4>(a, st);
   if (bm == 128 && bn == 128 && stages == 4 && nw == 8) return launch_fit<128, 128, EPI, 4, 1, 8>(a, st);
+  if (bm == 256 && bn == 256 && stages == 2 && nw == 4) return dllm::wide_gemm(a, EPI, st);
   if (bm == 256 && bn == 128 && stages == 3 && nw == 8) return launch_fit<256, 128, EPI, 3, 1, 8>(a, st);
   if (bm == 256 && bn == 256 && stages == 2 && nw == 8) return launch_fit<256, 256, EPI, 2, 1, 8>(a, st);
   return -20;

@@ -458,7 +458,7 @@ def moe_ffn_tg_resadd(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13
         from . import gemm
         return gemm.res_add_ssq(moe_ffn_tg(x, ids, wts, w13i, w2, frag=frag), r, ssq)
     return int(ext.moe_ffn_tg(x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, None,
-                              list(moe_plan(x.shape[0] * ids.shape[1])), 0, res=r, ssq=ssq, **moe_few(x, ids, frag)))
+                              list(moe_plan(x.shape[0] * ids.shape[1], w13i, w2)), 0, res=r, ssq=ssq, **moe_few(x, ids, frag)))
 
 
 def moe_ffn(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13: torch.Tensor,
@@ -479,8 +479,13 @@ MOE_PLANS = {  # (bm, bn13, stages13, ks13, nw13, bn2, stages2, ks2, nw2) by rou
     "decode": (64, 128, 3, 1, 4, 64, 6, 1, 4),        # P <= 128: weight streaming, 64-row tiles, 6-deep ring for
                                                       # the long-K down projection
     "mid": (128, 128, 4, 1, 8, 128, 4, 1, 8),         # P <= 1024
-    "prefill": (256, 256, 2, 1, 8, 128, 3, 1, 8),     # large P: 256x256 tiles (weight reuse)
+    "prefill": (256, 256, 2, 1, 4, 128, 3, 1, 8),     # large P: 256x256 tiles (weight reuse)
+    "wide": (256, 256, 2, 1, 4, 256, 2, 1, 4),        # ... of both products, where the second's fill half the CUs
 }
+# Row tiles of 256 where an expert has half of one and they fill more than half the CUs.  Layer of experts, us 128-row tiles / "prefill" / "wide":
+# 8 of 1024 x 1024 1200 tokens 52 / 63 / 68, 2100 79 / 73 / 72, 2800 85 / 74 / 77, 4001 124 / 120 / 106, 8048 207 / 187 / 173; 64 of
+# 1024 x 512 4001 (125 pairs an expert) 94 / 109 / 111, 8048 154 / 146 / 140; 8 of 4096 x 3584 600 265 / 228 / 229, 2800 729 / 548 / 491.
+MOE_WIDE_ROWS, MOE_WIDE_FIRST, MOE_WIDE_SECOND = 128, 0.55, 0.5
 
 
 # tokens and routed pairs up to which the experts run on their fragment-major copies (csrc/kernels/moe_decode.hip, whose pair list ends
@@ -515,8 +520,17 @@ def moe_few(x: torch.Tensor, ids: torch.Tensor, frag) -> dict:
     return dict(w13f=frag[0], w2f=frag[1], few_ks=1 if in_order else 4)
 
 
-def moe_plan(pairs: int) -> Tuple[int, ...]:
-    return MOE_PLANS["decode" if pairs <= 128 else "mid" if pairs <= 1024 else "prefill"]
+def moe_plan(pairs: int, w1: Optional[torch.Tensor] = None, w2: Optional[torch.Tensor] = None) -> Tuple[int, ...]:
+    """``w1`` [E, N1, K1], ``w2`` [E, N2, K2]: the experts' weights, for the tiles of prompt steps."""
+    if pairs <= 1024 or w1 is None:
+        return MOE_PLANS["decode" if pairs <= 128 else "mid" if pairs <= 1024 else "prefill"]
+    from .gemm import _P
+    E = w1.shape[0]
+    rows = max(E, pairs / 256 + E / 2)      # row tiles; an expert's last one is half full on average
+    fill = lambda w: rows * -(-w.shape[1] // 256) / _P.cus  # noqa: E731
+    if pairs < MOE_WIDE_ROWS * E or fill(w1) < MOE_WIDE_FIRST:
+        return MOE_PLANS["mid"]
+    return MOE_PLANS["wide" if fill(w2) >= MOE_WIDE_SECOND else "prefill"]
 
 
 def moe_ffn_tg(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torch.Tensor, w2: torch.Tensor,
@@ -536,7 +550,7 @@ def moe_ffn_tg(x: torch.Tensor, ids: torch.Tensor, wts: torch.Tensor, w13i: torc
         out = ref.moe_ffn(x, ids, wts, w13, w2)
         return out if tail is None else moe_tail(out, tail)
     if plan is None:
-        plan = moe_plan(x.shape[0] * ids.shape[1])
+        plan = moe_plan(x.shape[0] * ids.shape[1], w13i, w2)
     return moe_run_tg(ext, x, ids.to(torch.int32).contiguous(), wts.float().contiguous(), w13i, w2, plan, 0, tail, frag)
 
 

@@ -299,7 +299,7 @@ def _splits_together(M: int, N: int, K: int, plan: Tuple) -> int:
 # a prefill chunk uses the plan of the smallest bucket that holds it.  Rounds 4-5 measured it
 # slower or neutral end to end (profiles/r4_prefill_gemm.md); with the grouped tile raster and the
 # 8-loader 256 x 128 plans among the candidates (round 6) tgemm takes 8 of TinyLlama's 12 (bucket,
-# shape) pairs (gate|up at 8K rows: 368 vs 448 us).  End to end it is within noise (+0.3 % over 7
+# shape) pairs (gate|up at 8K rows: 368 vs 448 us; 309 on four waves, csrc/kernels/wide_gemm.hip).  End to end it is within noise (+0.3 % over 7
 # same-box arms of the driver command, prefill step time lower in 2 of 3; profiles/r6_prefill_core.md),
 # and it is the default: the fused-epilogue kernel runs where it measured faster, hipBLASLt elsewhere.
 PREFILL_MS = (2048, 4096, 8192)
@@ -313,12 +313,13 @@ SPLIT_MARGIN = 1.03
 # decode (v_new given): the standalone QKV epilogue hands V over row-major too, as the one-launch
 # tgemm does, and the attention kernel writes the newest V^T (no 2-byte stores 32 B apart)
 QKV_POST_VROWS = True
-_PF_PLANS = ((256, 256, 2, 1, 1, 8), (256, 128, 3, 1, 1, 8), (192, 128, 3, 1, 1, 8), (128, 128, 3, 1, 1, 8),
+_PF_PLANS = ((256, 256, 2, 1, 1, 4), (256, 256, 2, 1, 1, 4, 1, 0, 0, 64, 16, 8),      # csrc/kernels/wide_gemm.hip
+             (256, 128, 3, 1, 1, 8), (192, 128, 3, 1, 1, 8), (128, 128, 3, 1, 1, 8),
              # 32-deep k-steps: 5-13 % ahead of the 64-deep tiles at 2-4K rows (profiles/r5_decode_gemm_lab.md)
              (256, 256, 4, 1, 1, 8, 1, 0, 0, 32),
              # grouped tile raster (plan element 12: m-tiles per group), the 8-loader 256 x 128 tile: the
              # fastest tgemm forms at 2-8K rows in scripts/exp/raster_probe.py (profiles/r6_gemm_fill_path.md)
-             (256, 256, 2, 1, 1, 8, 1, 0, 0, 64, 16, 8), (256, 256, 4, 1, 1, 8, 1, 0, 0, 32, 16, 8),
+             (256, 256, 4, 1, 1, 8, 1, 0, 0, 32, 16, 8),
              (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 0), (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 2),
              (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 8))
 

@@ -291,7 +291,7 @@ def moe_ffn_relu2(x, ids, wts, w1, w2, tail: Optional[tuple] = None, frag=None) 
         return out if tail is None else moe_tail(out, tail)
     ids, wts = ids.to(torch.int32).contiguous(), wts.float().contiguous()
     if moe_ffn_relu2_tg_ok(x, w1):
-        return moe_run_tg(ext, x, ids, wts, w1, w2, moe_plan(x.shape[0] * ids.shape[1]), 1, tail, frag)
+        return moe_run_tg(ext, x, ids, wts, w1, w2, moe_plan(x.shape[0] * ids.shape[1], w1, w2), 1, tail, frag)
     out = torch.empty((x.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
     ext.moe_ffn(x, ids, wts, w1, w2, out, 1)
     return out if tail is None else moe_tail(out, tail)
