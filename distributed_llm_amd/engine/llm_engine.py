@@ -1184,7 +1184,9 @@ class LLMEngine:
         h[o[6] + rows] = lens
         self._sync_bt(non_blocking=self._in_join_burst)
         h[o[7]] = self._split_len(int(lens.sum()))
-        if self.fused_sampler:
+        if self.fused_sampler and self._feeding:       # nothing is sampled; the step's seed is drawn all the same
+            self._next_seed()
+        elif self.fused_sampler:
             self._fill_sampler(h, hf, self._so, self.buckets[-1], running, bs)
         nu = len(self._bt_upd) // 2
         h[o[8]] = nu
@@ -1826,8 +1828,11 @@ class LLMEngine:
                 if s is not None:
                     self._release(s)
             return torch.empty((0, self.cfg.vocab))
+        decode, table = True, (self._bt_dirty, self._bt_rows)
+        opened: List[int] = []
         for key, toks, _ in entries:
             toks = [int(t) for t in toks]
+            decode = decode and len(toks) == 1 and key in self._streams and self._streams[key].num_computed > 0
             if not toks:
                 raise ValueError("an entry needs at least one token")
             s = self._streams.get(key)
@@ -1855,20 +1860,25 @@ class LLMEngine:
                         nblk = (len(s.prompt) + BS - 1) // BS
                         self.bt_host[s.row, nblk - 1] = slot // BS
                         self._bt_hw = max(self._bt_hw, nblk)
-                        self._bt_dirty = True      # the next decode step copies the table (_sync_bt)
+                        self._bt_dirty = True      # the step copies the table (_sync_bt)
                         self._mark_bt_row(s.row)
+                        opened += (s.row * self.max_blocks + nblk - 1, slot // BS)
             seqs.append(s)
         n_want = sum(len(w) for _, _, w in entries)
-        decode = all(len(t) == 1 and s.num_computed > 0 for s, (_, t, _) in zip(seqs, entries))
+        if decode and not table[0]:
+            # blocks opened by single tokens travel with the step's inputs (its scatter applies them, as in generation): the table's
+            # copy of a few columns waits for the device, 40-48 us of a step
+            self._bt_dirty, self._bt_rows = table
+            self._bt_upd.extend(opened)
         if decode:
             if self.d_logits is None:
                 self.d_logits = torch.zeros((self.buckets[-1], self.cfg.vocab), dtype=torch.float32, device=self.device)
             B = len(seqs)
             lens = np.fromiter((s.length for s in seqs), dtype=np.int64, count=B)
             last = np.fromiter((s.prompt[-1] for s in seqs), dtype=np.int64, count=B)
-            bs = self._prep_decode(seqs, lens, last, 0)
             self._feeding = True
             try:
+                bs = self._prep_decode(seqs, lens, last, 0)
                 if self.use_graphs:
                     self._replay(bs, 0)
                 else:
@@ -1877,6 +1887,7 @@ class LLMEngine:
                 self._feeding = False
             self.steps["decode"] += 1
             self.steps["decode_tokens"] += B
+            self._fed(seqs)             # (the step runs meanwhile)
             rows = [i for i, (_, _, w) in enumerate(entries) for _ in w]
             # the step must finish before the next one restages its pinned inputs (generation reads
             # the step's tokens back at this point)
@@ -1904,15 +1915,18 @@ class LLMEngine:
                 out = torch.empty((0, self.cfg.vocab))
                 if self.on_gpu:
                     torch.cuda.current_stream(self.device).synchronize()
-        for s in seqs:
-            s.num_computed = s.length
-            self.bm.commit(s.id, s.length)
+            self._fed(seqs)
         for key in end:
             s = self._streams.pop(key, None)
             if s is not None:
                 self._release(s)
         assert out.shape[0] == n_want
         return out
+
+    def _fed(self, seqs: List[_Seq]) -> None:
+        for s in seqs:
+            s.num_computed = s.length
+            self.bm.commit(s.id, s.length)
 
     # ------------------------------------------------------------------ outputs
     def _finalize_text(self, s: _Seq) -> str:
