@@ -209,10 +209,10 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       mloc = lane_max(mloc, 32);
       const float m_new = fmaxf(m_run, mloc);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = exp2f(m_run - m_safe);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);
       float lsum = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) { p[j] = exp2f(p[j] - m_safe); lsum += p[j]; }
+      for (int j = 0; j < 8; ++j) { p[j] = __builtin_amdgcn_exp2f(p[j] - m_safe); lsum += p[j]; }
       lsum = lane_add(lsum, 16);
       lsum = lane_add(lsum, 32);
       l_run = l_run * alpha + lsum;
@@ -282,7 +282,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
     if (wave < WAVES) {
       const float mo = s_m[wave][rl], lo = s_l[wave][rl];
       const float mn = fmaxf(m_run, mo), ms = (mn == -INFINITY) ? 0.f : mn;
-      const float fa = exp2f(m_run - ms), fb = exp2f(mo - ms);
+      const float fa = __builtin_amdgcn_exp2f(m_run - ms), fb = __builtin_amdgcn_exp2f(mo - ms);
       l_run = l_run * fa + lo * fb;
       m_run = mn;
 #pragma unroll
@@ -312,7 +312,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       float L = 0.f, O = 0.f;
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) {
-        const float f = exp2f(s_m[w][row] - Ms);
+        const float f = __builtin_amdgcn_exp2f(s_m[w][row] - Ms);
         L += s_l[w][row] * f;
         O += s_o[w][row][col] * f;
       }
@@ -337,7 +337,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
     float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const float f = exp2f(s_m[w][row] - Ms);
+      const float f = __builtin_amdgcn_exp2f(s_m[w][row] - Ms);
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] += s_o[w][row][col + j] * f;
     }
@@ -354,7 +354,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       const float Ms = (M == -INFINITY) ? 0.f : M;
       float L = 0.f;
 #pragma unroll
-      for (int w = 0; w < WAVES; ++w) L += s_l[w][row] * exp2f(s_m[w][row] - Ms);
+      for (int w = 0; w < WAVES; ++w) L += s_l[w][row] * __builtin_amdgcn_exp2f(s_m[w][row] - Ms);
       ml[2 * h] = M;
       ml[2 * h + 1] = L;
     }
@@ -387,7 +387,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, s_pm[sp * 16 + row]);
       const float Ms = (M == -INFINITY) ? 0.f : M;
       float L = 0.f;
-      for (int sp = 0; sp < nsplit; ++sp) L += s_pl[sp * 16 + row] * exp2f(s_pm[sp * 16 + row] - Ms);
+      for (int sp = 0; sp < nsplit; ++sp) L += s_pl[sp * 16 + row] * __builtin_amdgcn_exp2f(s_pm[sp * 16 + row] - Ms);
       s_m[0][row] = Ms;
       s_l[0][row] = L;
     }
@@ -404,7 +404,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
 #pragma unroll
       for (int sp = 0; sp < COMBINE_MAXS; ++sp) {
         if (sp < nsplit) {
-          const float f = exp2f(s_pm[sp * 16 + row] - s_m[0][row]);
+          const float f = __builtin_amdgcn_exp2f(s_pm[sp * 16 + row] - s_m[0][row]);
           o[0] += q[sp].x * f; o[1] += q[sp].y * f; o[2] += q[sp].z * f; o[3] += q[sp].w * f;
         }
       }
@@ -427,7 +427,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
     for (int sp = 0; sp < nsplit; ++sp) {
       const float4 q = ld_wt16(rml, (unsigned)((tbase + sp * 16 + (row & ~1)) * 2 * 4));
       const float m = (row & 1) ? q.z : q.x, l = (row & 1) ? q.w : q.y;
-      L += l * exp2f(m - Ms);
+      L += l * __builtin_amdgcn_exp2f(m - Ms);
     }
     s_m[0][row] = Ms;
     s_l[0][row] = L;
@@ -440,7 +440,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
     float o[4] = {0.f, 0.f, 0.f, 0.f};
     for (int sp = 0; sp < nsplit; ++sp) {
       const float4 mq = ld_wt16(rml, (unsigned)((tbase + sp * 16 + (row & ~1)) * 2 * 4));
-      const float f = exp2f(((row & 1) ? mq.z : mq.x) - s_m[0][row]);
+      const float f = __builtin_amdgcn_exp2f(((row & 1) ? mq.z : mq.x) - s_m[0][row]);
       const float4 q = ld_wt16(ro, (unsigned)(((tbase + sp * 16 + row) * D + col) * 4));
       o[0] += q.x * f; o[1] += q.y * f; o[2] += q.z * f; o[3] += q.w * f;
     }

@@ -389,11 +389,19 @@ class LLMEngine:
     # MI355X, TinyLlama) it cut B=1 from 1.14 to 0.89 ms and B=16 from 1.51 to 1.29 ms vs the
     # static split grid (a kernel-only sweep had B=16-64 about even)
     ATTN_WL_MIN_BS = 1
-    # shortest key range of one work-list unit (split-K granularity)
-    # (256: with the parallel split combine, batch 1-8 steps at 2k context are 2-3 % faster than at
-    # 512 and equal at 8k, microbench decode sweep; it only matters while batch x context < 64k
-    # tokens, above that the target unit count sets the chunk)
+    # shortest key range of one work-list unit (split-K granularity).  It only matters while batch x context < 64k tokens, above
+    # that the target unit count sets the chunk.  A unit's eight waves take 256 keys a trip, 1.2 us; parts that meet cost 2 to 3 us (slabs past
+    # L2, a ticket, the last one's sum).  us of a launch, TinyLlama's heads, chunk of 128 / 256 / whole: 24 requests of 20-300
+    # keys 8.2 / 8.5 / 6.2, 48 of 40-424 10.1 / 10.0 / 8.1, 64 of 300-900 18.7 / 18.8 / 12.5, 2 of 500-1000 8.0 / 8.8 / 10.0, 8 of
+    # 2000-5000 14.4 / 13.9 / 19.6.
     ATTN_MIN_CHUNK = 256
+
+    def _min_chunk(self, lens: np.ndarray) -> int:
+        longest, heads = int(lens.max()), len(lens) * self._nkv
+        if longest <= 512 or (longest <= 1024 and heads >= 128):      # two trips, or four that fill half the CUs: whole
+            return 1024
+        return 128 if int((-(-lens // 128)).sum()) * self._nkv <= 128 else self.ATTN_MIN_CHUNK
+
     def _use_worklist(self, bs: int) -> bool:
         return self.attn_worklist and bs >= self.ATTN_WL_MIN_BS
 
@@ -1176,7 +1184,7 @@ class LLMEngine:
             target = self.ATTN_ITEMS_PER_WG * grid
             items_t, items = self._items_bufs[p]
             ops.decode_work_items(lens[order], self._nkv, self.max_splits, target,
-                                  min_chunk=self.ATTN_MIN_CHUNK, out=items, seq=rows[order], qstart=order)
+                                  min_chunk=self._min_chunk(lens), out=items, seq=rows[order], qstart=order)
             n_items = ops.work_items_len(items)
         h[o[4]:o[6] + R + 1] = 0
         h[o[4] + rows] = np.arange(B)

@@ -53,3 +53,16 @@ def test_work_items_extended_form():
     tile = u[:, 0] & 0xFFFF
     assert (u[:, 2] & 0xFFFF == seq[tile]).all() and (u[:, 2] >> 16 == qstart[tile]).all()
     assert (u[:, 3] == ctx[tile]).all()
+
+
+@pytest.mark.parametrize("lens,nkv,want", [([512], 4, 1024), ([513], 4, 128), ([4000], 4, 128), ([300] * 48, 4, 1024), ([513] + [40] * 30, 4, 256),
+                                           ([1024] * 32, 4, 1024), ([1024] * 31, 4, 256), ([1025] * 32, 4, 256)])
+def test_chunk_of_a_batch(lens, nkv, want):
+    """Whole up to two trips of 256 keys, or four where the heads fill half the CUs; short parts where there are few."""
+    from distributed_llm_amd.engine.llm_engine import LLMEngine
+    eng = LLMEngine.__new__(LLMEngine)
+    eng._nkv = nkv
+    got = eng._min_chunk(np.array(lens))
+    assert got == want
+    if want == 1024:
+        assert ops.decode_work_items(np.array(lens), nkv, 16, 512, min_chunk=got)[0] == len(lens) * nkv
