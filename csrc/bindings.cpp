@@ -26,18 +26,18 @@ int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, const int*
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
 int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, const void*, float, void*, hipStream_t);
 int dllm_scatter_pairs(int*, const int*, int, hipStream_t);
-int dllm_step_fetch(const int*, int*, int, int, int, int, const int*, const int*, int*, int, hipStream_t);
+int dllm_step_fetch(const int*, int*, int, int, int, int, const int*, const int*, int*, int, int*, int, int, hipStream_t);
 int dllm_step_store(const int*, int*, int, hipStream_t);
 int dllm_argmax(const void*, long, int, int, int, int*, hipStream_t);
 int dllm_sample_topp(const float*, const long*, int, int, const float*, const float*, const float*, int*, hipStream_t);
 int dllm_cosine_scores(const float*, const float*, float*, int, int, int, hipStream_t);
 int dllm_sample_rows(const void*, long, int, int, const float*, const float*, const int*, const unsigned*, int*,
-                     hipStream_t);
+                     int*, hipStream_t);
 int dllm_tp_cands_k();
 int dllm_tp_cands(const void*, long, int, int, int, void*, hipStream_t);
 int dllm_tp_sample(const void*, int, int, const float*, const float*, const int*, const unsigned*, int*, hipStream_t);
 int dllm_sample_split(const void*, long, int, int, int, const float*, const float*, const int*, const unsigned*, void*,
-                      long, int*, int*, hipStream_t);
+                      long, int*, int*, int*, hipStream_t);
 int dllm_sample_split_maxp();
 int dllm_sample_split_kmax();
 int dllm_skinny_epi(const void*, long, const void*, int, void*, long, int, int, int, int, int, int, float*, int*, void*,
@@ -123,6 +123,7 @@ int dllm_latent_expand_ok(int, int, int, int);
 int dllm_latent_expand(const void*, const int*, int, int, int, int, const int*, int, int, int, int, const void*, const void*, void*,
                        void*, int, hipStream_t);
 int dllm_gate_heads(const void*, int, const void*, long, void*, long, int, int, long, int, hipStream_t);
+int dllm_embed_rows(const int*, const void*, int, long, float, float*, float*, void*, const float*, float, void*, long, int, hipStream_t);
 int dllm_scaled_resadd_rms(const void*, long, int, float, int, const float*, float*, const float*, void*, long, long, int, float,
                            hipStream_t);
 int dllm_relu2_scale(const void*, int, const float*, int, int, void*, long, int, hipStream_t);
@@ -505,10 +506,15 @@ static void* mapped_ptr(const torch::Tensor& t, const char* what) {
 // Decode-step inputs from the pinned staging buffer (device-mapped) into dec_dev, with the
 // pipelined id gather (ids[i] = d_out[src[i]] where src[i] >= 0) and the attention work list.
 void step_fetch(torch::Tensor dec_host, torch::Tensor dec_dev, int64_t ids_off, int64_t src_off, int64_t n_ids,
-                torch::Tensor d_out, c10::optional<torch::Tensor> items_host, c10::optional<torch::Tensor> items_dev) {
+                torch::Tensor d_out, c10::optional<torch::Tensor> items_host, c10::optional<torch::Tensor> items_dev,
+                c10::optional<torch::Tensor> sc_dst, int64_t sc_off, int64_t sc_cap) {
   TORCH_CHECK(dec_dev.is_cuda() && dec_dev.scalar_type() == torch::kInt && dec_dev.is_contiguous() &&
                   dec_dev.numel() == dec_host.numel(), "step_fetch: dec_dev int32 like dec_host");
   TORCH_CHECK(d_out.is_cuda() && d_out.scalar_type() == torch::kInt && d_out.numel() > n_ids, "step_fetch: d_out");
+  if (sc_dst) {
+    check_i32(*sc_dst, "sc_dst");
+    TORCH_CHECK(sc_dst->is_contiguous() && sc_off >= 0 && sc_cap >= 0 && sc_off + 1 + 2 * sc_cap <= dec_host.numel(), "step_fetch: updates");
+  }
   const int* ih = nullptr;
   int* idv = nullptr;
   int cap = 0;
@@ -521,7 +527,7 @@ void step_fetch(torch::Tensor dec_host, torch::Tensor dec_dev, int64_t ids_off, 
   }
   ok(dllm_step_fetch((const int*)mapped_ptr(dec_host, "step_fetch dec_host"), dec_dev.data_ptr<int>(),
                      (int)dec_host.numel(), (int)ids_off, (int)src_off, (int)n_ids, d_out.data_ptr<int>(), ih, idv, cap,
-                     stream()),
+                     sc_dst ? sc_dst->data_ptr<int>() : nullptr, (int)sc_off, (int)sc_cap, stream()),
      "step_fetch");
 }
 
@@ -572,10 +578,17 @@ void sample_topp(torch::Tensor vals, torch::Tensor idx, torch::Tensor temp, torc
      "sample_topp");
 }
 
+// Where a sampler writes its tokens a second time: mapped host memory (none: nullptr)
+static int* tokens_host(const c10::optional<torch::Tensor>& t, int B) {
+  if (!t) return nullptr;
+  TORCH_CHECK(t->numel() >= B, "out_host: a token a row");
+  return (int*)mapped_ptr(*t, "out_host");
+}
+
 // Fused per-row sampler: temp <= 0 -> arg-max; else exact top-k (k <= 256; 0 -> 256), temperature,
 // top-p and an inverse-CDF draw with u = hash(seed, row).  seed: int32 device scalar.
 void sample_rows(torch::Tensor logits, torch::Tensor temp, torch::Tensor top_p, torch::Tensor top_k,
-                 torch::Tensor seed, torch::Tensor out) {
+                 torch::Tensor seed, torch::Tensor out, c10::optional<torch::Tensor> out_host) {
   check_bf16(logits, "logits");
   TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1 && logits.stride(0) % 8 == 0,
               "logits [B, V] row-major, 16-B aligned rows");
@@ -590,7 +603,7 @@ void sample_rows(torch::Tensor logits, torch::Tensor temp, torch::Tensor top_p, 
               "per-row parameter lengths");
   ok(dllm_sample_rows(logits.data_ptr(), logits.stride(0), B, logits.size(1), temp.data_ptr<float>(),
                       top_p.data_ptr<float>(), top_k.data_ptr<int>(), (const unsigned*)seed.data_ptr<int>(),
-                      out.data_ptr<int>(), stream()),
+                      out.data_ptr<int>(), tokens_host(out_host, B), stream()),
      "sample_rows");
 }
 
@@ -599,7 +612,8 @@ void sample_rows(torch::Tensor logits, torch::Tensor temp, torch::Tensor top_p, 
 int64_t sample_split_maxp() { return dllm_sample_split_maxp(); }
 int64_t sample_split_kmax() { return dllm_sample_split_kmax(); }
 void sample_split(torch::Tensor logits, torch::Tensor temp, torch::Tensor top_p, torch::Tensor top_k,
-                  torch::Tensor seed, torch::Tensor part, torch::Tensor counters, torch::Tensor out, int64_t P) {
+                  torch::Tensor seed, torch::Tensor part, torch::Tensor counters, torch::Tensor out, int64_t P,
+                  c10::optional<torch::Tensor> out_host) {
   check_bf16(logits, "logits");
   TORCH_CHECK(logits.dim() == 2 && logits.stride(1) == 1 && logits.stride(0) % 8 == 0,
               "logits [B, V] row-major, 16-B aligned rows");
@@ -617,7 +631,8 @@ void sample_split(torch::Tensor logits, torch::Tensor temp, torch::Tensor top_p,
   TORCH_CHECK(P >= 1 && P <= dllm_sample_split_maxp(), "shards P");
   ok(dllm_sample_split(logits.data_ptr(), logits.stride(0), B, logits.size(1), (int)P, temp.data_ptr<float>(),
                        top_p.data_ptr<float>(), top_k.data_ptr<int>(), (const unsigned*)seed.data_ptr<int>(),
-                       part.data_ptr(), (long)part.numel() * 4, counters.data_ptr<int>(), out.data_ptr<int>(), stream()),
+                       part.data_ptr(), (long)part.numel() * 4, counters.data_ptr<int>(), out.data_ptr<int>(), tokens_host(out_host, B),
+                       stream()),
      "sample_split");
 }
 
@@ -2265,6 +2280,34 @@ void scaled_resadd_rms(torch::Tensor x, c10::optional<torch::Tensor> y, double m
      "scaled_resadd_rms");
 }
 
+// Embedding rows to the f32 stream (x, and x2), their rounding (lp) and the first norm of the stream (h), in one launch
+bool embed_rows(torch::Tensor ids, torch::Tensor table, double scale, torch::Tensor x, c10::optional<torch::Tensor> x2,
+                c10::optional<torch::Tensor> lp, c10::optional<torch::Tensor> w, double eps, c10::optional<torch::Tensor> h) {
+  check_i32(ids, "ids");
+  const bool f = act_f32(table, "table");
+  check_f32(x, "x");
+  TORCH_CHECK(table.dim() == 2 && table.is_contiguous() && x.dim() == 2 && x.is_contiguous() && x.size(1) == table.size(1) &&
+                  ids.numel() == x.size(0) && ids.is_contiguous(), "table [V, width], ids [T], x [T, width] f32");
+  TORCH_CHECK(w.has_value() == h.has_value(), "a norm weight and its output");
+  if (x2) {
+    check_f32(*x2, "x2");
+    TORCH_CHECK(x2->is_contiguous() && x2->sizes() == x.sizes(), "x2 like x");
+  }
+  for (auto* t : {&lp, &h})
+    if (*t) TORCH_CHECK((*t)->is_cuda() && (*t)->scalar_type() == table.scalar_type() && (*t)->is_contiguous() && (*t)->sizes() == x.sizes(),
+                        "[T, width] of the table's type");
+  if (w) {
+    check_f32(*w, "norm weight");
+    TORCH_CHECK(w->is_contiguous() && w->numel() == x.size(1), "norm weight [width]");
+  }
+  const int rc = dllm_embed_rows(ids.data_ptr<int>(), table.data_ptr(), f, table.size(0), (float)scale, x.data_ptr<float>(),
+                                 x2 ? x2->data_ptr<float>() : nullptr, lp ? lp->data_ptr() : nullptr, w ? w->data_ptr<float>() : nullptr,
+                                 (float)eps, h ? h->data_ptr() : nullptr, (long)x.size(0), (int)x.size(1), stream());
+  if (rc == -1) return false;      // a width or alignment the launch does not take
+  ok(rc, "embed_rows");
+  return true;
+}
+
 // ---- differential attention, Mamba-2 / mLSTM recurrences, PolyNorm, grouped router (gqa.hip, outer_scan.hip, seqmix.hip)
 void qk_norm_prep(torch::Tensor proj, c10::optional<torch::Tensor> bias, int64_t H, int64_t G, int64_t M, int64_t d, int64_t dv,
                   torch::Tensor qw, torch::Tensor kw, torch::Tensor cos_sin, int64_t rot, double eps, double qscale,
@@ -2867,6 +2910,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("latent_q_prep", &latent_q_prep);
   m.def("gate_heads", &gate_heads);
   m.def("scaled_resadd_rms", &scaled_resadd_rms);
+  m.def("embed_rows", &embed_rows);
   m.def("gqa_tile_tokens",
         [](int64_t H, int64_t G, bool mfma) { return (int64_t)dllm_gqa_tile_tokens((int)H, (int)G, (int)mfma); });
   m.def("gqa_mfma_ok", [](bool f32, int64_t H, int64_t G, int64_t d, int64_t dv, int64_t bs) {
@@ -2929,11 +2973,15 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("eps") = 0.0, py::arg("xn") = py::none());
   m.def("argmax", &argmax);
   m.def("scatter_pairs", &scatter_pairs);
-  m.def("step_fetch", &step_fetch);
+  m.def("step_fetch", &step_fetch, py::arg("dec_host"), py::arg("dec_dev"), py::arg("ids_off"), py::arg("src_off"), py::arg("n_ids"),
+        py::arg("d_out"), py::arg("items_host") = py::none(), py::arg("items_dev") = py::none(), py::arg("sc_dst") = py::none(),
+        py::arg("sc_off") = 0, py::arg("sc_cap") = 0);
   m.def("step_store", &step_store);
   m.def("sample_topp", &sample_topp);
-  m.def("sample_rows", &sample_rows);
-  m.def("sample_split", &sample_split);
+  m.def("sample_rows", &sample_rows, py::arg("logits"), py::arg("temp"), py::arg("top_p"), py::arg("top_k"), py::arg("seed"), py::arg("out"),
+        py::arg("out_host") = py::none());
+  m.def("sample_split", &sample_split, py::arg("logits"), py::arg("temp"), py::arg("top_p"), py::arg("top_k"), py::arg("seed"), py::arg("part"),
+        py::arg("counters"), py::arg("out"), py::arg("P"), py::arg("out_host") = py::none());
   m.def("sample_split_maxp", &sample_split_maxp);
   m.def("sample_split_kmax", &sample_split_kmax);
   m.def("tp_cands_k", &tp_cands_k);

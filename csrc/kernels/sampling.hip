@@ -149,8 +149,6 @@ struct SrShared {
   float w_r[SR_KMAX];           // value by rank
   int i_r[SR_KMAX];             // token id by rank
   unsigned wsum[SR_THREADS / 64];
-  float sv[SR_THREADS / 64];
-  int si[SR_THREADS / 64];
   int s_bin, s_above, s_n, s_nt, s_lo, s_amax;
   float s_m;
 };
@@ -458,49 +456,92 @@ static __device__ __forceinline__ int draw_rank(const SrShared& sh, int kk, floa
   return pick;
 }
 
-__global__ void __launch_bounds__(SR_THREADS) sample_rows_kernel(const u16* __restrict__ logits, long stride, int V,
-                                                                 const float* __restrict__ temp,
-                                                                 const float* __restrict__ top_p,
-                                                                 const int* __restrict__ top_k,
-                                                                 const unsigned* __restrict__ seed,
-                                                                 int* __restrict__ out) {
-  __shared__ SrShared sh;
-  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const u16* l = logits + (long)row * stride;
-  const int nv = V >> 3;
-  const float t = temp[row];
-
-  if (!(t > 0.f)) {  // greedy row: arg-max, ties -> lowest index
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-    for_each_vec<SR_THREADS>(l, nv, tid, [&](const uint4 v, int c) {
-      float f[8];
-      unpack8(v, f);
+// The arg-max of l[0, V) by all NT threads (ties -> lowest index, NaN never chosen, nothing to choose -> 0x7fffffff), in thread 0.
+// Four vectors a thread in flight; a thread's indices ascend, so a vector takes the place of the best one only if its largest is larger,
+// and the entry is looked for once at the end (entry by entry the row's comparisons were a third of the launch).
+struct BestShared { float v[16]; int i[16]; };
+template <int NT>
+static __device__ __forceinline__ int row_argmax(const u16* __restrict__ l, int V, BestShared& sh, float& best) {
+  const int nv = V >> 3, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  float bv = -INFINITY;
+  int bc = -1;
+  uint4 bq = make_uint4(0u, 0u, 0u, 0u);
+  for (int c0 = tid; c0 < nv; c0 += 4 * NT) {
+    uint4 v[4];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) better(bv, bi, f[j], c * 8 + j);
-    });
-    for (int i = (nv << 3) + tid; i < V; i += SR_THREADS) better(bv, bi, bf2f(l[i]), i);
+    for (int u = 0; u < 4; ++u) v[u] = ld16(l + (long)min(c0 + u * NT, nv - 1) * 8);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float f[8];
+      unpack8(v[u], f);
+      const float m = fmaxf(fmaxf(fmaxf(f[0], f[1]), fmaxf(f[2], f[3])), fmaxf(fmaxf(f[4], f[5]), fmaxf(f[6], f[7])));
+      if (c0 + u * NT < nv && (m > bv || (m == bv && bc < 0))) { bv = m; bc = c0 + u * NT; bq = v[u]; }
+    }
+  }
+  int bi = 0x7fffffff;
+  if (bc >= 0) {
+    float f[8];
+    unpack8(bq, f);
+#pragma unroll
+    for (int j = 7; j >= 0; --j) bi = f[j] == bv ? bc * 8 + j : bi;
+  }
+  for (int i = (nv << 3) + tid; i < V; i += NT) better(bv, bi, bf2f(l[i]), i);
+  auto reduce = [&](const int from) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
+      if (o > from) continue;
       const float ov = lane_xor(bv, o);
       const int oi = lane_xor(bi, o);
       better(bv, bi, ov, oi);
     }
-    if (lane == 0) { sh.sv[wid] = bv; sh.si[wid] = bi; }
-    __syncthreads();
+  };
+  reduce(32);
+  if (lane == 0) { sh.v[wid] = bv; sh.i[wid] = bi; }
+  __syncthreads();
+  if (wid == 0) {
+    bv = lane < NT / 64 ? sh.v[lane] : -INFINITY;
+    bi = lane < NT / 64 ? sh.i[lane] : 0x7fffffff;
+    reduce(8);
+  }
+  best = bv;
+  return bi;
+}
+
+// NT 1024 where every row has a CU for itself: a greedy row is read by sixteen waves, any other by the first four.
+// out_host: the tokens once more, in mapped host memory (null: no)
+template <int NT>
+__global__ void __launch_bounds__(NT) sample_rows_kernel(const u16* __restrict__ logits, long stride, int V,
+                                                         const float* __restrict__ temp, const float* __restrict__ top_p,
+                                                         const int* __restrict__ top_k, const unsigned* __restrict__ seed,
+                                                         int* __restrict__ out, int* __restrict__ out_host) {
+  __shared__ SrShared sh;
+  __shared__ BestShared bs;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const u16* l = logits + (long)row * stride;
+  const float t = temp[row];
+
+  if (!(t > 0.f)) {  // greedy row
+    float bv;
+    const int bi = row_argmax<NT>(l, V, bs, bv);
     if (tid == 0) {
-      for (int w = 1; w < SR_THREADS / 64; ++w) better(bv, bi, sh.sv[w], sh.si[w]);
-      out[row] = (bi == 0x7fffffff) ? 0 : bi;
+      const int id = bi == 0x7fffffff ? 0 : bi;
+      out[row] = id;
+      if (out_host) out_host[row] = id;
     }
     return;
   }
+  if (tid >= SR_THREADS) return;      // (whole waves, ahead of every barrier)
   int k = top_k[row];
   if (k <= 0 || k > SR_KMAX) k = SR_KMAX;
   if (k > V) k = V;
   const int n = row_topk(l, V, k, sh);
   if (wid == 0) {
     const int pick = draw_rank(sh, min(k, n), t, top_p[row], *seed, (unsigned)row);
-    if (lane == 0) out[row] = pick >= 0 ? sh.i_r[pick] : 0;   // an all-NaN row yields token 0
+    if (lane == 0) {
+      const int id = pick >= 0 ? sh.i_r[pick] : 0;   // an all-NaN row yields token 0
+      out[row] = id;
+      if (out_host) out_host[row] = id;
+    }
   }
 }
 
@@ -598,10 +639,11 @@ __global__ void __launch_bounds__(SR_THREADS) sample_split_kernel(const u16* __r
                                                                   const int* __restrict__ top_k,
                                                                   const unsigned* __restrict__ seed, void* part,
                                                                   unsigned part_bytes, int* __restrict__ counters,
-                                                                  int* __restrict__ out) {
+                                                                  int* __restrict__ out, int* __restrict__ out_host) {
   __shared__ SrShared sh;
   __shared__ int2 lists[SS_MAXP * SR_KMAX];
   __shared__ int s_last;
+  __shared__ BestShared bs;
   const int p = blockIdx.x, row = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int start = p * vs, len = min(vs, V - start);
   const u16* l = logits + (long)row * stride + start;
@@ -614,28 +656,10 @@ __global__ void __launch_bounds__(SR_THREADS) sample_split_kernel(const u16* __r
   const __amdgpu_buffer_rsrc_t rs = make_rsrc(part, part_bytes);
   const unsigned base = (unsigned)(((long)row * P + p) * SR_KMAX * 8);
   if (greedy) {                                   // shard arg-max, ties -> lowest index
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-    const int nv = len >> 3;
-    for_each_vec<SR_THREADS>(l, nv, tid, [&](const uint4 v, int c) {
-      float f[8];
-      unpack8(v, f);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) better(bv, bi, f[j], start + c * 8 + j);
-    });
-    for (int i = (nv << 3) + tid; i < len; i += SR_THREADS) better(bv, bi, bf2f(l[i]), start + i);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = lane_xor(bv, o);
-      const int oi = lane_xor(bi, o);
-      better(bv, bi, ov, oi);
-    }
-    if (lane == 0) { sh.sv[wid] = bv; sh.si[wid] = bi; }
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < SR_THREADS / 64; ++w) better(bv, bi, sh.sv[w], sh.si[w]);
-      st_wt16(rs, base, make_float4(bv, __int_as_float(bi), -INFINITY, __int_as_float(0x7fffffff)));
-    }
+    float bv;
+    const int bi = row_argmax<SR_THREADS>(l, len, bs, bv);
+    if (tid == 0)
+      st_wt16(rs, base, make_float4(bv, __int_as_float(bi == 0x7fffffff ? bi : start + bi), -INFINITY, __int_as_float(0x7fffffff)));
   } else {
     const int n = min(row_topk(l, len, min(k, len), sh), k);
     for (int r2 = tid; 2 * r2 < kp; r2 += SR_THREADS) {
@@ -662,7 +686,9 @@ __global__ void __launch_bounds__(SR_THREADS) sample_split_kernel(const u16* __r
       float bv = -INFINITY;
       int bi = 0x7fffffff;
       for (int q = 0; q < P; ++q) better(bv, bi, __int_as_float(lists[q * kp].x), lists[q * kp].y);
-      out[row] = (bi == 0x7fffffff) ? 0 : bi;
+      const int id = bi == 0x7fffffff ? 0 : bi;
+      out[row] = id;
+      if (out_host) out_host[row] = id;
     }
     return;
   }
@@ -690,7 +716,11 @@ __global__ void __launch_bounds__(SR_THREADS) sample_split_kernel(const u16* __r
   const int kk = min(k, sh.s_n);
   if (wid == 0) {
     const int pick = draw_rank(sh, kk, t, top_p[row], *seed, (unsigned)row);
-    if (lane == 0) out[row] = pick >= 0 ? sh.i_r[pick] : 0;
+    if (lane == 0) {
+      const int id = pick >= 0 ? sh.i_r[pick] : 0;
+      out[row] = id;
+      if (out_host) out_host[row] = id;
+    }
   }
 }
 }  // namespace
@@ -702,7 +732,7 @@ extern "C" int dllm_sample_split_kmax() { return SR_KMAX; }
 // part >= B * P * SR_KMAX int2, counters >= B ints, zero.  Same tokens as dllm_sample_rows.
 extern "C" int dllm_sample_split(const void* logits, long stride, int B, int V, int P, const float* temp,
                                  const float* top_p, const int* top_k, const unsigned* seed, void* part,
-                                 long part_bytes, int* counters, int* out, hipStream_t stream) {
+                                 long part_bytes, int* counters, int* out, int* out_host, hipStream_t stream) {
   if (B <= 0) return 0;
   if (V <= 0 || stride % 8 != 0 || P < 1 || P > SS_MAXP) return -1;
   const int vs = ((V + P - 1) / P + 7) / 8 * 8;
@@ -710,16 +740,21 @@ extern "C" int dllm_sample_split(const void* logits, long stride, int B, int V, 
   const long need = (long)B * P * SR_KMAX * 8;
   if (part_bytes < need || need > 0x7fffffffL) return -3;
   hipLaunchKernelGGL(sample_split_kernel, dim3(P, B), dim3(SR_THREADS), 0, stream, (const u16*)logits, stride, V, P,
-                     vs, temp, top_p, top_k, seed, part, (unsigned)need, counters, out);
+                     vs, temp, top_p, top_k, seed, part, (unsigned)need, counters, out, out_host);
   return (int)hipGetLastError();
 }
 
 extern "C" int dllm_sample_rows(const void* logits, long stride, int B, int V, const float* temp, const float* top_p,
-                                const int* top_k, const unsigned* seed, int* out, hipStream_t stream) {
+                                const int* top_k, const unsigned* seed, int* out, int* out_host, hipStream_t stream) {
   if (B <= 0) return 0;
   if (V <= 0 || stride % 8 != 0) return -1;
-  hipLaunchKernelGGL(sample_rows_kernel, dim3(B), dim3(SR_THREADS), 0, stream, (const u16*)logits, stride, V, temp,
-                     top_p, top_k, seed, out);
+  // (sixteen waves of the sampled path's registers are a CU; past one row a CU they would take turns)
+  if (B <= 256)
+    hipLaunchKernelGGL((sample_rows_kernel<1024>), dim3(B), dim3(1024), 0, stream, (const u16*)logits, stride, V, temp, top_p, top_k,
+                       seed, out, out_host);
+  else
+    hipLaunchKernelGGL((sample_rows_kernel<SR_THREADS>), dim3(B), dim3(SR_THREADS), 0, stream, (const u16*)logits, stride, V, temp,
+                       top_p, top_k, seed, out, out_host);
   return (int)hipGetLastError();
 }
 

@@ -1716,16 +1716,19 @@ class LLMEngine:
         if self._gio:
             o, mb = self._off, self.buckets[-1]
             items = (self._items_bufs[p][0], self.items_dev) if self.attn_worklist else (None, None)
-            ops.step_fetch(self._dec_bufs[p][0], self.dec_dev, o[0], o[9], mb, self.d_out, *items)
-        self._decode_body(bs)
-        if self._gio and not self._feeding:
+            # (and this step's block-table updates)
+            ops.step_fetch(self._dec_bufs[p][0], self.dec_dev, o[0], o[9], mb, self.d_out, *items, updates=(self.bt_dev, o[8], self.R))
+        # one rank: the sampler's launch writes the tokens' pinned copy as well
+        host = self._out_bufs[p] if self._gio and self.fused_sampler and self.par.tp_size == 1 and self.par.custom_ar is None else None
+        self._decode_body(bs, host)
+        if self._gio and not self._feeding and host is None:
             ops.step_store(self.d_out, self._out_bufs[p], bs + 1)
 
-    def _decode_body(self, bs: int) -> None:
-        # this step's block-table updates (inside the graph; the fused layer applies them in its
+    def _decode_body(self, bs: int, host: Optional[torch.Tensor] = None) -> None:
+        # without the step I/O kernels the step's block-table updates are applied here (the fused layer does it in its
         # embedding launch)
         hid = self.model.hidden_states(self.d_ids[:bs], self.d_pos[:bs], self._decode_meta(bs), self.kv_caches,
-                                       scatter=(self.bt_dev, self.d_upd))
+                                       scatter=None if self._gio else (self.bt_dev, self.d_upd))
         if self._feeding:      # given tokens: the step ends in its logits, nothing is sampled
             lf = getattr(self.model, "logits_f32", None)
             if lf is None or self.model.plain_logits:
@@ -1735,7 +1738,7 @@ class LLMEngine:
             return
         if self.fused_sampler:
             self.model.sample(hid, self.d_temp[:bs], self.d_topp[:bs], self.d_topk[:bs], self.d_seed,
-                              self.d_out[:bs])
+                              self.d_out[:bs], **({} if host is None else {"host": host}))
             if self.par.custom_ar is not None:
                 self.par.graph_error_flag(self.d_out[bs:bs + 1])
             return

@@ -1131,6 +1131,11 @@ class HybridModel:
         return y
 
     # ------------------------------------------------------------------ forward
+    def _embed(self, ids: torch.Tensor) -> torch.Tensor:
+        if self.dtype == torch.bfloat16 and self.cfg.hidden % 8 == 0:      # (the gather kernel moves 16-byte vectors)
+            return ops.embedding(ids, self.embed)
+        return self.embed.index_select(0, ids.long())
+
     def hidden_states(self, input_ids: torch.Tensor, positions: torch.Tensor, meta, kv_caches: List[tuple],
                       scatter: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
         """Final-normed hidden states of the packed rows ``meta.last_idx`` (every row when
@@ -1138,36 +1143,32 @@ class HybridModel:
         cfg, eps = self.cfg, self.cfg.rms_eps
         if scatter is not None:
             ops.scatter_pairs(*scatter)
-        if self.dtype == torch.bfloat16:
-            if cfg.hidden % 8 == 0:
-                xl = ops.embedding(input_ids, self.embed)
-            else:      # the gather kernel moves 16-byte vectors
-                xl = self.embed.index_select(0, input_ids.long())
-            x = xl.float()
-        else:
-            x = self.embed.index_select(0, input_ids.long())
-            xl = None
-        if cfg.embed_scale != 1.0:
-            x = x * cfg.embed_scale      # f32; the pre-norm layers read their own normed copy
-            xl = None if xl is None else x.to(self.dtype)
+        T, W, nL = input_ids.shape[0], cfg.hidden, len(self.layers)
+        ln, rms = cfg.norm_kind == "layer", cfg.pre_norm and cfg.norm_kind != "layer" and not cfg.parallel_ff
+        # depth average: an f32 stack of the embedding output and every layer's result; layer i works in place on slot i + 1, which the
+        # previous layer's weighted sum has filled with its input
+        X = torch.empty((nL + 2, T, W), dtype=torch.float32, device=input_ids.device) if cfg.depth_average and not cfg.parallel_ff else None
+        x = X[0] if X is not None else torch.empty((T, W), dtype=torch.float32, device=input_ids.device)
+        xl = torch.empty((T, W), dtype=self.dtype, device=x.device) if self.dtype == torch.bfloat16 and not rms and not ln else None
+        h = torch.empty((T, W), dtype=self.dtype, device=x.device) if rms else None
+        n1 = self.layers[0]["norm1"]
+        if not seqmix.embed_rows(input_ids, self.embed, cfg.embed_scale, x, None if X is None else X[1], xl, n1 if rms else None, eps, h):
+            e = self._embed(input_ids)
+            x.copy_(e)
+            if cfg.embed_scale != 1.0:
+                x.mul_(cfg.embed_scale)      # f32; the pre-norm layers read their own normed copy
+            if X is not None:
+                X[1].copy_(x)
+            if xl is not None:
+                xl.copy_(x)
+            if rms:
+                seqmix.scaled_resadd_rms(x, eps, w=n1, out=h)
+        if X is not None:
+            x = X[1]
         if cfg.parallel_ff:
             return self._hidden_parallel(x, xl, positions, meta, kv_caches)
-        T, W, nL = x.shape[0], cfg.hidden, len(self.layers)
-        X = None
-        if cfg.depth_average:
-            # f32 stack of the embedding output and every layer's result; layer i works in place on
-            # slot i + 1, which the previous layer's weighted sum has filled with its input
-            X = torch.empty((nL + 2, T, W), dtype=torch.float32, device=x.device)
-            X[0].copy_(x)
-            X[1].copy_(x)
-            x = X[1]
-        h = None
-        ln = cfg.norm_kind == "layer"
         if ln:
-            h = seqmix.ls_resadd_ln(x, self.layers[0]["norm1"], self.layers[0]["norm1.b"], eps, self.dtype)
-        elif cfg.pre_norm:
-            h = torch.empty((T, W), dtype=self.dtype, device=x.device)
-            seqmix.scaled_resadd_rms(x, eps, w=self.layers[0]["norm1"], out=h)
+            h = seqmix.ls_resadd_ln(x, n1, self.layers[0]["norm1.b"], eps, self.dtype)
         for i, (L, S, cache) in enumerate(zip(self.layers, cfg.layers, kv_caches)):
             m = S.mixer
             if not cfg.pre_norm:
@@ -1273,8 +1274,8 @@ class HybridModel:
     def greedy(self, hidden: torch.Tensor) -> torch.Tensor:
         return ops.argmax(self._sampler_logits(hidden))
 
-    def sample(self, hidden, temperature, top_p, top_k, seed, out):
-        return ops.sample_rows(self._sampler_logits(hidden), temperature, top_p, top_k, seed, out=out)
+    def sample(self, hidden, temperature, top_p, top_k, seed, out, host=None):
+        return ops.sample_rows(self._sampler_logits(hidden), temperature, top_p, top_k, seed, out=out, host=host)
 
     def topk_candidates(self, hidden: torch.Tensor, k: int):
         v, i = torch.topk(self.logits(hidden).float(), min(k, self.cfg.vocab), dim=-1)

@@ -565,7 +565,7 @@ class LlamaModel:
         return allp[..., 1].gather(0, best.unsqueeze(0)).squeeze(0).to(torch.int32)
 
     def sample(self, hidden: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor, top_k: torch.Tensor,
-               seed: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+               seed: torch.Tensor, out: torch.Tensor, host: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Fused per-row sampling (greedy / exact top-k + top-p, ops.sample_rows) over the LM head.
 
         Under TP the vocab is sharded: every rank reduces its shard to its ranked top-256
@@ -573,10 +573,11 @@ class LlamaModel:
         replaces the [S, V] logits, and every rank merges the tp sorted lists and draws with the
         same seed (ops.tp_sample, one launch) -> the same token on all ranks, and the token the
         unsharded sampler would draw (the global top-k of any k <= 256 is inside the union of the
-        per-shard top-256).  Graph-capturable: three launches, no host sync, no torch.topk."""
+        per-shard top-256).  Graph-capturable: three launches, no host sync, no torch.topk.  ``host`` (one rank only): pinned
+        tokens, written by the same launch."""
         lg = self.logits(hidden)
         if self.par.tp_size == 1:
-            return ops.sample_rows(lg, temperature, top_p, top_k, seed, out=out)
+            return ops.sample_rows(lg, temperature, top_p, top_k, seed, out=out, host=host)
         cand = ops.tp_candidates(lg, self.vocab_shard.start)
         return ops.tp_sample(self.par.all_gather(cand), temperature, top_p, top_k, seed, out=out)
 

@@ -596,16 +596,20 @@ def sample_top_p(cand_vals: torch.Tensor, cand_idx: torch.Tensor, temperature: t
 
 
 def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Tensor, top_k: torch.Tensor,
-                seed: torch.Tensor, out: Optional[torch.Tensor] = None, shards: Optional[int] = None) -> torch.Tensor:
+                seed: torch.Tensor, out: Optional[torch.Tensor] = None, shards: Optional[int] = None,
+                host: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One-launch sampler over bf16 logits [B, V] (csrc/kernels/sampling.hip sample_rows_kernel):
     per row, temperature <= 0 -> arg-max, else exact top-k (top_k <= 0 -> 256 candidates),
     temperature, top-p and an inverse-CDF draw with u = hash(seed, row).  All parameters are
     device tensors (f32 / int32, ``seed`` an int32 scalar), so the call is graph-capturable.
     Small batches of large-vocab rows run sample_split_kernel instead (the row's vocab on up to 8
-    workgroups, same tokens; ``sample_split_shards``); ``shards`` forces a shard count (1: never)."""
+    workgroups, same tokens; ``sample_split_shards``); ``shards`` forces a shard count (1: never).
+    ``host`` (pinned int32): receives the tokens too."""
     ext = _native(logits)
     if ext is None:
         r = ref.sample_rows(logits, temperature.cpu(), top_p.cpu(), top_k.cpu(), int(seed.reshape(-1)[0]))
+        if host is not None:
+            host[:r.numel()].copy_(r)
         if out is not None:
             out[:r.numel()].copy_(r)
             return out
@@ -618,9 +622,9 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_p: torch.Te
         # (sample_split_kernel); the ranked lists go through the owner's split-K workspace
         from . import gemm as _gemm
         part, counters = _gemm._P.workspace(logits.device, B * P * SAMPLE_SPLIT_KMAX * 2, B)
-        ext.sample_split(logits, temperature, top_p, top_k, seed, part, counters, o, P)
+        ext.sample_split(logits, temperature, top_p, top_k, seed, part, counters, o, P, host)
     else:
-        ext.sample_rows(logits, temperature, top_p, top_k, seed, o)
+        ext.sample_rows(logits, temperature, top_p, top_k, seed, o, host)
     return o
 
 
@@ -766,11 +770,12 @@ from .gemm import autotune as gemm_autotune, linear, linear_swiglu, norm_linear 
 
 def step_fetch(dec_host: torch.Tensor, dec_dev: torch.Tensor, ids_off: int, src_off: int, n_ids: int,
                d_out: torch.Tensor, items_host: Optional[torch.Tensor] = None,
-               items_dev: Optional[torch.Tensor] = None) -> None:
+               items_dev: Optional[torch.Tensor] = None, updates: Optional[Tuple[torch.Tensor, int, int]] = None) -> None:
     """Decode-step inputs from a pinned host buffer into ``dec_dev`` by a kernel (graph-capturable,
     no copy engine): ``dec_dev[:] = dec_host`` except ids ``[ids_off, ids_off + n_ids)``, which take
     ``d_out[src[i]]`` where ``src[i] = dec_host[src_off + i] >= 0`` (the previous step's tokens);
-    and the work list ``items_dev <- items_host`` (its header's length)."""
+    and the work list ``items_dev <- items_host`` (its header's length).  ``updates`` = (int32 tensor, place of [n, index, value, ...]
+    in ``dec_host``, most pairs): ``scatter_pairs`` of them."""
     ext = _native(dec_dev)
     if ext is None:
         h = dec_host.to(dec_dev.device)
@@ -783,8 +788,10 @@ def step_fetch(dec_host: torch.Tensor, dec_dev: torch.Tensor, ids_off: int, src_
         if items_host is not None:
             n = work_items_len(items_host.numpy())
             items_dev[:n].copy_(items_host[:n])
+        if updates is not None:
+            scatter_pairs(updates[0], h[updates[1]:updates[1] + 1 + 2 * updates[2]])
         return
-    ext.step_fetch(dec_host, dec_dev, int(ids_off), int(src_off), int(n_ids), d_out, items_host, items_dev)
+    ext.step_fetch(dec_host, dec_dev, int(ids_off), int(src_off), int(n_ids), d_out, items_host, items_dev, *(updates or ()))
 
 
 def step_store(d_out: torch.Tensor, out_host: torch.Tensor, n: int) -> None:

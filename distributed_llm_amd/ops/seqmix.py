@@ -774,6 +774,15 @@ def scaled_resadd_rms(x: torch.Tensor, eps: float, y: Optional[torch.Tensor] = N
     ext.scaled_resadd_rms(x, y, float(mult), bool(set_), vec, w, float(eps), out)
 
 
+def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float, x: torch.Tensor, x2: Optional[torch.Tensor] = None,
+               lp: Optional[torch.Tensor] = None, w: Optional[torch.Tensor] = None, eps: float = 0.0,
+               h: Optional[torch.Tensor] = None) -> bool:
+    """The start of a step in one launch: table[ids] * scale as the f32 stream x [T, width] (and x2), its rounding lp, and
+    rmsnorm(x) * w in h (lp, h: the table's type).  False where there is no such launch (nothing is written then)."""
+    ext = _native(x)
+    return ext is not None and ext.embed_rows(ids, table, float(scale), x, x2, lp, w, float(eps), h)
+
+
 def rope_prep(proj, heads, kv_heads, dim, vdim, cos_sin, rot_dims, qscale, positions, slots, k_cache, v_cache, ucol: int = 0,
               act: Optional[torch.Tensor] = None, zero_rows: Optional[torch.Tensor] = None,
               bias: Optional[torch.Tensor] = None, qtab: Optional[torch.Tensor] = None) -> torch.Tensor:
