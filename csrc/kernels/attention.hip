@@ -94,7 +94,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
   auto& s_m = sm.m;
   auto& s_l = sm.l;
   const int splits = a.split_stride;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, rl = lane & 15;
   const int seq = tm.seq;
   const int G = a.G, tpt = 16 / G;

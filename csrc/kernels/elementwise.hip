@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256) embed_kernel(const int* __restrict__ ids,
     for (int i = threadIdx.x; i < n; i += blockDim.x) sc_dst[sc_buf[1 + 2 * i]] = sc_buf[2 + 2 * i];
     return;
   }
-  const long t = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const long t = blockIdx.x * 4L + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (t >= T) return;
   const long r = ids[t] - lo;
   const bool ok = r >= 0 && r < rows;
@@ -198,7 +198,7 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
                                                          int* __restrict__ ids, float* __restrict__ w,
                                                          float* __restrict__ logits, int shared, float scale,
                                                          const u16* __restrict__ norm_w, float eps, u16* __restrict__ xn) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int t = blockIdx.x * 4 + wv;
   if (t >= T) return;  // whole wave; no block barrier below
   const int nc = H >> 3;

@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   }
   __syncthreads();
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, rl = lane & 15;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, rl = lane & 15;
   const int q0 = (int)blockIdx.x * 64 + wave * 16;  // this wave's first query row
   const int q = q0 + rl;                             // this lane's query row
   if (q0 >= S) return;                               // wave-uniform: no barrier follows
@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict
                                                            int K) {
   constexpr int KS = 3, RS = 20;      // 384 = 4 waves of 3 steps, 1536 = 16 of 3; LDS rows of 16 + 4 floats reach every bank
   __shared__ __attribute__((aligned(16))) float red[NW][MT * 16][RS];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.x * 16;
   const int steps = K / 32, per = (steps + NW - 1) / NW, s0 = w * per, s1 = min(steps, s0 + per);
   const u16* wr = W + (long)(col0 + lr) * K + 8 * g;
@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ 
                                                         u16* __restrict__ Y, int M, int N, int K, const u16* __restrict__ lnw,
                                                         const u16* __restrict__ lnb, float eps, u16* __restrict__ Xn, u16* __restrict__ Vt) {
   __shared__ __attribute__((aligned(16))) u16 sx[FEW_M * FEW_LD];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.x * 16, steps = K / 32, c = 8 * lane;
   uint4 xv = {}, gw = {}, gb = {};
   FewW wf;
@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __r
                                                                   int Smax) {
   constexpr int KST = D / 32, NT = D / 16;
   __shared__ __attribute__((aligned(16))) u16 so[FEW_M * FEW_LD];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.x * 16, H = nh * D, steps = H / 32;
   const u16* qp = qkv + (long)min(lr, M - 1) * (3 * H) + w * D + 8 * g;
   bf16x8 qf[KST], kf[KST], vf[NT];

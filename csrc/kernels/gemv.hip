@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(256) gemv_kernel(const u16* __restrict__ X, lo
   float* s_ri = reinterpret_cast<float*>(xs + (XG ? 0L : (long)M * K)) + (NORM ? 4 * M : 0);
   float* s_ep = s_ri + M;
   float* s_red = s_ep + 4 * R * M;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr bool PAIRED = EPI == GV_QKV || EPI == GV_SWIGLU;
   // Virtual blocks: the launch may cap the grid below the column blocks (gemv_grid), and then a
   // workgroup walks blocks vb, vb + gridDim.x, ... with X staged ONCE: at batch 2-8 a per-block

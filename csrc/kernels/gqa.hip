@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(const T* __restrict__ pr
                                                         const int* __restrict__ slots, T* __restrict__ kc,
                                                         T* __restrict__ vc, T* __restrict__ q, int BSZ) {
   const long tok = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T* r = proj + tok * ld;
   const int slot = slots[tok];
   const long blk = slot >= 0 ? slot / BSZ : 0;
@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(256) attn_prep_vec_kernel(const u16* __restric
                                                             const int* __restrict__ slots, u16* __restrict__ kc, u16* __restrict__ vc,
                                                             u16* __restrict__ q, int BSZ, int T, int ny) {
   constexpr int LPH = D / 8, TW = APV_T / 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t0 = blockIdx.x * APV_T;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = blockIdx.x * APV_T;
   if ((int)blockIdx.y < ny) {
     const int hh = (blockIdx.y * 64 + lane) / LPH, c = lane % LPH * 8, half = rot >> 1;
     const int hx = min(hh, H + G - 1), f = c < half ? c : c - half;
@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(256) qk_norm_prep_kernel(const T* __restrict__
                                                            const int* __restrict__ slots, T* __restrict__ kc,
                                                            T* __restrict__ vc, T* __restrict__ q, int BSZ) {
   const long tok = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T* r = proj + tok * ld;
   const int slot = kc ? slots[tok] : -1;
   const long blk = slot >= 0 ? slot / BSZ : 0;
@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(256) rope_prep_kernel(const T* __restrict__ pr
 template <typename T>
 __global__ void __launch_bounds__(256) diff_combine_kernel(const float* __restrict__ a, T* __restrict__ out, long units, int H,
                                                            int G, int dv, float lam, float eps, float scale) {
-  const long u = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long u = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (u >= units) return;
   const long tok = u / H;
@@ -1251,7 +1251,7 @@ __global__ void __launch_bounds__(256) gqa_combine_kernel(const float* __restric
   // the first row's partials are asked for before it is known that there is such a row (every row has its place), and with their
   // weights: this is bound by trips to memory one behind the other (four users, 16 splits: 6.0 -> 4.6 us)
   constexpr int NZ = 16;
-  const int g = blockIdx.y, R = H / G, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = blockIdx.y, R = H / G, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long zs = (long)GM_ROWS * (dv + 2);
   const float* pt = part + ((long)blockIdx.x * G + g) * splits * zs;
   int row = blockIdx.z * 4 + wave;

@@ -68,7 +68,7 @@ __global__ void __launch_bounds__(256) latent_kv_write_kernel(const T* __restric
                                                               T* __restrict__ zl, int zh, int zc, long zn, long zt) {
   constexpr int NR = 8;      // values a lane keeps
   __shared__ float red[3];
-  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = slots[t];
   if (zl && slot < 0)
     for (int i = threadIdx.x; i < zh * zc; i += blockDim.x) stf(zl + i / zc * zn + t * zt + i % zc, 0.f);

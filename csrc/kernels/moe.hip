@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(256) moe_combine_resadd_kernel(const u16* __re
                                                                  const float* __restrict__ wts, int k, int H, int T,
                                                                  u16* __restrict__ r, long ldr, float* __restrict__ ssq, long ssq_ld,
                                                                  int cw) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= T) return;
   u16* rr = r + (long)row * ldr;
   const int c1 = min(H, (int)(blockIdx.y + 1) * cw);
@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(256) moe_gemm13_kernel(const u16* __restrict__
                                                          int H) {
   const int tile = blockIdx.x;
   if (tile >= *n_tiles) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col0 = blockIdx.y * 64 + wave * 16;
   if (col0 >= I) return;  // whole wave; the kernel has no block-level barrier
   const int e = tile_e[tile], r0 = tile_r0[tile], nrows = tile_n[tile];
@@ -270,7 +270,7 @@ __global__ void __launch_bounds__(256) moe_gemm2_kernel(const u16* __restrict__ 
                                                         float* __restrict__ y, int I, int H) {
   const int tile = blockIdx.x;
   if (tile >= *n_tiles) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col0 = blockIdx.y * 128 + wave * 32;
   if (col0 >= H) return;
   const int e = tile_e[tile], r0 = tile_r0[tile], nrows = tile_n[tile];

@@ -90,7 +90,7 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
     }
   };
   if constexpr (KS > 1) {
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __syncthreads();      // (a second pass of rows: the first one's sums are read)
 #pragma unroll
     for (int m = 0; m < MT; ++m)

@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const float* __rest
                                                              const float* __restrict__ w, T* __restrict__ out, long units,
                                                              int H, int dv, float eps, const int* __restrict__ qstart,
                                                              const int* __restrict__ qlen, int S) {
-  const long u = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long u = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (u >= units) return;
   const long tok = u / H;

@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256) rms_rows_kernel(const TI* __restrict__ x,
                                                        TO* __restrict__ y, long ldy, int rows, int n, float eps,
                                                        int groups) {
   // a wave per (row, part): `groups` equal consecutive parts of a row, each by its own root mean square
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (unit >= rows * groups) return;
   const int row = unit / groups, c0 = (unit % groups) * n;
   const TI* xr = x + (long)row * ldx + c0;
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256) rms_rows_kernel(const TI* __restrict__ x,
 template <typename TI, typename TO, int NE>
 __global__ void __launch_bounds__(256) rms_rows_reg_kernel(const TI* __restrict__ x, long ldx, const float* __restrict__ w,
                                                            TO* __restrict__ y, long ldy, int rows, int n, float eps, int groups) {
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (unit >= rows * groups) return;
   const int row = unit / groups, c0 = (unit % groups) * n;
   const TI* xr = x + (long)row * ldx + c0;
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restri
   constexpr bool EARLY = NE <= 16;     // the stream and the weights in flight with the row, where the registers allow
   constexpr int ST = PARTS ? 64 : 256;
   const long row = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, u = PARTS ? lane : (int)threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u = PARTS ? lane : (int)threadIdx.x;
   const int n = H / groups;
   float* xr = x + row * (long)H;
   for (int p = PARTS ? wave : 0; p < groups; p += 4) {
@@ -469,7 +469,7 @@ __global__ void __launch_bounds__(256) conv_silu_kernel(const T* x, long ldx, co
   const int step = 4 * gridDim.z;
   const float bias = b[c];
   float x0 = 0.f;     // the first token's own input (read before its output is stored)
-  for (int j = blockIdx.z * 4 + (threadIdx.x >> 6); j < n; j += step) {
+  for (int j = blockIdx.z * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); j < n; j += step) {
     float acc = bias;
     for (int k = 0; k + 1 < K; ++k) {
       const int i = j - (K - 1) + k;
@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(256) conv_vec_kernel(const u16* __restrict__ x
     for (int k = 0; k < K; ++k) wk[k][e] = w[(c + e) * K + k];
   }
   const int stride = 4 * gridDim.z * CV_RUN;
-  for (int j0 = (blockIdx.z * 4 + (threadIdx.x >> 6)) * CV_RUN; j0 < n; j0 += stride) {
+  for (int j0 = (blockIdx.z * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * CV_RUN; j0 < n; j0 += stride) {
     float hist[K > 1 ? K - 1 : 1][8];
 #pragma unroll
     for (int k = 0; k + 1 < K; ++k) {
@@ -1033,7 +1033,7 @@ __global__ void __launch_bounds__(256) retention_finish_kernel(const float* __re
                                                                long ld, int H, int d, int dv, float eps,
                                                                const int* __restrict__ qstart, const int* __restrict__ qlen,
                                                                int S, T* __restrict__ out, long rows_total) {
-  const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long r = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (r >= rows_total) return;
   const int lane = threadIdx.x & 63;
   const long tok = r / H;
@@ -1230,7 +1230,7 @@ __global__ void __launch_bounds__(256) route_topk_kernel(const float* __restrict
                                                          const float* __restrict__ corr, int real, int* __restrict__ ids,
                                                          float* __restrict__ wts, float* __restrict__ idw) {
   extern __shared__ float rsm[];
-  const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = blockIdx.x * 4 + wave;
   if (t >= T) return;
   route_one(logits + (long)t * ld, rsm + wave * route_patch(E), t, E, top, count, keep, smode, gmode, corr, real, ids, wts, idw);
 }
@@ -1283,7 +1283,7 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const u16* __restrict_
                                                           int* __restrict__ ids, float* __restrict__ wts, float* __restrict__ idw) {
   constexpr int EB = XC <= 4 ? 2 : 1;
   extern __shared__ float rsm[];        // [n] logits, then route_one's patch
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long t = blockIdx.x;
   router_dots<XC>(x + t * ldx, w, n, H, wave * EB, n, 4 * EB, rsm);
   __syncthreads();
@@ -1297,7 +1297,7 @@ template <int XC>
 __global__ void __launch_bounds__(256) router_logits_kernel(const u16* __restrict__ x, long ldx, const float* __restrict__ w, int n, int H,
                                                             float* __restrict__ logits) {
   constexpr int EB = XC <= 4 ? 2 : 1;
-  const int e0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * EB;
+  const int e0 = (blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * EB;
   const long t = blockIdx.x;
   router_dots<XC>(x + t * ldx, w, n, H, e0, min(n, e0 + EB), EB, logits + t * n);
 }
@@ -1330,7 +1330,7 @@ template <typename T>
 __global__ void __launch_bounds__(256) gated_group_norm_kernel(const float* __restrict__ y, const T* __restrict__ z, long ldz,
                                                                const float* __restrict__ w, T* __restrict__ out, int rows,
                                                                int n, int groups, float eps) {
-  const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int unit = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (unit >= rows * groups) return;
   const int row = unit / groups, c0 = (unit % groups) * n;
   const float* yr = y + (long)row * n * groups + c0;

@@ -138,7 +138,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
   float* s_red = s_rsp + TPR * BM;
   int* s_last = reinterpret_cast<int*>(s_red + 2 * BM);
 
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool loader = NL > 0 && wid >= NC;
   const int kg = loader ? 0 : wid / NW, wave = loader ? 0 : wid % NW;
   const int wm = wave / NWN, wn = wave % NWN;
