@@ -429,12 +429,12 @@ def tg_plan(M: int, N: int, K: int) -> Tuple[int, ...]:
             p = (_small(M, N, K) or (None,))[0]
     if p is not None:
         return tuple(p) + (1, 4)[len(p) - 4:] if len(p) < 6 else tuple(p)
-    mt128, nt128 = -(-M // 128), -(-N // 128)
-    if mt128 * nt128 >= 224:   # 8 waves: ~10 % ahead of 4 (profiles/r2_tgemm_tune_8b_shapes.log:25)
-        return (128, 128, 3, 1, 1, 8)
     mt64, nt64 = -(-M // 64), -(-N // 64)
-    if mt64 * nt128 >= 200:
-        return (64, 128, 3, 1, 1, 4)
+    # 64 x 128 tiles of eight waves from 150 of them on, two workgroups a CU.  us 128 x 128 / here / 64 x 64 (GELU epilogue): 3800 rows
+    # 1536 x 384 18 / 14 / 14, 384 x 1536 21 / 15 / 17, 8000 rows 1536 x 384 29 / 24 / 33, 1200 rows 3072 x 2048 27 / 25 / 32, 500 rows 1536 x
+    # 384 9 / 7 / 7; at 500 rows of 1152 x 1536 (72 tiles) 21 / 14 / 12.
+    if mt64 * -(-N // 128) >= 150:
+        return (64, 128, 3, 1, 1, 8)
     tiles = mt64 * nt64
     splits = 1
     while tiles * splits * 2 <= 512 and K // (splits * 2) >= 256 and splits < 8:
