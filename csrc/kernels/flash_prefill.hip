@@ -314,9 +314,10 @@ __global__ void __launch_bounds__(512, MINW) flash_prefill_kernel(FlashArgs a) {
       pv_chunk<D, NB, tail.value>(acc, vbase, pf, kb, kmax, rl, h);
     }
   };
-  const int whole = min(nchunks, kmax / CK);
+  const int whole = PIPE ? nchunks : min(nchunks, kmax / CK);      // (PIPE: the last chunk's P.V is behind the loop anyway)
   for (int t = c0; t < whole; ++t) chunk(t, std::false_type{});
-  if (max(whole, c0) < nchunks) chunk(max(whole, c0), std::true_type{});
+  if constexpr (!PIPE)
+    if (max(whole, c0) < nchunks) chunk(max(whole, c0), std::true_type{});
   if constexpr (PIPE) {
     if (kb_prev >= 0) pv_chunk<D, NB>(acc, vprev, pf_prev, kb_prev, kmax, rl, h);
   }
