@@ -360,17 +360,20 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(const T* __restrict__ q
   }
 }
 
+typedef float f32x3 __attribute__((ext_vector_type(3)));
+
 // A workgroup owns 16 value columns of one (sequence, head); its four waves own a quarter of the key dims each, as the
 // accumulators of the last product, which are at once the right operand of S^T k and S^T q.  The waves' parts meet in LDS, a
 // thread sums one element of each, and U = (I + A)^-1 R comes out as the right operand of the state's update.  Serial over the
 // tiles, so the chain of one tile bounds it: two products, one exchange, two small products, the update.  Sums of more than four terms go in
-// parts that are added pairwise, or the largest last.  bf16, 16 heads of 128 x 128: 6 sequences of 1400 tokens 363 us with the two
-// launches beside it against 617 token by token, one of 4096 tokens 536 against 1219 (358 and 520 without the look for infinities and
-// NaN; before that, with one chain a sum, 314 and 472, with outputs up to 1.5 times as far off as token by token).  f32 errors against 64 bits over 385 tokens, state and outputs, token by token
+// parts that are added pairwise, or the largest last.  Three workgroups of the wide-load form fit a CU (its registers are bounded for
+// that: with two, 6 sequences are a second pass and take 437 us).  bf16, 16 heads of 128 x 128, with the two launches beside it: 6
+// sequences of 1400 tokens 373 us, one of 4096 tokens 433 (421 and 535 with waits for loads just issued, 617 and 1219 token by token).
+// f32 errors against 64 bits over 385 tokens, state and outputs, token by token
 // in brackets: decays near 1 1.5e-7 (5.6e-7), 1.7e-7 (2.6e-7); a model's (0.01 to 0.3 a token) 1.2e-7 (1.9e-7), 1.6e-7 (1.7e-7); up
 // to 4 a token 1.0e-7 (1.05e-7), 1.53e-7 (1.49e-7).
 template <typename T, int NS, bool VL>
-__global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ qkv, long ldq, int H, int G, int d, int dv,
+__global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __restrict__ qkv, long ldq, int H, int G, int d, int dv,
                                                          float* __restrict__ state, const int* __restrict__ qstart,
                                                          const int* __restrict__ qlen, const int* __restrict__ ctx,
                                                          const int* __restrict__ rows, const float* __restrict__ pre,
@@ -384,7 +387,7 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
   const int h = blockIdx.y, s = blockIdx.z;
   const int n = qlen[s];
   if (n <= 0) return;   // the whole workgroup
-  const int tid = threadIdx.x, lr = tid & 15, row = tid >> 4, w = tid >> 6, g4 = (tid >> 4) & 3;
+  const int tid = threadIdx.x, lr = tid & 15, row = tid >> 4, w = __builtin_amdgcn_readfirstlane(tid >> 6), g4 = (tid >> 4) & 3;
   const int j = blockIdx.x * 16 + lr;
   const bool live = j < dv;
   const int q0 = qstart[s], p0 = ctx[s] - n;
@@ -406,66 +409,62 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
   }
   const long oq = (long)(h / (H / G)) * d, ok = (long)G * d + oq, ov = 2L * G * d + (long)h * dv + (live ? j : dv - 1);
   // two tiles' inputs travel while one is computed: NS dims of one token's q and k with their factors; one value and its
-  // scalars, four entries of a row of (I + A)^-1 and of P
+  // scalars, four entries of a row of (I + A)^-1 and of P.  No load stands behind a condition or is copied on from tile to tile (rows past
+  // the end read the last token's and become zeros where they are used; two tiles take turns with two sets of registers): the
+  // compiler then knows which are in flight, where it waited for all of them at the head of every tile
+  const int kcol = NS * lr < d ? NS * lr : 0;
   row_t rq, rk;
   float2 fac = make_float2(0.f, 0.f);
   auto fetch_keys = [&](int t0) {
-    rq = row_t(T(0));
-    rk = row_t(T(0));
-    if (t0 + row < n) {
-      const T* x = qkv + (long)(q0 + t0 + row) * ldq;
-      if constexpr (VL) {
-        if (NS * lr < d) {
-          rq = *reinterpret_cast<const row_t*>(x + oq + NS * lr);
-          rk = *reinterpret_cast<const row_t*>(x + ok + NS * lr);
-        }
-      } else {
+    const int at = q0 + min(t0 + row, n - 1);
+    const T* x = qkv + (long)at * ldq;
+    if constexpr (VL) {
+      rq = *reinterpret_cast<const row_t*>(x + oq + kcol);
+      rk = *reinterpret_cast<const row_t*>(x + ok + kcol);
+    } else {
 #pragma unroll
-        for (int r = 0; r < NS; ++r)
-          if (NS * lr + r < d) {
-            rq[r] = x[oq + NS * lr + r];
-            rk[r] = x[ok + NS * lr + r];
-          }
+      for (int r = 0; r < NS; ++r) {
+        rq[r] = x[oq + min(kcol + r, d - 1)];
+        rk[r] = x[ok + min(kcol + r, d - 1)];
       }
-      fac = *reinterpret_cast<const float2*>(pre + ((long)(q0 + t0 + row) * H + h) * DT_W + 2 * DT_L + 4);
     }
+    fac = *reinterpret_cast<const float2*>(pre + ((long)at * H + h) * DT_W + 2 * DT_L + 4);
   };
-  auto stage_keys = [&](int buf) {
+  auto stage_keys = [&](int buf, int t0) {
+    const bool in = t0 + row < n;
 #pragma unroll
     for (int r = 0; r < NS; r += 4) {
       f32x4 a, b;
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const T y = rq[r + x], z = rk[r + x];
-        a[x] = ldf(&y) * fac.x;
-        b[x] = ldf(&z) * fac.y;
+        const bool on = in && NS * lr + r + x < d;
+        a[x] = on ? ldf(&y) * fac.x : 0.f;
+        b[x] = on ? ldf(&z) * fac.y : 0.f;
       }
       *reinterpret_cast<f32x4*>(qs[buf] + row * LD + NS * lr + r) = a;
       *reinterpret_cast<f32x4*>(ks[buf] + row * LD + NS * lr + r) = b;
     }
   };
-  struct Tile { T v; f32x4 sc, inv, p; };
-  auto fetch_tile = [&](int t0) {
-    Tile t;
-    t.v = T(0);
-    t.sc = t.inv = t.p = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (t0 + row < n) {
-      t.v = qkv[(long)(q0 + t0 + row) * ldq + ov];
-      t.sc = *reinterpret_cast<const f32x4*>(pre + ((long)(q0 + t0 + row) * H + h) * DT_W + 2 * DT_L);
-    }
-    if (t0 + lr < n) {
-      const float* x = pre + ((long)(q0 + t0 + lr) * H + h) * DT_W + 4 * g4;
-      t.inv = *reinterpret_cast<const f32x4*>(x);
-      t.p = *reinterpret_cast<const f32x4*>(x + DT_L);
-    }
-    return t;
+  // (three scalars: a register that a load writes and nobody reads is given away while the load is under way, and its next owner waits)
+  struct Tile { T v; f32x3 sc; f32x4 inv, p; };
+  auto fetch_tile = [&](Tile& t, int t0) {
+    const int at = q0 + min(t0 + row, n - 1);
+    t.v = qkv[(long)at * ldq + ov];
+    t.sc = *reinterpret_cast<const f32x3*>(pre + ((long)at * H + h) * DT_W + 2 * DT_L);
+    const float* x = pre + ((long)(q0 + min(t0 + lr, n - 1)) * H + h) * DT_W + 4 * g4;
+    t.inv = *reinterpret_cast<const f32x4*>(x);
+    t.p = *reinterpret_cast<const f32x4*>(x + DT_L);
   };
+  __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): the state has landed, so that no tile waits for it
   fetch_keys(0);
-  Tile cur = fetch_tile(0), nxt = fetch_tile(DT_L);
-  stage_keys(0);
+  Tile even, odd;
+  fetch_tile(even, 0);
+  fetch_tile(odd, DT_L);
+  stage_keys(0, 0);
   fetch_keys(DT_L);
   __syncthreads();
-  for (int t0 = 0, buf = 0; t0 < n; t0 += DT_L, buf ^= 1) {
+  auto tile = [&](const int t0, const int buf, Tile& cur) {
     const int nt = min(DT_L, n - t0);
     {
       f32x4 tk[4], tq[4];
@@ -486,6 +485,10 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
       *reinterpret_cast<f32x4*>(p + TP) = (tq[0] + tq[1]) + (tq[2] + tq[3]);
     }
     __syncthreads();
+    if (nt < DT_L) {      // the last tile: zeros behind the end
+      if (row >= nt) cur.sc = f32x3{0.f, 0.f, 0.f};
+      if (lr >= nt) cur.inv = cur.p = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     {   // token `row`, column lr
       const float* p = part + lr * DT_P + row;
       const float ek = (p[0] + p[2 * TP]) + (p[4 * TP] + p[6 * TP]), eq = (p[TP] + p[3 * TP]) + (p[5 * TP] + p[7 * TP]);
@@ -494,10 +497,8 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
       if (lr == 0) ws[row] = cur.sc[2];
       if (tid == 16 * (nt - 1)) last = cur.sc[0];
     }
-    if (t0 + DT_L < n) {
-      stage_keys(buf ^ 1);
-      fetch_keys(t0 + 2 * DT_L);
-    }
+    stage_keys(buf ^ 1, t0 + DT_L);      // (behind the last tile: zeros that nobody reads)
+    fetch_keys(t0 + 2 * DT_L);
     __syncthreads();
     f32x4 r = *reinterpret_cast<const f32x4*>(Rs + lr * DT_P + 4 * g4);
     // An infinity or NaN of a token must not reach those before it, whose zeros in (I + A)^-1 and P it would meet: it leaves the
@@ -555,9 +556,15 @@ __global__ void __launch_bounds__(256) delta_tile_kernel(const T* __restrict__ q
       for (int x = 0; x < 4; ++x)
         if (live && 4 * g4 + x < nt) raw[((long)(q0 + t0 + 4 * g4 + x) * H + h) * dv + j] = o[x];
     }
-    cur = nxt;
-    nxt = fetch_tile(t0 + 2 * DT_L);
+    fetch_tile(cur, t0 + 2 * DT_L);
+  };
+  // pairs of tiles and perhaps one more: a way out between two of a pair would meet the way back in a block, with its loads under way
+  const int tiles = (n + DT_L - 1) / DT_L;
+  for (int i = 0; i < tiles / 2; ++i) {
+    tile(2 * i * DT_L, 0, even);
+    tile((2 * i + 1) * DT_L, 1, odd);
   }
+  if (tiles & 1) tile((tiles - 1) * DT_L, 0, even);
   if (!live) return;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
