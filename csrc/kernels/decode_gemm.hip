@@ -57,6 +57,12 @@ __device__ __forceinline__ uint4 ldb16(__amdgpu_buffer_rsrc_t r, unsigned off) {
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
 }
 
+// the loads of a stage stay together, behind the products before them
+__device__ __forceinline__ void keep_order() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int MT, int NT, int VS, int EPI>
 struct Dg {
   static constexpr int WV = 4 * VS, T = 64 * WV, NC = 16 * NT, MR = 16 * MT, LD = NC + 4;
@@ -69,7 +75,8 @@ struct Dg {
   static constexpr int LDS = WV * REG + (SQ ? WV * MR * 4 : MR * (NC / 4) * 4) + 16;
 };
 
-template <int MT, int NT, int VS, int EPI>
+// ONE: a wave's K is one stage (a second one, all out of range, cost the products of a 1024-wide layer 3 %)
+template <int MT, int NT, int VS, int EPI, bool ONE>
 __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   using C = Dg<MT, NT, VS, EPI>;
   constexpr int NC = C::NC, MR = C::MR, LD = C::LD, U = C::U, WV = C::WV, T = C::T, NI = C::NI, PX = C::PX;
@@ -116,9 +123,9 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     if constexpr (SQ) sq[m] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const int nt16 = (N + 15) >> 4;
-  const u16* wt[NT];      // wave-uniform: the lane's 16 bytes are a 32-bit offset of the load
+  __amdgpu_buffer_rsrc_t wt[NT];      // a tile's weights up to the wave's last k: reads behind it are zeros that cost no traffic
 #pragma unroll
-  for (int n = 0; n < NT; ++n) wt[n] = a.W + (long)min(tile * NT + n, nt16 - 1) * 16 * K;
+  for (int n = 0; n < NT; ++n) wt[n] = make_rsrc(a.W + (long)min(tile * NT + n, nt16 - 1) * 16 * K, (unsigned)wk1 * 32);
   // X: fragments (row r16, 8 k of group g), or rows (XL): 4 U lanes a row
   constexpr int LR = 4 * U, RPI = 64 / LR;
   const int xr = XL ? lane / LR : r16, xc = XL ? lane % LR : g;
@@ -127,23 +134,28 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   const unsigned x0 = (unsigned)(xr * (int)a.ldx + 8 * xc) * 2;
   unsigned char* mine = dg_smem + wave * C::REG;
 
+  // A stage's rows first: they go through LDS while its weights are on their way.  No load stands behind a condition (past the wave's
+  // k they are out of the buffers' ranges): where ways with and without a load meet, the compiler waits for all that are in flight, and
+  // with `if (there is a next stage) load` in the loop it had one stage's latency for every two.  us in a captured graph, weights from HBM, 48
+  // rows: 11264 x 2048 SwiGLU 13.0 -> 11.8, 2560 x 2048 QKV 8.4 -> 7.6, 2048 x 2048 6.8 -> 6.6, 2048 x 5632 10.2 -> 10.1; 16 rows 10.3 -> 9.8, 6.0 -> 5.7,
+  // 8.9 -> 8.6 (the last).  Three stages of two steps: 12.3, 7.7, 6.9, 10.0.
   struct Stage { bf16x8 w[U][NT]; uint4 x[U * MT]; };
-  auto load = [&](Stage& st, int k0, int cnt) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (u < cnt) {
-#pragma unroll
-        for (int n = 0; n < NT; ++n) st.w[u][n] = ldnt_bf16x8(wt[n] + (long)(k0 + 32 * u) * 16 + (unsigned)lane * 8);
-      }
+  auto load = [&](Stage& st, int k0) {
+    keep_order();
+    const unsigned wo = (unsigned)(k0 * 32 + lane * 16), xo = k0 < wk1 ? x0 + (unsigned)k0 * 2 : 0x40000000u;
     if constexpr (XL) {
       // (a short stage reads on into other k: never multiplied)
 #pragma unroll
-      for (int i = 0; i < U * MT; ++i) st.x[i] = ldb16(xb, x0 + (unsigned)(RPI * i * (int)a.ldx + k0) * 2);
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (u < cnt) st.x[u] = ldb16(xb, x0 + (unsigned)(k0 + 32 * u) * 2);
+      for (int i = 0; i < U * MT; ++i) st.x[i] = ldb16(xb, xo + (unsigned)(RPI * i * (int)a.ldx) * 2);
     }
+    keep_order();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) st.w[u][n] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wt[n], wo + u * 1024, 0, 2));
+      if constexpr (!XL) st.x[u] = ldb16(xb, xo + u * 64);
+    }
+    keep_order();
   };
   auto compute = [&](const Stage& st, int cnt) {
     if constexpr (XL) {
@@ -164,9 +176,10 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
         }
       }
   };
-  const int steps = (wk1 - wk0) / 32, nblk = steps / U, tail = steps - nblk * U;
+  const int steps = (wk1 - wk0) / 32;
   Stage A, B;
-  if (nblk > 0) load(A, wk0, U);
+  load(A, wk0);
+  if constexpr (!ONE) load(B, wk0 + 32 * U);
   float4 e_co[EPI == DG_QKV ? NI : 1], e_si[EPI == DG_QKV ? NI : 1];
   if constexpr (EPI == DG_QKV) {
     const int hd = a.d / 2, qk = (a.nq + a.nkv) * a.d;
@@ -181,20 +194,17 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
       }
     }
   }
-  int kb = wk0;
-  for (int i = 0; i < nblk; i += 2) {
-    if (i + 1 < nblk) load(B, kb + 32 * U, U);
-    compute(A, U);
-    if (i + 1 < nblk) {
-      if (i + 2 < nblk) load(A, kb + 64 * U, U);
+  int i = 0;
+  if constexpr (!ONE) {
+    for (; i + 2 * U < steps; i += 2 * U) {
+      compute(A, U);
+      load(A, wk0 + (i + 2 * U) * 32);
       compute(B, U);
+      load(B, wk0 + (i + 3 * U) * 32);
     }
-    kb += 64 * U;
   }
-  if (tail > 0) {
-    load(A, wk0 + nblk * 32 * U, tail);
-    compute(A, tail);
-  }
+  if (steps > i) compute(A, steps - i);
+  if (!ONE && steps > i + U) compute(B, steps - i - U);
 
   // ---- the waves' partial tiles meet in LDS (each wave's own piece: its staged rows are read).  acc[m][n][r] = C[16m + 4g + r][16n + r16]
   float* pt = reinterpret_cast<float*>(mine);
@@ -401,15 +411,17 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   }
 }
 
-template <int MT, int NT, int VS, int EPI>
+template <int MT, int NT, int VS, int EPI, bool ONE = false>
 int launch(const DgArgs& a, int gy, hipStream_t st) {
   using C = Dg<MT, NT, VS, EPI>;
   static_assert(C::LDS <= 160 * 1024, "LDS of a workgroup");
+  if constexpr (VS == 4 && !ONE)
+    if (a.kchunk <= 128 * C::U) return launch<MT, NT, VS, EPI, true>(a, gy, st);
   static const int rc = C::LDS <= 64 * 1024 ? 0      // raised once: no attribute call inside a later stream capture
-                            : (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI>,
+                            : (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI, ONE>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
   if (rc) return rc;
-  hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI>), dim3((a.N + C::NC - 1) / C::NC, gy), dim3(C::T), C::LDS, st, a);
+  hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, ONE>), dim3((a.N + C::NC - 1) / C::NC, gy), dim3(C::T), C::LDS, st, a);
   return (int)hipGetLastError();
 }
 
