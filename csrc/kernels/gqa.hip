@@ -845,8 +845,8 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(c
   uint4 pk_[NFK], pv_[NFV];
   // A thread moves the same (key, chunk) and (dim, page, half) of every tile (tiles start at multiples
   // of 64 keys), so only the page ids change from tile to tile: offsets inside a page are kept.
-  int koff[NFK], voff[NFV];      // inside a page
-  int kkey[NFK], vpg[NFV];
+  int koff[NFK], voff[NFV];      // inside a page (past d or dv: the row's first, and zeros when staged)
+  int kkey[NFK];
   bool kon[NFK], von[NFV];
   const long kpage = (long)G * GM_BS * d, vpage = (long)GV * dv * GM_BS;
   const int gv = g / (G / GV);
@@ -856,29 +856,32 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(c
     const int kk = e / KCH, c = (e % KCH) * 8;
     kkey[f] = kk;
     kon[f] = c < d;
-    koff[f] = (g * GM_BS + (kk & 15)) * d + c;
+    koff[f] = (g * GM_BS + (kk & 15)) * d + (kon[f] ? c : 0);
   }
+  const int vpg = (tid % (GM_KT / 8)) >> 1;      // the page a thread's values are on
 #pragma unroll
   for (int f = 0; f < NFV; ++f) {
     const int e = tid + 256 * f;
     const int j = e / (GM_KT / 8), cc = e % (GM_KT / 8);
-    vpg[f] = cc >> 1;
     von[f] = j < dv;
-    voff[f] = (gv * dv + j) * GM_BS + 8 * (cc & 1);
+    voff[f] = (gv * dv + (von[f] ? j : 0)) * GM_BS + 8 * (cc & 1);
   }
-  auto fetch = [&](int k0) {
-    const int nk = min(GM_KT, last + 1 - k0);
-    const int* pg = btr + (k0 >> 4);
+  // A tile's page ids are loaded a tile ahead of its keys, and no load stands behind a condition of its own (pages past the newest key:
+  // its page again, and zeros when staged): a load that waits for its page id waits for all loads before it, and a tile took one
+  // latency per chunk (us, then -> now: 16 heads of 96 / 64, 4001 tokens 183 -> 143; 16 / 4 of 128, four sequences of 2900 66 -> 54; 16 of 256, 1500
+  // tokens 180 -> 121; 32 / 8 of 64, six of 1400 224 -> 211)
+  int kid[NFK], vid;
+  const int page_last = last >> 4;
+  auto fetch_ids = [&](int k0) {
 #pragma unroll
-    for (int f = 0; f < NFK; ++f) {
-      pk_[f] = make_uint4(0u, 0u, 0u, 0u);
-      if (kon[f] && kkey[f] < nk) pk_[f] = *reinterpret_cast<const uint4*>(kc + pg[kkey[f] >> 4] * kpage + koff[f]);
-    }
+    for (int f = 0; f < NFK; ++f) kid[f] = btr[min((k0 + kkey[f]) >> 4, page_last)];
+    vid = btr[min((k0 >> 4) + vpg, page_last)];
+  };
+  auto fetch = [&] {
 #pragma unroll
-    for (int f = 0; f < NFV; ++f) {
-      pv_[f] = make_uint4(0u, 0u, 0u, 0u);
-      if (von[f] && 16 * vpg[f] < nk) pv_[f] = *reinterpret_cast<const uint4*>(vc + pg[vpg[f]] * vpage + voff[f]);
-    }
+    for (int f = 0; f < NFK; ++f) pk_[f] = *reinterpret_cast<const uint4*>(kc + kid[f] * kpage + koff[f]);
+#pragma unroll
+    for (int f = 0; f < NFV; ++f) pv_[f] = *reinterpret_cast<const uint4*>(vc + vid * vpage + voff[f]);
   };
   // small grids (decode steps) split a row's key tiles over `splits` workgroups; each leaves its
   // running maximum, sum and unnormalised output in `part`, gqa_combine merges them
@@ -890,10 +893,23 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(c
   const int vbeg = (int)((long)ntiles * blockIdx.z / splits);
   const int vend = (int)((long)ntiles * (blockIdx.z + 1) / splits);   // exclusive
   auto tile_k0 = [&](int v) { return (v < nkeep ? v : tfirst + v - nkeep) * GM_KT; };
-  if (vbeg < vend) fetch(tile_k0(vbeg));
+  if (vbeg < vend) {
+    fetch_ids(tile_k0(vbeg));
+    fetch();
+    fetch_ids(tile_k0(min(vbeg + 1, vend - 1)));
+  }
   for (int vt = vbeg; vt < vend; ++vt) {
     const int k0 = tile_k0(vt);
     __syncthreads();   // the previous tile is consumed
+    const int nk = last + 1 - k0;
+    if (nk < GM_KT || d < KD || dv < VD) {
+#pragma unroll
+      for (int f = 0; f < NFK; ++f)
+        if (!(kon[f] & (kkey[f] < nk))) pk_[f] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int f = 0; f < NFV; ++f)
+        if (!(von[f] & (16 * vpg < nk))) pv_[f] = make_uint4(0u, 0u, 0u, 0u);
+    }
 #pragma unroll
     for (int f = 0; f < NFK; ++f) {
       const int e = tid + 256 * f;
@@ -906,7 +922,10 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(c
       const int j = e / (GM_KT / 8), cc = e % (GM_KT / 8);
       *reinterpret_cast<uint4*>(vtr + j * VSTR + 8 * cc) = pv_[f];
     }
-    if (vt + 1 < vend) fetch(tile_k0(vt + 1));   // the next tile's loads fly under this tile's products
+    if (vt + 1 < vend) {      // the next tile's loads fly under this tile's products
+      fetch();
+      fetch_ids(tile_k0(min(vt + 2, vend - 1)));
+    }
     __syncthreads();
     if (k0 > wave_last) continue;   // this wave's rows see nothing of the tile (the barriers above are uniform)
     if (k0 >= keep && k0 + GM_KT <= wave_lo) continue;   // ... or the tile lies before every row's window / chunk
