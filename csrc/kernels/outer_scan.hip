@@ -70,51 +70,73 @@ __global__ void __launch_bounds__(256) outer_scan_kernel(const T* __restrict__ k
   float* Ms = Gb + OS_TG;               // [TG]  mLSTM: m_t
   float* Ps = Ms + OS_TG;               // [TG][STRIPS][CW] partial sums
   const int kh = h / kq_heads_div;      // SSD: the head's group; mLSTM: the head
+  // A group's inputs are loaded a group ahead, the first ones beside the state, and no load stands behind a condition (entries that do
+  // not exist read a neighbour and are zeros where they are staged).  us, then -> now, 32 heads of 128 x 64: 8 sequences of 200 to 600 tokens 244
+  // -> 197 (the walk over the tokens, whose rows come from LDS, bounds it), a step of 12 sequences 15.1 -> 13.5
+  constexpr int EK = (OS_TG * NP + 255) / 256, EV = (OS_TG * CW + 255) / 256;
+  T fk[EK], fq[EK], fv[EV], fa, fb;
+  auto fetch = [&](int t0) {
+    const int tl = n_new - 1;
+#pragma unroll
+    for (int i = 0; i < EK; ++i) {
+      const int e = tid + 256 * i;
+      const T* r = kq + (long)(q0 + min(t0 + e / NP, tl)) * ld_kq + (long)kh * N + min(e % NP, N - 1);
+      fk[i] = r[k_off];
+      fq[i] = r[q_off];
+    }
+#pragma unroll
+    for (int i = 0; i < EV; ++i) {
+      const int e = tid + 256 * i;
+      fv[i] = vsrc[(long)(q0 + min(t0 + e / CW, tl)) * ld_v + v_off + (long)h * dv + min(v0 + e % CW, dv - 1)];
+    }
+    const T* g = gsrc + (long)(q0 + min(t0 + (tid & (OS_TG - 1)), tl)) * ld_g;
+    fa = g[g_off + h];
+    if constexpr (MLSTM) fb = g[g_off2 + h];
+  };
   float S[NPT];
   float* sp = state + (((long)slot * H + h) * N) * dv + v0 + c;
   float* np = MLSTM ? nm + (((long)slot * H + h) * NCB + cb) * (N + 1) : nullptr;
 #pragma unroll
-  for (int k = 0; k < NPT; ++k) {
-    const int n = strip + k * STRIPS;
-    float v = 0.f;
-    if (col_ok && n < N && p0 > 0) v = is_norm ? np[n] : sp[(long)n * dv];
-    S[k] = v;
-  }
+  for (int k = 0; k < NPT; ++k) S[k] = 0.f;
   float m = 0.f;
-  if (MLSTM && p0 > 0) m = np[N];
+  if (p0 > 0) {
+    const float* s0 = is_norm ? np : sp + (col_ok ? 0 : -c);
+    const long ss = is_norm ? 1 : dv;
+#pragma unroll
+    for (int k = 0; k < NPT; ++k) S[k] = s0[min(strip + k * STRIPS, N - 1) * ss];
+    if (MLSTM) m = np[N];
+  }
   const float hp0 = p0v ? p0v[h] : 0.f, hp1 = p1v ? p1v[h] : 0.f, hp2 = p2v ? p2v[h] : 0.f;
+  fetch(0);
+#pragma unroll
+  for (int k = 0; k < NPT; ++k) S[k] = col_ok & (strip + k * STRIPS < N) ? S[k] : 0.f;
   for (int t0 = 0; t0 < n_new; t0 += OS_TG) {
     const int nt = min(OS_TG, n_new - t0);
     __syncthreads();     // the previous group's sums are stored
-    for (int e = tid; e < nt * NP; e += 256) {
-      const int t = e / NP, n = e % NP;
-      float2 v = make_float2(0.f, 0.f);
-      if (n < N) {
-        const T* r = kq + (long)(q0 + t0 + t) * ld_kq + (long)kh * N + n;
-        v = make_float2(ldf(r + k_off), ldf(r + q_off) * qscale);
-      }
-      KQ[e] = v;
+#pragma unroll
+    for (int i = 0; i < EK; ++i) {
+      const int e = tid + 256 * i;
+      const bool on = e % NP < N;
+      if (e < OS_TG * NP) KQ[e] = make_float2(on ? ldf(&fk[i]) : 0.f, on ? ldf(&fq[i]) * qscale : 0.f);
     }
-    for (int e = tid; e < nt * CW; e += 256) {
-      const int t = e / CW, cc = e % CW;
-      float v = 0.f;
-      if (MLSTM && cc == OS_COLS) v = 1.f;
-      else if (v0 + cc < dv) v = ldf(vsrc + (long)(q0 + t0 + t) * ld_v + v_off + (long)h * dv + v0 + cc);
-      Vs[e] = v;
+#pragma unroll
+    for (int i = 0; i < EV; ++i) {
+      const int e = tid + 256 * i, cc = e % CW;
+      if (e < OS_TG * CW) Vs[e] = MLSTM && cc == OS_COLS ? 1.f : v0 + cc < dv ? ldf(&fv[i]) : 0.f;
     }
     if (tid < nt) {
-      const T* g = gsrc + (long)(q0 + t0 + tid) * ld_g;
       if (MLSTM) {
         // hp0 / hp1: the input and forget gates' biases
-        Ga[tid] = cap * tanhf((ldf(g + g_off + h) + hp0) / cap);
-        Gb[tid] = logsigmoid_f(cap * tanhf((ldf(g + g_off2 + h) + hp1) / cap));
+        Ga[tid] = cap * tanhf((ldf(&fa) + hp0) / cap);
+        Gb[tid] = logsigmoid_f(cap * tanhf((ldf(&fb) + hp1) / cap));
       } else {
         // hp0: step bias, hp1: -exp(A_log)
-        const float dt = softplus_f(ldf(g + g_off + h) + hp0);
+        const float dt = softplus_f(ldf(&fa) + hp0);
         Ga[tid] = expf(hp1 * dt);
         Gb[tid] = dt;
       }
     }
+    if (t0 + OS_TG < n_new) fetch(t0 + OS_TG);
     __syncthreads();
     if (live) {
       for (int t = 0; t < nt; ++t) {
