@@ -22,28 +22,33 @@ namespace {
 constexpr int MD_PAIRS = 256;
 constexpr int MD_TILES = 2;      // column tiles a workgroup of KS 1: the 64 x 9 waves of a 1024-wide layer reach every CU
 
+// 32 k of a tile's weights; past the buffer's last k zeros that cost no traffic
+__device__ __forceinline__ bf16x8 md_w(__amdgpu_buffer_rsrc_t r, int k) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, (unsigned)k * 32 + (threadIdx.x & 63) * 16, 0, 0));
+}
+
 template <int ACT, int MT, int KS>
-__device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx, int div, const u16* __restrict__ wt, int kb, int K,
+__device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx, int div, __amdgpu_buffer_rsrc_t wt, int kb, int K,
                                             const int* list, int row0, int n, int c0, void* __restrict__ out, long ldo,
                                             const bf16x8 (&w0)[4], float (*s_acc)[KS > 1 ? 32 : 1][17]) {      // k in [kb, K)
   const int lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
+  // no load stands behind a condition (rows past n read the last one's, k past the end nothing or the last step's; neither is used):
+  // where ways with and without a load meet the compiler waits for all loads in flight
   const u16* xr[MT];
-  bool ok[MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    ok[m] = row0 + 16 * m + r16 < n;
-    xr[m] = x + (long)(list[min(row0 + 16 * m + r16, n - 1)] / div) * ldx + 8 * g;
-  }
+  for (int m = 0; m < MT; ++m) xr[m] = x + (long)(list[min(row0 + 16 * m + r16, n - 1)] / div) * ldx + 8 * g;
   constexpr int U = MT > 2 || (KS > 1 && MT > 1) ? 2 : 4;
+  const int klast = max(K - 32, 0);
   struct Stage { bf16x8 w[U]; uint4 x[U][MT]; };
-  auto load = [&](Stage& st, int k0, bool first) {
+  auto load = [&](Stage& st, int k0, int first) {      // `first`: the stage's place among the weights loaded ahead (-1: not there)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (k0 + 32 * u >= K) break;      // (uniform)
-      st.w[u] = first ? w0[u] : __builtin_bit_cast(bf16x8, ld16(wt + (long)(k0 + 32 * u) * 16 + (unsigned)lane * 8));
+      st.w[u] = first >= 0 ? w0[first + u] : md_w(wt, k0 + 32 * u);
 #pragma unroll
-      for (int m = 0; m < MT; ++m) st.x[u][m] = ok[m] ? ld16(xr[m] + k0 + 32 * u) : make_uint4(0, 0, 0, 0);
+      for (int m = 0; m < MT; ++m) st.x[u][m] = ld16(xr[m] + min(k0 + 32 * u, klast));
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
   f32x4 acc[MT];
 #pragma unroll
@@ -51,32 +56,39 @@ __device__ __forceinline__ void expert_rows(const u16* __restrict__ x, long ldx,
   auto compute = [&](const Stage& st, int k0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (k0 + 32 * u >= K) break;
+      if (k0 + 32 * u >= K) break;      // (uniform)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
         acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, st.x[u][m]), st.w[u], acc[m], 0, 0, 0);
     }
   };
   Stage A, B;
-  load(A, kb, true);
-  load(B, kb + 32 * U, false);
+  load(A, kb, 0);
+  load(B, kb + 32 * U, U == 2 ? 2 : -1);
+  int k0 = kb;
   if constexpr (KS > 1) {      // a quarter of K is two stages or little more
-    for (int k0 = kb; k0 < K; k0 += 64 * U) {
+    for (; k0 + 64 * U < K; k0 += 64 * U) {
       compute(A, k0);
-      load(A, k0 + 64 * U, false);
+      load(A, k0 + 64 * U, -1);
       compute(B, k0 + 32 * U);
-      load(B, k0 + 96 * U, false);
+      load(B, k0 + 96 * U, -1);
     }
+    compute(A, k0);
+    compute(B, k0 + 32 * U);
   } else {
     Stage C;      // two stages ahead of the one that is multiplied
-    for (int k0 = kb; k0 < K; k0 += 96 * U) {
-      load(C, k0 + 64 * U, false);
+    load(C, k0 + 64 * U, -1);
+    for (; k0 + 96 * U < K; k0 += 96 * U) {
       compute(A, k0);
-      load(A, k0 + 96 * U, false);
+      load(A, k0 + 96 * U, -1);
       compute(B, k0 + 32 * U);
-      load(B, k0 + 128 * U, false);
+      load(B, k0 + 128 * U, -1);
       compute(C, k0 + 64 * U);
+      load(C, k0 + 160 * U, -1);
     }
+    compute(A, k0);
+    compute(B, k0 + 32 * U);
+    compute(C, k0 + 64 * U);
   }
   auto put = [&](int row, int c, float a, float u) {
     if (row >= n) return;
@@ -125,12 +137,11 @@ __global__ void __launch_bounds__(KS > 1 ? 64 * KS : 64 * MD_TILES, KS > 1 ? 4 :
   const int e = blockIdx.y, tile = KS > 1 ? blockIdx.x : blockIdx.x * MD_TILES + wave;
   if (tile * 16 >= N) return;      // (KS 1: no barrier below)
   const int kq = KS > 1 ? (K / KS + 31) & ~31 : K, kb = KS > 1 ? min(K, wave * kq) : 0, ke = min(K, kb + kq);
-  const u16* wt = w + ((long)e * (N / 16) + tile) * 16 * K;
+  const __amdgpu_buffer_rsrc_t wt = make_rsrc(w + ((long)e * (N / 16) + tile) * 16 * K, (unsigned)ke * 32);
   bf16x8 w0[4];
   auto first = [&] {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (kb + 32 * u < ke) w0[u] = __builtin_bit_cast(bf16x8, ld16(wt + kb * 16 + 512 * u + (unsigned)lane * 8));
+    for (int u = 0; u < 4; ++u) w0[u] = md_w(wt, kb + 32 * u);
   };
   // the first weights are under way while the ids come, unless most experts have no pair and would stream them for nothing (two tokens of 4
   // of 64 experts of 2048 x 1408: 74 us always ahead, 34)
