@@ -53,7 +53,7 @@ int dllm_moe_max_tiles(int, int);
 int dllm_moe_ffn(const void*, long, long, int, const int*, const float*, int, int, const void*, const void*, int, int*,
                  int*, void*, float*, void*, int, hipStream_t);
 int dllm_rms_rows(const void*, long, int, const float*, void*, long, int, int, int, float, int, hipStream_t);
-int dllm_norm_resadd(const void*, long, int, const float*, float*, void*, int, int, float, int, const float*, hipStream_t);
+int dllm_norm_resadd(const void*, long, int, const float*, float*, void*, int, int, float, int, const float*, float*, hipStream_t);
 int dllm_polynorm(const void*, long, int, const float*, void*, long, int, float, hipStream_t);
 int dllm_router_topk(const void*, long, const float*, int, int, float*, int, int, int, int, int, int, int, const float*, int, int*, float*, float*,
                      int, hipStream_t);
@@ -75,7 +75,7 @@ int dllm_mlstm(const void*, long, int, int, int, int, const float*, float, float
                const int*, const int*, const int*, int, long, float*, void*, int, hipStream_t);
 int dllm_mlstm_chunk_ok(int, long, int, int);
 int dllm_qk_norm_prep(const void*, long, int, const float*, int, int, int, int, int, const float*, const float*, const float*,
-                      int, int, float, float, const int*, const int*, void*, void*, void*, long, int, hipStream_t);
+                      int, int, float, float, const int*, const int*, void*, void*, void*, long, int, void*, int, hipStream_t);
 int dllm_diff_combine(const float*, void*, int, long, int, int, int, float, float, float, hipStream_t);
 int dllm_conv_silu(const void*, long, int, const float*, const float*, void*, const int*, const int*, const int*,
                    const int*, void*, int, int, int, int, int, int, int, hipStream_t);
@@ -109,7 +109,7 @@ int dllm_delta_rule(const void*, long, const void*, long, int, int, int, int, in
                     float, float*, const int*, const int*, const int*, const int*, float*, void*, int, long, float*, hipStream_t);
 int dllm_delta_pre(int);
 int dllm_attn_prep(const void*, long, int, int, int, int, int, const float*, int, int, float, const float*, const int*,
-                   const int*, void*, void*, void*, long, int, hipStream_t);
+                   const int*, void*, void*, void*, long, int, void*, int, hipStream_t);
 int dllm_gqa_tile_tokens(int, int, int);
 int dllm_gqa_mfma_ok(int, int, int, int, int, int);
 int dllm_paged_gqa(const void*, const void*, const void*, int, const int*, int, int, const int*, const int*, const int*,
@@ -1686,7 +1686,7 @@ void rms_rows(torch::Tensor x, c10::optional<torch::Tensor> w, torch::Tensor y, 
 }
 
 void norm_resadd(torch::Tensor y, torch::Tensor w, double eps, torch::Tensor x, c10::optional<torch::Tensor> xl,
-                 int64_t groups, c10::optional<torch::Tensor> bias) {
+                 int64_t groups, c10::optional<torch::Tensor> bias, c10::optional<torch::Tensor> xw) {
   const bool f = act_f32(y, "y");
   check_rows2d(y, "y");
   check_f32(w, "w");
@@ -1705,8 +1705,12 @@ void norm_resadd(torch::Tensor y, torch::Tensor w, double eps, torch::Tensor x, 
     TORCH_CHECK(bias->numel() == x.size(1), "bias length");
     bp = bias->data_ptr<float>();
   }
+  if (xw) {
+    check_f32(*xw, "x_wide");
+    TORCH_CHECK(xl && xw->is_contiguous() && xw->sizes() == x.sizes(), "x_wide: beside x_lp, contiguous, the shape of x");
+  }
   ok(dllm_norm_resadd(y.data_ptr(), y.stride(0), f, w.data_ptr<float>(), x.data_ptr<float>(), lp, (int)x.size(0),
-                      (int)x.size(1), (float)eps, (int)groups, bp, stream()),
+                      (int)x.size(1), (float)eps, (int)groups, bp, xw ? xw->data_ptr<float>() : nullptr, stream()),
      "norm_resadd");
 }
 
@@ -2011,9 +2015,17 @@ void delta_rule(torch::Tensor qkv, torch::Tensor gba, int64_t H, int64_t G, int6
      "delta_rule");
 }
 
+// 4-byte words of a row of an optional contiguous [T, n] buffer that a prep launch clears
+int zero_words(const c10::optional<torch::Tensor>& z, int64_t T) {
+  if (!z) return 0;
+  TORCH_CHECK(z->is_cuda() && z->is_contiguous() && z->dim() == 2 && z->size(0) == T && z->size(1) * z->element_size() % 4 == 0,
+              "zero_rows: [T, n] of whole 4-byte words, contiguous");
+  return (int)(z->size(1) * z->element_size() / 4);
+}
+
 void attn_prep(torch::Tensor proj, int64_t H, int64_t G, int64_t d, int64_t dv, torch::Tensor cos_sin, int64_t rot,
                double eps, torch::Tensor qscale, torch::Tensor pos, torch::Tensor slots, torch::Tensor kc, torch::Tensor vc,
-               torch::Tensor q) {
+               torch::Tensor q, c10::optional<torch::Tensor> zero_rows) {
   const bool f = act_f32(proj, "proj");
   check_rows2d(proj, "proj");
   check_f32(cos_sin, "cos_sin");
@@ -2033,7 +2045,8 @@ void attn_prep(torch::Tensor proj, int64_t H, int64_t G, int64_t d, int64_t dv, 
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == proj.scalar_type() && q.is_contiguous() && q.numel() == T * H * d, "q [T, H, d]");
   ok(dllm_attn_prep(proj.data_ptr(), proj.stride(0), f, (int)H, (int)G, (int)d, (int)dv, cos_sin.data_ptr<float>(),
                     (int)cos_sin.size(1), (int)rot, (float)eps, qscale.data_ptr<float>(), pos.data_ptr<int>(),
-                    slots.data_ptr<int>(), kc.data_ptr(), vc.data_ptr(), q.data_ptr(), (long)T, (int)kc.size(2), stream()),
+                    slots.data_ptr<int>(), kc.data_ptr(), vc.data_ptr(), q.data_ptr(), (long)T, (int)kc.size(2),
+                    zero_rows ? zero_rows->data_ptr() : nullptr, zero_words(zero_rows, T), stream()),
      "attn_prep");
 }
 
@@ -2312,7 +2325,7 @@ bool embed_rows(torch::Tensor ids, torch::Tensor table, double scale, torch::Ten
 void qk_norm_prep(torch::Tensor proj, c10::optional<torch::Tensor> bias, int64_t H, int64_t G, int64_t M, int64_t d, int64_t dv,
                   torch::Tensor qw, torch::Tensor kw, torch::Tensor cos_sin, int64_t rot, double eps, double qscale,
                   torch::Tensor pos, torch::Tensor slots, c10::optional<torch::Tensor> kc, c10::optional<torch::Tensor> vc,
-                  torch::Tensor q) {
+                  torch::Tensor q, c10::optional<torch::Tensor> zero_rows) {
   const bool f = act_f32(proj, "proj");
   check_rows2d(proj, "proj");
   check_f32(cos_sin, "cos_sin");
@@ -2351,7 +2364,8 @@ void qk_norm_prep(torch::Tensor proj, c10::optional<torch::Tensor> bias, int64_t
               "q [T, H M, d]");
   ok(dllm_qk_norm_prep(proj.data_ptr(), proj.stride(0), f, bp, (int)H, (int)G, (int)M, (int)d, (int)dv, qw.data_ptr<float>(),
                        kw.data_ptr<float>(), cos_sin.data_ptr<float>(), (int)cos_sin.size(1), (int)rot, (float)eps,
-                       (float)qscale, pos.data_ptr<int>(), slots.data_ptr<int>(), kp, vp, q.data_ptr(), (long)T, bsz, stream()),
+                       (float)qscale, pos.data_ptr<int>(), slots.data_ptr<int>(), kp, vp, q.data_ptr(), (long)T, bsz,
+                       zero_rows ? zero_rows->data_ptr() : nullptr, zero_words(zero_rows, T), stream()),
      "qk_norm_prep");
 }
 
@@ -2857,7 +2871,7 @@ void latent_attention(torch::Tensor qa, torch::Tensor q, int64_t dim, int64_t ro
 PYBIND11_MODULE(_hip_kernels, m) {
   m.def("rms_rows", &rms_rows, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("eps"), py::arg("groups") = 1);
   m.def("norm_resadd", &norm_resadd, py::arg("y"), py::arg("w"), py::arg("eps"), py::arg("x"), py::arg("x_lp"),
-        py::arg("groups") = 1, py::arg("bias") = py::none());
+        py::arg("groups") = 1, py::arg("bias") = py::none(), py::arg("x_wide") = py::none());
   m.def("polynorm", &polynorm);
   m.def("group_router", &group_router);
   m.def("swiglu_scale", &swiglu_scale);

@@ -64,13 +64,22 @@ __device__ __forceinline__ float cap_fast(float s, float cap, float two_over_cap
   return cap - 2.f * cap * __builtin_amdgcn_rcpf(__expf(s * two_over_cap) + 1.f);
 }
 
+// this workgroup's share of a token's row of a [T, zw] buffer of 4-byte words, cleared: the attention output of a step with padding rows,
+// which no attention tile writes (a fill of its own: 4.7 us a layer of a decode step)
+__device__ __forceinline__ void clear_row(uint32_t* zrow, int zw, long tok) {
+  if (zrow)
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < zw; i += gridDim.y * 256) zrow[tok * zw + i] = 0u;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) attn_prep_kernel(const T* __restrict__ proj, long ld, int H, int G, int d, int dv,
                                                         const float* __restrict__ cos_sin, int tab_w, int rot, float eps,
                                                         const float* __restrict__ qscale, const int* __restrict__ pos,
                                                         const int* __restrict__ slots, T* __restrict__ kc,
-                                                        T* __restrict__ vc, T* __restrict__ q, int BSZ) {
+                                                        T* __restrict__ vc, T* __restrict__ q, int BSZ, uint32_t* __restrict__ zrow,
+                                                        int zw) {
   const long tok = blockIdx.x;
+  clear_row(zrow, zw, tok);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T* r = proj + tok * ld;
   const int slot = slots[tok];
@@ -126,9 +135,11 @@ __global__ void __launch_bounds__(256) attn_prep_vec_kernel(const u16* __restric
                                                             const float* __restrict__ cos_sin, int tab_w, int rot, float eps,
                                                             const float* __restrict__ qscale, const int* __restrict__ pos,
                                                             const int* __restrict__ slots, u16* __restrict__ kc, u16* __restrict__ vc,
-                                                            u16* __restrict__ q, int BSZ, int T, int ny) {
+                                                            u16* __restrict__ q, int BSZ, int T, int ny,
+                                                            uint32_t* __restrict__ zrow, int zw) {
   constexpr int LPH = D / 8, TW = APV_T / 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = blockIdx.x * APV_T;
+  for (int t = t0; t < min(t0 + APV_T, T); ++t) clear_row(zrow, zw, t);
   if ((int)blockIdx.y < ny) {
     const int hh = (blockIdx.y * 64 + lane) / LPH, c = lane % LPH * 8, half = rot >> 1;
     const int hx = min(hh, H + G - 1), f = c < half ? c : c - half;
@@ -206,8 +217,10 @@ __global__ void __launch_bounds__(256) qk_norm_prep_kernel(const T* __restrict__
                                                            const float* __restrict__ cos_sin, int tab_w, int rot, float eps,
                                                            float qscale, const int* __restrict__ pos,
                                                            const int* __restrict__ slots, T* __restrict__ kc,
-                                                           T* __restrict__ vc, T* __restrict__ q, int BSZ) {
+                                                           T* __restrict__ vc, T* __restrict__ q, int BSZ,
+                                                           uint32_t* __restrict__ zrow, int zw) {
   const long tok = blockIdx.x;
+  clear_row(zrow, zw, tok);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const T* r = proj + tok * ld;
   const int slot = kc ? slots[tok] : -1;
@@ -1366,9 +1379,10 @@ int launch_gqa_t(int nj, dim3 grid, long lds, hipStream_t st, const void* q, con
 
 extern "C" int dllm_attn_prep(const void* proj, long ld, int f32, int H, int G, int d, int dv, const float* cos_sin,
                               int tab_w, int rot, float eps, const float* qscale, const int* pos, const int* slots, void* kc,
-                              void* vc, void* q, long T, int BSZ, hipStream_t st) {
+                              void* vc, void* q, long T, int BSZ, void* zero_rows, int zw, hipStream_t st) {
   if (T <= 0) return 0;
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w) return -1;
+  uint32_t* const z = (uint32_t*)zero_rows;
   // whole vectors: heads of 32 to 256, halves of the rotation and values in eights, 16-byte aligned rows; and enough of them: 16 tokens a
   // workgroup leave few steps' worth of waves, of which each waits for all its loads (element by element / here, us, heads + key heads
   // x width: 40 x 64, 6 tokens 3.2 / 4.0, 64 3.8 / 5.8, 192 5.4 / 5.9, 256 6.3 / 6.0; 20 x 64, 384 5.4 / 5.9, 512 6.4 / 6.0; 5 x 256, 700 6.0 / 6.3,
@@ -1379,7 +1393,7 @@ extern "C" int dllm_attn_prep(const void* proj, long ld, int f32, int H, int G, 
     const dim3 g(((unsigned)T + APV_T - 1) / APV_T, ny + (G * dv + APV_V - 1) / APV_V);
 #define APV(D)                                                                                                                     \
   hipLaunchKernelGGL(attn_prep_vec_kernel<D>, g, dim3(256), 0, st, (const u16*)proj, ld, H, G, dv, cos_sin, tab_w, rot, eps, qscale, pos, \
-                     slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ, (int)T, ny)
+                     slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ, (int)T, ny, z, zw)
     if (d == 32) APV(32);
     else if (d == 64) APV(64);
     else if (d == 128) APV(128);
@@ -1390,10 +1404,10 @@ extern "C" int dllm_attn_prep(const void* proj, long ld, int f32, int H, int G, 
   const dim3 grid((unsigned)T, (H + G + 3) / 4);
   if (f32)
     hipLaunchKernelGGL(attn_prep_kernel<float>, grid, dim3(256), 0, st, (const float*)proj, ld, H, G, d, dv, cos_sin, tab_w, rot,
-                       eps, qscale, pos, slots, (float*)kc, (float*)vc, (float*)q, BSZ);
+                       eps, qscale, pos, slots, (float*)kc, (float*)vc, (float*)q, BSZ, z, zw);
   else
     hipLaunchKernelGGL(attn_prep_kernel<u16>, grid, dim3(256), 0, st, (const u16*)proj, ld, H, G, d, dv, cos_sin, tab_w, rot, eps,
-                       qscale, pos, slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ);
+                       qscale, pos, slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ, z, zw);
   return (int)hipGetLastError();
 }
 
@@ -1520,17 +1534,17 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
 extern "C" int dllm_qk_norm_prep(const void* proj, long ld, int f32, const float* bias, int H, int G, int M, int d, int dv,
                                  const float* qw, const float* kw, const float* cos_sin, int tab_w, int rot, float eps,
                                  float qscale, const int* pos, const int* slots, void* kc, void* vc, void* q, long T, int BSZ,
-                                 hipStream_t st) {
+                                 void* zero_rows, int zw, hipStream_t st) {
   if (T <= 0) return 0;
   if (rot < 0 || rot > d || (rot & 1) || rot > tab_w || H < 1 || G < 1 || H % G || M < 1) return -1;
   const int units = H * M + (kc ? G * M : 0);
   const dim3 grid((unsigned)T, (units + 3) / 4);
   if (f32)
     hipLaunchKernelGGL(qk_norm_prep_kernel<float>, grid, dim3(256), 0, st, (const float*)proj, ld, bias, H, G, M, d, dv, qw, kw,
-                       cos_sin, tab_w, rot, eps, qscale, pos, slots, (float*)kc, (float*)vc, (float*)q, BSZ);
+                       cos_sin, tab_w, rot, eps, qscale, pos, slots, (float*)kc, (float*)vc, (float*)q, BSZ, (uint32_t*)zero_rows, zw);
   else
     hipLaunchKernelGGL(qk_norm_prep_kernel<u16>, grid, dim3(256), 0, st, (const u16*)proj, ld, bias, H, G, M, d, dv, qw, kw,
-                       cos_sin, tab_w, rot, eps, qscale, pos, slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ);
+                       cos_sin, tab_w, rot, eps, qscale, pos, slots, (u16*)kc, (u16*)vc, (u16*)q, BSZ, (uint32_t*)zero_rows, zw);
   return (int)hipGetLastError();
 }
 

@@ -101,10 +101,18 @@ __global__ void __launch_bounds__(256) rms_rows_reg_kernel(const TI* __restrict_
 }
 
 // ---------------------------------------------------------------- norm_resadd
+// an entry of the rounded stream, and of its widened copy
+template <typename T>
+__device__ __forceinline__ void put_lp(T* xl, float* xw, long i, float v) {
+  if (!xl) return;
+  stf(xl + i, v);
+  if (xw) xw[i] = sizeof(T) == 2 ? bf2f(f2bf(v)) : v;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ y, long ldy, const float* __restrict__ w,
                                                           float* __restrict__ x, T* __restrict__ xl, int H, float eps,
-                                                          int groups, const float* __restrict__ bias) {
+                                                          int groups, const float* __restrict__ bias, float* __restrict__ xw) {
   __shared__ float red[16];
   const long row = blockIdx.x;
   const T* yr = y + row * ldy;
@@ -119,7 +127,7 @@ __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ 
       for (int i = lane; i < n; i += 64) {
         const float v = xr[c0 + i] + (ldf(yr + c0 + i) + (bias ? bias[c0 + i] : 0.f)) * r * w[c0 + i];
         xr[c0 + i] = v;
-        if (xl) stf(xl + row * (long)H + c0 + i, v);
+        put_lp(xl, xw, row * (long)H + c0 + i, v);
       }
     }
     return;
@@ -130,7 +138,7 @@ __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ 
   for (int i = threadIdx.x; i < H; i += 256) {
     const float v = xr[i] + (ldf(yr + i) + (bias ? bias[i] : 0.f)) * r * w[i];
     xr[i] = v;
-    if (xl) stf(xl + row * (long)H + i, v);
+    put_lp(xl, xw, row * (long)H + i, v);
   }
 }
 
@@ -143,7 +151,8 @@ template <typename T, typename TY, int NE, bool PARTS>
 __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restrict__ y, long ldy, const float* __restrict__ w,
                                                               float* __restrict__ x, T* __restrict__ xl, int H, float eps,
                                                               int groups, const float* __restrict__ bias,
-                                                              const int* __restrict__ inv, const float* __restrict__ wts, int k) {
+                                                              const int* __restrict__ inv, const float* __restrict__ wts, int k,
+                                                              float* __restrict__ xw) {
   __shared__ float red[4];
   constexpr bool EARLY = NE <= 16;     // the stream and the weights in flight with the row, where the registers allow
   constexpr int ST = PARTS ? 64 : 256;
@@ -203,7 +212,7 @@ __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restri
       if (c >= c1) continue;
       const float v = (EARLY ? s[EARLY ? j : 0] : xr[c]) + a[j] * r * (EARLY ? g[EARLY ? j : 0] : w[c]);
       xr[c] = v;
-      if (xl) stf(xl + row * (long)H + c, v);
+      put_lp(xl, xw, row * (long)H + c, v);
     }
     if constexpr (!PARTS) break;
   }
@@ -1598,11 +1607,11 @@ int norm_resadd_entries(int H, int groups) {
 }
 template <typename T, typename TY>
 int norm_resadd_reg(const void* y, long ldy, const float* w, float* x, void* xl, long rows, int H, float eps, int groups,
-                    const float* bias, const int* inv, const float* wts, int k, hipStream_t st) {
+                    const float* bias, const int* inv, const float* wts, int k, hipStream_t st, float* xw = nullptr) {
   const int e = norm_resadd_entries(H, groups);
 #define NRV(NE, PARTS)                                                                                                                   \
   hipLaunchKernelGGL((norm_resadd_reg_kernel<T, TY, NE, PARTS>), dim3((unsigned)rows), dim3(256), 0, st, (const TY*)y, ldy, w, x, (T*)xl, H, \
-                     eps, groups, bias, inv, wts, k)
+                     eps, groups, bias, inv, wts, k, xw)
   if (groups == 1) {
     if (e <= 4) NRV(4, false); else if (e <= 8) NRV(8, false); else if (e <= 16) NRV(16, false); else NRV(32, false);
   } else {
@@ -1627,19 +1636,20 @@ extern "C" int dllm_moe_norm_resadd(const void* y, int f32, const int* inv, cons
              : norm_resadd_reg<u16, u16>(y, H, w, x, xl, T, H, eps, groups, nullptr, inv, wts, k, st);
 }
 
+// xw (with xl): the rounded stream again, as f32
 extern "C" int dllm_norm_resadd(const void* y, long ldy, int f32, const float* w, float* x, void* xl, int rows, int H,
-                                float eps, int groups, const float* bias, hipStream_t st) {
+                                float eps, int groups, const float* bias, float* xw, hipStream_t st) {
   if (rows <= 0) return rows == 0 ? 0 : -1;
   if (groups < 1 || H % groups) return -1;
   // f32 rows of 8192 (parts of 2048) hold 32 entries a thread, and many of them stream better in two passes of more waves: 4000 x 8192
   // 151 us in registers, 126 in two passes; 300 rows 11.9, 15.4
   const int e = norm_resadd_entries(H, groups);
   if (e && !(f32 && e > 16 && rows > 1024))
-    return f32 ? norm_resadd_reg<float, float>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st)
-               : norm_resadd_reg<u16, u16>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st);
+    return f32 ? norm_resadd_reg<float, float>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st, xw)
+               : norm_resadd_reg<u16, u16>(y, ldy, w, x, xl, rows, H, eps, groups, bias, nullptr, nullptr, 0, st, xw);
   BY_T(f32,
-       hipLaunchKernelGGL(norm_resadd_kernel<u16>, dim3(rows), dim3(256), 0, st, (const u16*)y, ldy, w, x, (u16*)xl, H, eps, groups, bias),
-       hipLaunchKernelGGL(norm_resadd_kernel<float>, dim3(rows), dim3(256), 0, st, (const float*)y, ldy, w, x, (float*)xl, H, eps, groups, bias))
+       hipLaunchKernelGGL(norm_resadd_kernel<u16>, dim3(rows), dim3(256), 0, st, (const u16*)y, ldy, w, x, (u16*)xl, H, eps, groups, bias, xw),
+       hipLaunchKernelGGL(norm_resadd_kernel<float>, dim3(rows), dim3(256), 0, st, (const float*)y, ldy, w, x, (float*)xl, H, eps, groups, bias, xw))
   return (int)hipGetLastError();
 }
 

@@ -836,14 +836,16 @@ class HybridModel:
         nl = self._left_cols(a)
         rot = a.rot.dims if a.rot is not None else 0
         table = self._table(a) if rot else self._any_table()
+        all_rows = self._all_rows(x, meta)      # else the prep launch clears the attention output's padding rows
+        out = self._cleared_in_prep(all_rows, x.shape[0], a.heads * a.vdim, x.dtype)
         q = seqmix.attn_prep(proj, a.heads, a.kv_heads, a.dim, a.vdim, table, rot, eps, L["qscale"], positions,
-                             meta.slots, k_cache, v_cache)
+                             meta.slots, k_cache, v_cache, out)
         mfma = seqmix.gqa_use_mfma(q, a.heads, a.kv_heads, a.dim, a.vdim, k_cache.shape[2])
         ts, tt = meta.latent_tiles(1, self.device, seqmix.gqa_tokens_per_tile(a.heads, a.kv_heads, mfma))
         gate = proj[:, nl - a.heads * a.vdim:nl]
         splits = seqmix.gqa_splits(int(ts.numel()), a.kv_heads, meta.max_ctx) if mfma else 1
         lo = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
-                                        gate, mfma, splits)
+                                        gate, mfma, splits, all_rows=all_rows, out=out)
         ro = seqmix.lightning_attention(proj[:, nl:], b.heads, b.dim, b.vdim, L["decay"], state, eps, L["rnorm"],
                                         meta.qstart, meta.qlen, meta.ctx, meta.state_rows, longest=self._longest(meta))
         return _pm(lo, L, "lo"), _pm(ro, L, "ro")
@@ -856,15 +858,17 @@ class HybridModel:
         proj = _pm(x, L, "proj")
         rot = m.rot.dims if m.rot is not None else 0
         table = self._table(m) if rot else self._any_table()
+        all_rows = self._all_rows(x, meta)
+        out = self._cleared_in_prep(all_rows, x.shape[0], 2 * m.heads * m.vdim, torch.float32)
         q = seqmix.qk_norm_prep(proj, L["bias"], m.heads, m.kv_heads, 2, m.dim, m.vdim, L["qnorm"], L["knorm"], table, rot,
                                 self.cfg.rms_eps, m.scale, positions, meta.slots, k_cache if own else None,
-                                v_cache if own else None)
+                                v_cache if own else None, out)
         H2, G2 = 2 * m.heads, 2 * m.kv_heads
         mfma = seqmix.gqa_use_mfma(q, H2, G2, m.dim, m.vdim, k_cache.shape[2])
         ts, tt = meta.latent_tiles(1, self.device, seqmix.gqa_tokens_per_tile(H2, G2, mfma))
         splits = seqmix.gqa_splits(int(ts.numel()), G2, meta.max_ctx, m.window) if mfma else 1
         a = seqmix.paged_gqa_attention(q, k_cache, v_cache, meta.block_tables, meta.qstart, meta.qlen, meta.ctx, ts, tt,
-                                       None, mfma, splits, window=m.window, out_f32=True)
+                                       None, mfma, splits, window=m.window, out_f32=True, all_rows=all_rows, out=out)
         o = seqmix.diff_combine(a, m.heads, m.kv_heads, m.vdim, L["lam"], self.cfg.rms_eps, 1.0 - m.diff, self.dtype)
         return _pm(o, L, "o")
 
@@ -1018,6 +1022,12 @@ class HybridModel:
         """A step of prompt portions whose sequences cover every packed row (no padding rows)."""
         return meta.host_qlen is not None and sum(int(n) for n in meta.host_qlen) == x.shape[0]
 
+    def _cleared_in_prep(self, all_rows: bool, rows: int, cols: int, dtype) -> Optional[torch.Tensor]:
+        """An attention output for the launch before it to clear; None where nothing needs clearing, or its rows are not whole words."""
+        if all_rows or cols * dtype.itemsize % 4:
+            return None
+        return torch.empty((rows, cols), dtype=dtype, device=self.device)
+
     def _mamba2(self, L, m: MixerSpec, x, meta, cache):
         conv_state, state = cache
         rows = meta.state_rows
@@ -1060,13 +1070,14 @@ class HybridModel:
                 a = seqmix.gelu_erf(z) if act[0] == "gelu" else seqmix.glu_act(z, L.get("up_b"), *act)
         return _pm(a, L, "down")
 
-    def _experts_swiglu(self, L, f: MoESpec, x, tail=None):
+    def _experts_swiglu(self, L, f: MoESpec, x, tail=None, wide=None):
         """Sigmoid router in f32 with group-limited top-k, weights = the chosen scores; SwiGLU experts
         on the grouped MFMA kernels, or in the dense form (all experts' columns in two GEMMs, unused
         experts gated to zero) for f32 models and widths the grouped kernels do not take.  The logits are the
-        vendor's f32 product: ``seqmix.router_topk`` sums in another order (16 rows 6 us instead of 14), and the mLSTM
+        vendor's f32 product (of ``wide``, x in f32, where the launch before has written that):
+        ``seqmix.router_topk`` sums in another order (16 rows 6 us instead of 14), and the mLSTM
         layers of these models turn the last bit of a weight into tenths of a logit."""
-        logits = F.linear(x.float(), L["router"])
+        logits = F.linear(x.float() if wide is None else wide, L["router"])
         ids, w = seqmix.group_router(logits, f.top, f.group_count, f.group_keep)
         if f.scale != 1.0:
             w = w * f.scale
@@ -1102,11 +1113,11 @@ class HybridModel:
         a = seqmix.swiglu_scale(_mm(x, L["w1"].view(f.experts * 2 * f.ff, -1)), g, f.ff)
         return _pm(a, L, "w2d")
 
-    def _experts(self, L, f: MoESpec, x, tail=None):
+    def _experts(self, L, f: MoESpec, x, tail=None, wide=None):
         """``tail`` (ops.moe_ffn_tg): where the experts run on the grouped GEMM, their sum ends in the stream and None is
         returned; elsewhere the caller adds what is returned."""
         if f.act == "swiglu":
-            return self._experts_swiglu(L, f, x, tail)
+            return self._experts_swiglu(L, f, x, tail, wide)
         if "shared_in" in L:
             ids, w = ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
             return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], tail, L.get("experts_r"))
@@ -1226,11 +1237,12 @@ class HybridModel:
                     seqmix.resadd_norm(a, post, eps, x, nxt, h, bias=bias, **pair)
             else:
                 ng = cfg.norm_groups
-                seqmix.norm_resadd(y, L["norm1"], eps, x, xl, groups=ng, bias=L.get("ob"))
+                xw = torch.empty_like(x) if xl is not None and isinstance(S.mlp, MoESpec) and S.mlp.act == "swiglu" else None
+                seqmix.norm_resadd(y, L["norm1"], eps, x, xl, groups=ng, bias=L.get("ob"), x_wide=xw)
                 if S.mlp is not None:
                     hin = x if xl is None else xl
                     y = self._dense(L, S.mlp, hin) if isinstance(S.mlp, DenseSpec) else \
-                        self._experts(L, S.mlp, hin, (L["norm2"], eps, x, xl, ng))
+                        self._experts(L, S.mlp, hin, (L["norm2"], eps, x, xl, ng), xw)
                     if y is not None:
                         seqmix.norm_resadd(y, L["norm2"], eps, x, xl, groups=ng)
                 if X is not None:

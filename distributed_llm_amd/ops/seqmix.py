@@ -48,14 +48,20 @@ def rms_rows(x: torch.Tensor, w: Optional[torch.Tensor], eps: float, out_dtype=N
 
 
 def norm_resadd(y: torch.Tensor, w: torch.Tensor, eps: float, x: torch.Tensor,
-                x_lp: Optional[torch.Tensor] = None, groups: int = 1, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+                x_lp: Optional[torch.Tensor] = None, groups: int = 1, bias: Optional[torch.Tensor] = None,
+                x_wide: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Residual update in f32: ``x += rmsnorm(y) * w`` in place (x f32 [T, H]); ``x_lp`` (the model
     dtype) receives the rounded stream for the next projections, in the same launch.  ``groups`` as
-    in ``rms_rows``; ``bias`` (the sublayer's output bias) is added to y before the norm."""
+    in ``rms_rows``; ``bias`` (the sublayer's output bias) is added to y before the norm.
+    ``x_wide`` (f32, beside ``x_lp``): the rounded stream widened again, for a router that multiplies in f32 (its copy
+    was a launch of its own: 5 us a layer of a decode step)."""
     ext = _native(y)
     if ext is None:
-        return ref.norm_resadd(y, w, eps, x, x_lp, groups, bias)
-    ext.norm_resadd(y, w, float(eps), x, x_lp, int(groups), bias)
+        ref.norm_resadd(y, w, eps, x, x_lp, groups, bias)
+        if x_wide is not None:
+            x_wide.copy_(x_lp)
+        return x
+    ext.norm_resadd(y, w, float(eps), x, x_lp, int(groups), bias, x_wide)
     return x
 
 
@@ -386,17 +392,20 @@ def gqa_tokens_per_tile(heads: int, kv_heads: int, mfma: bool = False) -> int:
 
 
 def attn_prep(proj, heads, kv_heads, dim, vdim, cos_sin, rot_dims, eps, qscale, positions, slots, k_cache,
-              v_cache) -> torch.Tensor:
+              v_cache, zero_rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Rotate q and k (rotate-half, first ``rot_dims`` dims), bring every head to unit RMS, scale q
     per head, write k and v to their page slots (k_cache [blocks, kv_heads, block, dim], v_cache
-    [blocks, kv_heads, vdim, block]); returns q [T, heads, dim]."""
+    [blocks, kv_heads, vdim, block]); returns q [T, heads, dim].  ``zero_rows`` [T, n] (whole 4-byte words a row) is
+    cleared in the same launch: the attention output of a step with padding rows."""
     ext = _native(proj)
     if ext is None:
+        if zero_rows is not None:
+            zero_rows.zero_()
         return ref.attn_prep(proj, heads, kv_heads, dim, vdim, cos_sin, rot_dims, eps, qscale, positions, slots,
                              k_cache, v_cache)
     q = torch.empty((proj.shape[0], heads, dim), dtype=proj.dtype, device=proj.device)     # every row is written
     ext.attn_prep(proj, int(heads), int(kv_heads), int(dim), int(vdim), cos_sin, int(rot_dims), float(eps), qscale,
-                  positions, slots, k_cache, v_cache, q)
+                  positions, slots, k_cache, v_cache, q, zero_rows)
     return q
 
 
@@ -460,21 +469,23 @@ def paged_gqa_attention(q, k_cache, v_cache, block_tables, qstart, qlen, ctx, ti
 # ----------------------------------------------------------------------------- differential attention
 
 def qk_norm_prep(proj, bias, heads, kv_heads, maps, dim, vdim, qnorm_w, knorm_w, cos_sin, rot_dims, eps, qscale,
-                 positions, slots, k_cache, v_cache) -> torch.Tensor:
+                 positions, slots, k_cache, v_cache, zero_rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Attention inputs with a weighted RMS norm of every q / k vector BEFORE its rotation, biases,
     and ``maps`` score maps per head (differential attention: 2).  proj [T, q | k | v] (+ ``bias``
     f32 over the same columns); returns q [T, heads maps, dim], scaled by ``qscale``, the query rows
     of one key/value head ordered (map, head in group), so that the grouped-query kernels pair row r
     with key row r // (heads / kv_heads) of k_cache [blocks, kv_heads maps, block, dim].  v goes to
     v_cache [blocks, kv_heads, vdim, block].  ``k_cache`` None (a layer that reads another layer's
-    keys and values): proj holds q alone."""
+    keys and values): proj holds q alone.  ``zero_rows``: as in ``attn_prep``."""
     ext = _native(proj)
     if ext is None:
+        if zero_rows is not None:
+            zero_rows.zero_()
         return ref.qk_norm_prep(proj, bias, heads, kv_heads, maps, dim, vdim, qnorm_w, knorm_w, cos_sin, rot_dims, eps,
                                 qscale, positions, slots, k_cache, v_cache)
     q = torch.empty((proj.shape[0], heads * maps, dim), dtype=proj.dtype, device=proj.device)     # every row is written
     ext.qk_norm_prep(proj, bias, int(heads), int(kv_heads), int(maps), int(dim), int(vdim), qnorm_w, knorm_w, cos_sin,
-                     int(rot_dims), float(eps), float(qscale), positions, slots, k_cache, v_cache, q)
+                     int(rot_dims), float(eps), float(qscale), positions, slots, k_cache, v_cache, q, zero_rows)
     return q
 
 
