@@ -131,6 +131,12 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
 // the launch and the exchange; the LDS-tiled GEMM adds a ring's fill and, for long K, a split's exchange through memory: 16 rows,
 // 384 -> 1152 / 384 -> 384 / 384 -> 1536 / 1536 -> 384 columns 2.9 / 3.5 / 3.5 / 5.4 us against 5.4 / 5.6 / 7.7 / 9.4.
 enum { ENC_PLAIN = 0, ENC_RESADD = 1, ENC_QKV = 2, ENC_GELU = 4 };
+
+// Loads of values that are used behind conditions, waited for at once: left to itself the compiler moves each to its use, and each then
+// has a latency of its own (in a layer of 16 rows, us: attention and output 6.1 -> 5.2, the two products of rows 6.0 -> 4.9 and 5.3 -> 4.5, down 5.6 -> 5.4)
+template <typename F>
+__device__ __forceinline__ void arrived(F& f) { asm volatile("" : "+v"(f)); }
+
 template <int MT, int NW, int EPI>
 __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict__ X, long ldx, const u16* __restrict__ W,
                                                            const u16* __restrict__ bias, u16* __restrict__ Y, long ldy, int M, int N,
@@ -144,6 +150,10 @@ __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict
   const u16* xr[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) xr[m] = X + (long)min(16 * m + lr, M - 1) * ldx + 8 * g;   // rows past M repeat the last and are dropped
+  const int row = threadIdx.x >> 2, c = 4 * (threadIdx.x & 3);     // this thread's outputs below: 64 rows a pass
+  const u16x4 b = *reinterpret_cast<const u16x4*>(bias + col0 + c);
+  u16x4 r = {};
+  if (EPI == ENC_RESADD) r = *reinterpret_cast<const u16x4*>(Y + (long)min(row, M - 1) * ldy + col0 + c);
   f32x4 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -158,14 +168,17 @@ __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict
     }
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
+      arrived(wf[u]);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) arrived(xf[u][m]);
+    }
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
       if (s + u >= s1) break;
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[u][m], wf[u], acc[m], 0, 0, 0);
     }
   }
-  const int row = threadIdx.x >> 2, c = 4 * (threadIdx.x & 3);     // this thread's outputs below: 64 rows a pass
-  u16x4 r = {}, b = *reinterpret_cast<const u16x4*>(bias + col0 + c);
-  if (EPI == ENC_RESADD && row < M) r = *reinterpret_cast<const u16x4*>(Y + (long)row * ldy + col0 + c);
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -216,13 +229,16 @@ struct FewW {
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < 3; ++u)
+    for (int u = 0; u < 3; ++u) {
+      bf16x8 x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int s = j * per + u;
-        if (u < per && s < steps)
-          acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a + 32 * s)), f[j][u], acc[j], 0, 0, 0);
-      }
+      for (int j = 0; j < 4; ++j) x[j] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a + 32 * min(j * per + u, steps - 1)));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) arrived(x[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (u < per && j * per + u < steps) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[j], f[j][u], acc[j], 0, 0, 0);
+    }
     return ((acc[0] + acc[1]) + acc[2]) + acc[3];
   }
 };
@@ -309,11 +325,7 @@ __global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __r
     const uint2 x = *reinterpret_cast<const uint2*>(Vt + (long)(w * D + 16 * n + lr) * FEW_M + 4 * g);
     vf[n] = __builtin_bit_cast(bf16x8, make_uint4(x.x, x.y, 0, 0));
   }
-  int ts = 0, tn = 0;                  // text `lane`: first row, rows
-  if (lane < B) {
-    ts = min(max(starts[lane], 0), M);
-    tn = min(min(max(lens[lane], 0), Smax), M - ts);
-  }
+  int ts = starts[min(lane, B - 1)], tn = lens[min(lane, B - 1)];
   FewW wf;
   float b = 0.f, r[4] = {};
   if (w == 0) {
@@ -322,6 +334,10 @@ __global__ void __launch_bounds__(64 * FEW_K / D) attn_out_kernel(const u16* __r
 #pragma unroll
     for (int i = 0; i < 4; ++i) r[i] = bf2f(Y[(long)min(4 * g + i, M - 1) * H + col0 + lr]);
   }
+  arrived(ts);
+  arrived(tn);
+  ts = lane < B ? min(max(ts, 0), M) : 0;      // text `lane`: first row, rows
+  tn = lane < B ? min(min(max(tn, 0), Smax), M - ts) : 0;
   int q0 = 0, q1 = 0;                  // the keys of this lane's query
   for (int t = 0; t < B; ++t) {
     const int a = __builtin_amdgcn_readlane(ts, t), e = a + __builtin_amdgcn_readlane(tn, t);
