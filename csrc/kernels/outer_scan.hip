@@ -206,20 +206,40 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const float* __rest
   if (u >= units) return;
   const long tok = u / H;
   const int h = (int)(u % H);
+  // up to 256 columns stay in registers, and all that is read is under way at once (columns past the row read its last): in passes, each
+  // with its loads, every one was a trip to memory (one token of 8 heads 5.2 -> 3.6 us)
+  constexpr int NR = 4;
+  const float* r = raw + u * dv;
+  const T* gr = gate + tok * ldg + (long)h * dv;
+  const float* wr = w + h * dv;
+  float x[NR], wt[NR];
+  T gt[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) {
+    const int i = min(lane + 64 * j, dv - 1);
+    x[j] = r[i];
+    gt[j] = gr[i];
+    wt[j] = wr[i];
+  }
   bool live = false;
   for (int s = lane; s < S; s += 64) live |= tok >= qstart[s] && tok < qstart[s] + qlen[s];
   if (!__any(live)) {
     for (int i = lane; i < dv; i += 64) stf(out + u * dv + i, 0.f);
     return;
   }
-  const float* r = raw + u * dv;
-  float s = 0.f;
-  for (int i = lane; i < dv; i += 64) s += r[i] * r[i];
-  const float sc = 1.f / sqrtf(wave_sum(s) / (float)dv + eps);
-  for (int i = lane; i < dv; i += 64) {
-    const float g = ldf(gate + tok * ldg + (long)h * dv + i);
-    stf(out + u * dv + i, r[i] * sc * w[h * dv + i] / (1.f + expf(-g)));
+  float s = 0.f, g[NR];
+#pragma unroll
+  for (int j = 0; j < NR; ++j) {
+    g[j] = ldf(&gt[j]);
+    asm volatile("" : "+v"(x[j]), "+v"(g[j]), "+v"(wt[j]));
+    if (lane + 64 * j < dv) s += x[j] * x[j];
   }
+  for (int i = lane + 64 * NR; i < dv; i += 64) s += r[i] * r[i];
+  const float sc = 1.f / sqrtf(wave_sum(s) / (float)dv + eps);
+#pragma unroll
+  for (int j = 0; j < NR; ++j)
+    if (lane + 64 * j < dv) stf(out + u * dv + lane + 64 * j, x[j] * sc * wt[j] / (1.f + expf(-g[j])));
+  for (int i = lane + 64 * NR; i < dv; i += 64) stf(out + u * dv + i, r[i] * sc * wr[i] / (1.f + expf(-ldf(gr + i))));
 }
 
 constexpr int OS_NPT[] = {1, 2, 3, 4, 5, 6, 8, 9, 10, 12, 16, 20, 24, 32};   // instantiated rows per thread

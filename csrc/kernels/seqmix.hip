@@ -303,7 +303,11 @@ template <> struct vec4<u16> {
 // resadd_norm for rows of whole 4-entry vectors, NV vectors a thread: the row stays in registers, and the slots of a
 // sum over depth are read four vectors ahead.  Bound by memory: n slots are n
 // rows of f32 a token in and two out.  8k tokens of width 2048, the 18 launches of 12 layers whose sums take 2 to 13
-// slots (7.4 GB, 1.4 ms at 5.2 TB/s): 3.8 ms entry by entry, 1.7 ms here.
+// slots (7.4 GB, 1.4 ms at 5.2 TB/s): 3.8 ms entry by entry, 1.7 ms here.  A decode step's rows are bound by latency: every weight is under way
+// with the row (and held by `here`: the compiler moves a load to its use behind the sums, a trip to memory of
+// its own; one row of 1024 4.2 -> 3.6 us).
+__device__ __forceinline__ void here(float4& f) { asm volatile("" : "+v"(f.x), "+v"(f.y), "+v"(f.z), "+v"(f.w)); }
+
 template <typename T, int NV, bool TWO, bool DEPTH>
 __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restrict__ a, long lda, const T* __restrict__ b, long ldb,
                                                               const float* __restrict__ wa, const float* __restrict__ wb,
@@ -314,21 +318,50 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
   __shared__ float red[16];
   const long row = blockIdx.x;
   float* xr = x + row * (long)H;
-  float4 y[NV], v[NV], z[TWO ? NV : 1];
+  constexpr bool EARLY = NV <= 2;      // (longer rows are many registers: 4 vectors 148 with two branches)
+  constexpr int NE = EARLY ? NV : 1, NG = EARLY && TWO ? NV : 1;
+  float4 y[NV], v[NV], z[TWO ? NV : 1], wp[NE], wn[NE], ga[NG], gb[NG], bi[NE];
+  auto weight = [](const float4* early, const float* w, int j, int c) { return EARLY ? early[j] : *reinterpret_cast<const float4*>(w + c); };
   float ss = 0.f, sb = 0.f;
+  const float* const wnx = w_next ? w_next : w_post;
+  const float* const bip = bias ? bias : w_post;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {      // (a vector past the row reads the first and is zero)
+    const int c0 = 4 * (j * 256 + (int)threadIdx.x), c = c0 < H ? c0 : 0;
+    y[j] = vec4<T>::ld(a + row * lda + c);
+    if constexpr (TWO) z[j] = vec4<T>::ld(b + row * ldb + c);
+    v[j] = *reinterpret_cast<const float4*>(xr + c);
+    if constexpr (EARLY) {
+      bi[j] = *reinterpret_cast<const float4*>(bip + c);
+      wp[j] = *reinterpret_cast<const float4*>(w_post + c);
+      wn[j] = *reinterpret_cast<const float4*>(wnx + c);
+      if constexpr (TWO) {
+        ga[j] = *reinterpret_cast<const float4*>(wa + c);
+        gb[j] = *reinterpret_cast<const float4*>(wb + c);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    here(y[j]);
+    here(v[j]);
+    if constexpr (TWO) here(z[j]);
+    if constexpr (EARLY) {
+      here(bi[j]);
+      here(wp[j]);
+      here(wn[j]);
+      if constexpr (TWO) { here(ga[j]); here(gb[j]); }
+    }
+  }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int c = 4 * (j * 256 + (int)threadIdx.x);
-    y[j] = v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if constexpr (TWO) z[j] = y[j];
-    if (c < H) {
-      y[j] = vec4<T>::ld(a + row * lda + c);
-      if constexpr (TWO) z[j] = vec4<T>::ld(b + row * ldb + c);
-      v[j] = *reinterpret_cast<const float4*>(xr + c);     // in flight under the first sum
-      if (!TWO && bias) {
-        const float4 g = *reinterpret_cast<const float4*>(bias + c);
-        y[j].x += g.x; y[j].y += g.y; y[j].z += g.z; y[j].w += g.w;
-      }
+    if (c >= H) {
+      y[j] = v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if constexpr (TWO) z[j] = y[j];
+    } else if (!TWO && bias) {
+      const float4 g = weight(bi, bip, j, c);
+      y[j].x += g.x; y[j].y += g.y; y[j].z += g.z; y[j].w += g.w;
     }
     ss += y[j].x * y[j].x + y[j].y * y[j].y + y[j].z * y[j].z + y[j].w * y[j].w;
     if constexpr (TWO) sb += z[j].x * z[j].x + z[j].y * z[j].y + z[j].z * z[j].z + z[j].w * z[j].w;
@@ -341,11 +374,11 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
     for (int j = 0; j < NV; ++j) {
       const int c = 4 * (j * 256 + (int)threadIdx.x);
       if (c < H) {
-        const float4 g = *reinterpret_cast<const float4*>(wa + c), h = *reinterpret_cast<const float4*>(wb + c);
+        const float4 g = weight(ga, wa, j, c), h = weight(gb, wb, j, c);
         y[j] = make_float4(y[j].x * ra * g.x + z[j].x * rb * h.x, y[j].y * ra * g.y + z[j].y * rb * h.y,
                            y[j].z * ra * g.z + z[j].z * rb * h.z, y[j].w * ra * g.w + z[j].w * rb * h.w);
         if (bias) {
-          const float4 e = *reinterpret_cast<const float4*>(bias + c);
+          const float4 e = weight(bi, bip, j, c);
           y[j].x += e.x; y[j].y += e.y; y[j].z += e.z; y[j].w += e.w;
         }
       }
@@ -358,7 +391,7 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
   for (int j = 0; j < NV; ++j) {
     const int c = 4 * (j * 256 + (int)threadIdx.x);
     if (c < H) {
-      const float4 g = *reinterpret_cast<const float4*>(w_post + c);
+      const float4 g = weight(wp, w_post, j, c);
       v[j].x += y[j].x * ry * g.x; v[j].y += y[j].y * ry * g.y; v[j].z += y[j].z * ry * g.z; v[j].w += y[j].w * ry * g.w;
       *reinterpret_cast<float4*>(xr + c) = v[j];
       if constexpr (DEPTH) {     // the layer's weighted sum over slots 0 .. dn - 1 of the stack, the last of them being this row
@@ -388,7 +421,7 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
   for (int j = 0; j < NV; ++j) {
     const int c = 4 * (j * 256 + (int)threadIdx.x);
     if (c < H) {
-      const float4 g = *reinterpret_cast<const float4*>(w_next + c);
+      const float4 g = weight(wn, wnx, j, c);
       vec4<T>::st(xn + row * (long)H + c, make_float4(v[j].x * rx * g.x, v[j].y * rx * g.y, v[j].z * rx * g.z, v[j].w * rx * g.w));
     }
   }
