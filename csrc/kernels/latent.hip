@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(256) latent_kv_write_kernel(const T* __restric
     wt[j] = g[i];
   }
   const int half = rot >> 1;
-  const float* cs = cos_sin + (long)pos[t] * tab_w;
+  const float* cs = cos_sin + (slot >= 0 ? (long)pos[t] * tab_w : 0);      // (a padding token's position is nobody's)
   const float turned = !is_q && lane < rot ? rotated(r + rank, lane, half, hf, cs) : 0.f;
 #pragma unroll
   for (int j = 0; j < NR; ++j) {

@@ -59,3 +59,23 @@ def test_norm_resadd_widens(T, H, groups, dtype):
     got, lp2, wide = x.clone(), torch.empty_like(lp), torch.empty_like(x)
     seqmix.norm_resadd(y, w, 1e-6, got, lp2, groups, x_wide=wide)
     assert torch.equal(want, got) and torch.equal(lp, lp2) and torch.equal(lp.float(), wide)
+
+
+# less than a wave, more values than a lane keeps, more rotated columns than a wave has lanes; f32 sums of up to 700 squares: some 20
+# roundings on the longest way, 2e-5 leaves ten times that
+@pytest.mark.parametrize("rank,rot,qn", [(5, 2, 3), (64, 64, 0), (256, 32, 192), (700, 130, 1600)])
+@pytest.mark.parametrize("half", [False, True])
+def test_latent_write_edges(rank, rot, qn, half):
+    from distributed_llm_amd.ops import reference as ref
+    T, g = 4, torch.Generator(device="cuda").manual_seed(rank)
+    R = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    row, w, wq, table = R(T, qn + rank + rot), torch.rand(rank, device="cuda"), torch.rand(max(qn, 1), device="cuda"), R(16, rot)
+    slots = torch.tensor([3, -1, 17, 0], device="cuda", dtype=torch.int32)
+    pos = torch.tensor([0, 16, 15, 7], device="cuda", dtype=torch.int32)      # the padding token's lies behind the table
+    c1, c2 = torch.zeros(2, 16, rank + rot, device="cuda"), torch.zeros(2, 16, rank + rot, device="cuda")
+    q = (row[:, :qn], wq) if qn else (None, None)
+    a = seqmix.latent_kv_write(row[:, qn:], rank, w, 1e-6, pos, table, slots, c1, half, *q)
+    b = ref.latent_kv_write(row[:, qn:], rank, w, 1e-6, pos.clamp(max=15), table, slots, c2, half, *q)
+    torch.testing.assert_close(c1, c2, rtol=2e-5, atol=2e-5)
+    if qn:
+        torch.testing.assert_close(a, b, rtol=2e-5, atol=2e-5)
