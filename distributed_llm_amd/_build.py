@@ -50,6 +50,13 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
+# What every kernel is compiled with; tests/test_kernel_resources.py looks at the registers of exactly this code
+HIP_FLAGS = ["-fPIC", "-O3", "-std=c++17", f"--offload-arch={ARCH}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             "-Wno-unused-result", "-Wno-deprecated-declarations",
+             # no packed-f32 VALU forms (device pass only; the host pass warns that it ignores it)
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+
+
 def build_hip(force: bool = False, jobs: int = 8) -> str:
     kdir = os.path.join(CSRC, "kernels")
     kernels = sorted(os.path.join(kdir, f) for f in os.listdir(kdir) if f.endswith(".hip"))
@@ -61,10 +68,6 @@ def build_hip(force: bool = False, jobs: int = 8) -> str:
     from torch.utils import cpp_extension as ce
     os.makedirs(BUILD, exist_ok=True)
     hipcc = _hipcc()
-    common = ["-fPIC", "-O3", "-std=c++17", f"--offload-arch={ARCH}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-              "-Wno-unused-result", "-Wno-deprecated-declarations",
-              # no packed-f32 VALU forms (device pass only; the host pass warns that it ignores it)
-              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     torch_inc = []
     for p in ce.include_paths(device_type="cuda"):
@@ -73,9 +76,9 @@ def build_hip(force: bool = False, jobs: int = 8) -> str:
     jobs_list = []
     for src in kernels:
         obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-        jobs_list.append([hipcc, *common, "-I", kdir, "-c", src, "-o", obj])
+        jobs_list.append([hipcc, *HIP_FLAGS, "-I", kdir, "-c", src, "-o", obj])
     bind_obj = os.path.join(BUILD, "bindings.o")
-    jobs_list.append([hipcc, *common, *torch_inc, *py_inc, f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+    jobs_list.append([hipcc, *HIP_FLAGS, *torch_inc, *py_inc, f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
                       "-DTORCH_EXTENSION_NAME=_hip_kernels", "-DTORCH_API_INCLUDE_EXTENSION_H",
                       "-c", bind, "-o", bind_obj])
     objs = [j[-1] for j in jobs_list]

@@ -3,7 +3,7 @@
 A kernel that spills to scratch turns its K/V stream into extra memory round trips per lane; a
 harmless-looking refactor (a by-reference lambda around the attention work unit) once made every
 paged-attention instantiation spill 176 B/lane and run ~1.3x slower on MI355X.  This compiles the
-kernels with ``-Rpass-analysis=kernel-resource-usage`` and fails on any scratch use.
+kernels with the flags of the build and ``-Rpass-analysis=kernel-resource-usage`` and fails on any scratch use.
 """
 import os
 import re
@@ -12,12 +12,14 @@ import subprocess
 
 import pytest
 
+from distributed_llm_amd._build import HIP_FLAGS
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 KERNELS = ["attention.hip", "gemv.hip", "skinny_gemm.hip", "sampling.hip", "moe.hip",
            "flash_prefill.hip", "tgemm.hip", "encoder.hip", "gqa.hip", "delta.hip", "mlstm_chunk.hip",
            "chunk_scan.hip", "scan_chunk.hip", "seqmix.hip", "elementwise.hip", "decode_gemm.hip", "moe_decode.hip", "f32_gemm.hip",
-           "latent.hip"]
+           "latent.hip", "wide_gemm.hip", "outer_scan.hip", "norm.hip", "rope_kv.hip", "cosine.hip"]
 # measured exceptions (bytes/lane allowed): the d=64 flash prefill at 4 waves per SIMD (128-VGPR cap,
 # two workgroups per CU) keeps ~5 values in scratch around the chunk loop and is still 1.14-1.17x
 # faster than the spill-free one-workgroup build (profiles/r2_flash_prefill_microbench.md)
@@ -28,8 +30,7 @@ ALLOW = {r"flash_prefill_kernelILi64ELi4E": 32}
 @pytest.mark.parametrize("src", KERNELS)
 def test_no_scratch_spills(src, tmp_path):
     path = os.path.join(ROOT, "csrc", "kernels", src)
-    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-I", os.path.dirname(path), "-c", path,
-                        "-o", str(tmp_path / "k.o"), "-Rpass-analysis=kernel-resource-usage"],
+    r = subprocess.run([HIPCC, *HIP_FLAGS, "-I", os.path.dirname(path), "-c", path, "-o", str(tmp_path / "k.o"), "-Rpass-analysis=kernel-resource-usage"],
                        capture_output=True, text=True, timeout=600)
     assert r.returncode == 0, r.stderr[-2000:]
     names = re.findall(r"Function Name: (\S+)", r.stderr)
