@@ -39,3 +39,58 @@ def test_no_scratch_spills(src, tmp_path):
     budget = lambda n: max([v for k, v in ALLOW.items() if re.search(k, n)] or [0])
     spilled = [(n, s) for n, s in zip(names, scratch) if s > budget(n)]
     assert not spilled, f"scratch spills: {spilled}"
+
+
+def _registers(operand):
+    m = re.fullmatch(r"([va])(?:\[(\d+):(\d+)\]|(\d+))", operand)
+    return {(m[1], i) for i in range(int(m[2] or m[4]), int(m[3] or m[4]) + 1)} if m else set()
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_inline_products_of_wide_gemm(tmp_path):
+    """The compiler does not know that the inline instruction of wide_gemm.hip is a matrix product and keeps no distance from it: a
+    vector instruction must not write an operand within two wait states ahead of one, and from the first product up to the wait behind the
+    last nothing else may touch the accumulators."""
+    path, out = os.path.join(ROOT, "csrc", "kernels", "wide_gemm.hip"), tmp_path / "k.s"
+    r = subprocess.run([HIPCC, *HIP_FLAGS, "-I", os.path.dirname(path), "--cuda-device-only", "-S", path, "-o", str(out)],
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernels = 0
+    for text in re.split(r"\n(?=_Z\w+:)", out.read_text().split(".section\t.AMDGPU.metadata")[0])[1:]:
+        ins, at = [], {}
+        for line in text.split("\n"):
+            line = line.split(";")[0].strip()
+            if re.fullmatch(r"\.L\w+:", line):
+                at[line[:-1]] = len(ins)
+            elif re.match(r"[a-z]\w+(\s|$)", line):
+                ins.append((line.split()[0], re.split(r",\s*", line.split(None, 1)[1]) if " " in line or "\t" in line else []))
+        mul = [i for i, (op, _) in enumerate(ins) if op.startswith("v_mfma")]
+        if not mul:
+            continue
+        kernels += 1
+        ways = {}      # instruction: where a jump comes from
+        for i, (op, args) in enumerate(ins):
+            if "branch" in op and args and args[-1] in at:
+                ways.setdefault(at[args[-1]], []).append(i)
+
+        def ahead(i, states):
+            """Instructions that can run within ``states`` wait states ahead of instruction i."""
+            if states <= 0 or i < 0:
+                return
+            for j in [i - 1] + ways.get(i, []):
+                if j >= 0 and (j != i - 1 or ins[j][0] not in ("s_branch", "s_endpgm")):
+                    yield j
+                    yield from ahead(j, states - (1 + int(ins[j][1][0]) if ins[j][0] == "s_nop" else 1))
+
+        for i in mul:
+            read = set().union(*(_registers(a) for a in ins[i][1][1:]))
+            for j in ahead(i, 2):
+                op, args = ins[j]
+                assert not (op.startswith("v_") and not op.startswith("v_mfma") and _registers(args[0]) & read), (ins[j], ins[i])
+        # (program order is the order of the steps: the loop, the stage before the last, the last)
+        end = next(i for i in range(mul[-1], len(ins)) if ins[i][0] == "s_nop" and ins[i + 1][0] == "s_nop")
+        assert int(ins[end][1][0]) + int(ins[end + 1][1][0]) + 2 >= 18
+        for i in range(mul[0], end):
+            if i not in mul:
+                assert not any(x[0] == "a" for arg in ins[i][1] for x in _registers(arg)), ins[i]
+    assert kernels == 7      # the epilogues
