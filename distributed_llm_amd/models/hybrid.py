@@ -1154,7 +1154,7 @@ class HybridModel:
         cfg, eps = self.cfg, self.cfg.rms_eps
         if scatter is not None:
             ops.scatter_pairs(*scatter)
-        T, W, nL = input_ids.shape[0], cfg.hidden, len(self.layers)
+        T, W, nL = input_ids.numel(), cfg.hidden, len(self.layers)
         ln, rms = cfg.norm_kind == "layer", cfg.pre_norm and cfg.norm_kind != "layer" and not cfg.parallel_ff
         # depth average: an f32 stack of the embedding output and every layer's result; layer i works in place on slot i + 1, which the
         # previous layer's weighted sum has filled with its input

@@ -791,7 +791,9 @@ def embed_rows(ids: torch.Tensor, table: torch.Tensor, scale: float, x: torch.Te
     """The start of a step in one launch: table[ids] * scale as the f32 stream x [T, width] (and x2), its rounding lp, and
     rmsnorm(x) * w in h (lp, h: the table's type).  False where there is no such launch (nothing is written then)."""
     ext = _native(x)
-    return ext is not None and ext.embed_rows(ids, table, float(scale), x, x2, lp, w, float(eps), h)
+    if ext is None or ids.dim() != 1:
+        return False
+    return ext.embed_rows(ids.to(torch.int32).contiguous(), table, float(scale), x, x2, lp, w, float(eps), h)
 
 
 def rope_prep(proj, heads, kv_heads, dim, vdim, cos_sin, rot_dims, qscale, positions, slots, k_cache, v_cache, ucol: int = 0,

@@ -76,6 +76,17 @@ def test_embed_rows_of_other_widths():
     assert bool((x == 3.0).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embed_rows_of_any_ids(dtype):
+    """Whole numbers of another width and strided ones, as the gather takes them; ids of other shapes go its way."""
+    table, x = torch.randn(50, 64, device="cuda").to(dtype), torch.empty(6, 64, device="cuda")
+    ids = torch.randint(0, 50, (6, 2), device="cuda")
+    for some in (ids[:, 0], ids[:, 1].int(), ids[:, 0].to(torch.int16)):
+        assert seqmix.embed_rows(some, table, 2.0, x.zero_())
+        assert torch.equal(x, table[some.long()].float() * 2.0)
+    assert not seqmix.embed_rows(ids[:, :1], table, 2.0, x)
+
+
 @pytest.mark.parametrize("n", [0, 1, 64])
 def test_updates_with_the_inputs(n):
     """The block-table pairs of the pinned buffer, as many as it says."""
