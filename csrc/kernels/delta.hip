@@ -366,10 +366,9 @@ typedef float f32x3 __attribute__((ext_vector_type(3)));
 // accumulators of the last product, which are at once the right operand of S^T k and S^T q.  The waves' parts meet in LDS, a
 // thread sums one element of each, and U = (I + A)^-1 R comes out as the right operand of the state's update.  Serial over the
 // tiles, so the chain of one tile bounds it: two products, one exchange, two small products, the update.  Sums of more than four terms go in
-// parts that are added pairwise, or the largest last.  Three workgroups of the wide-load form fit a CU (with
-// two, 6 sequences are a second pass and take 437 us).  bf16, 16 heads of 128 x 128, with the two launches beside it: 6 sequences of 1400
-// tokens 380 us, one of 4096 tokens 465 (415 and 535 with waits for loads just issued, 617 and 1219 token by token; a second set of
-// registers for the row's inputs 373 and 433, but they spill where the compiler pairs f32 operations).
+// parts that are added pairwise, or the largest last.  Three workgroups of the wide-load form fit a CU (its registers are bounded for
+// that: with two, 6 sequences are a second pass and take 437 us).  bf16, 16 heads of 128 x 128, with the two launches beside it: 6
+// sequences of 1400 tokens 373 us, one of 4096 tokens 433 (421 and 535 with waits for loads just issued, 617 and 1219 token by token).
 // f32 errors against 64 bits over 385 tokens, state and outputs, token by token
 // in brackets: decays near 1 1.5e-7 (5.6e-7), 1.7e-7 (2.6e-7); a model's (0.01 to 0.3 a token) 1.2e-7 (1.9e-7), 1.6e-7 (1.7e-7); up
 // to 4 a token 1.0e-7 (1.05e-7), 1.53e-7 (1.49e-7).
@@ -409,10 +408,10 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
     }
   }
   const long oq = (long)(h / (H / G)) * d, ok = (long)G * d + oq, ov = 2L * G * d + (long)h * dv + (live ? j : dv - 1);
-  // a tile's inputs travel while the one before is computed, its keys two tiles ahead: NS dims of one token's q and k with their factors; one value and its
-  // scalars, four entries of a row of (I + A)^-1 and of P, each loaded again where it has been used.  No load stands behind a condition or
-  // is copied on from tile to tile (rows past the end read the last token's and become zeros where they are used): the compiler then
-  // knows which are in flight, where it waited for all of them at the head of every tile
+  // two tiles' inputs travel while one is computed: NS dims of one token's q and k with their factors; one value and its
+  // scalars, four entries of a row of (I + A)^-1 and of P.  No load stands behind a condition or is copied on from tile to tile (rows past
+  // the end read the last token's and become zeros where they are used; two tiles take turns with two sets of registers): the
+  // compiler then knows which are in flight, where it waited for all of them at the head of every tile
   const int kcol = NS * lr < d ? NS * lr : 0;
   row_t rq, rk;
   float2 fac = make_float2(0.f, 0.f);
@@ -449,22 +448,23 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
   };
   // (three scalars: a register that a load writes and nobody reads is given away while the load is under way, and its next owner waits)
   struct Tile { T v; f32x3 sc; f32x4 inv, p; };
-  Tile cur;
-  auto fetch_row = [&](int t0) {
+  auto fetch_tile = [&](Tile& t, int t0) {
     const int at = q0 + min(t0 + row, n - 1);
-    cur.v = qkv[(long)at * ldq + ov];
-    cur.sc = *reinterpret_cast<const f32x3*>(pre + ((long)at * H + h) * DT_W + 2 * DT_L);
+    t.v = qkv[(long)at * ldq + ov];
+    t.sc = *reinterpret_cast<const f32x3*>(pre + ((long)at * H + h) * DT_W + 2 * DT_L);
+    const float* x = pre + ((long)(q0 + min(t0 + lr, n - 1)) * H + h) * DT_W + 4 * g4;
+    t.inv = *reinterpret_cast<const f32x4*>(x);
+    t.p = *reinterpret_cast<const f32x4*>(x + DT_L);
   };
-  auto entries = [&](int t0) { return pre + ((long)(q0 + min(t0 + lr, n - 1)) * H + h) * DT_W + 4 * g4; };
   __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): the state has landed, so that no tile waits for it
   fetch_keys(0);
-  fetch_row(0);
-  cur.inv = *reinterpret_cast<const f32x4*>(entries(0));
-  cur.p = *reinterpret_cast<const f32x4*>(entries(0) + DT_L);
+  Tile even, odd;
+  fetch_tile(even, 0);
+  fetch_tile(odd, DT_L);
   stage_keys(0, 0);
   fetch_keys(DT_L);
   __syncthreads();
-  for (int t0 = 0, buf = 0; t0 < n; t0 += DT_L, buf ^= 1) {
+  auto tile = [&](const int t0, const int buf, Tile& cur) {
     const int nt = min(DT_L, n - t0);
     {
       f32x4 tk[4], tq[4];
@@ -485,15 +485,18 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
       *reinterpret_cast<f32x4*>(p + TP) = (tq[0] + tq[1]) + (tq[2] + tq[3]);
     }
     __syncthreads();
+    if (nt < DT_L) {      // the last tile: zeros behind the end
+      if (row >= nt) cur.sc = f32x3{0.f, 0.f, 0.f};
+      if (lr >= nt) cur.inv = cur.p = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     {   // token `row`, column lr
       const float* p = part + lr * DT_P + row;
       const float ek = (p[0] + p[2 * TP]) + (p[4 * TP] + p[6 * TP]), eq = (p[TP] + p[3 * TP]) + (p[5 * TP] + p[7 * TP]);
       Rs[lr * DT_P + row] = row < nt ? cur.sc[1] * (ldf(&cur.v) - cur.sc[0] * ek) : 0.f;
       Os[lr * DT_P + row] = cur.sc[0] * eq;
-      if (lr == 0) ws[row] = row < nt ? cur.sc[2] : 0.f;
+      if (lr == 0) ws[row] = cur.sc[2];
       if (tid == 16 * (nt - 1)) last = cur.sc[0];
     }
-    fetch_row(t0 + DT_L);
     stage_keys(buf ^ 1, t0 + DT_L);      // (behind the last tile: zeros that nobody reads)
     fetch_keys(t0 + 2 * DT_L);
     __syncthreads();
@@ -519,8 +522,7 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
     const f32x4 we = *reinterpret_cast<const f32x4*>(ws + 4 * g4);
     const float gam = last;
 #pragma unroll
-    for (int x = 0; x < 4; ++x) u4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(lr < nt ? cur.inv[x] : 0.f, r[x], zero, 0, 0, 0);
-    cur.inv = *reinterpret_cast<const f32x4*>(entries(t0 + DT_L));
+    for (int x = 0; x < 4; ++x) u4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.inv[x], r[x], zero, 0, 0, 0);
     f32x4 u;
 #pragma unroll
     for (int e = 0; e < 4; ++e) u[e] = (u4[e ^ 1][e] + (u4[e ^ 2][e] + u4[e ^ 3][e])) + u4[e][e];
@@ -543,7 +545,7 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
     if (w == ((t0 >> 4) & 3)) {   // the waves take turns with the outputs
       f32x4 o4[4];
 #pragma unroll
-      for (int x = 0; x < 4; ++x) o4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(lr < nt ? cur.p[x] : 0.f, u[x], zero, 0, 0, 0);
+      for (int x = 0; x < 4; ++x) o4[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.p[x], u[x], zero, 0, 0, 0);
       f32x4 o = *reinterpret_cast<const f32x4*>(Os + lr * DT_P + 4 * g4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = (o[e] + (o4[e ^ 1][e] + (o4[e ^ 2][e] + o4[e ^ 3][e]))) + o4[e][e];
@@ -554,8 +556,15 @@ __global__ void __launch_bounds__(256, VL ? 3 : 2) delta_tile_kernel(const T* __
       for (int x = 0; x < 4; ++x)
         if (live && 4 * g4 + x < nt) raw[((long)(q0 + t0 + 4 * g4 + x) * H + h) * dv + j] = o[x];
     }
-    cur.p = *reinterpret_cast<const f32x4*>(entries(t0 + DT_L) + DT_L);
+    fetch_tile(cur, t0 + 2 * DT_L);
+  };
+  // pairs of tiles and perhaps one more: a way out between two of a pair would meet the way back in a block, with its loads under way
+  const int tiles = (n + DT_L - 1) / DT_L;
+  for (int i = 0; i < tiles / 2; ++i) {
+    tile(2 * i * DT_L, 0, even);
+    tile((2 * i + 1) * DT_L, 1, odd);
   }
+  if (tiles & 1) tile((tiles - 1) * DT_L, 0, even);
   if (!live) return;
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
