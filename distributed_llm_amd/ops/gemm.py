@@ -36,7 +36,7 @@ from typing import Dict, Iterable, Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from . import _native, reference as ref
+from . import _load as _load_ext, _native, reference as ref
 
 MAX_M = 1024       # decode buckets up to this size are autotuned
 SKINNY_MAX_M = 128
@@ -1020,9 +1020,30 @@ def _plan_key(k) -> str:
     return "%d,%d,%d,%d" % (k[0], k[1], k[2], int(k[3]))
 
 
-def _load_plans(path: str) -> None:
+# A plan file's key beside its plans: what they were timed with.  Times hold for the kernels that were timed, a choice for the candidates it
+# was made among: a file from before a kernel or a candidate plan would keep both out for good.
+_TIMED_WITH = "timed with"
+
+
+def _timed_with(dev) -> str:
+    """The candidates (this file), the kernels as built, the vendor's library and the device."""
+    import hashlib
+    h = hashlib.sha1()
+    for path in (__file__, getattr(_load_ext(), "__file__", "")):
+        if path and os.path.exists(path):
+            with open(path, "rb") as f:
+                h.update(f.read())
+    p = torch.cuda.get_device_properties(dev)
+    return "%s %s %d %s" % (torch.__version__, p.name, p.multi_processor_count, h.hexdigest())
+
+
+def _load_plans(path: str, timed_with: Optional[str] = None) -> None:
+    """``timed_with``: nothing of a file that was timed with anything else (None: any file)."""
     with open(path) as f:
-        for k, v in json.load(f).items():
+        d = json.load(f)
+        if d.pop(_TIMED_WITH, None) != timed_with and timed_with is not None:
+            return
+        for k, v in d.items():
             kind, *at = k.split(",")
             if kind == "t":
                 _P.tg_plans[tuple(map(int, at))] = tuple(v)
@@ -1041,7 +1062,7 @@ def _load_plans(path: str) -> None:
                 _P.plans[(int(kind), int(at[0]), int(at[1]), at[2] == "1")] = tuple(v)
 
 
-def _save_plans(path: str) -> None:
+def _save_plans(path: str, timed_with: str = "") -> None:
     d = {_plan_key(k): list(v) for k, v in _P.plans.items()}
     d.update({_plan_key(k): list(v) for k, v in _P.tg_plans.items()})
     d.update({"c,%d,%d,%d" % k: v for k, v in _P.fused_core.items()})
@@ -1049,6 +1070,7 @@ def _save_plans(path: str) -> None:
     d.update({"d,%d,%d,%d" % k: v and list(v) for k, v in _P.dg_plans.items()})
     d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
     d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
+    d[_TIMED_WITH] = timed_with
     if os.path.dirname(path):
         os.makedirs(os.path.dirname(path), exist_ok=True)
     with open(path, "w") as f:
@@ -1075,8 +1097,9 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
         _P.cus = _sk_grid(dev)
         _P.pf_parts.clear()
     cache = os.environ.get("DLLM_GEMM_PLANS")  # JSON plan cache: re-use a previous run's choices
+    made = _timed_with(dev) if cache else ""
     if cache and os.path.exists(cache):
-        _load_plans(cache)
+        _load_plans(cache, made)
     shapes = list(shapes)
     fused = list(fused)
     # the fused ops' tgemm plans stream the panel weight copies: time them in that layout
@@ -1089,7 +1112,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     if PREFILL_TUNE or prefill:
         _autotune_prefill(fused, dev, verbose, roles, qkv_dims)
     if cache:
-        _save_plans(cache)
+        _save_plans(cache, made)
 
 
 def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> None:

@@ -213,6 +213,54 @@ def test_plan_file(monkeypatch, tmp_path):
     assert G._P.fused_core == {(8, 2048, 2048): "tg"} and G._P.dg_plans == {(8, 2048, 2048): (1, 2, 4)} and not G._P.frag_core
 
 
+def test_plan_file_of_other_code(monkeypatch, tmp_path):
+    """Times hold for the kernels and candidates that were timed: nothing comes back from a file that was timed with others, or does not say."""
+    import json
+    from types import SimpleNamespace
+    _none_timed(monkeypatch)
+    cards = {0: SimpleNamespace(name="A", multi_processor_count=256), 1: SimpleNamespace(name="A", multi_processor_count=64)}
+    monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: cards[d])
+    built = tmp_path / "kernels.so"
+    monkeypatch.setattr(G, "_load_ext", lambda: SimpleNamespace(__file__=str(built)))
+    made = []
+    for content, card in ((b"one", 0), (b"two", 0), (b"one", 1)):
+        built.write_bytes(content)
+        made.append(G._timed_with(card))
+    assert len(set(made)) == 3 and built.write_bytes(b"one") and G._timed_with(0) == made[0]
+    k, path = (16, 2048, 2048), str(tmp_path / "plans.json")
+    G._P.tg_plans[k] = (64, 64, 3, 1, 1, 4)
+    G._save_plans(path, made[0])
+    for m, want in ((made[1], {}), (made[0], {k: (64, 64, 3, 1, 1, 4)})):
+        G._P.tg_plans.clear()
+        G._load_plans(path, m)
+        assert G._P.tg_plans == want
+    with open(path) as f:
+        d = json.load(f)
+    with open(path, "w") as f:
+        json.dump({k: v for k, v in d.items() if k.startswith("t,")}, f)
+    G._P.tg_plans.clear()
+    G._load_plans(path, made[0])
+    assert not G._P.tg_plans
+
+
+@pytest.mark.gpu
+def test_old_plan_file_is_timed_again(monkeypatch, tmp_path):
+    import json
+    _none_timed(monkeypatch)
+    monkeypatch.setattr(G, "PREFILL_TUNE", False)
+    path, key = str(tmp_path / "plans.json"), "%d,%d,%d,0" % (4, 1024, 768)
+    with open(path, "w") as f:
+        json.dump({key: ["skinny", 1, 1], "%d,%d,%d,0" % (4, 999, 768): ["blas"]}, f)
+    monkeypatch.setenv("DLLM_GEMM_PLANS", path)
+    G.autotune([(1024, 768, False)], [4], "cuda")
+    assert set(G._P.plans) == {(4, 1024, 768, False)}
+    timed = dict(G._P.plans)
+    _none_timed(monkeypatch)
+    monkeypatch.setattr(G, "_time", lambda *a, **k: pytest.fail("timed again"))
+    G.autotune([(1024, 768, False)], [4], "cuda")
+    assert G._P.plans == timed
+
+
 @pytest.mark.gpu
 def test_copies_are_timed_when_they_come_second(monkeypatch):
     """Shapes timed for a model without copies, then for one with them: the decode GEMM is timed, the earlier choices stand."""
