@@ -160,7 +160,7 @@ class LLMEngine:
         prefix_cache = prefix_cache and not self.recurrent
         geo = getattr(self.model, "attn_geometry", "llama")
         self._paged_attn = geo is not None       # softmax attention over paged K/V (split-K work lists)
-        self._nkv = self.model.nkv if self._paged_attn else 1
+        self._nkv, self._head_dim = (self.model.nkv, self.model.d) if self._paged_attn else (1, 1)
         if hasattr(self.model, "ensure_positions"):
             self.model.ensure_positions(self.max_model_len)
         self.max_num_seqs = max_num_seqs
@@ -191,6 +191,8 @@ class LLMEngine:
         self._memo_cap = 200_000
         self._memo_lock = threading.Lock()
         self.on_gpu = self.device.type == "cuda"
+        if self.on_gpu:
+            self._cus = torch.cuda.get_device_properties(self.device).multi_processor_count
         self._ws_owner = ("engine", id(self))   # split-K workspaces of this engine's kernels/graphs
         # expert-parallel MoE exchanges split sizes on the host (parallel.expert_parallel): eager
         # (an expert-parallel MoE model decodes on its TP-within-expert shards: graph-capturable)
@@ -390,17 +392,24 @@ class LLMEngine:
     # static split grid (a kernel-only sweep had B=16-64 about even)
     ATTN_WL_MIN_BS = 1
     # shortest key range of one work-list unit (split-K granularity).  It only matters while batch x context < 64k tokens, above
-    # that the target unit count sets the chunk.  A unit's eight waves take 256 keys a trip, 1.2 us; parts that meet cost 2 to 3 us (slabs past
-    # L2, a ticket, the last one's sum).  us of a launch, TinyLlama's heads, chunk of 128 / 256 / whole: 24 requests of 20-300
-    # keys 8.2 / 8.5 / 6.2, 48 of 40-424 10.1 / 10.0 / 8.1, 64 of 300-900 18.7 / 18.8 / 12.5, 2 of 500-1000 8.0 / 8.8 / 10.0, 8 of
-    # 2000-5000 14.4 / 13.9 / 19.6.
+    # that the target unit count sets the chunk.  A unit's eight waves take 256 keys a trip, 1.2 us (heads of 128: 2 to 2.5); parts that meet cost 2 to
+    # 3 us (slabs past L2, a ticket, the last one's sum).  us of a launch, chunk of 128 / 256 / whole.  Heads of 64 (TinyLlama's): 24 requests of
+    # 20-300 keys 8.2 / 8.5 / 6.2, 48 of 40-424 10.1 / 10.0 / 8.1, 64 of 300-900 18.7 / 18.8 / 12.5, 2 of 500-1000 8.0 / 8.8 / 10.0, 8 of
+    # 2000-5000 14.4 / 13.9 / 19.6; one request and one key head, 320 keys 7.3 / 7.1 / 5.4, 512 7.3 / 7.9 / 6.4; one request of 1800 9.0 / 8.4
+    # / 11.3 (eight key heads 9.6 / 8.7 / 11.7), 2500 9.1 / 8.6 / 11.3, 3500 9.5 / 9.6 / 11.7.  Heads of 128: one request of 350 8.3 / 8.8 / 8.3, 450
+    # 8.4 / 9.6 / 9.9, 1800 10.3 / 10.5 / 16.9; 32 of 100-384 on two key heads 9.4 / 9.9 / 9.3.
     ATTN_MIN_CHUNK = 256
+    _cus = 256               # CUs of the device
+    _head_dim = 64
 
     def _min_chunk(self, lens: np.ndarray) -> int:
-        longest, heads = int(lens.max()), len(lens) * self._nkv
-        if longest <= 512 or (longest <= 1024 and heads >= 128):      # two trips, or four that fill half the CUs: whole
+        longest, half, wide = int(lens.max()), self._cus // 2, self._head_dim > 96
+        # two trips (of the wider heads, whose trips are longer, up to where parts of 128 take over), or four that fill half the CUs: whole
+        if longest <= (384 if wide else 512) or (longest <= 1024 and len(lens) * self._nkv >= half):
             return 1024
-        return 128 if int((-(-lens // 128)).sum()) * self._nkv <= 128 else self.ATTN_MIN_CHUNK
+        if not wide and 1536 < longest <= 3072:      # (12 to 16 parts of 128: the sum of so many is what eats their gain)
+            return self.ATTN_MIN_CHUNK
+        return 128 if int((-(-lens // 128)).sum()) * self._nkv <= half else self.ATTN_MIN_CHUNK
 
     def _use_worklist(self, bs: int) -> bool:
         return self.attn_worklist and bs >= self.ATTN_WL_MIN_BS

@@ -66,3 +66,16 @@ def test_chunk_of_a_batch(lens, nkv, want):
     assert got == want
     if want == 1024:
         assert ops.decode_work_items(np.array(lens), nkv, 16, 512, min_chunk=got)[0] == len(lens) * nkv
+
+
+@pytest.mark.parametrize("lens,nkv,d,cus,want", [
+    ([512], 1, 64, 256, 1024), ([512], 1, 96, 256, 1024), ([384], 1, 128, 256, 1024), ([385], 1, 128, 256, 128),      # a trip of wide heads is longer
+    ([400] * 16, 4, 128, 256, 256), ([400] * 32, 4, 128, 256, 1024), ([1024] * 32, 4, 128, 256, 1024),
+    ([1536], 8, 64, 256, 128), ([1537], 8, 64, 256, 256), ([3072], 1, 96, 256, 256), ([3073], 1, 96, 256, 128), ([1800], 1, 128, 256, 128),
+    ([1024] * 31, 4, 64, 304, 256), ([1024] * 16, 4, 64, 128, 1024), ([1024] * 15, 4, 64, 128, 256), ([640] * 3, 4, 64, 128, 128),
+    ([640] * 4, 4, 64, 128, 256)])
+def test_chunk_by_head_width_and_device(lens, nkv, d, cus, want):
+    from distributed_llm_amd.engine.llm_engine import LLMEngine
+    eng = LLMEngine.__new__(LLMEngine)
+    eng._nkv, eng._head_dim, eng._cus = nkv, d, cus
+    assert eng._min_chunk(np.array(lens)) == want
