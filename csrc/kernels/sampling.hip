@@ -748,8 +748,10 @@ extern "C" int dllm_sample_rows(const void* logits, long stride, int B, int V, c
                                 const int* top_k, const unsigned* seed, int* out, int* out_host, hipStream_t stream) {
   if (B <= 0) return 0;
   if (V <= 0 || stride % 8 != 0) return -1;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -2;
   // (sixteen waves of the sampled path's registers are a CU; past one row a CU they would take turns)
-  if (B <= 256)
+  if (B <= cus)
     hipLaunchKernelGGL((sample_rows_kernel<1024>), dim3(B), dim3(1024), 0, stream, (const u16*)logits, stride, V, temp, top_p, top_k,
                        seed, out, out_host);
   else
