@@ -429,11 +429,18 @@ def tg_plan(M: int, N: int, K: int) -> Tuple[int, ...]:
             p = (_small(M, N, K) or (None,))[0]
     if p is not None:
         return tuple(p) + (1, 4)[len(p) - 4:] if len(p) < 6 else tuple(p)
-    mt64, nt64 = -(-M // 64), -(-N // 64)
+    mt64, nt64, nt128 = -(-M // 64), -(-N // 64), -(-N // 128)
     # 64 x 128 tiles of eight waves from 150 of them on, two workgroups a CU.  us 128 x 128 / here / 64 x 64 (GELU epilogue): 3800 rows
-    # 1536 x 384 18 / 14 / 14, 384 x 1536 21 / 15 / 17, 8000 rows 1536 x 384 29 / 24 / 33, 1200 rows 3072 x 2048 27 / 25 / 32, 500 rows 1536 x
-    # 384 9 / 7 / 7; at 500 rows of 1152 x 1536 (72 tiles) 21 / 14 / 12.
-    if mt64 * -(-N // 128) >= 150:
+    # 1536 x 384 18 / 14 / 14, 384 x 1536 21 / 15 / 17, 8000 rows 1536 x 384 29 / 24 / 33, 1200 rows 3072 x 2048 27 / 25 / 32, 16000 rows 4096 x
+    # 1024 260 / 232 / 292, 500 rows 1536 x 384 9 / 7 / 7; at 500 rows of 1152 x 1536 (72 tiles) 21 / 14 / 12.  More columns than rows are few
+    # tiles of many rows' worth of weights: 300 rows of 4096 x 4096 (160) 43 / 30 / 28, 600 of 2304 x 768 (180) 15 / 10.8 / 10.3, 600 of
+    # 3072 x 768 (240) 15 / 11.2 / 11.3.  A long K down to fewer columns (residual epilogue) reads less with 128 x 128, where its tiles are
+    # whole rounds: 1024 x 4096, 4000 rows (256 tiles) 45 / 49, 8000 89 / 97, 2000 (128) 41 / 30; 4096 x 4096, 2000 rows 88 / 92; 768 x 3072,
+    # 16000 rows (750) 104 / 108, 8000 (378) 64 / 57
+    tiles = -(-M // 128) * nt128
+    if K >= 2048 and N <= K and tiles >= 0.9 * _P.cus * -(-tiles // _P.cus):
+        return (128, 128, 3, 1, 1, 8)
+    if mt64 * nt128 >= (150 if M >= N else 185):
         return (64, 128, 3, 1, 1, 8)
     tiles = mt64 * nt64
     splits = 1

@@ -61,6 +61,20 @@ def test_rows_between_batch_sizes_take_the_next_ones_plan(monkeypatch):
     assert G.tg_slots(57, 256, 512) == 4 and G.tg_slots(70, 256, 512) == 2
 
 
+def test_untimed_tiles(monkeypatch):
+    """Both sides of each line of the rule for shapes that nobody timed."""
+    _none_timed(monkeypatch)
+    monkeypatch.setattr(G._P, "cus", 256)
+    tile = lambda M, N, K: G.tg_plan(M, N, K)[:2]  # noqa: E731
+    assert tile(3200, 384, 1536) == (64, 128) and tile(3136, 384, 1536) == (64, 64)      # 150 and 147 tiles
+    assert tile(600, 2304, 768) == (64, 64) and tile(640, 2432, 768) == (64, 128)         # 180 and 190, more columns than rows
+    assert tile(4000, 1024, 4096) == (128, 128) and tile(2000, 1024, 4096) == tile(4200, 1024, 4096) == (64, 128)
+    assert tile(16000, 768, 3072) == (128, 128) and tile(8000, 768, 3072) == (64, 128)
+    assert tile(4000, 1024, 1984) == tile(16000, 4096, 1024) == tile(1000, 8192, 2048) == (64, 128)
+    monkeypatch.setattr(G._P, "cus", 128)
+    assert tile(2000, 1024, 4096) == (128, 128)
+
+
 def _timed(monkeypatch, N, K, us, small):
     """Tables as the autotuner leaves them: a round of 256 tiles of 256 x 256 and of 256 x 128, and plans of small tiles."""
     big, half = (256, 256, 2, 1, 1, 8), (256, 128, 3, 1, 1, 8)
