@@ -177,7 +177,9 @@ class _Planner:
         self.fused_opts: Dict[Tuple[int, int, int], Dict[str, float]] = {}   # measured us per core choice
         self.pf_times: Dict[Tuple[int, int], list] = {}      # (N, K) of prompts: [(plan, rows, us)]
         self.pf_small: Dict[Tuple[int, int, int], Tuple] = {}        # (rows of PF_SMALL_MS, N, K): (fastest plan, its us)
+        self.pf_lin: Dict[Tuple[int, int], list] = {}        # (N, K) of prompts: [(rows, us)] of the vendor's product and its epilogue
         self.pf_parts: Dict[Tuple[int, int, int], Tuple] = {}        # prompt_parts' answers
+        self.pf_vendor: Dict[Tuple[int, int, int], bool] = {}        # use_vendor_core's, for rows that are no bucket
         self.cus = 256            # CUs of the device the prompt plans were timed on
         self.ws: Dict[Tuple, Tuple[torch.Tensor, torch.Tensor]] = {}
         self.sk_tables: Dict[Tuple, Tuple[torch.Tensor, int]] = {}   # stream-K segment lists per shape
@@ -355,6 +357,35 @@ def _round_us(N: int, K: int):
     return out
 
 
+def _parts_us(M: int, N: int, K: int) -> Tuple[float, Optional[Tuple]]:
+    """(us, parts): ``prompt_parts`` worked out."""
+    best, us, parts, cus = float("inf"), float("inf"), None, _P.cus
+    rounds, usual = _round_us(N, K), tg_plan(M, N, K)
+    tiles = lambda rows, plan: -(-rows // plan[0]) * -(-N // plan[1])
+    if usual in rounds:
+        us, parts = _rounds(tiles(M, usual), cus) * rounds[usual], ((M, usual),)
+        best = _PART_GAIN * us
+    for plan, u in rounds.items():
+        t = _rounds(tiles(M, plan), cus) * u
+        if t < best:
+            best, us, parts = t, t, ((M, plan),)
+        for k in range(1, -(-tiles(M, plan) // cus)):      # k rounds of it, and the rows they leave
+            rows = k * cus // -(-N // plan[1]) * plan[0]
+            tail = _small(M - rows, N, K) if 0 < rows < M else None
+            if tail is not None:
+                t = _rounds(tiles(rows, plan), cus) * u + tail[1] + _PART_US
+                if t < best:
+                    best, us, parts = t, t, ((rows, plan), (M - rows, tail[0]))
+    return us, parts
+
+
+def _keep(answers: dict, key, answer):
+    if len(answers) > 4096:
+        answers.clear()
+    answers[key] = answer
+    return answer
+
+
 def prompt_parts(M: int, N: int, K: int) -> Optional[Tuple]:
     """How the one-launch form of a fused product of a prompt's M > MAX_M rows runs: ((rows, plan), ...) one behind the other, or None
     where nothing was timed.  A large tile costs by rounds over the CUs: 8928 rows of 2048 columns are 280 tiles of 256 x 256, two
@@ -363,27 +394,29 @@ def prompt_parts(M: int, N: int, K: int) -> Optional[Tuple]:
     key = (M, N, K)
     if key in _P.pf_parts:
         return _P.pf_parts[key]
-    best, parts, cus = float("inf"), None, _P.cus
-    rounds, usual = _round_us(N, K), tg_plan(M, N, K)
-    tiles = lambda rows, plan: -(-rows // plan[0]) * -(-N // plan[1])
-    if usual in rounds:
-        best, parts = _PART_GAIN * _rounds(tiles(M, usual), cus) * rounds[usual], ((M, usual),)
-    for plan, u in rounds.items():
-        t = _rounds(tiles(M, plan), cus) * u
-        if t < best:
-            best, parts = t, ((M, plan),)
-        for k in range(1, -(-tiles(M, plan) // cus)):      # k rounds of it, and the rows they leave
-            rows = k * cus // -(-N // plan[1]) * plan[0]
-            tail = _small(M - rows, N, K) if 0 < rows < M else None
-            if tail is not None:
-                t = _rounds(tiles(rows, plan), cus) * u + tail[1] + _PART_US
-                if t < best:
-                    best, parts = t, ((rows, plan), (M - rows, tail[0]))
-    if parts is not None:
-        if len(_P.pf_parts) > 4096:
-            _P.pf_parts.clear()
-        _P.pf_parts[key] = parts
-    return parts
+    parts = _parts_us(M, N, K)[1]
+    return None if parts is None else _keep(_P.pf_parts, key, parts)
+
+
+# Row counts beside the buckets at which the vendor's product and its epilogue are timed
+PF_LIN_MS = (1280, 3072, 5120, 6144, 10240, 12288, 14336, 16384)
+_VENDOR_GAIN = 0.97       # the other form than the bucket's, where it is that much shorter
+
+
+def _vendor_at(M: int, N: int, K: int, bucket: bool) -> bool:
+    """Whether a prompt's M rows run on the vendor's product and its epilogue: as their ``bucket``, unless the other form is the shorter one by
+    what is timed around M.  Both go by rounds of tiles, of other sizes; between two timed sizes the vendor's takes as long as at the larger
+    one, or longer.  us, vendor / one launch, TinyLlama: down 4500 rows 94 / 110, 8192 140 / 137, 8928 193 / 171, 10000 202 / 241, 11679 244 / 255,
+    13000 246 / 241; output 4500 47 / 52, 8192 70 / 61, 10000 94 / 107, 11679 106 / 111; QKV 4096 58 / 72, 7000 104 / 100, 11679 138 / 136,
+    14500 200 / 178.  Over 424 row counts of ten products this is 1.9 % above the shorter form, 3.2 % by the bucket alone."""
+    key = (M, N, K)
+    if key in _P.pf_vendor:
+        return _P.pf_vendor[key]
+    at, us = sorted(_P.pf_lin.get((N, K), ())), _parts_us(M, N, K)[0]
+    if not at or us == float("inf"):
+        return bucket
+    lin = next((t for m, t in at if M <= m), at[-1][1] * M / at[-1][0])
+    return _keep(_P.pf_vendor, key, us >= _VENDOR_GAIN * lin if bucket else lin < _VENDOR_GAIN * us)
 
 
 def _row_parts(M: int, N: int, K: int, frag: bool = False) -> list:
@@ -723,6 +756,8 @@ def use_vendor_core(M: int, N: int, K: int, frag: bool = False) -> bool:
     c = _core_of(M, N, K, frag)
     if c is None and M > MAX_M and PREFILL_MS:
         c = _P.fused_core.get((prefill_bucket(M), N, K))
+        if c is not None:
+            return _vendor_at(M, N, K, c != "tg")
     if c is not None:
         return c != "tg"
     return M > MAX_M
@@ -1056,6 +1091,8 @@ def _load_plans(path: str, timed_with: Optional[str] = None) -> None:
                 _P.tg_plans[tuple(map(int, at))] = tuple(v)
             elif kind == "s":
                 _P.pf_small[tuple(map(int, at))] = (tuple(v[0]), v[1])
+            elif kind == "l":
+                _P.pf_lin[tuple(map(int, at))] = [tuple(e) for e in v]
             elif kind == "p":
                 _P.pf_times[tuple(map(int, at))] = [(tuple(q), m, t) for q, m, t in v]
             elif kind == "d":
@@ -1077,6 +1114,7 @@ def _save_plans(path: str, timed_with: str = "") -> None:
     d.update({"d,%d,%d,%d" % k: v and list(v) for k, v in _P.dg_plans.items()})
     d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
     d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
+    d.update({"l,%d,%d" % k: v for k, v in _P.pf_lin.items()})
     d[_TIMED_WITH] = timed_with
     if os.path.dirname(path):
         os.makedirs(os.path.dirname(path), exist_ok=True)
@@ -1103,6 +1141,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
     if _P.cus != _sk_grid(dev):
         _P.cus = _sk_grid(dev)
         _P.pf_parts.clear()
+        _P.pf_vendor.clear()
     cache = os.environ.get("DLLM_GEMM_PLANS")  # JSON plan cache: re-use a previous run's choices
     made = _timed_with(dev) if cache else ""
     if cache and os.path.exists(cache):
@@ -1123,10 +1162,10 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
 
 
 def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> None:
-    """Fused-op core at the prefill buckets: one tgemm launch with the epilogue fused (PLAIN timed,
-    the fused epilogues write the same tile or less) against hipBLASLt + the standalone epilogue
-    kernel; the tgemm plans stream the K-panel weight copy the model keeps (W_PANEL).  Among the tgemm plans
-    ``prompt_parts`` chooses by times with the epilogue; plans of the sizes below the buckets are timed too."""
+    """Fused-op core at the prefill buckets: one tgemm launch with the epilogue fused against hipBLASLt + the standalone epilogue kernel,
+    both timed through the fused op (by their plain products TinyLlama's QKV of 4096 rows went to one launch of 72 us from
+    58; where a shape has no fused op: PLAIN, and the vendor's plus ``_post_us``), the vendor's at PF_LIN_MS as well (``_vendor_at``);
+    the tgemm plans stream the K-panel weight copy the model keeps (W_PANEL).  Plans of the sizes below the buckets are timed too."""
     roles = roles or {}
     for (N, K) in {tuple(f) for f in fused}:
         todo = [M for M in PREFILL_MS if (M, N, K) not in _P.fused_core]
@@ -1135,12 +1174,23 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
         copies = max(2, min(8, (256 << 20) // (N * K * 2)))
         ws = [(torch.randn(N, K, device=dev) * 0.02).to(torch.bfloat16) for _ in range(copies)]
         wps = [panel_weight(w) for w in ws] if W_PANEL else ws
+        lins = {}
+        for M in sorted({*todo, *PF_LIN_MS}) if (N, K) in roles else ():
+            whole = _fused_call(roles[(N, K)], torch.randn(M, K, device=dev).to(torch.bfloat16), ws, wps, qkv_dims, dev)
+            try:
+                _P.fused_core[(M, N, K)] = "lin"
+                lins[M] = _time(whole, iters=8)
+            except Exception:  # noqa: BLE001 - no such fused op
+                continue
+            finally:
+                _P.fused_core.pop((M, N, K), None)
+        _P.pf_lin[(N, K)] = sorted({**dict(_P.pf_lin.get((N, K), ())), **lins}.items())
         for M in todo:
             x = torch.randn(M, K, device=dev).to(torch.bfloat16)
             y = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
             ext = _native(x)
-            lin = _time(lambda i: torch.matmul(x, ws[i % copies].t(), out=y), iters=8) + _post_us(M, N, dev)
-            best, best_t = None, float("inf")
+            lin = lins.get(M) or _time(lambda i: torch.matmul(x, ws[i % copies].t(), out=y), iters=8) + _post_us(M, N, dev)
+            best, best_t, best_whole = None, float("inf"), float("inf")
             times = _P.pf_times.setdefault((N, K), [])
             whole = _fused_call(roles.get((N, K)), x, ws, wps, qkv_dims, dev)
             for p in _PF_PLANS:
@@ -1156,12 +1206,13 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
                     _P.fused_core.pop((M, N, K), None)      # (not timed yet: ``todo``)
                 if t < best_t:
                     best, best_t = p, t
+                best_whole = min(best_whole, t_whole)
                 times.append((p, M, t_whole))
             if best is not None:
                 _P.tg_plans[(M, N, K)] = best
-            _P.fused_core[(M, N, K)] = "tg" if best is not None and best_t < lin else "lin"
+            _P.fused_core[(M, N, K)] = "tg" if best_whole < lin else "lin"
             if verbose:
-                print(f"gemm prefill M={M} N={N} K={K}: blas+post {lin:.1f}us, tgemm {best} {best_t:.1f}us "
+                print(f"gemm prefill M={M} N={N} K={K}: blas+post {lin:.1f}us, tgemm {best} {best_whole:.1f}us "
                       f"-> {_P.fused_core[(M, N, K)]}", flush=True)
             del x, y
         for M in PF_SMALL_MS:
@@ -1180,6 +1231,7 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
             if verbose and best is not None:
                 print(f"gemm rows M={M} N={N} K={K}: {best} {res[best]:.1f}us", flush=True)
         _P.pf_parts.clear()
+        _P.pf_vendor.clear()
         del ws, wps
 
 

@@ -106,6 +106,35 @@ def test_prompt_parts(monkeypatch, N, us, small):
     assert G.prompt_parts(8928, N, 256) is None
 
 
+def test_vendor_core_by_the_rows_at_hand(monkeypatch):
+    """Times as TinyLlama's down product has them: one round of 256 x 256 tiles at 8192 rows beats the vendor's product, two at 10000 do not,
+    two full ones do again; a bucket's own choice stands, and rows that nothing was timed for go by their bucket."""
+    monkeypatch.delenv("DLLM_FUSED_CORE", raising=False)
+    _none_timed(monkeypatch)
+    N, K, wide = 2048, 5632, (256, 256, 2, 1, 1, 4)
+    monkeypatch.setattr(G._P, "cus", 256)
+    G._P.pf_times[N, K] = [(wide, m, t) for m, t in ((2048, 120.0), (4096, 122.0), (8192, 137.0))]
+    G._P.pf_lin[N, K] = [(1280, 45.0), (2048, 53.0), (4096, 86.0), (6144, 118.0), (8192, 140.0), (10240, 205.0), (12288, 250.0), (16384, 298.0)]
+    G._P.tg_plans.update({(m, N, K): wide for m in G.PREFILL_MS})
+    G._P.pf_small.update({(m, N, K): ((128, 128, 3, 1, 1, 8), 30.0) for m in G.PF_SMALL_MS})
+    G._P.fused_core.update({(2048, N, K): "lin", (4096, N, K): "lin", (8192, N, K): "tg"})
+    want = {1100: True, 2048: True, 4096: True, 4500: True, 6000: True, 8000: False, 8192: False, 8900: False, 10000: True, 11679: True,
+            12288: True, 13000: False, 16384: False, 20000: True}
+    for _ in range(2):      # (worked out, then looked up)
+        assert {M: G.use_vendor_core(M, N, K) for M in want} == want
+    parts = lambda M: [p == "lin" for _, _, p in G._row_parts(M, N, K)]  # noqa: E731
+    assert parts(10000) == [True] and parts(8900) == [False, False] and parts(16000) == [False]
+    # a choice is kept unless the other form is shorter by more than the times are uncertain by
+    G._P.fused_core[8192, N, K] = "lin"
+    G._P.pf_vendor.clear()
+    assert G.use_vendor_core(8000, N, K) and G.use_vendor_core(10000, N, K) and not G.use_vendor_core(8900, N, K)
+    G._P.fused_core[8192, N, K] = "tg"
+    for gone in ("pf_lin", "pf_times"):
+        monkeypatch.setattr(G._P, gone, {})
+        monkeypatch.setattr(G._P, "pf_vendor", {})
+        assert not G.use_vendor_core(10000, N, K) and G.use_vendor_core(3000, N, K)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("panel", [False, True])
 def test_parts_are_the_whole(monkeypatch, panel):
@@ -167,7 +196,7 @@ def test_decode_gemm_in_place_of_a_skinny_plan(monkeypatch):
 
 
 def _none_timed(monkeypatch):
-    for name in ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "fused_opts", "pf_times", "pf_small", "pf_parts"):
+    for name in ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "fused_opts", "pf_times", "pf_small", "pf_parts", "pf_lin", "pf_vendor"):
         monkeypatch.setattr(G._P, name, {})
 
 
@@ -214,7 +243,8 @@ def test_plan_file(monkeypatch, tmp_path):
     G._P.tg_plans[k], G._P.fused_core[k], G._P.frag_core[k] = (64, 64, 3, 1, 1, 4), "skE4", "dg1.2.2"
     G._P.dg_plans.update({k: (1, 2, 4), (8, 2048, 2048): None})
     G._P.pf_times[2048, 2048], G._P.pf_small[128, 2048, 2048] = [((256, 256, 2, 1, 1, 8), 2048, 50.0)], ((64, 64, 3, 1, 1, 4), 9.0)
-    tables = ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "pf_times", "pf_small")
+    G._P.pf_lin[2048, 2048] = [(2048, 40.0), (3072, 55.0)]
+    tables = ("plans", "tg_plans", "dg_plans", "fused_core", "frag_core", "pf_times", "pf_small", "pf_lin")
     want = {n: dict(getattr(G._P, n)) for n in tables}
     G._save_plans(str(tmp_path / "sub" / "plans.json"))
     _none_timed(monkeypatch)
