@@ -1848,7 +1848,7 @@ class LLMEngine:
                 if s is not None:
                     self._release(s)
             return torch.empty((0, self.cfg.vocab))
-        decode, table = True, (self._bt_dirty, self._bt_rows)
+        decode, synced = True, (self._bt_dirty, self._bt_rows)
         opened: List[int] = []
         for key, toks, _ in entries:
             toks = [int(t) for t in toks]
@@ -1885,10 +1885,10 @@ class LLMEngine:
                         opened += (s.row * self.max_blocks + nblk - 1, slot // BS)
             seqs.append(s)
         n_want = sum(len(w) for _, _, w in entries)
-        if decode and not table[0]:
+        if decode and not synced[0]:
             # blocks opened by single tokens travel with the step's inputs (its scatter applies them, as in generation): the table's
             # copy of a few columns waits for the device, 40-48 us of a step
-            self._bt_dirty, self._bt_rows = table
+            self._bt_dirty, self._bt_rows = synced
             self._bt_upd.extend(opened)
         if decode:
             if self.d_logits is None:
