@@ -994,6 +994,7 @@ int by_tile(int bm, int bn, int stages, int ks, int nw, int wk, const GemmArgs& 
     if (bm == 128 && bn == 128) return by_pipe_deep<128, 128, EPI, 8>(stages, ks, a, st);
     if (bm == 192 && bn == 128) return by_pipe<192, 128, EPI, 8>(stages, ks, a, st);
     if (bm == 256 && bn == 128) return by_pipe<256, 128, EPI, 8>(stages, ks, a, st);
+    // (for plans with splits of K; of one split the four-wave form is the faster, and the one that is timed)
     if (bm == 256 && bn == 256) return by_pipe<256, 256, EPI, 8>(stages, ks, a, st);
   }
   return -20;
@@ -1006,9 +1007,8 @@ int by_tile_grouped(int bm, int bn, int stages, int ks, int nw, const GemmArgs& 
   if (bm == 64 && bn == 128 && stages == 3 && nw == 4) return launch_fit<64, 128, EPI, 3, 1, 4>(a, st);
   if (bm == 64 && bn == 64 && stages == 6 && nw == 4) return launch_fit<64, 64, EPI, 6, 1, 4>(a, st);
   if (bm == 128 && bn == 128 && stages == 4 && nw == 8) return launch_fit<128, 128, EPI, 4, 1, 8>(a, st);
-  if (bm == 256 && bn == 256 && stages == 2 && nw == 4) return dllm::wide_gemm(a, EPI, st);
+  if (bm == 256 && bn == 256 && stages == 2) return dllm::wide_gemm(a, EPI, st);      // (plans of eight waves: the same bits)
   if (bm == 256 && bn == 128 && stages == 3 && nw == 8) return launch_fit<256, 128, EPI, 3, 1, 8>(a, st);
-  if (bm == 256 && bn == 256 && stages == 2 && nw == 8) return launch_fit<256, 256, EPI, 2, 1, 8>(a, st);
   return -20;
 }
 

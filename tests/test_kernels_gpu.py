@@ -460,7 +460,7 @@ def test_moe_ffn(T, H, I, E, k):
 
 
 _MOE_PLANS = [(64, 128, 3, 1, 4, 64, 3, 1, 4), (128, 128, 3, 1, 8, 128, 3, 1, 8), (64, 64, 2, 2, 4, 128, 2, 1, 4),
-              (256, 256, 2, 1, 8, 128, 3, 1, 8)]
+              (256, 256, 2, 1, 8, 128, 3, 1, 8), (256, 256, 2, 1, 4, 128, 3, 1, 8), (256, 256, 2, 1, 4, 256, 2, 1, 4)]
 
 
 @pytest.mark.parametrize("plan", _MOE_PLANS)

@@ -11,7 +11,8 @@ from distributed_llm_amd.ops import reference as ref
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 PLANS = [(64, 64, 3, 1, 1, 4), (64, 64, 3, 1, 2, 4, 1, 0, 0, 64, 32), (64, 64, 3, 2, 1, 4), (128, 128, 3, 1, 1, 8), (192, 128, 3, 1, 1, 8),
-         (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 2), (256, 256, 2, 1, 1, 8, 1, 0, 0, 64, 16, 8), (256, 256, 4, 1, 1, 8, 1, 0, 0, 32)]
+         (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 2), (256, 256, 2, 1, 1, 8, 1, 0, 0, 64, 16, 8), (256, 256, 4, 1, 1, 8, 1, 0, 0, 32),
+         (256, 256, 2, 1, 1, 4), (256, 256, 2, 1, 1, 4, 1, 0, 0, 64, 16, 8)]
 
 
 def _slots(kind, M):
