@@ -75,6 +75,24 @@ def test_untimed_tiles(monkeypatch):
     assert tile(2000, 1024, 4096) == (128, 128)
 
 
+def test_expert_tiles(monkeypatch):
+    """Both sides of each line of the rule for an expert layer's tiles: pairs, pairs an expert, CUs that each product's tiles fill."""
+    from distributed_llm_amd import ops
+    monkeypatch.setattr(G._P, "cus", 256)
+
+    def plan(pairs, E, N1, N2):
+        w1, w2 = torch.empty(E, N1, 64, device="meta"), torch.empty(E, N2, N1 // 2, device="meta")
+        return next(k for k, v in ops.MOE_PLANS.items() if v == ops.moe_plan(pairs, w1, w2))
+
+    assert [plan(p, 8, 14336, 4096) for p in (128, 129, 1024, 1025)] == ["decode", "mid", "mid", "wide"]
+    assert ops.moe_plan(5000) == ops.MOE_PLANS["prefill"]      # (no weights: by the pairs alone)
+    assert [plan(p, 64, 2048, 2048) for p in (64 * 128 - 1, 64 * 128)] == ["mid", "wide"]
+    # 8 experts of 1024 x 1024: 17.6 row tiles of the first product's 8 columns are 0.55 of the CUs, 32 of the second's 4 are half
+    assert [plan(p, 8, 2048, 1024) for p in (3481, 3482, 7167, 7168)] == ["mid", "prefill", "prefill", "wide"]
+    monkeypatch.setattr(G._P, "cus", 128)
+    assert [plan(p, 8, 2048, 1024) for p in (3000, 3482)] == ["prefill", "wide"]
+
+
 def _timed(monkeypatch, N, K, us, small):
     """Tables as the autotuner leaves them: a round of 256 tiles of 256 x 256 and of 256 x 128, and plans of small tiles."""
     big, half = (256, 256, 2, 1, 1, 8), (256, 128, 3, 1, 1, 8)
