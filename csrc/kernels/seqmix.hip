@@ -308,6 +308,14 @@ template <> struct vec4<u16> {
 // its own; one row of 1024 4.2 -> 3.6 us).
 __device__ __forceinline__ void here(float4& f) { asm volatile("" : "+v"(f.x), "+v"(f.y), "+v"(f.z), "+v"(f.w)); }
 
+// Here and where two products meet, the one that is fused is named: left to the compiler it was another from form to form, and a row's last
+// bits would hang on the number of rows beside it
+template <int NV>
+__device__ __forceinline__ float squares(const float4& q) {
+  const float xy = NV == 1 ? fmaf(q.y, q.y, q.x * q.x) : fmaf(q.x, q.x, q.y * q.y);
+  return fmaf(q.w, q.w, fmaf(q.z, q.z, xy));
+}
+
 template <typename T, int NV, bool TWO, bool DEPTH>
 __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restrict__ a, long lda, const T* __restrict__ b, long ldb,
                                                               const float* __restrict__ wa, const float* __restrict__ wb,
@@ -363,8 +371,8 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
       const float4 g = weight(bi, bip, j, c);
       y[j].x += g.x; y[j].y += g.y; y[j].z += g.z; y[j].w += g.w;
     }
-    ss += y[j].x * y[j].x + y[j].y * y[j].y + y[j].z * y[j].z + y[j].w * y[j].w;
-    if constexpr (TWO) sb += z[j].x * z[j].x + z[j].y * z[j].y + z[j].z * z[j].z + z[j].w * z[j].w;
+    ss += squares<NV>(y[j]);
+    if constexpr (TWO) sb += squares<NV>(z[j]);
   }
   float ry = 1.f / sqrtf(block_sum(ss, red) / (float)H + eps);
   if constexpr (TWO) {
@@ -375,14 +383,14 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
       const int c = 4 * (j * 256 + (int)threadIdx.x);
       if (c < H) {
         const float4 g = weight(ga, wa, j, c), h = weight(gb, wb, j, c);
-        y[j] = make_float4(y[j].x * ra * g.x + z[j].x * rb * h.x, y[j].y * ra * g.y + z[j].y * rb * h.y,
-                           y[j].z * ra * g.z + z[j].z * rb * h.z, y[j].w * ra * g.w + z[j].w * rb * h.w);
+        y[j] = make_float4(fmaf(y[j].x * ra, g.x, z[j].x * rb * h.x), fmaf(y[j].y * ra, g.y, z[j].y * rb * h.y),
+                           fmaf(y[j].z * ra, g.z, z[j].z * rb * h.z), fmaf(y[j].w * ra, g.w, z[j].w * rb * h.w));
         if (bias) {
           const float4 e = weight(bi, bip, j, c);
           y[j].x += e.x; y[j].y += e.y; y[j].z += e.z; y[j].w += e.w;
         }
       }
-      ss += y[j].x * y[j].x + y[j].y * y[j].y + y[j].z * y[j].z + y[j].w * y[j].w;
+      ss += squares<NV>(y[j]);
     }
     ry = 1.f / sqrtf(block_sum(ss, red) / (float)H + eps);
   }
@@ -413,7 +421,7 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
       }
       if (xn && !w_next) vec4<T>::st(xn + row * (long)H + c, v[j]);
     }
-    ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+    ss += squares<NV>(v[j]);
   }
   if (!xn || !w_next) return;   // uniform
   const float rx = 1.f / sqrtf(block_sum(ss, red) / (float)H + eps);

@@ -238,6 +238,18 @@ def test_resadd_norm(dt, n, pair, aligned):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n", [24, 512, 1024, 1032, 3000])
+def test_mean_of_two_branches_rounds_the_second_product(dt, n):
+    """An epsilon far above the rows makes every norm the same power of two: the update is half of fma(a, wa, b wb), to the bit (products of
+    a bf16 value and a float are whole in a double, and so are their sums but for far apart ones)."""
+    torch.manual_seed(n)
+    a, b = torch.randn(5, n, device=DEV).bfloat16().to(dt), torch.randn(5, n, device=DEV).bfloat16().to(dt)
+    wa, wb, x = torch.rand(n, device=DEV) + 0.5, torch.rand(n, device=DEV) + 0.5, torch.zeros(5, n, device=DEV)
+    seqmix.resadd_norm(a, torch.full((n,), 2.0 ** 60, device=DEV), 2.0 ** 60, x, b=b, wa=wa, wb=wb)
+    assert torch.equal(x, ((a.double() * wa.double() + (b.float() * wb).double()) / 2).float())
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("pair", [False, True])
 def test_resadd_norm_with_depth_average(dt, pair):
     """The layer-ending form: the residual update and the weighted sum over the stack in one launch."""
