@@ -316,7 +316,7 @@ __device__ __forceinline__ float squares(const float4& q) {
   return fmaf(q.w, q.w, fmaf(q.z, q.z, xy));
 }
 
-template <typename T, int NV, bool TWO, bool DEPTH>
+template <typename T, int NV, bool TWO, bool DEPTH, bool EARLY>
 __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restrict__ a, long lda, const T* __restrict__ b, long ldb,
                                                               const float* __restrict__ wa, const float* __restrict__ wb,
                                                               const float* __restrict__ w_post, float* __restrict__ x,
@@ -326,39 +326,40 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
   __shared__ float red[16];
   const long row = blockIdx.x;
   float* xr = x + row * (long)H;
-  constexpr bool EARLY = NV <= 2;      // (longer rows are many registers: 4 vectors 148 with two branches)
   constexpr int NE = EARLY ? NV : 1, NG = EARLY && TWO ? NV : 1;
   float4 y[NV], v[NV], z[TWO ? NV : 1], wp[NE], wn[NE], ga[NG], gb[NG], bi[NE];
   auto weight = [](const float4* early, const float* w, int j, int c) { return EARLY ? early[j] : *reinterpret_cast<const float4*>(w + c); };
   float ss = 0.f, sb = 0.f;
   const float* const wnx = w_next ? w_next : w_post;
   const float* const bip = bias ? bias : w_post;
+  if constexpr (EARLY || NV > 2) {
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {      // (a vector past the row reads the first and is zero)
-    const int c0 = 4 * (j * 256 + (int)threadIdx.x), c = c0 < H ? c0 : 0;
-    y[j] = vec4<T>::ld(a + row * lda + c);
-    if constexpr (TWO) z[j] = vec4<T>::ld(b + row * ldb + c);
-    v[j] = *reinterpret_cast<const float4*>(xr + c);
-    if constexpr (EARLY) {
-      bi[j] = *reinterpret_cast<const float4*>(bip + c);
-      wp[j] = *reinterpret_cast<const float4*>(w_post + c);
-      wn[j] = *reinterpret_cast<const float4*>(wnx + c);
-      if constexpr (TWO) {
-        ga[j] = *reinterpret_cast<const float4*>(wa + c);
-        gb[j] = *reinterpret_cast<const float4*>(wb + c);
+    for (int j = 0; j < NV; ++j) {      // (a vector past the row reads the first and is zero)
+      const int c0 = 4 * (j * 256 + (int)threadIdx.x), c = c0 < H ? c0 : 0;
+      y[j] = vec4<T>::ld(a + row * lda + c);
+      if constexpr (TWO) z[j] = vec4<T>::ld(b + row * ldb + c);
+      v[j] = *reinterpret_cast<const float4*>(xr + c);
+      if constexpr (EARLY) {
+        bi[j] = *reinterpret_cast<const float4*>(bip + c);
+        wp[j] = *reinterpret_cast<const float4*>(w_post + c);
+        wn[j] = *reinterpret_cast<const float4*>(wnx + c);
+        if constexpr (TWO) {
+          ga[j] = *reinterpret_cast<const float4*>(wa + c);
+          gb[j] = *reinterpret_cast<const float4*>(wb + c);
+        }
       }
     }
-  }
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    here(y[j]);
-    here(v[j]);
-    if constexpr (TWO) here(z[j]);
-    if constexpr (EARLY) {
-      here(bi[j]);
-      here(wp[j]);
-      here(wn[j]);
-      if constexpr (TWO) { here(ga[j]); here(gb[j]); }
+    for (int j = 0; j < NV; ++j) {
+      here(y[j]);
+      here(v[j]);
+      if constexpr (TWO) here(z[j]);
+      if constexpr (EARLY) {
+        here(bi[j]);
+        here(wp[j]);
+        here(wn[j]);
+        if constexpr (TWO) { here(ga[j]); here(gb[j]); }
+      }
     }
   }
 #pragma unroll
@@ -367,9 +368,16 @@ __global__ void __launch_bounds__(256) resadd_norm_vec_kernel(const T* __restric
     if (c >= H) {
       y[j] = v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
       if constexpr (TWO) z[j] = y[j];
-    } else if (!TWO && bias) {
-      const float4 g = weight(bi, bip, j, c);
-      y[j].x += g.x; y[j].y += g.y; y[j].z += g.z; y[j].w += g.w;
+    } else {
+      if constexpr (!EARLY && NV <= 2) {
+        y[j] = vec4<T>::ld(a + row * lda + c);
+        if constexpr (TWO) z[j] = vec4<T>::ld(b + row * ldb + c);
+        v[j] = *reinterpret_cast<const float4*>(xr + c);     // in flight under the first sum
+      }
+      if (!TWO && bias) {
+        const float4 g = weight(bi, bip, j, c);
+        y[j].x += g.x; y[j].y += g.y; y[j].z += g.z; y[j].w += g.w;
+      }
     }
     ss += squares<NV>(y[j]);
     if constexpr (TWO) sb += squares<NV>(z[j]);
@@ -1707,13 +1715,21 @@ extern "C" int dllm_resadd_norm(const void* a, long lda, const void* b, long ldb
   if (H % 4 == 0 && H <= 8192 && lda % 4 == 0 && (uintptr_t)a % ab == 0 && f16(x) && f16(w_post) && (!xn || (uintptr_t)xn % ab == 0) &&
       f16(w_next) && f16(bias) && (!b || (ldb % 4 == 0 && (uintptr_t)b % ab == 0 && f16(wa) && f16(wb)))) {
     const int nv = (H + 1023) / 1024;
-#define RN(T, NV, TWO, DEPTH)                                                                                                 \
-  hipLaunchKernelGGL((resadd_norm_vec_kernel<T, NV, TWO, DEPTH>), dim3(rows), dim3(256), 0, st, (const T*)a, lda, (const T*)b, ldb, wa, wb, \
+#define RN(T, NV, TWO, DEPTH, EARLY)                                                                                          \
+  hipLaunchKernelGGL((resadd_norm_vec_kernel<T, NV, TWO, DEPTH, EARLY>), dim3(rows), dim3(256), 0, st, (const T*)a, lda, (const T*)b, ldb, wa, wb, \
                      w_post, x, w_next, (T*)xn, H, eps, bias, dw, dn, (long)rows * H)
-#define RNB(T, NV) do { if (dw) { if (b) RN(T, NV, true, true); else RN(T, NV, false, true); } else { if (b) RN(T, NV, true, false); else RN(T, NV, false, false); } } while (0)
-#define RNT(T) do { if (nv <= 1) RNB(T, 1); else if (nv <= 2) RNB(T, 2); else if (nv <= 4) RNB(T, 4); else RNB(T, 8); } while (0)
+#define RNB(T, NV, EARLY) do { if (dw) { if (b) RN(T, NV, true, true, EARLY); else RN(T, NV, false, true, EARLY); } else { if (b) RN(T, NV, true, false, EARLY); else RN(T, NV, false, false, EARLY); } } while (0)
+#define RNE(T, NV) do { if (early) RNB(T, NV, true); else RNB(T, NV, false); } while (0)
+    // Every weight ahead but where one round of workgroups shares the CUs: there what the threads past a short row load in vain counts (1000
+    // rows, weights ahead / at their use, us: bf16 512 4.2 / 4.0, two branches 5.7 / 5.1, f32 512 5.7 / 5.2), while one or two rows a CU wait for
+    // the loads (100 rows of 2048 3.8 / 4.4) and over many rounds the loads ahead fill the gaps (8000 rows of 1536 bf16 23.7 / 25.7, f32 30.1 / 31.2).
+    // As many vectors as the row has: f32 rows of 5120 with three of eight past the end 5.4 for 5.0
+    const bool early = rows <= 512 || rows > 2048;
+#define RNT(T) do { if (nv <= 1) RNE(T, 1); else if (nv <= 2) RNE(T, 2); else if (nv <= 3) RNB(T, 3, false); else if (nv <= 4) RNB(T, 4, false); \
+                    else if (nv <= 5) RNB(T, 5, false); else if (nv <= 6) RNB(T, 6, false); else RNB(T, 8, false); } while (0)
     if (f32) RNT(float); else RNT(u16);
 #undef RNT
+#undef RNE
 #undef RNB
 #undef RN
     return (int)hipGetLastError();

@@ -238,6 +238,27 @@ def test_resadd_norm(dt, n, pair, aligned):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("R,n", [(512, 512), (513, 512), (2048, 1032), (2049, 1032), (513, 2048), (3, 2052), (3, 3072), (3, 4100), (3, 5120), (3, 6144), (3, 6148)])
+def test_resadd_norm_rows(dt, pair, R, n):
+    """Weights ahead of the sums and at their use, and every number of a thread's vectors."""
+    torch.manual_seed(n)
+    a, b = torch.randn(R, n, device=DEV).to(dt), torch.randn(R, n, device=DEV).to(dt) if pair else None
+    bias, wa, wb, wp, wn = (torch.randn(n, device=DEV) for _ in range(5))
+    kw = dict(b=b, wa=wa, wb=wb) if pair else dict(bias=bias)
+    x1 = torch.randn(R, n, device=DEV)
+    x2, x3, h1, h2 = x1.clone(), x1[:3].clone(), torch.empty_like(a), torch.empty_like(a)
+    few = dict(kw, b=b[:3]) if pair else kw
+    seqmix.resadd_norm(a[:3], wp, 1e-5, x3, wn, h1[:3], **few)
+    h3 = h1[:3].clone()
+    seqmix.resadd_norm(a, wp, 1e-5, x1, wn, h1, **kw)
+    assert torch.equal(x1[:3], x3) and torch.equal(h1[:3], h3)
+    ref.resadd_norm(a, wp, 1e-5, x2, wn, h2, **kw)
+    torch.testing.assert_close(x1, x2, atol=2e-5, rtol=2e-5)
+    torch.testing.assert_close(h1.float(), h2.float(), **tol(dt))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("n", [24, 512, 1024, 1032, 3000])
 def test_mean_of_two_branches_rounds_the_second_product(dt, n):
     """An epsilon far above the rows makes every norm the same power of two: the update is half of fma(a, wa, b wb), to the bit (products of
