@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256) norm_resadd_kernel(const T* __restrict__ 
 // (expert-sorted, TY), in the launch that uses it; a sum of bf16 rows is rounded to bf16 first, as the combine of its own
 // writes it.  Bound by latency at decode: 24 rows of 1024 2.9 us against 3.4 in two passes (of 4096
 // 4.2 against 6.8), 8000 rows 17.5 against 21.2; with the experts' sum 0.9 us more than the combine whose place it takes.
-template <typename T, typename TY, int NE, bool PARTS>
+template <typename T, typename TY, int NE, bool PARTS, bool WIDE>
 __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restrict__ y, long ldy, const float* __restrict__ w,
                                                               float* __restrict__ x, T* __restrict__ xl, int H, float eps,
                                                               int groups, const float* __restrict__ bias,
@@ -183,8 +183,12 @@ __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restri
       for (int e = 0; e < k; ++e) {
         const TY* yr = y + (inv ? (long)inv[row * k + e] : row * k + e) * ldy;
         const float wt = wts[row * k + e];
+        // (opaque: addresses kept from one expert to the next were 160 registers at 32 entries, and 1000 rows of 5120, without experts
+        // too, a second round of workgroups: 20.8 us for 14.8)
+        int c = c0;
+        asm volatile("" : "+v"(c));
 #pragma unroll
-        for (int j = 0; j < NE; ++j) a[j] += wt * ldf(yr + min(c0 + ST * j, c1 - 1));
+        for (int j = 0; j < NE; ++j) a[j] += wt * ldf(yr + min(c + ST * j, c1 - 1));
       }
       if constexpr (sizeof(TY) == 2) {
 #pragma unroll
@@ -212,7 +216,8 @@ __global__ void __launch_bounds__(256) norm_resadd_reg_kernel(const TY* __restri
       if (c >= c1) continue;
       const float v = (EARLY ? s[EARLY ? j : 0] : xr[c]) + a[j] * r * (EARLY ? g[EARLY ? j : 0] : w[c]);
       xr[c] = v;
-      put_lp(xl, xw, row * (long)H + c, v);
+      if constexpr (WIDE) put_lp(xl, xw, row * (long)H + c, v);      // (a row of f32 beside the rounded one; its test in every store cost 4096 wide rows 5 %)
+      else if (xl) stf(xl + row * (long)H + c, v);
     }
     if constexpr (!PARTS) break;
   }
@@ -1658,15 +1663,17 @@ template <typename T, typename TY>
 int norm_resadd_reg(const void* y, long ldy, const float* w, float* x, void* xl, long rows, int H, float eps, int groups,
                     const float* bias, const int* inv, const float* wts, int k, hipStream_t st, float* xw = nullptr) {
   const int e = norm_resadd_entries(H, groups);
-#define NRV(NE, PARTS)                                                                                                                   \
-  hipLaunchKernelGGL((norm_resadd_reg_kernel<T, TY, NE, PARTS>), dim3((unsigned)rows), dim3(256), 0, st, (const TY*)y, ldy, w, x, (T*)xl, H, \
+#define NRVW(NE, PARTS, WIDE)                                                                                                            \
+  hipLaunchKernelGGL((norm_resadd_reg_kernel<T, TY, NE, PARTS, WIDE>), dim3((unsigned)rows), dim3(256), 0, st, (const TY*)y, ldy, w, x, (T*)xl, H, \
                      eps, groups, bias, inv, wts, k, xw)
+#define NRV(NE, PARTS) do { if (xw) NRVW(NE, PARTS, true); else NRVW(NE, PARTS, false); } while (0)
   if (groups == 1) {
     if (e <= 4) NRV(4, false); else if (e <= 8) NRV(8, false); else if (e <= 16) NRV(16, false); else NRV(32, false);
   } else {
     if (e <= 4) NRV(4, true); else if (e <= 8) NRV(8, true); else if (e <= 16) NRV(16, true); else if (e <= 32) NRV(32, true); else NRV(64, true);
   }
 #undef NRV
+#undef NRVW
   return (int)hipGetLastError();
 }
 }  // namespace

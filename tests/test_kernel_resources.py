@@ -5,10 +5,12 @@ harmless-looking refactor (a by-reference lambda around the attention work unit)
 paged-attention instantiation spill 176 B/lane and run ~1.3x slower on MI355X.  This compiles the
 kernels with the flags of the build and ``-Rpass-analysis=kernel-resource-usage`` and fails on any scratch use.
 """
+import functools
 import os
 import re
 import shutil
 import subprocess
+import tempfile
 
 import pytest
 
@@ -26,19 +28,41 @@ KERNELS = ["attention.hip", "gemv.hip", "skinny_gemm.hip", "sampling.hip", "moe.
 ALLOW = {r"flash_prefill_kernelILi64ELi4E": 32}
 
 
+@functools.lru_cache(maxsize=None)
+def _usage(src):
+    path = os.path.join(ROOT, "csrc", "kernels", src)
+    with tempfile.TemporaryDirectory() as tmp:
+        r = subprocess.run([HIPCC, *HIP_FLAGS, "-I", os.path.dirname(path), "-c", path, "-o", os.path.join(tmp, "k.o"),
+                            "-Rpass-analysis=kernel-resource-usage"], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return r.stderr
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 @pytest.mark.parametrize("src", KERNELS)
-def test_no_scratch_spills(src, tmp_path):
-    path = os.path.join(ROOT, "csrc", "kernels", src)
-    r = subprocess.run([HIPCC, *HIP_FLAGS, "-I", os.path.dirname(path), "-c", path, "-o", str(tmp_path / "k.o"), "-Rpass-analysis=kernel-resource-usage"],
-                       capture_output=True, text=True, timeout=600)
-    assert r.returncode == 0, r.stderr[-2000:]
-    names = re.findall(r"Function Name: (\S+)", r.stderr)
-    scratch = [int(x) for x in re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", r.stderr)]
+def test_no_scratch_spills(src):
+    out = _usage(src)
+    names = re.findall(r"Function Name: (\S+)", out)
+    scratch = [int(x) for x in re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", out)]
     assert names and len(names) == len(scratch)
     budget = lambda n: max([v for k, v in ALLOW.items() if re.search(k, n)] or [0])
     spilled = [(n, s) for n, s in zip(names, scratch) if s > budget(n)]
     assert not spilled, f"scratch spills: {spilled}"
+
+
+# What a wave may hold of the registers, where one workgroup more or less on a CU is a round of the launch: (source, kernel, waves a SIMD)
+WAVES = [
+    ("seqmix.hip", r"norm_resadd_reg_kernelI\w\wLi(16|32)E", 4),      # 1000 rows of 5120: 15 us, 21 with three
+    ("seqmix.hip", r"norm_resadd_reg_kernelI\w\wLi64E", 2),
+]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+@pytest.mark.parametrize("src,kernel,waves", WAVES)
+def test_waves_of_a_simd(src, kernel, waves):
+    out = _usage(src)
+    got = {n: int(w) for n, w in re.findall(r"Function Name: (\S+).*?Occupancy \[waves/SIMD\]: (\d+)", out, re.S) if re.search(kernel, n)}
+    assert got and min(got.values()) >= waves, got
 
 
 def _registers(operand):
