@@ -38,7 +38,7 @@ __device__ __forceinline__ float logsigmoid_f(float x) { return x < 0.f ? x - lo
 // MLSTM = false: ssd_scan; true: mlstm.  NPT >= ceil(N / strips); the staged k / q rows are padded with
 // zeros to NPT * strips entries, so the walk over a thread's state rows has no bounds test (rows past
 // N stay zero) and its LDS reads (k and q of a row side by side, 8 bytes) can be issued together.
-template <typename T, bool MLSTM, int NPT>
+template <typename T, bool MLSTM, int NPT, bool AHEAD>
 __global__ void __launch_bounds__(256) outer_scan_kernel(const T* __restrict__ kq, long ld_kq, int k_off, int q_off, int kq_heads_div,
                                                          const T* __restrict__ vsrc, long ld_v, int v_off,
                                                          const T* __restrict__ gsrc, long ld_g, int g_off, int g_off2,
@@ -107,22 +107,39 @@ __global__ void __launch_bounds__(256) outer_scan_kernel(const T* __restrict__ k
     if (MLSTM) m = np[N];
   }
   const float hp0 = p0v ? p0v[h] : 0.f, hp1 = p1v ? p1v[h] : 0.f, hp2 = p2v ? p2v[h] : 0.f;
-  fetch(0);
+  if constexpr (AHEAD) fetch(0);
 #pragma unroll
   for (int k = 0; k < NPT; ++k) S[k] = col_ok & (strip + k * STRIPS < N) ? S[k] : 0.f;
   for (int t0 = 0; t0 < n_new; t0 += OS_TG) {
     const int nt = min(OS_TG, n_new - t0);
     __syncthreads();     // the previous group's sums are stored
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int i = 0; i < EK; ++i) {
-      const int e = tid + 256 * i;
-      const bool on = e % NP < N;
-      if (e < OS_TG * NP) KQ[e] = make_float2(on ? ldf(&fk[i]) : 0.f, on ? ldf(&fq[i]) * qscale : 0.f);
-    }
+      for (int i = 0; i < EK; ++i) {
+        const int e = tid + 256 * i;
+        const bool on = e % NP < N;
+        if (e < OS_TG * NP) KQ[e] = make_float2(on ? ldf(&fk[i]) : 0.f, on ? ldf(&fq[i]) * qscale : 0.f);
+      }
 #pragma unroll
-    for (int i = 0; i < EV; ++i) {
-      const int e = tid + 256 * i, cc = e % CW;
-      if (e < OS_TG * CW) Vs[e] = MLSTM && cc == OS_COLS ? 1.f : v0 + cc < dv ? ldf(&fv[i]) : 0.f;
+      for (int i = 0; i < EV; ++i) {
+        const int e = tid + 256 * i, cc = e % CW;
+        if (e < OS_TG * CW) Vs[e] = MLSTM && cc == OS_COLS ? 1.f : v0 + cc < dv ? ldf(&fv[i]) : 0.f;
+      }
+    } else {
+      for (int e = tid; e < nt * NP; e += 256) {
+        const int t = e / NP, n = e % NP;
+        const T* r = kq + (long)(q0 + t0 + t) * ld_kq + (long)kh * N + n;
+        KQ[e] = n < N ? make_float2(ldf(r + k_off), ldf(r + q_off) * qscale) : make_float2(0.f, 0.f);
+      }
+      for (int e = tid; e < nt * CW; e += 256) {
+        const int t = e / CW, cc = e % CW;
+        Vs[e] = MLSTM && cc == OS_COLS ? 1.f : v0 + cc < dv ? ldf(vsrc + (long)(q0 + t0 + t) * ld_v + v_off + (long)h * dv + v0 + cc) : 0.f;
+      }
+      if (tid < nt) {
+        const T* g = gsrc + (long)(q0 + t0 + tid) * ld_g;
+        fa = g[g_off + h];
+        if constexpr (MLSTM) fb = g[g_off2 + h];
+      }
     }
     if (tid < nt) {
       if (MLSTM) {
@@ -136,7 +153,8 @@ __global__ void __launch_bounds__(256) outer_scan_kernel(const T* __restrict__ k
         Gb[tid] = dt;
       }
     }
-    if (t0 + OS_TG < n_new) fetch(t0 + OS_TG);
+    if constexpr (AHEAD)
+      if (t0 + OS_TG < n_new) fetch(t0 + OS_TG);
     __syncthreads();
     if (live) {
       for (int t = 0; t < nt; ++t) {
@@ -274,11 +292,23 @@ int launch_outer(dim3 grid, long lds, hipStream_t st, const void* kq, long ld_kq
                  long ld_v, int v_off, const void* g, long ld_g, int g_off, int g_off2, const float* p0, const float* p1,
                  const float* p2, float cap, float qscale, float* state, float* nm, int NCB, const int* qstart,
                  const int* qlen, const int* ctx, const int* rows, float* out, int H, int N, int dv) {
-  ENSURE_LDS((outer_scan_kernel<T, MLSTM, NPT>), lds);
-  hipLaunchKernelGGL((outer_scan_kernel<T, MLSTM, NPT>), grid, dim3(256), lds, st, (const T*)kq, ld_kq, k_off, q_off, kdiv,
-                     (const T*)v, ld_v, v_off, (const T*)g, ld_g, g_off, g_off2, p0, p1, p2, cap, qscale, state, nm, NCB,
-                     qstart, qlen, ctx, rows, out, H, N, dv);
-  return (int)hipGetLastError();
+#define OUTER(AHEAD)                                                                                                              \
+  do {                                                                                                                            \
+    ENSURE_LDS((outer_scan_kernel<T, MLSTM, NPT, AHEAD>), lds);                                                                   \
+    hipLaunchKernelGGL((outer_scan_kernel<T, MLSTM, NPT, AHEAD>), grid, dim3(256), lds, st, (const T*)kq, ld_kq, k_off, q_off, kdiv, \
+                       (const T*)v, ld_v, v_off, (const T*)g, ld_g, g_off, g_off2, p0, p1, p2, cap, qscale, state, nm, NCB,       \
+                       qstart, qlen, ctx, rows, out, H, N, dv);                                                                   \
+    return (int)hipGetLastError();                                                                                                \
+  } while (0)
+  // With the longest rows and their inputs a group ahead a workgroup's registers fill its CU: workgroups that are not the only one of
+  // a CU load where they stage (mLSTM, 8 heads of 480 x 64, us ahead / not: 16 sequences of 33 tokens (512 workgroups) 87 / 66, 3 of 200 to 600 592 / 858)
+  if constexpr (MLSTM && NPT > 24) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -3;
+    if ((long)grid.x * grid.y * grid.z > cus) OUTER(false);
+  }
+  OUTER(true);
+#undef OUTER
 }
 
 template <typename T, bool MLSTM, typename... A>

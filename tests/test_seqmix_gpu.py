@@ -529,6 +529,28 @@ def test_mlstm(dt, case, H, d, dv):
     torch.testing.assert_close(nm1, nm2, atol=2e-4, rtol=2e-4)
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,d,dv", [(8, 480, 64), (5, 400, 96)])
+def test_mlstm_long_rows_of_many_sequences(dt, H, d, dv):
+    """More workgroups than CUs load their inputs where they stage them: the bits of each sequence by itself, a group ahead."""
+    torch.manual_seed(d)
+    qlens, starts = [9, 1, 17, 0, 8, 5, 2, 16] * 4, [0, 3] * 16
+    T, qstart, qlen, ctx, rows, _ = batch(qlens, starts)
+    assert H * len(qlens) * seqmix.scan_col_blocks(dv) > torch.cuda.get_device_properties(0).multi_processor_count
+    proj = torch.randn(T, 2 * H * (d + dv + 1), device=DEV).to(dt)
+    gate_b, w = torch.randn(2 * H, device=DEV), torch.rand(H * dv, device=DEV) + 0.5
+    s1 = torch.randn(len(qlens), H, d, dv, device=DEV)
+    nm1 = torch.randn(len(qlens), H, 1, d + 1, device=DEV).repeat(1, 1, seqmix.scan_col_blocks(dv), 1).contiguous()
+    s2, nm2 = s1.clone(), nm1.clone()
+    got = seqmix.mlstm(proj, H, d, dv, gate_b, 3.0, s1, nm1, 1e-5, w, qstart, qlen, ctx, rows, chunked=False)
+    for i, n in enumerate(qlens):
+        if n:
+            o = seqmix.mlstm(proj, H, d, dv, gate_b, 3.0, s2, nm2, 1e-5, w, qstart[i:i + 1], qlen[i:i + 1], ctx[i:i + 1], rows[i:i + 1], chunked=False)
+            t = int(qstart[i])
+            assert torch.equal(o[t:t + n], got[t:t + n])
+    assert torch.equal(s1, s2) and torch.equal(nm1, nm2)
+
+
 @pytest.mark.parametrize("case", CASES + [([200, 63, 1, 64], [0, 5, 9, 130]), ([129, 128], [0, 7])])
 @pytest.mark.parametrize("H,d,dv", [(4, 40, 48), (3, 64, 8), (2, 128, 128), (1, 8, 72), (2, 96, 40)])
 @pytest.mark.parametrize("cap,gain", [(3.0, 4.0), (15.0, 8.0), (6.0, 0.5)])
