@@ -137,11 +137,13 @@ enum { ENC_PLAIN = 0, ENC_RESADD = 1, ENC_QKV = 2, ENC_GELU = 4 };
 template <typename F>
 __device__ __forceinline__ void arrived(F& f) { asm volatile("" : "+v"(f)); }
 
-template <int MT, int NW, int EPI>
+// KS k-steps of a wave at a time, so many that a wave's come out even where that can be (loads that do not exist are taken from those that do:
+// 1024 -> 1024 columns on 64 rows, 16 waves of 2 steps, 9.4 us three at a time, 7.3)
+template <int MT, int NW, int EPI, int KS>
 __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict__ X, long ldx, const u16* __restrict__ W,
                                                            const u16* __restrict__ bias, u16* __restrict__ Y, long ldy, int M, int N,
                                                            int K) {
-  constexpr int KS = 3, RS = 20;      // 384 = 4 waves of 3 steps, 1536 = 16 of 3; LDS rows of 16 + 4 floats reach every bank
+  constexpr int RS = 20;      // LDS rows of 16 + 4 floats reach every bank
   __shared__ __attribute__((aligned(16))) float red[NW][MT * 16][RS];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.x * 16;
@@ -197,14 +199,23 @@ __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict
   *reinterpret_cast<u16x4*>(Y + (long)row * ldy + col0 + c) = o;
 }
 
-template <int MT, int NW>
+template <int MT, int NW, int KS>
 int launch_enc_gemm(const u16* x, long ldx, const u16* w, const u16* bias, u16* y, long ldy, int M, int N, int K, int epi, hipStream_t st) {
   const dim3 g(N / 16), b(64 * NW);
-  if (epi == ENC_PLAIN) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_PLAIN>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
-  else if (epi == ENC_RESADD) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_RESADD>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
-  else if (epi == ENC_GELU) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_GELU>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
+  if (epi == ENC_PLAIN) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_PLAIN, KS>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
+  else if (epi == ENC_RESADD) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_RESADD, KS>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
+  else if (epi == ENC_GELU) hipLaunchKernelGGL((enc_gemm_kernel<MT, NW, ENC_GELU, KS>), g, b, 0, st, x, ldx, w, bias, y, ldy, M, N, K);
   else return -1;
   return (int)hipGetLastError();
+}
+
+template <int MT, int NW>
+int launch_enc_gemm(const u16* x, long ldx, const u16* w, const u16* bias, u16* y, long ldy, int M, int N, int K, int epi, hipStream_t st) {
+  const int per = (K / 32 + NW - 1) / NW;      // k-steps a wave: 3 of 384 and 1536 columns
+  if (per % 3 == 0) return launch_enc_gemm<MT, NW, 3>(x, ldx, w, bias, y, ldy, M, N, K, epi, st);
+  if (per % 4 == 0) return launch_enc_gemm<MT, NW, 4>(x, ldx, w, bias, y, ldy, M, N, K, epi, st);
+  if (per % 2 == 0) return launch_enc_gemm<MT, NW, 2>(x, ldx, w, bias, y, ldy, M, N, K, epi, st);
+  return launch_enc_gemm<MT, NW, 3>(x, ldx, w, bias, y, ldy, M, N, K, epi, st);
 }
 
 // ---- whole layers of up to 16 rows (H <= 384) in four launches instead of seven: [LayerNorm +] QKV, attention + output + residual,

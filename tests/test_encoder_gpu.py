@@ -149,6 +149,13 @@ def test_few_row_projections(M, N, K):
     assert not ext.enc_gemm(_b(65, K), w, bias, _b(65, N), 0) and not ext.enc_gemm(x, _b(N + 8, K), _b(N + 8), _b(M, N + 8), 0)
 
 
+@pytest.mark.parametrize("M", [3, 16, 40, 64])
+@pytest.mark.parametrize("K", [128, 256, 448, 512, 896, 1024, 1280, 2048, 3072, 4096])
+def test_k_steps_at_a_time(M, K):
+    """Two, three and four k-steps of a wave at a time."""
+    test_few_row_projections(M, 48, K)
+
+
 @pytest.mark.parametrize("lens", [[1], [15], [16], [17], [9, 7], [1] * 16, [1, 0, 12]])
 @pytest.mark.parametrize("nh,d,inter", [(12, 32, 1536), (6, 64, 320), (3, 64, 96), (1, 32, 32), (5, 32, 64), (3, 64, 128), (2, 32, 64), (10, 32, 704),
                                         (1, 64, 64)])      # (widths that are no whole 64s take one launch an operation)
