@@ -20,6 +20,8 @@
 // all of its K range of X in fragments, and X . X^T's diagonal, one more MFMA per fragment, is the rows' sums of squares.
 // GLU and GELU are the activations of layer-list feed-forwards, on the rounded product as their own launches do them (a launch of its
 // own: 3.4 us and the gap before it).  QKV, SWIGLU and GLU weights are stored with the halves of a pair 8 columns apart in one tile (frag_weight).
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -75,8 +77,10 @@ struct Dg {
   static constexpr int LDS = WV * REG + (SQ ? WV * MR * 4 : MR * (NC / 4) * 4) + 16;
 };
 
-// ONE: a wave's K is one stage (a second one, all out of range, cost the products of a 1024-wide layer 3 %)
-template <int MT, int NT, int VS, int EPI, bool ONE>
+// HALVES: a wave's K is that many half stages or fewer (0: any number, two stages at a time).  A step that does not exist is no traffic to
+// memory but passes through the caches' pipe like any other: two stages for waves of three steps cost 16 rows of 11264 x 768 in two splits
+// 8.2 us for 6.6.  (As ways through one kernel the forms cost it registers, and a fourth of its waves.)
+template <int MT, int NT, int VS, int EPI, int HALVES>
 __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   using C = Dg<MT, NT, VS, EPI>;
   constexpr int NC = C::NC, MR = C::MR, LD = C::LD, U = C::U, WV = C::WV, T = C::T, NI = C::NI, PX = C::PX;
@@ -140,7 +144,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   // rows: 11264 x 2048 SwiGLU 13.0 -> 11.8, 2560 x 2048 QKV 8.4 -> 7.6, 2048 x 2048 6.8 -> 6.6, 2048 x 5632 10.2 -> 10.1; 16 rows 10.3 -> 9.8, 6.0 -> 5.7,
   // 8.9 -> 8.6 (the last).  Three stages of two steps: 12.3, 7.7, 6.9, 10.0.
   struct Stage { bf16x8 w[U][NT]; uint4 x[U * MT]; };
-  auto load = [&](Stage& st, int k0) {
+  auto load = [&](Stage& st, int k0, auto cnt) {      // the first cnt steps of a stage
     keep_order();
     const unsigned wo = (unsigned)(k0 * 32 + lane * 16), xo = k0 < wk1 ? x0 + (unsigned)k0 * 2 : 0x40000000u;
     if constexpr (XL) {
@@ -150,20 +154,20 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
     }
     keep_order();
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < cnt.value; ++u) {
 #pragma unroll
       for (int n = 0; n < NT; ++n) st.w[u][n] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wt[n], wo + u * 1024, 0, 2));
       if constexpr (!XL) st.x[u] = ldb16(xb, xo + u * 64);
     }
     keep_order();
   };
-  auto compute = [&](const Stage& st, int cnt) {
+  auto compute = [&](const Stage& st, int cnt, auto most) {
     if constexpr (XL) {
 #pragma unroll
       for (int i = 0; i < U * MT; ++i) *reinterpret_cast<uint4*>(mine + (RPI * i + xr) * PX + xc * 16) = st.x[i];
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < most.value; ++u)
       if (u < cnt) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -176,35 +180,50 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
         }
       }
   };
-  const int steps = (wk1 - wk0) / 32;
-  Stage A, B;
-  load(A, wk0);
-  if constexpr (!ONE) load(B, wk0 + 32 * U);
   float4 e_co[EPI == DG_QKV ? NI : 1], e_si[EPI == DG_QKV ? NI : 1];
-  if constexpr (EPI == DG_QKV) {
-    const int hd = a.d / 2, qk = (a.nq + a.nkv) * a.d;
+  auto angles = [&] {      // behind the first weights
+    if constexpr (EPI == DG_QKV) {
+      const int hd = a.d / 2, qk = (a.nq + a.nkv) * a.d;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int it = (threadIdx.x + i * T) % IPR, t16 = tile * NT + it / 2, cb = (t16 >> 1) * 32;
-      if (cb < qk) {
-        const int d1 = 16 * ((cb % a.d) >> 5) + 8 * (t16 & 1) + 4 * (it & 1);
-        const float* cs = a.cos_sin + (long)e_pos[i] * a.d + d1;
-        e_co[i] = *reinterpret_cast<const float4*>(cs);
-        e_si[i] = *reinterpret_cast<const float4*>(cs + hd);
+      for (int i = 0; i < NI; ++i) {
+        const int it = (threadIdx.x + i * T) % IPR, t16 = tile * NT + it / 2, cb = (t16 >> 1) * 32;
+        if (cb < qk) {
+          const int d1 = 16 * ((cb % a.d) >> 5) + 8 * (t16 & 1) + 4 * (it & 1);
+          const float* cs = a.cos_sin + (long)e_pos[i] * a.d + d1;
+          e_co[i] = *reinterpret_cast<const float4*>(cs);
+          e_si[i] = *reinterpret_cast<const float4*>(cs + hd);
+        }
       }
     }
-  }
-  int i = 0;
-  if constexpr (!ONE) {
-    for (; i + 2 * U < steps; i += 2 * U) {
-      compute(A, U);
-      load(A, wk0 + (i + 2 * U) * 32);
-      compute(B, U);
-      load(B, wk0 + (i + 3 * U) * 32);
+  };
+  const int steps = (wk1 - wk0) / 32;
+  constexpr std::integral_constant<int, U> whole{};
+  constexpr std::integral_constant<int, U / 2> half{};
+  if (steps <= 0) {      // a wave without k: a group past the last split
+    angles();
+  } else {
+    Stage A, B;
+    if constexpr (HALVES == 1) load(A, wk0, half);
+    else load(A, wk0, whole);
+    if constexpr (HALVES == 3) load(B, wk0 + 32 * U, half);
+    if constexpr (HALVES == 0) load(B, wk0 + 32 * U, whole);
+    angles();
+    if constexpr (HALVES == 0) {
+      int i = 0;
+      for (; i + 2 * U < steps; i += 2 * U) {
+        compute(A, U, whole);
+        load(A, wk0 + (i + 2 * U) * 32, whole);
+        compute(B, U, whole);
+        load(B, wk0 + (i + 3 * U) * 32, whole);
+      }
+      if (steps > i) compute(A, steps - i, whole);
+      if (steps > i + U) compute(B, steps - i - U, whole);
+    } else {
+      if constexpr (HALVES == 1) compute(A, steps, half);
+      else compute(A, steps, whole);
+      if constexpr (HALVES == 3) compute(B, steps - U, half);
     }
   }
-  if (steps > i) compute(A, steps - i);
-  if (!ONE && steps > i + U) compute(B, steps - i - U);
 
   // ---- the waves' partial tiles meet in LDS (each wave's own piece: its staged rows are read).  acc[m][n][r] = C[16m + 4g + r][16n + r16]
   float* pt = reinterpret_cast<float*>(mine);
@@ -411,18 +430,27 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
   }
 }
 
-template <int MT, int NT, int VS, int EPI, bool ONE = false>
-int launch(const DgArgs& a, int gy, hipStream_t st) {
+template <int MT, int NT, int VS, int EPI, int HALVES>
+int launch_as(const DgArgs& a, int gy, hipStream_t st) {
   using C = Dg<MT, NT, VS, EPI>;
   static_assert(C::LDS <= 160 * 1024, "LDS of a workgroup");
-  if constexpr (VS == 4 && !ONE)
-    if (a.kchunk <= 128 * C::U) return launch<MT, NT, VS, EPI, true>(a, gy, st);
   static const int rc = C::LDS <= 64 * 1024 ? 0      // raised once: no attribute call inside a later stream capture
-                            : (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI, ONE>,
+                            : (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI, HALVES>,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
   if (rc) return rc;
-  hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, ONE>), dim3((a.N + C::NC - 1) / C::NC, gy), dim3(C::T), C::LDS, st, a);
+  hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, HALVES>), dim3((a.N + C::NC - 1) / C::NC, gy), dim3(C::T), C::LDS, st, a);
   return (int)hipGetLastError();
+}
+
+template <int MT, int NT, int VS, int EPI>
+int launch(const DgArgs& a, int gy, hipStream_t st) {
+  constexpr int H = Dg<MT, NT, VS, EPI>::U / 2;
+  switch ((((a.kchunk + 3) / 4 + 31) / 32 + H - 1) / H) {      // half stages of the longest wave
+    case 1: return launch_as<MT, NT, VS, EPI, 1>(a, gy, st);
+    case 2: return launch_as<MT, NT, VS, EPI, 2>(a, gy, st);
+    case 3: return launch_as<MT, NT, VS, EPI, 3>(a, gy, st);
+    default: return launch_as<MT, NT, VS, EPI, 0>(a, gy, st);
+  }
 }
 
 template <int MT, int EPI>

@@ -167,3 +167,13 @@ def test_f32_rows(M, N, K):
     assert (err <= bound).all()
     got = G.f32_linear(x, wf, N, gelu=True).double()
     assert ((got - torch.nn.functional.gelu(want)).abs() <= 1.13 * bound + 4 * 2.0 ** -24 * (want.abs() + 1)).all()
+
+
+@pytest.mark.parametrize("plan", [(1, 1, 1), (3, 1, 1), (1, 2, 2), (1, 4, 4), (2, 2, 3), (1, 4, 3)])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 17])
+def test_stages_of_a_wave(plan, steps):
+    """One to three half stages have a form each, longer waves walk: on both sides of every line, with whole steps for all four waves of a
+    group, one more and one less."""
+    for M in (4, 24):
+        for K in (128 * steps * plan[2], 128 * steps * plan[2] + 32, 128 * steps * plan[2] - 32):
+            test_plain(M, plan, 48, K)
