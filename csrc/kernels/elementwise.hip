@@ -248,11 +248,13 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
     for (int y = 0; y < EB; ++y)
 #pragma unroll
       for (int c = 0; c < XC; ++c) wr[y][c] = ld16(wg + (long)min(e0 + y, E - 1) * H + 8 * min(lane + 64 * c, nc - 1));
+    if (nc < 64 * XC) {      // (uniform)
 #pragma unroll
-    for (int c = 0; c < XC; ++c)
-      if (lane + 64 * c >= nc)
+      for (int c = 0; c < XC; ++c)
+        if (lane + 64 * c >= nc)
 #pragma unroll
-        for (int y = 0; y < EB; ++y) wr[y][c] = make_uint4(0u, 0u, 0u, 0u);
+          for (int y = 0; y < EB; ++y) wr[y][c] = make_uint4(0u, 0u, 0u, 0u);
+    }
     float s[EB];
 #pragma unroll
     for (int x = 0; x < EB; ++x) {
@@ -427,10 +429,17 @@ extern "C" int dllm_moe_router(const void* x, long x_stride, const void* wg, int
       hipLaunchKernelGGL((moe_router_kernel<XC, EB, false>), grid, block, 0, stream, (const u16*)x, x_stride, (const u16*)wg, T, E, H, k, \
                          ids, w, logits, shared, scale, nullptr, 0.f, nullptr);                                                 \
   } while (0)
-  if (nc <= 128) ROUTER(2, 8);
-  else if (nc <= 256) ROUTER(4, 4);
-  else if (nc <= 512) ROUTER(8, 2);
-  else ROUTER(16, 2);
+  switch ((nc + 63) / 64) {      // (as many chunks a lane as the row has: none is loaded for nothing but in the last)
+    case 1: ROUTER(1, 8); break;
+    case 2: ROUTER(2, 8); break;
+    case 3: ROUTER(3, 4); break;
+    case 4: ROUTER(4, 4); break;
+    case 5: ROUTER(5, 2); break;
+    case 6: ROUTER(6, 2); break;
+    case 7: case 8: ROUTER(8, 2); break;
+    case 9: case 10: case 11: case 12: ROUTER(12, 2); break;
+    default: ROUTER(16, 2);
+  }
 #undef ROUTER
   return (int)hipGetLastError();
 }

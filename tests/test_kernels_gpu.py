@@ -502,6 +502,12 @@ def test_moe_router_matches_fp32_and_is_batch_invariant(H, E, k):
         assert torch.equal(i2, ids[:n]) and torch.equal(w2, w[:n])
 
 
+@pytest.mark.parametrize("H", [8, 504, 512, 520, 1024, 1032, 1536, 1544, 2056, 2560, 3072, 3080, 4104, 6144, 6152])
+def test_moe_router_widths(H):
+    """As many chunks a lane as the row has, full and not."""
+    test_moe_router_matches_fp32_and_is_batch_invariant(H, 8, 2)
+
+
 @pytest.mark.parametrize("T", [5, 700, 1500])
 def test_moe_ffn_grouped_bitwise_repeatable(T):
     """Routing places pairs in a stable order (no atomic arrival order), so repeated calls on the
