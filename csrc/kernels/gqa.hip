@@ -776,9 +776,10 @@ typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 constexpr float CAP_MAX = 64.f;
 // DIST: the scores fall with the distance (`slopes`); the score accumulators start at -slope * distance.
 // Up to 64-wide heads four workgroups fit a CU's LDS, and its registers if a wave keeps to 128 (6 sequences of 7300 tokens, 32 / 8 heads:
-// 266 us with three, 232 with four).
+// 266 us with three, 232 with four).  Up to 192 two must: left alone 192-wide heads took the registers of one (24 decode rows, 8 / 2 heads, 20.0 us
+// for 14.2; 3000 tokens under a window of 512 59.6 for 38.8).
 template <int KD, int VD, bool CAP, bool DIST>
-__global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(const u16* __restrict__ q, const u16* __restrict__ kc,
+__global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 192 ? 2 : 1) paged_gqa_mfma_kernel(const u16* __restrict__ q, const u16* __restrict__ kc,
                                                              const u16* __restrict__ vc, const int* __restrict__ bt,
                                                              int bt_ld, const int* __restrict__ qstart,
                                                              const int* __restrict__ qlen, const int* __restrict__ ctx,
@@ -1089,7 +1090,7 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : 1) paged_gqa_mfma_kernel(c
 // above.  With splits 16, merge included: four sequences of 1300, 8 heads of 64 with slopes 19 -> 13 us; six of 2600, 8 splits 28 -> 19.
 // More than 16 rows (a tile of a short portion) are walked 16 at a time.
 template <int KD, int VD, bool CAP, bool DIST>
-__global__ void __launch_bounds__(256) gqa_few_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
+__global__ void __launch_bounds__(256, 2) gqa_few_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
                                                       const int* __restrict__ bt, int bt_ld, const int* __restrict__ qstart,
                                                       const int* __restrict__ qlen, const int* __restrict__ ctx,
                                                       const int* __restrict__ tile_seq, const int* __restrict__ tile_tok0,

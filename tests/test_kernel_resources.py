@@ -54,6 +54,9 @@ def test_no_scratch_spills(src):
 WAVES = [
     ("seqmix.hip", r"norm_resadd_reg_kernelI\w\wLi(16|32)E", 4),      # 1000 rows of 5120: 15 us, 21 with three
     ("seqmix.hip", r"norm_resadd_reg_kernelI\w\wLi64E", 2),
+    ("gqa.hip", r"paged_gqa_mfma_kernelILi(128|192)E", 2),      # 24 decode rows of 192-wide heads: 14 us, 20 with one
+    ("gqa.hip", r"paged_gqa_mfma_kernelILi96E", 3),
+    ("gqa.hip", r"gqa_few_kernel", 2),
 ]
 
 
