@@ -431,26 +431,27 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
 }
 
 template <int MT, int NT, int VS, int EPI, int HALVES>
-int launch_as(const DgArgs& a, int gy, hipStream_t st) {
-  using C = Dg<MT, NT, VS, EPI>;
-  static_assert(C::LDS <= 160 * 1024, "LDS of a workgroup");
-  static const int rc = C::LDS <= 64 * 1024 ? 0      // raised once: no attribute call inside a later stream capture
-                            : (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI, HALVES>,
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-  if (rc) return rc;
-  hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, HALVES>), dim3((a.N + C::NC - 1) / C::NC, gy), dim3(C::T), C::LDS, st, a);
-  return (int)hipGetLastError();
+int raise_lds() {
+  return (int)hipFuncSetAttribute((const void*)dgemm_kernel<MT, NT, VS, EPI, HALVES>, hipFuncAttributeMaxDynamicSharedMemorySize, Dg<MT, NT, VS, EPI>::LDS);
 }
 
 template <int MT, int NT, int VS, int EPI>
 int launch(const DgArgs& a, int gy, hipStream_t st) {
-  constexpr int H = Dg<MT, NT, VS, EPI>::U / 2;
+  using C = Dg<MT, NT, VS, EPI>;
+  static_assert(C::LDS <= 160 * 1024, "LDS of a workgroup");
+  // raised once, for every length of K: no attribute call inside a later stream capture
+  static const int rc = C::LDS <= 64 * 1024 ? 0 : raise_lds<MT, NT, VS, EPI, 0>() | raise_lds<MT, NT, VS, EPI, 1>() |
+                                                      raise_lds<MT, NT, VS, EPI, 2>() | raise_lds<MT, NT, VS, EPI, 3>();
+  if (rc) return rc;
+  const dim3 grid((a.N + C::NC - 1) / C::NC, gy);
+  constexpr int H = C::U / 2;
   switch ((((a.kchunk + 3) / 4 + 31) / 32 + H - 1) / H) {      // half stages of the longest wave
-    case 1: return launch_as<MT, NT, VS, EPI, 1>(a, gy, st);
-    case 2: return launch_as<MT, NT, VS, EPI, 2>(a, gy, st);
-    case 3: return launch_as<MT, NT, VS, EPI, 3>(a, gy, st);
-    default: return launch_as<MT, NT, VS, EPI, 0>(a, gy, st);
+    case 1: hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, 1>), grid, dim3(C::T), C::LDS, st, a); break;
+    case 2: hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, 2>), grid, dim3(C::T), C::LDS, st, a); break;
+    case 3: hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, 3>), grid, dim3(C::T), C::LDS, st, a); break;
+    default: hipLaunchKernelGGL((dgemm_kernel<MT, NT, VS, EPI, 0>), grid, dim3(C::T), C::LDS, st, a);
   }
+  return (int)hipGetLastError();
 }
 
 template <int MT, int EPI>
