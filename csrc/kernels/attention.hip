@@ -209,6 +209,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
       mloc = lane_max(mloc, 32);
       const float m_new = fmaxf(m_run, mloc);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+      // (the instruction by itself, here and below: weights under 2^-126 become zero, which no f32 sum beside a weight of 1 would show)
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);
       float lsum = 0.f;
 #pragma unroll
