@@ -1076,7 +1076,8 @@ def _timed_with(dev) -> str:
             with open(path, "rb") as f:
                 h.update(f.read())
     p = torch.cuda.get_device_properties(dev)
-    return "%s %s %d %s" % (torch.__version__, p.name, p.multi_processor_count, h.hexdigest())
+    # (not by its name, which is empty under a profiler)
+    return "%s %s %d %s" % (torch.__version__, p.gcnArchName, p.multi_processor_count, h.hexdigest())
 
 
 def _load_plans(path: str, timed_with: Optional[str] = None) -> None:

@@ -280,7 +280,8 @@ def test_plan_file_of_other_code(monkeypatch, tmp_path):
     import json
     from types import SimpleNamespace
     _none_timed(monkeypatch)
-    cards = {0: SimpleNamespace(name="A", multi_processor_count=256), 1: SimpleNamespace(name="A", multi_processor_count=64)}
+    card = lambda name, cus: SimpleNamespace(name=name, gcnArchName="gfx950", multi_processor_count=cus)
+    cards = {0: card("A", 256), 1: card("A", 64), 2: card("", 256)}
     monkeypatch.setattr(torch.cuda, "get_device_properties", lambda d: cards[d])
     built = tmp_path / "kernels.so"
     monkeypatch.setattr(G, "_load_ext", lambda: SimpleNamespace(__file__=str(built)))
@@ -288,7 +289,7 @@ def test_plan_file_of_other_code(monkeypatch, tmp_path):
     for content, card in ((b"one", 0), (b"two", 0), (b"one", 1)):
         built.write_bytes(content)
         made.append(G._timed_with(card))
-    assert len(set(made)) == 3 and built.write_bytes(b"one") and G._timed_with(0) == made[0]
+    assert len(set(made)) == 3 and built.write_bytes(b"one") and G._timed_with(0) == made[0] == G._timed_with(2)      # (a profiler hides the name)
     k, path = (16, 2048, 2048), str(tmp_path / "plans.json")
     G._P.tg_plans[k] = (64, 64, 3, 1, 1, 4)
     G._save_plans(path, made[0])
