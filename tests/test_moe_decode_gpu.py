@@ -48,6 +48,16 @@ def test_bits_of_the_grouped_gemm(mode, T, E, k, H, I, same):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("T", [3, 24])
+@pytest.mark.parametrize("steps", range(1, 14))
+def test_stages_of_a_quarter(mode, T, steps):
+    """A wave's quarter of K ends in a first, second or third stage, whole and not, and the last waves have less of it or none."""
+    for K in (128 * steps, 128 * steps - 64):
+        test_bits_of_the_grouped_gemm(mode, T, 2, 2, K, K, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("T,groups", [(1, 1), (24, 4), (40, 1)])
 def test_sum_ends_in_the_stream(mode, T, groups):
     x, ids, wts, w1, w2, frag, run = _case(T, 9, 3, 1024, 256, mode, False)
