@@ -185,6 +185,13 @@ def test_latent_inputs(dt, half, T, H, dim, rot, rank, qr):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("rank,qr", [(128, 384), (129, 64), (64, 385), (256, 768), (257, 10), (100, 769), (512, 1537)])
+def test_latent_values_a_lane(dt, rank, qr):
+    """Both sides of two, four and eight values of a row in a lane."""
+    test_latent_inputs(dt, False, 9, 2, 16, 12, rank, qr)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 def test_relu2_and_dense_gate(dt):
     torch.manual_seed(4)
     T, E, ff, k = 9, 6, 20, 3
