@@ -273,7 +273,7 @@ class PipelinedConversations(Conversations):
 
     def wait_turns(self, n: int, records=None) -> None:
         """Block until ``n`` turns have completed in total; from then on record into ``records``."""
-        # DLLM_VERBOSE=1: a progress line every 30 s (long rehearsals; gpurun's silence watchdog)
+        # DLLM_VERBOSE=1: a progress line every 30 s (long rehearsals; watchers that take silence for a hang)
         verbose = os.environ.get("DLLM_VERBOSE") == "1"
         last = time.perf_counter()
         with self._cv:
