@@ -1177,11 +1177,11 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
         wps = [panel_weight(w) for w in ws] if W_PANEL else ws
         lins = {}
         for M in sorted({*todo, *PF_LIN_MS}) if (N, K) in roles else ():
-            whole = _fused_call(roles[(N, K)], torch.randn(M, K, device=dev).to(torch.bfloat16), ws, wps, qkv_dims, dev)
             try:
+                whole = _fused_call(roles[(N, K)], torch.randn(M, K, device=dev).to(torch.bfloat16), ws, wps, qkv_dims, dev)
                 _P.fused_core[(M, N, K)] = "lin"
                 lins[M] = _time(whole, iters=8)
-            except Exception:  # noqa: BLE001 - no such fused op
+            except Exception:  # noqa: BLE001 - no such fused op, or no memory for so many rows
                 continue
             finally:
                 _P.fused_core.pop((M, N, K), None)

@@ -153,6 +153,24 @@ def test_vendor_core_by_the_rows_at_hand(monkeypatch):
         assert not G.use_vendor_core(10000, N, K) and G.use_vendor_core(3000, N, K)
 
 
+def test_rows_that_do_not_fit_are_not_timed(monkeypatch):
+    """Beside a large model and its pool the largest row counts may find no memory: they are left out, and the engine starts."""
+    _none_timed(monkeypatch)
+    monkeypatch.setattr(G, "PREFILL_MS", (2048,))
+    monkeypatch.setattr(G, "PF_SMALL_MS", ())
+    monkeypatch.setattr(G, "PF_LIN_MS", (1280, 12288, 16384))
+
+    def call(role, x, *a):
+        if x.shape[0] > 12000:
+            raise torch.OutOfMemoryError("no memory")
+        return lambda i: None
+    monkeypatch.setattr(G, "_fused_call", call)
+    monkeypatch.setattr(G, "_native", lambda x: None)
+    monkeypatch.setattr(G, "_time", lambda fn, iters=24: 7.0)
+    G._autotune_prefill([(64, 64)], "cpu", False, {(64, 64): "resadd"})
+    assert G._P.pf_lin == {(64, 64): [(1280, 7.0), (2048, 7.0)]} and set(G._P.fused_core) == {(2048, 64, 64)}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("panel", [False, True])
 def test_parts_are_the_whole(monkeypatch, panel):
