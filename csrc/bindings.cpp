@@ -47,6 +47,8 @@ int dllm_f32_gemm(const float*, long, const float*, float*, long, int, int, int,
 int dllm_dgemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*, void*, long, float*, long,
                float, float, const int*, const float*, const int*, void*, void*, void*, void*, long, int, int, int, const float*, int, float,
                float, hipStream_t);
+int dllm_tail_gemm(const void*, long, const float*, float*, const float*, const float*, const float*, float, const void*, void*, long, int, int, int,
+                   int, int, const float*, int, float, float, hipStream_t);
 int dllm_skinny_gemm(const void*, long, const void*, void*, long, int, int, int, int, int, int, int, float*, int*,
                      hipStream_t);
 int dllm_moe_max_tiles(int, int);
@@ -873,6 +875,50 @@ int64_t dgemm(torch::Tensor x, torch::Tensor w, int64_t n_cols, int64_t epi, int
                 (float)limit, (float)alpha, stream()),
      "dgemm");
   return epi == 1 ? tiles : 0;
+}
+
+// resadd_norm (x2 = x + rmsnorm(y + bias) w_post, h = rmsnorm(x2) w_next) and the product h . W^T behind it in one launch
+// (csrc/kernels/tail_gemm.hip): y [M <= 16, K <= 1024], x and x2 [M, K] f32, not the same memory, w as dgemm's; glu: w paired, out [M, n_cols / 2] =
+// the gated activation `mode` of glu_act, with act_bias.  nt 1 or 2 tiles of 16 columns a workgroup.
+void tail_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor x2, torch::Tensor w_post, torch::Tensor w_next, c10::optional<torch::Tensor> bias,
+               double eps, torch::Tensor w, int64_t n_cols, torch::Tensor out, int64_t nt, bool glu, c10::optional<torch::Tensor> act_bias, int64_t mode,
+               double limit, double alpha) {
+  check_bf16(y, "y");
+  check_bf16(w, "w");
+  check_bf16(out, "out");
+  check_f32(x, "x");
+  check_f32(x2, "x2");
+  check_f32(w_post, "w_post");
+  check_f32(w_next, "w_next");
+  const int64_t M = y.size(0), K = y.dim() == 2 ? y.size(1) : 0, N = n_cols;
+  auto aligned = [](const torch::Tensor& t, int n) { return (uintptr_t)t.data_ptr() % n == 0; };
+  TORCH_CHECK(y.dim() == 2 && y.stride(1) == 1 && M >= 1 && M <= 16 && K >= 32 && K <= 1024 && K % 32 == 0, "y [M, K]: M <= 16, K <= 1024, K % 32 == 0");
+  TORCH_CHECK(y.stride(0) % 4 == 0 && aligned(y, 8) && (M == 1 || y.stride(0) >= K), "y: rows of 8 bytes");
+  TORCH_CHECK(x.sizes() == y.sizes() && x2.sizes() == y.sizes() && x.is_contiguous() && x2.is_contiguous() && aligned(x, 16) && aligned(x2, 16) &&
+                  (x.data_ptr<float>() + M * K <= x2.data_ptr<float>() || x2.data_ptr<float>() + M * K <= x.data_ptr<float>()),
+              "x, x2 [M, K], apart");
+  auto vec = [&](const torch::Tensor& t, int64_t n) { return t.is_contiguous() && t.numel() == n && aligned(t, 16); };
+  TORCH_CHECK(vec(w_post, K) && vec(w_next, K), "norm weights [K]");
+  TORCH_CHECK(w.dim() == 4 && w.is_contiguous() && w.size(0) == (N + 15) / 16 && w.size(1) == K / 32 && w.size(2) == 64 && w.size(3) == 8 && N >= 1 &&
+                  aligned(w, 16), "w: [ceil(N / 16), K / 32, 64, 8]");
+  TORCH_CHECK((nt == 1 || nt == 2) && mode >= 0 && mode <= 2 && (!glu || N % 16 == 0), "no such plan");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == (glu ? N / 2 : N) && out.stride(1) == 1 && out.stride(0) % 4 == 0 && aligned(out, 8) &&
+                  (M == 1 || out.stride(0) >= out.size(1)), "out: rows of 8 bytes");
+  const float *bp = nullptr, *ap = nullptr;
+  if (bias) {
+    check_f32(*bias, "bias");
+    TORCH_CHECK(vec(*bias, K), "bias [K]");
+    bp = bias->data_ptr<float>();
+  }
+  if (act_bias) {
+    check_f32(*act_bias, "act_bias");
+    TORCH_CHECK(glu && vec(*act_bias, N) && N % 8 == 0, "act_bias [n_cols]");
+    ap = act_bias->data_ptr<float>();
+  }
+  ok(dllm_tail_gemm(y.data_ptr(), y.stride(0), x.data_ptr<float>(), x2.data_ptr<float>(), w_post.data_ptr<float>(), w_next.data_ptr<float>(), bp,
+                    (float)eps, w.data_ptr(), out.data_ptr(), out.stride(0), (int)M, (int)N, (int)K, (int)nt, glu, ap, (int)mode, (float)limit,
+                    (float)alpha, stream()),
+     "tail_gemm");
 }
 
 // Small-batch (M <= 16) MFMA GEMM with a fused decoder epilogue (csrc/kernels/skinny_gemm.hip
@@ -3009,6 +3055,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("skinny_epi", &skinny_epi);
   m.def("f32_gemm", &f32_gemm, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("epi") = 0);
   m.def("dgemm", &dgemm);
+  m.def("tail_gemm", &tail_gemm);
   m.def("gemv", &gemv);
   m.def("gemv_norm", &gemv_norm);
   m.def("gemv_slots", &gemv_slots);

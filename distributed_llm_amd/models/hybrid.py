@@ -99,6 +99,10 @@ from .configs import DenseSpec, HybridConfig, LayerSpec, MixerSpec, MoESpec, QTe
 _PROJECTIONS = ("proj", "out", "dqkv", "uq", "o", "up", "down", "in", "x", "dt", "qkvg", "lo", "ro", "sh_up", "sh_down")
 
 
+# the one product that these mixers make of their input: it may take the tail ahead of it along (ops.gemm.Tail)
+_FIRST = {"biased_attention": "proj", "latent_attention": "dqkv", "mlstm": "proj"}
+
+
 def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
     """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy."""
     if wf is not None and ops.gemm.dg_takes(x):
@@ -114,6 +118,8 @@ def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, kee
 
 def _pm(x: torch.Tensor, L: Dict[str, torch.Tensor], name: str) -> torch.Tensor:
     wf = L.get(name + "_r")
+    if isinstance(x, ops.gemm.Tail):
+        return x.linear(L[name], wf)
     return _mm(x, L[name]) if wf is None else _mm(x, L[name], wf, L["order_kept"])
 
 
@@ -1058,7 +1064,9 @@ class HybridModel:
 
     def _dense(self, L, f: DenseSpec, x):
         act, a = self._act_args(f), None
-        if "up_act_r" in L:
+        if "up_act_r" in L and isinstance(x, ops.gemm.Tail):
+            a = x.linear(L["up"], L["up_act_r"], act[0], L.get("up_b"), act[1], act[2])
+        elif "up_act_r" in L:
             a = ops.gemm.linear_act(x, L["up"], L["up_act_r"], act[0], L.get("up_b"), act[1], act[2], L["order_kept"])
         elif "up_r" in L and act is not None and act[0] == "gelu" and ops.gemm.fg_takes(x, L["up"].shape[0]):
             a = ops.gemm.f32_linear(x, L["up_r"], L["up"].shape[0], gelu=True)
@@ -1140,6 +1148,21 @@ class HybridModel:
         if f.shared_ff:
             y = y + _pm(seqmix.relu2_scale(_pm(x, L, "sh_up")), L, "sh_down")
         return y
+
+    def _tail(self, y, w_post, x, w_next, bias=None, L=None, S: Optional[LayerSpec] = None):
+        """``x += rmsnorm(y + bias) * w_post`` and the next sublayer's input ``rmsnorm(x) * w_next``: (stream, input).  ``L``, ``S``: the
+        layer that reads the input, with its feed-forward (S None) or with its mixer; where its product takes the
+        tail along, the input is an ``ops.gemm.Tail`` and the stream is there once that product has run."""
+        if L is not None and self.tap is None:
+            name = "up" if S is None else _FIRST.get(S.mixer.kind)
+            wf = L.get("up_act_r", L.get("up_r")) if name == "up" else L.get(f"{name}_r")
+            if wf is not None and not L["order_kept"] and wf.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and x.is_contiguous() and \
+                    ops.gemm.tail_takes(y, L[name], w_post, w_next, bias, L.get("up_b") if name == "up" else None):
+                x2 = torch.empty_like(x)
+                return x2, ops.gemm.Tail(y, w_post, self.cfg.rms_eps, x, x2, w_next, bias)
+        h = torch.empty(x.shape, dtype=self.dtype, device=x.device)
+        seqmix.resadd_norm(y, w_post, self.cfg.rms_eps, x, w_next, h, bias=bias)
+        return x, h
 
     # ------------------------------------------------------------------ forward
     def _embed(self, ids: torch.Tensor) -> torch.Tensor:
@@ -1223,8 +1246,12 @@ class HybridModel:
                 pair = dict(b=y[1], wa=L["lout"], wb=L["rout"]) if isinstance(y, tuple) else {}
                 a, bias = y[0] if isinstance(y, tuple) else y, None
                 if S.mlp is not None:
-                    h = torch.empty((T, W), dtype=self.dtype, device=x.device)
-                    seqmix.resadd_norm(a, L["norm1b"], eps, x, L["norm2"], h, **pair)
+                    if pair:
+                        h = torch.empty((T, W), dtype=self.dtype, device=x.device)
+                        seqmix.resadd_norm(a, L["norm1b"], eps, x, L["norm2"], h, **pair)
+                    else:
+                        gated = isinstance(S.mlp, DenseSpec) and (self._act_args(S.mlp) or ("",))[0] != "gelu"
+                        x, h = self._tail(a, L["norm1b"], x, L["norm2"], L=L if gated and X is None else None)
                     y = self._dense(L, S.mlp, h) if isinstance(S.mlp, DenseSpec) else self._experts(L, S.mlp, h)
                     a, pair, post, bias = y, {}, L["norm2b"], L.get("down_b")
                 else:
@@ -1232,9 +1259,12 @@ class HybridModel:
                 if X is not None:     # ... and the layer's weighted sum over depth
                     h = torch.empty((T, W), dtype=self.dtype, device=x.device)
                     x = seqmix.resadd_norm(a, post, eps, x, nxt, h, depth=(X, L["dwa"], i + 2), bias=bias, **pair)
-                else:
+                elif pair:
                     h = torch.empty((T, W), dtype=self.dtype, device=x.device)
                     seqmix.resadd_norm(a, post, eps, x, nxt, h, bias=bias, **pair)
+                else:
+                    last = i + 1 == nL
+                    x, h = self._tail(a, post, x, nxt, bias, None if last else self.layers[i + 1], None if last else cfg.layers[i + 1])
             else:
                 ng = cfg.norm_groups
                 xw = torch.empty_like(x) if xl is not None and isinstance(S.mlp, MoESpec) and S.mlp.act == "swiglu" else None

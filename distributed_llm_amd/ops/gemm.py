@@ -692,6 +692,40 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, wf: torch.Tensor, act: str, bia
     return y
 
 
+TAIL_MAX_M, TAIL_MAX_K = 16, 1024      # tail_gemm.hip: rows and width of what a workgroup norms
+
+
+class Tail:
+    """A sublayer's tail that the product behind it takes along (csrc/kernels/tail_gemm.hip): ``x2 = x + rmsnorm(y + bias) * w_post``
+    (f32, another buffer than x), and the product's input ``rmsnorm(x2) * w_next``, which exists nowhere else.  Goes where that input
+    would (``shape``, ``device``, ``dtype`` are its own)."""
+
+    def __init__(self, y, w_post, eps, x, x2, w_next, bias=None):
+        self.y, self.w_post, self.eps, self.x, self.x2, self.w_next, self.bias = y, w_post, eps, x, x2, w_next, bias
+        self.shape, self.device, self.dtype, self.is_cuda = y.shape, y.device, y.dtype, y.is_cuda
+
+    def linear(self, w: torch.Tensor, wf: torch.Tensor, act: Optional[str] = None, act_bias: Optional[torch.Tensor] = None,
+               limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
+        """``linear`` of the input, or with ``act`` ``linear_act``'s gated form; once, and on the engine's stream before x2 is read."""
+        from .seqmix import GLU_MODES
+        N = w.shape[0]
+        out = torch.empty((self.shape[0], N if act is None else N // 2), dtype=self.dtype, device=self.device)
+        _native(self.y).tail_gemm(self.y, self.x, self.x2, self.w_post, self.w_next, self.bias, float(self.eps), wf, N, out,
+                                  1 if N <= 16 * _sk_grid(self.device) else 2, act is not None, act_bias,
+                                  0 if act is None else GLU_MODES[act], float(limit), float(alpha))
+        return out
+
+
+def tail_takes(y: torch.Tensor, w: torch.Tensor, *vectors: Optional[torch.Tensor]) -> bool:
+    """Does a ``Tail`` of y go into the product with w [N, K] (which has a fragment-major copy)?  Up to 16 rows of at most 1024, and
+    columns for one round of workgroups: each norms every row.  ``vectors``: the f32 vectors it reads."""
+    M, (N, K) = y.shape[0], w.shape
+    return (y.is_cuda and y.dtype == torch.bfloat16 and 0 < M <= TAIL_MAX_M and y.shape[1] == K <= TAIL_MAX_K and K % 32 == 0 and
+            y.stride(1) == 1 and y.stride(0) % 4 == 0 and (M == 1 or y.stride(0) >= K) and y.data_ptr() % 8 == 0 and
+            N <= 32 * _sk_grid(y.device) and os.environ.get("DLLM_GEMM") != "blas" and
+            all(v is None or (v.dtype == torch.float32 and v.is_contiguous() and v.data_ptr() % 16 == 0) for v in vectors))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
            wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
     """``x @ w.T`` on the shape's tuned plan; ``wp``: the panel copy a tgemm plan streams, ``wf``: the fragment-major copy of the
