@@ -24,6 +24,8 @@ int dllm_gemv(const void*, long, const void*, void*, long, int, int, int, int, i
 int dllm_gelu(const void*, void*, long, hipStream_t);
 int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, const int*, int, hipStream_t);
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
+int dllm_resadd_router(const void*, long, const float*, float, float*, void*, const float*, const void*, int, int, int, int, int*, float*, int, float,
+                       hipStream_t);
 int dllm_moe_router(const void*, long, const void*, int, int, int, int, int*, float*, float*, int, float, const void*, float, void*, hipStream_t);
 int dllm_scatter_pairs(int*, const int*, int, hipStream_t);
 int dllm_step_fetch(const int*, int*, int, int, int, int, const int*, const int*, int*, int, int*, int, int, hipStream_t);
@@ -493,6 +495,33 @@ void moe_router(torch::Tensor x, torch::Tensor wg, int64_t k, torch::Tensor ids,
                      lp, (int)shared, (float)scale, norm_w ? norm_w->data_ptr() : nullptr, (float)eps,
                      norm_w ? xn->data_ptr() : nullptr, stream()),
      "moe_router");
+}
+
+// norm_resadd of one group with its rounded copy, and moe_router of that, in one launch (H <= 2048)
+void resadd_router(torch::Tensor y, torch::Tensor w, double eps, torch::Tensor x, torch::Tensor xl, c10::optional<torch::Tensor> bias,
+                   torch::Tensor wg, int64_t k, torch::Tensor ids, torch::Tensor wts, bool shared, double scale) {
+  check_bf16(y, "y");
+  check_bf16(xl, "x_lp");
+  check_bf16(wg, "router weight");
+  check_f32(w, "w");
+  check_f32(x, "x");
+  check_i32(ids, "ids");
+  check_f32(wts, "weights");
+  TORCH_CHECK(y.dim() == 2 && y.stride(1) == 1 && x.is_contiguous() && xl.is_contiguous() && x.sizes() == y.sizes() && xl.sizes() == y.sizes() &&
+                  w.is_contiguous() && w.numel() == y.size(1),
+              "y, x, x_lp [T, H], w [H]");
+  TORCH_CHECK(wg.dim() == 2 && wg.is_contiguous() && wg.size(1) == y.size(1) && (uintptr_t)wg.data_ptr() % 16 == 0, "wg [E, H], 16-B aligned");
+  const int64_t T = y.size(0), n = T * (k + (shared ? 1 : 0));
+  TORCH_CHECK(ids.numel() == n && wts.numel() == n && ids.is_contiguous() && wts.is_contiguous(), "out shapes");
+  const float* bp = nullptr;
+  if (bias) {
+    check_f32(*bias, "bias");
+    TORCH_CHECK(bias->is_contiguous() && bias->numel() == y.size(1), "bias [H]");
+    bp = bias->data_ptr<float>();
+  }
+  ok(dllm_resadd_router(y.data_ptr(), y.stride(0), w.data_ptr<float>(), (float)eps, x.data_ptr<float>(), xl.data_ptr(), bp, wg.data_ptr(), (int)T,
+                        (int)wg.size(0), (int)y.size(1), (int)k, ids.data_ptr<int>(), wts.data_ptr<float>(), (int)shared, (float)scale, stream()),
+     "resadd_router");
 }
 
 // dst (int32, any shape, contiguous) flat[idx_i] = val_i for buf = [n, idx0, val0, ...]
@@ -3028,6 +3057,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
   m.def("gelu", &gelu);
   m.def("mean_pool_l2", &mean_pool_l2, py::arg("x"), py::arg("lens"), py::arg("out"), py::arg("starts") = py::none());
   m.def("moe_gate", &moe_gate);
+  m.def("resadd_router", &resadd_router);
   m.def("moe_router", &moe_router, py::arg("x"), py::arg("wg"), py::arg("k"), py::arg("ids"), py::arg("w"),
         py::arg("logits") = py::none(), py::arg("shared") = false, py::arg("scale") = 1.0, py::arg("norm_w") = py::none(),
         py::arg("eps") = 0.0, py::arg("xn") = py::none());

@@ -181,6 +181,32 @@ __global__ void moe_gate_kernel(const float* __restrict__ logits, int T, int E, 
   for (int i = 0; i < k; ++i) { sel[i] = __expf(sel[i] - m); s += sel[i]; }
   for (int i = 0; i < k; ++i) { ids[(long)t * k + i] = sid[i]; w[(long)t * k + i] = sel[i] / s; }
 }
+// A token's choice from its logits (lane e: expert e's; one wave): the k largest, the lower expert first among equals; NaN is never chosen, and
+// expert 0 where nothing is left to choose.  Softmax over all E then renormalise over the selected == softmax over the selected logits;
+// summed in the order of choice.  `o`: the token's first pair
+__device__ __forceinline__ void router_choice(float lg, int lane, int E, int k, long o, int* ids, float* w, int shared, float scale) {
+  float left = lane < E && lg > -INFINITY ? lg : -INFINITY, sel = -INFINITY;
+  int sid = 0;
+  for (int i = 0; i < k; ++i) {
+    float best = left;
+    int bi = lane;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const float ov = lane_xor(best, m);
+      const int oi = lane_xor(bi, m);
+      if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+    }
+    if (!(best > -INFINITY)) bi = 0;
+    if (lane == i) { sel = best; sid = bi; }
+    if (lane == bi) left = -INFINITY;
+  }
+  const float ex = __expf(sel - __shfl(sel, 0));
+  float sum = 0.f;
+  for (int i = 0; i < k; ++i) sum += __shfl(ex, i);
+  if (lane < k) { ids[o + lane] = sid; w[o + lane] = ex / sum * scale; }
+  if (shared && lane == k) { ids[o + k] = E; w[o + k] = 1.f; }
+}
+
 // Fused router: logits[t, e] = x[t] . wg[e] in fp32 (one wave per token: each lane holds XC 8-wide
 // chunks of its token's row in registers, every expert's dot product is summed in a fixed order and
 // reduced with an xor butterfly), then the same top-k / renormalised softmax as moe_gate_kernel.
@@ -276,29 +302,95 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const u16* __restrict__
     for (int x = 0; x < EB; ++x) lg = lane == e0 + x ? s[x] : lg;
   }
   if (logits != nullptr && lane < E) logits[(long)t * E + lane] = lg;
-  // the k largest, the lower expert first among equals; NaN is never chosen, and expert 0 where nothing is left to choose
-  float left = lane < E && lg > -INFINITY ? lg : -INFINITY, sel = -INFINITY;
-  int sid = 0;
-  for (int i = 0; i < k; ++i) {
-    float best = left;
-    int bi = lane;
+  router_choice(lg, lane, E, k, (long)t * (k + shared), ids, w, shared, scale);
+}
+
+// norm_resadd (seqmix.hip, one group: x += rmsnorm(y + bias) * w, xl = the rounded stream) and the router of that row: a workgroup a token, the
+// row's entries and sums as norm_resadd_reg_kernel has them, then two experts a wave at a time with moe_router_kernel's sums, the
+// first two's rows asked for beside the token's.  Both launches were latency: us in a captured graph, two / here, width 1024, 8 experts:
+// 1 token 5.6 / 3.6, 24 6.4 / 3.9, 300 6.9 / 4.5, 4000 15.6 / 12.4; 64 experts 24 tokens 13.4 / 6.9, 1000 15.1 / 11.3, 4000 32.3 / 30.2, but 12000 81 / 83
+// (and width 2048, 4000 54.9 / 55.8: many tokens of many experts stay apart, ops.resadd_moe_router).
+template <int NE, int XC>      // entries a thread, 8-wide chunks a lane
+__global__ void __launch_bounds__(256) resadd_router_kernel(const u16* __restrict__ y, long ldy, const float* __restrict__ w, float* __restrict__ x,
+                                                            u16* __restrict__ xl, int H, float eps, const float* __restrict__ bias,
+                                                            const u16* __restrict__ wg, int E, int k, int* __restrict__ ids,
+                                                            float* __restrict__ wts, int shared, float scale) {
+  __shared__ float red[4], lgs[64];
+  __shared__ __attribute__((aligned(16))) u16 rowb[512 * XC];
+  const long row = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nc = H >> 3;
+  float* xr = x + row * (long)H;
+  float a[NE], s[NE], g[NE], b[NE];
+  const float* bp = bias ? bias : w;
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      const float ov = lane_xor(best, m);
-      const int oi = lane_xor(bi, m);
-      if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
-    }
-    if (!(best > -INFINITY)) bi = 0;
-    if (lane == i) { sel = best; sid = bi; }
-    if (lane == bi) left = -INFINITY;
+  for (int j = 0; j < NE; ++j) {
+    const int c = min((int)threadIdx.x + 256 * j, H - 1);
+    s[j] = xr[c];
+    g[j] = w[c];
+    a[j] = bf2f(y[row * ldy + c]);
+    b[j] = bp[c];
   }
-  // softmax over all E then renormalise over the selected == softmax over the selected logits; summed in the order of choice
-  const float ex = __expf(sel - __shfl(sel, 0));
-  float sum = 0.f;
-  for (int i = 0; i < k; ++i) sum += __shfl(ex, i);
-  const long o = (long)t * (k + shared);
-  if (lane < k) { ids[o + lane] = sid; w[o + lane] = ex / sum * scale; }
-  if (shared && lane == k) { ids[o + k] = E; w[o + k] = 1.f; }
+  uint4 wr[2][XC];
+  auto rows = [&](int e0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int c = 0; c < XC; ++c) wr[i][c] = ld16(wg + (long)min(e0 + wave + 4 * i, E - 1) * H + 8 * min(lane + 64 * c, nc - 1));
+  };
+  rows(0);
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    if (bias) a[j] += b[j];
+    const float v = (int)threadIdx.x + 256 * j < H ? a[j] : 0.f;
+    q = fmaf(v, v, q);
+  }
+  q = wave_sum(q);
+  if (lane == 0) red[wave] = q;
+  __syncthreads();
+  q = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q += red[i];
+  const float r = 1.f / sqrtf(q / (float)H + eps);
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    const int c = threadIdx.x + 256 * j;
+    if (c >= H) continue;
+    const float v = s[j] + a[j] * r * g[j];
+    xr[c] = v;
+    const u16 o = f2bf(v);
+    xl[row * (long)H + c] = o;
+    rowb[c] = o;
+  }
+  __syncthreads();
+  uint4 xv[XC];
+#pragma unroll
+  for (int c = 0; c < XC; ++c) xv[c] = lane + 64 * c < nc ? ld16(rowb + 8 * (lane + 64 * c)) : make_uint4(0u, 0u, 0u, 0u);
+  for (int e0 = 0; e0 < E; e0 += 8) {
+    if (e0 > 0) rows(e0);
+    float d[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      d[i] = 0.f;
+#pragma unroll
+      for (int c = 0; c < XC; ++c) {
+        float f[8], h[8];
+        unpack8(lane + 64 * c < nc ? wr[i][c] : make_uint4(0u, 0u, 0u, 0u), f);
+        unpack8(xv[c], h);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) d[i] += h[u] * f[u];
+      }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) d[i] = lane_add(d[i], m);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (lane == 0 && e0 + wave + 4 * i < E) lgs[e0 + wave + 4 * i] = d[i];
+  }
+  __syncthreads();
+  if (wave == 0) router_choice(lane < E ? lgs[lane] : -INFINITY, lane, E, k, row * (k + shared), ids, wts, shared, scale);
 }
 
 // buf = [n, idx0, val0, idx1, val1, ...]: dst[idx_i] = val_i.  n is read on the device, so a
@@ -441,6 +533,19 @@ extern "C" int dllm_moe_router(const void* x, long x_stride, const void* wg, int
     default: ROUTER(16, 2);
   }
 #undef ROUTER
+  return (int)hipGetLastError();
+}
+
+// y [T, H] bf16 rows, x [T, H] f32 in place, xl [T, H] bf16; wg [E, H] bf16, rows of 16 bytes; ids and wts [T, k + shared]
+extern "C" int dllm_resadd_router(const void* y, long ldy, const float* w, float eps, float* x, void* xl, const float* bias, const void* wg, int T,
+                                  int E, int H, int k, int* ids, float* wts, int shared, float scale, hipStream_t stream) {
+  if (E < 1 || E > 64 || k < 1 || k > 8 || k > E || H < 8 || H % 8 || H > 2048) return -1;
+  if (T == 0) return 0;
+#define RR(NE, XC)                                                                                                                         \
+  hipLaunchKernelGGL((resadd_router_kernel<NE, XC>), dim3(T), dim3(256), 0, stream, (const u16*)y, ldy, w, x, (u16*)xl, H, eps, bias, (const u16*)wg, \
+                     E, k, ids, wts, shared, scale)
+  if (H <= 512) RR(2, 1); else if (H <= 1024) RR(4, 2); else RR(8, 4);
+#undef RR
   return (int)hipGetLastError();
 }
 

@@ -1121,13 +1121,13 @@ class HybridModel:
         a = seqmix.swiglu_scale(_mm(x, L["w1"].view(f.experts * 2 * f.ff, -1)), g, f.ff)
         return _pm(a, L, "w2d")
 
-    def _experts(self, L, f: MoESpec, x, tail=None, wide=None):
+    def _experts(self, L, f: MoESpec, x, tail=None, wide=None, routed=None):
         """``tail`` (ops.moe_ffn_tg): where the experts run on the grouped GEMM, their sum ends in the stream and None is
-        returned; elsewhere the caller adds what is returned."""
+        returned; elsewhere the caller adds what is returned.  ``routed``: (ids, weights), where the launch before has chosen."""
         if f.act == "swiglu":
             return self._experts_swiglu(L, f, x, tail, wide)
         if "shared_in" in L:
-            ids, w = ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
+            ids, w = routed or ops.moe_router(x, L["router"], f.top, shared=True, scale=f.scale)
             return seqmix.moe_ffn_relu2(x, ids, w, L["w1"], L["w2"], tail, L.get("experts_r"))
         if f.experts > 64 or f.top > 8:      # beyond the router kernels' register budget: library top-k
             val, ids = torch.topk(torch.softmax(F.linear(x.float(), L["router"].float()), -1), f.top, -1)
@@ -1268,11 +1268,15 @@ class HybridModel:
             else:
                 ng = cfg.norm_groups
                 xw = torch.empty_like(x) if xl is not None and isinstance(S.mlp, MoESpec) and S.mlp.act == "swiglu" else None
-                seqmix.norm_resadd(y, L["norm1"], eps, x, xl, groups=ng, bias=L.get("ob"), x_wide=xw)
+                routed = None
+                if xl is not None and ng == 1 and isinstance(S.mlp, MoESpec) and S.mlp.act != "swiglu" and "shared_in" in L:
+                    routed = ops.resadd_moe_router(y, L["norm1"], eps, x, xl, L["router"], S.mlp.top, True, S.mlp.scale, L.get("ob"))
+                else:
+                    seqmix.norm_resadd(y, L["norm1"], eps, x, xl, groups=ng, bias=L.get("ob"), x_wide=xw)
                 if S.mlp is not None:
                     hin = x if xl is None else xl
                     y = self._dense(L, S.mlp, hin) if isinstance(S.mlp, DenseSpec) else \
-                        self._experts(L, S.mlp, hin, (L["norm2"], eps, x, xl, ng), xw)
+                        self._experts(L, S.mlp, hin, (L["norm2"], eps, x, xl, ng), xw, routed)
                     if y is not None:
                         seqmix.norm_resadd(y, L["norm2"], eps, x, xl, groups=ng)
                 if X is not None:
