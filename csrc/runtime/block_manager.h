@@ -177,6 +177,17 @@ class BlockManager {
     return out;
   }
 
+  // Tokens, positions and slots of positions [start, end) of a sequence.
+  void inputs(int64_t id, int start, int end, int32_t* tok, int32_t* pos, int32_t* slot) {
+    const Seq& s = get(id);
+    if (start < 0 || start > end || end > (int)s.tokens.size() || end > (int)s.blocks.size() * bs_) throw std::out_of_range("token range");
+    std::copy(s.tokens.begin() + start, s.tokens.begin() + end, tok);
+    for (int p = start; p < end; ++p) {
+      *pos++ = p;
+      *slot++ = s.blocks[p / bs_] * bs_ + p % bs_;
+    }
+  }
+
   // Mark K/V of positions [0, n) as computed; registers newly completed full blocks.
   void commit(int64_t id, int n) {
     Seq& s = get(id);

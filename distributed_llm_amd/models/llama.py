@@ -35,6 +35,7 @@ import os
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -77,13 +78,10 @@ class AttnMeta:
             self._lat = {}
         tpe = max(1, rows // heads)
         if tpe not in self._lat:
-            ts, tt = [], []
-            for i, n in enumerate(self.host_qlen):
-                for t0 in range(0, int(n), tpe):
-                    ts.append(i)
-                    tt.append(t0)
-            self._lat[tpe] = (torch.tensor(ts, dtype=torch.int32, device=device),
-                              torch.tensor(tt, dtype=torch.int32, device=device))
+            both = torch.from_numpy(np.stack(ops.tile_table(np.asarray(self.host_qlen, dtype=np.int64), tpe)))
+            if torch.device(device).type == "cuda":      # (from pageable memory the copy waits for the launches before it)
+                both = both.pin_memory().to(device, non_blocking=True)
+            self._lat[tpe] = (both[0], both[1])
         return self._lat[tpe]
 
 

@@ -200,6 +200,14 @@ def flash_supported(d: int, group: int, max_blocks: int) -> bool:
         flash_lds_bytes(d, max_blocks) <= 160 * 1024 and os.environ.get("DLLM_FLASH_PREFILL", "1") == "1"
 
 
+def tile_table(q_lens: np.ndarray, tokens: int) -> Tuple[np.ndarray, np.ndarray]:
+    """``build_tiles`` / ``flash_tiles`` for tiles of ``tokens`` tokens, as int32 arrays."""
+    counts = -(-q_lens // tokens)
+    seq = np.repeat(np.arange(len(q_lens), dtype=np.int32), counts)
+    first = np.cumsum(counts) - counts
+    return seq, ((np.arange(len(seq)) - np.repeat(first, counts)) * tokens).astype(np.int32)
+
+
 def flash_tiles(q_lens, group: int) -> Tuple[list, list]:
     """Host tile table of the flash prefill kernel: 256 / group query tokens per tile."""
     tpt = FLASH_ROWS // group
