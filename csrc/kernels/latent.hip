@@ -692,8 +692,8 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
   }
   const int* btr = bt + (long)s * bt_w;
   const int ntiles = (kmax + KT - 1) / KT;
-  const int kbeg = (int)((long)ntiles * blockIdx.z / splits) * KT;
-  const int kend = min(kmax, (int)((long)ntiles * (blockIdx.z + 1) / splits) * KT);
+  // as many tiles a split as they come to, so the splits with keys are the first ones (what merges them reads no others)
+  const int per = (ntiles + splits - 1) / splits * KT, kbeg = (int)blockIdx.z * per, kend = min(kmax, kbeg + per);
   if (splits > 1 && kbeg >= kend) {        // more splits than tiles: nothing to leave but that (decode grids have them for the longest context)
     if (tid < RPB) {
       const long pr = (((long)entry * gridDim.x + blockIdx.x) * RPB + tid) * splits + blockIdx.z;
@@ -931,6 +931,22 @@ __global__ void __launch_bounds__(256) latent_attention_mfma_kernel(
   }
 }
 
+// o + sum_z w_z (split z's entry c), z from z0 to live, in order; 16 loads under way at a time, none behind a condition
+__device__ __forceinline__ float more_splits(float o, int z0, int live, float wz, const float* po, int rank, int c) {
+  const float* p = po + min(c, rank - 1);
+  for (int z = z0; z < live; z += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = p[(long)min(z + u, live - 1) * rank];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const float w = __shfl(wz, min(z + u, live - 1), 64);
+      if (z + u < live && w != 0.f) o += v[u] * w;       // a split that saw no key left nothing to read
+    }
+  }
+  return o;
+}
+
 // one workgroup per (entry, row): merge the splits' (max, sum, weighted latent) partials.  Lane z of every
 // wave holds split z's weight (splits <= 64), a thread owns latent dims tid, tid + 256, ...
 template <typename T>
@@ -965,6 +981,7 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
   float L = wave_sum(lz * ez);
   if (sinks && L > 0.f) L += expf(sinks[row % H] - M);
   const float wz = L > 0.f ? ez / L : 0.f;
+  const int live = 64 - __clzll((long long)__ballot(lz > 0.f));      // one past the last split with a key
   const long tok = q0 + tok0 + row / H;
   const int h = row % H;
   for (int c0 = 0; c0 < rank; c0 += 256) {     // every lane stays in the loop: the shuffles read all lanes
@@ -980,11 +997,7 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
       }
       z0 = min(splits, NZ);
     }
-#pragma unroll 8
-    for (int z = z0; z < splits; ++z) {
-      const float w = __shfl(wz, z, 64);
-      if (on && w != 0.f) o += po[(long)z * rank + c] * w;
-    }
+    o = more_splits(o, z0, live, wz, po, rank, c);
     if (on) stf(out + ((long)h * Ttot + tok) * rank + c, o);
   }
 }
@@ -1031,6 +1044,7 @@ __global__ void __launch_bounds__(256) latent_up_kernel(const float* __restrict_
   float L = wave_sum(lz * ez);
   if (sinks && L > 0.f) L += expf(sinks[h] - M);
   const float wz = L > 0.f ? ez / L : 0.f;
+  const int live = 64 - __clzll((long long)__ballot(lz > 0.f));      // one past the last split with a key
   for (int c0 = 0; c0 < rank; c0 += 256) {     // every lane stays in the loop: the shuffles read all lanes
     const int c = c0 + tid;
     float o = 0.f;
@@ -1043,11 +1057,7 @@ __global__ void __launch_bounds__(256) latent_up_kernel(const float* __restrict_
       }
       z0 = min(splits, NZ);
     }
-#pragma unroll 8
-    for (int z = z0; z < splits; ++z) {
-      const float w = __shfl(wz, z, 64);
-      if (c < rank && w != 0.f) o += po[(long)z * rank + c] * w;
-    }
+    o = more_splits(o, z0, live, wz, po, rank, c);
     if (c < rank) lat[c] = bf2f(f2bf(o));
   }
   __syncthreads();

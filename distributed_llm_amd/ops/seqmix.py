@@ -209,15 +209,20 @@ def latent_q_prep(q, heads, dim, rot_dim, positions, cos_sin, scale, half: bool 
     return out
 
 
-LAT_SPLIT_TARGET = 512     # workgroups a small latent-attention grid is split up to (over keys)
-LAT_SPLIT_MAX = 16
+LAT_SPLIT_TARGET = 256     # workgroups a small latent-attention grid is split up to (over keys): one a CU, what its LDS holds
+LAT_SPLIT_MAX = 64         # lanes of the wave that merges them
 
 
 def latent_splits(n_entries: int, heads: int, rows: int = LAT_ROWS) -> int:
-    """Key splits of a latent attention launch: grids with fewer than ``LAT_SPLIT_TARGET`` workgroups
-    (decode steps, short portions) split every row's keys over up to ``LAT_SPLIT_MAX`` workgroups."""
-    gx = ((1 if heads >= rows else rows // heads) * heads + rows - 1) // rows
-    return max(1, min(LAT_SPLIT_MAX, LAT_SPLIT_TARGET // max(1, n_entries * gx)))
+    """Key splits of a latent attention launch: grids with fewer than ``LAT_SPLIT_TARGET`` workgroups (decode steps, short portions) split
+    every row's keys over as many workgroups as one round of the CUs holds, up to ``LAT_SPLIT_MAX`` (splits without keys cost next to
+    nothing: those with keys are the first ones).  us with the merge, up to 16 splits and 512 workgroups / here, 16 heads: one of 4001 24.7
+    / 16.6, two of 8000 39.4 / 21.7, four of 300 to 1300 18.0 / 15.5, 24 of up to 316 17.4 / 15.1, 48 of 1000 34.0 / 28.3, a portion of 256 38.7 / 21.5.  More
+    than half a round of entries are split only into the three that nearly fill two: 150 tokens behind 1000 in one 68.8, in three 62.3."""
+    n = n_entries * (((1 if heads >= rows else rows // heads) * heads + rows - 1) // rows)
+    if n > LAT_SPLIT_TARGET // 2:
+        return 3 if 2 * LAT_SPLIT_TARGET // n >= 3 else 1
+    return min(LAT_SPLIT_MAX, LAT_SPLIT_TARGET // max(1, n))
 
 
 def latent_rows(x: torch.Tensor, rank: int, rot_dim: int, tokens: int, seqs: int) -> int:
