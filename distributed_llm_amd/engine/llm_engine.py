@@ -354,6 +354,7 @@ class LLMEngine:
                                       verbose=os.environ.get("DLLM_VERBOSE") == "1",
                                       frag=[] if m.lm_head_r is None else [b[:2] for b in big])
                     ops.gemm.reserve(self.device)
+            ops.gemm.autotune_prompts(m.prompt_shapes(), self.device)
             return
         shapes = set()
         L = m.layers[0]

@@ -103,8 +103,9 @@ _PROJECTIONS = ("proj", "out", "dqkv", "uq", "o", "up", "down", "in", "x", "dt",
 _FIRST = {"biased_attention": "proj", "latent_attention": "dqkv", "mlstm": "proj"}
 
 
-def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
-    """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy."""
+def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, keep_order: bool = False, prompt: bool = False) -> torch.Tensor:
+    """x @ w.T: the framework's tuned GEMM where it takes the shape, else the vendor GEMM.  ``wf``: the weight's fragment-major copy; ``prompt`` as
+    in ``ops.linear``."""
     if wf is not None and ops.gemm.dg_takes(x):
         return ops.linear(x, w, wf=wf, keep_order=keep_order)
     if wf is not None and ops.gemm.fg_takes(x, w.shape[0]):
@@ -112,7 +113,7 @@ def _mm(x: torch.Tensor, w: torch.Tensor, wf: Optional[torch.Tensor] = None, kee
     if (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1
             and x.shape[1] % 64 == 0 and w.shape[0] % 64 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and w.is_contiguous()):
-        return ops.linear(x, w)
+        return ops.linear(x, w, prompt=prompt)
     return F.linear(x, w)
 
 
@@ -120,7 +121,7 @@ def _pm(x: torch.Tensor, L: Dict[str, torch.Tensor], name: str) -> torch.Tensor:
     wf = L.get(name + "_r")
     if isinstance(x, ops.gemm.Tail):
         return x.linear(L[name], wf)
-    return _mm(x, L[name]) if wf is None else _mm(x, L[name], wf, L["order_kept"])
+    return _mm(x, L[name], wf, wf is not None and L["order_kept"], L["prompt"])
 
 
 class HybridModel:
@@ -162,6 +163,8 @@ class HybridModel:
         self._max_pos = 0
         raw = self._load(weights) if weights else self._random(seed, init_std)
         self._place(raw)
+        for L in self.layers:
+            L["prompt"] = dtype == torch.bfloat16 and not self.order_kept      # a prompt's products may take timed tiles (ops.linear)
         self.lm_head_r: Optional[torch.Tensor] = None
         if fragments:
             self.place_fragments()
@@ -619,6 +622,19 @@ class HybridModel:
             ([self.loop_in] if self.cfg.loop is not None else [])
         return sorted({tuple(w.shape) for w in ws if w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and w.numel() >= 1 << 22})
 
+    def prompt_shapes(self) -> List[Tuple[int, int, bool]]:
+        """(out, in, with a GELU behind it) of the projections that may take timed tiles for a prompt's rows: of a bf16 model that bears another
+        order of sums.  The engine times them."""
+        if self.dtype != torch.bfloat16 or self.order_kept:
+            return []
+        out = set()
+        for L, S in zip(self.layers, self.cfg.layers):
+            gelu = isinstance(S.mlp, DenseSpec) and not self.cfg.parallel_ff and (self._act_args(S.mlp) or ("",))[0] == "gelu"
+            for k in _PROJECTIONS:
+                if k in L and L[k].shape[0] % 64 == 0 and L[k].shape[1] % 64 == 0 and L[k].is_contiguous() and L[k].numel() >= 1 << 19:
+                    out.add((*L[k].shape, k == "up" and gelu))
+        return sorted(out)
+
     def weight_bytes(self) -> int:
         n = sum(x.numel() * x.element_size() for x in (self.embed, self.final_norm))
         if self.cfg.loop is not None:
@@ -1071,6 +1087,10 @@ class HybridModel:
         elif "up_r" in L and act is not None and act[0] == "gelu" and ops.gemm.fg_takes(x, L["up"].shape[0]):
             a = ops.gemm.f32_linear(x, L["up_r"], L["up"].shape[0], gelu=True)
         if a is None:
+            if act is not None and act[0] == "gelu" and L["prompt"]:
+                a = ops.gemm.prompt_gelu(x, L["up"])
+            if a is not None:
+                return _pm(a, L, "down")
             z = _pm(x, L, "up")
             if act is None:
                 a = seqmix.polynorm(z, L["act"], self.cfg.rms_eps)

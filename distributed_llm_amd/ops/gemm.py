@@ -180,6 +180,10 @@ class _Planner:
         self.pf_lin: Dict[Tuple[int, int], list] = {}        # (N, K) of prompts: [(rows, us)] of the vendor's product and its epilogue
         self.pf_parts: Dict[Tuple[int, int, int], Tuple] = {}        # prompt_parts' answers
         self.pf_vendor: Dict[Tuple[int, int, int], bool] = {}        # use_vendor_core's, for rows that are no bucket
+        # (N, K, 1 with a GELU behind it) of plain products of prompts: [(rows, us of the vendor's, GELU's launch included)], [(rows, us of
+        # each of _PP_PLANS)]
+        self.pp_times: Dict[Tuple[int, int, int], Tuple[list, list]] = {}
+        self.pp_plans: Dict[Tuple[int, int, int, int], Optional[Tuple]] = {}      # prompt_plan's answers
         self.cus = 256            # CUs of the device the prompt plans were timed on
         self.ws: Dict[Tuple, Tuple[torch.Tensor, torch.Tensor]] = {}
         self.sk_tables: Dict[Tuple, Tuple[torch.Tensor, int]] = {}   # stream-K segment lists per shape
@@ -417,6 +421,97 @@ def _vendor_at(M: int, N: int, K: int, bucket: bool) -> bool:
         return bucket
     lin = next((t for m, t in at if M <= m), at[-1][1] * M / at[-1][0])
     return _keep(_P.pf_vendor, key, us >= _VENDOR_GAIN * lin if bucket else lin < _VENDOR_GAIN * us)
+
+
+# Plain products of prompts (layer lists): the row counts at which the vendor's is timed, and the tiles timed beside it at some of them
+PP_MS = (*range(1280, 8193, 256), *range(8704, 12289, 512))
+PP_OWN_MS = (2048, 4096, 8192, 12288)
+_PP_PLANS = ((256, 256, 2, 1, 1, 4, 1, 0, 0, 64, 16, 8), (256, 128, 3, 1, 1, 8, 1, 8, 0, 64, 16, 8), (192, 128, 3, 1, 1, 8), (128, 128, 3, 1, 1, 8),
+             (64, 128, 3, 1, 1, 8))
+_PP_GAIN = 0.95           # estimates between timed sizes are within 5 % of what is measured
+
+
+def prompt_plan(M: int, N: int, K: int, gelu: bool = False) -> Optional[Tuple]:
+    """The tile on which M > MAX_M rows of x @ w.T [-> erf-GELU] run, or None: the vendor's product, or nothing was timed.  The vendor's time
+    steps up and down with the rows: 13312 x 2048 271 us at 6144 rows, 366 to 373 from 6200 to 7424, 349 from 7500 to 8192 (here 256,
+    291 to 316, 341 to 356), 6208 x 2048 111 at 5000, 190 at 7300, 155 at 7500 (105, 154, 152), 8192 x 2048 184 at 7308, 263 at 8193 (199, 242); so it is
+    timed every few hundred rows, and taken to cost what it does at the next of them.  A tile's time goes by rounds over the CUs."""
+    key = (M, N, K, int(gelu))
+    if key in _P.pp_plans:
+        return _P.pp_plans[key]
+    vendor, own = _P.pp_times.get(key[1:], ((), ()))
+    if not vendor or not own or M > 1.25 * vendor[-1][0]:
+        return None
+    us = next((t for m, t in vendor if M <= m), vendor[-1][1] * M / vendor[-1][0])
+    m0, times = next((e for e in own if M <= e[0]), own[-1])
+    best = None
+    for plan, t in zip(_PP_PLANS, times):
+        tiles = lambda m: -(-m // plan[0]) * -(-N // plan[1])
+        t *= _rounds(tiles(M), _P.cus) / _rounds(tiles(m0), _P.cus)
+        if 0 < t < _PP_GAIN * us and (best is None or t < best[0]):
+            best = (t, plan)
+    return _keep(_P.pp_plans, key, best and best[1])
+
+
+def autotune_prompts(shapes: Iterable[Tuple[int, int, bool]], device) -> None:
+    """Times the plain products of prompts, ``prompt_plan``'s choice: (N, K, with a GELU behind it) of each."""
+    from . import seqmix
+    dev = torch.device(device)
+    if dev.type != "cuda" or os.environ.get("DLLM_GEMM") == "blas":
+        return
+    cache = os.environ.get("DLLM_GEMM_PLANS")
+    made = _timed_with(dev) if cache else ""
+    if cache and os.path.exists(cache):
+        _load_plans(cache, made)
+    if _P.cus != _sk_grid(dev):
+        _P.cus = _sk_grid(dev)
+        _P.pf_parts.clear()
+        _P.pf_vendor.clear()
+        _P.pp_plans.clear()
+    for N, K, gelu in shapes:
+        key = (N, K, int(gelu))
+        if key in _P.pp_times:
+            continue
+        copies = max(2, min(8, (256 << 20) // (N * K * 2)))
+        ws = [(torch.randn(N, K, device=dev) * 0.02).to(torch.bfloat16) for _ in range(copies)]
+        most, vendor, own = PP_MS[-1], [], []
+        while most >= PP_MS[0]:      # (where so many rows find no memory, fewer are timed)
+            try:
+                X, Y = torch.randn(most, K, dtype=torch.bfloat16, device=dev), torch.empty(most, N, dtype=torch.bfloat16, device=dev)
+                break
+            except torch.OutOfMemoryError:
+                most //= 2
+        for M in (m for m in PP_MS if m <= most):
+            x, y = X[:M], Y[:M]
+
+            def call(i):
+                torch.matmul(x, ws[i % copies].t(), out=y)
+                if gelu:
+                    seqmix.gelu_erf(y)
+            vendor.append((M, _time(call, iters=4)))
+            if M in PP_OWN_MS:
+                epi, ext = EPI_GELU if gelu else EPI_PLAIN, _native(x)
+                own.append((M, [_time(lambda i: _tgemm(ext, x, ws[i % copies], epi, p, y=y), iters=4) for p in _PP_PLANS]))
+        _P.pp_times[key] = (vendor, own)
+    if cache:
+        _save_plans(cache, made)
+
+
+def prompt_gelu(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """``seqmix.gelu_erf(linear(x, w, prompt=True))`` in one launch where that is the faster form, else None."""
+    plan = prompt_plan(x.shape[0], *w.shape, True) if _prompt_rows(x, w) else None
+    if plan is None:
+        return None
+    y = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+    _tgemm(_native(x), x, w, EPI_GELU, plan, y=y)
+    return y
+
+
+def _prompt_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Rows and weights that the tiled GEMM reads, past the timed decode sizes."""
+    return (x.is_cuda and x.shape[0] > MAX_M and x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and
+            x.stride(0) >= x.shape[1] and w.is_contiguous() and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and
+            x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and os.environ.get("DLLM_GEMM") != "blas")
 
 
 def _row_parts(M: int, N: int, K: int, frag: bool = False) -> list:
@@ -727,12 +822,15 @@ def tail_takes(y: torch.Tensor, w: torch.Tensor, *vectors: Optional[torch.Tensor
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
-           wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None, keep_order: bool = False) -> torch.Tensor:
-    """``x @ w.T`` on the shape's tuned plan; ``wp``: the panel copy a tgemm plan streams, ``wf``: the fragment-major copy of the
+           wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None, keep_order: bool = False, prompt: bool = False) -> torch.Tensor:
+    """``x @ w.T`` on the shape's tuned plan; ``prompt``: many rows may take the tile timed for them (``prompt_plan``); ``wp``: the panel copy a tgemm plan streams, ``wf``: the fragment-major copy of the
     decode GEMM, which takes the untimed products of up to 64 rows with the splits and the order of sums they have without it, and
     timed ones where it was faster, or with ``keep_order`` where the plan is a skinny one, whose sums it keeps."""
     if not x.is_cuda or os.environ.get("DLLM_GEMM") == "blas":
         return F.linear(x, w) if out is None else torch.matmul(x, w.t(), out=out)
+    tile = prompt_plan(x.shape[0], *w.shape) if prompt and _prompt_rows(x, w) else None
+    if tile is not None:
+        return _run_plan(("tg",) + tile, x, w, False, out)
     plan, together, dg = _linear_plan(x, w, wf is not None, keep_order)
     if dg is not None and dg_takes(x):
         y = out if out is not None else torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
@@ -1128,6 +1226,8 @@ def _load_plans(path: str, timed_with: Optional[str] = None) -> None:
                 _P.pf_small[tuple(map(int, at))] = (tuple(v[0]), v[1])
             elif kind == "l":
                 _P.pf_lin[tuple(map(int, at))] = [tuple(e) for e in v]
+            elif kind == "m":
+                _P.pp_times[tuple(map(int, at))] = ([tuple(e) for e in v[0]], [(m, list(t)) for m, t in v[1]])
             elif kind == "p":
                 _P.pf_times[tuple(map(int, at))] = [(tuple(q), m, t) for q, m, t in v]
             elif kind == "d":
@@ -1150,6 +1250,7 @@ def _save_plans(path: str, timed_with: str = "") -> None:
     d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
     d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
     d.update({"l,%d,%d" % k: v for k, v in _P.pf_lin.items()})
+    d.update({"m,%d,%d,%d" % k: v for k, v in _P.pp_times.items()})
     d[_TIMED_WITH] = timed_with
     if os.path.dirname(path):
         os.makedirs(os.path.dirname(path), exist_ok=True)
@@ -1177,6 +1278,7 @@ def autotune(shapes: Iterable[Tuple[int, int, bool]], ms: Iterable[int], device,
         _P.cus = _sk_grid(dev)
         _P.pf_parts.clear()
         _P.pf_vendor.clear()
+        _P.pp_plans.clear()
     cache = os.environ.get("DLLM_GEMM_PLANS")  # JSON plan cache: re-use a previous run's choices
     made = _timed_with(dev) if cache else ""
     if cache and os.path.exists(cache):
