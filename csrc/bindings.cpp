@@ -22,6 +22,7 @@ int dllm_embed(const int*, const void*, void*, long, int, long, long, float*, in
 int dllm_gemv(const void*, long, const void*, void*, long, int, int, int, int, int, const void*, void*, const void*,
               float, hipStream_t);
 int dllm_gelu(const void*, void*, long, hipStream_t);
+int dllm_ln_pool_l2(const void*, const void*, const void*, float, const int*, float*, int, int, const int*, int, hipStream_t);
 int dllm_mean_pool_l2(const void*, const int*, float*, int, int, int, const int*, int, hipStream_t);
 int dllm_moe_gate(const float*, int, int, int, int*, float*, hipStream_t);
 int dllm_resadd_router(const void*, long, const float*, float, float*, void*, const float*, const void*, int, int, int, int, int*, float*, int, float,
@@ -159,7 +160,7 @@ int dllm_moe_tail_ok(int, int);
 int dllm_enc_gemm_ok(int, int, int);
 int dllm_enc_few_ok(int, int, int, int, int);
 int dllm_enc_few_layer(void*, void*, void*, void*, void*, const void* const*, const void*, const void*, int, int, int, int, float, float,
-                       const int*, const int*, int, int, hipStream_t);
+                       const int*, const int*, int, int, const int*, const int*, const void*, const void*, const void*, int, hipStream_t);
 int dllm_enc_gemm(const void*, long, const void*, const void*, void*, long, int, int, int, int, hipStream_t);
 int dllm_encoder_attention(const void*, const int*, void*, int, int, int, int, float, const int*, int, hipStream_t);
 int dllm_embed_ln(const int*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int,
@@ -1642,68 +1643,6 @@ bool enc_gemm(torch::Tensor x, torch::Tensor w, torch::Tensor bias, torch::Tenso
   return true;
 }
 
-// All layers of the sentence encoder over packed rows, in one call: seven launches a layer (four at up to 16 rows) back to back instead of seven calls
-// from the interpreter, whose 6 us each were most of a single text's 335 us.  weights: per layer QKV w, b, output w, b, norm w, b,
-// up w, b, down w, b, norm w, b.  plans (QKV, output, up, down): bm, bn, stages, splits, ks, waves, k-groups, loaders, k depth, mfma,
-// raster.  x [T, H] is overwritten; returns the last layer's rows.
-torch::Tensor encoder_layers(torch::Tensor x, torch::Tensor lens, torch::Tensor starts, int64_t S, int64_t nh, int64_t d, double eps,
-                             std::vector<torch::Tensor> weights, std::vector<std::vector<int64_t>> plans,
-                             c10::optional<torch::Tensor> part, c10::optional<torch::Tensor> counters) {
-  check_bf16(x, "x");
-  TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && x.size(1) == nh * d, "x [T, nh d]");
-  TORCH_CHECK(weights.size() % 12 == 0 && plans.size() == 4, "twelve tensors a layer, four plans");
-  for (auto& p : plans) TORCH_CHECK(p.size() == 11, "a plan has 11 entries");
-  const int64_t T = x.size(0), H = x.size(1), B = lens.numel();
-  if (weights.empty() || T == 0) return x;
-  const int64_t I = weights[6].size(0);
-  auto qkv = torch::empty({T, 3 * H}, x.options()), a = torch::empty({T, H}, x.options()), f = torch::empty({T, I}, x.options()),
-       y = torch::empty({T, H}, x.options());
-  const c10::optional<torch::Tensor> none;
-  const double scale = 1.0 / std::sqrt((double)d);
-  // up to 16 rows: four launches a layer (encoder.hip), if every weight is as those kernels read it
-  bool few = T <= 16 && dllm_enc_few_ok((int)T, (int)nh, (int)d, (int)I, (int)B) && S >= 1 && starts.numel() >= B && lens.is_contiguous() &&
-             starts.is_contiguous() && lens.scalar_type() == torch::kInt32 && starts.scalar_type() == torch::kInt32 && lens.is_cuda() &&
-             starts.is_cuda() && ((uintptr_t)x.data_ptr() & 15) == 0;
-  const int64_t rows[12] = {3 * H, 3 * H, H, H, H, H, I, I, H, H, H, H};
-  for (size_t i = 0; few && i < weights.size(); ++i) {
-    const auto& w = weights[i];
-    const int64_t k = i % 12, c = k == 0 || k == 2 || k == 6 ? H : k == 8 ? I : 0;
-    few = w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.is_contiguous() && ((uintptr_t)w.data_ptr() & 15) == 0 &&
-          (c ? w.dim() == 2 && w.size(0) == rows[k] && w.size(1) == c : w.numel() == rows[k]);
-  }
-  if (few) {
-    auto vt = torch::empty({H, 16}, x.options());
-    const void *ln_w = nullptr, *ln_b = nullptr;
-    for (size_t l = 0; l < weights.size(); l += 12) {
-      const void* w[10];
-      for (int i = 0; i < 10; ++i) w[i] = weights[l + i].data_ptr();
-      ok(dllm_enc_few_layer(x.data_ptr(), y.data_ptr(), qkv.data_ptr(), vt.data_ptr(), f.data_ptr(), w, ln_w, ln_b, (int)T, (int)nh, (int)d,
-                            (int)I, (float)eps, (float)scale, starts.data_ptr<int>(), lens.data_ptr<int>(), (int)B, (int)S, stream()),
-         "encoder layer");
-      ln_w = weights[l + 10].data_ptr();
-      ln_b = weights[l + 11].data_ptr();
-    }
-    norm(y, none, weights[weights.size() - 2], weights.back(), x, eps, true);
-    return x;
-  }
-  auto gemm = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& b, const torch::Tensor& out, int epi,
-                  const std::vector<int64_t>& p) {
-    if (!enc_gemm(in, w, b, out, epi)) tgemm(in, w, out, epi, p[0], p[1], p[2], p[3], p[4], p[5], part, counters, none, 0, 0.0, 0.0, none, none, none, none, none, none,
-          none, 0, 0, 0, b, p[6], p[7], none, 0, none, p[8], p[9], p[10]);
-  };
-  for (size_t l = 0; l < weights.size(); l += 12) {
-    const torch::Tensor* w = &weights[l];
-    gemm(x, w[0], w[1], qkv, 0, plans[0]);
-    encoder_attention(qkv, lens, a, B, S, nh, d, scale, starts);
-    gemm(a, w[2], w[3], x, 1, plans[1]);
-    norm(x, none, w[4], w[5], y, eps, true);
-    gemm(y, w[6], w[7], f, 4, plans[2]);
-    gemm(f, w[8], w[9], y, 1, plans[3]);
-    norm(y, none, w[10], w[11], x, eps, true);
-  }
-  return x;
-}
-
 void embed_ln(torch::Tensor ids, torch::Tensor word, torch::Tensor pos, torch::Tensor type0, torch::Tensor w,
               torch::Tensor b, torch::Tensor out, int64_t S, double eps, c10::optional<torch::Tensor> at) {
   check_i32(ids, "ids");
@@ -1723,6 +1662,111 @@ void embed_ln(torch::Tensor ids, torch::Tensor word, torch::Tensor pos, torch::T
                    out.data_ptr(), T, S, H, word.size(0), (float)eps, at ? at->data_ptr<int>() : nullptr, stream()),
      "embed_ln");
 }
+// All layers of the sentence encoder over packed rows, in one call: seven launches a layer (four at up to 16 rows) back to back instead of seven calls
+// from the interpreter, whose 6 us each were most of a single text's 335 us.  weights: per layer QKV w, b, output w, b, norm w, b,
+// up w, b, down w, b, norm w, b.  plans (QKV, output, up, down): bm, bn, stages, splits, ks, waves, k-groups, loaders, k depth, mfma,
+// raster.  x [T, H] is overwritten; returns the last layer's rows.  emb (ids [T], positions [T], word, pos, type0, norm w, b): x is made of them, up to
+// 16 rows in the first layer's first launch.  out [B, H] f32: the texts' unit means, of rows that the last LayerNorm's launch sums instead of storing.
+torch::Tensor encoder_layers(torch::Tensor x, torch::Tensor lens, torch::Tensor starts, int64_t S, int64_t nh, int64_t d, double eps,
+                             std::vector<torch::Tensor> weights, std::vector<std::vector<int64_t>> plans,
+                             c10::optional<torch::Tensor> part, c10::optional<torch::Tensor> counters, std::vector<torch::Tensor> emb,
+                             c10::optional<torch::Tensor> out) {
+  check_bf16(x, "x");
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && x.size(1) == nh * d, "x [T, nh d]");
+  TORCH_CHECK(emb.empty() || emb.size() == 7, "seven tensors make the rows");
+  TORCH_CHECK(weights.size() % 12 == 0 && plans.size() == 4, "twelve tensors a layer, four plans");
+  for (auto& p : plans) TORCH_CHECK(p.size() == 11, "a plan has 11 entries");
+  const int64_t T = x.size(0), H = x.size(1), B = lens.numel();
+  auto embed = [&] {
+    if (!emb.empty() && T) embed_ln(emb[0], emb[2], emb[3], emb[4], emb[5], emb[6], x, S, eps, emb[1]);
+  };
+  if (weights.empty() || T == 0) {
+    embed();
+    if (out) mean_pool_l2(x, lens, *out, starts);
+    return x;
+  }
+  // the last LayerNorm, of `from`, and what comes of its rows
+  auto last = [&](const torch::Tensor& from) {
+    const auto &w = weights[weights.size() - 2], &b = weights.back();
+    const auto aligned = [](const torch::Tensor& t) { return t.is_contiguous() && ((uintptr_t)t.data_ptr() & 15) == 0; };
+    if (!out || H > 512 || H % 8 || B == 0 || !aligned(from) || !aligned(w) || !aligned(b)) {
+      norm(from, c10::nullopt, w, b, x, eps, true);
+      if (out) mean_pool_l2(x, lens, *out, starts);
+      return;
+    }
+    check_bf16(w, "norm weight");
+    check_bf16(b, "norm bias");
+    check_i32(lens, "lens");
+    check_i32(starts, "starts");
+    check_f32(*out, "out");
+    TORCH_CHECK(w.numel() == H && b.numel() == H && lens.is_contiguous() && starts.is_contiguous() && starts.numel() >= B && out->is_contiguous() &&
+                    out->size(0) == B && out->size(1) == H, "shapes");
+    ok(dllm_ln_pool_l2(from.data_ptr(), w.data_ptr(), b.data_ptr(), (float)eps, lens.data_ptr<int>(), out->data_ptr<float>(), (int)B, (int)H,
+                       starts.data_ptr<int>(), (int)T, stream()),
+       "ln_pool_l2");
+  };
+  const int64_t I = weights[6].size(0);
+  auto qkv = torch::empty({T, 3 * H}, x.options()), a = torch::empty({T, H}, x.options()), f = torch::empty({T, I}, x.options()),
+       y = torch::empty({T, H}, x.options());
+  const c10::optional<torch::Tensor> none;
+  const double scale = 1.0 / std::sqrt((double)d);
+  // up to 16 rows: four launches a layer (encoder.hip), if every weight is as those kernels read it
+  bool few = T <= 16 && dllm_enc_few_ok((int)T, (int)nh, (int)d, (int)I, (int)B) && S >= 1 && starts.numel() >= B && lens.is_contiguous() &&
+             starts.is_contiguous() && lens.scalar_type() == torch::kInt32 && starts.scalar_type() == torch::kInt32 && lens.is_cuda() &&
+             starts.is_cuda() && ((uintptr_t)x.data_ptr() & 15) == 0;
+  const int64_t rows[12] = {3 * H, 3 * H, H, H, H, H, I, I, H, H, H, H};
+  for (size_t i = 0; few && i < weights.size(); ++i) {
+    const auto& w = weights[i];
+    const int64_t k = i % 12, c = k == 0 || k == 2 || k == 6 ? H : k == 8 ? I : 0;
+    few = w.is_cuda() && w.scalar_type() == torch::kBFloat16 && w.is_contiguous() && ((uintptr_t)w.data_ptr() & 15) == 0 &&
+          (c ? w.dim() == 2 && w.size(0) == rows[k] && w.size(1) == c : w.numel() == rows[k]);
+  }
+  if (few) {
+    auto vt = torch::empty({H, 16}, x.options());
+    const void *ln_w = nullptr, *ln_b = nullptr;      // of the LayerNorm that the next layer's first launch takes
+    // rows made in the first launch, where their operands are as it reads them
+    bool made = !emb.empty();
+    for (size_t i = 0; made && i < emb.size(); ++i) {
+      const auto& t = emb[i];
+      made = t.is_cuda() && t.is_contiguous() && t.scalar_type() == (i < 2 ? torch::kInt32 : torch::kBFloat16) && ((uintptr_t)t.data_ptr() & (i < 2 ? 3 : 15)) == 0 &&
+             (i < 2 ? t.numel() == T : i < 4 ? t.dim() == 2 && t.size(1) == H && t.size(0) >= (i == 3 ? S : 1) : t.numel() == H);
+    }
+    if (!made) embed();
+    else { ln_w = emb[5].data_ptr(); ln_b = emb[6].data_ptr(); }
+    for (size_t l = 0; l < weights.size(); l += 12) {
+      const void* w[10];
+      for (int i = 0; i < 10; ++i) w[i] = weights[l + i].data_ptr();
+      ok(dllm_enc_few_layer(x.data_ptr(), y.data_ptr(), qkv.data_ptr(), vt.data_ptr(), f.data_ptr(), w, ln_w, ln_b, (int)T, (int)nh, (int)d,
+                            (int)I, (float)eps, (float)scale, starts.data_ptr<int>(), lens.data_ptr<int>(), (int)B, (int)S,
+                            made && l == 0 ? emb[0].data_ptr<int>() : nullptr, made ? emb[1].data_ptr<int>() : nullptr, made ? emb[2].data_ptr() : nullptr,
+                            made ? emb[3].data_ptr() : nullptr, made ? emb[4].data_ptr() : nullptr, made ? (int)emb[2].size(0) : 0, stream()),
+         "encoder layer");
+      ln_w = weights[l + 10].data_ptr();
+      ln_b = weights[l + 11].data_ptr();
+    }
+    last(y);
+    return x;
+  }
+  embed();
+  auto gemm = [&](const torch::Tensor& in, const torch::Tensor& w, const torch::Tensor& b, const torch::Tensor& out, int epi,
+                  const std::vector<int64_t>& p) {
+    if (!enc_gemm(in, w, b, out, epi)) tgemm(in, w, out, epi, p[0], p[1], p[2], p[3], p[4], p[5], part, counters, none, 0, 0.0, 0.0, none, none, none, none, none, none,
+          none, 0, 0, 0, b, p[6], p[7], none, 0, none, p[8], p[9], p[10]);
+  };
+  for (size_t l = 0; l < weights.size(); l += 12) {
+    const torch::Tensor* w = &weights[l];
+    gemm(x, w[0], w[1], qkv, 0, plans[0]);
+    encoder_attention(qkv, lens, a, B, S, nh, d, scale, starts);
+    gemm(a, w[2], w[3], x, 1, plans[1]);
+    norm(x, none, w[4], w[5], y, eps, true);
+    gemm(y, w[6], w[7], f, 4, plans[2]);
+    gemm(f, w[8], w[9], y, 1, plans[3]);
+    if (l + 12 < weights.size()) norm(y, none, w[10], w[11], x, eps, true);
+  }
+  last(y);
+  return x;
+}
+
 // ---- sequence mixers and the f32 residual stream (csrc/kernels/seqmix.hip, latent.hip).
 // Activations are bf16 or f32; `act_f32` reports which and checks that a tensor is one of the two.
 bool act_f32(const torch::Tensor& t, const char* name) {
@@ -3015,7 +3059,9 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none(), py::arg("up_w") = py::none(),
         py::arg("gate") = py::none(), py::arg("up_out") = py::none());
   m.def("latent_mfma_ok", [](int64_t rank, int64_t rot, int64_t rows) { return dllm_latent_mfma_ok((int)rank, (int)rot, (int)rows) != 0; });
-  m.def("encoder_layers", &encoder_layers);
+  m.def("encoder_layers", &encoder_layers, py::arg("x"), py::arg("lens"), py::arg("starts"), py::arg("S"), py::arg("nh"), py::arg("d"), py::arg("eps"),
+        py::arg("weights"), py::arg("plans"), py::arg("part") = py::none(), py::arg("counters") = py::none(),
+        py::arg("emb") = std::vector<torch::Tensor>(), py::arg("out") = py::none());
   m.def("enc_gemm", &enc_gemm);
   m.def("encoder_attention", &encoder_attention, py::arg("qkv"), py::arg("lens"), py::arg("out"), py::arg("B"), py::arg("S"), py::arg("nh"), py::arg("d"), py::arg("scale"), py::arg("starts") = py::none());
   m.def("embed_ln", &embed_ln, py::arg("ids"), py::arg("word"), py::arg("pos"), py::arg("type0"), py::arg("w"), py::arg("b"), py::arg("out"), py::arg("S"), py::arg("eps"), py::arg("positions") = py::none());

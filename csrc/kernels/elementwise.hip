@@ -127,6 +127,57 @@ __global__ void __launch_bounds__(256) mean_pool_l2_kernel(const u16* __restrict
   }
 }
 
+// The same behind a LayerNorm (norm.hip's arithmetic, each row rounded as it leaves there), rows of at most 512: eight waves a text, each with four
+// rows in flight.  96 texts of up to 72 tokens x 384: 7.1 us, the two launches 11.2; one text of 12: 3.3.
+__global__ void __launch_bounds__(512) ln_pool_l2_kernel(const u16* __restrict__ x, const u16* __restrict__ w, const u16* __restrict__ bias, float eps,
+                                                         const int* __restrict__ lens, float* __restrict__ out, int H, const int* __restrict__ starts,
+                                                         int T) {
+  constexpr int NW = 8;
+  __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) float part[NW][512];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = 8 * lane;
+  const int row0 = min(max(starts[b], 0), T), n = min(max(lens[b], 0), T - row0);
+  const bool on = c < H;
+  const u16* xr = x + (long)row0 * H + (on ? c : 0);
+  float gw[8], gb[8], acc[8] = {};
+  unpack8(on ? ld16(w + c) : make_uint4(0u, 0u, 0u, 0u), gw);
+  unpack8(on ? ld16(bias + c) : make_uint4(0u, 0u, 0u, 0u), gb);
+  for (int s = wave; s < n; s += 4 * NW) {
+    uint4 r[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) r[u] = ld16(xr + (long)min(s + u * NW, n - 1) * H);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s + u * NW >= n) break;      // (uniform)
+      float v[8], sum = 0.f, q = 0.f, o[8];
+      unpack8(on ? r[u] : make_uint4(0u, 0u, 0u, 0u), v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum += v[j];
+      const float mean = wave_sum(sum) / H;
+      if (on)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) { const float d = v[j] - mean; q += d * d; }
+      const float rstd = rsqrtf(wave_sum(q) / H + eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (v[j] - mean) * rstd * gw[j] + gb[j];
+      unpack8(pack8(o), o);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] += o[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) part[wave][c + j] = acc[j];
+  __syncthreads();
+  float y = 0.f;
+  if ((int)threadIdx.x < H) {
+#pragma unroll
+    for (int g = 0; g < NW; ++g) y += part[g][threadIdx.x];
+    y *= n > 0 ? 1.f / n : 0.f;
+  }
+  const float sc = 1.f / fmaxf(sqrtf(block_sum(y * y, red)), 1e-12f);
+  if ((int)threadIdx.x < H) out[(long)b * H + threadIdx.x] = y * sc;
+}
+
 // widths that are no whole vectors (H <= 1024)
 __global__ void __launch_bounds__(256) mean_pool_any_kernel(const u16* __restrict__ x, const int* __restrict__ lens,
                                                             float* __restrict__ out, int S, int H,
@@ -477,6 +528,14 @@ extern "C" int dllm_gelu(const void* x, void* y, long n, hipStream_t stream) {
   if (n % 8 != 0) return -1;
   if (n == 0) return 0;
   hipLaunchKernelGGL(gelu_kernel, dim3(grid_for(n / 8, 256)), dim3(256), 0, stream, (const u16*)x, (u16*)y, n / 8);
+  return (int)hipGetLastError();
+}
+
+// x [T, H] packed rows, 16-byte aligned, H % 8 == 0 and H <= 512
+extern "C" int dllm_ln_pool_l2(const void* x, const void* w, const void* b, float eps, const int* lens, float* out, int B, int H, const int* starts,
+                               int T, hipStream_t stream) {
+  if (H < 8 || H % 8 || H > 512 || B < 1) return -1;
+  hipLaunchKernelGGL(ln_pool_l2_kernel, dim3(B), dim3(512), 0, stream, (const u16*)x, (const u16*)w, (const u16*)b, eps, lens, out, H, starts, T);
   return (int)hipGetLastError();
 }
 

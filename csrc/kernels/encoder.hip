@@ -42,6 +42,14 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   const u16* base = qkv + row0 * ld;
   const int len = min(lens[b], S);
 
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, rl = lane & 15;
+  const int q0 = (int)blockIdx.x * 64 + wave * 16;  // this wave's first query row
+  const int q = q0 + rl;                             // this lane's query row
+  bf16x8 qf[KSTEPS];                                 // on its way beside the keys: behind the barrier it was a trip of its own
+#pragma unroll
+  for (int s = 0; s < KSTEPS; ++s)
+    qf[s] = __builtin_bit_cast(bf16x8, q < S ? ld16(base + (long)q * ld + h * D + 8 * g + 32 * s) : make_uint4(0, 0, 0, 0));
+
   // ---- stage K rows and V^T for the whole sequence (zero past S)
   for (int e = threadIdx.x; e < SP * CPR; e += blockDim.x) {
     const int key = e / CPR, c = (e % CPR) * 8;
@@ -60,15 +68,7 @@ __global__ void __launch_bounds__(256) encoder_attn_kernel(const u16* __restrict
   }
   __syncthreads();
 
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, rl = lane & 15;
-  const int q0 = (int)blockIdx.x * 64 + wave * 16;  // this wave's first query row
-  const int q = q0 + rl;                             // this lane's query row
   if (q0 >= S) return;                               // wave-uniform: no barrier follows
-  bf16x8 qf[KSTEPS];
-#pragma unroll
-  for (int s = 0; s < KSTEPS; ++s)
-    qf[s] = __builtin_bit_cast(bf16x8, q < S ? ld16(base + (long)q * ld + h * D + 8 * g + 32 * s) : make_uint4(0, 0, 0, 0));
-
   f32x4 acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -254,21 +254,33 @@ struct FewW {
   }
 };
 
+// What a row is made of where the embeddings are summed in the launch (embed_ln_kernel's arithmetic)
+struct FewEmb { const int *ids, *at; const u16 *word, *pos, *type0; int S, vocab; };
+
 // EPI ENC_QKV: columns of q and k as they are, to Y; those of v transposed, to Vt [H][16], zero from row M on, as attn_out reads them.
-// ENC_GELU as in enc_gemm.  LN: X is the sum that a LayerNorm takes (norm.hip's arithmetic, a wave a row); the first workgroup stores
-// its rows to Xn for the residual sum that follows.
-template <int EPI, bool LN>
+// ENC_GELU as in enc_gemm.  IN 1: X is the sum that a LayerNorm takes (norm.hip's arithmetic, a wave a row); 2: that sum is made here, of
+// the embeddings `e` (6.2 us for 4.6: the ids come first; as a launch of its own 4 and the gap between two); the first workgroup stores its rows to Xn for the residual sum that follows.
+template <int EPI, int IN>
 __global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ X, const u16* __restrict__ W, const u16* __restrict__ bias,
                                                         u16* __restrict__ Y, int M, int N, int K, const u16* __restrict__ lnw,
-                                                        const u16* __restrict__ lnb, float eps, u16* __restrict__ Xn, u16* __restrict__ Vt) {
+                                                        const u16* __restrict__ lnb, float eps, u16* __restrict__ Xn, u16* __restrict__ Vt,
+                                                        FewEmb e) {
+  constexpr bool LN = IN != 0;
   __shared__ __attribute__((aligned(16))) u16 sx[FEW_M * FEW_LD];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.x * 16, steps = K / 32, c = 8 * lane;
-  uint4 xv = {}, gw = {}, gb = {};
+  uint4 xv = {}, gw = {}, gb = {}, pv = {}, tv = {};
   FewW wf;
   float b = 0.f;
+  const int t = min(w, M - 1);        // rows past M repeat the last and are dropped
+  const u16 *xr = X + (long)t * K, *pr = nullptr;
+  if constexpr (IN == 2) {
+    xr = e.word + (long)min(max(e.ids[t], 0), e.vocab - 1) * K;
+    pr = e.pos + (long)min(max(e.at[t], 0), e.S - 1) * K;
+  }
   if (c < K) {
-    xv = ld16(X + (long)min(w, M - 1) * K + c);        // rows past M repeat the last and are dropped
+    xv = ld16(xr + c);
+    if constexpr (IN == 2) { pv = ld16(pr + c); tv = ld16(e.type0 + c); }
     if (LN) { gw = ld16(lnw + c); gb = ld16(lnb + c); }
   }
   if (w == 0) {
@@ -278,6 +290,13 @@ __global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ 
   if (LN) {
     float v[8], s = 0.f, q = 0.f, ga[8], be[8];
     unpack8(xv, v);
+    if constexpr (IN == 2) {
+      float a[8], y[8];
+      unpack8(pv, a);
+      unpack8(tv, y);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = v[j] + a[j] + y[j];
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) s += v[j];
     const float mean = wave_sum(s) / K;
@@ -517,22 +536,25 @@ extern "C" int dllm_enc_few_ok(int M, int nh, int d, int I, int B) {
   return M >= 1 && M <= FEW_M && B >= 1 && B <= 64 && (d == 32 || d == 64) && nh >= 1 && nh * d <= FEW_K && I >= 32 && I % 32 == 0;
 }
 
-// One layer on M packed rows.  x [M, H]: the rows, or (ln0w) where they go: they are the LayerNorm of the sums in y.  Leaves the next
-// sums in y.  w: QKV w, b, output w, b, norm w, b, up w, b, down w, b.  qkv [M, 3H], vt [H, 16], f [M, I].  Operands 16-byte aligned,
-// rows contiguous.
+// One layer on M packed rows.  x [M, H]: the rows, or (ln0w) where they go: they are the LayerNorm of the sums in y, or with ids of the sums of
+// embeddings word[ids] + pos[at] + type0.  Leaves the next sums in y.  w: QKV w, b, output w, b, norm w, b, up w, b, down w, b.  qkv [M, 3H], vt [H, 16],
+// f [M, I].  Operands 16-byte aligned, rows contiguous.
 extern "C" int dllm_enc_few_layer(void* x, void* y, void* qkv, void* vt, void* f, const void* const* w, const void* ln0w, const void* ln0b,
                                   int M, int nh, int d, int I, float eps, float scale, const int* starts, const int* lens, int B, int S,
-                                  hipStream_t st) {
-  if (!dllm_enc_few_ok(M, nh, d, I, B)) return -1;
+                                  const int* ids, const int* at, const void* word, const void* pos, const void* type0, int vocab, hipStream_t st) {
+  if (!dllm_enc_few_ok(M, nh, d, I, B) || (ids && !ln0w)) return -1;
   u16 *X = (u16*)x, *Y = (u16*)y, *Q = (u16*)qkv, *V = (u16*)vt, *F = (u16*)f;
   const u16* const* W = reinterpret_cast<const u16* const*>(w);
   const int H = nh * d;
   const dim3 rows(64 * FEW_M), heads(64 * nh);
-  if (ln0w) hipLaunchKernelGGL((enc_rows_kernel<ENC_QKV, true>), dim3(3 * H / 16), rows, 0, st, Y, W[0], W[1], Q, M, 3 * H, H, (const u16*)ln0w, (const u16*)ln0b, eps, X, V);
-  else hipLaunchKernelGGL((enc_rows_kernel<ENC_QKV, false>), dim3(3 * H / 16), rows, 0, st, X, W[0], W[1], Q, M, 3 * H, H, nullptr, nullptr, eps, nullptr, V);
+  const FewEmb e{ids, at, (const u16*)word, (const u16*)pos, (const u16*)type0, S, vocab};
+#define QKV(IN, FROM) \
+  hipLaunchKernelGGL((enc_rows_kernel<ENC_QKV, IN>), dim3(3 * H / 16), rows, 0, st, FROM, W[0], W[1], Q, M, 3 * H, H, (const u16*)ln0w, (const u16*)ln0b, eps, X, V, e)
+  if (ids) QKV(2, X); else if (ln0w) QKV(1, Y); else QKV(0, X);
+#undef QKV
   if (d == 32) hipLaunchKernelGGL(attn_out_kernel<32>, dim3(H / 16), heads, 0, st, Q, V, W[2], W[3], X, M, nh, scale * LOG2E, starts, lens, B, S);
   else hipLaunchKernelGGL(attn_out_kernel<64>, dim3(H / 16), heads, 0, st, Q, V, W[2], W[3], X, M, nh, scale * LOG2E, starts, lens, B, S);
-  hipLaunchKernelGGL((enc_rows_kernel<ENC_GELU, true>), dim3(I / 16), rows, 0, st, X, W[6], W[7], F, M, I, H, W[4], W[5], eps, Y, nullptr);
+  hipLaunchKernelGGL((enc_rows_kernel<ENC_GELU, 1>), dim3(I / 16), rows, 0, st, X, W[6], W[7], F, M, I, H, W[4], W[5], eps, Y, nullptr, e);
   const int rc = (int)hipGetLastError();
   return rc ? rc : dllm_enc_gemm(F, I, W[8], W[9], Y, H, M, H, I, ENC_RESADD, st);
 }

@@ -153,16 +153,15 @@ class MiniLMEncoder:
     def _forward(self, texts: List[str], max_len: int) -> torch.Tensor:
         """One packed batch through the HIP encoder (the texts' rows one behind the other, no padding): fused embedding+LN,
         per layer 4 tgemm launches (QKV + bias, Wo + bias + residual, W1 + bias + GELU, W2 + bias + residual), the encoder
-        attention kernel and 2 LayerNorms; mean-pool + L2 (csrc/kernels/encoder.hip, tgemm.hip, norm.hip, elementwise.hip).
+        attention kernel and 2 LayerNorms, the last of which ends in the mean-pool + L2 (csrc/kernels/encoder.hip, tgemm.hip, norm.hip, elementwise.hip).
         CPU tensors run the same graph on ops.reference."""
         cfg = self.cfg
         packed, T, S = self.tok.pack(texts, max_len)
         B = len(texts)
         ids, at_d, starts_d, lens_d = packed.to(self.device).split([T, T, B, B])
         H, nh = cfg.hidden, cfg.heads
-        x = ops.embed_ln(ids, self.word, self.pos, self.type0, *self.emb_ln, S, cfg.eps, at_d)
-        x = ops.gemm.encoder_layers(x, lens_d, starts_d, S, nh, H // nh, cfg.eps, self.layers)
-        return ops.mean_pool_l2(x, lens_d, starts_d)
+        return ops.gemm.encoder_texts(ids, at_d, (self.word, self.pos, self.type0, *self.emb_ln), lens_d, starts_d, S, nh, H // nh, cfg.eps,
+                                      self.layers)
 
     @torch.no_grad()
     def reference_forward(self, texts: List[str], max_len: int = 256) -> torch.Tensor:

@@ -1113,31 +1113,56 @@ def encoder_layers(x: torch.Tensor, lens: torch.Tensor, starts: torch.Tensor, S:
     are overwritten: QKV, attention, output + residual, LayerNorm, up + GELU, down + residual, LayerNorm.  On the GPU one call
     launches them all."""
     from . import encoder_attention, layer_norm
-    T, H = x.shape
-    names = ("wqkv", "wo", "w1", "w2")
-    if T and layers and x.is_contiguous() and all(_enc_ok(x, L[n]) for L in layers for n in names):
-        shapes = [tuple(layers[0][n].shape) for n in names]
-        plans = [tg_plan(T, n, k) for n, k in shapes]
-        if all(tuple(L[n].shape) == s for L in layers for n, s in zip(names, shapes)) and not any(p[8:9] == (1,) for p in plans):
-            full, floats, tiles = [], 0, 0
-            for p, (n, k) in zip(plans, shapes):
-                p = p + (1, 4, 1, 0, 0, 64, 16, 0)[len(p) - 4:]
-                if k % (64 * p[4]):
-                    p = p[:4] + (1, p[5], 1) + p[7:]
-                if _tg_splits(k, p[3], p[4]) > 1:
-                    fl, ti = _need_tg(T, n, k, p[0], p[1], p[3], p[4])
-                    floats, tiles = max(floats, fl), max(tiles, ti)
-                full.append(list(p[:8] + p[9:]))
-            part, cnt = _P.workspace(x.device, floats, tiles) if tiles else (None, None)
-            return _native(x).encoder_layers(x, lens, starts, int(S), int(nh), int(d), float(eps),
-                                             [t for L in layers for t in (L["wqkv"], L["bqkv"], L["wo"], L["bo"], *L["ln1"], L["w1"], L["b1"],
-                                                                          L["w2"], L["b2"], *L["ln2"])], full, part, cnt)
+    plan = _encoder_plan(x, layers)
+    if plan:
+        return _native(x).encoder_layers(x, lens, starts, int(S), int(nh), int(d), float(eps), *plan)
     for L in layers:
         a = encoder_attention(linear_bias(x, L["wqkv"], L["bqkv"]), lens, lens.numel(), S, nh, d, starts=starts)
         x = layer_norm(linear_bias_residual(a, L["wo"], L["bo"], x), *L["ln1"], eps)
         f = linear_bias(x, L["w1"], L["b1"], gelu=True)
         x = layer_norm(linear_bias_residual(f, L["w2"], L["b2"], x), *L["ln2"], eps)
     return x
+
+
+def encoder_texts(ids: torch.Tensor, at: torch.Tensor, emb, lens: torch.Tensor, starts: torch.Tensor, S: int, nh: int, d: int, eps: float,
+                  layers) -> torch.Tensor:
+    """Unit vectors [B, nh d] (f32) of packed texts: embeddings (``emb``: word, pos, type0, norm w, b), ``encoder_layers``, mean over each text's
+    rows.  On the GPU one call, whose first and last launches hold the embeddings (up to 16 rows) and the mean."""
+    from . import embed_ln, mean_pool_l2
+    T, word = ids.numel(), emb[0]
+    # past 16 rows a launch of its own, under way while this call is prepared (inside it 96 texts took 10 us more)
+    few = T <= 16 and word.is_cuda
+    x = torch.empty((T, word.shape[1]), dtype=word.dtype, device=word.device) if few else embed_ln(ids, *emb, S, eps, at)
+    plan = _encoder_plan(x, layers)
+    if not plan:
+        x = embed_ln(ids, *emb, S, eps, at) if few else x
+        return mean_pool_l2(encoder_layers(x, lens, starts, S, nh, d, eps, layers), lens, starts)
+    out = torch.empty((lens.numel(), word.shape[1]), dtype=torch.float32, device=word.device)
+    _native(x).encoder_layers(x, lens, starts, int(S), int(nh), int(d), float(eps), *plan, [ids, at, *emb] if few else [], out)
+    return out
+
+
+def _encoder_plan(x: torch.Tensor, layers):
+    """Weights, plans and scratch of the native encoder on rows like x (None: not its shapes)."""
+    T, names = x.shape[0], ("wqkv", "wo", "w1", "w2")
+    if not (T and layers and x.is_contiguous() and all(_enc_ok(x, L[n]) for L in layers for n in names)):
+        return None
+    shapes = [tuple(layers[0][n].shape) for n in names]
+    plans = [tg_plan(T, n, k) for n, k in shapes]
+    if any(tuple(L[n].shape) != s for L in layers for n, s in zip(names, shapes)) or any(p[8:9] == (1,) for p in plans):
+        return None
+    full, floats, tiles = [], 0, 0
+    for p, (n, k) in zip(plans, shapes):
+        p = p + (1, 4, 1, 0, 0, 64, 16, 0)[len(p) - 4:]
+        if k % (64 * p[4]):
+            p = p[:4] + (1, p[5], 1) + p[7:]
+        if _tg_splits(k, p[3], p[4]) > 1:
+            fl, ti = _need_tg(T, n, k, p[0], p[1], p[3], p[4])
+            floats, tiles = max(floats, fl), max(tiles, ti)
+        full.append(list(p[:8] + p[9:]))
+    part, cnt = _P.workspace(x.device, floats, tiles) if tiles else (None, None)
+    weights = [t for L in layers for t in (L["wqkv"], L["bqkv"], L["wo"], L["bo"], *L["ln1"], L["w1"], L["b1"], L["w2"], L["b2"], *L["ln2"])]
+    return weights, full, part, cnt
 
 
 def max_slots(N: int, M: int = 0) -> int:
