@@ -333,7 +333,7 @@ __global__ void __launch_bounds__(256 * VS) dgemm_kernel(DgArgs a) {
         o.v[j] = f2bf(x1[i][j]);
         if constexpr (EPI == DG_GELU) {
           const float v = bf2f(o.v[j]);
-          o.v[j] = f2bf(0.5f * v * (1.f + erff(v * 0.70710678118654752f)));
+          o.v[j] = f2bf(gelu_bf(v));
         }
       }
       u16* y = a.Y + (long)m * a.ldy + c;

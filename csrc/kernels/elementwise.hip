@@ -70,7 +70,7 @@ __global__ void gelu_kernel(const u16* __restrict__ x, u16* __restrict__ y, long
     float f[8];
     unpack8(ld16(x + v * 8), f);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = 0.5f * f[j] * (1.f + erff(f[j] * 0.70710678118654752f));
+    for (int j = 0; j < 8; ++j) f[j] = gelu_bf(f[j]);
     st16(y + v * 8, pack8(f));
   }
 }

@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(64 * NW) enc_gemm_kernel(const u16* __restrict
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float z = bf2f(f2bf(v[i] + bf2f(b.v[i])));               // the projection's own rounding, as in the tiled form
-    o.v[i] = f2bf(EPI == ENC_GELU ? 0.5f * z * (1.f + erff(z * 0.70710678118654752f)) : EPI == ENC_RESADD ? z + bf2f(r.v[i]) : z);
+    o.v[i] = f2bf(EPI == ENC_GELU ? gelu_bf(z) : EPI == ENC_RESADD ? z + bf2f(r.v[i]) : z);
   }
   *reinterpret_cast<u16x4*>(Y + (long)row * ldy + col0 + c) = o;
 }
@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(1024) enc_rows_kernel(const u16* __restrict__ 
   for (int i = 0; i < 4; ++i)
     if (4 * g + i < M) {
       const float z = bf2f(f2bf(v[i] + b));
-      Y[(long)(4 * g + i) * N + col0 + lr] = f2bf(EPI == ENC_GELU ? 0.5f * z * (1.f + erff(z * 0.70710678118654752f)) : z);
+      Y[(long)(4 * g + i) * N + col0 + lr] = f2bf(EPI == ENC_GELU ? gelu_bf(z) : z);
     }
 }
 

@@ -75,7 +75,6 @@ __device__ __forceinline__ void block_sync_lds() {
 
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
 __device__ __forceinline__ float bfr(float x) { return bf2f(f2bf(x)); }
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 // KS: 64-deep k sub-tiles per ring stage (one barrier per stage); NW: waves per k-group, laid out
 // WGM (M) x NW/WGM (N), each wave a (BM/WGM) x (BN/(NW/WGM)) tile; WK: k-groups (1, or 2 with
@@ -658,7 +657,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
 #pragma unroll
             for (int j = 0; j < FN32; ++j) {
               float x = acc32[i][j][v] * ri + bcol[j];
-              if constexpr (EPI == EPI_GELU) x = gelu_erf(bfr(x));
+              if constexpr (EPI == EPI_GELU) x = gelu_bf(bfr(x));
               so[rl * OLD + wn * WN + 32 * j + lc] = f2bf(x);
             }
           }
@@ -711,7 +710,7 @@ __device__ __forceinline__ void tgemm_unit(const GemmArgs& a, unsigned char* sme
 #pragma unroll
           for (int j = 0; j < FN; ++j) {
             float v = acc[i][j][e] * rinv[i][e] + bcol[j];
-            if constexpr (EPI == EPI_GELU) v = gelu_erf(bfr(v));  // GELU of the bf16 linear output
+            if constexpr (EPI == EPI_GELU) v = gelu_bf(bfr(v));  // GELU of the bf16 linear output
             if constexpr (EPI == EPI_RELU2) v = fmaxf(v, 0.f) * fmaxf(v, 0.f);
             so[rl * OLD + wn * WN + 16 * j + cl] = f2bf(v);
           }

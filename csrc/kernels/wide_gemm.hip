@@ -30,7 +30,6 @@ constexpr int KD = 64, ROW = 2 * KD;      // k depth of a stage, bytes of a stag
 __device__ __forceinline__ int swizzle(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
 __device__ __forceinline__ float bfr(float x) { return bf2f(f2bf(x)); }
-__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 // Two fragments of a row (a lane holds columns 4 g .. 4 g + 3 of each): 16 bytes, columns 16 (g & 1) + 8 (g >> 1) .. + 7 of the 32
 __device__ __forceinline__ uint4 join(const float* a, const float* b) {
@@ -248,7 +247,7 @@ __global__ void __launch_bounds__(256) wide_gemm_kernel(GemmArgs a) {
             } else {
               float x = acc[i][2 * v + h][e] * ri;
               if constexpr (EPI != EPI_RELU2) x += bias[2 * v + h][e];
-              if constexpr (EPI == EPI_GELU) x = gelu_erf(bfr(x));      // GELU of the bf16 linear output
+              if constexpr (EPI == EPI_GELU) x = gelu_bf(bfr(x));      // GELU of the bf16 linear output
               if constexpr (EPI == EPI_RELU2) x = fmaxf(x, 0.f) * fmaxf(x, 0.f);
               p[h][e] = x;
             }
