@@ -177,6 +177,7 @@ class _Planner:
         self.fused_opts: Dict[Tuple[int, int, int], Dict[str, float]] = {}   # measured us per core choice
         self.pf_times: Dict[Tuple[int, int], list] = {}      # (N, K) of prompts: [(plan, rows, us)]
         self.pf_small: Dict[Tuple[int, int, int], Tuple] = {}        # (rows of PF_SMALL_MS, N, K): (fastest plan, its us)
+        self.pf_tail: Dict[Tuple[int, int, int], Tuple] = {}        # the same of PF_TAIL_MS
         self.pf_lin: Dict[Tuple[int, int], list] = {}        # (N, K) of prompts: [(rows, us)] of the vendor's product and its epilogue
         self.pf_parts: Dict[Tuple[int, int, int], Tuple] = {}        # prompt_parts' answers
         self.pf_vendor: Dict[Tuple[int, int, int], bool] = {}        # use_vendor_core's, for rows that are no bucket
@@ -333,6 +334,7 @@ _PF_PLANS = ((256, 256, 2, 1, 1, 4), (256, 256, 2, 1, 1, 4, 1, 0, 0, 64, 16, 8),
 # Row counts between the decode buckets and the prefill buckets, whose plans are timed once too: a short prompt's products, and what
 # prompt_parts leaves behind whole rounds of large tiles.
 PF_SMALL_MS = (128, 256, 384, 512, 768, 1024)
+PF_TAIL_MS = (1280, 1536, 1920, 2432, 3072, 3584, 3968)      # more of what is left (4096 rows of 2048 columns are a round of 256 x 128)
 _PF_SMALL = ((64, 64, 3, 1, 1, 4), (64, 64, 3, 2, 1, 4), (64, 64, 4, 1, 1, 4, 1, 8), (64, 128, 3, 1, 1, 8), (128, 64, 4, 1, 1, 4, 1, 8),
              (128, 128, 3, 1, 1, 8), (160, 128, 3, 1, 1, 8, 1, 6), (192, 128, 3, 1, 1, 8), (256, 128, 3, 1, 1, 8, 1, 8))
 _PART_US = 4.0            # a second launch of a product, and the clearing of row-sum slots it does not write
@@ -344,6 +346,12 @@ def _small(m: int, N: int, K: int):
     """(fastest plan, its us) timed for the next of PF_SMALL_MS, or None."""
     b = next((b for b in PF_SMALL_MS if m <= b), None)
     return None if b is None else _P.pf_small.get((b, N, K))
+
+
+def _left(m: int, N: int, K: int):
+    """The same, of PF_TAIL_MS too."""
+    b = next((b for b in PF_TAIL_MS if m <= b), None) if m > PF_SMALL_MS[-1] else None
+    return _small(m, N, K) if b is None else _P.pf_tail.get((b, N, K))
 
 
 def _rounds(tiles: int, cus: int) -> float:
@@ -375,7 +383,7 @@ def _parts_us(M: int, N: int, K: int) -> Tuple[float, Optional[Tuple]]:
             best, us, parts = t, t, ((M, plan),)
         for k in range(1, -(-tiles(M, plan) // cus)):      # k rounds of it, and the rows they leave
             rows = k * cus // -(-N // plan[1]) * plan[0]
-            tail = _small(M - rows, N, K) if 0 < rows < M else None
+            tail = _left(M - rows, N, K) if 0 < rows < M else None
             if tail is not None:
                 t = _rounds(tiles(rows, plan), cus) * u + tail[1] + _PART_US
                 if t < best:
@@ -394,7 +402,9 @@ def prompt_parts(M: int, N: int, K: int) -> Optional[Tuple]:
     """How the one-launch form of a fused product of a prompt's M > MAX_M rows runs: ((rows, plan), ...) one behind the other, or None
     where nothing was timed.  A large tile costs by rounds over the CUs: 8928 rows of 2048 columns are 280 tiles of 256 x 256, two
     rounds of which the second holds 24, so the last 736 rows go to a launch of small tiles.  us, one launch / here, TinyLlama: Wo
-    4500 rows 72 / 56, 8928 rows 140 / 94; gate|up 1500 rows 107 / 92, 3000 rows 196 / 157, 4500 rows 261 / 224."""
+    4500 rows 72 / 56, 8928 rows 140 / 94; gate|up 1500 rows 107 / 92, 3000 rows 196 / 157, 4500 rows 261 / 224.  What is left may be most of a
+    round: past 1024 rows of it, the shortest of the other forms (the vendor's and its epilogue too) / here, 11679 rows: down 241 / 222, Wo
+    109 / 102; QKV 8400 rows 100 / 87."""
     key = (M, N, K)
     if key in _P.pf_parts:
         return _P.pf_parts[key]
@@ -1249,6 +1259,8 @@ def _load_plans(path: str, timed_with: Optional[str] = None) -> None:
                 _P.tg_plans[tuple(map(int, at))] = tuple(v)
             elif kind == "s":
                 _P.pf_small[tuple(map(int, at))] = (tuple(v[0]), v[1])
+            elif kind == "e":
+                _P.pf_tail[tuple(map(int, at))] = (tuple(v[0]), v[1])
             elif kind == "l":
                 _P.pf_lin[tuple(map(int, at))] = [tuple(e) for e in v]
             elif kind == "m":
@@ -1273,6 +1285,7 @@ def _save_plans(path: str, timed_with: str = "") -> None:
     d.update({"r,%d,%d,%d" % k: v for k, v in _P.frag_core.items()})
     d.update({"d,%d,%d,%d" % k: v and list(v) for k, v in _P.dg_plans.items()})
     d.update({"s,%d,%d,%d" % k: list(v) for k, v in _P.pf_small.items()})
+    d.update({"e,%d,%d,%d" % k: list(v) for k, v in _P.pf_tail.items()})
     d.update({"p,%d,%d" % k: v for k, v in _P.pf_times.items()})
     d.update({"l,%d,%d" % k: v for k, v in _P.pf_lin.items()})
     d.update({"m,%d,%d,%d" % k: v for k, v in _P.pp_times.items()})
@@ -1377,11 +1390,13 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
                 print(f"gemm prefill M={M} N={N} K={K}: blas+post {lin:.1f}us, tgemm {best} {best_whole:.1f}us "
                       f"-> {_P.fused_core[(M, N, K)]}", flush=True)
             del x, y
-        for M in PF_SMALL_MS:
+        res: dict = {}
+        for M in PF_SMALL_MS + PF_TAIL_MS:
             x, y = torch.randn(M, K, device=dev).to(torch.bfloat16), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+            far = {p for p, t in res.items() if M in PF_TAIL_MS and t > 1.6 * min(res.values())}      # at the size before: not timed again
             ext, res = _native(x), {}
             for p in _PF_SMALL:
-                if p[0] > max(64, M) or (p[3] > 1 and _need_tg(M, N, K, p[0], p[1], p[3])[0] > WS_FLOATS) or _tg_splits(K, p[3]) != p[3]:
+                if p in far or p[0] > max(64, M) or (p[3] > 1 and _need_tg(M, N, K, p[0], p[1], p[3])[0] > WS_FLOATS) or _tg_splits(K, p[3]) != p[3]:
                     continue
                 try:
                     res[p] = _time(lambda i: _tgemm(ext, x, wps[i % copies], EPI_PLAIN, p, y=y), iters=8)
@@ -1389,7 +1404,7 @@ def _autotune_prefill(fused, dev, verbose: bool, roles=None, qkv_dims=None) -> N
                     continue
             best = min(res, key=res.get, default=None)
             if best is not None:
-                _P.pf_small[(M, N, K)] = (best, res[best])
+                (_P.pf_small if M in PF_SMALL_MS else _P.pf_tail)[(M, N, K)] = (best, res[best])
             if verbose and best is not None:
                 print(f"gemm rows M={M} N={N} K={K}: {best} {res[best]:.1f}us", flush=True)
         _P.pf_parts.clear()

@@ -434,3 +434,20 @@ def test_which_f32_products_are_taken(monkeypatch):
                          (16, 2048, 128, False), (9, 2048, 8192, False), (16, 2048, 512, True), (16, 2048, 4096, True), (17, 512, 512, False)]:
         assert G.fg_takes(rows(M, K), N) == yes and G.fg_takes(rows(M, K)) == (M <= 16)
     assert not G.fg_takes(torch.zeros(4, 520)[:, 1:513], 512) and not G.fg_takes(rows(4, 512).bfloat16(), 512)
+
+
+def test_prompt_parts_that_leave_most_of_a_round(monkeypatch, tmp_path):
+    """TinyLlama's down product: 3487 rows behind a round of large tiles run on what was timed for the next size, also from a plan file; more than
+    was timed is one launch."""
+    monkeypatch.delenv("DLLM_FUSED_CORE", raising=False)
+    N, K, big, tail = 2048, 5632, (256, 256, 2, 1, 1, 4), (256, 128, 3, 1, 1, 8, 1, 8)
+    monkeypatch.setattr(G._P, "pf_tail", {(m, N, K): (tail, 0.02 * m) for m in G.PF_TAIL_MS})
+    _none_timed(monkeypatch)
+    G._P.pf_times[N, K] = [(big, 8192, 135.0)]
+    G._save_plans(str(tmp_path / "plans.json"))
+    _none_timed(monkeypatch)
+    G._P.pf_tail.clear()
+    G._load_plans(str(tmp_path / "plans.json"))
+    for left, parts in ((1024, 1), (1025, 2), (1280, 2), (3487, 2), (3968, 2), (3969, 1)):
+        assert len(G.prompt_parts(8192 + left, N, K)) == parts
+    assert G.prompt_parts(11679, N, K) == ((8192, big), (3487, tail))
