@@ -730,16 +730,16 @@ def dg_takes(x: torch.Tensor) -> bool:
         (x.shape[0] == 1 or x.stride(0) >= x.shape[1]) and x.data_ptr() % 16 == 0
 
 
-FG_MAX_M, FG_MAX_K = 16, 2048      # f32_gemm.hip: past them the vendor GEMM is as fast
+FG_MAX_M, FG_MAX_K = 16, 8192      # f32_gemm.hip: past them the vendor GEMM is as fast
 
 
 def _fg_wins(M: int, N: int, K: int) -> bool:
     """Past eight rows the vendor GEMM is ahead on wide and on long products, us vendor / here: 16 rows 8192 x 2048 15.9 / 19.7, 32000 x 1536
-    44 / 52, 128 x 2048 6.8 / 7.5, 32000 x 512 17.2 / 17.7; but 4096 x 2048 12.6 / 11.5, 8192 x 1024 12.7 / 10.7, 12 rows 32000 x 1024 34.7 / 32.7.
+    44 / 52, 128 x 2048 6.8 / 7.5, 32000 x 512 17.2 / 17.7, 1024 x 4096 10.8 / 14.7; but 4096 x 2048 12.6 / 11.5, 8192 x 1024 12.7 / 10.7, 12 rows 32000 x 1024 34.7 / 32.7.
     Up to eight it is nowhere."""
     if M <= 8:
         return True
-    return (N <= 16384 or M <= 12) if K <= 1024 else 512 <= N <= 4096
+    return (N <= 16384 or M <= 12) if K <= 1024 else 512 <= N <= 4096 and K <= 2048
 
 
 def fg_takes(x: torch.Tensor, N: Optional[int] = None) -> bool:
