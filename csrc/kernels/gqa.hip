@@ -446,7 +446,8 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(const float* __restri
 
 constexpr int GA_ROWS = 16;   // rows per workgroup
 // up to a workgroup per CU, 8 waves share a workgroup's keys, past that 4 (16 heads of 64, us with 8 / 4: 128 workgroups of 400
-// keys 15.1 / 17.6, 8 of 2000 39.7 / 53.3, 480 of 60 12.9 / 8.8, 2016 of up to 250 65.5 / 48.9)
+// keys 11.9 / 14.8, 8 of 2000 34 / 49, 480 of 60 9.9 / 6.8, 2016 of up to 200 62 / 39; 16 waves, without registers for a page ahead: 8 of 400
+// keys 11.4 against 10.9, of 2000 31 against 34)
 constexpr int GQF_WIDE = 256;
 
 // KT keys per tile (64, or 32 when the tile would not fit the LDS), NJ = ceil(dv / 64)
@@ -593,9 +594,11 @@ __global__ void __launch_bounds__(256) paged_gqa_kernel(const T* __restrict__ q,
 // comes from where it lies, 16 bytes a lane (contraction step x of lane group g4 stands for dim 16 b + 4 g4 + x, or key
 // 4 g4 + x): no LDS and no barrier until the NW waves of a workgroup, which take every NW-th page, meet at the end.  The next
 // page's keys and values travel while one is computed.  Bounded by one page's load and 32 small products at decode, by the
-// f32 matrix rate (139 TF/s) over prompts.  16 query heads of 64 on 4 key heads: two sequences
-// of 400 keys 14 us a step against 104 of the general kernel above, a prompt of 2000 tokens 165 against 1087; errors against 64
-// bits 2e-7 either way.
+// f32 matrix rate (139 TF/s) over prompts.  At the end every wave leaves its sums in LDS and a thread an output adds them up, in the order of the
+// waves; its gate is asked for at the start.  (Halves of the waves adding to the other halves, two barriers each, and a last wave that then
+// read the gates of all rows were 4 us of any launch.)  16 query heads of 64 on 4 key heads: two sequences of 400 keys 11.0 us a step (14.8
+// with that end; 104 in the general kernel above), one of 60 5.6 (9.1), a prompt of 2000 tokens 138 (144; 1087); heads of 128, two of 400 keys
+// 19 (26).  Errors against 64 bits 2e-7 either way.
 template <int KB, int VB, int NW>
 __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc,
                                                           const float* __restrict__ vc, const int* __restrict__ bt, int bt_ld,
@@ -606,8 +609,9 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
                                                           int win, int keep, float sink, int chunk, float cap,
                                                           const float* __restrict__ sinks, long ldo,
                                                           const float* __restrict__ slopes, int ghead) {
-  __shared__ __attribute__((aligned(16))) f32x4 Om[NW / 2][VB * 64];
-  __shared__ float ml[NW][2][16];
+  constexpr int EPT = 4 * VB / NW;               // outputs a thread
+  __shared__ __attribute__((aligned(16))) f32x4 Om[NW][16][4 * VB + 1];
+  __shared__ float ml[NW][2][16], Ls[16];
   const int tile = gridDim.x - 1 - blockIdx.x;   // later tokens see more keys: start with the long rows
   const int s = tile_seq[tile];
   const int n = qlen[s], tok0 = tile_tok0[tile];
@@ -623,6 +627,14 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
   const int rpos = row ? p0 + tok0 + lr / Rh : -1, rlo = row ? oldest_key(rpos, win, chunk) : 0;
   const float slp = slopes ? slopes[h] : 0.f;
   f32x4 qf[KB];
+  float gv[EPT];
+  if (gate)
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const int i = threadIdx.x + e * 64 * NW, r = min(i / (16 * VB), nrows - 1), j = min(i % (16 * VB), dv - 1);
+      const int hh = g * R + r0 + r % Rh;
+      gv[e] = gate[(q0 + tok0 + r / Rh) * ldg + (ghead ? (long)hh : (long)hh * dv + j)];
+    }
   const float* qp = q + (tok * H + h) * d;
 #pragma unroll
   for (int b = 0; b < KB; ++b) {
@@ -718,31 +730,20 @@ __global__ void __launch_bounds__(64 * NW) gqa_f32_kernel(const float* __restric
   for (int x = 0; x < NW; ++x) L += ml[x][0][lr] > -INFINITY ? ml[x][1][lr] * expf(ml[x][0][lr] - M) : 0.f;
   const float f = m > -INFINITY ? expf(m - M) : 0.f;
 #pragma unroll
-  for (int b = 0; b < VB; ++b) O[b] *= f;
+  for (int b = 0; b < VB; ++b) Om[w][lr][(16 * b + 4 * g4) / 4] = O[b] * f;
+  if (w == 0 && g4 == 0) Ls[lr] = 1.f / (L + (sinks ? expf(sinks[h] - M) : sink > 0.f ? sink * expf(-M) : 0.f));
+  __syncthreads();
 #pragma unroll
-  for (int half = NW / 2; half; half >>= 1) {
-    if (w >= half && w < 2 * half)
+  for (int e = 0; e < EPT; ++e) {
+    const int i = threadIdx.x + e * 64 * NW, r = i / (16 * VB), j = i % (16 * VB);
+    if (r >= nrows || j >= dv) continue;
+    float o = 0.f;
 #pragma unroll
-      for (int b = 0; b < VB; ++b) Om[w - half][b * 64 + lane] = O[b];
-    __syncthreads();
-    if (w < half)
-#pragma unroll
-      for (int b = 0; b < VB; ++b) O[b] += Om[w][b * 64 + lane];
-    __syncthreads();
+    for (int x = 0; x < NW; ++x) o += reinterpret_cast<const float*>(&Om[x][r][0])[j];
+    o *= Ls[r];
+    if (gate) o *= 1.f / (1.f + expf(-gv[e]));
+    out[(q0 + tok0 + r / Rh) * ldo + (long)(g * R + r0 + r % Rh) * dv + j] = o;
   }
-  if (w || !row) return;
-  const float inv = 1.f / (L + (sinks ? expf(sinks[h] - M) : sink > 0.f ? sink * expf(-M) : 0.f));
-  const float gh = gate && ghead ? 1.f / (1.f + expf(-gate[tok * ldg + h])) : 1.f;
-#pragma unroll
-  for (int b = 0; b < VB; ++b)
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int j = 16 * b + 4 * g4 + x;
-      if (j >= dv) continue;
-      float o = O[b][x] * inv * gh;
-      if (gate && !ghead) o *= 1.f / (1.f + expf(-gate[tok * ldg + (long)h * dv + j]));
-      out[tok * ldo + (long)h * dv + j] = o;
-    }
 }
 
 // ---------------------------------------------------------------- bf16 on the matrix cores
