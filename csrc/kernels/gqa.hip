@@ -1083,6 +1083,283 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 192 ? 2 : 1) paged_g
   }
 }
 
+// The same with a row to a lane column:  S^T = K . Q^T  leaves 16 of a tile's scores of one row in a lane, so the row's maximum is eight instructions
+// and two lane exchanges where the form above takes seven for each of a lane's four rows, one exponential rescales it, and the weights are at
+// once the right operand of  O^T = V^T . P^T  where they went round by LDS.  (Row 16 kb + 4 g + i of the staged keys is key 32 (kb / 2) + 8 g + 4 (kb % 2) + i:
+// a lane's scores are then eight neighbouring keys of each half of a tile, as V^T lies.)  Vector instructions bound both forms, two thirds of
+// the cycles here: per tile and wave 95 of them and 28 products.  us, above / here: six sequences of 308 to 2600 tokens, 32 / 8 heads of 64 176 / 122,
+// with a window of 512 103 / 70; 4001 tokens, 16 heads of 96 / 64 128 / 103; 24 of 160 32.6 / 19.8; four of 200 to 1300, 16 / 4 of 64 with slopes 43 / 29;
+// four of 2900, 16 / 4 of 128 429 / 254; 3000, 8 / 2 of 192 / 128 125 / 94.  Two tiles in LDS with one barrier a tile took 139 for 132, chunks
+// swizzled for fewer bank conflicts nothing.
+// Scores stay below 2^127 (their maximum is taken times log2 e).
+template <int KD, int VD, bool CAP, bool DIST>
+__global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) : 2) gqa_cols_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
+                                                      const int* __restrict__ bt, int bt_ld, const int* __restrict__ qstart,
+                                                      const int* __restrict__ qlen, const int* __restrict__ ctx,
+                                                      const int* __restrict__ tile_seq, const int* __restrict__ tile_tok0,
+                                                      const u16* __restrict__ gate, long ldg, u16* __restrict__ out, int H, int G, int d,
+                                                      int dv, int TQ, int splits, float* __restrict__ part, int win, int keep,
+                                                      float sink, int chunk, float cap, const float* __restrict__ sinks, long ldo,
+                                                      const float* __restrict__ slopes, int ghead) {
+  constexpr int DS = KD / 32, VB = VD / 16, NKB = GM_KT / 16;
+  constexpr int KSTR = KD + 8, VSTR = GM_KT + 8;
+  constexpr float LOG2E = 1.44269504f;
+  __shared__ __attribute__((aligned(16))) u16 ksh[GM_KT * KSTR], vtr[VD * VSTR];      // keys; values transposed, [dim][key]
+  const int g = blockIdx.x % G, tile = (gridDim.x - 1 - blockIdx.x) / G;
+  const int s = tile_seq[tile];
+  const int n = qlen[s];
+  const int tok0 = tile_tok0[tile];
+  if (n <= 0 || tok0 >= n) return;   // the whole workgroup (padding tiles)
+  const int R = H / G;
+  const int nq = min(TQ, n - tok0), nrows = nq * R;
+  const int q0 = qstart[s], p0 = ctx[s] - n;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, g4 = lane >> 4;
+  // this lane's row -> (token tok0 + row / R, query head g R + row % R)
+  const int row = 16 * wave + lr;
+  const bool live = row < nrows;
+  const int tl = live ? row / R : 0, h = g * R + (live ? row % R : 0);
+  const int rpos = live ? p0 + tok0 + tl : -1, rlo = live ? oldest_key(rpos, win, chunk) : 0;      // -1: sees no key
+  const float slp = DIST && live ? slopes[h] : 0.f;
+  const long tok = q0 + tok0 + tl;
+  bf16x8 qb[DS];
+#pragma unroll
+  for (int st = 0; st < DS; ++st) {
+    const int c = st * 32 + 8 * g4;
+    qb[st] = __builtin_bit_cast(bf16x8, live && c < d ? ld16(q + (tok * H + h) * d + c) : make_uint4(0u, 0u, 0u, 0u));
+  }
+  float m = CAP ? 0.f : -INFINITY;
+  // the weights' sum is one more row of  V^T . P^T,  of ones: four products where 16 additions are a twelfth of a tile's vector instructions
+  f32x4 l = {0.f, 0.f, 0.f, 0.f};
+  // {-1, 0} in a register: as an inline constant the compiler writes it the way the instruction reads {0, -1}
+  uint32_t neg = 0xbf80u;
+  asm volatile("" : "+s"(neg));
+  const bf16x2v minus = __builtin_bit_cast(bf16x2v, neg);
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+  f32x4 acc[VB];
+#pragma unroll
+  for (int cb = 0; cb < VB; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int wave_last = 16 * wave < nrows ? p0 + tok0 + (min(16 * wave + 15, nrows - 1)) / R : -1;
+  // the oldest row of the wave; idle rows (past nrows) are masked, so a wave that has any never skips the mask
+  const int wave_first = 16 * wave + 15 < nrows ? p0 + tok0 + (16 * wave) / R : -1;
+  // the oldest keys the wave's oldest and newest live rows see (a tile wholly before the first is
+  // skipped; one not before the second needs no mask at its old end)
+  const int wave_lo = 16 * wave < nrows ? oldest_key(p0 + tok0 + (16 * wave) / R, win, chunk) : 0;
+  const int wave_lo_last = wave_last >= 0 ? oldest_key(wave_last, win, chunk) : 0;
+  // CAP: exponents in base 2
+  const float cap2 = cap > 0.f ? (CAP ? 2.88539008f : 2.f) / cap : 0.f;
+  const float capl = 1.44269504f * cap;
+  const int last = p0 + tok0 + nq - 1;   // the newest key any row sees
+  const int* btr = bt + (long)s * bt_ld;
+  // A wave stages a page of the tile's four: its number is a scalar, and a lane's places in it are the same in every tile.  Page ids are
+  // loaded a tile ahead of the keys, and no load stands behind a condition (pages past the newest key: its page again, and zeros when staged).
+  constexpr int KCH = KD / 8, NFK = KD / 32, NFV = VD / 32;      // 16-byte chunks of a key row; chunks of K, and of V, a lane moves per tile
+  uint4 pk_[NFK], pv_[NFV];
+  int koff[NFK], voff[NFV], klds[NFK], kkey[NFK];      // in a page (past d or dv: the row's first, and zeros when staged), in LDS
+  bool kon[NFK], von[NFV];
+#pragma unroll
+  for (int f = 0; f < NFK; ++f) {
+    const int e = lane + 64 * f, c = (e % KCH) * 8, kk = 16 * wave + e / KCH;
+    kkey[f] = kk;
+    kon[f] = c < d;
+    koff[f] = (e / KCH) * d + (kon[f] ? c : 0);
+    klds[f] = (32 * (kk >> 5) + 16 * ((kk >> 2) & 1) + 4 * ((kk >> 3) & 3) + (kk & 3)) * KSTR + c;
+  }
+#pragma unroll
+  for (int f = 0; f < NFV; ++f) {
+    const int j = (lane >> 1) + 32 * f;
+    von[f] = j < dv;
+    voff[f] = (von[f] ? j : 0) * GM_BS + 8 * (lane & 1);
+  }
+  const u16 *kg = kc + (long)g * GM_BS * d, *vg = vc + (long)g * dv * GM_BS;
+  const long kpage = (long)G * GM_BS * d, vpage = (long)G * dv * GM_BS;
+  const int page_last = last >> 4;
+  int id;
+  auto fetch_ids = [&](int k0) { id = btr[min((k0 >> 4) + wave, page_last)]; };
+  auto fetch = [&] {
+    const u16 *kp = kg + id * kpage, *vp = vg + id * vpage;
+#pragma unroll
+    for (int f = 0; f < NFK; ++f) pk_[f] = ld16(kp + koff[f]);
+#pragma unroll
+    for (int f = 0; f < NFV; ++f) pv_[f] = ld16(vp + voff[f]);
+  };
+  const int tfirst = oldest_key(p0 + tok0, win, chunk) / GM_KT;   // the oldest tile of the window / chunk any row sees
+  const int nkeep = min(tfirst, (keep + GM_KT - 1) / GM_KT);
+  const int ntiles = last / GM_KT + 1 - tfirst + nkeep;
+  const int vbeg = (int)((long)ntiles * blockIdx.z / splits);
+  const int vend = (int)((long)ntiles * (blockIdx.z + 1) / splits);   // exclusive
+  auto tile_k0 = [&](int v) { return (v < nkeep ? v : tfirst + v - nkeep) * GM_KT; };
+  if (vbeg < vend) {
+    fetch_ids(tile_k0(vbeg));
+    fetch();
+    fetch_ids(tile_k0(min(vbeg + 1, vend - 1)));
+  }
+  for (int vt = vbeg; vt < vend; ++vt) {
+    const int k0 = tile_k0(vt);
+    __syncthreads();   // the previous tile is consumed
+    const int nk = last + 1 - k0;
+    if (nk < GM_KT || d < KD || dv < VD) {
+#pragma unroll
+      for (int f = 0; f < NFK; ++f)
+        if (!(kon[f] & (kkey[f] < nk))) pk_[f] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int f = 0; f < NFV; ++f)
+        if (!(von[f] & (16 * wave < nk))) pv_[f] = make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int f = 0; f < NFK; ++f) st16(ksh + klds[f], pk_[f]);
+#pragma unroll
+    for (int f = 0; f < NFV; ++f) st16(vtr + ((lane >> 1) + 32 * f) * VSTR + 16 * wave + 8 * (lane & 1), pv_[f]);
+    if (vt + 1 < vend) {      // the next tile's loads fly under this tile's products
+      fetch();
+      fetch_ids(tile_k0(min(vt + 2, vend - 1)));
+    }
+    __syncthreads();
+    if (k0 > wave_last) continue;   // this wave's rows see nothing of the tile (the barriers above are uniform)
+    if (k0 >= keep && k0 + GM_KT <= wave_lo) continue;   // ... or the tile lies before every row's window / chunk
+    const int key0 = k0 + 8 * g4;      // score (kb, i) is of key key0 + 32 (kb / 2) + 4 (kb % 2) + i
+    f32x4 sc[NKB];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+      sc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (DIST) {
+        const float d0 = slp * (float)(key0 + 32 * (kb >> 1) + 4 * (kb & 1) - rpos);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[kb][i] = fmaf(slp, (float)i, d0);
+      }
+    }
+#pragma unroll
+    for (int st = 0; st < DS; ++st)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) {
+        const bf16x8 a = __builtin_bit_cast(bf16x8, ld16(ksh + (16 * kb + lr) * KSTR + 8 * g4 + st * 32));
+        sc[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qb[st], sc[kb], 0, 0, 0);
+      }
+    if (!CAP && !DIST && cap > 0.f) {
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sc[kb][i] = cap_fast(sc[kb][i], cap, cap2);
+    }
+    if constexpr (CAP) {   // log2(e) times the capped score
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          sc[kb][i] = capl - 2.f * capl * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(sc[kb][i] * cap2) + 1.f);
+    }
+    // a tile inside every row's range needs no mask (wave-uniform, a scalar branch; bitwise as above)
+    if (!(k0 + GM_KT - 1 <= wave_first && k0 >= wave_lo_last)) {
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = key0 + 32 * (kb >> 1) + 4 * (kb & 1) + i;
+          const bool vis = (key <= rpos) & ((key >= rlo) | (key < keep));
+          sc[kb][i] = vis ? sc[kb][i] : -INFINITY;
+        }
+    }
+    float c2 = 0.f, alpha = 1.f;
+    if constexpr (!CAP) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kb][i]);
+      mx = lane_max(mx, 16);
+      mx = fmaxf(m, lane_max(mx, 32));
+      c2 = mx > -INFINITY ? mx * LOG2E : 0.f;      // before the first visible key: weights, acc and l are 0
+      alpha = __builtin_amdgcn_exp2f(fmaf(m, LOG2E, -c2));
+      m = mx;
+    }
+    bf16x8 ph[NKB / 2], pl[NKB / 2];      // p = hi + lo with both parts bf16 (the packed conversions round to nearest even)
+#pragma unroll
+    for (int ks = 0; ks < NKB / 2; ++ks) {
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x = sc[2 * ks + (j >> 2)][j & 3];
+        p[j] = __builtin_amdgcn_exp2f(CAP ? x : fmaf(x, LOG2E, -c2));      // exp(-inf) = 0 for masked keys
+      }
+      uint32_t hi[4], lo[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        hi[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2v{p[2 * j], p[2 * j + 1]}, bf16x2v));
+        const bf16x2v hb = __builtin_bit_cast(bf16x2v, hi[j]);
+        const f32x2v r = {__builtin_amdgcn_fdot2_f32_bf16(hb, minus, p[2 * j], false),
+                          __builtin_amdgcn_fdot2_f32_bf16(hb, bf16x2v{0.f, -1.f}, p[2 * j + 1], false)};      // p - hi, exact
+        lo[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2v));
+      }
+      ph[ks] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+      pl[ks] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+    }
+    if constexpr (!CAP) {
+      if (__any(alpha != 1.f)) {      // (once the running maxima have settled no row of the wave rescales)
+        l *= alpha;
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) acc[cb] *= alpha;
+      }
+    }
+    __builtin_amdgcn_s_setprio(1);      // (ahead of the other waves' vector instructions: 132 -> 122 us)
+#pragma unroll
+    for (int ks = 0; ks < NKB / 2; ++ks) {
+      if constexpr (VB <= 4) {
+        bf16x8 v[VB];
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) v[cb] = __builtin_bit_cast(bf16x8, ld16(vtr + (16 * cb + lr) * VSTR + 8 * g4 + 32 * ks));
+        l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, ph[ks], l, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[cb], ph[ks], acc[cb], 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl[ks], l, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[cb], pl[ks], acc[cb], 0, 0, 0);
+      } else {      // (with all of eight blocks' values at hand 304 us for 255)
+        l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, ph[ks], l, 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pl[ks], l, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) {
+          const bf16x8 v = __builtin_bit_cast(bf16x8, ld16(vtr + (16 * cb + lr) * VSTR + 8 * g4 + 32 * ks));
+          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, ph[ks], acc[cb], 0, 0, 0);
+          acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pl[ks], acc[cb], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  }
+  if (!live) return;
+  if (part) {
+    float* pr = part + ((((long)tile * G + g) * splits + blockIdx.z) * GM_ROWS + row) * (dv + 2);
+    if (g4 == 0) { pr[0] = m; pr[1] = l[0]; }
+#pragma unroll
+    for (int cb = 0; cb < VB; ++cb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (16 * cb + 4 * g4 + i < dv) pr[2 + 16 * cb + 4 * g4 + i] = acc[cb][i];
+    return;
+  }
+  float inv = 1.f / (l[0] + (sinks ? __expf(sinks[h] - m) : sink > 0.f ? sink * __expf(-m) : 0.f));
+  if (gate && ghead) inv *= 1.f / (1.f + expf(-bf2f(gate[tok * ldg + h])));
+  auto recip = [](float x) { const float r = __builtin_amdgcn_rcpf(x); return x < 1e38f ? r * fmaf(-x, r, 2.f) : r; };
+  const u16* gr = gate && !ghead ? gate + tok * ldg + (long)h * dv : nullptr;
+  u16* o = out + tok * ldo + (long)h * dv;
+  const bool whole = dv % 4 == 0 && ldo % 4 == 0 && ldg % 4 == 0 && (((uintptr_t)out | (uintptr_t)gate) & 7) == 0;      // four outputs at a time
+#pragma unroll
+  for (int cb = 0; cb < VB; ++cb) {
+    const int j = 16 * cb + 4 * g4;
+    u16x4 y;
+    if (whole && j < dv) {
+      const u16x4 z = gr ? *reinterpret_cast<const u16x4*>(gr + j) : u16x4{};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y.v[i] = f2bf(acc[cb][i] * inv * (gr ? recip(1.f + expf(-bf2f(z.v[i]))) : 1.f));
+      *reinterpret_cast<u16x4*>(o + j) = y;
+    } else
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j + i < dv) o[j + i] = f2bf(acc[cb][i] * inv * (gr ? recip(1.f + expf(-bf2f(gr[j + i]))) : 1.f));
+  }
+}
+
 // The same for few rows a tile (decode steps: a token's R <= 16 heads): there paged_gqa_mfma has one wave of four with live rows, which
 // walks every tile of its split behind two barriers (3 us a tile).  Here each wave takes 32-key chunks of its own and keeps its own
 // maximum, sum and O^T; keys and values come from the pages straight to registers, the next chunk's while this one is multiplied, and
@@ -1479,6 +1756,23 @@ extern "C" int dllm_paged_gqa(const void* q, const void* kc, const void* vc, int
       else GQF(false, false);
 #undef GQF
 #undef GQM
+    } else if (GV == G && !out32 && d <= 192 && dv <= 128) {      // (wider heads' accumulators and keys take more registers than a wave has)
+#define GQC(KD, VD, CAP, DIST)                                                                                                    \
+  hipLaunchKernelGGL((gqa_cols_kernel<KD, VD, CAP, DIST>), grid, dim3(256), 0, st, (const u16*)q, (const u16*)kc, (const u16*)vc, bt, \
+                     bt_ld, qstart, qlen, ctx, tile_seq, tile_tok0, (const u16*)gate, ldg, (u16*)out, H, G, d, dv, TQ, splits, pp, win, keep, \
+                     sink, chunk, cap, sinks, ldo, slopes, ghead)
+#define GQL(CAP, DIST)                                         \
+  do {                                                         \
+    if (d <= 64 && dv <= 64) GQC(64, 64, CAP, DIST);           \
+    else if (d <= 96 && dv <= 64) GQC(96, 64, CAP, DIST);      \
+    else if (d <= 128 && dv <= 128) GQC(128, 128, CAP, DIST);  \
+    else GQC(192, 128, CAP, DIST);                             \
+  } while (0)
+      if (cap > 0.f && cap <= CAP_MAX) GQL(true, false);
+      else if (slopes) GQL(false, true);
+      else GQL(false, false);
+#undef GQL
+#undef GQC
     } else if (cap > 0.f && cap <= CAP_MAX) GQZ(true, false);
     else if (slopes) GQZ(false, true);
     else GQZ(false, false);
