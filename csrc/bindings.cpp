@@ -138,6 +138,7 @@ int dllm_latent_kv_write(const void*, long, int, int, int, const float*, float, 
 int dllm_latent_attention(const void*, const void*, long, int, int, int, int, int, long, const float*, int, const void*,
                           const int*, int, const int*, const int*, const int*, const int*, const int*, int, float, void*,
                           int, float*, float*, int, int, int, const float*, const void*, int, const void*, long, int, void*, long, hipStream_t);
+int dllm_latent_absorb(const void*, long, int, const void*, void*, int, int, int, int, hipStream_t);
 int dllm_latent_mfma_ok(int, int, int);
 int dllm_car_alloc(long, void**);
 int dllm_car_get_handle(void*, char*);
@@ -2169,6 +2170,20 @@ void attn_prep(torch::Tensor proj, int64_t H, int64_t G, int64_t d, int64_t dv, 
      "attn_prep");
 }
 
+// qa [H, T, rank] = q[:, h, :dim] . uk[h] with w [H, rank, dim] (latent.hip); q [T, H, dim], its rows and heads may be parts of wider ones
+void latent_absorb(torch::Tensor q, torch::Tensor w, torch::Tensor out) {
+  for (auto* t : {&q, &w, &out}) {
+    check_bf16(*t, "latent_absorb operand");
+    TORCH_CHECK(t->dim() == 3 && t->stride(2) == 1, "matrices of unit column stride");
+  }
+  const int64_t T = q.size(0), H = q.size(1), dim = q.size(2), rank = w.size(1);
+  TORCH_CHECK(w.is_contiguous() && out.is_contiguous() && w.size(0) == H && w.size(2) == dim && out.size(0) == H && out.size(1) == T && out.size(2) == rank &&
+                  T >= 1, "q [T, H, dim], w [H, rank, dim], out [H, T, rank]");
+  ok(dllm_latent_absorb(q.data_ptr(), T > 1 ? q.stride(0) : H * dim, (int)(H > 1 ? q.stride(1) : dim), w.data_ptr(), out.data_ptr(), (int)T, (int)H, (int)dim, (int)rank,
+                        stream()),
+     "latent_absorb");
+}
+
 void paged_gqa_attention(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tensor bt, torch::Tensor qstart,
                          torch::Tensor qlen, torch::Tensor ctx, torch::Tensor tile_seq, torch::Tensor tile_tok0,
                          c10::optional<torch::Tensor> gate, torch::Tensor out, bool mfma, int64_t splits,
@@ -3058,6 +3073,7 @@ PYBIND11_MODULE(_hip_kernels, m) {
         py::arg("splits") = 1, py::arg("part_o") = py::none(), py::arg("part_ml") = py::none(), py::arg("mfma") = true,
         py::arg("rows") = 16, py::arg("half") = false, py::arg("sinks") = py::none(), py::arg("up_w") = py::none(),
         py::arg("gate") = py::none(), py::arg("up_out") = py::none());
+  m.def("latent_absorb", &latent_absorb);
   m.def("latent_mfma_ok", [](int64_t rank, int64_t rot, int64_t rows) { return dllm_latent_mfma_ok((int)rank, (int)rot, (int)rows) != 0; });
   m.def("encoder_layers", &encoder_layers, py::arg("x"), py::arg("lens"), py::arg("starts"), py::arg("S"), py::arg("nh"), py::arg("d"), py::arg("eps"),
         py::arg("weights"), py::arg("plans"), py::arg("part") = py::none(), py::arg("counters") = py::none(),

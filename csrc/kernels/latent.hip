@@ -1002,6 +1002,25 @@ __global__ void __launch_bounds__(256) latent_combine_kernel(const float* __rest
   }
 }
 
+// The key up-projection on the queries' unrotated dims for steps of few tokens:  qa[h] = q[:, h, :dim] . uk[h]  with uk stored [H, rank, dim].  A wave
+// takes 16 ranks of a head and 16 tokens; weights are the first operand, so that a lane holds four neighbouring ranks of one token.  Bounded by
+// one trip to memory: us, the vendor's batched product / here, 16 heads of 64 -> 256: 4
+// tokens 4.3 / 2.3, 24 4.7 / 2.4, 64 5.1 / 2.4; 32 heads of 64 -> 512: 6.3 / 2.3, 3.9 / 2.8, 4.4 / 3.9 (128 5.1 / 5.9, where the weights are read once
+// per 16 tokens); 8 of 128 -> 512: 3.8 / 2.5, 4.0 / 2.8, 4.0 / 2.9.
+__global__ void __launch_bounds__(256) latent_absorb_kernel(const u16* __restrict__ q, long ldq, int hstep, const u16* __restrict__ W,
+                                                            u16* __restrict__ out, int T, int dim, int rank) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, g4 = lane >> 4;
+  const int n0 = 64 * blockIdx.x + 16 * wave, h = blockIdx.y, t = 16 * blockIdx.z + lr;
+  if (n0 >= rank) return;      // (no barrier)
+  const u16* wr = W + ((long)h * rank + n0 + lr) * dim + 8 * g4;
+  const u16* qr = q + (long)min(t, T - 1) * ldq + (long)h * hstep + 8 * g4;      // rows past T repeat the last and are dropped
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = 0; k < dim; k += 32)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ld16(wr + k)), __builtin_bit_cast(bf16x8, ld16(qr + k)), acc, 0, 0, 0);
+  if (t < T) *reinterpret_cast<uint2*>(out + ((long)h * T + t) * rank + n0 + 4 * g4) = make_uint2(f2bf2(acc[0], acc[1]), f2bf2(acc[2], acc[3]));
+}
+
 // latent_combine, the head's value up-projection and its gate in one launch, for steps of few tokens: a workgroup merges a (token,
 // head) row's splits, rounds it to bf16 and multiplies it with the head's W [rank, 8 NV], a thread NV-th of the columns and some of
 // the ranks; weights, partials and gate are all asked for at the start.  As launches of their own the batched product of the vendor's
@@ -1207,6 +1226,15 @@ int launch_latent_mfma(dim3 g, hipStream_t st, const u16* qa, const u16* q, long
   return (int)hipGetLastError();
 }
 }  // namespace
+
+// q [T, H, >= dim] rows ldq apart, heads hstep, W [H, rank, dim], out [H, T, rank]: 16-byte aligned; dim % 32 == 0, rank % 16 == 0, strides % 8 == 0
+extern "C" int dllm_latent_absorb(const void* q, long ldq, int hstep, const void* W, void* out, int T, int H, int dim, int rank, hipStream_t st) {
+  if (T < 1 || H < 1 || dim < 32 || dim % 32 || rank < 16 || rank % 16 || ldq % 8 || hstep % 8 || (((uintptr_t)q | (uintptr_t)W | (uintptr_t)out) & 15))
+    return -1;
+  hipLaunchKernelGGL(latent_absorb_kernel, dim3((rank + 63) / 64, H, (T + 15) / 16), dim3(256), 0, st, (const u16*)q, ldq, hstep, (const u16*)W, (u16*)out,
+                     T, dim, rank);
+  return (int)hipGetLastError();
+}
 
 // 1 when the matrix-core kernel takes this shape with `rows` (16 or 32) rows per workgroup (bf16, even
 // widths, a 32-key tile fits the LDS)

@@ -467,6 +467,7 @@ class HybridModel:
                 D["dq_norm"], D["dkv_norm"] = f32(t[p + "mix.dq.norm"]), f32(t[p + "mix.dkv.norm"])
                 D["uq"], D["o"] = put(t[p + "mix.uq"]), put(t[p + "mix.o"])
                 D["uk"] = put(t[p + "mix.uk"].view(m.heads, m.dim, m.kv_rank))                       # [H, d, r]
+                self._place_absorb(D)
                 D["uv"] = put(t[p + "mix.uv"].view(m.heads, m.vdim, m.kv_rank))                      # [H, dv, r]
                 D["uvT"] = D["uv"].transpose(1, 2).contiguous()                                      # [H, r, dv]
                 if m.sinks:
@@ -591,6 +592,11 @@ class HybridModel:
             w = torch.cat([w, w.new_zeros(-n % 64, w.shape[1])], 0)
         return put(w), n
 
+    def _place_absorb(self, D) -> None:
+        """The key up-projection as [H, r, d], for the steps of few tokens of a bf16 model on the GPU that bears another order of sums."""
+        if self.dtype == torch.bfloat16 and self.device.type == "cuda" and not self.order_kept:
+            D["uk_r"] = D["uk"].transpose(1, 2).contiguous()
+
     def _place_parallel(self, D, L: LayerSpec, t, p: str, put, f32) -> None:
         """A layer whose mixer and feed-forward read the same input and are added together: one
         projection for everything that reads it, one for everything that is added."""
@@ -606,6 +612,7 @@ class HybridModel:
         else:
             D["dkv_norm"] = f32(t[p + "mix.dkv.norm"])
             D["uk"] = put(t[p + "mix.uk"].view(m.heads, m.dim, m.kv_rank))                       # [H, d, r]
+            self._place_absorb(D)
             D["uv"] = put(t[p + "mix.uv"].view(m.heads, m.vdim, m.kv_rank))                      # [H, dv, r]
             D["uvT"] = D["uv"].transpose(1, 2).contiguous()                                      # [H, r, dv]
             n = m.heads * m.dim + m.kv_rank
@@ -817,8 +824,8 @@ class HybridModel:
             o = seqmix.paged_gqa_attention(q, k, v, pages, meta.qstart, meta.qlen, meta.ctx, ts, tt, gate, mfma, splits,
                                            all_rows=True, sinks=L.get("sink"))
             return _pm(o, L, "o")
-        qn = q.view(T, H, m.dim + rd)[:, :, :m.dim].transpose(0, 1)
-        qa = torch.bmm(qn, L["uk"])                                     # key up-projection absorbed: [H, T, rank]
+        # key up-projection absorbed: [H, T, rank]
+        qa = seqmix.latent_absorb(q.view(T, H, m.dim + rd)[:, :, :m.dim], L["uk"], L.get("uk_r"))
         lat = seqmix.latent_attention(qa, q, m.dim, rd, positions, table, cache[0], meta.block_tables, meta.qstart,
                                       meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat, half=m.rot_half,
                                       sinks=L.get("sink"), up=up)
@@ -994,7 +1001,7 @@ class HybridModel:
         seqmix.latent_prep(proj, c0, L["dkv_norm"], self.cfg.rms_eps, meta.slots, cache[0], g0 + hv, act,
                            zero=lat if up is None else both[:, :hv][None])
         q = proj[:, :c0]
-        qa = torch.bmm(q.unflatten(1, (H, m.dim)).transpose(0, 1), L["uk"])     # key up-projection absorbed: [H, T, rank]
+        qa = seqmix.latent_absorb(q.unflatten(1, (H, m.dim)), L["uk"], L.get("uk_r"))     # key up-projection absorbed: [H, T, rank]
         lat = seqmix.latent_attention(qa, q, m.dim, 0, positions, self._any_table(), cache[0], meta.block_tables, meta.qstart,
                                       meta.qlen, meta.ctx, ts, tr, m.scale, rows=rows, out=lat, up=up)
         if up is None:

@@ -240,6 +240,22 @@ def latent_rows(x: torch.Tensor, rank: int, rot_dim: int, tokens: int, seqs: int
 LAT_UP_TOKENS = 64     # latent_up_kernel: past it the batched product reads the weights less often
 
 
+LAT_ABSORB_TOKENS = 64      # up to here the own kernel is ahead of the vendor's batched product at every width (csrc/kernels/latent.hip)
+
+
+def latent_absorb(q: torch.Tensor, uk: torch.Tensor, ukT: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """q [T, heads, dim] (parts of wider rows) times uk [heads, dim, rank]: [heads, T, rank], the query that meets the cached latents.  ``ukT``: uk as
+    [heads, rank, dim], for steps of few tokens."""
+    T, H, dim = q.shape
+    if (ukT is not None and 0 < T <= LAT_ABSORB_TOKENS and q.is_cuda and q.dtype == ukT.dtype == torch.bfloat16 and ukT.is_contiguous() and dim % 32 == 0 and
+            ukT.shape[1] % 16 == 0 and q.stride(2) == 1 and q.stride(1) % 8 == 0 and q.stride(0) % 8 == 0 and
+            q.data_ptr() % 16 == 0 and ukT.data_ptr() % 16 == 0):
+        out = torch.empty((H, T, ukT.shape[1]), dtype=q.dtype, device=q.device)
+        _native(q).latent_absorb(q, ukT, out)
+        return out
+    return torch.bmm(q.transpose(0, 1), uk)
+
+
 def latent_up_ok(x: torch.Tensor, heads: int, tokens: int, entries: int, rank: int, rot_dim: int, uv: torch.Tensor, rows: int) -> bool:
     """Does a latent attention launch over ``entries`` tiles merge its splits together with the value up-projection ``uv``
     [heads, rank, vdim] (``latent_attention``'s ``up``)?"""
