@@ -26,7 +26,10 @@
 
 namespace {
 constexpr int BS = 16;     // tokens per KV block
-constexpr int WAVES = 4;   // LDS combine slots; a workgroup runs W = 4 or 8 waves
+// LDS combine slots of W = 4 or 8 waves.  Eight of 64-wide heads have one each: the upper four folding into the lower ones first is two barriers
+// and a pass over LDS on every launch's way (us, folded / here: one request of
+// 57 keys 4.78 / 4.41, of 300 6.1 / 5.75, 48 of 40 to 424 7.1 / 6.7, 64 of 300 to 900 11.5 / 11.15, two of 6001 and 2900 in parts 10.85 / 10.6)
+constexpr int slots(int W, int D) { return W == 8 && D == 64 ? 8 : 4; }
 constexpr int COMBINE_MAXS = 16;  // split counts up to this take the parallel last-arriver combine
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -61,11 +64,12 @@ struct AttnArgs {
 // for short contexts ran 1.5-4.7x slower than the same work with z = 1, so the engine uses static
 // split counts sized to the batch and keeps the dynamic split for explicit opt-in.
 
-template <int D>
+template <int D, int SL>
 struct AttnSmem {
-  float o[WAVES][16][D + 1];
-  float m[WAVES][16];
-  float l[WAVES][16];
+  static constexpr int PITCH = SL == 8 ? D + 4 : D + 1;      // (+ 4: 16-byte stores of 16 rows reach every bank)
+  __attribute__((aligned(16))) float o[SL][16][PITCH];
+  float m[SL][16];
+  float l[SL][16];
   int last;
 };
 
@@ -85,11 +89,12 @@ __device__ __forceinline__ TileMeta load_tile_meta(const AttnArgs& a, int tile) 
 }
 
 template <int D, int W, bool VN>
-__device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, const int tile, const int kvh,
+__device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D, slots(W, D)>& sm, const int tile, const int kvh,
                                           const int split, int nsplit, const TileMeta tm) {
   constexpr int CH = 1;   // 32-key chunks per wave trip (2, and a block-table prefetch one trip ahead, measured no gain)
   constexpr int KSTEPS = D / 32;
   constexpr int NT = D / 16;
+  constexpr int WAVES = slots(W, D);
   auto& s_o = sm.o;
   auto& s_m = sm.m;
   auto& s_l = sm.l;
@@ -271,7 +276,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
   }
 
   // ---- combine the waves through LDS.  acc[n][r] = O^T[dim 16n + 4g + r][row rl]
-  if constexpr (W == 8) {  // waves 4..7 fold into waves 0..3 first (keeps LDS at 4 slots)
+  if constexpr (W == 8 && WAVES == 4) {  // waves 4..7 fold into waves 0..3 first (keeps LDS at 4 slots)
     if (wave >= WAVES) {
       if (g == 0) { s_m[wave - WAVES][rl] = m_run; s_l[wave - WAVES][rl] = l_run; }
 #pragma unroll
@@ -296,13 +301,41 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
   if (wave < WAVES) {
     if (g == 0) { s_m[wave][rl] = m_run; s_l[wave][rl] = l_run; }
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+    for (int n = 0; n < NT; ++n) {
+      if constexpr (WAVES == 8) *reinterpret_cast<f32x4*>(&s_o[wave][rl][16 * n + 4 * g]) = acc[n];
+      else
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s_o[wave][rl][16 * n + 4 * g + r] = acc[n][r];
+        for (int r = 0; r < 4; ++r) s_o[wave][rl][16 * n + 4 * g + r] = acc[n][r];
+    }
   }
   __syncthreads();
 
   const int G_ = G;
+  if (WAVES == 8 && nsplit == 1) {
+    for (int e = 2 * threadIdx.x; e < 16 * D; e += 2 * blockDim.x) {      // two neighbouring columns
+      const int row = e / D, col = e % D;
+      float f[WAVES], M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) M = fmaxf(M, f[w] = s_m[w][row]);
+      const float Ms = (M == -INFINITY) ? 0.f : M;
+      float L = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        f[w] = __builtin_amdgcn_exp2f(f[w] - Ms);
+        const float2 o = *reinterpret_cast<const float2*>(&s_o[w][row][col]);
+        L += s_l[w][row] * f[w];
+        o0 += o.x * f[w];
+        o1 += o.y * f[w];
+      }
+      const int tok = tok0 + row / G_, head = kvh * G_ + row % G_;
+      if (seq < 0 || tok >= qlen) continue;
+      u16* y = a.out + ((long)(qstart + tok) * a.nq + head) * D + col;
+      const uint32_t v = L > 0.f ? f2bf2(o0 / L, o1 / L) : 0u;
+      if (((uintptr_t)a.out & 3) == 0) *reinterpret_cast<uint32_t*>(y) = v;
+      else { y[0] = (u16)v; y[1] = (u16)(v >> 16); }
+    }
+    return;
+  }
   if (nsplit == 1) {
     for (int e = threadIdx.x; e < 16 * D; e += blockDim.x) {
       const int row = e / D, col = e % D;
@@ -454,7 +487,7 @@ __device__ __forceinline__ void attn_unit(const AttnArgs& a, AttnSmem<D>& sm, co
 
 template <int D, int W, bool VN>
 __global__ void __launch_bounds__(64 * W) paged_attn_kernel(AttnArgs a) {
-  __shared__ AttnSmem<D> sm;
+  __shared__ AttnSmem<D, slots(W, D)> sm;
   if (a.items != nullptr) {
     // Persistent decode: a fixed grid (graph-capturable) walks a host-built list of equal-sized
     // key ranges, longest sequences first, so a batch of very different context lengths costs
