@@ -121,6 +121,8 @@ def _pm(x: torch.Tensor, L: Dict[str, torch.Tensor], name: str) -> torch.Tensor:
     wf = L.get(name + "_r")
     if isinstance(x, ops.gemm.Tail):
         return x.linear(L[name], wf)
+    if wf is None and not L["prompt"]:
+        return _mm(x, L[name])
     return _mm(x, L[name], wf, wf is not None and L["order_kept"], L["prompt"])
 
 
