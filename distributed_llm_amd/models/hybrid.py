@@ -469,7 +469,6 @@ class HybridModel:
                 D["dq_norm"], D["dkv_norm"] = f32(t[p + "mix.dq.norm"]), f32(t[p + "mix.dkv.norm"])
                 D["uq"], D["o"] = put(t[p + "mix.uq"]), put(t[p + "mix.o"])
                 D["uk"] = put(t[p + "mix.uk"].view(m.heads, m.dim, m.kv_rank))                       # [H, d, r]
-                self._place_absorb(D)
                 D["uv"] = put(t[p + "mix.uv"].view(m.heads, m.vdim, m.kv_rank))                      # [H, dv, r]
                 D["uvT"] = D["uv"].transpose(1, 2).contiguous()                                      # [H, r, dv]
                 if m.sinks:
@@ -562,9 +561,14 @@ class HybridModel:
         else:
             takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
         todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
-        extra = sum(L[n].numel() * L[n].element_size() for L, n in todo) + self.lm_head.numel() * self.lm_head.element_size()
+        # the key up-projections of latent attention with the ranks as rows (seqmix.latent_absorb)
+        absorb = [L for L in self.layers if "uk" in L and not f32 and not self.order_kept]
+        extra = (sum(L[n].numel() * L[n].element_size() for L, n in todo + [(L, "uk") for L in absorb]) +
+                 self.lm_head.numel() * self.lm_head.element_size())
         if not ops.gemm.copies_fit(extra, self.device, spare):
             return
+        for L in absorb:
+            L["uk_r"] = L["uk"].transpose(1, 2).contiguous()
         for L, S in zip(self.layers, self.cfg.layers):
             f = S.mlp
             act = self._act_args(f) if isinstance(f, DenseSpec) and not self.cfg.parallel_ff else None
@@ -594,11 +598,6 @@ class HybridModel:
             w = torch.cat([w, w.new_zeros(-n % 64, w.shape[1])], 0)
         return put(w), n
 
-    def _place_absorb(self, D) -> None:
-        """The key up-projection as [H, r, d], for the steps of few tokens of a bf16 model on the GPU that bears another order of sums."""
-        if self.dtype == torch.bfloat16 and self.device.type == "cuda" and not self.order_kept:
-            D["uk_r"] = D["uk"].transpose(1, 2).contiguous()
-
     def _place_parallel(self, D, L: LayerSpec, t, p: str, put, f32) -> None:
         """A layer whose mixer and feed-forward read the same input and are added together: one
         projection for everything that reads it, one for everything that is added."""
@@ -614,7 +613,6 @@ class HybridModel:
         else:
             D["dkv_norm"] = f32(t[p + "mix.dkv.norm"])
             D["uk"] = put(t[p + "mix.uk"].view(m.heads, m.dim, m.kv_rank))                       # [H, d, r]
-            self._place_absorb(D)
             D["uv"] = put(t[p + "mix.uv"].view(m.heads, m.vdim, m.kv_rank))                      # [H, dv, r]
             D["uvT"] = D["uv"].transpose(1, 2).contiguous()                                      # [H, r, dv]
             n = m.heads * m.dim + m.kv_rank
