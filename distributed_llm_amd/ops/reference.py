@@ -671,8 +671,9 @@ def paged_gqa_attention(q, k_cache, v_cache, block_tables, qstart, qlen, ctx, ga
     every softmax denominator (it has no value): p_j = exp(s_j) / (sink + sum exp(s_j)).  ``sinks``
     [heads] f32: that term's score per head instead, with weight 1.  ``chunk`` > 0: position i sees the
     keys j <= i of its own chunk, j >= i - i % chunk.  ``softcap``: s <- softcap tanh(s / softcap).
-    ``slopes`` [heads]: s <- s - slopes[head] (i - j).  ``out``: written there."""
+    ``slopes`` [heads]: s <- s - slopes[head] (i - j).  ``out``: written there.  Computed in f32, 64-bit inputs in 64 bits."""
     T, H, d = q.shape
+    wide = torch.float64 if q.dtype == torch.float64 else torch.float32
     G, BSz, dv = k_cache.shape[1], k_cache.shape[2], v_cache.shape[2]
     vrep = G // v_cache.shape[1]
     if out is None:
@@ -684,10 +685,10 @@ def paged_gqa_attention(q, k_cache, v_cache, block_tables, qstart, qlen, ctx, ga
             continue
         nb = (c + BSz - 1) // BSz
         blocks = block_tables[s, :nb].long()
-        K = k_cache[blocks].transpose(1, 2).reshape(nb * BSz, G, d)[:c].float().repeat_interleave(H // G, 1)
-        V = v_cache[blocks].permute(0, 3, 1, 2).reshape(nb * BSz, G // vrep, dv)[:c].float().repeat_interleave(
+        K = k_cache[blocks].transpose(1, 2).reshape(nb * BSz, G, d)[:c].to(wide).repeat_interleave(H // G, 1)
+        V = v_cache[blocks].permute(0, 3, 1, 2).reshape(nb * BSz, G // vrep, dv)[:c].to(wide).repeat_interleave(
             vrep * (H // G), 1)
-        qq = q[qs[s]:qs[s] + n].float()
+        qq = q[qs[s]:qs[s] + n].to(wide)
         sc = torch.einsum("thd,uhd->htu", qq, K)
         pos = torch.arange(c - n, c, device=q.device)
         mask = torch.arange(c, device=q.device)[None, :] > pos[:, None]
@@ -700,10 +701,10 @@ def paged_gqa_attention(q, k_cache, v_cache, block_tables, qstart, qlen, ctx, ga
         if softcap > 0:
             sc = softcap * torch.tanh(sc / softcap)
         if slopes is not None:
-            sc = sc - slopes.float()[:, None, None] * (pos[:, None] - torch.arange(c, device=q.device)[None, :])[None]
+            sc = sc - slopes.to(wide)[:, None, None] * (pos[:, None] - torch.arange(c, device=q.device)[None, :])[None]
         sc = sc.masked_fill(mask[None], float("-inf"))
         if sinks is not None:
-            sc = torch.cat([sc, sinks.float()[:, None, None].expand(H, n, 1)], -1)
+            sc = torch.cat([sc, sinks.to(wide)[:, None, None].expand(H, n, 1)], -1)
             pr = torch.softmax(sc, -1)[..., :-1]
         elif sink > 0:
             mx = sc.max(-1, keepdim=True).values.clamp_min(0.0)
@@ -713,7 +714,7 @@ def paged_gqa_attention(q, k_cache, v_cache, block_tables, qstart, qlen, ctx, ga
             pr = torch.softmax(sc, -1)
         o = torch.einsum("htu,uhv->thv", pr, V).reshape(n, H * dv)
         if gate is not None:
-            gt = torch.sigmoid(gate[qs[s]:qs[s] + n].float())
+            gt = torch.sigmoid(gate[qs[s]:qs[s] + n].to(wide))
             o = o * (gt.repeat_interleave(dv, 1) if gt.shape[1] == H else gt)
         out[qs[s]:qs[s] + n] = o.to(out.dtype)
     return out
