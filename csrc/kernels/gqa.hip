@@ -1091,7 +1091,6 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 192 ? 2 : 1) paged_g
 // with a window of 512 103 / 70; 4001 tokens, 16 heads of 96 / 64 128 / 103; 24 of 160 32.6 / 19.8; four of 200 to 1300, 16 / 4 of 64 with slopes 43 / 29;
 // four of 2900, 16 / 4 of 128 429 / 254; 3000, 8 / 2 of 192 / 128 125 / 94.  Two tiles in LDS with one barrier a tile took 139 for 132, chunks
 // swizzled for fewer bank conflicts nothing.
-// Scores stay below 2^127 (their maximum is taken times log2 e).
 template <int KD, int VD, bool CAP, bool DIST>
 __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) : 2) gqa_cols_kernel(const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
                                                       const int* __restrict__ bt, int bt_ld, const int* __restrict__ qstart,
@@ -1128,7 +1127,13 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) :
     const int c = st * 32 + 8 * g4;
     qb[st] = __builtin_bit_cast(bf16x8, live && c < d ? ld16(q + (tok * H + h) * d + c) : make_uint4(0u, 0u, 0u, 0u));
   }
-  float m = CAP ? 0.f : -INFINITY;
+  // The sums hold weights relative to 2^c2, log2 e times the row's maximum m and rounded: what rescales them is how far c2 moves, exactly 1 where the
+  // maximum has stayed.  (From m times log2 e unrounded it was off by c2's rounding on every tile: 24000 keys with scores of 100 lost 4e-4 of the oldest keys'
+  // weights, here 4e-6, the output's own rounding; time as it was: 153 us for 152 to 155 on the six prompts, 101 for 103 at 96 / 64, 95.6 for
+  // 93.2 at 192 / 128.)  Lowest before the first visible key: weights and sums are 0.
+  constexpr float LOWEST = -0x1.fffffep127f;
+  float m = CAP ? 0.f : -INFINITY, c2 = CAP ? 0.f : LOWEST;
+  bool huge = false;      // a maximum that may leave f32's range times log2 e, in any row of the wave: from there on relative to e^m
   // the weights' sum is one more row of  V^T . P^T,  of ones: four products where 16 additions are a twelfth of a tile's vector instructions
   f32x4 l = {0.f, 0.f, 0.f, 0.f};
   // {-1, 0} in a register: as an inline constant the compiler writes it the way the instruction reads {0, -1}
@@ -1259,7 +1264,6 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) :
           sc[kb][i] = vis ? sc[kb][i] : -INFINITY;
         }
     }
-    float c2 = 0.f, alpha = 1.f;
     if constexpr (!CAP) {
       float mx = -INFINITY;
 #pragma unroll
@@ -1268,9 +1272,24 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) :
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kb][i]);
       mx = lane_max(mx, 16);
       mx = fmaxf(m, lane_max(mx, 32));
-      c2 = mx > -INFINITY ? mx * LOG2E : 0.f;      // before the first visible key: weights, acc and l are 0
-      alpha = __builtin_amdgcn_exp2f(fmaf(m, LOG2E, -c2));
-      m = mx;
+      const float cm = fmaxf(mx * LOG2E, LOWEST);
+      if (__any(mx != m)) {      // (once the running maxima have settled no row of the wave rescales; rows that see no key never do)
+        huge = huge || __any(fabsf(mx) > 0x1p126f && mx > -INFINITY);
+        const float cn = huge ? 0.f : cm;
+        const float alpha = mx == m ? 1.f : __builtin_amdgcn_exp2f(huge ? (m - mx) * LOG2E : c2 - cn);
+        m = mx;
+        c2 = cn;
+        l *= alpha;
+#pragma unroll
+        for (int cb = 0; cb < VB; ++cb) acc[cb] *= alpha;
+      }
+      if (__builtin_expect(huge, 0)) {
+        const float mf = fmaxf(m, LOWEST);
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[kb][i] -= mf;
+      }
     }
     bf16x8 ph[NKB / 2], pl[NKB / 2];      // p = hi + lo with both parts bf16 (the packed conversions round to nearest even)
 #pragma unroll
@@ -1292,13 +1311,6 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) :
       }
       ph[ks] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
       pl[ks] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
-    }
-    if constexpr (!CAP) {
-      if (__any(alpha != 1.f)) {      // (once the running maxima have settled no row of the wave rescales)
-        l *= alpha;
-#pragma unroll
-        for (int cb = 0; cb < VB; ++cb) acc[cb] *= alpha;
-      }
     }
     __builtin_amdgcn_s_setprio(1);      // (ahead of the other waves' vector instructions: 132 -> 122 us)
 #pragma unroll
@@ -1328,17 +1340,19 @@ __global__ void __launch_bounds__(256, KD <= 64 ? 4 : KD <= 96 ? (CAP ? 3 : 4) :
     __builtin_amdgcn_s_setprio(0);
   }
   if (!live) return;
-  if (part) {
+  if (part) {      // relative to e^m, as what merges them takes them
     float* pr = part + ((((long)tile * G + g) * splits + blockIdx.z) * GM_ROWS + row) * (dv + 2);
-    if (g4 == 0) { pr[0] = m; pr[1] = l[0]; }
+    const float f = CAP || huge || !(m > -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(-fmaf(m, LOG2E, -c2));
+    if (g4 == 0) { pr[0] = m; pr[1] = l[0] * f; }
 #pragma unroll
     for (int cb = 0; cb < VB; ++cb)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (16 * cb + 4 * g4 + i < dv) pr[2 + 16 * cb + 4 * g4 + i] = acc[cb][i];
+        if (16 * cb + 4 * g4 + i < dv) pr[2 + 16 * cb + 4 * g4 + i] = acc[cb][i] * f;
     return;
   }
-  float inv = 1.f / (l[0] + (sinks ? __expf(sinks[h] - m) : sink > 0.f ? sink * __expf(-m) : 0.f));
+  auto weight = [&](float x) { return huge ? __expf(x - m) : __builtin_amdgcn_exp2f(fmaf(x, LOG2E, -c2)); };
+  float inv = 1.f / (l[0] + (sinks ? weight(sinks[h]) : sink > 0.f ? sink * weight(0.f) : 0.f));
   if (gate && ghead) inv *= 1.f / (1.f + expf(-bf2f(gate[tok * ldg + h])));
   auto recip = [](float x) { const float r = __builtin_amdgcn_rcpf(x); return x < 1e38f ? r * fmaf(-x, r, 2.f) : r; };
   const u16* gr = gate && !ghead ? gate + tok * ldg + (long)h * dv : nullptr;

@@ -92,3 +92,43 @@ def test_rows_that_see_what_is_not_finite(bad):
         if cache == 1:      # (a key of weight 0 instead of its own)
             same[64:150, 1] = False
         assert torch.equal(got.view(190, 2, 4, 64)[same], clean.view(190, 2, 4, 64)[same])
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (96, 64), (128, 128)])
+@pytest.mark.parametrize("mean,splits", [(0.0, 1), (20.0, 1), (20.0, 3), (100.0, 1)])
+def test_long_contexts_keep_their_oldest_keys_weights(mean, splits, d, dv):
+    """Every key of the older half (values 1) is there again in the newer half (values -1), scores `mean` +- 1: outputs near 0 (the newest rows see a few
+    keys of the newer half less), and a weight that loses or gains a share a tile is off by all of that share.  Weights are in two bf16 parts: 2^-17 of each at
+    most, in any direction; scores are f32 sums, off by some 2^-24 of the largest, alike for a key and its copy."""
+    n, T = 24000, 40
+    q, kc, vc, bt, qs, ql, cx, ts, tt = setup(4, 2, d, dv, [T], [n])
+    q, page = torch.zeros_like(q), bt[0].long()
+    q[:, :, 0], q[:, :, 1] = 4.0, 1.0
+    half = torch.randn(n // 2, 2, d, device=DEV)
+    half[:, :, 0] = mean / 4
+    keys = torch.cat([half, half[torch.randperm(n // 2, device=DEV)]]).bfloat16()
+    kc[page] = keys.view(-1, 16, 2, d).transpose(1, 2)
+    vc[page[:n // 32]], vc[page[n // 32:]] = 1.0, -1.0
+    a = (q, kc, vc, bt, qs, ql, cx, ts, tt)
+    want = ref.paged_gqa_attention(q.double(), kc.double(), vc.double(), bt, qs, ql, cx, None, 0, False, 0, 0.0, 0, 0.0, None, None, None)
+    got, old = (seqmix.paged_gqa_attention(*a, None, mfma=True, splits=splits, out_f32=f) for f in (False, True))
+    assert want.abs().max() < 0.02
+    err, err_old = ((x.double() - want).abs().max().item() for x in (got, old))
+    print("keys %d, scores %g, %d split(s): off by %.2g, other form %.2g" % (n, mean, splits, err, err_old))
+    assert err <= 2.0 ** -9 * want.abs().max().item() + 2.0 ** -18
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_scores_that_leave_f32_times_log2_e(sign, splits):
+    """Scores of 2.5e38 and -2.5e38 are f32 numbers and 1.44 times them are not: the row's largest takes all, the rows without one are as ever."""
+    q, kc, vc, bt, qs, ql, cx, ts, tt = setup(8, 2, 64, 64, [150, 70], [150, 70])
+    q[:, :, 0] = 0.0
+    q[64:90, 1, 0] = 2.0 ** 64
+    kc[:, :, :, 0] = sign * 2.0 ** 63 * (1.0 + torch.arange(16, device=DEV)[None, None] / 32)      # scores to 2^127 (1 + 15 / 32)
+    a = (q, kc.bfloat16(), vc, bt, qs, ql, cx, ts, tt)
+    want = ref.paged_gqa_attention(q.double(), kc.double(), vc.double(), bt, qs, ql, cx, None, 0, False, 0, 0.0, 0, 0.0, None, None, None)
+    got, old = (seqmix.paged_gqa_attention(*a, None, mfma=True, splits=splits, out_f32=f) for f in (False, True))
+    size = want.abs().amax(1, keepdim=True).clamp_min(1.0)
+    assert ((old.double() - want).abs() <= 2.0 ** -14 * size).all()
+    assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * size).all()
