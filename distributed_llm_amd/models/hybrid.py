@@ -1180,7 +1180,8 @@ class HybridModel:
         """``x += rmsnorm(y + bias) * w_post`` and the next sublayer's input ``rmsnorm(x) * w_next``: (stream, input).  ``L``, ``S``: the
         layer that reads the input, with its feed-forward (S None) or with its mixer; where its product takes the
         tail along, the input is an ``ops.gemm.Tail`` and the stream is there once that product has run."""
-        if L is not None and self.tap is None:
+        # (an input convolution reads its rows itself)
+        if L is not None and self.tap is None and (S is None or not self.cfg.input_conv):
             name = "up" if S is None else _FIRST.get(S.mixer.kind)
             wf = L.get("up_act_r", L.get("up_r")) if name == "up" else L.get(f"{name}_r")
             if wf is not None and not L["order_kept"] and wf.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and x.is_contiguous() and \

@@ -75,6 +75,22 @@ def test_not_taken(K):
     assert not G.tail_takes(rnd(4, 64).bfloat16(), rnd(64, 64).bfloat16(), rnd(65)[1:])      # (a vector 4 bytes off)
 
 
+@pytest.mark.parametrize("taps", [0, 3])
+def test_an_input_convolution_reads_rows(monkeypatch, taps):
+    """What a mixer's product takes along exists nowhere else: not where a convolution stands ahead of the mixer.  A feed-forward has none."""
+    from types import SimpleNamespace as NS
+
+    from distributed_llm_amd.models.hybrid import HybridModel
+    monkeypatch.setattr(G, "tail_takes", lambda *a: True)
+    monkeypatch.setattr(seqmix, "resadd_norm", lambda *a, **k: None)
+    m = object.__new__(HybridModel)
+    m.tap, m.dtype, m.cfg = None, torch.bfloat16, NS(rms_eps=1e-5, input_conv=taps)
+    w, v, x = torch.zeros(64, 64, dtype=torch.bfloat16), torch.zeros(64), torch.zeros(2, 64)
+    L = {"proj": w, "proj_r": w, "up": w, "up_act_r": w, "order_kept": False}
+    taken = lambda S: isinstance(m._tail(w[:2], v, x, v, None, L, S)[1], G.Tail)  # noqa: E731
+    assert taken(NS(mixer=NS(kind="mlstm"))) == (taps == 0) and taken(None)
+
+
 @GPU
 def test_replays():
     """In a captured graph, with eager work between: the stream goes on from buffer to buffer."""
