@@ -393,6 +393,21 @@ __global__ void __launch_bounds__(256) latent_attention_kernel(
   float* psh = ksh + KT * kstride;              // [16][64]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int half = rot >> 1;
+  // causal horizon of the block: the last row's position
+  const int last_row = min(row0 + LROWS, nrows) - 1;
+  const int kmax = p0 + tok0 + last_row / H + 1;
+  // split over keys (small grids): the first splits, as many as there are key tiles, share these evenly and leave unnormalised partials, which
+  // latent_combine merges; one without keys leaves nothing but that
+  const int ntiles = (kmax + KT - 1) / KT, sp = min(splits, ntiles), z = min((int)blockIdx.z, sp);
+  const int kbeg = (int)((long)ntiles * z / sp) * KT, kend = min(kmax, (int)((long)ntiles * (z + 1) / sp) * KT);
+  if ((int)blockIdx.z >= sp) {
+    if (tid < LROWS) {
+      const long pr = (((long)entry * gridDim.x + blockIdx.x) * LROWS + tid) * splits + blockIdx.z;
+      part_ml[2 * pr] = -INFINITY;
+      part_ml[2 * pr + 1] = 0.f;
+    }
+    return;
+  }
   // stage the rows' queries (f32, scaled): latent part from qa [H, T, rank], rotated part from q
   for (int e = tid; e < LROWS * Dp; e += 256) {
     const int rr = e / Dp, c = e % Dp, row = row0 + rr;
@@ -409,9 +424,6 @@ __global__ void __launch_bounds__(256) latent_attention_kernel(
     }
     qsh[e] = v;
   }
-  // causal horizon of the block: the last row's position
-  const int last_row = min(row0 + LROWS, nrows) - 1;
-  const int kmax = p0 + tok0 + last_row / H + 1;
   int rpos[4];
   bool rok[4];
 #pragma unroll
@@ -429,11 +441,6 @@ __global__ void __launch_bounds__(256) latent_attention_kernel(
     for (int i = 0; i < RI; ++i) acc[a][i] = 0.f;
   }
   const int* btr = bt + (long)s * bt_w;
-  // split over keys (small grids): split z of `splits` walks its share of the key tiles and leaves
-  // unnormalised partials; latent_combine merges them
-  const int ntiles = (kmax + KT - 1) / KT;
-  const int kbeg = (int)((long)ntiles * blockIdx.z / splits) * KT;
-  const int kend = min(kmax, (int)((long)ntiles * (blockIdx.z + 1) / splits) * KT);
   for (int k0 = kbeg; k0 < kend; k0 += KT) {
     const int nk = min(KT, kend - k0);
     __syncthreads();   // the previous tile is consumed (and the queries are staged)

@@ -209,20 +209,41 @@ def latent_q_prep(q, heads, dim, rot_dim, positions, cos_sin, scale, half: bool 
     return out
 
 
-LAT_SPLIT_TARGET = 256     # workgroups a small latent-attention grid is split up to (over keys): one a CU, what its LDS holds
-LAT_SPLIT_MAX = 64         # lanes of the wave that merges them
+LAT_SPLIT_MAX = 64         # lanes of the wave that merges a latent attention launch's key splits
 
 
-def latent_splits(n_entries: int, heads: int, rows: int = LAT_ROWS) -> int:
-    """Key splits of a latent attention launch: grids with fewer than ``LAT_SPLIT_TARGET`` workgroups (decode steps, short portions) split
-    every row's keys over as many workgroups as one round of the CUs holds, up to ``LAT_SPLIT_MAX`` (splits without keys cost next to
+def latent_splits(n_entries: int, heads: int, rows: int = LAT_ROWS, cus: int = 256, vector: int = 0) -> int:
+    """Key splits of a latent attention launch: grids with fewer workgroups than ``cus`` (decode steps, short portions) split every row's keys over
+    as many as one round of the CUs holds (the LDS of one holds one workgroup), up to ``LAT_SPLIT_MAX`` (splits without keys cost next to
     nothing: those with keys are the first ones).  us with the merge, up to 16 splits and 512 workgroups / here, 16 heads: one of 4001 24.7
     / 16.6, two of 8000 39.4 / 21.7, four of 300 to 1300 18.0 / 15.5, 24 of up to 316 17.4 / 15.1, 48 of 1000 34.0 / 28.3, a portion of 256 38.7 / 21.5.  More
-    than half a round of entries are split only into the three that nearly fill two: 150 tokens behind 1000 in one 68.8, in three 62.3."""
-    n = n_entries * (((1 if heads >= rows else rows // heads) * heads + rows - 1) // rows)
-    if n > LAT_SPLIT_TARGET // 2:
-        return 3 if 2 * LAT_SPLIT_TARGET // n >= 3 else 1
-    return min(LAT_SPLIT_MAX, LAT_SPLIT_TARGET // max(1, n))
+    than half a round of entries are split only into the three that nearly fill two: 150 tokens behind 1000 in one 68.8, in three 62.3.  From there to a
+    whole round nothing is gained, 171 / 256 entries in one and in two: 60 keys 10.6 / 10.7 and 19.0 / 23.2, 1000 65 / 66 and 79 / 83, 2500 147 / 152
+    and 161 / 168, 64 heads of 50 tokens with the value up-projection in the merge 70.6 and 86.1 (as a product of its own in the first).
+    ``vector``: the workgroups a CU holds of the form that f32 models run (``latent_vector_wgs``): a round of those too, or two where one leaves a
+    seventh of it idle and two do not.  us, up to 16 splits and 512 workgroups, keys over all of them / here: 16 heads, rank 256, one of 400 33.0 / 33.6, of
+    4001 96 / 36.5, four of 300 to 1300 54 / 34.7, 24 of up to 316 42.5 / 34.5, 48 of 1000 156 / 143, 100 of 300 93.3 / 95.0 (in two 113); 32 heads, rank
+    512, 51 / 41, 259 / 78, 112 / 97, 120 / 92, 619 / 533; 8 heads, rank 128, two workgroups a CU, 22.5 / 22.4, 66 / 25, 37 / 23.4, 24.3 / 23.0, 57.7 / 57.9
+    (in five 85), 200 of 300 79 / 67."""
+    n = max(1, n_entries * (((1 if heads >= rows else rows // heads) * heads + rows - 1) // rows))
+    if vector:
+        slots = vector * cus
+        sp = slots // n
+        if 7 * sp * n < 6 * slots and n <= cus and 2 * slots // n > 2 * sp:
+            sp = 2 * slots // n
+        return max(1, min(LAT_SPLIT_MAX, sp))
+    if n > cus // 2:
+        return 3 if 2 * cus // n >= 3 else 1
+    return min(LAT_SPLIT_MAX, cus // n)
+
+
+def latent_vector_wgs(rank: int, rot_dim: int) -> int:
+    """Workgroups of the vector form that the LDS of a CU holds: the queries of 16 rows, up to 64 keys and their weights in f32."""
+    return 2 if 4 * (80 * (rank + rot_dim) + 1280) <= 80 << 10 else 1
+
+
+def _cus(x: torch.Tensor) -> int:
+    return torch.cuda.get_device_properties(x.device).multi_processor_count
 
 
 def latent_rows(x: torch.Tensor, rank: int, rot_dim: int, tokens: int, seqs: int) -> int:
@@ -263,7 +284,7 @@ def latent_up_ok(x: torch.Tensor, heads: int, tokens: int, entries: int, rank: i
         return False
     ext = _native(x)
     return (ext is not None and uv.shape[2] in (32, 64, 128) and uv.is_contiguous() and uv.data_ptr() % 16 == 0 and
-            latent_splits(entries, heads, rows) > 1 and bool(ext.latent_mfma_ok(int(rank), int(rot_dim), int(rows))))
+            latent_splits(entries, heads, rows, _cus(x)) > 1 and bool(ext.latent_mfma_ok(int(rank), int(rot_dim), int(rows))))
 
 
 def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_tables, qstart, qlen, ctx, tile_seq,
@@ -284,15 +305,17 @@ def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_table
     if out is None:
         out = torch.zeros_like(qa) if up is None else qa      # with splits and an up-projection nothing is written there
     H, n_entries = qa.shape[0], int(tile_seq.numel())
-    sp = latent_splits(n_entries, H, rows) if splits is None else int(splits)
+    if mfma is None:
+        mfma = os.environ.get("DLLM_LATENT_MFMA", "1") == "1"
+    matrix = bool(mfma) and qa.dtype == torch.bfloat16 and bool(ext.latent_mfma_ok(int(qa.shape[2]), int(rot_dim), int(rows)))
+    vector = 0 if matrix else latent_vector_wgs(qa.shape[2], rot_dim)
+    sp = latent_splits(n_entries, H, rows, _cus(qa), vector) if splits is None else int(splits)
     po = pml = None
     if sp > 1:
         gx = ((1 if H >= rows else rows // H) * H + rows - 1) // rows
         prow = n_entries * gx * rows * sp
         po = torch.empty(prow * qa.shape[2], dtype=torch.float32, device=qa.device)
         pml = torch.empty(prow * 2, dtype=torch.float32, device=qa.device)
-    if mfma is None:
-        mfma = os.environ.get("DLLM_LATENT_MFMA", "1") == "1"
     ext.latent_attention(qa, q, int(dim), int(rot_dim), positions, cos_sin, cache, block_tables, qstart, qlen, ctx,
                          tile_seq, tile_tok0, float(scale), out, sp, po, pml, bool(mfma), int(rows), bool(half), sinks, *(up or ()))
     return out if up is None else up[2]

@@ -15,6 +15,46 @@ def test_one_round_of_workgroups():
     assert seqmix.latent_splits(4, 8) == 64 and seqmix.latent_splits(40, 128) == 1      # (eight 16-row blocks an entry)
 
 
+def test_rounds_of_the_device_and_of_the_vector_form():
+    assert [seqmix.latent_splits(n, 16, cus=64) for n in (1, 4, 24, 32, 33, 42, 43, 100)] == [64, 16, 2, 2, 3, 3, 1, 1]
+    assert [seqmix.latent_splits(n, 16, vector=1) for n in (1, 4, 5, 24, 48, 75, 100, 128, 150, 200, 219, 220, 256, 257, 900)] == \
+        [64, 64, 51, 10, 5, 3, 5, 2, 3, 1, 1, 1, 1, 1, 1]
+    assert [seqmix.latent_splits(n, 16, vector=2) for n in (1, 8, 9, 48, 150, 200, 256, 257, 400, 900)] == [64, 64, 56, 10, 3, 5, 2, 1, 1, 1]
+    assert [seqmix.latent_vector_wgs(*r) for r in ((128, 32), (240, 0), (241, 0), (256, 32))] == [2, 2, 1, 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,rank,rd", [(16, 256, 32), (4, 128, 6), (32, 512, 64)])
+def test_f32_splits_against_64_bits(H, rank, rd):
+    """The vector form, whose tiles are 64 keys, or 32 at rank 512: splits with and without keys, more of them than tiles, the rule's own."""
+    torch.manual_seed(H)
+    dim, dev, ctxs = 32, "cuda", [1, 31, 64, 65, 700, 1025, 2300]
+    n, per = len(ctxs), [(c + 15) // 16 for c in ctxs]
+    I = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    bt, at = torch.zeros(n, max(per), dtype=torch.int32), 1
+    for i, m in enumerate(per):
+        bt[i, :m] = torch.arange(at, at + m)
+        at += m
+    cache = torch.randn(at, 16, rank + rd, device=dev)
+    qa, q = torch.randn(H, n, rank, device=dev), torch.randn(n, H * (dim + rd), device=dev)
+    table, pos, scale, sinks = ops.rope_cos_sin(4096, rd, 10000.0, torch.device(dev)), I([c - 1 for c in ctxs]), 0.05, torch.randn(H, device=dev)
+    args = (qa, q, dim, rd, pos, table, cache, bt.to(dev), I(list(range(n))), I([1] * n), I(ctxs), I(list(range(n))), I([0] * n), scale)
+    want = torch.empty(H, n, rank, dtype=torch.float64, device=dev)
+    for i, c in enumerate(ctxs):
+        kv = cache[bt[i, :per[i]].long().to(dev)].flatten(0, 1)[:c].double()
+        cs, sn = (x.double() for x in ref._rot_table(table, pos[i:i + 1], rd // 2))
+        qr = ref._rope_interleaved(q[i:i + 1].double().view(1, H, dim + rd)[..., dim:], cs[:, None], sn[:, None])[0]
+        sc = torch.cat([(qa[:, i].double() @ kv[:, :rank].t() + qr @ kv[:, rank:].t()) * scale, sinks.double()[:, None]], 1)
+        want[:, i] = torch.softmax(sc, 1)[:, :c] @ kv[:, :rank]
+    one = None
+    for splits in (1, 2, 10, 16, 33, 64, None):
+        got = seqmix.latent_attention(*args, splits=splits, sinks=sinks)
+        err = float((got - want).norm() / want.norm())
+        one = err if one is None else one
+        print("H %d rank %d splits %s: off by %.2g" % (H, rank, splits, err))
+        assert err <= 4e-6 and err <= 1.5 * one      # f32 sums, whose shorter parts are no worse
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [1, 2, 16, 17, 33, 64])
 @pytest.mark.parametrize("sink", [False, True])
