@@ -354,7 +354,8 @@ class LLMEngine:
                                       verbose=os.environ.get("DLLM_VERBOSE") == "1",
                                       frag=[] if m.lm_head_r is None else [b[:2] for b in big])
                     ops.gemm.reserve(self.device)
-            ops.gemm.autotune_prompts(m.prompt_shapes(), self.device)
+            # rows of one chunk: generation's have max_prefill_tokens at most, a program's own (``feed``) what rows and pool hold
+            ops.gemm.autotune_prompts(m.prompt_shapes(), self.device, min(self.max_num_seqs * self.max_model_len, self.num_blocks * BS))
             return
         shapes = set()
         L = m.layers[0]

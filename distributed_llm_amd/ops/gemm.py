@@ -31,7 +31,7 @@ import contextvars
 import json
 import math
 import os
-from typing import Dict, Iterable, Optional, Tuple
+from typing import Dict, Iterable, List, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -463,11 +463,12 @@ def prompt_plan(M: int, N: int, K: int, gelu: bool = False) -> Optional[Tuple]:
     return _keep(_P.pp_plans, key, best and best[1])
 
 
-def autotune_prompts(shapes: Iterable[Tuple[int, int, bool]], device) -> None:
-    """Times the plain products of prompts, ``prompt_plan``'s choice: (N, K, with a GELU behind it) of each."""
+def autotune_prompts(shapes: Iterable[Tuple[int, int, bool]], device, most: int = PP_MS[-1]) -> None:
+    """Times the plain products of prompts, ``prompt_plan``'s choice: (N, K, with a GELU behind it) of each, up to the timed size that holds ``most``
+    rows.  What was timed before stands.  Where there is no memory for a size, that and the longer ones are left to the vendor's product."""
     from . import seqmix
     dev = torch.device(device)
-    if dev.type != "cuda" or os.environ.get("DLLM_GEMM") == "blas":
+    if dev.type != "cuda" or most <= MAX_M or os.environ.get("DLLM_GEMM") == "blas":
         return
     cache = os.environ.get("DLLM_GEMM_PLANS")
     made = _timed_with(dev) if cache else ""
@@ -480,31 +481,40 @@ def autotune_prompts(shapes: Iterable[Tuple[int, int, bool]], device) -> None:
         _P.pp_plans.clear()
     for N, K, gelu in shapes:
         key = (N, K, int(gelu))
-        if key in _P.pp_times:
+        vendor, own = _P.pp_times.setdefault(key, ([], []))
+        ms, own_ms = _pp_left(PP_MS, vendor, most), _pp_left(PP_OWN_MS, own, most)
+        if not ms and not own_ms:
             continue
-        copies = max(2, min(8, (256 << 20) // (N * K * 2)))
-        ws = [(torch.randn(N, K, device=dev) * 0.02).to(torch.bfloat16) for _ in range(copies)]
-        most, vendor, own = PP_MS[-1], [], []
-        while most >= PP_MS[0]:      # (where so many rows find no memory, fewer are timed)
-            try:
-                X, Y = torch.randn(most, K, dtype=torch.bfloat16, device=dev), torch.empty(most, N, dtype=torch.bfloat16, device=dev)
-                break
-            except torch.OutOfMemoryError:
-                most //= 2
-        for M in (m for m in PP_MS if m <= most):
-            x, y = X[:M], Y[:M]
+        try:
+            copies = max(2, min(8, (256 << 20) // (N * K * 2)))
+            ws = [torch.randn(N, K, dtype=torch.bfloat16, device=dev).mul_(0.02) for _ in range(copies)]
+            for M in sorted({*ms, *own_ms}):
+                x, y = torch.randn(M, K, dtype=torch.bfloat16, device=dev), torch.empty(M, N, dtype=torch.bfloat16, device=dev)
 
-            def call(i):
-                torch.matmul(x, ws[i % copies].t(), out=y)
-                if gelu:
-                    seqmix.gelu_erf(y)
-            vendor.append((M, _time(call, iters=4)))
-            if M in PP_OWN_MS:
-                epi, ext = EPI_GELU if gelu else EPI_PLAIN, _native(x)
-                own.append((M, [_time(lambda i: _tgemm(ext, x, ws[i % copies], epi, p, y=y), iters=4) for p in _PP_PLANS]))
-        _P.pp_times[key] = (vendor, own)
+                def call(i):
+                    torch.matmul(x, ws[i % copies].t(), out=y)
+                    if gelu:
+                        seqmix.gelu_erf(y)
+                us = _time(call, iters=4) if M in ms else None
+                if M in own_ms:
+                    epi, ext = EPI_GELU if gelu else EPI_PLAIN, _native(x)
+                    own.append((M, [_time(lambda i: _tgemm(ext, x, ws[i % copies], epi, p, y=y), iters=4) for p in _PP_PLANS]))
+                if us is not None:
+                    vendor.append((M, us))
+                del x, y
+        except torch.OutOfMemoryError:
+            continue
+        finally:
+            for k in list(_P.pp_plans):      # (rows past what was timed have another answer now)
+                if k[1:] == key:
+                    _P.pp_plans.pop(k, None)
     if cache:
         _save_plans(cache, made)
+
+
+def _pp_left(sizes: Iterable[int], have: list, most: int) -> List[int]:
+    """The row counts that are left to time for prompts of up to ``most`` rows: up to the next one that holds them."""
+    return [m for i, m in enumerate(sizes) if (i == 0 or sizes[i - 1] < most) and m > (have[-1][0] if have else 0)]
 
 
 def prompt_gelu(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:

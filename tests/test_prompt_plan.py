@@ -50,6 +50,59 @@ def test_answers_are_bounded_and_kept_in_plan_files(tmp_path):
     assert G._P.pp_times == want
 
 
+def test_sizes_that_an_engine_has_no_rows_for_are_not_timed():
+    left = lambda most, have=(): G._pp_left((1280, 2048, 4096, 8192), [(m, 1.0) for m in have], most)  # noqa: E731
+    assert left(1025) == left(1280) == [1280] and left(1281) == left(2048) == [1280, 2048] and left(9000) == [1280, 2048, 4096, 8192]
+    assert left(2000, (1280, 2048)) == [] and left(2049, (1280, 2048)) == [4096]      # what was timed stands
+
+
+class Timing:
+    """Stands in for the device and its clock; memory for tensors of ``rows``."""
+
+    def __init__(self, monkeypatch, rows=1 << 20):
+        self.rows, self.seen = rows, []
+        randn = torch.randn
+
+        def made(*s, dtype=None, device=None):
+            if s[0] > self.rows:
+                raise torch.OutOfMemoryError("no room")
+            self.seen.append(s[0])
+            return randn(1, 1)
+        monkeypatch.setattr(torch, "randn", made)
+        monkeypatch.setattr(torch, "empty", lambda *s, **k: None)
+        monkeypatch.setattr(G, "_sk_grid", lambda d: 256)
+        monkeypatch.setattr(G, "_native", lambda t: None)
+        monkeypatch.setattr(G, "_time", lambda f, iters: 100.0)
+
+
+def test_an_engine_times_what_it_can_hold(monkeypatch):
+    t = Timing(monkeypatch)
+    G.autotune_prompts([(1024, 512, False)], "cuda", 1024)
+    assert not t.seen and not G._P.pp_times
+    G.autotune_prompts([(1024, 512, False)], "cuda", 1500)
+    assert [m for m, _ in G._P.pp_times[(1024, 512, 0)][0]] == [1280, 1536] and [m for m, _ in G._P.pp_times[(1024, 512, 0)][1]] == [2048]
+    assert G.prompt_plan(1500, 1024, 512) is None and G.prompt_plan(9000, 1024, 512) is None
+    first, G._P.pp_times[(1024, 512, 0)][0][0] = G._P.pp_times[(1024, 512, 0)], (1280, 77.0)
+    t.seen.clear()
+    G.autotune_prompts([(1024, 512, False)], "cuda", 1 << 20)      # a larger engine times the rest
+    vendor, own = G._P.pp_times[(1024, 512, 0)]
+    assert vendor is first[0] and vendor[0] == (1280, 77.0) and [m for m, _ in vendor] == list(G.PP_MS) and [m for m, _ in own] == list(G.PP_OWN_MS)
+    assert t.seen.count(1280) == t.seen.count(2048) - 1 == 0 and (9000, 1024, 512, 0) not in G._P.pp_plans
+
+
+@pytest.mark.parametrize("rows,vendor,own", [(5000, 4864, 4096), (1500, 1280, None), (600, None, None)])
+def test_sizes_without_memory_are_left_to_the_vendor(monkeypatch, rows, vendor, own):
+    Timing(monkeypatch, rows)
+    G.autotune_prompts([(1024, 512, False), (256, 128, True)], "cuda")
+    for key in ((1024, 512, 0), (256, 128, 1)):
+        a, b = G._P.pp_times[key]
+        if key[0] > rows:      # no room for its weights either
+            assert not a and not b
+            continue
+        assert (a[-1][0] if a else None) == (vendor if vendor else None) and (b[-1][0] if b else None) == own
+    assert G.prompt_plan(12000, 1024, 512) is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1025, 64, 64), (1300, 1600, 192), (2049, 3136, 1024), (4000, 264, 128)])
 @pytest.mark.parametrize("plan", G._PP_PLANS)
