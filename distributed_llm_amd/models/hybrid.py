@@ -561,14 +561,14 @@ class HybridModel:
         else:
             takes = lambda w: w.shape[1] % 64 == 0 and w.shape[0] % (64 if self.order_kept else 8) == 0
         todo = [(L, n) for L in self.layers for n in _PROJECTIONS if n in L and takes(L[n])]
-        # the key up-projections of latent attention with the ranks as rows (seqmix.latent_absorb)
+        # what saves least of a step for its bytes comes last and does not cost the others their place: long f32 rows, and the key
+        # up-projections of latent attention with the ranks as rows (seqmix.latent_absorb)
+        later = [(L, n) for L, n in todo if f32 and L[n].shape[1] > 2048]
+        todo = [(L, n) for L, n in todo if not any(l is L and m == n for l, m in later)]
         absorb = [L for L in self.layers if "uk" in L and not f32 and not self.order_kept]
-        extra = (sum(L[n].numel() * L[n].element_size() for L, n in todo + [(L, "uk") for L in absorb]) +
-                 self.lm_head.numel() * self.lm_head.element_size())
-        if not ops.gemm.copies_fit(extra, self.device, spare):
+        size = lambda which: sum(L[n].numel() * L[n].element_size() for L, n in which)  # noqa: E731
+        if not ops.gemm.copies_fit(size(todo) + self.lm_head.numel() * self.lm_head.element_size(), self.device, spare):
             return
-        for L in absorb:
-            L["uk_r"] = L["uk"].transpose(1, 2).contiguous()
         for L, S in zip(self.layers, self.cfg.layers):
             f = S.mlp
             act = self._act_args(f) if isinstance(f, DenseSpec) and not self.cfg.parallel_ff else None
@@ -582,12 +582,16 @@ class HybridModel:
         ex = [(L, S.mlp) for L, S in zip(self.layers, self.cfg.layers)
               if not f32 and isinstance(S.mlp, MoESpec) and "w2" in L and L["w1"].shape[1] % 64 == 0 and L["w1"].shape[2] % 64 == 0
               and L["w2"].shape[2] % 64 == 0 and (S.mlp.act != "swiglu" or L.get("tg"))]
-        extra = sum(L[n].numel() * L[n].element_size() for L, _ in ex for n in ("w1", "w2"))
-        if ops.gemm.copies_fit(extra, self.device, spare):
+        if ops.gemm.copies_fit(size((L, n) for L, _ in ex for n in ("w1", "w2")), self.device, spare):
             for L, f in ex:
                 L["experts_r"] = (ops.frag_experts(L["w1"], paired=f.act == "swiglu"), ops.frag_experts(L["w2"]), self.order_kept)
         if takes(self.lm_head):
             self.lm_head_r = ops.gemm.frag_weight(self.lm_head)
+        if ops.gemm.copies_fit(size(later + [(L, "uk") for L in absorb]), self.device, spare):
+            for L, n in later:
+                L[n + "_r"], L["order_kept"] = ops.gemm.frag_weight(L[n]), self.order_kept
+            for L in absorb:
+                L["uk_r"] = L["uk"].transpose(1, 2).contiguous()
 
     def _fuse(self, parts: List[torch.Tensor], put) -> Tuple[torch.Tensor, int]:
         """One projection for several that read the same input, and its rows; bf16 models on the GPU get

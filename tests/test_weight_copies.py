@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from distributed_llm_amd.models.configs import ModelConfig, filevik_config
+from distributed_llm_amd.models.configs import ModelConfig, filevik_config, sedopel_config
 from distributed_llm_amd.models.registry import build_model
 from distributed_llm_amd.ops import gemm as G
 
@@ -72,3 +72,23 @@ def test_the_pool_comes_first(monkeypatch, cfg, some):
     got = torch.cat(steps(without))
     # other plans: bf16 roundings of a few layers
     assert float((got - want).norm() / want.norm()) < 2.0 ** -5
+
+
+LONG = sedopel_config({"architecture": "Sedopel", "width": 128, "vocab": 512, "norm": {"eps": 1e-6}, "layers": [
+    {"type": "delta", "mlp": {"kind": "dense", "ff": 4096}, "mixer": {"heads": 2, "kv_heads": 1, "dim": 64, "vdim": 64, "conv": 4}}] * 2})
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg,dtype,last", [(LONG, torch.float32, "down_r"), (LAYERS, torch.bfloat16, "uk_r")], ids=["long f32 rows", "uk"])
+def test_the_last_copies_cost_no_other_its_place(monkeypatch, cfg, dtype, last):
+    """Room for all but the long rows of an f32 model, or all but the key up-projections: only those are missing."""
+    asked, room = [], [1 << 40]
+    monkeypatch.setattr(G, "copies_fit", lambda extra, device, spare=0: (asked.append(extra), extra <= room[0])[1])
+    every = set(_copies(build_model(cfg, dtype=dtype)))
+    assert last in every
+    mine = sum(asked[:1])      # the projections and the head; what else there is was asked for behind them
+    base, asked[:] = set(every) - {last}, []
+    room[0] = mine
+    monkeypatch.setattr(G, "copies_fit", lambda extra, device, spare=0: (asked.append(extra), len(asked) == 1 and extra <= room[0])[1])
+    got = set(_copies(build_model(cfg, dtype=dtype)))
+    assert got == base - {"experts_r"} and got
