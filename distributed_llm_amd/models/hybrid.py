@@ -121,9 +121,8 @@ def _pm(x: torch.Tensor, L: Dict[str, torch.Tensor], name: str) -> torch.Tensor:
     wf = L.get(name + "_r")
     if isinstance(x, ops.gemm.Tail):
         return x.linear(L[name], wf)
-    if wf is None and not L["prompt"]:
-        return _mm(x, L[name])
-    return _mm(x, L[name], wf, wf is not None and L["order_kept"], L["prompt"])
+    more = {} if wf is None else {"wf": wf, "keep_order": L["order_kept"]}
+    return _mm(x, L[name], prompt=True, **more) if L["prompt"] else _mm(x, L[name], **more)
 
 
 class HybridModel:
