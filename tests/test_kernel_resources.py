@@ -57,6 +57,8 @@ WAVES = [
     ("gqa.hip", r"paged_gqa_mfma_kernelILi(128|192)E", 2),      # 24 decode rows of 192-wide heads: 14 us, 20 with one
     ("gqa.hip", r"paged_gqa_mfma_kernelILi96E", 3),
     ("gqa.hip", r"gqa_few_kernel", 2),
+    ("gqa.hip", r"gqa_cols_kernelILi(64|96)E", 4),      # 96 / 64 with slopes holds 124 of 128
+    ("gqa.hip", r"gqa_cols_kernelILi(128|192)E", 2),
 ]
 
 
