@@ -149,8 +149,8 @@ static __device__ __forceinline__ float block_sum(float v, float* red) {
 // x (1 + erf(x / sqrt 2)) / 2 for values that end in bf16: max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, with erfc(z) = exp(-z^2) t P(t), t = 1 / (1 + z / 2);
 // 2 P: a fit of erfcx(z) / t on z from 0 to 10 to the least largest relative error (4.3e-8, reweighted least squares).  Half of erff's instructions, which
 // were most of an epilogue, and no cancellation where 1 + erf is small: the largest relative error against 64 bits is 3e-7 from -1 to 1 and 7e-7 to -3,
-// 9e-6 below (with erff 1.4e-7, 7e-6, 4e-2 to -5 and 1), and of the 65280 finite bf16 inputs none rounds to another bf16 than the exact
-// value (197 with erff).  3571 x 1536 x 384 with it: 16.0 us, with erff 16.9.  NaN and infinities as there (-inf: NaN).
+// 9e-6 below (with erff 1.4e-7, 7e-6, 4e-2 to -5 and 1), and of the 65280 finite bf16 inputs none whose result is 2^-125 or more rounds to another bf16
+// than the exact value (197 with erff; smaller results, at x below -13, may be 0: the exponential's instruction has no subnormal numbers).  3571 x 1536 x 384 with it: 16.0 us, with erff 16.9.  NaN and infinities as there (-inf: NaN).
 static __device__ __forceinline__ float gelu_bf(float x) {
   const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.35355339059327373f, 1.f)), u = x * 0.84932180028801907f;      // sqrt(log2(e) / 2)
   float p = fmaf(t, -0.029534505680203438f, 0.14228759706020355f);

@@ -66,7 +66,8 @@ __global__ void __launch_bounds__(64 * NW) f32_gemm_kernel(const float* __restri
 // (pieces of a k 16 bytes off the power of two: at eight rows of 1024 x 1024 4.4 us without, here 4.0).  us, the kernel above / here (the
 // vendor's): 2 rows 512 x 512 2.96 / 2.68 (4.4), 2048 x 512 3.4 / 3.1 (5.8), 1024 x 1024 4.1 / 3.5 (8.1), 1024 x 2048 6.2 / 4.4 (8.5), 2048 x
 // 2048 6.1 / 5.0 (8.7), 1024 x 4096 10.2 / 6.1 (10.1), 2048 x 8192 22.3 / 18.1 (22.7), 32000 x 1024 25.1 / 23.0 (32.4); 8 rows 2048 x 512 3.6 /
-// 3.5, 1024 x 1024 4.5 / 4.0, 2048 x 2048 7.4 / 5.5, 1024 x 4096 12.3 / 7.5 (10.1).  Sums of K / 64 terms: 1.4e-7 from 64 bits at 2048 k, 3.0e-7 above.
+// 3.5, 1024 x 1024 4.5 / 4.0, 2048 x 2048 7.4 / 5.5, 1024 x 4096 12.3 / 7.5 (10.1).  Sums of K / 64 terms with sixteen waves, K / 32 with
+// eight (K up to 512, and the weights of 64 MB and more): with sixteen 1.4e-7 from 64 bits at 2048 k, 3.0e-7 above.
 template <int EPI, int RB, int NWV, int KS>
 __global__ void __launch_bounds__(64 * NWV) f32_few_kernel(const float* __restrict__ X, long ldx, const float* __restrict__ W, float* __restrict__ Y,
                                                            long ldy, int M, int N, int K) {
