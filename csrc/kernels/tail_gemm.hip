@@ -12,7 +12,8 @@
 //     tiles through LDS, the same order of sums.  NT tiles of 16 columns a workgroup: one while a round of workgroups holds them, else two.
 // us in a captured graph, width 1024, two launches / here: 1088 columns 1 row 6.1 / 3.9, 4 rows 6.2 / 3.9, 8 6.4 / 4.7, 16 6.8 / 6.3; 3136 columns
 // 6.5 / 4.2, 6.5 / 4.1, 6.8 / 4.8, 7.0 / 6.4; 5632 gated 8.4 / 4.9, 8.5 / 5.2, 9.3 / 5.9, 9.3 / 7.8; 8192 7.5 / 5.0, 7.6 / 5.5, 7.8 / 5.7, 7.9 / 7.3
-// (two rows a SIMD and more add their arithmetic, 0.2 us a row).
+// (two rows a SIMD and more add their arithmetic, 0.2 us a row: widths up to 512 win with up to 12 rows, ops.gemm.tail_wins; 3136 columns of 512 1 row 5.6 /
+// 3.8, 8 6.0 / 4.8, 12 6.1 / 5.5, of 768 5.8 / 4.0, 6.4 / 4.8, 16 6.7 / 6.4).
 #include "common.h"
 
 namespace {

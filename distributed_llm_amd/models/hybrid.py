@@ -1188,7 +1188,7 @@ class HybridModel:
             name = "up" if S is None else _FIRST.get(S.mixer.kind)
             wf = L.get("up_act_r", L.get("up_r")) if name == "up" else L.get(f"{name}_r")
             if wf is not None and not L["order_kept"] and wf.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 and x.is_contiguous() and \
-                    ops.gemm.tail_takes(y, L[name], w_post, w_next, bias, L.get("up_b") if name == "up" else None):
+                    ops.gemm.tail_wins(*y.shape) and ops.gemm.tail_takes(y, L[name], w_post, w_next, bias, L.get("up_b") if name == "up" else None):
                 x2 = torch.empty_like(x)
                 return x2, ops.gemm.Tail(y, w_post, self.cfg.rms_eps, x, x2, w_next, bias)
         h = torch.empty(x.shape, dtype=self.dtype, device=x.device)

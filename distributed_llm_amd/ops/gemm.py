@@ -841,6 +841,13 @@ def tail_takes(y: torch.Tensor, w: torch.Tensor, *vectors: Optional[torch.Tensor
             all(v is None or (v.dtype == torch.float32 and v.is_contiguous() and v.data_ptr() % 16 == 0) for v in vectors))
 
 
+def tail_wins(M: int, K: int) -> bool:
+    """Is one launch the faster form?  From the 13th row on a SIMD norms four, which widths up to 512 do not bear: us, two launches / one, 3136 columns, 8,
+    12, 13 and 16 rows of 256 5.4 / 4.8, 5.5 / 5.5, 5.4 / 5.9, 5.5 / 6.1; of 512 6.0 / 4.8, 6.1 / 5.5, 6.1 / 6.0, 6.1 / 6.3; of 576 6.2 / 4.8, 6.3 / 5.7,
+    6.2 / 6.0, 6.5 / 6.4; of 768 and 16 6.7 / 6.4."""
+    return M <= 12 or K > 512
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
            wp: Optional[torch.Tensor] = None, wf: Optional[torch.Tensor] = None, keep_order: bool = False, prompt: bool = False) -> torch.Tensor:
     """``x @ w.T`` on the shape's tuned plan; ``prompt``: many rows may take the tile timed for them (``prompt_plan``); ``wp``: the panel copy a tgemm plan streams, ``wf``: the fragment-major copy of the

@@ -91,6 +91,20 @@ def test_an_input_convolution_reads_rows(monkeypatch, taps):
     assert taken(NS(mixer=NS(kind="mlstm"))) == (taps == 0) and taken(None)
 
 
+@pytest.mark.parametrize("M,K,one", [(1, 64, True), (12, 512, True), (13, 512, False), (16, 256, False), (13, 576, True), (16, 1024, True)])
+def test_rows_and_widths_of_one_launch(monkeypatch, M, K, one):
+    from types import SimpleNamespace as NS
+
+    from distributed_llm_amd.models.hybrid import HybridModel
+    monkeypatch.setattr(G, "tail_takes", lambda *a: True)
+    monkeypatch.setattr(seqmix, "resadd_norm", lambda *a, **k: None)
+    m = object.__new__(HybridModel)
+    m.tap, m.dtype, m.cfg = None, torch.bfloat16, NS(rms_eps=1e-5, input_conv=0)
+    w, v = torch.zeros(64, K, dtype=torch.bfloat16), torch.zeros(K)
+    L = {"up": w, "up_act_r": w, "order_kept": False}
+    assert isinstance(m._tail(w[:M], v, torch.zeros(M, K), v, None, L)[1], G.Tail) == one
+
+
 @GPU
 def test_replays():
     """In a captured graph, with eager work between: the stream goes on from buffer to buffer."""
