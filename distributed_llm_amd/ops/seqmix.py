@@ -25,6 +25,7 @@ sequence whose first new position is 0 starts from a zero state, so a re-used sl
 """
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional, Tuple
 
@@ -242,8 +243,9 @@ def latent_vector_wgs(rank: int, rot_dim: int) -> int:
     return 2 if 4 * (80 * (rank + rot_dim) + 1280) <= 80 << 10 else 1
 
 
-def _cus(x: torch.Tensor) -> int:
-    return torch.cuda.get_device_properties(x.device).multi_processor_count
+@functools.lru_cache(maxsize=None)
+def _cus(device: torch.device) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
 
 
 def latent_rows(x: torch.Tensor, rank: int, rot_dim: int, tokens: int, seqs: int) -> int:
@@ -284,7 +286,7 @@ def latent_up_ok(x: torch.Tensor, heads: int, tokens: int, entries: int, rank: i
         return False
     ext = _native(x)
     return (ext is not None and uv.shape[2] in (32, 64, 128) and uv.is_contiguous() and uv.data_ptr() % 16 == 0 and
-            latent_splits(entries, heads, rows, _cus(x)) > 1 and bool(ext.latent_mfma_ok(int(rank), int(rot_dim), int(rows))))
+            latent_splits(entries, heads, rows, _cus(x.device)) > 1 and bool(ext.latent_mfma_ok(int(rank), int(rot_dim), int(rows))))
 
 
 def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_tables, qstart, qlen, ctx, tile_seq,
@@ -307,9 +309,10 @@ def latent_attention(qa, q, dim, rot_dim, positions, cos_sin, cache, block_table
     H, n_entries = qa.shape[0], int(tile_seq.numel())
     if mfma is None:
         mfma = os.environ.get("DLLM_LATENT_MFMA", "1") == "1"
-    matrix = bool(mfma) and qa.dtype == torch.bfloat16 and bool(ext.latent_mfma_ok(int(qa.shape[2]), int(rot_dim), int(rows)))
-    vector = 0 if matrix else latent_vector_wgs(qa.shape[2], rot_dim)
-    sp = latent_splits(n_entries, H, rows, _cus(qa), vector) if splits is None else int(splits)
+    if splits is None:      # (``up`` is the matrix-core form's)
+        matrix = up is not None or (bool(mfma) and qa.dtype == torch.bfloat16 and bool(ext.latent_mfma_ok(int(qa.shape[2]), int(rot_dim), int(rows))))
+        splits = latent_splits(n_entries, H, rows, _cus(qa.device), 0 if matrix else latent_vector_wgs(qa.shape[2], rot_dim))
+    sp = int(splits)
     po = pml = None
     if sp > 1:
         gx = ((1 if H >= rows else rows // H) * H + rows - 1) // rows
